@@ -1,7 +1,10 @@
 // GEMM entry point of the Gemm / SmoothQuantGemm / WeightOnlyQuantMatmul plugins.
 //   M <= 8  -> the streaming GEMV (gemv.hip), the decode path;
-//   M  > 8  -> MFMA tiles: LDS-DMA staged (gemm_glds.hip: SQ / fp16, K-bytes % 128 == 0), else register staged with
-//              in-flight dequantisation (gemm_mfma.hip: weight-only types, odd K), else 8-row GEMV slabs.
+//   M 9..31 -> the weight-streaming MFMA product (gemm_slim.hip): a 19-token prompt's projections are bound by the weights, not by MFMA tiles
+//              (weight-only int8, 12288 x 4096 at 19 rows: 26 us; the 128 x 128 register-staged tiles took 116);
+//   M >= 32 -> MFMA tiles: LDS-DMA staged (gemm_glds.hip: SQ / fp16, K-bytes % 128 == 0; gemm_woq.hip: weight-only), else register staged
+//              with in-flight dequantisation (gemm_mfma.hip: odd K);
+//   shapes that none of these serves -> 8-row GEMV slabs.
 #include "dev_utils.h"
 #include <cstdlib>
 #include "kernels.h"
@@ -14,6 +17,7 @@ namespace kernels
 
 int launch_gemm_mfma(const GemmParams& p, hipStream_t stream); // gemm_mfma.hip; returns 1 when the shape is unsupported
 int launch_gemm_woq(const GemmParams& p, hipStream_t stream);  // gemm_woq.hip (weight-only, dequantisation in the main loop); same
+int launch_gemm_slim(const GemmParams& p, hipStream_t stream); // gemm_slim.hip (few rows, every type); same
 int launch_gemm_glds(const GemmParams& p, hipStream_t stream); // gemm_glds.hip (SQ / fp16, LDS-DMA staged); same convention
 
 using namespace dev;
@@ -78,7 +82,7 @@ int launch_gemm(const GemmParams& pin, hipStream_t stream)
             // weight-only at prefill sizes: the u8 / nibble tile by LDS-DMA, dequantised between LDS and the MFMA fragments -
             // no fp16 image of the weights (r01 / r02 expanded the matrix to fp16 in a scratch buffer on every call: 3 N K bytes
             // of HBM traffic the algorithm does not have; removed in r05, profiles/r03_woq_gemm_sweep.txt).  Shapes it does not
-            // serve (K % 64 != 0, M < 32) take the register-staged kernel below.
+            // serve (M < 32, K % 64 != 0) take the kernels below.
             const int r = launch_gemm_woq(pin, stream);
             if (r <= 0)
                 return r;
@@ -110,7 +114,9 @@ int launch_gemm(const GemmParams& pin, hipStream_t stream)
     };
     if (p.M > 8)
     {
-        const int r = launch_gemm_mfma(p, stream);
+        int r = p.M < 32 ? launch_gemm_slim(p, stream) : 1;
+        if (r > 0)
+            r = launch_gemm_mfma(p, stream);
         if (r <= 0)
             return finish(r);
     }

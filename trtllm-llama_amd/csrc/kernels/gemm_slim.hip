@@ -1,0 +1,112 @@
+// Products of 9 .. 31 rows on the LLaMA path (short prompts): fp16, SmoothQuant int8, weight-only int8 / int4 weights through the
+// weight-streaming main loop of gemm_slim_impl.h.  The epilogue has the rounding points of the tiles in gemm_mfma.hip.
+#include "gemm_slim_impl.h"
+#include "kernels.h"
+#include "launch_util.h"
+#include "weight_layout.h"
+
+namespace tllm
+{
+namespace kernels
+{
+using namespace dev;
+
+namespace
+{
+
+template <int WT, int MT, int D, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void gemm_slim_kernel(const GemmParams p)
+{
+    __shared__ __attribute__((aligned(16))) char lds[slim::lds_bytes<MT, WAVES>()];
+    constexpr bool SQ = WT == W_INT8_SQ;
+    const int lane = threadIdx.x & 63;
+    const int n0 = blockIdx.x * 16;
+    const char* xrow[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+    {
+        const int m = 16 * t + (lane & 15);
+        xrow[t] = reinterpret_cast<const char*>(p.a) + (int64_t) (m < p.M ? m : p.M - 1) * p.lda * (SQ ? 1 : 2);
+    }
+    const int wbytes = WT == W_FP16 ? p.K * 2 : (WT == W_INT4_WOQ ? p.K / 2 : p.K);
+    slim::product<WT, MT, D, WAVES>(lds, reinterpret_cast<const char*>(p.w) + (int64_t) n0 * p.ldw, p.ldw, p.N - n0, wbytes, xrow,
+        [&](int t, const typename slim::Traits<WT>::acc_t& acc) {
+            const int row = 16 * t + (lane & 15), col0 = n0 + 4 * (lane >> 4);
+            if (row >= p.M)
+                return;
+            const float sr = SQ ? (p.per_token ? p.scale_row[row] : p.scale_row[0]) : 1.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+            {
+                const int col = col0 + e;
+                if (col >= p.N)
+                    continue;
+                float v;
+                if constexpr (SQ)
+                    v = (float) acc[e] * ((p.per_channel ? reinterpret_cast<const float*>(p.scale_col)[col] : reinterpret_cast<const float*>(p.scale_col)[0]) * sr);
+                else if constexpr (WT == W_FP16)
+                    v = acc[e];
+                else
+                    v = acc[e] * h2f(reinterpret_cast<const uint16_t*>(p.scale_col)[col]);
+                const int64_t o = (int64_t) row * p.ldc + col;
+                if (p.out_dtype == DT_HALF)
+                    reinterpret_cast<uint16_t*>(p.c)[o] = f2h(v);
+                else if (SQ && p.out_dtype == DT_INT32)
+                    reinterpret_cast<int32_t*>(p.c)[o] = f2i32_rni_sat(v);
+                else
+                    reinterpret_cast<float*>(p.c)[o] = v;
+            }
+        });
+}
+
+template <int WT, int MT, int D, int WAVES>
+int go(const GemmParams& p, hipStream_t stream)
+{
+    hipLaunchKernelGGL((gemm_slim_kernel<WT, MT, D, WAVES>), dim3((p.N + 15) / 16), dim3(WAVES * 64), 0, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+    {
+        set_error("gemm_slim launch failed: %s", hipGetErrorString(e));
+        return -1;
+    }
+    return 0;
+}
+
+template <int WT>
+int launch_wt(const GemmParams& p, hipStream_t stream)
+{
+    // (the line between the launch shapes: gemm_slim_impl.h.  Two row tiles: 12288 x 4096 weight-only int8 at 19 rows 26.0 us on 4 waves,
+    // 27.9 on 8; 4096 x 11008 26.8 and 21.1)
+    const bool many = (p.N + 15) / 16 * 4 >= launch_util::device_cus() * 5;
+    if (p.M <= 16)
+        return many ? go<WT, 1, 1, 4>(p, stream) : go<WT, 1, 1, 8>(p, stream);
+    return many ? go<WT, 2, 1, 4>(p, stream) : go<WT, 2, 1, 8>(p, stream);
+}
+
+} // namespace
+
+// 0: launched, -1: launch error, 1: not served (row counts, alignment)
+int launch_gemm_slim(const GemmParams& p, hipStream_t stream)
+{
+    const int a_es = p.wtype == W_INT8_SQ ? 1 : 2;
+    if (p.M < 1 || p.M > 32 || p.N < 1 || p.K < 1 || p.residual || p.silu_gate)
+        return 1;
+    // 16-byte loads of both operands; 32-bit offsets of a workgroup's W rows
+    if ((reinterpret_cast<uintptr_t>(p.a) & 15) || ((p.lda * a_es) & 15) || (reinterpret_cast<uintptr_t>(p.w) & 15) || (p.ldw & 15) || p.ldw > (1 << 26))
+        return 1;
+    if ((p.K * a_es) % 16 || (p.wtype == W_INT8_WOQ && p.K % 16) || (p.wtype == W_INT4_WOQ && p.K % 32))
+        return 1;
+    if (p.out_dtype != DT_HALF && p.out_dtype != DT_FLOAT && !(p.out_dtype == DT_INT32 && p.wtype == W_INT8_SQ))
+        return 1;
+    switch (p.wtype)
+    {
+    case W_FP16: return launch_wt<W_FP16>(p, stream);
+    case W_INT8_SQ: return launch_wt<W_INT8_SQ>(p, stream);
+    case W_INT8_WOQ: return launch_wt<W_INT8_WOQ>(p, stream);
+    case W_INT4_WOQ: return launch_wt<W_INT4_WOQ>(p, stream);
+    default: return 1;
+    }
+}
+
+} // namespace kernels
+} // namespace tllm

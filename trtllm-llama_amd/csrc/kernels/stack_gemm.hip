@@ -2,14 +2,16 @@
 //
 //   bfloat16, M >= 32, K % 64 == 0: the LDS-DMA staged MFMA tiles of gemm_glds_impl.h instantiated for bfloat16 operands
 //                     (v_mfma_f32_32x32x16_bf16), tile shape by the same rounds x area rule as the fp16 form;
-//   bfloat16, other M > 8: the register-staged MFMA tiles of gemm_mfma.hip;
-//   bfloat16, M <= 8: skinny_kernel below - HBM-bound, a wave streams R weight rows with 16-byte non-temporal loads and keeps the
-//                     M activation rows' chunks in registers; fp32 accumulation, DPP reduction;
+//   bfloat16, other M >= 32: the register-staged MFMA tiles of gemm_mfma.hip;
+//   bfloat16, M <= 31: slim_kernel below - HBM-bound, the weight-streaming MFMA main loop of gemm_slim_impl.h;
+//   bfloat16, M = 1 but for long rows of few columns: skinny_kernel - a wave streams 2 weight rows with 16-byte non-temporal loads and keeps the
+//                     activation row's chunks in registers; fp32 accumulation, DPP reduction; few columns, M <= 8: its form whose waves split K;
 //   float32         : fma_tile_kernel - 64 x 64 tiles of plain fp32 FMAs through LDS (no reduced-precision matrix mode), any shape;
 //                     also the fallback for bfloat16 operands whose rows are not 16-byte aligned.
 #include "dev_utils.h"
 #include "gemm_glds_impl.h"
 #include "gemm_seam.h"
+#include "gemm_slim_impl.h"
 #include "stack_kernels.h"
 #include <cstdlib>
 
@@ -74,11 +76,10 @@ __device__ __forceinline__ void seam_pair(const StackGemmParams& p, int row, int
     seam_store_pair<DT == DT_FLOAT>(p.seam, p.act, p.c, p.ldc, p.out_f32 != 0, row, col, v0, v1, has1);
 }
 
-// operands of product blockIdx.z of a batched launch
+// operands of product b of a batched launch
 template <int DT>
-__device__ __forceinline__ StackGemmParams batch_slice(StackGemmParams p)
+__device__ __forceinline__ StackGemmParams batch_slice(StackGemmParams p, int64_t b)
 {
-    const int64_t b = blockIdx.z;
     constexpr int ES = DT == DT_BF16 ? 2 : 4;
     p.a = reinterpret_cast<const char*>(p.a) + b * p.stride_a * ES;
     p.w = reinterpret_cast<const char*>(p.w) + b * p.stride_w * ES;
@@ -104,7 +105,7 @@ constexpr int TM = 64, TN = 64, TK = 16;
 template <int DT>
 __global__ __launch_bounds__(256) void fma_tile_kernel(const StackGemmParams p_in)
 {
-    const StackGemmParams p = batch_slice<DT>(p_in);
+    const StackGemmParams p = batch_slice<DT>(p_in, blockIdx.z);
     __shared__ int64_t row_s[TM]; // where the tile's rows of a start
     __shared__ float As[TK][TM + 4];
     __shared__ float Ws[TK][TN + 4];
@@ -160,28 +161,42 @@ __global__ __launch_bounds__(256) void fma_tile_kernel(const StackGemmParams p_i
         }
 }
 
-// bfloat16, M <= MR rows: 4 waves per workgroup, R weight rows per wave
+// Group blockIdx.z of a grouped launch whose grid holds fewer products than there are groups: the blockIdx.z-th one that has rows (a step of
+// few tokens reaches few experts; 32 x 352 workgroups of which 4 x 352 have work cost more to start than to run).  -1: there is none.
+__device__ __forceinline__ int nth_group(const int32_t* off, int groups, int nth)
+{
+    const int lane = threadIdx.x & 63;
+    for (int g0 = 0; g0 < groups; g0 += 64)
+    {
+        const int g = g0 + lane;
+        uint64_t has = __ballot(g < groups && off[g + 1] > off[g]);
+        const int n = __popcll(has);
+        if (nth < n)
+        {
+            for (; nth > 0; --nth)
+                has &= has - 1;
+            return g0 + __ffsll((unsigned long long) has) - 1;
+        }
+        nth -= n;
+    }
+    return -1;
+}
+
+// bfloat16, one row: 4 waves per workgroup, SK_R weight rows per wave
 constexpr int SK_R = 2;
 
-template <int MR>
-__global__ __launch_bounds__(256) void skinny_kernel(const StackGemmParams p_in)
+__global__ __launch_bounds__(256) void skinny_kernel(const StackGemmParams p_in, int groups)
 {
-    const StackGemmParams p = batch_slice<DT_BF16>(p_in);
+    int b = blockIdx.z;
+    if (groups && (b = nth_group(p_in.group_off, groups, b)) < 0)
+        return;
+    const StackGemmParams p = batch_slice<DT_BF16>(p_in, b);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int n0 = (blockIdx.x * 4 + wid) * SK_R;
     if (n0 >= p.N || p.M <= 0)
         return;
-    float acc[SK_R][MR];
-#pragma unroll
-    for (int r = 0; r < SK_R; ++r)
-#pragma unroll
-        for (int m = 0; m < MR; ++m)
-            acc[r][m] = 0.f;
-    const uint16_t* a = reinterpret_cast<const uint16_t*>(p.a);
-    int64_t arow[MR]; // where the rows of a start (p.M of them)
-#pragma unroll
-    for (int m = 0; m < MR; ++m)
-        arow[m] = m < p.M ? (int64_t) (p.a_rows ? p.a_rows[m] : m) * p.lda : 0;
+    float acc[SK_R] = {0.f, 0.f};
+    const uint16_t* a = reinterpret_cast<const uint16_t*>(p.a) + (int64_t) (p.a_rows ? p.a_rows[0] : 0) * p.lda;
     const uint16_t* w = reinterpret_cast<const uint16_t*>(p.w);
     for (int k = lane * 8; k < p.K; k += 64 * 8)
     {
@@ -189,34 +204,62 @@ __global__ __launch_bounds__(256) void skinny_kernel(const StackGemmParams p_in)
 #pragma unroll
         for (int r = 0; r < SK_R; ++r)
             wv[r] = n0 + r < p.N ? ld_nt16(w + (int64_t) (n0 + r) * p.ldw + k) : make_uint4(0, 0, 0, 0);
+        const uint4 xv = *reinterpret_cast<const uint4*>(a + k);
+        const uint32_t xs[4] = {xv.x, xv.y, xv.z, xv.w};
 #pragma unroll
-        for (int m = 0; m < MR; ++m)
+        for (int r = 0; r < SK_R; ++r)
         {
-            if (m >= p.M)
-                break;
-            const uint4 xv = *reinterpret_cast<const uint4*>(a + arow[m] + k);
-            const uint32_t xs[4] = {xv.x, xv.y, xv.z, xv.w};
+            const uint32_t ws[4] = {wv[r].x, wv[r].y, wv[r].z, wv[r].w};
 #pragma unroll
-            for (int r = 0; r < SK_R; ++r)
+            for (int i = 0; i < 4; ++i)
             {
-                const uint32_t ws[4] = {wv[r].x, wv[r].y, wv[r].z, wv[r].w};
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                {
-                    acc[r][m] = fmaf(__builtin_bit_cast(float, xs[i] << 16), __builtin_bit_cast(float, ws[i] << 16), acc[r][m]);
-                    acc[r][m] = fmaf(__builtin_bit_cast(float, xs[i] & 0xffff0000u), __builtin_bit_cast(float, ws[i] & 0xffff0000u), acc[r][m]);
-                }
+                acc[r] = fmaf(__builtin_bit_cast(float, xs[i] << 16), __builtin_bit_cast(float, ws[i] << 16), acc[r]);
+                acc[r] = fmaf(__builtin_bit_cast(float, xs[i] & 0xffff0000u), __builtin_bit_cast(float, ws[i] & 0xffff0000u), acc[r]);
             }
         }
     }
     static_assert(SK_R == 2, "a wave's rows are one pair of columns");
+    const float s0 = wave_sum(acc[0]), s1 = wave_sum(acc[1]);
+    if (lane == 0)
+        seam_pair<DT_BF16>(p, 0, n0, s0, s1);
+}
+
+// bfloat16, M <= 16 * MT rows: the main loop of gemm_slim_impl.h, a workgroup per 16 columns and product
+template <int MT, int D, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void slim_kernel(const StackGemmParams p_in, int groups)
+{
+    __shared__ __attribute__((aligned(16))) char lds[slim::lds_bytes<MT, WAVES>()];
+    int b = blockIdx.z;
+    if (groups && (b = nth_group(p_in.group_off, groups, b)) < 0)
+        return;
+    const StackGemmParams p = batch_slice<DT_BF16>(p_in, b);
+    if (p.M <= 0)
+        return;
+    const int lane = threadIdx.x & 63, n0 = blockIdx.x * 16;
+    const char* xrow[MT];
 #pragma unroll
-    for (int m = 0; m < MR; ++m)
+    for (int t = 0; t < MT; ++t)
     {
-        const float s0 = wave_sum(acc[0][m]), s1 = wave_sum(acc[1][m]);
-        if (lane == 0 && m < p.M)
-            seam_pair<DT_BF16>(p, m, n0, s0, s1);
+        int m = 16 * t + (lane & 15);
+        m = m < p.M ? m : p.M - 1;
+        xrow[t] = reinterpret_cast<const char*>(p.a) + (int64_t) (p.a_rows ? p.a_rows[m] : m) * p.lda * 2;
     }
+    slim::product<W_BF16, MT, D, WAVES>(lds, reinterpret_cast<const char*>(p.w) + (int64_t) n0 * p.ldw * 2, p.ldw * 2, p.N - n0, p.K * 2, xrow,
+        [&](int t, const slim::f32x4& acc) {
+            const int row = 16 * t + (lane & 15), col = n0 + 4 * (lane >> 4);
+            if (row >= p.M)
+                return;
+            if (col < p.N)
+                seam_pair<DT_BF16>(p, row, col, acc[0], acc[1]);
+            if (col + 2 < p.N)
+                seam_pair<DT_BF16>(p, row, col + 2, acc[2], acc[3]);
+        });
+}
+
+template <int MT, int D, int WAVES>
+void launch_slim(const StackGemmParams& p, int products, int groups, hipStream_t stream)
+{
+    hipLaunchKernelGGL((slim_kernel<MT, D, WAVES>), dim3((p.N + 15) / 16, 1, products), dim3(WAVES * 64), 0, stream, p, groups);
 }
 
 // The same for products of few rows of W (a token input's gate): a workgroup per SK_R rows whose 4 waves split K, so that the weights are
@@ -388,11 +431,16 @@ int launch_stack_gemm(const StackGemmParams& p_in, hipStream_t stream)
     }
     const bool aligned = !(reinterpret_cast<uintptr_t>(p.a) & 15) && !(reinterpret_cast<uintptr_t>(p.w) & 15) && p.K % 8 == 0 && p.lda % 8 == 0 && p.ldw % 8 == 0
         && (p.batch == 1 || (p.stride_a % 8 == 0 && p.stride_w % 8 == 0));
-    if (aligned && p.M <= 8)
+    if (aligned && p.M < 32 && p.ldw < (1 << 26))
     {
-        const dim3 grid((p.N + 4 * SK_R - 1) / (4 * SK_R), 1, p.batch);
-        if (p.batch == 1 && !p.group_off && (int) grid.x * 2 <= launch_util::device_cus() && p.K >= 2048)
+        const int cus = launch_util::device_cus();
+        // a grouped step of few rows: as many products as groups can have rows
+        const bool few = p.group_off && p.group_total < p.batch;
+        const int products = few ? p.group_total : p.batch, groups = few ? p.batch : 0;
+        const int64_t slim_wgs = (int64_t) ((p.N + 15) / 16) * products;
+        if (p.batch == 1 && !p.group_off && p.M <= 8 && (p.N + 7) / 8 * 2 <= cus && p.K >= 2048)
         {
+            // 1024 x 2048: 3.4 / 4.0 / 5.2 us at one / four / eight rows, the MFMA form 5.1 .. 6.2
             const dim3 kg((p.N + SK_R - 1) / SK_R);
             if (p.M <= 1)
                 hipLaunchKernelGGL((skinny_ksplit_kernel<1>), kg, dim3(256), 0, stream, p);
@@ -402,13 +450,19 @@ int launch_stack_gemm(const StackGemmParams& p_in, hipStream_t stream)
                 hipLaunchKernelGGL((skinny_ksplit_kernel<8>), kg, dim3(256), 0, stream, p);
             return launched("stack_gemm skinny (K over waves)");
         }
-        if (p.M <= 1)
-            hipLaunchKernelGGL((skinny_kernel<1>), grid, dim3(256), 0, stream, p);
-        else if (p.M <= 4)
-            hipLaunchKernelGGL((skinny_kernel<4>), grid, dim3(256), 0, stream, p);
+        if (p.M <= 1 && (slim_wgs > cus || p.K < 4096))
+        {
+            // one row: 32000 x 2048 22.4 us against the MFMA form's 28.0, 11008 x 2048 10.4 / 12.3, 2048 x 2048 5.4 / 6.2; long rows of few
+            // columns want the MFMA form, whose waves split K: 4096 x 4096 9.7 against 10.8, 4096 x 11008 20.3 / 21.4, 2048 x 5504 9.7 / 10.3
+            hipLaunchKernelGGL(skinny_kernel, dim3((p.N + 4 * SK_R - 1) / (4 * SK_R), 1, products), dim3(256), 0, stream, p, groups);
+            return launched("stack_gemm skinny");
+        }
+        const bool many = slim_wgs * 4 >= cus * 5; // (gemm_slim_impl.h)
+        if (p.M <= 16)
+            many ? launch_slim<1, 1, 4>(p, products, groups, stream) : launch_slim<1, 2, 8>(p, products, groups, stream);
         else
-            hipLaunchKernelGGL((skinny_kernel<8>), grid, dim3(256), 0, stream, p);
-        return launched("stack_gemm skinny");
+            many ? launch_slim<2, 1, 4>(p, products, groups, stream) : launch_slim<2, 1, 8>(p, products, groups, stream);
+        return launched("stack_gemm slim");
     }
     const int64_t tiles128 = (int64_t) ((p.M + 127) / 128) * ((p.N + 127) / 128);
     if (aligned && p.split_ws && p.batch == 1 && p.M >= 32 && tiles128 * 2 <= launch_util::device_cus())
