@@ -1,0 +1,712 @@
+// The recurrences of the stack engine's state layers (HGRN2, gated delta rule, Mamba-2) over prompts, 16 rows at a time.
+//
+// All three are  S <- diag(f_t) S + k_t u_t^T,  o_t = S^T q_t  with a state S [D, V] per head in fp32 (HGRN2: u = v, k = 1 - f; delta rule: u_t =
+// beta_t (v_t - (diag(f_t) S)^T k_t); Mamba-2: one f per head, k = dt B, u = x).  Row by row that is a chain of rows: 1.0 ms for 1024 rows
+// whatever the width, the chip idle (a row took 1 us of dependent latency).  With b_t = f_1 ... f_t inside a chunk of 16 rows,
+//   o_t = (b_t q_t)^T S_0 + sum_{s <= t} P[t, s] u_s,   P[t, s] = sum_d q_t[d] k_s[d] f_{s+1}[d] ... f_t[d]
+//   S_16 = b_16 S_0 + sum_s (k_s f_{s+1} ... f_16) u_s^T
+//   delta rule:  u = T (v - (b k)^T S_0),  T = (I + diag(beta) M)^-1 diag(beta),  M[t, s] = sum_d k_t[d] k_s[d] f_{s+1}[d] ... f_t[d], s < t
+// so only S_0 -> S_16 is a chain, of matrix products.  Every decay is a product of the factors between two rows (never a quotient of cumulative
+// products: nothing underflows into 0 / 0 whatever the gates), all sums are fp32 (v_mfma_f32_16x16x4_f32, no reduced-precision matrix
+// mode) in both element types.
+//
+// Two launches.  chunk_prepare_kernel / ssm_prepare_kernel: a workgroup per (chunk, head), resp. (chunk, group), all chunks at once: gates, unit
+// norms, the decayed vectors, P, M and T into scratch.  chunk_walk_kernel: a workgroup per (entry, head, 16 columns of V) walks the chunks; its
+// four waves keep the state's rows in turn, 16 at a time, in registers in the MFMA's accumulator layout (lane: column lane & 15, rows 4 (lane >> 4)
+// + i), which is also its B-operand layout when the four K = 4 steps of 16 rows take rows 4 g + i in step i: S, u and v go from product to
+// product without moving, and what comes from scratch is 16 bytes per lane.  One barrier per chunk, where the waves' partial o (and S^T k)
+// meet; the next chunk's operands are in flight under this one's products.
+//
+// Measured (us, both launches, 16 heads): HGRN2 128 x 128, 1024 rows 1024 -> 68; delta rule 128 x 128, three prompts of 683 rows in all 1740 1193 -> 119;
+// Mamba-2 64 heads 128 x 64, 1021 rows 400 -> 70.
+#include "dev_utils.h"
+#include "launch_util.h"
+#include "stack_chunk.h"
+#include "stack_kernels.h"
+#include <algorithm>
+#include <type_traits>
+
+namespace tllm
+{
+namespace kernels
+{
+using namespace dev;
+
+namespace
+{
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <int DT>
+__device__ __forceinline__ float ld_el(const void* p, int64_t i)
+{
+    if constexpr (DT == DT_BF16)
+        return bf2f(reinterpret_cast<const uint16_t*>(p)[i]);
+    else
+        return reinterpret_cast<const float*>(p)[i];
+}
+
+enum Mode
+{
+    HGRN = 0,
+    DELTA = 1,
+    SSM = 2
+};
+
+// What the three kinds have in common, filled by the launchers below.
+struct ChunkArgs
+{
+    int32_t heads = 0, D = 0, V = 0, groups = 1, entries = 0, slots = 0;
+    // HGRN: q at proj column h D, f at heads D + h D, v at 2 heads D + h V.  DELTA: x = [q | k | v].  SSM: xbc = [x | B | C], proj = [z | ... | dt]
+    const void* proj = nullptr;
+    int64_t ldp = 0;
+    const void* xbc = nullptr;
+    int64_t ldx = 0;
+    int32_t qk_heads = 0;
+    const float* f_bias = nullptr; // HGRN
+    const float* lower = nullptr;
+    const float* decay_raw = nullptr; // DELTA
+    const float* dt_bias = nullptr;   // DELTA, SSM
+    const float* a_log = nullptr;
+    const void* beta_raw = nullptr;
+    int64_t ld_beta = 0;
+    const float* d_skip = nullptr; // SSM
+    float* state = nullptr;
+    float* out = nullptr; // [tokens, heads V]
+    const int32_t* ent_slot = nullptr;
+    const int32_t* ent_first = nullptr;
+    const int32_t* ent_count = nullptr;
+    const int32_t* ent_pos0 = nullptr;
+    // scratch, by chunk slot c and head: the slot of an entry's chunk j is ent_first / 16 + entry + j
+    float* qt = nullptr; // [c][heads | groups][16][D]  b_t q_t, SSM: C
+    float* kb = nullptr; // [c][heads][16][D]  b_t k_t                        (DELTA)
+    float* kt = nullptr; // [c][heads | groups][D][16]  k_s f_{s+1} ... f_16, SSM: B transposed
+    float* pm = nullptr; // [c][heads][16][16] P
+    float* tm = nullptr; // [c][heads][16][16] T                              (DELTA)
+    float* bc = nullptr; // [c][heads][D] f_1 ... f_16; SSM: [c][heads][48] = {b_t}, {dt_s f_{s+1} ... f_16}, f_1 ... f_16 in [32]
+};
+
+// entry and chunk of a slot; false where the slot belongs to none
+__device__ __forceinline__ bool find_chunk(const ChunkArgs& a, int slot, int& e, int& j)
+{
+    const int lane = threadIdx.x & 63;
+    for (int e0 = 0; e0 < a.entries; e0 += 64)
+    {
+        const int i = e0 + lane;
+        int at = 0, n = 0;
+        if (i < a.entries)
+        {
+            at = a.ent_first[i] / CHUNK_ROWS + i;
+            n = (a.ent_count[i] + CHUNK_ROWS - 1) / CHUNK_ROWS;
+        }
+        const uint64_t mine = __ballot(slot >= at && slot < at + n);
+        if (mine)
+        {
+            const int l = __ffsll((unsigned long long) mine) - 1;
+            e = e0 + l;
+            j = slot - __shfl(at, l, 64);
+            return true;
+        }
+    }
+    return false;
+}
+
+__device__ __forceinline__ float sigmoid_f(float z)
+{
+    return 1.f / (1.f + expf(-z));
+}
+__device__ __forceinline__ float softplus_f(float z)
+{
+    return z > 20.f ? z : log1pf(expf(z));
+}
+// exp(-rate softplus(z)) as the row-by-row kernel takes it (stack_delta.hip)
+template <int DT>
+__device__ __forceinline__ float decay_of(float rate, float z)
+{
+    if constexpr (DT == DT_BF16)
+    {
+        constexpr float LOG2E = 1.4426950408889634f;
+        const float sp2 = z > 20.f ? z * LOG2E : __builtin_amdgcn_logf(1.f + __builtin_amdgcn_exp2f(z * LOG2E));
+        return __builtin_amdgcn_exp2f(-rate * sp2);
+    }
+    else
+        return expf(-rate * softplus_f(z));
+}
+
+constexpr int R = CHUNK_ROWS;
+
+// HGRN2 and delta rule: a workgroup per (chunk, head), D a multiple of 64 up to 256
+template <int DT, int MODE>
+__global__ __launch_bounds__(256) void chunk_prepare_kernel(const ChunkArgs a)
+{
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    const int D = a.D, h = blockIdx.y, slot = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    int e, j;
+    if (!find_chunk(a, slot, e, j))
+        return;
+    const int t0 = a.ent_first[e] + j * R, nt = min(R, a.ent_count[e] - j * R);
+    float* fs = sm;          // [R][D] decay
+    float* ks = fs + R * D;  // [R][D]
+    float* qs = ks + R * D;  // [R][D]
+    float* ms = qs + R * D;  // [R][R] M
+    float* bs = ms + R * R;  // [R] beta
+    const int hk = MODE == DELTA ? h / (a.heads / a.qk_heads) : 0;
+    const float rate = MODE == DELTA ? expf(a.a_log[h]) : 0.f;
+    for (int i = tid; i < R * D; i += 256)
+    {
+        const int t = i / D, d = i % D;
+        float f = 1.f, k = 0.f, q = 0.f; // a row past the entry's end leaves the state as it is
+        if (t < nt)
+        {
+            const int64_t r = t0 + t;
+            if constexpr (MODE == HGRN)
+            {
+                q = ld_el<DT>(a.proj, r * a.ldp + h * D + d);
+                q = q / (1.f + expf(-q));
+                if (DT == DT_BF16)
+                    q = bf2f(f2bf(q)); // the projection's activation is a bfloat16 value; everything behind it is fp32
+                const float lo = a.lower[h * D + d];
+                f = lo + (1.f - lo) * sigmoid_f(ld_el<DT>(a.proj, r * a.ldp + (a.heads + h) * D + d) + a.f_bias[h * D + d]);
+                k = 1.f - f;
+            }
+            else
+            {
+                q = ld_el<DT>(a.xbc, r * a.ldx + hk * D + d);
+                k = ld_el<DT>(a.xbc, r * a.ldx + (a.qk_heads + hk) * D + d);
+                f = decay_of<DT>(rate, a.decay_raw[r * a.heads * D + h * D + d] + a.dt_bias[h * D + d]);
+            }
+        }
+        fs[i] = f;
+        ks[i] = k;
+        qs[i] = q;
+    }
+    if (MODE == DELTA && tid < R)
+        bs[tid] = tid < nt ? sigmoid_f(ld_el<DT>(a.beta_raw, (int64_t) (t0 + tid) * a.ld_beta + h)) : 0.f;
+    __syncthreads();
+    if constexpr (MODE == DELTA)
+    {
+        // unit q (times dim^-1/2) and k: a wave per row
+        for (int t = wid; t < R; t += 4)
+        {
+            float sq = 0.f, sk = 0.f;
+            for (int d = lane; d < D; d += 64)
+            {
+                sq = fmaf(qs[t * D + d], qs[t * D + d], sq);
+                sk = fmaf(ks[t * D + d], ks[t * D + d], sk);
+            }
+            const float iq = 1.f / (sqrtf((float) D) * sqrtf(wave_sum(sq) + 1e-6f)), ik = 1.f / sqrtf(wave_sum(sk) + 1e-6f);
+            for (int d = lane; d < D; d += 64)
+            {
+                qs[t * D + d] *= iq;
+                ks[t * D + d] *= ik;
+            }
+        }
+        __syncthreads();
+    }
+    const int64_t ch = (int64_t) slot * a.heads + h;
+    // P and M: thread (row pair, channel pair): rows tp and 15 - tp against every row s, the decay between them built up as s goes down
+    {
+        const int dg = tid & 31, tp = tid >> 5;
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+        {
+            const int t = half ? R - 1 - tp : tp;
+            float pa[R], ma[R];
+#pragma unroll
+            for (int s = 0; s < R; ++s)
+                pa[s] = ma[s] = 0.f;
+            for (int d = dg * 2; d < D; d += 64)
+            {
+                float2 q = *reinterpret_cast<const float2*>(qs + t * D + d), k = *reinterpret_cast<const float2*>(ks + t * D + d);
+#pragma unroll
+                for (int s = R - 1; s >= 0; --s)
+                {
+                    if (s > t)
+                        continue;
+                    const float2 ksv = *reinterpret_cast<const float2*>(ks + s * D + d), f = *reinterpret_cast<const float2*>(fs + s * D + d);
+                    pa[s] = fmaf(q.x, ksv.x, fmaf(q.y, ksv.y, pa[s]));
+                    if (MODE == DELTA)
+                    {
+                        ma[s] = fmaf(k.x, ksv.x, fmaf(k.y, ksv.y, ma[s]));
+                        k.x *= f.x;
+                        k.y *= f.y;
+                    }
+                    q.x *= f.x; // q_t f_s ... f_t meets k_{s - 1}
+                    q.y *= f.y;
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < R; ++s)
+            {
+                pa[s] = group_sum<32>(pa[s]);
+                if (MODE == DELTA)
+                    ma[s] = group_sum<32>(ma[s]);
+            }
+            if (dg == 0)
+            {
+#pragma unroll
+                for (int s = 0; s < R; s += 4)
+                {
+                    *reinterpret_cast<float4*>(a.pm + ch * R * R + t * R + s) = make_float4(pa[s], pa[s + 1], pa[s + 2], pa[s + 3]);
+                    if (MODE == DELTA)
+                        *reinterpret_cast<float4*>(ms + t * R + s) = make_float4(ma[s], ma[s + 1], ma[s + 2], ma[s + 3]);
+                }
+            }
+        }
+    }
+    // the decayed vectors: forward from the chunk's start, backward from its end
+    for (int i = tid; i < 2 * D; i += 256)
+    {
+        const int d = i % D;
+        float w = 1.f;
+        if (i < D)
+        {
+#pragma unroll
+            for (int t = 0; t < R; ++t)
+            {
+                w *= fs[t * D + d];
+                a.qt[(ch * R + t) * D + d] = qs[t * D + d] * w;
+                if (MODE == DELTA)
+                    a.kb[(ch * R + t) * D + d] = ks[t * D + d] * w;
+            }
+            a.bc[ch * D + d] = w;
+        }
+        else
+        {
+            float o[R];
+#pragma unroll
+            for (int s = R - 1; s >= 0; --s)
+            {
+                o[s] = ks[s * D + d] * w;
+                w *= fs[s * D + d];
+            }
+#pragma unroll
+            for (int s = 0; s < R; s += 4)
+                *reinterpret_cast<float4*>(a.kt + (ch * D + d) * R + s) = make_float4(o[s], o[s + 1], o[s + 2], o[s + 3]);
+        }
+    }
+    if constexpr (MODE == DELTA)
+    {
+        __syncthreads();
+        // T by forward substitution, a thread per column
+        if (tid < R)
+        {
+            float x[R];
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+            {
+                float s0 = 0.f;
+#pragma unroll
+                for (int s = 0; s < i; ++s)
+                    s0 = fmaf(ms[i * R + s], x[s], s0);
+                x[i] = (i == tid ? 1.f : 0.f) - bs[i] * s0;
+            }
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+                a.tm[ch * R * R + i * R + tid] = x[i] * bs[tid];
+        }
+    }
+}
+
+// Mamba-2: a workgroup per (chunk, group): B transposed, C B^T once for the group's heads, then each head's decays
+template <int DT>
+__global__ __launch_bounds__(256) void ssm_prepare_kernel(const ChunkArgs a)
+{
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    const int D = a.D, g = blockIdx.y, slot = blockIdx.x, tid = threadIdx.x;
+    int e, j;
+    if (!find_chunk(a, slot, e, j))
+        return;
+    const int t0 = a.ent_first[e] + j * R, nt = min(R, a.ent_count[e] - j * R);
+    const int per = a.heads / a.groups, inner = a.heads * a.V, GN = a.groups * D, DP = D + 4;
+    float* bs = sm;            // [R][DP] (a row's end is padded: the rows of a column then fall on different banks)
+    float* cs = bs + R * DP;   // [R][DP]
+    float* dts = cs + R * DP;  // [per][R] step size
+    float* fs = dts + per * R; // [per][R] decay
+    for (int i = tid; i < R * D; i += 256)
+    {
+        const int t = i / D, d = i % D;
+        const int64_t r = t0 + min(t, nt - 1);
+        const float c = ld_el<DT>(a.xbc, r * a.ldx + inner + GN + g * D + d);
+        bs[t * DP + d] = ld_el<DT>(a.xbc, r * a.ldx + inner + g * D + d);
+        cs[t * DP + d] = c;
+        a.qt[((int64_t) slot * a.groups + g) * R * D + i] = c;
+    }
+    for (int i = tid; i < per * R; i += 256)
+    {
+        const int h = g * per + i / R, t = i % R;
+        float dt = 0.f, f = 1.f; // a row past the entry's end leaves the state as it is
+        if (t < nt)
+        {
+            dt = softplus_f(ld_el<DT>(a.proj, (int64_t) (t0 + t) * a.ldp + 2 * inner + 2 * GN + h) + a.dt_bias[h]);
+            f = expf(-expf(a.a_log[h]) * dt);
+        }
+        dts[i] = dt;
+        fs[i] = f;
+    }
+    __syncthreads();
+    const int64_t cg = (int64_t) slot * a.groups + g;
+    for (int i = tid; i < D * (R / 4); i += 256)
+    {
+        const int d = i / (R / 4), s = i % (R / 4) * 4;
+        *reinterpret_cast<float4*>(a.kt + (cg * D + d) * R + s) = make_float4(bs[s * DP + d], bs[(s + 1) * DP + d], bs[(s + 2) * DP + d], bs[(s + 3) * DP + d]);
+    }
+    const int t = tid >> 4, s = tid & 15;
+    float cb[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int d = 0; d < D; d += 4)
+    {
+        const float4 c4 = *reinterpret_cast<const float4*>(cs + t * DP + d), b4 = *reinterpret_cast<const float4*>(bs + s * DP + d);
+        cb[0] = fmaf(c4.x, b4.x, cb[0]);
+        cb[1] = fmaf(c4.y, b4.y, cb[1]);
+        cb[2] = fmaf(c4.z, b4.z, cb[2]);
+        cb[3] = fmaf(c4.w, b4.w, cb[3]);
+    }
+    const float dot = (cb[0] + cb[1]) + (cb[2] + cb[3]);
+    for (int i = 0; i < per; ++i)
+    {
+        const int64_t ch = (int64_t) slot * a.heads + g * per + i;
+        float w = s <= t ? dts[i * R + s] : 0.f;
+        for (int k = s + 1; k <= t; ++k)
+            w *= fs[i * R + k];
+        a.pm[ch * R * R + tid] = dot * w;
+    }
+    for (int i = tid; i < per * R; i += 256)
+    {
+        const int hh = i / R, tt = i % R;
+        float b = 1.f, w = dts[i];
+        for (int k = 0; k <= tt; ++k)
+            b *= fs[hh * R + k];
+        for (int k = tt + 1; k < R; ++k)
+            w *= fs[hh * R + k];
+        float* o = a.bc + ((int64_t) slot * a.heads + g * per + hh) * 48;
+        o[tt] = b;
+        o[R + tt] = w;
+        if (tt == R - 1)
+            o[2 * R] = b;
+    }
+}
+
+// One workgroup per (entry, head, 16 columns of V): TILES * 64 rows of state (D), wave w keeps rows 16 (w + 4 j) .. + 16
+template <int DT, int MODE, int TILES>
+__global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
+{
+    __shared__ f32x4 po[2][4][64], pr[MODE == DELTA ? 2 : 1][MODE == DELTA ? 4 : 1][64];
+    constexpr int D = TILES * 64;
+    const int e = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int c16 = lane & 15, g4 = lane >> 4;
+    const int v = blockIdx.z * 16 + c16, V = a.V, vc = v < V ? v : V - 1;
+    const int first = a.ent_first[e], count = a.ent_count[e], nchunk = (count + R - 1) / R;
+    const int64_t slot0 = first / R + e;
+    const int grp = MODE == SSM ? h / (a.heads / a.groups) : 0;
+    float* st = a.state + ((int64_t) a.ent_slot[e] * a.heads + h) * D * V;
+    const bool live = v < V, carry = a.ent_pos0[e] > 0;
+
+    f32x4 S[TILES];
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            S[j][i] = live && carry ? st[(int64_t) (16 * (wid + 4 * j) + 4 * g4 + i) * V + v] : 0.f;
+    const float dsk = MODE == SSM ? a.d_skip[h] : 0.f;
+
+    // a chunk's operands as this lane holds them; `raw` ones are converted where they are used, so that nothing waits at its load
+    typedef typename std::conditional<DT == DT_BF16, uint16_t, float>::type Raw;
+    struct Ops
+    {
+        f32x4 q[TILES], kb[MODE == DELTA ? TILES : 1], kt[TILES], b[MODE == SSM ? 1 : TILES], p, t;
+        f32x4 bt, ws; // SSM: b_t of this lane's rows, dt_s f_{s+1} ... f_16
+        Raw v[4], z;
+        float b16;
+    };
+    const Raw* vsrc = reinterpret_cast<const Raw*>(MODE == HGRN ? a.proj : a.xbc);
+    const int64_t vld = MODE == HGRN ? a.ldp : a.ldx;
+    const int64_t vcol = (MODE == HGRN ? 2 * a.heads * D : MODE == DELTA ? 2 * a.qk_heads * D : 0) + h * V + vc;
+    auto request = [&](int j, Ops& o) {
+        const int64_t slot = slot0 + j, ch = slot * a.heads + h, kg = MODE == SSM ? slot * a.groups + grp : ch;
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
+        {
+            const int d0 = 16 * (wid + 4 * n);
+            o.kt[n] = *reinterpret_cast<const f32x4*>(a.kt + (kg * D + d0 + c16) * R + 4 * g4);
+            o.q[n] = *reinterpret_cast<const f32x4*>(a.qt + (kg * R + c16) * D + d0 + 4 * g4);
+            if constexpr (MODE != SSM)
+                o.b[n] = *reinterpret_cast<const f32x4*>(a.bc + ch * D + d0 + 4 * g4);
+            if constexpr (MODE == DELTA)
+                o.kb[n] = *reinterpret_cast<const f32x4*>(a.kb + (ch * R + c16) * D + d0 + 4 * g4);
+        }
+        o.p = *reinterpret_cast<const f32x4*>(a.pm + ch * R * R + c16 * R + 4 * g4);
+        if constexpr (MODE == DELTA)
+            o.t = *reinterpret_cast<const f32x4*>(a.tm + ch * R * R + c16 * R + 4 * g4);
+        if constexpr (MODE == SSM)
+        {
+            o.bt = *reinterpret_cast<const f32x4*>(a.bc + ch * 48 + 4 * g4);
+            o.ws = *reinterpret_cast<const f32x4*>(a.bc + ch * 48 + R + 4 * g4);
+            o.b16 = a.bc[ch * 48 + 2 * R];
+            o.z = reinterpret_cast<const Raw*>(a.proj)[(int64_t) (first + min(j * R + 4 * g4 + wid, count - 1)) * a.ldp + h * V + vc];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            o.v[i] = vsrc[(int64_t) (first + min(j * R + 4 * g4 + i, count - 1)) * vld + vcol];
+    };
+    auto cvt = [](Raw r) -> float {
+        if constexpr (DT == DT_BF16)
+            return bf2f(r);
+        else
+            return r;
+    };
+    auto pick = [](const f32x4& x, int i) { return i < 2 ? (i ? x[1] : x[0]) : (i == 2 ? x[2] : x[3]); };
+
+    auto chunk = [&](int j, const Ops& o) {
+        const int buf = j & 1;
+        f32x4 u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            u[i] = cvt(o.v[i]);
+        // two sums per product: a product's next step waits for the one before
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc1 = acc, accr = acc, accr1 = acc;
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2)
+            {
+                if constexpr (MODE == DELTA)
+                {
+                    accr = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kb[n][i], S[n][i], accr, 0, 0, 0);
+                    accr1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kb[n][i + 1], S[n][i + 1], accr1, 0, 0, 0);
+                }
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[n][i], S[n][i], acc, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[n][i + 1], S[n][i + 1], acc1, 0, 0, 0);
+            }
+        acc = acc + acc1;
+        accr = accr + accr1;
+        if constexpr (MODE == SSM)
+            acc = acc * o.bt;
+        if constexpr (MODE != DELTA) // this wave's quarter of P u
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pick(o.p, wid), pick(u, wid), acc, 0, 0, 0);
+        po[buf][wid][lane] = acc;
+        if constexpr (MODE == DELTA)
+            pr[buf][wid][lane] = accr;
+        __syncthreads();
+        f32x4 out = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (MODE == DELTA)
+        {
+            const f32x4 x = u - ((pr[buf][0][lane] + pr[buf][1][lane]) + (pr[buf][2][lane] + pr[buf][3][lane]));
+            u = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                u = __builtin_amdgcn_mfma_f32_16x16x4f32(o.t[i], x[i], u, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                out = __builtin_amdgcn_mfma_f32_16x16x4f32(o.p[i], u[i], out, 0, 0, 0);
+        }
+        const f32x4 us = MODE == SSM ? u * o.ws : u;
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
+        {
+            if constexpr (MODE == SSM)
+                S[n] = S[n] * o.b16;
+            else
+                S[n] = S[n] * o.b[n];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                S[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kt[n][i], us[i], S[n], 0, 0, 0);
+        }
+        // wave w finishes rows 4 g + w
+        const float* pf = reinterpret_cast<const float*>(&po[buf][0][0]);
+        float y = ((pf[lane * 4 + wid] + pf[256 + lane * 4 + wid]) + (pf[512 + lane * 4 + wid] + pf[768 + lane * 4 + wid])) + pick(out, wid);
+        const int row = j * R + 4 * g4 + wid;
+        if constexpr (MODE == SSM)
+        {
+            const float z = cvt(o.z);
+            y = fmaf(dsk, pick(u, wid), y) * (z / (1.f + expf(-z)));
+        }
+        if (live && row < count)
+            a.out[(int64_t) (first + row) * (a.heads * V) + h * V + v] = y;
+    };
+
+    // Three sets of operands: a chunk's are requested two chunks ahead.  Every request is made (past the end the last chunk's once more): one
+    // under a condition would have the compiler wait as if it had not been made, for all that is in flight.
+    const int last = nchunk - 1;
+    if (last < 0)
+        return;
+    Ops o0, o1, o2;
+    request(0, o0);
+    request(min(1, last), o1);
+    for (int j = 0;; j += 3)
+    {
+        request(min(j + 2, last), o2);
+        chunk(j, o0);
+        if (j + 1 > last)
+            break;
+        request(min(j + 3, last), o0);
+        chunk(j + 1, o1);
+        if (j + 2 > last)
+            break;
+        request(min(j + 4, last), o1);
+        chunk(j + 2, o2);
+        if (j + 3 > last)
+            break;
+    }
+    if (live)
+    {
+#pragma unroll
+        for (int j = 0; j < TILES; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                st[(int64_t) (16 * (wid + 4 * j) + 4 * g4 + i) * V + v] = S[j][i];
+    }
+}
+
+inline int launched(const char* what)
+{
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+    {
+        set_error("%s launch failed: %s", what, hipGetErrorString(e));
+        return -1;
+    }
+    return 0;
+}
+
+template <int DT, int MODE>
+void walk(const ChunkArgs& a, hipStream_t stream)
+{
+    const dim3 grid(a.entries, a.heads, (a.V + 15) / 16);
+    switch (a.D / 64)
+    {
+    case 1: hipLaunchKernelGGL((chunk_walk_kernel<DT, MODE, 1>), grid, dim3(256), 0, stream, a); break;
+    case 2: hipLaunchKernelGGL((chunk_walk_kernel<DT, MODE, 2>), grid, dim3(256), 0, stream, a); break;
+    case 3: hipLaunchKernelGGL((chunk_walk_kernel<DT, MODE, 3>), grid, dim3(256), 0, stream, a); break;
+    default: hipLaunchKernelGGL((chunk_walk_kernel<DT, MODE, 4>), grid, dim3(256), 0, stream, a); break;
+    }
+}
+
+template <int DT, int MODE>
+int run(const ChunkArgs& a, hipStream_t stream)
+{
+    if constexpr (MODE == SSM)
+    {
+        const size_t lds = sizeof(float) * ((size_t) 2 * R * (a.D + 4) + 2 * (size_t) (a.heads / a.groups) * R);
+        hipLaunchKernelGGL((ssm_prepare_kernel<DT>), dim3(a.slots, a.groups), dim3(256), lds, stream, a);
+    }
+    else
+    {
+        const size_t lds = sizeof(float) * ((size_t) 3 * R * a.D + R * R + R);
+        hipLaunchKernelGGL((chunk_prepare_kernel<DT, MODE>), dim3(a.slots, a.heads), dim3(256), lds, stream, a);
+    }
+    walk<DT, MODE>(a, stream);
+    return launched("stack_chunk");
+}
+
+// carves the scratch; false where it does not hold the step
+bool carve(ChunkArgs& a, int mode, int tokens, float* ws, size_t floats)
+{
+    a.slots = stack_chunk_slots(tokens, a.entries);
+    const size_t c = a.slots, hd = (size_t) a.heads * a.D;
+    float* at = ws;
+    auto take = [&](size_t n) {
+        float* p = at;
+        at += n;
+        return p;
+    };
+    a.qt = take(c * (mode == SSM ? (size_t) a.groups * a.D : hd) * R);
+    if (mode == DELTA)
+        a.kb = take(c * hd * R);
+    a.kt = take(c * (mode == SSM ? (size_t) a.groups * a.D : hd) * R);
+    a.pm = take(c * a.heads * R * R);
+    if (mode == DELTA)
+        a.tm = take(c * a.heads * R * R);
+    a.bc = take(c * (mode == SSM ? (size_t) a.heads * 48 : hd));
+    return ws && (size_t) (at - ws) <= floats;
+}
+
+} // namespace
+
+size_t stack_chunk_floats(int32_t tokens, int32_t entries, int32_t heads, int32_t dim, int32_t copies)
+{
+    // copies: 2 vectors per row and head (HGRN2), 3 (delta rule); Mamba-2's B per group is no more than one per head
+    return (size_t) stack_chunk_slots(tokens, entries) * heads * ((size_t) dim * (R * copies + 1) + 2 * R * R + 48);
+}
+
+bool stack_chunk_serves(int32_t dim, int32_t max_count)
+{
+    // from two chunks on: a portion of 32 rows takes 32 us row by row
+    return dim % 64 == 0 && dim >= 64 && dim <= 256 && max_count >= 2 * R;
+}
+
+int launch_stack_chunk_hgrn2(const StackHgrnParams& p, hipStream_t stream)
+{
+    ChunkArgs a;
+    a.heads = p.heads;
+    a.D = p.dim;
+    a.V = p.vdim;
+    a.entries = p.entries;
+    a.proj = p.proj;
+    a.ldp = p.ldp;
+    a.f_bias = p.f_bias;
+    a.lower = p.lower;
+    a.state = p.state;
+    a.out = p.o32;
+    a.ent_slot = p.ent_slot;
+    a.ent_first = p.ent_first;
+    a.ent_count = p.ent_count;
+    a.ent_pos0 = p.ent_pos0;
+    if (!stack_chunk_serves(p.dim, p.max_count) || !carve(a, HGRN, p.tokens, p.chunk_ws, p.chunk_floats))
+        return 1;
+    return p.dtype == DT_BF16 ? run<DT_BF16, HGRN>(a, stream) : run<DT_FLOAT, HGRN>(a, stream);
+}
+
+int launch_stack_chunk_delta(const StackDeltaParams& p, hipStream_t stream)
+{
+    ChunkArgs a;
+    a.heads = p.heads;
+    a.qk_heads = p.qk_heads;
+    a.D = p.dim;
+    a.V = p.vdim;
+    a.entries = p.entries;
+    a.xbc = p.x;
+    a.ldx = 2 * (int64_t) p.qk_heads * p.dim + (int64_t) p.heads * p.vdim;
+    a.decay_raw = p.decay_raw;
+    a.dt_bias = p.dt_bias;
+    a.a_log = p.a_log;
+    a.beta_raw = p.beta_raw;
+    a.ld_beta = p.ld_beta;
+    a.state = p.state;
+    a.out = p.o32;
+    a.ent_slot = p.ent_slot;
+    a.ent_first = p.ent_first;
+    a.ent_count = p.ent_count;
+    a.ent_pos0 = p.ent_pos0;
+    if (!stack_chunk_serves(p.dim, p.max_count) || !carve(a, DELTA, p.tokens, p.chunk_ws, p.chunk_floats))
+        return 1;
+    return p.dtype == DT_BF16 ? run<DT_BF16, DELTA>(a, stream) : run<DT_FLOAT, DELTA>(a, stream);
+}
+
+int launch_stack_chunk_ssm(const StackSsmParams& p, hipStream_t stream)
+{
+    ChunkArgs a;
+    a.heads = p.heads;
+    a.groups = p.groups;
+    a.D = p.state;
+    a.V = p.vdim;
+    a.entries = p.entries;
+    a.proj = p.proj;
+    a.ldp = p.ldp;
+    a.xbc = p.xbc;
+    a.ldx = (int64_t) p.heads * p.vdim + 2 * (int64_t) p.groups * p.state;
+    a.dt_bias = p.dt_bias;
+    a.a_log = p.a_log;
+    a.d_skip = p.d_skip;
+    a.state = p.ssm_state;
+    a.out = p.y32;
+    a.ent_slot = p.ent_slot;
+    a.ent_first = p.ent_first;
+    a.ent_count = p.ent_count;
+    a.ent_pos0 = p.ent_pos0;
+    // (the heads of a group share a workgroup's LDS in the first launch)
+    if (!stack_chunk_serves(p.state, p.max_count) || p.heads / p.groups > 128 || !carve(a, SSM, p.tokens, p.chunk_ws, p.chunk_floats))
+        return 1;
+    return p.dtype == DT_BF16 ? run<DT_BF16, SSM>(a, stream) : run<DT_FLOAT, SSM>(a, stream);
+}
+
+} // namespace kernels
+} // namespace tllm

@@ -3,6 +3,7 @@
 // read-out are fp32 in both element types; `DT` is the storage type of the convolution's output and of the layer's output.
 #include "dev_utils.h"
 #include "launch_util.h"
+#include "stack_chunk.h"
 #include "stack_kernels.h"
 #include <algorithm>
 #include <cstdlib>
@@ -376,6 +377,10 @@ int launch_stack_delta_scan(const StackDeltaParams& p, hipStream_t stream)
         set_error("stack_delta_scan: a missing operand");
         return -1;
     }
+    // prompts: 16 rows at a time through matrix products
+    const int rc = launch_stack_chunk_delta(p, stream);
+    if (rc <= 0)
+        return rc;
     return p.dtype == DT_BF16 ? launch_scan<DT_BF16>(p, stream) : launch_scan<DT_FLOAT>(p, stream);
 }
 

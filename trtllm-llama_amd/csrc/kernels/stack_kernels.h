@@ -300,7 +300,12 @@ struct StackHgrnParams
     int32_t max_count = 0;         // host: the largest ent_count of the step
     float* o32 = nullptr;          // scratch [tokens, heads * vdim]
     void* out = nullptr;           // [tokens, heads * vdim]
+    float* chunk_ws = nullptr;     // optional scratch of the chunked form (stack_chunk_floats); without it rows go one by one
+    size_t chunk_floats = 0;
 };
+// floats of scratch that the chunked recurrences want for a step (stack_chunk.hip); copies: 2 HGRN2 and Mamba-2, 3 delta rule
+size_t stack_chunk_floats(int32_t tokens, int32_t entries, int32_t heads, int32_t dim, int32_t copies);
+bool stack_chunk_serves(int32_t dim, int32_t max_count); // a state of dim rows, the largest entry of the step
 int launch_stack_hgrn2(const StackHgrnParams& p, hipStream_t stream);
 bool stack_hgrn2_serves(int32_t dim, int32_t vdim); // shapes one of its two forms takes
 
@@ -340,6 +345,9 @@ struct StackSsmParams
     const int32_t* ent_first = nullptr;
     const int32_t* ent_count = nullptr;
     const int32_t* ent_pos0 = nullptr;
+    int32_t max_count = 0;          // host: the largest ent_count of the step
+    float* chunk_ws = nullptr;      // optional scratch of the chunked form, as above
+    size_t chunk_floats = 0;
 };
 int launch_stack_ssm_conv(const StackSsmParams& p, hipStream_t stream);
 int launch_stack_ssm_scan(const StackSsmParams& p, hipStream_t stream);
@@ -423,6 +431,8 @@ struct StackDeltaParams
     const int32_t* ent_count = nullptr;
     const int32_t* ent_pos0 = nullptr;
     int32_t max_count = 0;            // host: the largest ent_count of the step
+    float* chunk_ws = nullptr;        // optional scratch of the chunked form, as above
+    size_t chunk_floats = 0;
 };
 int launch_stack_delta_scan(const StackDeltaParams& p, hipStream_t stream);
 int launch_stack_delta_out(const StackDeltaParams& p, hipStream_t stream);

@@ -2,6 +2,7 @@
 // Everything that a norm, a softmax, a recurrence or the residual stream touches is fp32; `DT` is the storage type of
 // activations, weights and caches (bfloat16 or fp32).
 #include "dev_utils.h"
+#include "stack_chunk.h"
 #include "stack_kernels.h"
 #include <algorithm>
 #include <cmath>
@@ -1979,8 +1980,22 @@ int launch_stack_hgrn2(const StackHgrnParams& p, hipStream_t stream)
         set_error("stack_hgrn2: heads %d, dim %d, vdim %d is not a shape it serves (dim up to 512)", p.heads, p.dim, p.vdim);
         return -1;
     }
+    const int64_t nh = (int64_t) p.tokens * p.heads;
+    auto norm = [&]() {
+        const dim3 grid((unsigned) ((nh + 3) / 4));
+        if (p.dtype == DT_BF16)
+            hipLaunchKernelGGL((head_rmsnorm_kernel<DT_BF16>), grid, dim3(256), 0, stream, p.out, p.o32, p.norm_w, nh, p.vdim, p.eps);
+        else
+            hipLaunchKernelGGL((head_rmsnorm_kernel<DT_FLOAT>), grid, dim3(256), 0, stream, p.out, p.o32, p.norm_w, nh, p.vdim, p.eps);
+        return launched("stack_hgrn2 norm");
+    };
     {
-        // Long portions (a prompt): a head is cut into groups of 16 columns, one workgroup each, so that the sequential walk over
+        const int rc = launch_stack_chunk_hgrn2(p, stream); // prompts: 16 rows at a time through matrix products
+        if (rc <= 0)
+            return rc ? rc : norm();
+    }
+    {
+        // Long portions (a prompt) of shapes the chunked form does not serve: a head is cut into groups of 16 columns, one workgroup each, so that the sequential walk over
         // the rows runs on many CUs at once; the head norm is then a pass of its own.  Short portions and decoded tokens: one
         // workgroup holds the whole head (vdim <= 256) and norms it in the same launch.
         bool spread = p.max_count >= 32 || p.vdim > 256;
@@ -2036,14 +2051,7 @@ int launch_stack_hgrn2(const StackHgrnParams& p, hipStream_t stream)
                 return -1;
             if (fuse)
                 return 0;
-            const int64_t nh = (int64_t) p.tokens * p.heads;
-            if (p.dtype == DT_BF16)
-                hipLaunchKernelGGL((head_rmsnorm_kernel<DT_BF16>), dim3((unsigned) ((nh + 3) / 4)), dim3(256), 0, stream, p.out, p.o32, p.norm_w,
-                    nh, p.vdim, p.eps);
-            else
-                hipLaunchKernelGGL((head_rmsnorm_kernel<DT_FLOAT>), dim3((unsigned) ((nh + 3) / 4)), dim3(256), 0, stream, p.out, p.o32, p.norm_w,
-                    nh, p.vdim, p.eps);
-            return launched("stack_hgrn2 norm");
+            return norm();
         }
     }
     if (p.dim > 128)
@@ -2073,14 +2081,7 @@ int launch_stack_hgrn2(const StackHgrnParams& p, hipStream_t stream)
 #undef TLLM_HGRN
     if (launched("stack_hgrn2 scan"))
         return -1;
-    const int64_t nh = (int64_t) p.tokens * p.heads;
-    if (p.dtype == DT_BF16)
-        hipLaunchKernelGGL((head_rmsnorm_kernel<DT_BF16>), dim3((unsigned) ((nh + 3) / 4)), dim3(256), 0, stream, p.out, p.o32, p.norm_w, nh,
-            p.vdim, p.eps);
-    else
-        hipLaunchKernelGGL((head_rmsnorm_kernel<DT_FLOAT>), dim3((unsigned) ((nh + 3) / 4)), dim3(256), 0, stream, p.out, p.o32, p.norm_w, nh,
-            p.vdim, p.eps);
-    return launched("stack_hgrn2 norm");
+    return norm();
 }
 
 } // namespace kernels

@@ -3,6 +3,7 @@
 // enters the recurrence are fp32 in both element types; `DT` is the storage type of the projection and of the convolution's output.
 #include "dev_utils.h"
 #include "launch_util.h"
+#include "stack_chunk.h"
 #include "stack_kernels.h"
 #include <algorithm>
 #include <cstdlib>
@@ -432,6 +433,11 @@ int launch_stack_ssm_scan(const StackSsmParams& p, hipStream_t stream)
         return 0;
     if (!ssm_ok(p, "stack_ssm_scan"))
         return -1;
+    {
+        const int rc = launch_stack_chunk_ssm(p, stream); // prompts: 16 rows at a time through matrix products
+        if (rc <= 0)
+            return rc;
+    }
     static const bool plain_only = [] {
         const char* v = std::getenv("TLLM_STACK_SSM_PLAIN"); // measurement knob: 1 = every shape on the form without prefetch
         return v && v[0] == '1';

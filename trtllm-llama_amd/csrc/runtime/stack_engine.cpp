@@ -169,6 +169,8 @@ struct tllm_stack
     std::vector<void*> owned;
     // scratch, grown to the largest step seen
     int cap_tokens = 0, cap_want = 0, cap_ints = 0;
+    float* chunk_ws = nullptr; // scratch of the chunked recurrences
+    size_t chunk_floats = 0;
     float *x = nullptr, *x0 = nullptr, *o32 = nullptr, *logits = nullptr, *tap = nullptr, *y32 = nullptr;
     void *h1 = nullptr, *h2 = nullptr, *proj = nullptr, *q = nullptr, *ctx = nullptr, *act = nullptr, *hw = nullptr, *lat = nullptr;
     int32_t *ints = nullptr, *ids_out = nullptr, *pinned = nullptr;
@@ -195,14 +197,15 @@ struct tllm_stack
     }
     void free_scratch()
     {
-        void* all[] = {v_first, shared_z, split_ws, x_el, side_act, act_sh, route_z, x, x0, o32, logits, tap, y32, h1, h2, proj, q, ctx, act, hw, lat, ints, ids_out, xbc, cq, qfull, moe_a, moe_y, moe_w, moe_i,
+        void* all[] = {chunk_ws, v_first, shared_z, split_ws, x_el, side_act, act_sh, route_z, x, x0, o32, logits, tap, y32, h1, h2, proj, q, ctx, act, hw, lat, ints, ids_out, xbc, cq, qfull, moe_a, moe_y, moe_w, moe_i,
             h32, dl_a, dl_g, pairs};
         for (void* p : all)
             if (p)
                 (void) hipFree(p);
         x_el = side_act = act_sh = nullptr;
         v_first = nullptr;
-        route_z = split_ws = shared_z = nullptr;
+        route_z = split_ws = shared_z = chunk_ws = nullptr;
+        chunk_floats = 0;
         x = x0 = o32 = logits = tap = y32 = nullptr;
         h1 = h2 = proj = q = ctx = act = hw = lat = nullptr;
         ints = ids_out = nullptr;
@@ -387,6 +390,19 @@ int ensure_scratch(tllm_stack* s, int tokens, int want, int n_ints)
         HIP_OK(hipMalloc(&s->qfull, T * std::max(s->max_qfull, 1) * es));
         HIP_OK(hipMalloc((void**) &s->h32, (s->token_shift ? T * wd : 1) * 4));
         HIP_OK(hipMalloc(&s->pairs, T * std::max(s->max_pairs, 1) * es));
+        for (const auto& l : s->layers)
+        {
+            const int copies = l.kind == MIX_DELTA ? 3 : (l.kind == MIX_HGRN2 || l.kind == MIX_MAMBA2 ? 2 : 0);
+            if (copies && T >= 2 * 16 && stack_chunk_serves(l.dim, (int) T))
+                s->chunk_floats = std::max(s->chunk_floats, stack_chunk_floats((int) T, std::min((int) T, s->slots), l.heads, l.dim, copies));
+        }
+        if (s->chunk_floats && hipMalloc((void**) &s->chunk_ws, s->chunk_floats * 4) != hipSuccess)
+        {
+            // no room: such rows go one by one
+            (void) hipGetLastError();
+            s->chunk_ws = nullptr;
+            s->chunk_floats = 0;
+        }
         HIP_OK(hipMalloc((void**) &s->dl_a, T * std::max(s->max_hd, 1) * 4));
         HIP_OK(hipMalloc((void**) &s->dl_g, (s->max_hd ? T * std::max(s->max_ctx, 1) : 1) * 4));
         {
@@ -1504,6 +1520,8 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             dp.ent_count = d_count;
             dp.ent_pos0 = d_pos0;
             dp.max_count = max_count;
+            dp.chunk_ws = s->chunk_ws;
+            dp.chunk_floats = s->chunk_floats;
             return (launch_stack_delta_scan(dp, stream) || launch_stack_delta_out(dp, stream)) ? -1 : 0;
         }
         if (l.kind == MIX_MAMBA2)
@@ -1534,6 +1552,9 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             sp.ent_first = d_first;
             sp.ent_count = d_count;
             sp.ent_pos0 = d_pos0;
+            sp.max_count = max_count;
+            sp.chunk_ws = s->chunk_ws;
+            sp.chunk_floats = s->chunk_floats;
             // convolution + silu (and the sequence's new tail), the recurrence with skip and gate, the norm in parts of the row
             if (launch_stack_ssm_conv(sp, stream) || launch_stack_ssm_scan(sp, stream))
                 return -1;
@@ -1561,6 +1582,8 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             hp.ent_count = d_count;
             hp.ent_pos0 = d_pos0;
             hp.max_count = max_count;
+            hp.chunk_ws = s->chunk_ws;
+            hp.chunk_floats = s->chunk_floats;
             hp.o32 = s->o32;
             hp.out = s->ctx;
             return launch_stack_hgrn2(hp, stream);
