@@ -594,15 +594,17 @@ __global__ __launch_bounds__(64 * (WM * WN * KG + LW)) void gemm_glds_kernel(con
     {
         // plain fp32 rows (stored, or added to the residual stream): a 32 x 32 block at a time through the wave's LDS scratch, 16 bytes per
         // lane and access.  Element by element this was the longest part of a short product.
-        const bool plain = !p.bias && !p.act && !(N & 3) && !(p.seam.n_sec > 0 && n0 + BN > p.seam.sec[0].col0);
-        float* dst = p.resid ? (p.gate ? nullptr : p.resid) : (p.out_dtype == DT_FLOAT ? reinterpret_cast<float*>(p.c) : nullptr);
+        // (a gated residual as well: 1024 x 2048 x 2048 with a gate 19 us in 16-byte pieces, 57 element by element)
+        const bool plain = !p.bias && !p.act && !(N & 3) && !(p.seam.n_sec > 0 && n0 + BN > p.seam.sec[0].col0)
+            && (!p.gate || (!(p.ldg & 3) && !(reinterpret_cast<uintptr_t>(p.gate) & 7) && !(reinterpret_cast<uintptr_t>(p.gate_bias) & 15)));
+        float* dst = p.resid ? p.resid : (p.out_dtype == DT_FLOAT ? reinterpret_cast<float*>(p.c) : nullptr);
         const int64_t ldd = p.resid ? p.ldr : p.ldc;
         if (plain && dst && !(ldd & 3) && !(reinterpret_cast<uintptr_t>(dst) & 15))
         {
             constexpr int P4 = 36; // floats per scratch row: 16-byte aligned, rows spread over the banks
-            static_assert(32 * P4 * 4 <= 32 * (NT * 64 + 16), "the scratch of a wave");
+            static_assert((size_t) WM * WN * 32 * P4 * 4 <= (size_t) S * STAGE, "the waves' scratch must fit the operand stages");
             __syncthreads(); // every wave has finished reading the operand buffers
-            float* scr = reinterpret_cast<float*>(lds + wid * (32 * (NT * 64 + 16)));
+            float* scr = reinterpret_cast<float*>(lds + wid * (32 * P4 * 4));
 #pragma unroll
             for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -623,6 +625,15 @@ __global__ __launch_bounds__(64 * (WM * WN * KG + LW)) void gemm_glds_kernel(con
                             if (p.resid)
                             {
                                 const float4 o = *at;
+                                if (p.gate)
+                                {
+                                    const uint2 z2 = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(p.gate) + (int64_t) grow * p.ldg + gcol);
+                                    const float4 b4 = p.gate_bias ? *reinterpret_cast<const float4*>(p.gate_bias + gcol) : make_float4(0.f, 0.f, 0.f, 0.f);
+                                    v.x *= 1.f / (1.f + __expf(-(bf2f((uint16_t) z2.x) + b4.x)));
+                                    v.y *= 1.f / (1.f + __expf(-(bf2f((uint16_t) (z2.x >> 16)) + b4.y)));
+                                    v.z *= 1.f / (1.f + __expf(-(bf2f((uint16_t) z2.y) + b4.z)));
+                                    v.w *= 1.f / (1.f + __expf(-(bf2f((uint16_t) (z2.y >> 16)) + b4.w)));
+                                }
                                 v = make_float4(o.x + v.x, o.y + v.y, o.z + v.z, o.w + v.w);
                             }
                             *at = v;

@@ -343,18 +343,19 @@ inline int launched(const char* what)
     return 0;
 }
 
-// the lock-step tile shapes of the LDS-DMA kernel and what a tile of each kind costs per area (measured on fp16 operands; the
-// bfloat16 MFMA has the same rate and byte geometry): fewest workgroup rounds x area x cost
+// The tile shapes of the LDS-DMA kernel, all with stages of whole 128-byte lines and 8 waves, and what a tile of each kind costs per area when
+// the chip is full of them (measured, relative to 256 x 256; M 2048 .. 512, N 2048 .. 22016, K 2048 .. 11008): fewest workgroup rounds x
+// area x cost.  us, M x N x K, in brackets the 64-byte stages and 4-wave tiles these replaced:
+//   1024 x 2048 x 5504   128 x 64  38 (49)      2048 x 4096 x 4096   128 x 256  62 (81)      2048 x 22016 x 4096   256 x 256  332 (380)
+//   1024 x 6144 x 2048   128 x 192 30 (43)      2048 x 6144 x 4096   256 x 192  94 (102)     1024 x 13056 x 2048   256 x 256   57 (61)
 int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0)
 {
-    // m_expected: the rows a product of a grouped launch has on average (g.M is their bound, which sizes the grid): the tile shape is
-    // chosen for what is expected, or tall tiles would run half empty on every group
     struct Shape
     {
         int id, bm, bn;
         double f;
     };
-    static const Shape shapes[] = {{0, 128, 128, 1.40}, {1, 256, 192, 1.0}, {2, 256, 256, 1.04}, {3, 128, 256, 1.39}};
+    static const Shape shapes[] = {{0, 128, 128, 1.49}, {1, 256, 192, 1.16}, {2, 256, 256, 1.0}, {3, 128, 256, 1.15}, {4, 128, 192, 1.28}, {5, 128, 64, 2.15}};
     const int cus = launch_util::device_cus();
     double best = 1e30;
     int pick = 0;
@@ -369,19 +370,10 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
             pick = sh.id;
         }
     }
-    if (m_expected > 0)
-    {
-        // groups of up to two 128-row tiles: the small square tile (more, shorter workgroups behind the ones that leave at once)
-        // measured 9 % ahead of the three larger shapes on a 1024-token prompt over 32 experts
-        if (m_expected <= 256)
-            pick = 0;
-        static const int forced = [] {
-            const char* v = std::getenv("TLLM_STACK_GROUP_TILE"); // measurement knob: tile shape 0 .. 3 for grouped products
-            return v && v[0] >= '0' && v[0] <= '3' ? v[0] - '0' : -1;
-        }();
-        if (forced >= 0)
-            pick = forced;
-    }
+    // Grouped: m_expected rows in a group on average (g.M is their bound); up to three 128-row tiles the groups' last ones decide.  32 groups of 8096 rows: 128 x 256 151 us against 160 for 128 x 128 and
+    // 167 for 256 x 192 (N 2816, K 2048), 255 / 307 / 291 (4096, 2752); of 1944 rows 128 x 128 92 us, the wider ones 95 and more (2816, 2048)
+    if (m_expected > 0 && m_expected <= 384)
+        pick = m_expected > 64 ? 3 : 0;
     if (g.act == ACT_SCALE_CAP || g.act == ACT_GELU_MUL)
         pick = 0; // the shape whose epilogue has them
     const int gated = g.act >= ACT_GATE_SILU ? (g.seam.n_sec > 0 ? g.seam.sec[0].col0 : g.N) : 0;
@@ -389,10 +381,12 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
         pick = 0; // gated rows that do not leave in 16-byte pieces
     switch (pick)
     {
-    case 1: return launch_cfg<W_BF16, 4, 2, 2, 3, 1, 64, 5>(g, stream);
-    case 2: return launch_cfg<W_BF16, 2, 4, 4, 2, 1, 64, 4>(g, stream);
-    case 3: return launch_cfg<W_BF16, 2, 2, 2, 4, 1, 64, 4>(g, stream);
-    default: return launch_cfg<W_BF16, 2, 2, 2, 2, 1, 128, 4>(g, stream);
+    case 1: return launch_cfg<W_BF16, 4, 2, 2, 3, 1, 128, 2>(g, stream);
+    case 2: return launch_cfg<W_BF16, 2, 4, 4, 2, 1, 128, 2>(g, stream);
+    case 3: return launch_cfg<W_BF16, 2, 4, 2, 2, 1, 128, 3>(g, stream);
+    case 4: return launch_cfg<W_BF16, 4, 2, 1, 3, 1, 128, 4>(g, stream);
+    case 5: return launch_cfg<W_BF16, 4, 2, 1, 1, 1, 128, 4>(g, stream);
+    default: return launch_cfg<W_BF16, 2, 4, 2, 1, 1, 128, 4>(g, stream);
     }
 }
 
