@@ -670,6 +670,375 @@ __global__ __launch_bounds__(256, DK >= 10 ? 1 : 2) void attn_prefill_kernel(con
     }
 }
 
+// The same two over the lanes 16, 32 and 48 further on without the LDS crossbar: a half's and a row's values change places (v_permlane32_swap,
+// v_permlane16_swap: the two results together hold both partners' values)
+__device__ __forceinline__ float rows_max_swap(float v)
+{
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const uint32_t x = __builtin_bit_cast(uint32_t, fmaxf(__builtin_bit_cast(float, (uint32_t) h[0]), __builtin_bit_cast(float, (uint32_t) h[1])));
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return fmaxf(__builtin_bit_cast(float, (uint32_t) r[0]), __builtin_bit_cast(float, (uint32_t) r[1]));
+}
+
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+// one LDS-DMA instruction: 64 lanes x 16 bytes, wave-uniform base + per-lane offset -> LDS [lds_byte + lane * 16] (the kernel waits by hand)
+__device__ __forceinline__ void dma16(const char* base, uint32_t off, uint32_t lds_byte)
+{
+    uint32_t m0_keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(m0_keep) : "v"(off), "s"(base), "s"(lds_byte) : "memory");
+}
+
+// softmax_block over the 16 NN keys of a unit (or of a wave's half of it): score [n][i] of the lane is key key_lane0 + 32 (n / 2) + 4 (n % 2) + i.  `plain`: nothing but a positive
+// scale stands between the product and the exponent, which then is one multiply-add and one exponential per score.
+template <int VT, int NN>
+__device__ __forceinline__ void softmax_unit(f32x4 (&s)[NN], float& m_run, float& l_run, f32x4 (&acc)[VT], uint4 (&pf)[NN / 2], const HeadMods& hm, bool plain,
+    bool masked, int key_lane0, int qpos, int klo)
+{
+    if (!plain)
+    {
+#pragma unroll
+        for (int n = 0; n < NN; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                float v;
+                if (hm.cap2 > 0.f)
+                {
+                    const float t2 = __builtin_amdgcn_exp2f(fminf(fmaxf(s[n][i] * hm.cap_arg, -43.f), 43.f)); // (softmax_block)
+                    v = hm.cap2 * (t2 - 1.f) * __builtin_amdgcn_rcpf(t2 + 1.f);
+                }
+                else
+                    v = s[n][i] * hm.scale2;
+                if (hm.pen)
+                {
+                    const float dist = (float) (qpos - (key_lane0 + 32 * (n >> 1) + 4 * (n & 1) + i));
+                    v -= hm.slope2 * dist;
+                    if (hm.r1 != 0.f)
+                        v -= hm.r1 * __builtin_amdgcn_logf(fmaxf(1.f + hm.r2 * dist, 1e-30f));
+                }
+                s[n][i] = v;
+            }
+    }
+    if (masked)
+    {
+#pragma unroll
+        for (int n = 0; n < NN; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                const int kidx = key_lane0 + 32 * (n >> 1) + 4 * (n & 1) + i;
+                if (kidx > qpos || (kidx < klo && kidx >= hm.keep))
+                    s[n][i] = -INFINITY;
+            }
+    }
+    if (hm.sigm)
+    {
+#pragma unroll
+        for (int n = 0; n < NN; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                s[n][i] = s[n][i] == -INFINITY ? 0.f : __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(s[n][i] + hm.wb2)));
+    }
+    else
+    {
+        float bm = -INFINITY;
+#pragma unroll
+        for (int n = 0; n < NN; ++n)
+            bm = fmaxf(bm, fmaxf(fmaxf(s[n][0], s[n][1]), fmaxf(s[n][2], s[n][3])));
+        const float sc = plain ? hm.scale2 : 1.f;
+        const float mn = fmaxf(m_run, rows_max_swap(bm) * sc);
+        const bool none = mn == -INFINITY; // this row sees no key of this unit (nor of any before)
+        const float corr = none ? 1.f : __builtin_amdgcn_exp2f(m_run - mn), off = none ? 0.f : -mn;
+        float rs = 0.f;
+#pragma unroll
+        for (int n = 0; n < NN; ++n)
+        {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                s[n][i] = __builtin_amdgcn_exp2f(fmaf(s[n][i], sc, off));
+            rs += (s[n][0] + s[n][1]) + (s[n][2] + s[n][3]);
+        }
+        l_run = l_run * corr + rs; // (the lane's own keys: the rows' sums meet behind the last unit)
+        m_run = mn;
+        if (__builtin_amdgcn_ballot_w64(corr != 1.f) != 0) // (softmax_block)
+        {
+#pragma unroll
+            for (int ct = 0; ct < VT; ++ct)
+                acc[ct] *= corr;
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < NN / 2; ++b)
+        pf[b] = make_uint4(pack_bf16(s[2 * b][0], s[2 * b][1]), pack_bf16(s[2 * b][2], s[2 * b][3]), pack_bf16(s[2 * b + 1][0], s[2 * b + 1][1]),
+            pack_bf16(s[2 * b + 1][2], s[2 * b + 1][3]));
+}
+
+// attn_prompt_kernel: prompts, heads of 64 / 128 / 192 query and 64 / 128 value dimensions, pages of a multiple of 64 keys.  The products of
+// attn_prefill_kernel, with what bounded it taken out (2 us per 32-key block and workgroup, of which the products are 0.1 and the softmax 0.2: the
+// staging through registers, two barriers and the shuffles of one block stood one after another):
+//   - a unit is 64 keys; its K and V^T rows go to LDS by LDS-DMA, the next unit's in flight under this one's arithmetic (two buffers, ONE barrier per
+//     unit); the 16-byte pieces of a row are permuted at the source so that the fragment reads fall on different banks;
+//   - a wave owns RT tiles of 16 rows (a workgroup 64 RT rows): every fragment read from LDS feeds all of them;
+//   - tile t of a half unit holds keys 8 (r / 4) + 4 t + r % 4 in row r, so that a lane's eight scores are eight neighbouring keys and the V^T fragment
+//     that meets them is one 16-byte read;
+//   - a row's maximum meets over the lanes by register swaps;
+//   - KS = 2 (few workgroups): eight waves, two to a row tile, each with its half of every unit's keys; they meet behind the last unit.
+// Workgroups: the heaviest tiles of all heads first, the heads of one key/value head on one XCD.
+// Measured (us): 32 heads over 8, 192 / 128, 2048 rows at contexts 0 and 2048 on average 402 -> 164; 128 / 128 272 -> 151; 16 heads of 2 x 64 / 128 with a soft
+// cap, 1024 rows 90 -> 57.
+template <int MAPS, int DK, int VT, int RT, int KS>
+__global__ __launch_bounds__(256 * KS, 2 / KS) void attn_prompt_kernel(const StackAttnParams p, int min_count, int tiles)
+{
+    constexpr int D = DK * 32, V = VT * 16, ROWS = 64 * RT;
+    constexpr int KPR = D / 8;                                    // 16-byte pieces of a K row
+    constexpr int NW = 4 * KS, NN = 4 / KS;                       // waves; score tiles of 16 keys per wave and unit
+    constexpr int KI = MAPS * KPR / NW, VI = V / 8 / NW;          // DMA instructions per wave and unit
+    constexpr int KB = MAPS * 64 * D * 2, BUF = KB + V * 128;     // bytes
+    static_assert(KPR % 8 == 0 && V % 64 == 0 && MAPS * KPR % NW == 0, "head sizes");
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    // blockIdx.x = tile level x (entries x heads), heaviest tiles first; inside a level the key/value heads run fastest
+    const int per = p.entries * p.heads;
+    const int level = blockIdx.x / per, q_ = blockIdx.x % per, e = q_ / p.heads, hi = q_ % p.heads;
+    const int h = p.cross_values ? hi : hi % p.kv_heads * (p.heads / p.kv_heads) + hi / p.kv_heads;
+    const int count = p.ent_count[e];
+    if (count < min_count)
+        return;
+    const int tile = (count + ROWS - 1) / ROWS - 1 - level;
+    if (tile < 0)
+        return;
+    const int first = p.ent_first[e], pos0 = p.ent_pos0[e];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, g4 = lane >> 4, wr = w & 3, half = w >> 2; // row tile, and which half of a unit's keys (KS = 2)
+    const HeadMap hd = head_map(p, h);
+    const int page = p.page, upp = page / 64; // units per page
+    const int32_t* table = p.block_table + (int64_t) e * p.max_blocks;
+    const HeadMods hm = head_mods(p, h);
+    const bool plain = hm.cap2 == 0.f && !hm.pen && !hm.sigm && hm.scale2 > 0.f;
+
+    int r0[RT], qpos[RT], klo[RT], my_last[RT], my_lo[RT], klo_last[RT];
+    bf16x8 qf[RT][MAPS][DK];
+    float m_run[RT][MAPS], l_run[RT][MAPS];
+    f32x4 acc[RT][MAPS][VT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+    {
+        r0[rt] = tile * ROWS + (wr * RT + rt) * 16;
+        const bool rows_ok = r0[rt] < count; // wave-uniform
+        const int qrow = r0[rt] + col < count ? r0[rt] + col : count - 1;
+        qpos[rt] = pos0 + qrow;
+        klo[rt] = first_visible(p, qpos[rt]);
+#pragma unroll
+        for (int m = 0; m < MAPS; ++m)
+        {
+#pragma unroll
+            for (int ks = 0; ks < DK; ++ks)
+                qf[rt][m][ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
+                    reinterpret_cast<const uint16_t*>(p.q) + (((int64_t) (first + qrow) * hd.q_heads + hd.qh) * MAPS + m) * D + ks * 32 + 8 * g4));
+            m_run[rt][m] = -INFINITY;
+            l_run[rt][m] = 0.f;
+#pragma unroll
+            for (int ct = 0; ct < VT; ++ct)
+                acc[rt][m][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        const int last = r0[rt] + 15 < count ? r0[rt] + 15 : count - 1;
+        my_last[rt] = rows_ok ? (pos0 + last) / 64 : -1; // the tile's last unit that holds a visible key, and its first
+        my_lo[rt] = rows_ok ? first_visible(p, pos0 + r0[rt]) / 64 : 0;
+        klo_last[rt] = rows_ok ? first_visible(p, pos0 + last) : 0;
+    }
+    const int wg_last = tile * ROWS + ROWS - 1 < count ? tile * ROWS + ROWS - 1 : count - 1;
+    // the units the workgroup walks: the ones with kept first keys, then from its first row's first visible key on
+    const int lo = first_visible(p, pos0 + tile * ROWS) / 64;
+    const int keep_u = (p.mask == MASK_WINDOW && p.mask_keep > 0) ? (p.mask_keep + 63) / 64 : 0, nkeep = keep_u < lo ? keep_u : lo;
+    const int n_units = nkeep + (pos0 + wg_last) / 64 + 1 - lo;
+    auto unit_at = [&](int v) { return v < nkeep ? v : v - nkeep + lo; };
+
+    // this lane's part of a unit's DMA: instruction i of wave w fills LDS pieces (NW i + w) 64 + lane
+    uint32_t koff[KI], voff[VI];
+#pragma unroll
+    for (int i = 0; i < KI; ++i)
+    {
+        const int L = (i * NW + w) * 64 + lane, row = L / KPR, pc = L % KPR, r = row % 64;
+        const int x = KPR % 16 == 0 ? ((r >> 3) & 3) << 2 | (r & 3) : ((r >> 3) & 3) << 1 | ((r >> 1) & 1);
+        koff[i] = (uint32_t) ((row / 64 * page + r) * D * 2 + (pc ^ x) * 16);
+    }
+#pragma unroll
+    for (int i = 0; i < VI; ++i)
+    {
+        const int L = (i * NW + w) * 64 + lane, row = L / 8, pc = L % 8;
+        voff[i] = (uint32_t) (row * page * 2 + (pc ^ ((row >> 1) & 7)) * 16);
+    }
+    const uint32_t lds0 = (uint32_t) (uintptr_t) (lds_void_t*) smem + w * 1024;
+    auto request = [&](int u, int blk, int buf) {
+        const int off = upp == 1 ? 0 : u % upp * 64;
+        const char* kb = reinterpret_cast<const char*>(p.k_pool) + (((int64_t) blk * (p.kv_heads * MAPS) + hd.kh * MAPS) * page + off) * D * 2;
+        const char* vb = reinterpret_cast<const char*>(p.v_pool) + (((int64_t) blk * p.kv_heads + hd.vh) * V * page + off) * 2;
+#pragma unroll
+        for (int i = 0; i < KI; ++i)
+            dma16(kb, koff[i], lds0 + buf * BUF + i * NW * 1024);
+#pragma unroll
+        for (int i = 0; i < VI; ++i)
+            dma16(vb, voff[i], lds0 + buf * BUF + KB + i * NW * 1024);
+    };
+    auto block_of = [&](int u) { return __builtin_amdgcn_readfirstlane(table[upp == 1 ? u : u / upp]); };
+
+    request(unit_at(0), block_of(unit_at(0)), 0);
+    int blk_next = n_units > 1 ? block_of(unit_at(1)) : 0;
+    for (int v = 0; v < n_units; ++v)
+    {
+        const int u = unit_at(v);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads(); // the unit has landed for every wave, and every wave is through with the one before it
+        if (v + 1 < n_units)
+        {
+            request(unit_at(v + 1), blk_next, (v + 1) & 1);
+            if (v + 2 < n_units)
+                blk_next = block_of(unit_at(v + 2));
+        }
+        bool on[RT], any = false; // wave-uniform
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+        {
+            on[rt] = u <= my_last[rt] && (u >= my_lo[rt] || u < keep_u);
+            any = any || on[rt];
+        }
+        if (!any)
+            continue;
+        const char* ks_ = smem + (v & 1) * BUF;
+        const char* vs_ = ks_ + KB;
+        const int key0 = u * 64 + (KS == 2 ? half * 32 : 0);
+        uint4 pf[RT][MAPS][NN / 2];
+#pragma unroll
+        for (int m = 0; m < MAPS; ++m)
+        {
+            f32x4 s[RT][NN];
+#pragma unroll
+            for (int n = 0; n < NN; ++n)
+            {
+                const int r = 32 * (KS == 2 ? half : n >> 1) + 8 * (col >> 2) + 4 * (n & 1) + (col & 3);
+                const int x = KPR % 16 == 0 ? ((r >> 3) & 3) << 2 | (r & 3) : ((r >> 3) & 3) << 1 | ((r >> 1) & 1);
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+                    s[rt][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < DK; ++ks)
+                {
+                    const bf16x8 kf = as_bf16x8(*reinterpret_cast<const uint4*>(ks_ + (m * 64 + r) * (D * 2) + (((ks * 4 + g4) ^ x) << 4)));
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) // (no branches among the products: a tile that is off has its scores dropped below)
+                        s[rt][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[rt][m][ks], s[rt][n], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+            {
+                pf[rt][m][0] = pf[rt][m][NN / 2 - 1] = make_uint4(0, 0, 0, 0);
+                if (RT == 1 || on[rt])
+                {
+                    const bool masked = key0 + 16 * NN - 1 > pos0 + r0[rt] || key0 < klo_last[rt];
+                    softmax_unit<VT, NN>(s[rt], m_run[rt][m], l_run[rt][m], acc[rt][m], pf[rt][m], hm, plain, masked, key0 + 8 * g4, qpos[rt], klo[rt]);
+                }
+            }
+        }
+#pragma unroll
+        for (int ct = 0; ct < VT; ++ct)
+#pragma unroll
+            for (int b = 0; b < NN / 2; ++b)
+            {
+                const int row = ct * 16 + col;
+                const bf16x8 vf = as_bf16x8(*reinterpret_cast<const uint4*>(vs_ + row * 128 + ((((KS == 2 ? half : b) * 4 + g4) ^ ((row >> 1) & 7)) << 4)));
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                    for (int m = 0; m < MAPS; ++m)
+                        acc[rt][m][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, as_bf16x8(pf[rt][m][b]), acc[rt][m][ct], 0, 0, 0);
+            }
+    }
+    if constexpr (KS == 2)
+    {
+        // the two halves of the keys meet: waves 4 .. 7 leave theirs in LDS
+        static_assert(RT == 1, "one row tile per wave");
+        constexpr int PER = (VT * 4 + 2) * 64; // floats per wave and map
+        float* x = reinterpret_cast<float*>(smem) + wr * PER * MAPS + lane;
+        __syncthreads();
+        if (half)
+        {
+#pragma unroll
+            for (int m = 0; m < MAPS; ++m)
+            {
+                x[m * PER] = m_run[0][m];
+                x[m * PER + 64] = l_run[0][m];
+#pragma unroll
+                for (int ct = 0; ct < VT; ++ct)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        x[m * PER + (2 + ct * 4 + i) * 64] = acc[0][m][ct][i];
+            }
+        }
+        __syncthreads();
+        if (half)
+            return;
+#pragma unroll
+        for (int m = 0; m < MAPS; ++m)
+        {
+            const float m1 = x[m * PER], M = fmaxf(m_run[0][m], m1);
+            const float f0 = hm.sigm ? 1.f : (m_run[0][m] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[0][m] - M));
+            const float f1 = hm.sigm ? 1.f : (m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - M));
+            m_run[0][m] = M;
+            l_run[0][m] = l_run[0][m] * f0 + x[m * PER + 64] * f1;
+#pragma unroll
+            for (int ct = 0; ct < VT; ++ct)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[0][m][ct][i] = acc[0][m][ct][i] * f0 + x[m * PER + (2 + ct * 4 + i) * 64] * f1;
+        }
+    }
+    // lane (col, g4) holds, for row col of a tile, channels ct * 16 + 4 g4 + i
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+    {
+        float inv[MAPS];
+#pragma unroll
+        for (int m = 0; m < MAPS; ++m)
+            inv[m] = finish_factor(p, h, m_run[rt][m], rows_sum(l_run[rt][m]));
+        float ss = 0.f;
+#pragma unroll
+        for (int ct = 0; ct < VT; ++ct)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                float o = acc[rt][0][ct][i] * inv[0];
+                if (MAPS == 2)
+                    o -= p.lambda * (acc[rt][MAPS - 1][ct][i] * inv[MAPS - 1]);
+                acc[rt][0][ct][i] = o;
+                ss += o * o;
+            }
+        float mul = 1.f;
+        if (p.head_norm)
+            mul = p.out_scale / sqrtf(rows_sum(ss) / (float) V + p.eps);
+        if (r0[rt] + col < count)
+        {
+            mul *= out_gate_of(p, first + r0[rt] + col, h);
+            uint16_t* out = reinterpret_cast<uint16_t*>(p.out) + ((int64_t) (first + r0[rt] + col) * p.heads + h) * V + 4 * g4;
+#pragma unroll
+            for (int ct = 0; ct < VT; ++ct)
+                *reinterpret_cast<uint2*>(out + ct * 16) = make_uint2(pack_bf16(acc[rt][0][ct][0] * mul, acc[rt][0][ct][1] * mul),
+                    pack_bf16(acc[rt][0][ct][2] * mul, acc[rt][0][ct][3] * mul));
+        }
+    }
+}
+
+template <int MAPS, int DK, int VT, int RT, int KS>
+void launch_prompt(const StackAttnParams& p, int min_count, hipStream_t stream)
+{
+    constexpr size_t stages = 2 * ((size_t) MAPS * 64 * DK * 64 + VT * 16 * 128), merge = KS == 2 ? (size_t) 4 * MAPS * (VT * 4 + 2) * 256 : 0;
+    constexpr size_t lds = stages > merge ? stages : merge;
+    launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_prompt_kernel<MAPS, DK, VT, RT, KS>), lds);
+    const int tiles = (p.max_count + 64 * RT - 1) / (64 * RT);
+    hipLaunchKernelGGL((attn_prompt_kernel<MAPS, DK, VT, RT, KS>), dim3((unsigned) ((int64_t) tiles * p.entries * p.heads)), dim3(256 * KS), lds, stream, p, min_count, tiles);
+}
+
 // attn_prefill_wide_kernel: the staged form for one map and long rows (dim of 160 and more), where the fragment reads out of LDS, not
 // the matrix pipe, bound attn_prefill_kernel: a wave owns TWO 16-row tiles (a workgroup 128 rows) and every K and V^T fragment it reads
 // from LDS feeds both, which halves the LDS traffic per score.  Same staging, same products, same finish.
@@ -953,7 +1322,34 @@ int launch_tile(const StackAttnParams& p, hipStream_t stream)
                 hipLaunchKernelGGL((attn_prefill_wide_kernel<DK, VT>), pg, dim3(256), 0, stream, p, PREFILL_ROWS);
             }
         }
-        if (!wide)
+        // heads of the usual sizes over pages of whole 64-key units (16-byte DMA from both pools)
+        constexpr bool prompt_form = (DK == 2 || DK == 4 || (DK == 6 && MAPS == 1)) && (VT == 4 || VT == 8);
+        bool prompt = false;
+        if constexpr (prompt_form)
+        {
+            prompt = p.page % 64 == 0 && !(reinterpret_cast<uintptr_t>(p.v_pool) & 15) && !wide
+                && (int64_t) ((p.max_count + 63) / 64) * p.entries * p.heads < (1 << 30);
+            if (prompt)
+            {
+                // two row tiles per wave where such workgroups still make two per CU; waves that share a unit's keys where workgroups of 64 rows
+                // would leave one wave to a SIMD
+                const int64_t wgs = (int64_t) ((p.max_count + 63) / 64) * p.entries * p.heads, cus = launch_util::device_cus();
+                bool two = false;
+                if constexpr (MAPS == 1)
+                {
+                    two = (int64_t) ((p.max_count + 127) / 128) * p.entries * p.heads >= 2 * cus;
+                    if (two)
+                        launch_prompt<MAPS, DK, VT, 2, 1>(p, PREFILL_ROWS, stream);
+                }
+                if (two)
+                    ;
+                else if (wgs <= cus)
+                    launch_prompt<MAPS, DK, VT, 1, 2>(p, PREFILL_ROWS, stream);
+                else
+                    launch_prompt<MAPS, DK, VT, 1, 1>(p, PREFILL_ROWS, stream);
+            }
+        }
+        if (!wide && !prompt)
         {
             const dim3 pg((p.max_count + 63) / 64, p.entries, p.heads);
             hipLaunchKernelGGL((attn_prefill_kernel<MAPS, DK, VT>), pg, dim3(256), 0, stream, p, PREFILL_ROWS);
