@@ -229,10 +229,13 @@ __device__ __forceinline__ float out_gate_of(const StackAttnParams& p, int64_t t
 template <int MAPS, int DK, int VT, int NW>
 __global__ __launch_bounds__(NW * 64) void attn_tile_kernel(const StackAttnParams p, int below_count, int ks, int head_rows)
 {
-    constexpr int D = DK * 32, V = VT * 16;
+    // VP: 16 floats behind a row's channels put the 16 rows x 4 pieces that a wave stores at once on all banks alike.  (Rows of V floats, a
+    // float per store, met on one bank 16 at a time: one decoded token took 10.7 us with two maps of 64 x 128 at 154 keys, 13.7 us with
+    // latent keys of 320 x 256 under a window of 512; 8.1 and 11.5 us this way.)
+    constexpr int D = DK * 32, V = VT * 16, VP = V + 16;
     extern __shared__ float lds[];
-    float* o_part = lds;                          // [NW][MAPS][16][V]
-    float* ml_part = lds + NW * MAPS * 16 * V;    // [NW][MAPS][16][2]
+    float* o_part = lds;                          // [NW][MAPS][16][VP]
+    float* ml_part = lds + NW * MAPS * 16 * VP;    // [NW][MAPS][16][2]
     // ks == 1: blockIdx.x is the entry's 16-row tile.  ks > 1 (decoding steps: every entry one tile): blockIdx.x is the key split -
     // workgroup `split` of an (entry, head) takes the key blocks split * NW + w, + ks * NW, ... and leaves an unnormalised partial
     // (max, sum, O per map and row) in split_ws; attn_split_merge_kernel finishes the rows.
@@ -367,9 +370,7 @@ __global__ __launch_bounds__(NW * 64) void attn_tile_kernel(const StackAttnParam
         }
 #pragma unroll
         for (int ct = 0; ct < VT; ++ct)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                o_part[((w * MAPS + m) * 16 + col) * V + ct * 16 + 4 * g4 + i] = acc[m][ct][i];
+            *reinterpret_cast<f32x4*>(&o_part[((w * MAPS + m) * 16 + col) * VP + ct * 16 + 4 * g4]) = acc[m][ct];
     }
     __syncthreads();
     // 16 threads per row at NW = 4 (NW * 4 in general), each a strided set of channels
@@ -433,7 +434,7 @@ __global__ __launch_bounds__(NW * 64) void attn_tile_kernel(const StackAttnParam
                         float a = 0.f;
 #pragma unroll
                         for (int ww = 0; ww < NW; ++ww)
-                            a += wgt[m][ww] * o_part[((ww * MAPS + m) * 16 + row) * V + ch];
+                            a += wgt[m][ww] * o_part[((ww * MAPS + m) * 16 + row) * VP + ch];
                         ws[ch] = a;
                     }
                 }
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(NW * 64) void attn_tile_kernel(const StackAttnParam
                 a[m] = 0.f;
 #pragma unroll
                 for (int ww = 0; ww < NW; ++ww)
-                    a[m] += wgt[m][ww] * o_part[((ww * MAPS + m) * 16 + row) * V + ch];
+                    a[m] += wgt[m][ww] * o_part[((ww * MAPS + m) * 16 + row) * VP + ch];
             }
             o[c] = MAPS == 2 ? a[0] - p.lambda * a[MAPS - 1] : a[0];
             ss += o[c] * o[c];
@@ -1293,7 +1294,7 @@ template <int MAPS, int DK, int VT>
 int launch_tile(const StackAttnParams& p, hipStream_t stream)
 {
     constexpr int NW = 4;
-    const size_t lds = sizeof(float) * ((size_t) NW * MAPS * 16 * VT * 16 + (size_t) NW * MAPS * 16 * 2);
+    const size_t lds = sizeof(float) * ((size_t) NW * MAPS * 16 * (VT * 16 + 16) + (size_t) NW * MAPS * 16 * 2);
     const void* fn = reinterpret_cast<const void*>(&attn_tile_kernel<MAPS, DK, VT, NW>);
     launch_util::ensure_dynamic_lds(fn, lds);
     // entries of PREFILL_ROWS rows and more go to the staged form, the rest (decoded tokens, short portions) to the key-split form;
