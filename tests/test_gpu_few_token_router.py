@@ -1,0 +1,29 @@
+"""Router of a few tokens in one launch (stack_moe.hip moe_route_few_kernel): logits spread over workgroups, the last of them chooses and
+orders.  Outputs that end inside a workgroup or take many of them, more than 64 choices' worth of lanes, groups, equal scores (the lowest
+outputs win), rows that are not whole 16-byte pieces, and 1, 7, 8 and 9 tokens (the most the launch takes, and one more), several steps
+in a row so that its ticket is armed again each time."""
+import numpy as np
+import pytest
+
+from rofozen_cases import make_config, mamba_layer, moe, random_weights
+from test_gpu_rofozen import O, as_f64, check, replay, session_for, tokens_for, tol_of
+
+pytestmark = pytest.mark.gpu
+
+ROUTERS = [dict(experts=1, identity=0, top=1, count=1, keep=1), dict(experts=6, identity=3, top=2, count=3, keep=2), dict(experts=17, identity=0, top=5, count=1, keep=1),
+           dict(experts=150, identity=10, top=7, count=8, keep=3), dict(experts=70, identity=0, top=64, count=1, keep=1)]
+
+
+@pytest.mark.parametrize('equal', [False, True], ids=['apart', 'equal'])
+@pytest.mark.parametrize('width', [96, 100])
+@pytest.mark.parametrize('router', ROUTERS, ids=lambda r: f"{r['experts']}+{r['identity']}top{r['top']}")
+def test_few_token_router(router, width, equal):
+    cfg = make_config([mamba_layer(mlp=moe(ff=8, **router)), mamba_layer(mlp=moe(ff=8, **router))], width=width)
+    w = random_weights(cfg, 5)
+    if equal:  # every output's score is the same number: the first ones are chosen
+        for name in w:
+            if name.endswith(('mlp.router', 'mlp.correction')):
+                w[name] = np.zeros_like(w[name])
+    toks = tokens_for(cfg, 29, 7)
+    got = replay(session_for(cfg, w, 'float32'), {'a': toks}, [[('a', k)] for k in (1, 7, 8, 9, 1, 1, 2)])['a']
+    check(got, O.logits(toks, as_f64(w), cfg), tol_of('float32'), 'a')

@@ -385,6 +385,7 @@ struct StackMoeParams
     int32_t* tok_of_slot = nullptr;   // [tokens * top] or null: the token of every used slot (grouped products read h through it: a_rows)
     void* a_sorted = nullptr;         // [tokens * top, width]; null: no rows are copied (not with weight_input)
     int32_t normalize = 0;            // 1: the chosen experts' scores are divided by their sum (+ 1e-20)
+    uint32_t* ticket = nullptr;       // a word that is zero between launches (a few tokens are routed and ordered in one launch), or null
     int32_t have_logits = 0;          // 1: `logits` already holds the router's logits (a projection's fp32 columns)
     // launch_stack_moe_combine: y += the sum instead of y = it; y_el (or null) receives the resulting rows in the element type
     // accumulate_gate (fp32 [tokens] or null): y's old row is scaled by sigmoid(accumulate_gate[t]) first

@@ -42,54 +42,68 @@ inline int launched(const char* what)
     return 0;
 }
 
-// the lane that holds the largest value of the wave, the lowest index among equals; every lane gets (value, index)
+// the lane that holds the largest value of the wave, the lowest index among equals; every lane gets (value, index).  The maximum goes
+// through DPP moves, and a lane that holds it alone gives its index by a lane read: a twelve-shuffle tree costs twice the time of a choice.
 __device__ __forceinline__ void wave_argmax(float& v, int& idx)
 {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1)
+    const float m = wave_max(v);
+    const uint64_t at = __ballot(v == m);
+    if (__popcll(at) == 1)
+        idx = __builtin_amdgcn_readlane(idx, (int) __builtin_ctzll(at));
+    else
     {
-        const float ov = __shfl_xor(v, d, 64);
-        const int oi = __shfl_xor(idx, d, 64);
-        if (ov > v || (ov == v && oi < idx))
+        int best = v == m ? idx : 0x7fffffff;
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1)
         {
-            v = ov;
-            idx = oi;
+            const int o = __shfl_xor(best, d, 64);
+            best = o < best ? o : best;
         }
+        idx = best;
     }
+    v = m;
 }
 
 constexpr int RT = 8;         // tokens per logits workgroup: a router row is read once for all of them
 constexpr int MAX_OUT = 1024; // router outputs (experts + identities)
 constexpr int MAX_TOP = 64;
-constexpr int FEW_TOKENS = 8; // steps of this many tokens or fewer route in one launch and gather inside the sort
+constexpr int RANKED_PAIRS = 64; // pairs up to which every thread compares all of them
+constexpr int FEW_TOKENS = RT; // steps of this many tokens or fewer are routed and ordered in one launch (and gather inside it)
 
-// Router logits, fp32: workgroup (x, y) = 4 router rows (one per wave) x RT tokens; lanes split the width in float4 pieces where
-// rows are 16-byte aligned.  z [tokens, outputs].
+// acc[r] = this lane's share of router row e times the rows t0 .. t0 + nt of h; lanes split the width in float4 pieces where rows are
+// 16-byte aligned
 template <int DT>
-__global__ __launch_bounds__(256) void moe_logits_kernel(const StackMoeParams p, float* z)
+__device__ __forceinline__ void router_row(const StackMoeParams& p, int e, int t0, int nt, int lane, float (&acc)[RT])
 {
-    const int NE = p.experts + p.identity, W = p.width;
-    const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, t0 = blockIdx.y * RT;
-    if (e >= NE)
-        return;
-    float acc[RT];
+    const int W = p.width;
 #pragma unroll
     for (int r = 0; r < RT; ++r)
         acc[r] = 0.f;
     const float* wr = p.router_w + (int64_t) e * W;
-    const int nt = p.tokens - t0 < RT ? p.tokens - t0 : RT;
     if ((W & 7) == 0)
     {
-        for (int k = lane * 8; k < W; k += 64 * 8)
+        // AHEAD pieces of the row are requested before the first is used (a piece behind the row: its first one again, unused)
+        constexpr int AHEAD = 4;
+        for (int k0 = lane * 8; k0 < W; k0 += AHEAD * 64 * 8)
         {
-            const float4 w0 = *reinterpret_cast<const float4*>(wr + k), w1 = *reinterpret_cast<const float4*>(wr + k + 4);
-            const float wv[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+            float4 w[AHEAD][2];
+#pragma unroll
+            for (int a = 0; a < AHEAD; ++a)
+            {
+                const int k = k0 + a * 64 * 8 < W ? k0 + a * 64 * 8 : k0;
+                w[a][0] = *reinterpret_cast<const float4*>(wr + k);
+                w[a][1] = *reinterpret_cast<const float4*>(wr + k + 4);
+            }
 #pragma unroll
             for (int r = 0; r < RT; ++r)
             {
-                if (r < nt)
+                if (r >= nt)
+                    break;
+                float hv[AHEAD][8];
+#pragma unroll
+                for (int a = 0; a < AHEAD; ++a)
                 {
-                    float hv[8];
+                    const int k = k0 + a * 64 * 8 < W ? k0 + a * 64 * 8 : k0;
                     if constexpr (DT == DT_BF16)
                     {
                         const uint4 u = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.h) + (int64_t) (t0 + r) * W + k);
@@ -97,19 +111,27 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const StackMoeParams p,
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
                         {
-                            hv[2 * i] = __builtin_bit_cast(float, us[i] << 16);
-                            hv[2 * i + 1] = __builtin_bit_cast(float, us[i] & 0xffff0000u);
+                            hv[a][2 * i] = __builtin_bit_cast(float, us[i] << 16);
+                            hv[a][2 * i + 1] = __builtin_bit_cast(float, us[i] & 0xffff0000u);
                         }
                     }
                     else
                     {
                         const float* hp = reinterpret_cast<const float*>(p.h) + (int64_t) (t0 + r) * W + k;
                         const float4 h0 = *reinterpret_cast<const float4*>(hp), h1 = *reinterpret_cast<const float4*>(hp + 4);
-                        hv[0] = h0.x, hv[1] = h0.y, hv[2] = h0.z, hv[3] = h0.w, hv[4] = h1.x, hv[5] = h1.y, hv[6] = h1.z, hv[7] = h1.w;
+                        hv[a][0] = h0.x, hv[a][1] = h0.y, hv[a][2] = h0.z, hv[a][3] = h0.w;
+                        hv[a][4] = h1.x, hv[a][5] = h1.y, hv[a][6] = h1.z, hv[a][7] = h1.w;
                     }
+                }
+#pragma unroll
+                for (int a = 0; a < AHEAD; ++a)
+                {
+                    if (k0 + a * 64 * 8 >= W)
+                        break;
+                    const float wv[8] = {w[a][0].x, w[a][0].y, w[a][0].z, w[a][0].w, w[a][1].x, w[a][1].y, w[a][1].z, w[a][1].w};
 #pragma unroll
                     for (int i = 0; i < 8; ++i)
-                        acc[r] = fmaf(wv[i], hv[i], acc[r]);
+                        acc[r] = fmaf(wv[i], hv[a][i], acc[r]);
                 }
             }
         }
@@ -125,6 +147,19 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const StackMoeParams p,
                     acc[r] = fmaf(wv, ld_el<DT>(p.h, (int64_t) (t0 + r) * W + k), acc[r]);
         }
     }
+}
+
+// Router logits, fp32: workgroup (x, y) = 4 router rows (one per wave) x RT tokens.  z [tokens, outputs].
+template <int DT>
+__global__ __launch_bounds__(256) void moe_logits_kernel(const StackMoeParams p, float* z)
+{
+    const int NE = p.experts + p.identity;
+    const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, t0 = blockIdx.y * RT;
+    if (e >= NE)
+        return;
+    const int nt = p.tokens - t0 < RT ? p.tokens - t0 : RT;
+    float acc[RT];
+    router_row<DT>(p, e, t0, nt, lane, acc);
 #pragma unroll
     for (int r = 0; r < RT; ++r)
     {
@@ -134,13 +169,12 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const StackMoeParams p,
     }
 }
 
-// One wave finishes one token: zr [outputs] holds its logits (LDS) and leaves as scores, cr [outputs] is room for the choice values.
-__device__ __forceinline__ void select_token(const StackMoeParams& p, float* zr, float* cr, int lane, int t)
+// One wave finishes one token: zr [outputs] holds its logits with the bias (LDS) and leaves as scores, cr [outputs] holds the corrections
+// and leaves as choice values,
+// lane k < top gets choice k.
+__device__ __forceinline__ int select_token(const StackMoeParams& p, float* zr, float* cr, int lane, int t)
 {
     const int NE = p.experts + p.identity;
-    if (p.bias)
-        for (int e = lane; e < NE; e += 64)
-            zr[e] += p.bias[e];
     if (p.score == ROUTE_SIGMOID)
     {
         // every output's score by itself
@@ -148,7 +182,7 @@ __device__ __forceinline__ void select_token(const StackMoeParams& p, float* zr,
         {
             const float s = 1.f / (1.f + expf(-zr[e]));
             zr[e] = s;
-            cr[e] = s + (p.correction ? p.correction[e] : 0.f);
+            cr[e] += s;
         }
     }
     else
@@ -170,7 +204,7 @@ __device__ __forceinline__ void select_token(const StackMoeParams& p, float* zr,
         {
             const float s = zr[e] * inv;
             zr[e] = s;
-            cr[e] = s + (p.correction ? p.correction[e] : 0.f);
+            cr[e] += s;
         }
     }
     __builtin_amdgcn_wave_barrier();
@@ -219,7 +253,8 @@ __device__ __forceinline__ void select_token(const StackMoeParams& p, float* zr,
         }
         __builtin_amdgcn_wave_barrier();
     }
-    float mine = 0.f, total = 0.f; // lane k keeps choice k's score; every lane their sum
+    float mine = 0.f, total = 0.f; // lane k keeps choice k and its score; every lane the scores' sum
+    int chosen = 0;
     for (int k = 0; k < p.top; ++k)
     {
         float bv = -INFINITY;
@@ -239,16 +274,17 @@ __device__ __forceinline__ void select_token(const StackMoeParams& p, float* zr,
         const float s = bv == -INFINITY ? 0.f : zr[bi];
         total += s;
         if (lane == k)
-            mine = s;
-        if (lane == 0)
         {
-            p.topk_idx[(int64_t) t * p.top + k] = bi;
-            cr[bi] = -INFINITY;
+            mine = s;
+            chosen = bi;
         }
+        if (lane == 0)
+            cr[bi] = -INFINITY;
         __builtin_amdgcn_wave_barrier();
     }
     if (lane < p.top)
         p.topk_w[(int64_t) t * p.top + lane] = (p.normalize ? mine / (total + 1e-20f) : mine) * p.scale;
+    return chosen;
 }
 
 // One wave per token (4 per workgroup): softmax over the logits, choice values, the kept groups, the top-k among them.
@@ -261,73 +297,35 @@ __global__ __launch_bounds__(256) void moe_select_kernel(const StackMoeParams p,
     const int t0 = blockIdx.x * 4, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (t0 + wid < p.tokens)
         for (int e = lane; e < NE; e += 64)
-            z[wid * NE + e] = zg[(int64_t) (t0 + wid) * NE + e];
+        {
+            z[wid * NE + e] = zg[(int64_t) (t0 + wid) * NE + e] + (p.bias ? p.bias[e] : 0.f);
+            ch[wid * NE + e] = p.correction ? p.correction[e] : 0.f;
+        }
     __syncthreads();
     const int t = t0 + wid;
     if (t >= p.tokens)
         return;
-    select_token(p, z + wid * NE, ch + wid * NE, lane, t);
-}
-
-// Few tokens (a step of decoded tokens): one workgroup of 16 waves per token computes its logits (a wave per router row, 16-byte
-// pieces) and wave 0 finishes the token, in one launch.
-template <int DT>
-__global__ __launch_bounds__(1024) void moe_route_few_kernel(const StackMoeParams p)
-{
-    extern __shared__ float sm[];
-    const int NE = p.experts + p.identity, W = p.width, t = blockIdx.x;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    for (int e = wid; e < NE; e += 16)
-    {
-        const float* wr = p.router_w + (int64_t) e * W;
-        float acc = 0.f;
-        if ((W & 7) == 0)
-        {
-            for (int k = lane * 8; k < W; k += 64 * 8)
-            {
-                const float4 w0 = *reinterpret_cast<const float4*>(wr + k), w1 = *reinterpret_cast<const float4*>(wr + k + 4);
-                const float wv[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-                float hv[8];
-                if constexpr (DT == DT_BF16)
-                {
-                    const uint4 u = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.h) + (int64_t) t * W + k);
-                    const uint32_t us[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                    {
-                        hv[2 * i] = __builtin_bit_cast(float, us[i] << 16);
-                        hv[2 * i + 1] = __builtin_bit_cast(float, us[i] & 0xffff0000u);
-                    }
-                }
-                else
-                {
-                    const float* hp = reinterpret_cast<const float*>(p.h) + (int64_t) t * W + k;
-                    const float4 h0 = *reinterpret_cast<const float4*>(hp), h1 = *reinterpret_cast<const float4*>(hp + 4);
-                    hv[0] = h0.x, hv[1] = h0.y, hv[2] = h0.z, hv[3] = h0.w, hv[4] = h1.x, hv[5] = h1.y, hv[6] = h1.z, hv[7] = h1.w;
-                }
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    acc = fmaf(wv[i], hv[i], acc);
-            }
-        }
-        else
-        {
-            for (int k = lane; k < W; k += 64)
-                acc = fmaf(wr[k], ld_el<DT>(p.h, (int64_t) t * W + k), acc);
-        }
-        acc = wave_sum(acc);
-        if (lane == 0)
-            sm[e] = acc;
-    }
-    __syncthreads();
-    if (wid == 0)
-        select_token(p, sm, sm + NE, lane, t);
+    const int chosen = select_token(p, z + wid * NE, ch + wid * NE, lane, t);
+    if (lane < p.top)
+        p.topk_idx[(int64_t) t * p.top + lane] = chosen;
 }
 
 // dst[:] = w * src[:] over one row of the element type (the weight of a pair applied to the expert's input), thread `i` of `n`
 __device__ __forceinline__ void scaled_row(const StackMoeParams& p, char* dst, const char* src, float w, int i, int n)
 {
-    if (p.dtype == DT_BF16)
+    if (p.dtype == DT_BF16 && (p.width & 7) == 0) // (16-byte rows of 16-byte operands: h and a_sorted are allocations)
+        for (int c = i * 8; c < p.width; c += n * 8)
+        {
+            const uint4 u = *reinterpret_cast<const uint4*>(src + c * 2);
+            const uint32_t us[4] = {u.x, u.y, u.z, u.w};
+            uint32_t o[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                o[k] = (uint32_t) f2bf(w * __builtin_bit_cast(float, us[k] << 16))
+                    | ((uint32_t) f2bf(w * __builtin_bit_cast(float, us[k] & 0xffff0000u)) << 16);
+            *reinterpret_cast<uint4*>(dst + c * 2) = make_uint4(o[0], o[1], o[2], o[3]);
+        }
+    else if (p.dtype == DT_BF16)
         for (int c = i; c < p.width; c += n)
             reinterpret_cast<uint16_t*>(dst)[c] = f2bf(w * bf2f(reinterpret_cast<const uint16_t*>(src)[c]));
     else
@@ -335,63 +333,11 @@ __device__ __forceinline__ void scaled_row(const StackMoeParams& p, char* dst, c
             reinterpret_cast<float*>(dst)[c] = w * reinterpret_cast<const float*>(src)[c];
 }
 
-// One workgroup: counts per expert, offsets, a slot per pair.  Which of an expert's slots a pair gets depends on the order of the
-// atomics; a row's product does not depend on its neighbours in a tile, so the results do not.  si: LDS, 2 * experts + 1 ints.
-__device__ __forceinline__ void sort_pairs(const StackMoeParams& p, int gather_row_bytes, int* si)
+// The rows of few pairs are copied by the launch that orders them, a wave per pair, instead of by one of their own
+__device__ __forceinline__ void gather_pairs(const StackMoeParams& p, int gather_row_bytes)
 {
-    int* cnt = si;                  // [experts]
-    int* off = cnt + p.experts;     // [experts + 1]
-    const int pairs = p.tokens * p.top, tid = threadIdx.x, NT = blockDim.x;
-    for (int e = tid; e < p.experts; e += NT)
-        cnt[e] = 0;
-    __syncthreads();
-    for (int i = tid; i < pairs; i += NT)
-    {
-        const int e = p.topk_idx[i];
-        if (e < p.experts)
-            atomicAdd(&cnt[e], 1);
-    }
-    __syncthreads();
-    if (tid == 0)
-    {
-        int run = 0;
-        for (int e = 0; e < p.experts; ++e)
-        {
-            off[e] = run;
-            run += cnt[e];
-        }
-        off[p.experts] = run;
-    }
-    __syncthreads();
-    for (int e = tid; e <= p.experts; e += NT)
-    {
-        p.group_off[e] = off[e];
-        if (e < p.experts)
-            cnt[e] = 0;
-    }
-    const int used = off[p.experts];
-    for (int i = used + tid; i < pairs; i += NT)
-        p.pair_of_slot[i] = -1;
-    __syncthreads();
-    for (int i = tid; i < pairs; i += NT)
-    {
-        const int e = p.topk_idx[i];
-        int slot = -1;
-        if (e < p.experts)
-        {
-            slot = off[e] + atomicAdd(&cnt[e], 1);
-            p.pair_of_slot[slot] = i;
-            if (p.tok_of_slot)
-                p.tok_of_slot[slot] = i / p.top;
-        }
-        p.slot_of_pair[i] = slot;
-    }
-    if (gather_row_bytes <= 0)
-        return;
-    // few pairs: the rows are copied here (a wave per pair) instead of by a launch of their own
-    __syncthreads();
-    const int lane = tid & 63;
-    for (int i = tid >> 6; i < pairs; i += NT >> 6)
+    const int pairs = p.tokens * p.top, NT = blockDim.x, lane = threadIdx.x & 63;
+    for (int i = threadIdx.x >> 6; i < pairs; i += NT >> 6)
     {
         const int slot = p.slot_of_pair[i];
         if (slot < 0)
@@ -409,27 +355,213 @@ __device__ __forceinline__ void sort_pairs(const StackMoeParams& p, int gather_r
     }
 }
 
+// One workgroup: counts per expert, offsets, a slot per pair.  Which of an expert's slots a pair gets depends on the order of the
+// atomics; a row's product does not depend on its neighbours in a tile, so the results do not.  choice [tokens * top]: the chosen
+// outputs; si: LDS, 2 * experts + 1 ints.
+__device__ __forceinline__ void sort_pairs(const StackMoeParams& p, const int* choice, int gather_row_bytes, int* si)
+{
+    int* cnt = si;                  // [experts]
+    int* off = cnt + p.experts;     // [experts + 1]
+    const int pairs = p.tokens * p.top, tid = threadIdx.x, NT = blockDim.x;
+    for (int e = tid; e < p.experts; e += NT)
+        cnt[e] = 0;
+    __syncthreads();
+    for (int i = tid; i < pairs; i += NT)
+    {
+        const int e = choice[i];
+        if (e < p.experts)
+            atomicAdd(&cnt[e], 1);
+    }
+    __syncthreads();
+    if (tid < 64) // one wave sums the counts, 64 experts at a time
+    {
+        int run = 0;
+        for (int e0 = 0; e0 < p.experts; e0 += 64)
+        {
+            const int e = e0 + tid, own = e < p.experts ? cnt[e] : 0;
+            int upto = own;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1)
+            {
+                const int below = __shfl_up(upto, d, 64);
+                upto += tid >= d ? below : 0;
+            }
+            if (e < p.experts)
+                off[e] = run + upto - own;
+            run += __builtin_amdgcn_readlane(upto, 63);
+        }
+        if (tid == 0)
+            off[p.experts] = run;
+    }
+    __syncthreads();
+    for (int e = tid; e <= p.experts; e += NT)
+    {
+        p.group_off[e] = off[e];
+        if (e < p.experts)
+            cnt[e] = 0;
+    }
+    const int used = off[p.experts];
+    for (int i = used + tid; i < pairs; i += NT)
+        p.pair_of_slot[i] = -1;
+    __syncthreads();
+    for (int i = tid; i < pairs; i += NT)
+    {
+        const int e = choice[i];
+        int slot = -1;
+        if (e < p.experts)
+        {
+            slot = off[e] + atomicAdd(&cnt[e], 1);
+            p.pair_of_slot[slot] = i;
+            if (p.tok_of_slot)
+                p.tok_of_slot[slot] = i / p.top;
+        }
+        p.slot_of_pair[i] = slot;
+    }
+    if (gather_row_bytes <= 0)
+        return;
+    __syncthreads();
+    gather_pairs(p, gather_row_bytes);
+}
+
+// The same for a few pairs: an expert's first slot is how many pairs chose a lower one, a pair's slot counts the equal ones ahead of it.
+// Every thread reads all choices, which no barrier or atomic separates: they cost less than the counting form's five barriers.
+__device__ __forceinline__ void rank_pairs(const StackMoeParams& p, const int* choice, int gather_row_bytes)
+{
+    const int pairs = p.tokens * p.top, tid = threadIdx.x, NT = blockDim.x;
+    for (int e = tid; e <= p.experts; e += NT)
+    {
+        int below = 0;
+        for (int j = 0; j < pairs; ++j)
+            below += choice[j] < e ? 1 : 0;
+        p.group_off[e] = below;
+    }
+    for (int i = tid; i < pairs; i += NT)
+    {
+        const int own = choice[i];
+        int below = 0, used = 0;
+        for (int j = 0; j < pairs; ++j)
+        {
+            const int c = choice[j];
+            below += (c < own || (c == own && j < i)) ? 1 : 0;
+            used += c < p.experts ? 1 : 0;
+        }
+        const bool routed = own < p.experts;
+        p.slot_of_pair[i] = routed ? below : -1;
+        if (routed)
+        {
+            p.pair_of_slot[below] = i;
+            if (p.tok_of_slot)
+                p.tok_of_slot[below] = i / p.top;
+        }
+        if (i >= used)
+            p.pair_of_slot[i] = -1;
+    }
+    if (gather_row_bytes <= 0)
+        return;
+    __syncthreads();
+    gather_pairs(p, gather_row_bytes);
+}
+
 __global__ __launch_bounds__(1024) void moe_sort_kernel(const StackMoeParams p, int gather_row_bytes)
 {
     extern __shared__ int si[];
-    sort_pairs(p, gather_row_bytes, si);
+    sort_pairs(p, p.topk_idx, gather_row_bytes, si);
 }
 
-// Few tokens whose logits are there already: wave t finishes token t, then the workgroup orders the pairs.
-__global__ __launch_bounds__(1024) void moe_plan_few_kernel(const StackMoeParams p, int gather_row_bytes)
+// LDS of a launch that chooses for a few tokens and orders their pairs: scores and choice values first, then counts and choices
+inline size_t plan_lds_bytes(const StackMoeParams& p)
 {
-    extern __shared__ float sm[];
+    const size_t NE = (size_t) (p.experts + p.identity), T = (size_t) p.tokens;
+    return sizeof(int) * std::max(2 * NE * T, 2 * (size_t) p.experts + 1 + T * (size_t) p.top);
+}
+
+// Wave t finishes token t, then the workgroup orders the pairs.  SPREAD: the logits come from other workgroups of this launch, bias and
+// corrections are in LDS already.
+template <bool SPREAD>
+__device__ __forceinline__ void plan_few(const StackMoeParams& p, int gather_row_bytes, float* sm)
+{
     const int NE = p.experts + p.identity, lane = threadIdx.x & 63, t = threadIdx.x >> 6;
+    int* choice = reinterpret_cast<int*>(sm) + 2 * p.experts + 1;
+    int chosen = 0;
     if (t < p.tokens)
     {
         float* z = sm + (int64_t) t * 2 * NE;
         for (int e = lane; e < NE; e += 64)
-            z[e] = p.logits[(int64_t) t * NE + e];
+        {
+            const float* src = p.logits + (int64_t) t * NE + e;
+            if constexpr (SPREAD)
+                z[e] += __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else
+            {
+                z[e] = *src + (p.bias ? p.bias[e] : 0.f);
+                z[NE + e] = p.correction ? p.correction[e] : 0.f;
+            }
+        }
         __builtin_amdgcn_wave_barrier();
-        select_token(p, z, z + NE, lane, t);
+        chosen = select_token(p, z, z + NE, lane, t);
     }
-    __syncthreads(); // the choices (global, this workgroup's own) are visible to all its waves
-    sort_pairs(p, gather_row_bytes, reinterpret_cast<int*>(sm));
+    __syncthreads(); // the scores' place is free
+    if (t < p.tokens && lane < p.top)
+        choice[t * p.top + lane] = chosen;
+    __syncthreads();
+    if (p.tokens * p.top <= RANKED_PAIRS)
+        rank_pairs(p, choice, gather_row_bytes);
+    else
+        sort_pairs(p, choice, gather_row_bytes, reinterpret_cast<int*>(sm));
+}
+
+// Few tokens whose logits are there already.
+__global__ __launch_bounds__(1024) void moe_plan_few_kernel(const StackMoeParams p, int gather_row_bytes)
+{
+    extern __shared__ float sm[];
+    plan_few<false>(p, gather_row_bytes, sm);
+}
+
+// The same with the logits computed here, a router row per wave.  The rows are spread over workgroups, and the last one to arrive chooses
+// and orders: a logit is written through to where every XCD sees it and waited for before its workgroup takes a ticket, the last one
+// reads them past its own caches, and the ticket word is zero again for the next launch.  Bound by latencies in a row (row, ticket,
+// logits, choices).  One workgroup for all rows draws too little bandwidth: one token, top 4, us alone / spread: 32 outputs of width
+// 1024 8.2 / 7.6, 64 of 2048 13.7 / 8.1, 256 of 4096 110 / 13.5; eight tokens 15.6 / 12.8, 38 / 15.4, 295 / 25.  In a decode step
+// (cold rows), 40 outputs of width 2048: 14.7 as a one-workgroup router and a sort, 9.8 here.
+template <int DT>
+__global__ __launch_bounds__(512) void moe_route_few_kernel(const StackMoeParams p, int gather_row_bytes)
+{
+    extern __shared__ float sm[];
+    __shared__ uint32_t ticket;
+    const int NE = p.experts + p.identity, lane = threadIdx.x & 63, e = blockIdx.x * 8 + (threadIdx.x >> 6);
+    // what the choice adds to the logits comes in under the product
+    for (int i = threadIdx.x; i < NE; i += 512)
+    {
+        const float b = p.bias ? p.bias[i] : 0.f, c = p.correction ? p.correction[i] : 0.f;
+        for (int t = 0; t < p.tokens; ++t)
+        {
+            sm[t * 2 * NE + i] = b;
+            sm[t * 2 * NE + NE + i] = c;
+        }
+    }
+    if (e < NE)
+    {
+        float acc[RT];
+        router_row<DT>(p, e, 0, p.tokens, lane, acc);
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+            if (r < p.tokens)
+            {
+                const float sum = wave_sum(acc[r]);
+                if (lane == 0)
+                    __hip_atomic_store(p.logits + (int64_t) r * NE + e, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+        ticket = __hip_atomic_fetch_add(p.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (ticket != gridDim.x - 1)
+        return;
+    if (threadIdx.x == 0)
+        __hip_atomic_store(p.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    plan_few<true>(p, gather_row_bytes, sm);
 }
 
 // a_sorted[slot, :] = h[token of the slot's pair, :]; 16 bytes per thread where the rows allow it
@@ -584,14 +716,6 @@ int launch_stack_moe_route(const StackMoeParams& p, hipStream_t stream)
         hipLaunchKernelGGL(moe_select_kernel, dim3((p.tokens + 3) / 4), dim3(256), sizeof(float) * 2 * 4 * NE, stream, p, p.logits);
         return launched("stack_moe_select");
     }
-    if (p.tokens <= FEW_TOKENS)
-    {
-        if (p.dtype == DT_BF16)
-            hipLaunchKernelGGL((moe_route_few_kernel<DT_BF16>), dim3(p.tokens), dim3(1024), sizeof(float) * 2 * NE, stream, p);
-        else
-            hipLaunchKernelGGL((moe_route_few_kernel<DT_FLOAT>), dim3(p.tokens), dim3(1024), sizeof(float) * 2 * NE, stream, p);
-        return launched("stack_moe_route (few tokens)");
-    }
     const dim3 lg((NE + 3) / 4, (p.tokens + RT - 1) / RT);
     if (p.dtype == DT_BF16)
         hipLaunchKernelGGL((moe_logits_kernel<DT_BF16>), lg, dim3(256), 0, stream, p, p.logits);
@@ -629,19 +753,27 @@ int launch_stack_moe_plan(const StackMoeParams& p, hipStream_t stream)
 {
     if (p.tokens <= 0)
         return 0;
-    if (!p.have_logits || p.tokens > FEW_TOKENS)
+    if (p.tokens > FEW_TOKENS || !(p.have_logits || p.ticket))
         return (launch_stack_moe_route(p, stream) || launch_stack_moe_sort(p, stream)) ? -1 : 0;
     if (!moe_ok(p, "stack_moe_plan"))
         return -1;
-    const size_t NE = (size_t) (p.experts + p.identity);
-    const size_t lds = std::max(sizeof(float) * 2 * NE * (size_t) p.tokens, sizeof(int) * (2 * (size_t) p.experts + 1));
+    const size_t lds = plan_lds_bytes(p);
     if (!p.logits || (p.weight_input && !p.a_sorted) || lds > 64 * 1024)
     {
-        set_error("stack_moe_plan: %d tokens x %d outputs, or a missing operand", p.tokens, (int) NE);
+        set_error("stack_moe_plan: %d tokens x %d outputs, or a missing operand", p.tokens, p.experts + p.identity);
         return -1;
     }
     const int row_bytes = p.a_sorted ? p.width * (p.dtype == DT_BF16 ? 2 : 4) : 0;
-    hipLaunchKernelGGL(moe_plan_few_kernel, dim3(1), dim3(1024), lds, stream, p, row_bytes);
+    if (p.have_logits)
+        hipLaunchKernelGGL(moe_plan_few_kernel, dim3(1), dim3(1024), lds, stream, p, row_bytes);
+    else
+    {
+        const dim3 grid((p.experts + p.identity + 7) / 8);
+        if (p.dtype == DT_BF16)
+            hipLaunchKernelGGL((moe_route_few_kernel<DT_BF16>), grid, dim3(512), lds, stream, p, row_bytes);
+        else
+            hipLaunchKernelGGL((moe_route_few_kernel<DT_FLOAT>), grid, dim3(512), lds, stream, p, row_bytes);
+    }
     return launched("stack_moe_plan");
 }
 

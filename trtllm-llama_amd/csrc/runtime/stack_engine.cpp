@@ -177,6 +177,7 @@ struct tllm_stack
     void *xbc = nullptr, *cq = nullptr, *qfull = nullptr, *moe_a = nullptr;
     float *moe_y = nullptr, *moe_w = nullptr;
     int32_t* moe_i = nullptr;
+    uint32_t* moe_ticket = nullptr; // behind moe_i's values: zero between launches
     // pair embedding (a hashed row per (previous token, token)) and token shift; the previous token of every slot's sequence
     int pair_buckets = 0, pair_mul_prev = 0, pair_mul_cur = 0, token_shift = 0;
     void* pair_table = nullptr;
@@ -212,6 +213,7 @@ struct tllm_stack
         xbc = cq = qfull = moe_a = nullptr;
         moe_y = moe_w = nullptr;
         moe_i = nullptr;
+        moe_ticket = nullptr;
         h32 = dl_a = dl_g = nullptr;
         pairs = nullptr;
     }
@@ -411,7 +413,11 @@ int ensure_scratch(tllm_stack* s, int tokens, int want, int n_ints)
             HIP_OK(hipMalloc(&s->moe_a, (s->max_top ? pairs * wd : 1) * es));
             HIP_OK(hipMalloc((void**) &s->moe_y, (s->max_top ? pairs * wd : 1) * 4));
             HIP_OK(hipMalloc((void**) &s->moe_w, (pairs + T * (size_t) (s->max_outputs + 1)) * 4));
-            HIP_OK(hipMalloc((void**) &s->moe_i, (4 * pairs + (size_t) s->max_experts + 1) * 4));
+            const size_t n_moe_i = 4 * pairs + (size_t) s->max_experts + 1;
+            HIP_OK(hipMalloc((void**) &s->moe_i, (n_moe_i + 1) * 4));
+            s->moe_ticket = (uint32_t*) s->moe_i + n_moe_i;
+            const uint32_t none = 0;
+            HIP_OK(hipMemcpy(s->moe_ticket, &none, sizeof(none), hipMemcpyHostToDevice));
         }
         HIP_OK(hipHostMalloc((void**) &s->pinned, NI * 4, hipHostMallocDefault));
         if (s->taps)
@@ -1761,6 +1767,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         mp.topk_w = s->moe_w;
         mp.logits = s->plain ? s->route_z : s->moe_w + pairs;
         mp.have_logits = s->plain ? 1 : 0;
+        mp.ticket = s->moe_ticket;
         mp.a_sorted = l.route_weight_input ? s->moe_a : nullptr; // otherwise the products read h1 through the slots' tokens
         mp.accumulate = accumulate ? 1 : 0;
         mp.accumulate_gate = l.shared_gate ? s->shared_z : nullptr;
