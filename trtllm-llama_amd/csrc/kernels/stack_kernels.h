@@ -72,6 +72,26 @@ int launch_stack_gemm(const StackGemmParams& p, hipStream_t stream);
 // ---------------------------------------------------------------------------------------------
 // Pointwise pieces.
 // ---------------------------------------------------------------------------------------------
+// dst[i] = src[i]: a step's metadata from pinned host memory, n a multiple of 4, both 16-byte aligned
+int launch_stack_fetch(int32_t* dst, const int32_t* host_src, int32_t n, hipStream_t stream);
+// A few wanted rows leave for pinned host memory in one launch: rows (null: not wanted) receives logits [n, vocab], choice
+// [n, stack_choice_parts(vocab)] the largest value of each part of a row and its lowest place (0x7fffffff: none), from which
+// stack_choose picks on the host: the largest, the lowest place among equals, 0 in a row without a number.
+struct StackChoice
+{
+    float value;
+    int32_t at;
+};
+int stack_choice_parts(int32_t vocab);
+int launch_stack_deliver(float* rows, StackChoice* choice, const float* logits, int32_t n, int32_t vocab, hipStream_t stream);
+inline int32_t stack_choose(const StackChoice* c, int parts)
+{
+    StackChoice best = c[0];
+    for (int i = 1; i < parts; ++i)
+        if (c[i].value > best.value || (c[i].value == best.value && c[i].at < best.at))
+            best = c[i];
+    return best.at == 0x7fffffff ? 0 : best.at;
+}
 // x[t, :] = table[ids[t], :] * scale (fp32 residual stream); keep (optional) receives the same rows; copies > 1: the row is also
 // written to x + c * copy_stride, c < copies (residual streams that all start from the embedding output)
 int launch_stack_embed(float* x, float* keep, const int32_t* ids, const void* table, int32_t dtype, int32_t tokens, int32_t width,
