@@ -455,6 +455,8 @@ struct StackDeltaParams
     float* chunk_ws = nullptr;        // optional scratch of the chunked form, as above
     size_t chunk_floats = 0;
 };
+// both, in one launch for a step of single rows
+int launch_stack_delta(const StackDeltaParams& p, hipStream_t stream);
 int launch_stack_delta_scan(const StackDeltaParams& p, hipStream_t stream);
 int launch_stack_delta_out(const StackDeltaParams& p, hipStream_t stream);
 bool stack_delta_serves(int32_t dim, int32_t vdim);

@@ -369,6 +369,91 @@ __global__ __launch_bounds__(1024) void ssm_scan_pipe_kernel(const StackSsmParam
     }
 }
 
+// One row per entry (a step of decoded tokens): nothing is walked, so the launch is bound by the latency of what it reads.  A workgroup per
+// (entry, head), thread (r, c) keeps rows 8 r .. 8 r + 7 of columns 4 c .. 4 c + 3: the state comes in 16-byte pieces, B and C as one
+// 8-value read each, all requested before the step size is known; one barrier for the sum over rows.  64 heads of 128 x 64, one
+// entry: 4.4 us, 7.9 us as a walk of one row.
+template <int DT>
+__global__ __launch_bounds__(1024) void ssm_step_kernel(const StackSsmParams p)
+{
+    extern __shared__ float part[]; // [N / 8][PH]
+    const int PH = p.vdim, N = p.state, H = p.heads, G = p.groups;
+    const int inner = H * PH, GN = G * N, CH = inner + 2 * GN;
+    const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, CT = PH >> 2;
+    const int r = tid / CT, c = tid - r * CT;
+    const bool live = r < N >> 3;
+    const int64_t row = p.ent_first[e];
+    float* sp = p.ssm_state + (((int64_t) p.ent_slot[e] * H + h) * N + 8 * (live ? r : 0)) * PH + 4 * c;
+    const int64_t bcol = row * CH + inner + (int64_t) (h / (H / G)) * N + 8 * (live ? r : 0), xcol = row * CH + h * PH;
+    typedef typename std::conditional<DT == DT_BF16, uint16_t, float>::type Raw;
+    typedef Raw Raw4 __attribute__((ext_vector_type(4)));
+    const Raw* xbc = reinterpret_cast<const Raw*>(p.xbc);
+    const Raw* prj = reinterpret_cast<const Raw*>(p.proj) + row * p.ldp;
+    auto cvt = [](Raw v) -> float {
+        if constexpr (DT == DT_BF16)
+            return bf2f(v);
+        else
+            return v;
+    };
+    const Raw rdt = prj[2 * inner + 2 * GN + h];
+    Raw4 rb[2], rc[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+    {
+        rb[k] = *reinterpret_cast<const Raw4*>(xbc + bcol + 4 * k);
+        rc[k] = *reinterpret_cast<const Raw4*>(xbc + bcol + GN + 4 * k);
+    }
+    const Raw4 rx = *reinterpret_cast<const Raw4*>(xbc + xcol + 4 * c);
+    const int v = tid < PH ? tid : PH - 1; // the column this thread finishes
+    const Raw vx = xbc[xcol + v], vz = prj[h * PH + v];
+    float4 S[8];
+    if (p.ent_pos0[e] > 0)
+    {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            S[j] = *reinterpret_cast<const float4*>(sp + (int64_t) j * PH);
+    }
+    else
+    {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            S[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    const float z = cvt(rdt) + p.dt_bias[h], dt = z > 20.f ? z : log1pf(expf(z));
+    const float a = expf(-expf(p.a_log[h]) * dt);
+    const float x[4] = {cvt(rx[0]) * dt, cvt(rx[1]) * dt, cvt(rx[2]) * dt, cvt(rx[3]) * dt};
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+    {
+        const float b = cvt(rb[j >> 2][j & 3]), cc = cvt(rc[j >> 2][j & 3]);
+        S[j].x = fmaf(a, S[j].x, b * x[0]);
+        S[j].y = fmaf(a, S[j].y, b * x[1]);
+        S[j].z = fmaf(a, S[j].z, b * x[2]);
+        S[j].w = fmaf(a, S[j].w, b * x[3]);
+        o.x = fmaf(S[j].x, cc, o.x);
+        o.y = fmaf(S[j].y, cc, o.y);
+        o.z = fmaf(S[j].z, cc, o.z);
+        o.w = fmaf(S[j].w, cc, o.w);
+    }
+    if (live)
+    {
+        *reinterpret_cast<float4*>(part + r * PH + 4 * c) = o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            *reinterpret_cast<float4*>(sp + (int64_t) j * PH) = S[j];
+    }
+    __syncthreads();
+    for (int i = tid; i < PH; i += blockDim.x)
+    {
+        float y = 0.f;
+        for (int k = 0; k < N >> 3; ++k)
+            y += part[k * PH + i];
+        const float xi = i == tid ? cvt(vx) : cvt(xbc[xcol + i]), zi = i == tid ? cvt(vz) : cvt(prj[h * PH + i]);
+        p.y32[row * inner + h * PH + i] = fmaf(p.d_skip[h], xi, y) * silu_f(zi);
+    }
+}
+
 // rows of state a thread keeps, for a head of P columns and N rows: the fewest that fit the workgroup, at least 4
 inline int slice_rows(int P, int N)
 {
@@ -437,6 +522,17 @@ int launch_stack_ssm_scan(const StackSsmParams& p, hipStream_t stream)
         const int rc = launch_stack_chunk_ssm(p, stream); // prompts: 16 rows at a time through matrix products
         if (rc <= 0)
             return rc;
+    }
+    if (p.max_count == 1 && p.state % 8 == 0 && p.vdim % 4 == 0 && (p.heads * p.vdim) % 8 == 0)
+    {
+        // (a thread per 8 x 4 values of state: at most 1024, the shapes that are served have at most 1024 x 32)
+        const int threads = (p.vdim / 4 * (p.state / 8) + 63) / 64 * 64;
+        const size_t lds = sizeof(float) * (size_t) (p.state / 8) * p.vdim;
+        if (p.dtype == DT_BF16)
+            hipLaunchKernelGGL((ssm_step_kernel<DT_BF16>), dim3(p.entries, p.heads), dim3(threads), lds, stream, p);
+        else
+            hipLaunchKernelGGL((ssm_step_kernel<DT_FLOAT>), dim3(p.entries, p.heads), dim3(threads), lds, stream, p);
+        return launched("stack_ssm_scan (one row)");
     }
     static const bool plain_only = [] {
         const char* v = std::getenv("TLLM_STACK_SSM_PLAIN"); // measurement knob: 1 = every shape on the form without prefetch

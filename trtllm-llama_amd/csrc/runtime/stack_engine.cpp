@@ -1567,7 +1567,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             dp.max_count = max_count;
             dp.chunk_ws = s->chunk_ws;
             dp.chunk_floats = s->chunk_floats;
-            return (launch_stack_delta_scan(dp, stream) || launch_stack_delta_out(dp, stream)) ? -1 : 0;
+            return launch_stack_delta(dp, stream);
         }
         if (l.kind == MIX_MAMBA2)
         {
