@@ -27,3 +27,16 @@ def test_few_token_router(router, width, equal):
     toks = tokens_for(cfg, 29, 7)
     got = replay(session_for(cfg, w, 'float32'), {'a': toks}, [[('a', k)] for k in (1, 7, 8, 9, 1, 1, 2)])['a']
     check(got, O.logits(toks, as_f64(w), cfg), tol_of('float32'), 'a')
+
+
+@pytest.mark.parametrize('n', [256, 257, 300])
+@pytest.mark.parametrize('router', [ROUTERS[1], ROUTERS[2], ROUTERS[3]], ids=lambda r: f"{r['experts']}+{r['identity']}")
+@pytest.mark.parametrize('width', [96, 128, 1056])
+def test_prompt_router(width, router, n):
+    """Logits of prompts through fp32 matrix products (from 257 tokens on, widths of whole 32-value pieces): tokens and outputs that end inside
+    a tile, widths shorter than the waves' first round and longer."""
+    cfg = make_config([mamba_layer(mlp=moe(ff=8, **router))], width=width)
+    w = random_weights(cfg, 6)
+    toks = tokens_for(cfg, n, 8)
+    got = replay(session_for(cfg, w, 'float32'), {'a': toks}, [[('a', n)]])['a']
+    check(got, O.logits(toks, as_f64(w), cfg), tol_of('float32'), 'a')

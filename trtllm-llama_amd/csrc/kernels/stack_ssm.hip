@@ -53,33 +53,12 @@ inline int launched(const char* what)
 
 constexpr int MAX_TAPS = 16;
 
-// Workgroups [0, tokens): row t, 256 channels each (blockIdx.y): rows that lie at least taps - 1 tokens into their entry read
-// nothing but the step's own projection rows.  Workgroups [tokens, tokens + entries): the first taps - 1 rows of an entry, which
-// reach into the sequence's tail of raw inputs, and the new tail - one thread per (entry, channel) reads the old tail before it
-// writes, so the launch has no ordering between workgroups to keep.
+// An entry's first taps - 1 rows of channel c, which reach into the sequence's tail of raw inputs, and the new tail: one thread per (entry,
+// channel) reads the old tail before it writes, so the launch has no ordering between workgroups to keep
 template <int DT>
-__global__ __launch_bounds__(256) void ssm_conv_kernel(const StackSsmParams p)
+__device__ __forceinline__ void conv_edges(const StackSsmParams& p, int e, int c, int CH, int64_t col, const float* w, float bias)
 {
-    const int inner = p.heads * p.vdim, CH = p.conv_channels > 0 ? p.conv_channels : inner + 2 * p.groups * p.state, K = p.taps;
-    const int c = blockIdx.y * 256 + threadIdx.x;
-    if (c >= CH)
-        return;
-    const float* w = p.conv_w + (int64_t) c * K;
-    const float bias = p.conv_b ? p.conv_b[c] : 0.f;
-    const int64_t col = (p.conv_channels > 0 ? p.conv_col : inner) + c; // mamba2: the convolution's inputs sit behind the z columns
-    if ((int) blockIdx.x < p.tokens)
-    {
-        const int t = blockIdx.x, e = p.tok_entry[t];
-        const int i = p.tok_pos[t] - p.ent_pos0[e];
-        if (i < K - 1)
-            return;
-        float acc = bias;
-        for (int k = 0; k < K; ++k)
-            acc = fmaf(w[k], ld_el<DT>(p.proj, (int64_t) (t - (K - 1) + k) * p.ldp + col), acc);
-        st_el<DT>(p.xbc, (int64_t) t * CH + c, silu_f(acc));
-        return;
-    }
-    const int e = blockIdx.x - p.tokens;
+    const int K = p.taps;
     const int first = p.ent_first[e], count = p.ent_count[e];
     float* tail = p.conv_state + (int64_t) p.ent_slot[e] * (K - 1) * CH + c;
     float old[MAX_TAPS - 1];
@@ -106,6 +85,107 @@ __global__ __launch_bounds__(256) void ssm_conv_kernel(const StackSsmParams p)
     }
     for (int j = 0; j < K - 1; ++j)
         tail[(int64_t) j * CH] = input(count - (K - 1) + j);
+}
+
+// Workgroups [0, tokens): row t, 256 channels each (blockIdx.y): rows that lie at least taps - 1 tokens into their entry read
+// nothing but the step's own projection rows.  Workgroups [tokens, tokens + entries): the entries' edges.
+template <int DT>
+__global__ __launch_bounds__(256) void ssm_conv_kernel(const StackSsmParams p)
+{
+    const int inner = p.heads * p.vdim, CH = p.conv_channels > 0 ? p.conv_channels : inner + 2 * p.groups * p.state, K = p.taps;
+    const int c = blockIdx.y * 256 + threadIdx.x;
+    if (c >= CH)
+        return;
+    const float* w = p.conv_w + (int64_t) c * K;
+    const float bias = p.conv_b ? p.conv_b[c] : 0.f;
+    const int64_t col = (p.conv_channels > 0 ? p.conv_col : inner) + c; // mamba2: the convolution's inputs sit behind the z columns
+    if ((int) blockIdx.x < p.tokens)
+    {
+        const int t = blockIdx.x, e = p.tok_entry[t];
+        const int i = p.tok_pos[t] - p.ent_pos0[e];
+        if (i < K - 1)
+            return;
+        float acc = bias;
+        for (int k = 0; k < K; ++k)
+            acc = fmaf(w[k], ld_el<DT>(p.proj, (int64_t) (t - (K - 1) + k) * p.ldp + col), acc);
+        st_el<DT>(p.xbc, (int64_t) t * CH + c, silu_f(acc));
+        return;
+    }
+    conv_edges<DT>(p, blockIdx.x - p.tokens, c, CH, col, w, bias);
+}
+
+// The rows behind an entry's first taps - 1, for prompts: a thread takes 4 neighbouring channels of RUN rows in turn and keeps the last
+// TAPS - 1 of them in registers, so that every input is read once, in 8-byte pieces, and every row's requests are out before the first is
+// used.  Bound by memory (the projection's columns in, xbc out).  What ssm_conv_kernel adds up, in its order.  A channel and a row per
+// thread read every input `taps` times, two bytes at a time: 1672 rows of 4096 channels, 4 taps, 40 us; 15 us here.
+template <int DT, int TAPS, int RUN>
+__global__ __launch_bounds__(256) void ssm_conv_run_kernel(const StackSsmParams p, int runs)
+{
+    const int inner = p.heads * p.vdim, CH = p.conv_channels > 0 ? p.conv_channels : inner + 2 * p.groups * p.state;
+    const int64_t col0 = p.conv_channels > 0 ? p.conv_col : inner;
+    if ((int) blockIdx.x >= runs) // the entries' edges, a channel per thread
+    {
+        const int c = blockIdx.y * 256 + threadIdx.x;
+        if (c < CH)
+            conv_edges<DT>(p, blockIdx.x - runs, c, CH, col0 + c, p.conv_w + (int64_t) c * TAPS, p.conv_b ? p.conv_b[c] : 0.f);
+        return;
+    }
+    const int c = (blockIdx.y * 64 + (threadIdx.x & 63)) * 4, t0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RUN;
+    if (c >= CH || t0 >= p.tokens)
+        return;
+    typedef typename std::conditional<DT == DT_BF16, uint16_t, float>::type Raw;
+    typedef Raw Raw4 __attribute__((ext_vector_type(4)));
+    const Raw* in = reinterpret_cast<const Raw*>(p.proj) + col0 + c;
+    Raw4 x[RUN + TAPS - 1]; // rows t0 - (TAPS - 1) .. t0 + RUN - 1, clamped into the step
+    int place[RUN];         // rows into its entry
+#pragma unroll
+    for (int i = 0; i < RUN + TAPS - 1; ++i)
+    {
+        const int t = t0 - (TAPS - 1) + i;
+        x[i] = *reinterpret_cast<const Raw4*>(in + (int64_t) (t < 0 ? 0 : t < p.tokens ? t : p.tokens - 1) * p.ldp);
+    }
+#pragma unroll
+    for (int i = 0; i < RUN; ++i)
+    {
+        const int t = t0 + i < p.tokens ? t0 + i : p.tokens - 1;
+        place[i] = t0 + i < p.tokens ? p.tok_pos[t] - p.ent_pos0[p.tok_entry[t]] : 0;
+    }
+    float w[4][TAPS], bias[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+    {
+        bias[j] = p.conv_b ? p.conv_b[c + j] : 0.f;
+#pragma unroll
+        for (int k = 0; k < TAPS; ++k)
+            w[j][k] = p.conv_w[(int64_t) (c + j) * TAPS + k];
+    }
+    auto cvt = [](Raw v) -> float {
+        if constexpr (DT == DT_BF16)
+            return bf2f(v);
+        else
+            return v;
+    };
+#pragma unroll
+    for (int i = 0; i < RUN; ++i)
+    {
+        if (place[i] < TAPS - 1) // (an entry's first rows, and rows behind the step's last)
+            continue;
+        Raw4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+        {
+            float acc = bias[j];
+#pragma unroll
+            for (int k = 0; k < TAPS; ++k)
+                acc = fmaf(w[j][k], cvt(x[i + k][j]), acc);
+            acc = silu_f(acc);
+            if constexpr (DT == DT_BF16)
+                o[j] = f2bf(acc);
+            else
+                o[j] = acc;
+        }
+        *reinterpret_cast<Raw4*>(reinterpret_cast<Raw*>(p.xbc) + (int64_t) (t0 + i) * CH + c) = o;
+    }
 }
 
 // One workgroup per (entry, head): thread (s, v) keeps rows [s NSZ, (s + 1) NSZ) of state column S[:, v] in registers.  Rows go
@@ -504,6 +584,22 @@ int launch_stack_ssm_conv(const StackSsmParams& p, hipStream_t stream)
     else if (!ssm_ok(p, "stack_ssm_conv"))
         return -1;
     const int CH = p.conv_channels > 0 ? p.conv_channels : p.heads * p.vdim + 2 * p.groups * p.state;
+    // prompts of 4 taps (the usual number) in runs of rows
+    constexpr int RUN = 8;
+    const int64_t col = p.conv_channels > 0 ? p.conv_col : p.heads * p.vdim;
+    const uintptr_t piece = p.dtype == DT_BF16 ? 7 : 15;
+    const bool runs = p.taps == 4 && p.tokens >= 64 && CH % 4 == 0 && col % 4 == 0 && p.ldp % 4 == 0
+        && !((reinterpret_cast<uintptr_t>(p.proj) | reinterpret_cast<uintptr_t>(p.xbc)) & piece);
+    if (runs)
+    {
+        const int n = (p.tokens + 4 * RUN - 1) / (4 * RUN);
+        const dim3 rg(n + p.entries, (CH + 255) / 256);
+        if (p.dtype == DT_BF16)
+            hipLaunchKernelGGL((ssm_conv_run_kernel<DT_BF16, 4, RUN>), rg, dim3(256), 0, stream, p, n);
+        else
+            hipLaunchKernelGGL((ssm_conv_run_kernel<DT_FLOAT, 4, RUN>), rg, dim3(256), 0, stream, p, n);
+        return launched("stack_ssm_conv (runs)");
+    }
     const dim3 grid(p.tokens + p.entries, (CH + 255) / 256);
     if (p.dtype == DT_BF16)
         hipLaunchKernelGGL((ssm_conv_kernel<DT_BF16>), grid, dim3(256), 0, stream, p);
