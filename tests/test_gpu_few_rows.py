@@ -1,4 +1,4 @@
-"""Products of 2 .. 31 rows through the weight-streaming MFMA kernels (gemm_slim_impl.h): LLaMA plugins in every weight type and the stack
+"""Products of few rows (2 .. 31; LLaMA: from 5, int4 weights from 3) through the weight-streaming MFMA kernels (gemm_slim_impl.h): LLaMA plugins in every weight type and the stack
 engine, at the edges of the row tiles (9, 16, 17, 31 rows), ragged columns, rows of W that end inside a 256-byte block or are shorter
 than the waves' first round, and both launch shapes (from 5120 columns on)."""
 import numpy as np
@@ -11,7 +11,7 @@ from tensorrt_llm.plugin import capi
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(9, 13, 64), (16, 40, 320), (17, 272, 1184), (31, 1003, 2080), (24, 64, 4096), (31, 5136, 544), (12, 5121, 256)]
+SHAPES = [(3, 64, 1184), (5, 40, 320), (8, 1003, 2080), (9, 13, 64), (16, 40, 320), (17, 272, 1184), (31, 1003, 2080), (24, 64, 4096), (31, 5136, 544), (12, 5121, 256)]
 
 
 @pytest.mark.parametrize('m,n,k', SHAPES)
@@ -74,3 +74,40 @@ def test_stack_decode_of_many_requests(requests):
     got = replay(session_for(cfg, w, 'bfloat16', max_tokens=64 * requests, max_sequences=requests), reqs, schedule)
     for i, toks in reqs.items():
         check_rows(got[i], toks, w, cfg, 'bfloat16', i)
+
+
+@pytest.mark.parametrize('mode,int8_kv', [('fp16', 0), ('woq8', 1), ('woq4', 0)])
+@pytest.mark.parametrize('batch', [2, 3, 5, 8, 17, 32, 33])
+def test_llama_decode_of_several_sequences(batch, mode, int8_kv):
+    """Generation steps whose products take the norm ahead of them and the residual or SwiGLU behind them, on both sides of the rows where
+    that form starts and ends, eager and captured; bounds of test_gpu_session.test_quantised_paths_vs_oracle."""
+    from oracle import quant_oracle as QO
+    from tensorrt_llm.runtime.native import NativeSession
+    from test_gpu_session import synth_model
+    cfg, w = synth_model(11)
+    S, NEW = 6, 4
+    r = np.random.default_rng(batch)
+    ids = r.integers(3, cfg['vocab_size'], (batch, S)).astype(np.int32)
+    lens = r.integers(2, S + 1, batch).astype(np.int32)
+    lens[0] = S
+    for b in range(batch):
+        ids[b, lens[b]:] = 2
+    q = QO.quantise_model(cfg, w, mode, int8_kv, calib_ids=ids, calib_lens=lens)
+    s = NativeSession(dict(cfg, quant_mode=q['quant_mode']))
+    for k, v in q['engine_tensors'].items():
+        s.set_tensor(k, v)
+    s.finalize()
+    s.setup(batch, S, NEW)
+    s.context(ids, lens)
+    got = [s.logits()]
+    s.step(1, use_graph=False)
+    got.append(s.logits())
+    s.step(2, use_graph=True)
+    got.append(s.logits())
+    out = s.output_ids()
+    s.close()
+    ref, _ = QO.run_model(q, ids, lens, NEW, feed_ids=out[:, S:S + NEW])
+    scale = max(np.abs(ref[0]).max(), 1.0)
+    for g, want in ((got[0], ref[0]), (got[1], ref[1]), (got[2], ref[3])):
+        np.testing.assert_allclose(g, want, atol=1e-2 * scale)
+        assert np.abs(g - want).mean() < 2.5e-3 * scale

@@ -1,7 +1,7 @@
 // GEMM entry point of the Gemm / SmoothQuantGemm / WeightOnlyQuantMatmul plugins.
-//   M <= 8  -> the streaming GEMV (gemv.hip), the decode path;
-//   M 9..31 -> the weight-streaming MFMA product (gemm_slim.hip): a 19-token prompt's projections are bound by the weights, not by MFMA tiles
-//              (weight-only int8, 12288 x 4096 at 19 rows: 26 us; the 128 x 128 register-staged tiles took 116);
+//   a few   -> the streaming GEMV (gemv.hip), the decode path;
+//   M 5..31 -> (int4 weights 3..31) the weight-streaming MFMA product (gemm_slim.hip): a 19-token prompt's projections are bound by the weights,
+//              not by MFMA tiles (weight-only int8, 12288 x 4096 at 19 rows: 26 us; the 128 x 128 register-staged tiles took 116);
 //   M >= 32 -> MFMA tiles: LDS-DMA staged (gemm_glds.hip: SQ / fp16, K-bytes % 128 == 0; gemm_woq.hip: weight-only), else register staged
 //              with in-flight dequantisation (gemm_mfma.hip: odd K);
 //   shapes that none of these serves -> 8-row GEMV slabs.
@@ -17,7 +17,6 @@ namespace kernels
 
 int launch_gemm_mfma(const GemmParams& p, hipStream_t stream); // gemm_mfma.hip; returns 1 when the shape is unsupported
 int launch_gemm_woq(const GemmParams& p, hipStream_t stream);  // gemm_woq.hip (weight-only, dequantisation in the main loop); same
-int launch_gemm_slim(const GemmParams& p, hipStream_t stream); // gemm_slim.hip (few rows, every type); same
 int launch_gemm_glds(const GemmParams& p, hipStream_t stream); // gemm_glds.hip (SQ / fp16, LDS-DMA staged); same convention
 
 using namespace dev;
@@ -112,11 +111,15 @@ int launch_gemm(const GemmParams& pin, hipStream_t stream)
             return launch_swiglu(pin.c, pin.silu_gate, pin.c, (int64_t) pin.M * pin.N, stream); // elementwise: in place is fine
         return rc;
     };
+    if (pin.M < 32 && pin.M >= gemm_slim_rows(pin.wtype))
+    {
+        const int r = launch_gemm_slim(pin, stream); // fuses both
+        if (r <= 0)
+            return r;
+    }
     if (p.M > 8)
     {
-        int r = p.M < 32 ? launch_gemm_slim(p, stream) : 1;
-        if (r > 0)
-            r = launch_gemm_mfma(p, stream);
+        const int r = launch_gemm_mfma(p, stream);
         if (r <= 0)
             return finish(r);
     }

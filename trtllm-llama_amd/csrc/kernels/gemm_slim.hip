@@ -50,7 +50,17 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_slim_kernel(const GemmParams 
                     v = acc[e] * h2f(reinterpret_cast<const uint16_t*>(p.scale_col)[col]);
                 const int64_t o = (int64_t) row * p.ldc + col;
                 if (p.out_dtype == DT_HALF)
-                    reinterpret_cast<uint16_t*>(p.c)[o] = f2h(v);
+                {
+                    uint16_t y = f2h(v); // (what follows: the pointwise passes' own rounding points)
+                    if (p.residual)
+                        y = f2h(h2f(y) + h2f(reinterpret_cast<const uint16_t*>(p.residual)[o]));
+                    else if (p.silu_gate)
+                    {
+                        const float g = h2f(reinterpret_cast<const uint16_t*>(p.silu_gate)[o]);
+                        y = f2h(h2f(f2h(g / (1.f + __expf(-g)))) * h2f(y));
+                    }
+                    reinterpret_cast<uint16_t*>(p.c)[o] = y;
+                }
                 else if (SQ && p.out_dtype == DT_INT32)
                     reinterpret_cast<int32_t*>(p.c)[o] = f2i32_rni_sat(v);
                 else
@@ -85,11 +95,20 @@ int launch_wt(const GemmParams& p, hipStream_t stream)
 
 } // namespace
 
-// 0: launched, -1: launch error, 1: not served (row counts, alignment)
+// Rows from which this form is the quicker one (the streaming GEMV's time grows with the rows: dot products on the vector pipe, and LDS for
+// every row's activations).  Cold weights, us at 4 / 5 / 8 rows by the GEMV and at 9 here: fp16 4096 x 4096 9.3 / 11.5 / 12.0, 9.8; fp16
+// 4096 x 11008 19.9 / 36.8 / 39.3, 19.8; SmoothQuant 4096 x 11008 12.9 / 15.5 / 16.5, 12.7; int8 weights 12288 x 4096 16.0 / 28.6 / 28.9,
+// 16.8; int4 weights 12288 x 4096 at 2 / 4 / 5 rows 16.4 / 31.5 / 195, 15.0.
+int gemm_slim_rows(int wtype)
+{
+    return wtype == W_INT4_WOQ ? 3 : 5;
+}
+
+// 0: launched, -1: launch error, 1: not served (row counts, alignment).  residual and silu_gate share c's rows; c may be the residual itself
 int launch_gemm_slim(const GemmParams& p, hipStream_t stream)
 {
     const int a_es = p.wtype == W_INT8_SQ ? 1 : 2;
-    if (p.M < 1 || p.M > 32 || p.N < 1 || p.K < 1 || p.residual || p.silu_gate)
+    if (p.M < 1 || p.M > 32 || p.N < 1 || p.K < 1 || ((p.residual || p.silu_gate) && p.out_dtype != DT_HALF))
         return 1;
     // 16-byte loads of both operands; 32-bit offsets of a workgroup's W rows
     if ((reinterpret_cast<uintptr_t>(p.a) & 15) || ((p.lda * a_es) & 15) || (reinterpret_cast<uintptr_t>(p.w) & 15) || (p.ldw & 15) || p.ldw > (1 << 26))

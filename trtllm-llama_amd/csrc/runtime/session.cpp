@@ -431,11 +431,75 @@ struct tllm_session
     }
 
     // ------------------------------------------------------------------------------------------ GEMM wrappers
+    // decode of several sequences with fp16 or weight-only weights: the norm, then the weight-streaming MFMA product (one pass over the
+    // weights for up to 32 rows) with the residual or the SwiGLU in its epilogue.  -> whether this form serves the call (rc: its status)
+    bool few_rows(const Linear& L, int M, int pro, int epi, const void* xin, int64_t ldx, const void* gamma, const void* residual, void* y,
+        int64_t ldy, int out_dtype, const Linear* up, hipStream_t st, int& rc)
+    {
+        const bool norm = pro == PRO_RMSNORM, swiglu = epi == EPI_SWIGLU;
+        if ((pro != PRO_NONE && !norm) || (epi != EPI_NONE && epi != EPI_RESIDUAL && !swiglu) || (out_dtype != DT_HALF && (epi != EPI_NONE || out_dtype != DT_FLOAT))
+            || (swiglu && (!up || up->wtype != L.wtype || up->N != L.N || up->K != L.K || L.N > Ir || ldy != L.N || (reinterpret_cast<uintptr_t>(up->w) & 15) || (up->ldw & 15))) || (norm && (L.K != hidden || ldx != hidden || xin == tmp || !tmp)))
+            return false;
+        GemmParams g;
+        g.wtype = L.wtype;
+        g.out_dtype = swiglu ? (int) DT_HALF : out_dtype;
+        g.M = M;
+        g.N = L.N;
+        g.K = L.K;
+        g.a = norm ? tmp : xin;
+        g.lda = norm ? hidden : ldx;
+        g.w = L.w;
+        g.ldw = L.ldw;
+        g.scale_col = L.scale_col;
+        g.scale_row = L.act_scale;
+        g.per_channel = L.per_channel;
+        g.c = swiglu ? this->g : y;
+        g.ldc = swiglu ? (int64_t) L.N : ldy;
+        g.residual = epi == EPI_RESIDUAL ? residual : nullptr;
+        // the products refuse a shape before they launch, but the norm is ahead of them: what decides is asked here
+        if ((g.lda * 2) % 16 || (reinterpret_cast<uintptr_t>(g.a) & 15) || (reinterpret_cast<uintptr_t>(g.w) & 15) || (g.ldw & 15) || L.K % 32)
+            return false;
+        rc = timed(gemv_cls, st, [&] {
+            if (norm)
+            {
+                RmsnormParams r;
+                r.M = M;
+                r.N = hidden;
+                r.x = xin;
+                r.gamma = gamma;
+                r.eps = eps;
+                r.y = tmp;
+                RUN(launch_rmsnorm(r, st));
+            }
+            if (launch_gemm_slim(g, st))
+                return 1;
+            if (!swiglu)
+                return 0;
+            GemmParams q = g;
+            q.w = up->w;
+            q.ldw = up->ldw;
+            q.scale_col = up->scale_col;
+            q.scale_row = up->act_scale;
+            q.per_channel = up->per_channel;
+            q.c = y;
+            q.ldc = ldy;
+            q.silu_gate = this->g;
+            return launch_gemm_slim(q, st) ? 1 : 0;
+        });
+        return true;
+    }
+
     // decode: fused skinny GEMM
     int gemv(const Linear& L, int M, int pro, int epi, const void* xin, int64_t ldx, const void* gamma,
         const float* in_qscale, const void* residual, const float* epi_scale, void* y, int64_t ldy, int out_dtype,
         const Linear* up, hipStream_t st, const float* row_scales = nullptr)
     {
+        if (L.wtype != W_INT8_SQ && M >= gemm_slim_rows(L.wtype) && M <= 32 && !row_scales && !tap_dst)
+        {
+            int rc = 1;
+            if (few_rows(L, M, pro, epi, xin, ldx, gamma, residual, y, ldy, out_dtype, up, st, rc))
+                return rc;
+        }
         GemvParams p;
         p.wtype = L.wtype;
         p.pro = pro;
