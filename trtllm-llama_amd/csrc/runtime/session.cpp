@@ -432,17 +432,18 @@ struct tllm_session
 
     // ------------------------------------------------------------------------------------------ GEMM wrappers
     // decode of several sequences with fp16 or weight-only weights: the norm, then the weight-streaming MFMA product (one pass over the
-    // weights for up to 32 rows) with the residual or the SwiGLU in its epilogue.  -> whether this form serves the call (rc: its status)
+    // weights for up to 32 rows) with the residual or the SwiGLU in its epilogue.  (The head stays with
+    // launch_gemv: a sequence's fp32 logits are the same bits alone and in a batch.)  -> whether this form serves the call (rc: its status)
     bool few_rows(const Linear& L, int M, int pro, int epi, const void* xin, int64_t ldx, const void* gamma, const void* residual, void* y,
         int64_t ldy, int out_dtype, const Linear* up, hipStream_t st, int& rc)
     {
         const bool norm = pro == PRO_RMSNORM, swiglu = epi == EPI_SWIGLU;
-        if ((pro != PRO_NONE && !norm) || (epi != EPI_NONE && epi != EPI_RESIDUAL && !swiglu) || (out_dtype != DT_HALF && (epi != EPI_NONE || out_dtype != DT_FLOAT))
+        if ((pro != PRO_NONE && !norm) || (epi != EPI_NONE && epi != EPI_RESIDUAL && !swiglu) || out_dtype != DT_HALF
             || (swiglu && (!up || up->wtype != L.wtype || up->N != L.N || up->K != L.K || L.N > Ir || ldy != L.N || (reinterpret_cast<uintptr_t>(up->w) & 15) || (up->ldw & 15))) || (norm && (L.K != hidden || ldx != hidden || xin == tmp || !tmp)))
             return false;
         GemmParams g;
         g.wtype = L.wtype;
-        g.out_dtype = swiglu ? (int) DT_HALF : out_dtype;
+        g.out_dtype = DT_HALF;
         g.M = M;
         g.N = L.N;
         g.K = L.K;
