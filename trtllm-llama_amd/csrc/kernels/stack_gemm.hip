@@ -13,7 +13,6 @@
 #include "gemm_seam.h"
 #include "gemm_slim_impl.h"
 #include "stack_kernels.h"
-#include <cstdlib>
 
 namespace tllm
 {
