@@ -588,6 +588,8 @@ struct tllm_session
         g.per_token = per_tok;
         g.c = c;
         g.ldc = L.N;
+        if (residual && M < 32) // in place: launch_gemm leaves that to the kernels of many rows
+            return launch_gemm_slim(g, st) ? 1 : 0;
         return launch_gemm(g, st) ? 1 : 0;
     }
 
@@ -731,8 +733,11 @@ struct tllm_session
             }
             // (weight-only: gemm_woq.hip adds the residual in its epilogue too - same two roundings; its own serve conditions)
             const bool woq_w = L.dense.wtype == W_INT8_WOQ || L.dense.wtype == W_INT4_WOQ;
-            const bool fuse_res = tp == 1 && !force_comm && M >= 32 && D % 8 == 0
-                && (woq_w ? (L.dense.K % 64 == 0 && L.proj.K % 64 == 0)
+            // (short prompts: gemm_slim.hip serves rows of whole 32-value pieces, in place)
+            const bool few_res = M < 32 && M >= gemm_slim_rows(L.dense.wtype) && L.dense.wtype == L.proj.wtype && L.dense.K % 32 == 0
+                && L.proj.K % 32 == 0 && !(L.dense.ldw & 15) && !(L.proj.ldw & 15);
+            const bool fuse_res = tp == 1 && !force_comm && (few_res || (M >= 32 && D % 8 == 0))
+                && (few_res ? true : woq_w ? (L.dense.K % 64 == 0 && L.proj.K % 64 == 0)
                           : ((L.dense.wtype == W_INT8_SQ || L.dense.wtype == W_FP16)
                               && (L.dense.K * (L.dense.wtype == W_FP16 ? 2 : 1)) % 128 == 0
                               && (L.proj.K * (L.proj.wtype == W_FP16 ? 2 : 1)) % 128 == 0));
