@@ -36,6 +36,13 @@ SCHEDULES = {
 }
 
 
+def check_request(mod, kind, got, toks, w, cfg, dtype, rid):
+    if kind == 'mamba2':
+        mod.check(got, mod.O.logits(toks, mod.as_f64(w), cfg), mod.tol_of(dtype), rid)
+    else:
+        mod.check_rows(got, toks, w, cfg, dtype, rid)
+
+
 def run(kind, dim, vdim, dtype, schedule, extreme=False):
     mod, cfg, decay = KINDS[kind](dim, vdim)
     steps = SCHEDULES[schedule]
@@ -53,10 +60,7 @@ def run(kind, dim, vdim, dtype, schedule, extreme=False):
             w['l0.mix.lower'] = np.zeros_like(w['l0.mix.lower'])
     got = mod.replay(mod.session_for(cfg, w, dtype), reqs, steps)
     for rid, toks in reqs.items():
-        if kind == 'mamba2':
-            mod.check(got[rid], mod.O.logits(toks, mod.as_f64(w), cfg), mod.tol_of(dtype), rid)
-        else:
-            mod.check_rows(got[rid], toks, w, cfg, dtype, rid)
+        check_request(mod, kind, got[rid], toks, w, cfg, dtype, rid)
 
 
 @pytest.mark.parametrize('schedule', sorted(SCHEDULES))
@@ -70,3 +74,35 @@ def test_portions(kind, dim, vdim, dtype, schedule):
 @pytest.mark.parametrize('kind', sorted(KINDS))
 def test_decays_from_none_to_all_in_one_chunk(kind):
     run(kind, 64, 24, 'float32', 'unequal', extreme=True)
+
+
+@pytest.mark.parametrize('where', [33, 47, 96])
+@pytest.mark.parametrize('what', ['row', 'value'])
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('kind', sorted(KINDS))
+def test_a_row_without_finite_numbers_leaves_the_earlier_ones_alone(kind, dtype, what, where):
+    """Row `where` of a request is NaN in every channel, or its values overflow: the rows before it, in the same chunk too, are what the oracle
+    has for the prompt that ends there, and the request beside it is untouched.  (The last place is a chunk of one row.)"""
+    dim, vdim = 64, 24
+    mod, cfg, _ = KINDS[kind](dim, vdim)
+    toks, other = mod.tokens_for(cfg, 97, 3), mod.tokens_for(cfg, 20, 4)
+    bad = next(t for t in range(cfg['vocab']) if t not in toks and t not in other)
+    w = mod.random_weights(cfg, 11)
+    if what == 'row':
+        w['embed'][bad] = np.nan
+    else:  # channel 0 is the bad token's alone, and the values read it with a weight near the type's largest
+        for name in ('embed', 'bigram'):
+            if name in w:
+                w[name][:, 0] = 0.0
+        w['embed'][bad, 0] = 20.0
+        w['l0.norm1'][0] = 1.0
+        if kind == 'mamba2':
+            inner = 4 * vdim
+            w['l0.mix.in'][inner:2 * inner, 0] = tolenex_cases.bf16_round(np.float32(3e38))
+        else:
+            w['l0.mix.v'][:, 0] = tolenex_cases.bf16_round(np.float32(3e38))
+    toks[where] = bad
+    got = mod.replay(mod.session_for(cfg, w, dtype), {'b': other, 'a': toks}, [[('b', 20), ('a', 97)]])
+    assert not np.isfinite(got['a'][where]).all()
+    check_request(mod, kind, got['a'][:where], toks[:where], w, cfg, dtype, 'a')
+    check_request(mod, kind, got['b'], other, w, cfg, dtype, 'b')

@@ -367,7 +367,7 @@ __global__ __launch_bounds__(256) void ssm_prepare_kernel(const ChunkArgs a)
         float w = s <= t ? dts[i * R + s] : 0.f;
         for (int k = s + 1; k <= t; ++k)
             w *= fs[i * R + k];
-        a.pm[ch * R * R + tid] = dot * w;
+        a.pm[ch * R * R + tid] = s <= t ? dot * w : 0.f; // (the dot of an overflowed row times 0 is no 0)
     }
     for (int i = tid; i < per * R; i += 256)
     {
@@ -383,6 +383,38 @@ __global__ __launch_bounds__(256) void ssm_prepare_kernel(const ChunkArgs a)
         if (tt == R - 1)
             o[2 * R] = b;
     }
+}
+
+// whether any lane of the wave holds an infinity, a NaN or a value near them
+__device__ __forceinline__ bool any_large(const f32x4& x)
+{
+    return __builtin_amdgcn_ballot_w64(!((fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3])) < 1e30f)) != 0;
+}
+__device__ __forceinline__ float pick(const f32x4& x, int i)
+{
+    return i < 2 ? (i ? x[1] : x[0]) : (i == 2 ? x[2] : x[3]);
+}
+
+// acc + M x of a lower triangular M [16, 16] (A-operand layout: M[lane & 15][4 (lane >> 4) + j] in element j) and x (B-operand layout: row
+// 4 (lane >> 4) + j), j in [j0, j1), over the rows s <= t alone
+__device__ __forceinline__ f32x4 lower_product(const f32x4& m, const f32x4& x, int j0, int j1, f32x4 acc)
+{
+    const int lane = threadIdx.x & 63, g4 = lane >> 4;
+#pragma unroll 1
+    for (int g = 0; g < 4; ++g)
+#pragma unroll 1
+        for (int j = j0; j < j1; ++j)
+        {
+            const float mj = pick(m, j), xs = __shfl(pick(x, j), (lane & 15) + 16 * g, 64);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                const int t = 4 * g4 + i;
+                const float mt = __shfl(mj, t + 16 * g, 64);
+                acc[i] = 4 * g + j <= t ? fmaf(mt, xs, acc[i]) : acc[i];
+            }
+        }
+    return acc;
 }
 
 // One workgroup per (entry, head, 16 columns of V): TILES * 64 rows of state (D), wave w keeps rows 16 (w + 4 j) .. + 16
@@ -453,7 +485,6 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
         else
             return r;
     };
-    auto pick = [](const f32x4& x, int i) { return i < 2 ? (i ? x[1] : x[0]) : (i == 2 ? x[2] : x[3]); };
 
     auto chunk = [&](int j, const Ops& o) {
         const int buf = j & 1;
@@ -480,25 +511,16 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
         accr = accr + accr1;
         if constexpr (MODE == SSM)
             acc = acc * o.bt;
+        const f32x4 past = acc; // what the rows ahead of the chunk give
         if constexpr (MODE != DELTA) // this wave's quarter of P u
             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pick(o.p, wid), pick(u, wid), acc, 0, 0, 0);
         po[buf][wid][lane] = acc;
         if constexpr (MODE == DELTA)
             pr[buf][wid][lane] = accr;
         __syncthreads();
-        f32x4 out = {0.f, 0.f, 0.f, 0.f};
+        f32x4 out = {0.f, 0.f, 0.f, 0.f}, x = u;
         if constexpr (MODE == DELTA)
-        {
-            const f32x4 x = u - ((pr[buf][0][lane] + pr[buf][1][lane]) + (pr[buf][2][lane] + pr[buf][3][lane]));
-            u = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                u = __builtin_amdgcn_mfma_f32_16x16x4f32(o.t[i], x[i], u, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                out = __builtin_amdgcn_mfma_f32_16x16x4f32(o.p[i], u[i], out, 0, 0, 0);
-        }
-        const f32x4 us = MODE == SSM ? u * o.ws : u;
+            x = u - ((pr[buf][0][lane] + pr[buf][1][lane]) + (pr[buf][2][lane] + pr[buf][3][lane]));
 #pragma unroll
         for (int n = 0; n < TILES; ++n)
         {
@@ -506,10 +528,39 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
                 S[n] = S[n] * o.b16;
             else
                 S[n] = S[n] * o.b[n];
+        }
+        // The zeros of P and T above their diagonals meet every row in a matrix product, and 0 times an infinity or a NaN is a NaN: where a row
+        // has one, the outputs are formed again row by row, without what follows a row (the state takes every row in any case).  All waves hold
+        // the same x, so that the branch is the workgroup's.  (Delta rule: u overflows only where x is near it, T's entries are below 2^15.)
+        const bool large = any_large(x);
+        if (large)
+        {
+            if constexpr (MODE == DELTA)
+                out = lower_product(o.p, lower_product(o.t, x, 0, 4, out), 0, 4, out);
+            else
+            {
+                po[buf][wid][lane] = lower_product(o.p, u, wid, wid + 1, past); // (nobody reads this chunk's po ahead of the barrier below)
+                __syncthreads();
+            }
+        }
+        if constexpr (MODE == DELTA)
+        {
+            u = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                u = __builtin_amdgcn_mfma_f32_16x16x4f32(o.t[i], x[i], u, 0, 0, 0);
+            f32x4 pu = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                pu = __builtin_amdgcn_mfma_f32_16x16x4f32(o.p[i], u[i], pu, 0, 0, 0);
+            out = large ? out : pu;
+        }
+        const f32x4 us = MODE == SSM ? u * o.ws : u;
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 S[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kt[n][i], us[i], S[n], 0, 0, 0);
-        }
         // wave w finishes rows 4 g + w
         const float* pf = reinterpret_cast<const float*>(&po[buf][0][0]);
         float y = ((pf[lane * 4 + wid] + pf[256 + lane * 4 + wid]) + (pf[512 + lane * 4 + wid] + pf[768 + lane * 4 + wid])) + pick(out, wid);
