@@ -1,0 +1,134 @@
+// A HIP runtime for tests of the stack engine's host side on a machine without a GPU: loaded ahead of libtllm_stack_engine.so, it takes the
+// place of the 20 runtime calls that the library makes.  Device memory is host memory within a budget, launches are recorded and compute
+// nothing.  Launch limits are the runtime's documented ones: fewer than 2^32 threads per grid dimension, 65535 workgroups in y and z.
+#include <hip/hip_runtime_api.h>
+#include <cstdint>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+
+namespace
+{
+struct Config
+{
+    dim3 grid, block;
+    size_t shared;
+    hipStream_t stream;
+};
+std::vector<Config> g_configs;
+std::map<void*, size_t> g_device, g_pinned;
+std::map<const void*, std::string> g_names;
+std::string g_launched;
+size_t g_live = 0, g_budget = ~size_t(0), g_largest = 0;
+int g_host_mallocs = 0, g_syncs = 0;
+hipError_t g_last = hipSuccess;
+
+hipError_t done(hipError_t e)
+{
+    if (e != hipSuccess)
+        g_last = e;
+    return e;
+}
+hipError_t release(std::map<void*, size_t>& from, void* p)
+{
+    if (!p)
+        return hipSuccess;
+    auto it = from.find(p);
+    if (it == from.end())
+        return done(hipErrorInvalidValue);
+    if (&from == &g_device)
+        g_live -= it->second;
+    from.erase(it);
+    std::free(p);
+    return hipSuccess;
+}
+} // namespace
+
+extern "C" {
+// what the tests ask
+void stub_budget(size_t bytes) { g_budget = bytes; }
+size_t stub_live() { return g_live; }
+int stub_has_allocation(size_t bytes)
+{
+    for (auto& a : g_device)
+        if (a.second == bytes)
+            return 1;
+    return 0;
+}
+int stub_host_mallocs() { return g_host_mallocs; }
+int stub_device_syncs() { return g_syncs; }
+size_t stub_pinned_bytes()
+{
+    size_t n = 0;
+    for (auto& a : g_pinned)
+        n += a.second;
+    return n;
+}
+const char* stub_launched() { return g_launched.c_str(); } // kernel names since the last stub_forget, a line each
+void stub_forget() { g_launched.clear(); }
+
+hipError_t hipMalloc(void** p, size_t n)
+{
+    if (n > g_budget || g_live > g_budget - n)
+        return done(hipErrorOutOfMemory);
+    *p = std::malloc(n ? n : 1); // (large ones are mapped on demand: nothing computes on them)
+    g_device[*p] = n;
+    g_live += n;
+    return hipSuccess;
+}
+hipError_t hipFree(void* p) { return release(g_device, p); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned int)
+{
+    ++g_host_mallocs;
+    *p = std::calloc(1, n ? n : 1);
+    g_pinned[*p] = n;
+    return hipSuccess;
+}
+hipError_t hipHostFree(void* p) { return release(g_pinned, p); }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { return std::memmove(d, s, n), hipSuccess; }
+hipError_t hipMemset(void*, int, size_t) { return hipSuccess; }
+hipError_t hipDeviceSynchronize() { return ++g_syncs, hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : e == hipSuccess ? "no error" : "invalid configuration"; }
+hipError_t hipGetLastError()
+{
+    const hipError_t e = g_last;
+    g_last = hipSuccess;
+    return e;
+}
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void**, size_t, hipStream_t)
+{
+    auto it = g_names.find(f);
+    g_launched += (it == g_names.end() ? std::string("?") : it->second) + "\n";
+    const bool fits = grid.x && grid.y && grid.z && (uint64_t) grid.x * block.x < (1ull << 32) && grid.y <= 65535 && grid.z <= 65535;
+    return done(fits ? hipSuccess : hipErrorInvalidConfiguration);
+}
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t shared, hipStream_t stream)
+{
+    g_configs.push_back({grid, block, shared, stream});
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shared, hipStream_t* stream)
+{
+    const Config c = g_configs.back();
+    g_configs.pop_back();
+    *grid = c.grid;
+    *block = c.block;
+    *shared = c.shared;
+    *stream = c.stream;
+    return hipSuccess;
+}
+void** __hipRegisterFatBinary(const void*)
+{
+    static void* module = nullptr;
+    return &module;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned int, void*, void*, void*, void*, int*) { g_names[host] = name; }
+}

@@ -1,0 +1,84 @@
+"""Host side of the stack engine's step - scratch, pinned memory, launch shapes - over a stand-in for the HIP runtime (hip_stub.cpp), without a
+GPU: nothing is computed, but every allocation and launch is the real code's.  Each scenario runs in a process of its own, with the stand-in
+loaded ahead of the library."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope='module')
+def stub(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp('stub') / 'hip_stub.so')
+    subprocess.run(['g++', '-shared', '-fPIC', '-std=c++17', '-O1', '-D__HIP_PLATFORM_AMD__', '-I/opt/rocm/include', os.path.join(HERE, 'hip_stub.cpp'), '-o', out],
+                   check=True)
+    return out
+
+
+def run(stub, scenario, *args):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), stub, scenario, *map(str, args)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+# ------------------------------------------------------------------------------------------------------------ in the child process
+class Stub:
+    def __init__(self, path):
+        self.lib = ctypes.CDLL(path, mode=ctypes.RTLD_GLOBAL)
+        self.lib.stub_budget.argtypes = self.lib.stub_has_allocation.argtypes = [ctypes.c_size_t]
+        self.lib.stub_live.restype = self.lib.stub_pinned_bytes.restype = ctypes.c_size_t
+        self.lib.stub_launched.restype = ctypes.c_char_p
+        for p in (os.path.dirname(HERE), os.path.join(os.path.dirname(HERE), 'trtllm-llama_amd'), HERE):
+            sys.path.insert(0, p)
+
+    def __getattr__(self, name):
+        return getattr(self.lib, 'stub_' + name)
+
+    def kernels(self):
+        return self.launched().decode().split()
+
+
+def engine(cfg, cases, dtype='bfloat16', **kw):
+    from tensorrt_llm.runtime import RaggedGenerationSession
+    return RaggedGenerationSession(cases.as_model(cfg, cases.random_weights(cfg, 1)), dtype=dtype, **kw)
+
+
+def step(s, rid, n, want=1, **kw):
+    return s.step([(rid, [1] * n, list(range(want)))], end=(rid,), **kw)
+
+
+def chunk_floats(tokens, entries, heads, vector_heads, dim, vectors, mamba=False):
+    """Per chunk of 16 rows: `vectors` of them per row and head (Mamba-2: per group), a 16 x 16 matrix per head (delta rule: two) and the decays over
+    the chunk (Mamba-2: 48 numbers)."""
+    chunks = tokens // 16 + entries + 1
+    return chunks * (vectors * 16 * dim * vector_heads + heads * (256 * (vectors - 1) + (48 if mamba else dim)))
+
+
+def scratch_of_the_state_layers(stub):
+    """What the chunked recurrences keep is what is allocated: Mamba-2's vectors once per group, not per head."""
+    import narurax_cases as N
+    import rofozen_cases as M
+    import tolenex_cases as H
+    for cases, layer, size in ((M, M.mamba_layer(heads=64, vdim=16, state=128, groups=8), (64, 8, 128, 2)),
+                               (M, M.mamba_layer(heads=6, vdim=16, state=64, groups=6), (6, 6, 64, 2)),
+                               (N, N.delta_layer(heads=8, kv_heads=2, dim=128, vdim=64), (8, 8, 128, 3)),
+                               (H, H.hgrn2_layer(heads=4, dim=192, vdim=32), (4, 4, 192, 2))):
+        s = engine(cases.make_config([layer]), cases, max_tokens=2048, max_sequences=4)
+        stub.forget()
+        step(s, 'a', 2000)
+        assert any('chunk_walk_kernel' in k for k in stub.kernels())
+        heads, vector_heads, dim, vectors = size
+        floats = chunk_floats(2000, 4, heads, vector_heads, dim, vectors, mamba=cases is M)
+        assert stub.has_allocation(4 * floats), (layer, 4 * floats)
+
+
+if __name__ == '__main__':
+    globals()[sys.argv[2]](Stub(sys.argv[1]), *sys.argv[3:])
+    print('ok')
+else:
+    def test_scratch_of_the_state_layers(stub):
+        run(stub, 'scratch_of_the_state_layers')

@@ -45,12 +45,7 @@ __device__ __forceinline__ float ld_el(const void* p, int64_t i)
         return reinterpret_cast<const float*>(p)[i];
 }
 
-enum Mode
-{
-    HGRN = 0,
-    DELTA = 1,
-    SSM = 2
-};
+constexpr int HGRN = CHUNK_HGRN2, DELTA = CHUNK_DELTA, SSM = CHUNK_SSM;
 
 // What the three kinds have in common, filled by the launchers below.
 struct ChunkArgs
@@ -648,34 +643,38 @@ int run(const ChunkArgs& a, hipStream_t stream)
     return launched("stack_chunk");
 }
 
-// carves the scratch; false where it does not hold the step
-bool carve(ChunkArgs& a, int mode, int tokens, float* ws, size_t floats)
+// Lays the scratch of a step out in ws -> the floats it takes (ws null: only that)
+size_t carve(ChunkArgs& a, int mode, int tokens, float* ws)
 {
     a.slots = stack_chunk_slots(tokens, a.entries);
-    const size_t c = a.slots, hd = (size_t) a.heads * a.D;
-    float* at = ws;
+    const size_t c = a.slots, hd = (size_t) a.heads * a.D, vectors = mode == SSM ? (size_t) a.groups * a.D : hd;
+    size_t at = 0;
     auto take = [&](size_t n) {
-        float* p = at;
+        float* p = ws ? ws + at : nullptr;
         at += n;
         return p;
     };
-    a.qt = take(c * (mode == SSM ? (size_t) a.groups * a.D : hd) * R);
+    a.qt = take(c * vectors * R);
     if (mode == DELTA)
         a.kb = take(c * hd * R);
-    a.kt = take(c * (mode == SSM ? (size_t) a.groups * a.D : hd) * R);
+    a.kt = take(c * vectors * R);
     a.pm = take(c * a.heads * R * R);
     if (mode == DELTA)
         a.tm = take(c * a.heads * R * R);
     a.bc = take(c * (mode == SSM ? (size_t) a.heads * 48 : hd));
-    return ws && (size_t) (at - ws) <= floats;
+    return at;
 }
 
 } // namespace
 
-size_t stack_chunk_floats(int32_t tokens, int32_t entries, int32_t heads, int32_t dim, int32_t copies)
+size_t stack_chunk_floats(StackChunkKind kind, int32_t tokens, int32_t entries, int32_t heads, int32_t groups, int32_t dim)
 {
-    // copies: 2 vectors per row and head (HGRN2), 3 (delta rule); Mamba-2's B per group is no more than one per head
-    return (size_t) stack_chunk_slots(tokens, entries) * heads * ((size_t) dim * (R * copies + 1) + 2 * R * R + 48);
+    ChunkArgs a;
+    a.heads = heads;
+    a.groups = groups;
+    a.D = dim;
+    a.entries = entries;
+    return carve(a, kind, tokens, nullptr);
 }
 
 bool stack_chunk_serves(int32_t dim, int32_t max_count)
@@ -701,7 +700,7 @@ int launch_stack_chunk_hgrn2(const StackHgrnParams& p, hipStream_t stream)
     a.ent_first = p.ent_first;
     a.ent_count = p.ent_count;
     a.ent_pos0 = p.ent_pos0;
-    if (!stack_chunk_serves(p.dim, p.max_count) || !carve(a, HGRN, p.tokens, p.chunk_ws, p.chunk_floats))
+    if (!stack_chunk_serves(p.dim, p.max_count) || !p.chunk_ws || carve(a, HGRN, p.tokens, p.chunk_ws) > p.chunk_floats)
         return 1;
     return p.dtype == DT_BF16 ? run<DT_BF16, HGRN>(a, stream) : run<DT_FLOAT, HGRN>(a, stream);
 }
@@ -727,7 +726,7 @@ int launch_stack_chunk_delta(const StackDeltaParams& p, hipStream_t stream)
     a.ent_first = p.ent_first;
     a.ent_count = p.ent_count;
     a.ent_pos0 = p.ent_pos0;
-    if (!stack_chunk_serves(p.dim, p.max_count) || !carve(a, DELTA, p.tokens, p.chunk_ws, p.chunk_floats))
+    if (!stack_chunk_serves(p.dim, p.max_count) || !p.chunk_ws || carve(a, DELTA, p.tokens, p.chunk_ws) > p.chunk_floats)
         return 1;
     return p.dtype == DT_BF16 ? run<DT_BF16, DELTA>(a, stream) : run<DT_FLOAT, DELTA>(a, stream);
 }
@@ -754,7 +753,7 @@ int launch_stack_chunk_ssm(const StackSsmParams& p, hipStream_t stream)
     a.ent_count = p.ent_count;
     a.ent_pos0 = p.ent_pos0;
     // (the heads of a group share a workgroup's LDS in the first launch)
-    if (!stack_chunk_serves(p.state, p.max_count) || p.heads / p.groups > 128 || !carve(a, SSM, p.tokens, p.chunk_ws, p.chunk_floats))
+    if (!stack_chunk_serves(p.state, p.max_count) || p.heads / p.groups > 128 || !p.chunk_ws || carve(a, SSM, p.tokens, p.chunk_ws) > p.chunk_floats)
         return 1;
     return p.dtype == DT_BF16 ? run<DT_BF16, SSM>(a, stream) : run<DT_FLOAT, SSM>(a, stream);
 }

@@ -323,8 +323,14 @@ struct StackHgrnParams
     float* chunk_ws = nullptr;     // optional scratch of the chunked form (stack_chunk_floats); without it rows go one by one
     size_t chunk_floats = 0;
 };
-// floats of scratch that the chunked recurrences want for a step (stack_chunk.hip); copies: 2 HGRN2 and Mamba-2, 3 delta rule
-size_t stack_chunk_floats(int32_t tokens, int32_t entries, int32_t heads, int32_t dim, int32_t copies);
+// floats of scratch that the chunked recurrences want for a step (stack_chunk.hip); groups: Mamba-2's, whose vectors its heads share
+enum StackChunkKind
+{
+    CHUNK_HGRN2 = 0,
+    CHUNK_DELTA = 1,
+    CHUNK_SSM = 2
+};
+size_t stack_chunk_floats(StackChunkKind kind, int32_t tokens, int32_t entries, int32_t heads, int32_t groups, int32_t dim);
 bool stack_chunk_serves(int32_t dim, int32_t max_count); // a state of dim rows, the largest entry of the step
 int launch_stack_hgrn2(const StackHgrnParams& p, hipStream_t stream);
 bool stack_hgrn2_serves(int32_t dim, int32_t vdim); // shapes one of its two forms takes

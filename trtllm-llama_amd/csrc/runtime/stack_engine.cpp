@@ -431,9 +431,9 @@ int ensure_scratch(tllm_stack* s, int tokens, int want, int n_ints)
         HIP_OK(hipMalloc(&s->pairs, T * std::max(s->max_pairs, 1) * es));
         for (const auto& l : s->layers)
         {
-            const int copies = l.kind == MIX_DELTA ? 3 : (l.kind == MIX_HGRN2 || l.kind == MIX_MAMBA2 ? 2 : 0);
-            if (copies && T >= 2 * 16 && stack_chunk_serves(l.dim, (int) T))
-                s->chunk_floats = std::max(s->chunk_floats, stack_chunk_floats((int) T, std::min((int) T, s->slots), l.heads, l.dim, copies));
+            if ((l.kind == MIX_DELTA || l.kind == MIX_HGRN2 || l.kind == MIX_MAMBA2) && stack_chunk_serves(l.dim, (int) T))
+                s->chunk_floats = std::max(s->chunk_floats, stack_chunk_floats(l.kind == MIX_DELTA ? CHUNK_DELTA : l.kind == MIX_HGRN2 ? CHUNK_HGRN2 : CHUNK_SSM,
+                                                                (int) T, std::min((int) T, s->slots), l.heads, l.groups, l.dim));
         }
         if (s->chunk_floats && hipMalloc((void**) &s->chunk_ws, s->chunk_floats * 4) != hipSuccess)
         {
