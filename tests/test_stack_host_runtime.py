@@ -76,9 +76,30 @@ def scratch_of_the_state_layers(stub):
         assert stub.has_allocation(4 * floats), (layer, 4 * floats)
 
 
+def scratch_that_leaves_room(stub):
+    """With the last free bytes short of the state layers' scratch, a step still has its mandatory buffers, and walks row by row."""
+    import narurax_cases as N
+    cfg = N.make_config([N.delta_layer(heads=8, kv_heads=2, dim=128, vdim=64)])
+    s = engine(cfg, N, max_tokens=2048, max_sequences=4)
+    before = stub.live()
+    step(s, 'a', 1024)
+    need, floats = stub.live() - before, chunk_floats(1024, 4, 8, 8, 128, 3)
+    assert any('chunk_walk_kernel' in k for k in stub.kernels())
+    for spare in (floats // 16, 2 * floats, 4 * floats - 4096):
+        s = engine(cfg, N, max_tokens=2048, max_sequences=4)
+        stub.budget(stub.live() + need - 4 * floats + spare)
+        stub.forget()
+        step(s, 'a', 1024)
+        assert stub.kernels() and not any('chunk_walk_kernel' in k for k in stub.kernels())
+        stub.budget(2 ** 64 - 1)
+
+
 if __name__ == '__main__':
     globals()[sys.argv[2]](Stub(sys.argv[1]), *sys.argv[3:])
     print('ok')
 else:
     def test_scratch_of_the_state_layers(stub):
         run(stub, 'scratch_of_the_state_layers')
+
+    def test_a_step_fits_where_only_the_optional_scratch_does_not(stub):
+        run(stub, 'scratch_that_leaves_room')

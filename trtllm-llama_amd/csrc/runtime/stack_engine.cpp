@@ -429,19 +429,6 @@ int ensure_scratch(tllm_stack* s, int tokens, int want, int n_ints)
         HIP_OK(hipMalloc(&s->qfull, T * std::max(s->max_qfull, 1) * es));
         HIP_OK(hipMalloc((void**) &s->h32, (s->token_shift ? T * wd : 1) * 4));
         HIP_OK(hipMalloc(&s->pairs, T * std::max(s->max_pairs, 1) * es));
-        for (const auto& l : s->layers)
-        {
-            if ((l.kind == MIX_DELTA || l.kind == MIX_HGRN2 || l.kind == MIX_MAMBA2) && stack_chunk_serves(l.dim, (int) T))
-                s->chunk_floats = std::max(s->chunk_floats, stack_chunk_floats(l.kind == MIX_DELTA ? CHUNK_DELTA : l.kind == MIX_HGRN2 ? CHUNK_HGRN2 : CHUNK_SSM,
-                                                                (int) T, std::min((int) T, s->slots), l.heads, l.groups, l.dim));
-        }
-        if (s->chunk_floats && hipMalloc((void**) &s->chunk_ws, s->chunk_floats * 4) != hipSuccess)
-        {
-            // no room: such rows go one by one
-            (void) hipGetLastError();
-            s->chunk_ws = nullptr;
-            s->chunk_floats = 0;
-        }
         HIP_OK(hipMalloc((void**) &s->dl_a, T * std::max(s->max_hd, 1) * 4));
         HIP_OK(hipMalloc((void**) &s->dl_g, (s->max_hd ? T * std::max(s->max_ctx, 1) : 1) * 4));
         {
@@ -459,6 +446,17 @@ int ensure_scratch(tllm_stack* s, int tokens, int want, int n_ints)
         HIP_OK(hipHostMalloc((void**) &s->pinned, NI * 4, hipHostMallocDefault));
         if (s->taps)
             HIP_OK(hipMalloc((void**) &s->tap, s->runs.size() * T * wd * 4));
+        // last, since a step does without it: where there is no room for it, its rows go one by one
+        for (const auto& l : s->layers)
+            if ((l.kind == MIX_DELTA || l.kind == MIX_HGRN2 || l.kind == MIX_MAMBA2) && stack_chunk_serves(l.dim, (int) T))
+                s->chunk_floats = std::max(s->chunk_floats, stack_chunk_floats(l.kind == MIX_DELTA ? CHUNK_DELTA : l.kind == MIX_HGRN2 ? CHUNK_HGRN2 : CHUNK_SSM,
+                                                                (int) T, std::min((int) T, s->slots), l.heads, l.groups, l.dim));
+        if (s->chunk_floats && hipMalloc((void**) &s->chunk_ws, s->chunk_floats * 4) != hipSuccess)
+        {
+            (void) hipGetLastError();
+            s->chunk_ws = nullptr;
+            s->chunk_floats = 0;
+        }
         s->cap_tokens = (int) T;
         s->cap_want = (int) W;
         s->cap_ints = (int) NI;
