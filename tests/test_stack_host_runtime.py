@@ -94,6 +94,25 @@ def scratch_that_leaves_room(stub):
         stub.budget(2 ** 64 - 1)
 
 
+def step_behind_one_that_found_no_memory(stub):
+    """A step that fails for want of memory gives its scratch back; a smaller one behind it makes its own."""
+    import narurax_cases as N
+    cfg = N.make_config([N.delta_layer(heads=8, kv_heads=2, dim=128, vdim=64)])
+    s = engine(cfg, N, max_tokens=2048, max_sequences=4)
+    step(s, 'a', 100)
+    stub.budget(stub.live() + (64 << 10))
+    try:
+        step(s, 'b', 1500)
+    except RuntimeError as e:
+        assert 'out of memory' in str(e)
+    else:
+        raise AssertionError('the budget holds the step')
+    stub.budget(2 ** 64 - 1)
+    stub.forget()
+    step(s, 'c', 20)
+    assert stub.kernels()
+
+
 if __name__ == '__main__':
     globals()[sys.argv[2]](Stub(sys.argv[1]), *sys.argv[3:])
     print('ok')
@@ -103,3 +122,6 @@ else:
 
     def test_a_step_fits_where_only_the_optional_scratch_does_not(stub):
         run(stub, 'scratch_that_leaves_room')
+
+    def test_a_step_behind_one_that_found_no_memory(stub):
+        run(stub, 'step_behind_one_that_found_no_memory')

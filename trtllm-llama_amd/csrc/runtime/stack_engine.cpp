@@ -234,6 +234,7 @@ namespace
         const hipError_t e_ = (call);                                                                                               \
         if (e_ != hipSuccess)                                                                                                       \
         {                                                                                                                           \
+            (void) hipGetLastError(); /* reported here: the next launch's check must not find it */                                \
             set_error("stack engine: %s failed: %s", #call, hipGetErrorString(e_));                                               \
             return -1;                                                                                                              \
         }                                                                                                                           \
@@ -401,6 +402,7 @@ int ensure_scratch(tllm_stack* s, int tokens, int want, int n_ints)
         }
         const size_t T = (size_t) std::max(tokens, s->cap_tokens), W = (size_t) std::max(want, s->cap_want);
         const size_t NI = (size_t) std::max(n_ints, s->cap_ints);
+        s->cap_tokens = s->cap_want = s->cap_ints = 0; // (nothing is there until all of it is)
         const size_t es = s->es, wd = s->width;
         HIP_OK(hipMalloc((void**) &s->x, T * wd * 4 * (size_t) s->streams));
         HIP_OK(hipMalloc((void**) &s->y32, T * wd * 4));
