@@ -113,6 +113,28 @@ def step_behind_one_that_found_no_memory(stub):
     assert stub.kernels()
 
 
+def pinned_rows(stub):
+    """Requests come in one by one: the pinned room for wanted rows grows by doubling, up to 8 MiB of logits, and nothing is pinned for rows that
+    go to nobody."""
+    import rofozen_cases as M
+    cfg = M.make_config([M.mamba_layer(heads=2, vdim=8, state=16, groups=1)], vocab=32000)
+    s = engine(cfg, M, max_tokens=2048, max_sequences=4)
+    step(s, 0, 70, 0)  # (the step's scratch and its pinned metadata are made here)
+    lib, none = s.engine._h, stub.host_mallocs()
+    import tensorrt_llm.runtime.stack as stack
+    one, pos, slot, table = (np.array(v, np.int32) for v in ([3], [0], [0], [[0]]))
+    b = stack.Batch(1, 1, 1, 1, one.ctypes.data, (count := np.array([1], np.int32)).ctypes.data, pos.ctypes.data, slot.ctypes.data, table.ctypes.data, pos.ctypes.data)
+    assert stack.load_library().tllm_stack_step(lib, ctypes.byref(b), None, None, None) == 0
+    assert stub.host_mallocs() == none
+    step(s, 1, 70, 70)  # (rows by copy; the scratch for the most rows)
+    scratch = stub.host_mallocs()
+    for n in range(1, 66):
+        logits, ids = step(s, n + 1, 70, n)
+        assert logits.shape == (n, 32000) and 'deliver_kernel' in stub.launched().decode()
+    assert stub.host_mallocs() - scratch == 8  # 1, 2, 4, ... 64 and 65 rows
+    assert stub.pinned_bytes() <= (8 << 20) + 65 * 64 * 8 + (64 << 10)
+
+
 if __name__ == '__main__':
     globals()[sys.argv[2]](Stub(sys.argv[1]), *sys.argv[3:])
     print('ok')
@@ -125,3 +147,6 @@ else:
 
     def test_a_step_behind_one_that_found_no_memory(stub):
         run(stub, 'step_behind_one_that_found_no_memory')
+
+    def test_pinned_rows(stub):
+        run(stub, 'pinned_rows')

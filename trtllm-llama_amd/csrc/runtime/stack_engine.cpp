@@ -374,18 +374,20 @@ bool ensure_landing(tllm_stack* s, int want)
         (void) hipDeviceSynchronize(); // (a step that ended in an error may still be under way)
         (void) hipHostFree(s->land_choice);
     }
+    // (twice the rows at least: as requests come in one by one, few of their steps pin anew)
+    const size_t rows = std::min(kLandBytes / row, std::max((size_t) want, 2 * (size_t) s->land_cap));
     s->land_choice = nullptr;
     s->land_cap = 0;
-    const size_t head = (sizeof(StackChoice) * parts * want + 63) / 64 * 64;
+    const size_t head = (sizeof(StackChoice) * parts * rows + 63) / 64 * 64;
     void* m = nullptr;
-    if (hipHostMalloc(&m, head + row * want, hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc(&m, head + row * rows, hipHostMallocDefault) != hipSuccess)
     {
         (void) hipGetLastError();
         return false;
     }
     s->land_choice = (StackChoice*) m;
     s->land_rows = (float*) ((char*) m + head);
-    s->land_cap = want;
+    s->land_cap = (int) rows;
     return true;
 }
 
@@ -1415,7 +1417,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
     const size_t n_ints = (size_t) 4 * T + (size_t) 4 * E + (size_t) E * MB + NW;
     if (ensure_scratch(s, T, std::max(NW, 1), (int) (n_ints + 3) / 4 * 4))
         return -1;
-    const bool deliver = ensure_landing(s, NW);
+    const bool deliver = (logits_out || next_ids_out) && ensure_landing(s, NW);
     int32_t* h = s->pinned;
     int32_t *h_tok = h, *h_tent = h + T, *h_tpos = h + 2 * T, *h_first = h + 3 * T, *h_count = h_first + E, *h_pos0 = h_count + E,
             *h_slot = h_pos0 + E, *h_table = h_slot + E, *h_want = h_table + (size_t) E * MB, *h_prev = h_want + NW;
