@@ -135,6 +135,20 @@ def pinned_rows(stub):
     assert stub.pinned_bytes() <= (8 << 20) + 65 * 64 * 8 + (64 << 10)
 
 
+def huge_step(stub):
+    """One prompt of 131072 tokens beside 300 decoded ones, 64 heads: tiles x entries x heads of one launch are more than a grid's x dimension takes."""
+    import ruzinex_cases as Z
+    cfg = Z.make_config([Z.layer(heads=64, kv_heads=8, dim=64, vdim=64, rot_dims=32)], width=64)
+    s = engine(cfg, Z, max_tokens=160000, max_sequences=301)
+    for i in range(300):
+        s.step([(i, [1], [0])])
+    stub.forget()
+    s.step([('long', [1] * 131072, [0])] + [(i, [1], [0]) for i in range(300)])
+    assert any('attn_prefill_kernel' in k for k in stub.kernels())
+    s.step([('long', [1] * 40, [0])] + [(i, [1], [0]) for i in range(300)])
+    assert any('attn_prompt_kernel' in k for k in stub.kernels())
+
+
 if __name__ == '__main__':
     globals()[sys.argv[2]](Stub(sys.argv[1]), *sys.argv[3:])
     print('ok')
@@ -150,3 +164,6 @@ else:
 
     def test_pinned_rows(stub):
         run(stub, 'pinned_rows')
+
+    def test_a_step_with_more_tiles_than_a_grid_dimension(stub):
+        run(stub, 'huge_step')

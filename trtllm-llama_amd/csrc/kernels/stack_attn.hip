@@ -671,8 +671,8 @@ __global__ __launch_bounds__(256, DK >= 10 ? 1 : 2) void attn_prefill_kernel(con
     }
 }
 
-// The same two over the lanes 16, 32 and 48 further on without the LDS crossbar: a half's and a row's values change places (v_permlane32_swap,
-// v_permlane16_swap: the two results together hold both partners' values)
+// the largest of a value over the lanes 16, 32 and 48 further on, without the LDS crossbar: a half's and a row's values change places
+// (v_permlane32_swap, v_permlane16_swap: the two results together hold both partners' values)
 __device__ __forceinline__ float rows_max_swap(float v)
 {
     const uint32_t u = __builtin_bit_cast(uint32_t, v);
@@ -1323,13 +1323,14 @@ int launch_tile(const StackAttnParams& p, hipStream_t stream)
                 hipLaunchKernelGGL((attn_prefill_wide_kernel<DK, VT>), pg, dim3(256), 0, stream, p, PREFILL_ROWS);
             }
         }
-        // heads of the usual sizes over pages of whole 64-key units (16-byte DMA from both pools)
+        // heads of the usual sizes over pages of whole 64-key units (16-byte DMA from both pools); its grid is one-dimensional, and a grid
+        // dimension holds fewer than 2^32 threads
         constexpr bool prompt_form = (DK == 2 || DK == 4 || (DK == 6 && MAPS == 1)) && (VT == 4 || VT == 8);
         bool prompt = false;
         if constexpr (prompt_form)
         {
             prompt = p.page % 64 == 0 && !(reinterpret_cast<uintptr_t>(p.v_pool) & 15) && !wide
-                && (int64_t) ((p.max_count + 63) / 64) * p.entries * p.heads < (1 << 30);
+                && (int64_t) ((p.max_count + 63) / 64) * p.entries * p.heads < (1 << 24);
             if (prompt)
             {
                 // two row tiles per wave where such workgroups still make two per CU; waves that share a unit's keys where workgroups of 64 rows
