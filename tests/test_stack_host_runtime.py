@@ -149,6 +149,15 @@ def huge_step(stub):
     assert any('attn_prompt_kernel' in k for k in stub.kernels())
 
 
+def many_small_rows(stub):
+    """More wanted rows of a small vocabulary than a grid has in y."""
+    import rofozen_cases as M
+    cfg = M.make_config([M.mamba_layer(heads=2, vdim=8, state=16, groups=1)], vocab=16, width=32)
+    s = engine(cfg, M, max_tokens=80000, max_sequences=1)
+    logits, ids = step(s, 'a', 70000, 70000)
+    assert logits.shape == (70000, 16) and ids.shape == (70000,)
+
+
 if __name__ == '__main__':
     globals()[sys.argv[2]](Stub(sys.argv[1]), *sys.argv[3:])
     print('ok')
@@ -167,3 +176,6 @@ else:
 
     def test_a_step_with_more_tiles_than_a_grid_dimension(stub):
         run(stub, 'huge_step')
+
+    def test_more_wanted_rows_than_a_grid_dimension(stub):
+        run(stub, 'many_small_rows')

@@ -365,7 +365,7 @@ constexpr size_t kLandBytes = 8 << 20;
 bool ensure_landing(tllm_stack* s, int want)
 {
     const size_t row = (size_t) s->vocab * 4, parts = (size_t) stack_choice_parts(s->vocab);
-    if (want < 1 || row * want > kLandBytes)
+    if (want < 1 || row * want > kLandBytes || want > 65535) // (a row is a workgroup row of the launch)
         return false;
     if (want <= s->land_cap)
         return true;
