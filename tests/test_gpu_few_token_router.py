@@ -40,3 +40,12 @@ def test_prompt_router(width, router, n):
     toks = tokens_for(cfg, n, 8)
     got = replay(session_for(cfg, w, 'float32'), {'a': toks}, [[('a', n)]])['a']
     check(got, O.logits(toks, as_f64(w), cfg), tol_of('float32'), 'a')
+
+
+def test_the_most_outputs_and_tokens_of_one_launch():
+    """1024 outputs, 8 tokens: scores and choice values are 64 KiB of LDS, and the launch's ticket comes on top."""
+    cfg = make_config([mamba_layer(mlp=moe(experts=1000, identity=24, top=3, count=1, keep=1, ff=8))], width=64)
+    w = random_weights(cfg, 9)
+    toks = tokens_for(cfg, 16, 10)
+    got = replay(session_for(cfg, w, 'float32'), {'a': toks}, [[('a', 8)], [('a', 7)], [('a', 1)]])['a']
+    check(got, O.logits(toks, as_f64(w), cfg), tol_of('float32'), 'a')

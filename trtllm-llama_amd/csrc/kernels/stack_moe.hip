@@ -1,6 +1,7 @@
 // Routed mixture of experts of the ragged-batch stack engine (stack_kernels.h): the fp32 router with its grouped top-k choice,
 // the ordering of (token, chosen expert) pairs by expert for the grouped products, and the weighted sum of the experts' outputs.
 #include "dev_utils.h"
+#include "launch_util.h"
 #include "stack_kernels.h"
 #include <algorithm>
 
@@ -854,6 +855,9 @@ int launch_stack_moe_plan(const StackMoeParams& p, hipStream_t stream)
     else
     {
         const dim3 grid((p.experts + p.identity + 7) / 8);
+        // (eight tokens of 1024 outputs take all of the default 64 KiB, and the kernel's ticket stands beside them)
+        const void* fn = p.dtype == DT_BF16 ? reinterpret_cast<const void*>(&moe_route_few_kernel<DT_BF16>) : reinterpret_cast<const void*>(&moe_route_few_kernel<DT_FLOAT>);
+        launch_util::ensure_dynamic_lds(fn, lds + sizeof(uint32_t));
         if (p.dtype == DT_BF16)
             hipLaunchKernelGGL((moe_route_few_kernel<DT_BF16>), grid, dim3(512), lds, stream, p, row_bytes);
         else
