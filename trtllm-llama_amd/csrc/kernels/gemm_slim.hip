@@ -1,5 +1,7 @@
-// Products of 9 .. 31 rows on the LLaMA path (short prompts): fp16, SmoothQuant int8, weight-only int8 / int4 weights through the
-// weight-streaming main loop of gemm_slim_impl.h.  The epilogue has the rounding points of the tiles in gemm_mfma.hip.
+// Products of few rows on the LLaMA path: fp16, SmoothQuant int8, weight-only int8 / int4 weights through the weight-streaming main loop of
+// gemm_slim_impl.h.  Short prompts and plain calls of 5 .. 31 rows (int4 weights 3 .. 31), generation steps of 5 .. 32 sequences with fp16 or
+// weight-only weights (int4 3 .. 32).  The epilogue has the rounding points of the tiles in gemm_mfma.hip.  The sums' order is not the
+// streaming GEMV's, which serves fewer rows: a sequence's fp16 rows differ in their last bits with the number of rows beside it.
 #include "gemm_slim_impl.h"
 #include "kernels.h"
 #include "launch_util.h"
@@ -104,26 +106,32 @@ int gemm_slim_rows(int wtype)
     return wtype == W_INT4_WOQ ? 3 : 5;
 }
 
-// 0: launched, -1: launch error, 1: not served (row counts, alignment).  residual and silu_gate share c's rows; c may be the residual itself
-int launch_gemm_slim(const GemmParams& p, hipStream_t stream)
+bool gemm_slim_serves(const GemmParams& p)
 {
+    if (p.wtype != W_FP16 && p.wtype != W_INT8_SQ && p.wtype != W_INT8_WOQ && p.wtype != W_INT4_WOQ)
+        return false;
     const int a_es = p.wtype == W_INT8_SQ ? 1 : 2;
     if (p.M < 1 || p.M > 32 || p.N < 1 || p.K < 1 || ((p.residual || p.silu_gate) && p.out_dtype != DT_HALF))
-        return 1;
+        return false;
     // 16-byte loads of both operands; 32-bit offsets of a workgroup's W rows
     if ((reinterpret_cast<uintptr_t>(p.a) & 15) || ((p.lda * a_es) & 15) || (reinterpret_cast<uintptr_t>(p.w) & 15) || (p.ldw & 15) || p.ldw > (1 << 26))
-        return 1;
+        return false;
     if ((p.K * a_es) % 16 || (p.wtype == W_INT8_WOQ && p.K % 16) || (p.wtype == W_INT4_WOQ && p.K % 32))
-        return 1;
-    if (p.out_dtype != DT_HALF && p.out_dtype != DT_FLOAT && !(p.out_dtype == DT_INT32 && p.wtype == W_INT8_SQ))
+        return false;
+    return p.out_dtype == DT_HALF || p.out_dtype == DT_FLOAT || (p.out_dtype == DT_INT32 && p.wtype == W_INT8_SQ);
+}
+
+// 0: launched, -1: launch error, 1: not served.  residual and silu_gate share c's rows; c may be the residual itself
+int launch_gemm_slim(const GemmParams& p, hipStream_t stream)
+{
+    if (!gemm_slim_serves(p))
         return 1;
     switch (p.wtype)
     {
     case W_FP16: return launch_wt<W_FP16>(p, stream);
     case W_INT8_SQ: return launch_wt<W_INT8_SQ>(p, stream);
     case W_INT8_WOQ: return launch_wt<W_INT8_WOQ>(p, stream);
-    case W_INT4_WOQ: return launch_wt<W_INT4_WOQ>(p, stream);
-    default: return 1;
+    default: return launch_wt<W_INT4_WOQ>(p, stream);
     }
 }
 

@@ -407,9 +407,10 @@ struct GemmParams
     void* ksplit_ws = nullptr;
 };
 int launch_gemm(const GemmParams& p, hipStream_t stream);
-// gemm_slim.hip: up to 32 rows of any weight type, residual (which may be c) or silu_gate in the epilogue; 1: a shape it does not serve.
-// gemm_slim_rows: the rows from which it is quicker than launch_gemv
+// gemm_slim.hip: up to 32 rows of any weight type, residual (which may be c) or silu_gate in the epilogue; 1: a call that gemm_slim_serves
+// says no to.  gemm_slim_rows: the rows from which it is quicker than launch_gemv
 int launch_gemm_slim(const GemmParams& p, hipStream_t stream);
+bool gemm_slim_serves(const GemmParams& p);
 int gemm_slim_rows(int wtype);
 // fc and gate projections of the SmoothQuant MLP in one kernel with SwiGLU + static int8 quantisation in its epilogue
 // (gemm_sqp.hip); returns 1 when the problem is not served (caller runs the two GEMMs + launch_swiglu_quant instead)

@@ -432,14 +432,18 @@ struct tllm_session
 
     // ------------------------------------------------------------------------------------------ GEMM wrappers
     // decode of several sequences with fp16 or weight-only weights: the norm, then the weight-streaming MFMA product (one pass over the
-    // weights for up to 32 rows) with the residual or the SwiGLU in its epilogue.  (The head stays with
-    // launch_gemv: a sequence's fp32 logits are the same bits alone and in a batch.)  -> whether this form serves the call (rc: its status)
+    // weights for up to 32 rows) with the residual or the SwiGLU in its epilogue.  The layers' sums then run in another order than with
+    // fewer sequences (launch_gemv); the head stays with launch_gemv, whose sum for a row does not depend on how many there are.
+    // -> whether this form serves the call (rc: its status)
     bool few_rows(const Linear& L, int M, int pro, int epi, const void* xin, int64_t ldx, const void* gamma, const void* residual, void* y,
         int64_t ldy, int out_dtype, const Linear* up, hipStream_t st, int& rc)
     {
         const bool norm = pro == PRO_RMSNORM, swiglu = epi == EPI_SWIGLU;
-        if ((pro != PRO_NONE && !norm) || (epi != EPI_NONE && epi != EPI_RESIDUAL && !swiglu) || out_dtype != DT_HALF
-            || (swiglu && (!up || up->wtype != L.wtype || up->N != L.N || up->K != L.K || L.N > Ir || ldy != L.N || (reinterpret_cast<uintptr_t>(up->w) & 15) || (up->ldw & 15))) || (norm && (L.K != hidden || ldx != hidden || xin == tmp || !tmp)))
+        if ((pro != PRO_NONE && !norm) || (epi != EPI_NONE && epi != EPI_RESIDUAL && !swiglu) || out_dtype != DT_HALF || L.K % 32)
+            return false;
+        if (norm && (L.K != hidden || ldx != hidden || xin == tmp || !tmp))
+            return false;
+        if (swiglu && (!up || up->wtype != L.wtype || up->N != L.N || up->K != L.K || L.N > Ir || ldy != L.N))
             return false;
         GemmParams g;
         g.wtype = L.wtype;
@@ -457,8 +461,19 @@ struct tllm_session
         g.c = swiglu ? this->g : y;
         g.ldc = swiglu ? (int64_t) L.N : ldy;
         g.residual = epi == EPI_RESIDUAL ? residual : nullptr;
-        // the products refuse a shape before they launch, but the norm is ahead of them: what decides is asked here
-        if ((g.lda * 2) % 16 || (reinterpret_cast<uintptr_t>(g.a) & 15) || (reinterpret_cast<uintptr_t>(g.w) & 15) || (g.ldw & 15) || L.K % 32)
+        GemmParams q = g; // the other half of a SwiGLU
+        if (swiglu)
+        {
+            q.w = up->w;
+            q.ldw = up->ldw;
+            q.scale_col = up->scale_col;
+            q.scale_row = up->act_scale;
+            q.per_channel = up->per_channel;
+            q.c = y;
+            q.ldc = ldy;
+            q.silu_gate = this->g;
+        }
+        if (!gemm_slim_serves(g) || !gemm_slim_serves(q)) // (asked ahead of the norm)
             return false;
         rc = timed(gemv_cls, st, [&] {
             if (norm)
@@ -472,20 +487,7 @@ struct tllm_session
                 r.y = tmp;
                 RUN(launch_rmsnorm(r, st));
             }
-            if (launch_gemm_slim(g, st))
-                return 1;
-            if (!swiglu)
-                return 0;
-            GemmParams q = g;
-            q.w = up->w;
-            q.ldw = up->ldw;
-            q.scale_col = up->scale_col;
-            q.scale_row = up->act_scale;
-            q.per_channel = up->per_channel;
-            q.c = y;
-            q.ldc = ldy;
-            q.silu_gate = this->g;
-            return launch_gemm_slim(q, st) ? 1 : 0;
+            return launch_gemm_slim(g, st) || (swiglu && launch_gemm_slim(q, st)) ? 1 : 0;
         });
         return true;
     }
@@ -567,8 +569,8 @@ struct tllm_session
     }
 
     // context: plain GEMM on M rows (activation already in the operand type)
-    int gemm(const Linear& L, int M, const void* a, const float* scale_row, int per_tok, void* c, int out_dtype,
-        hipStream_t st, const void* residual = nullptr, const void* silu_gate = nullptr)
+    static GemmParams gemm_params(const Linear& L, int M, const void* a, const float* scale_row, int per_tok, void* c, int out_dtype,
+        const void* residual = nullptr, const void* silu_gate = nullptr)
     {
         GemmParams g;
         g.residual = residual;
@@ -588,9 +590,22 @@ struct tllm_session
         g.per_token = per_tok;
         g.c = c;
         g.ldc = L.N;
-        if (residual && M < 32) // in place: launch_gemm leaves that to the kernels of many rows
-            return launch_gemm_slim(g, st) ? 1 : 0;
-        return launch_gemm(g, st) ? 1 : 0;
+        return g;
+    }
+    int gemm(const Linear& L, int M, const void* a, const float* scale_row, int per_tok, void* c, int out_dtype,
+        hipStream_t st, const void* residual = nullptr, const void* silu_gate = nullptr)
+    {
+        return launch_gemm(gemm_params(L, M, a, scale_row, per_tok, c, out_dtype, residual, silu_gate), st) ? 1 : 0;
+    }
+    // x += the product of few rows, in place (launch_gemm leaves that to the kernels of many rows)
+    bool adds_few_rows(const Linear& L, int M, const void* a) const
+    {
+        return M < 32 && M >= gemm_slim_rows(L.wtype) && L.K % 32 == 0 && gemm_slim_serves(gemm_params(L, M, a, nullptr, 0, x, DT_HALF, x));
+    }
+    int gemm_add(const Linear& L, int M, const void* a, const float* scale_row, int per_tok, hipStream_t st)
+    {
+        const GemmParams g = gemm_params(L, M, a, scale_row, per_tok, x, DT_HALF, x);
+        return (M < 32 ? launch_gemm_slim(g, st) : launch_gemm(g, st)) ? 1 : 0;
     }
 
     // On-device tactic selection (kernels/gemm_tactics.hip; reference: int8_gemm_template.h:372-457, stored per M bucket in the
@@ -733,9 +748,8 @@ struct tllm_session
             }
             // (weight-only: gemm_woq.hip adds the residual in its epilogue too - same two roundings; its own serve conditions)
             const bool woq_w = L.dense.wtype == W_INT8_WOQ || L.dense.wtype == W_INT4_WOQ;
-            // (short prompts: gemm_slim.hip serves rows of whole 32-value pieces, in place)
-            const bool few_res = M < 32 && M >= gemm_slim_rows(L.dense.wtype) && L.dense.wtype == L.proj.wtype && L.dense.K % 32 == 0
-                && L.proj.K % 32 == 0 && !(L.dense.ldw & 15) && !(L.proj.ldw & 15);
+            // (short prompts: both products in place, or neither)
+            const bool few_res = adds_few_rows(L.dense, M, d_in) && adds_few_rows(L.proj, M, sq ? q8 : inter_buf);
             const bool fuse_res = tp == 1 && !force_comm && (few_res || (M >= 32 && D % 8 == 0))
                 && (few_res ? true : woq_w ? (L.dense.K % 64 == 0 && L.proj.K % 64 == 0)
                           : ((L.dense.wtype == W_INT8_SQ || L.dense.wtype == W_FP16)
@@ -744,7 +758,7 @@ struct tllm_session
             if (fuse_res)
             {
                 // x <- x + O(ctx): residual fused into the GEMM epilogue (same rounding: fp16(gemm) then fp16(sum))
-                RUN(gemm(L.dense, M, d_in, sq && per_token ? qscale : nullptr, sq && per_token, x, DT_HALF, st, x));
+                RUN(gemm_add(L.dense, M, d_in, sq && per_token ? qscale : nullptr, sq && per_token, st));
             }
             else
             {
@@ -839,7 +853,7 @@ struct tllm_session
             }
             if (fuse_res)
             {
-                RUN(gemm(L.proj, M, p_in, sq && per_token ? qscale : nullptr, sq && per_token, x, DT_HALF, st, x));
+                RUN(gemm_add(L.proj, M, p_in, sq && per_token ? qscale : nullptr, sq && per_token, st));
             }
             else
             {
