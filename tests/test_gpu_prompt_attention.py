@@ -89,3 +89,34 @@ def test_many_workgroups(kind, steps):
 @pytest.mark.parametrize('kind', sorted(KINDS))
 def test_pages_of_other_sizes(kind, page):
     run(kind, 4, 2, 64, 64, SCHEDULES['portions'], page)
+
+
+@pytest.mark.parametrize('heads,steps', [(4, [[('a', 193)]]), (64, [[('a', 260)]]), (64, [[('b', 390), ('a', 130)]])], ids=['few', 'more', 'many'])
+@pytest.mark.parametrize('where', [40, 100])
+@pytest.mark.parametrize('kind', sorted(KINDS))
+def test_a_row_without_finite_numbers_reaches_no_row_that_does_not_see_it(kind, heads, steps, where):
+    """Row `where` of a request is NaN in every channel.  The rows before it, and with a window the ones that have left it behind, are what they
+    are with another token in its place."""
+    mod, cfg = KINDS[kind](heads, heads // 4 if heads == 64 else 2, 64, 64)
+    toks, other = mod.tokens_for(cfg, sum(k for step in steps for rid, k in step if rid == 'a'), 3), mod.tokens_for(cfg, 390, 4)
+    bad = next(t for t in range(cfg['vocab']) if t not in toks and t not in other)
+    w = mod.random_weights(cfg, 13)
+    finite = dict(w, embed=w['embed'].copy())
+    w['embed'][bad] = np.nan
+    toks[where] = bad
+    reqs = {'a': toks, 'b': other}
+    got = mod.replay(mod.session_for(cfg, w, 'bfloat16', max_tokens=2048), {r: reqs[r] for step in steps for r, _ in step}, steps)
+    assert not np.isfinite(got['a'][where]).any()
+    for rid, rows in got.items():
+        sees = np.zeros(len(rows), bool)
+        if rid == 'a':
+            sees[where:where + 70 if kind == 'window' else None] = True
+        if mod is test_gpu_vetipel:
+            want = mod.O.logits(reqs[rid], as_f64(finite), cfg)
+            mod.check(rows[~sees], want[~sees], mod.tol_of('bfloat16'), rid)
+        else:
+            n = int((~sees).sum())
+            assert not sees[:n].any()
+            if kind == 'ruzinex':  # (its head is its embedding: the bad token's own column is NaN in every row)
+                rows[:n, bad] = mod.O.logits(reqs[rid][:n], as_f64(finite), cfg)[:, bad]
+            mod.check_rows(rows[:n], reqs[rid][:n], finite, cfg, 'bfloat16', rid)

@@ -14,6 +14,7 @@
 #include "stack_kernels.h"
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 namespace tllm
 {
@@ -776,6 +777,31 @@ __device__ __forceinline__ void softmax_unit(f32x4 (&s)[NN], float& m_run, float
             pack_bf16(s[2 * b + 1][2], s[2 * b + 1][3]));
 }
 
+// the bfloat16 infinities and NaNs of x leave it as zeros -> 1.0 in their places
+__device__ __forceinline__ uint4 take_specials(uint4& x)
+{
+    uint32_t v[4] = {x.x, x.y, x.z, x.w}, o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+    {
+        const uint32_t top = ((v[i] & 0x7fff7fffu) + 0x00800080u) >> 15 & 0x00010001u; // an exponent of ones carries into the sign's place
+        v[i] &= ~(top * 0xffffu);
+        o[i] = top * 0x3f80u;
+    }
+    x = make_uint4(v[0], v[1], v[2], v[3]);
+    return make_uint4(o[0], o[1], o[2], o[3]);
+}
+// 1.0 where a bfloat16 of x is not zero
+__device__ __forceinline__ uint4 ones_where(const uint4& x)
+{
+    const uint32_t v[4] = {x.x, x.y, x.z, x.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        o[i] = (v[i] & 0x7fffu ? 0x3f80u : 0u) | (v[i] & 0x7fff0000u ? 0x3f800000u : 0u);
+    return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
 // attn_prompt_kernel: prompts, heads of 64 / 128 / 192 query and 64 / 128 value dimensions, pages of a multiple of 64 keys.  The products of
 // attn_prefill_kernel, with what bounded it taken out (2 us per 32-key block and workgroup, of which the products are 0.1 and the softmax 0.2: the
 // staging through registers, two barriers and the shuffles of one block stood one after another):
@@ -837,11 +863,6 @@ __global__ __launch_bounds__(256 * KS, 2 / KS) void attn_prompt_kernel(const Sta
             for (int ks = 0; ks < DK; ++ks)
                 qf[rt][m][ks] = as_bf16x8(*reinterpret_cast<const uint4*>(
                     reinterpret_cast<const uint16_t*>(p.q) + (((int64_t) (first + qrow) * hd.q_heads + hd.qh) * MAPS + m) * D + ks * 32 + 8 * g4));
-            m_run[rt][m] = -INFINITY;
-            l_run[rt][m] = 0.f;
-#pragma unroll
-            for (int ct = 0; ct < VT; ++ct)
-                acc[rt][m][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
         const int last = r0[rt] + 15 < count ? r0[rt] + 15 : count - 1;
         my_last[rt] = rows_ok ? (pos0 + last) / 64 : -1; // the tile's last unit that holds a visible key, and its first
@@ -884,77 +905,131 @@ __global__ __launch_bounds__(256 * KS, 2 / KS) void attn_prompt_kernel(const Sta
     };
     auto block_of = [&](int u) { return __builtin_amdgcn_readfirstlane(table[upp == 1 ? u : u / upp]); };
 
-    request(unit_at(0), block_of(unit_at(0)), 0);
-    int blk_next = n_units > 1 ? block_of(unit_at(1)) : 0;
-    for (int v = 0; v < n_units; ++v)
-    {
-        const int u = unit_at(v);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads(); // the unit has landed for every wave, and every wave is through with the one before it
-        if (v + 1 < n_units)
-        {
-            request(unit_at(v + 1), blk_next, (v + 1) & 1);
-            if (v + 2 < n_units)
-                blk_next = block_of(unit_at(v + 2));
-        }
-        bool on[RT], any = false; // wave-uniform
+    // CAREFUL: a value that is no finite number meets only the rows that see its key (a weight of 0 times it would make it everyone's)
+    auto walk = [&](auto careful) {
+        constexpr bool CAREFUL = decltype(careful)::value;
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
-        {
-            on[rt] = u <= my_last[rt] && (u >= my_lo[rt] || u < keep_u);
-            any = any || on[rt];
-        }
-        if (!any)
-            continue;
-        const char* ks_ = smem + (v & 1) * BUF;
-        const char* vs_ = ks_ + KB;
-        const int key0 = u * 64 + (KS == 2 ? half * 32 : 0);
-        uint4 pf[RT][MAPS][NN / 2];
 #pragma unroll
-        for (int m = 0; m < MAPS; ++m)
-        {
-            f32x4 s[RT][NN];
-#pragma unroll
-            for (int n = 0; n < NN; ++n)
+            for (int m = 0; m < MAPS; ++m)
             {
-                const int r = 32 * (KS == 2 ? half : n >> 1) + 8 * (col >> 2) + 4 * (n & 1) + (col & 3);
-                const int x = KPR % 16 == 0 ? ((r >> 3) & 3) << 2 | (r & 3) : ((r >> 3) & 3) << 1 | ((r >> 1) & 1);
+                m_run[rt][m] = -INFINITY;
+                l_run[rt][m] = 0.f;
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt)
-                    s[rt][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int ks = 0; ks < DK; ++ks)
-                {
-                    const bf16x8 kf = as_bf16x8(*reinterpret_cast<const uint4*>(ks_ + (m * 64 + r) * (D * 2) + (((ks * 4 + g4) ^ x) << 4)));
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) // (no branches among the products: a tile that is off has its scores dropped below)
-                        s[rt][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[rt][m][ks], s[rt][n], 0, 0, 0);
-                }
+                for (int ct = 0; ct < VT; ++ct)
+                    acc[rt][m][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
+        request(unit_at(0), block_of(unit_at(0)), 0);
+        int blk_next = n_units > 1 ? block_of(unit_at(1)) : 0;
+        for (int v = 0; v < n_units; ++v)
+        {
+            const int u = unit_at(v);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads(); // the unit has landed for every wave, and every wave is through with the one before it
+            if (v + 1 < n_units)
+            {
+                request(unit_at(v + 1), blk_next, (v + 1) & 1);
+                if (v + 2 < n_units)
+                    blk_next = block_of(unit_at(v + 2));
+            }
+            bool on[RT], any = false; // wave-uniform
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt)
             {
-                pf[rt][m][0] = pf[rt][m][NN / 2 - 1] = make_uint4(0, 0, 0, 0);
-                if (RT == 1 || on[rt])
-                {
-                    const bool masked = key0 + 16 * NN - 1 > pos0 + r0[rt] || key0 < klo_last[rt];
-                    softmax_unit<VT, NN>(s[rt], m_run[rt][m], l_run[rt][m], acc[rt][m], pf[rt][m], hm, plain, masked, key0 + 8 * g4, qpos[rt], klo[rt]);
-                }
+                on[rt] = u <= my_last[rt] && (u >= my_lo[rt] || u < keep_u);
+                any = any || on[rt];
             }
-        }
+            if (!any)
+                continue;
+            const char* ks_ = smem + (v & 1) * BUF;
+            const char* vs_ = ks_ + KB;
+            const int key0 = u * 64 + (KS == 2 ? half * 32 : 0);
+            uint4 pf[RT][MAPS][NN / 2];
 #pragma unroll
-        for (int ct = 0; ct < VT; ++ct)
-#pragma unroll
-            for (int b = 0; b < NN / 2; ++b)
+            for (int m = 0; m < MAPS; ++m)
             {
-                const int row = ct * 16 + col;
-                const bf16x8 vf = as_bf16x8(*reinterpret_cast<const uint4*>(vs_ + row * 128 + ((((KS == 2 ? half : b) * 4 + g4) ^ ((row >> 1) & 7)) << 4)));
+                f32x4 s[RT][NN];
+#pragma unroll
+                for (int n = 0; n < NN; ++n)
+                {
+                    const int r = 32 * (KS == 2 ? half : n >> 1) + 8 * (col >> 2) + 4 * (n & 1) + (col & 3);
+                    const int x = KPR % 16 == 0 ? ((r >> 3) & 3) << 2 | (r & 3) : ((r >> 3) & 3) << 1 | ((r >> 1) & 1);
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt)
+                        s[rt][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int ks = 0; ks < DK; ++ks)
+                    {
+                        const bf16x8 kf = as_bf16x8(*reinterpret_cast<const uint4*>(ks_ + (m * 64 + r) * (D * 2) + (((ks * 4 + g4) ^ x) << 4)));
+#pragma unroll
+                        for (int rt = 0; rt < RT; ++rt) // (no branches among the products: a tile that is off has its scores dropped below)
+                            s[rt][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[rt][m][ks], s[rt][n], 0, 0, 0);
+                    }
+                }
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                    for (int m = 0; m < MAPS; ++m)
-                        acc[rt][m][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, as_bf16x8(pf[rt][m][b]), acc[rt][m][ct], 0, 0, 0);
+                {
+                    pf[rt][m][0] = pf[rt][m][NN / 2 - 1] = make_uint4(0, 0, 0, 0);
+                    if (RT == 1 || on[rt])
+                    {
+                        const bool masked = key0 + 16 * NN - 1 > pos0 + r0[rt] || key0 < klo_last[rt];
+                        softmax_unit<VT, NN>(s[rt], m_run[rt][m], l_run[rt][m], acc[rt][m], pf[rt][m], hm, plain, masked, key0 + 8 * g4, qpos[rt], klo[rt]);
+                    }
+                }
             }
+#pragma unroll
+            for (int ct = 0; ct < VT; ++ct)
+#pragma unroll
+                for (int b = 0; b < NN / 2; ++b)
+                {
+                    const int row = ct * 16 + col;
+                    uint4 vr = *reinterpret_cast<const uint4*>(vs_ + row * 128 + ((((KS == 2 ? half : b) * 4 + g4) ^ ((row >> 1) & 7)) << 4));
+                    uint4 vbad = make_uint4(0, 0, 0, 0);
+                    if constexpr (CAREFUL)
+                        vbad = take_specials(vr);
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                        for (int m = 0; m < MAPS; ++m)
+                        {
+                            acc[rt][m][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vr), as_bf16x8(pf[rt][m][b]), acc[rt][m][ct], 0, 0, 0);
+                            if constexpr (CAREFUL)
+                            {
+                                const f32x4 n = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vbad), as_bf16x8(ones_where(pf[rt][m][b])), f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                                for (int i = 0; i < 4; ++i)
+                                    acc[rt][m][ct][i] = n[i] > 0.f ? __builtin_nanf("") : acc[rt][m][ct][i];
+                            }
+                        }
+                }
+        }
+    };
+    walk(std::false_type());
+    {
+        // A row that is not finite, in any wave: once more, carefully.  (Asked once, behind the last unit.)
+        bool finite = true;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int m = 0; m < MAPS; ++m)
+#pragma unroll
+                for (int ct = 0; ct < VT; ++ct)
+                    finite = finite && (fabsf(acc[rt][m][ct][0]) + fabsf(acc[rt][m][ct][1])) + (fabsf(acc[rt][m][ct][2]) + fabsf(acc[rt][m][ct][3])) < INFINITY;
+        int* flags = reinterpret_cast<int*>(smem);
+        const bool mine = __builtin_amdgcn_ballot_w64(!finite) != 0;
+        __syncthreads(); // (the waves are through with the last unit)
+        if (lane == 0)
+            flags[w] = mine ? 1 : 0;
+        __syncthreads();
+        int any = 0;
+#pragma unroll
+        for (int i = 0; i < NW; ++i)
+            any |= flags[i];
+        if (__builtin_amdgcn_readfirstlane(any))
+        {
+            __syncthreads(); // (the flags' place is the first unit's)
+            walk(std::true_type());
+        }
     }
     if constexpr (KS == 2)
     {
