@@ -85,6 +85,13 @@ def test_many_workgroups(kind, steps):
     run(kind, 64, 16, 64, 64, steps)
 
 
+@pytest.mark.parametrize('steps', [[[('a', 260)]], [[('a', 390), ('b', 130)], [('b', 390), ('a', 65)]]], ids=['more', 'many'])
+@pytest.mark.parametrize('kind,dim,vdim', [('ruzinex', 128, 128), ('kept', 128, 64), ('ruzinex', 192, 128), ('kept', 192, 64), ('window', 64, 128), ('tolenex', 128, 128)])
+def test_many_workgroups_of_wider_heads(kind, dim, vdim, steps):
+    """The same with heads of 128 and 192 query and 64 and 128 value dimensions."""
+    run(kind, 64, 16, dim, vdim, steps)
+
+
 @pytest.mark.parametrize('page', [32, 128])
 @pytest.mark.parametrize('kind', sorted(KINDS))
 def test_pages_of_other_sizes(kind, page):

@@ -247,8 +247,8 @@ def test_both_prompt_forms_of_wide_keys(wide, monkeypatch):
 @pytest.mark.parametrize('mlp', [dense(ff=3000), dense(ff=6000), dense(ff=8000), moe(experts=2, top=2, ff=1536, shared=3000), moe(experts=3, top=3, ff=1544, shared=1003),
                                  moe(experts=2, top=2, ff=64, shared=6000)], ids=lambda m: f"{m['kind']}{m.get('ff') or (m['expert']['ff'], m['shared']['ff'])}")
 def test_gated_products_of_every_tile_shape(mlp):
-    """Feed-forwards wide enough, over prompts long enough, that the products take each of the tile shapes; the columns behind the shared
-    expert's start inside a tile."""
+    """Feed-forwards wide enough, over prompts long enough, that the products take several of the tile shapes (every one, over more lengths of K:
+    test_gpu_product_tiles.py); the columns behind the shared expert's start inside a tile."""
     cfg = make_config([layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=mlp)], width=64)
     toks = tokens_for(cfg, 1000, 97)
     w = random_weights(cfg, 98)

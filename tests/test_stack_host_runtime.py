@@ -3,6 +3,7 @@ GPU: nothing is computed, but every allocation and launch is the real code's.  E
 loaded ahead of the library."""
 import ctypes
 import os
+import re
 import subprocess
 import sys
 
@@ -158,6 +159,30 @@ def many_small_rows(stub):
     assert logits.shape == (70000, 16) and ids.shape == (70000,)
 
 
+def tile_shapes(stub):
+    """The sizes of test_gpu_product_tiles.py take the tile shapes they are listed under."""
+    import test_gpu_product_tiles as P
+    import ruzinex_cases as Z
+    import tolenex_cases as T
+
+    def shapes(cfg, cases, rows, want=1):
+        s = engine(cfg, cases, max_tokens=2048, max_sequences=1)
+        stub.forget()
+        step(s, 'a', rows, want)
+        found = [re.search(r'gemm_glds_kernelILi\d+ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)', k) for k in stub.kernels()]
+        return [(32 * int(m[1]) * int(m[3]), 32 * int(m[2]) * int(m[4])) for m in found if m]
+
+    for shape, (columns, ff, grouped) in P.SHAPES.items():
+        for c in (columns, columns - 1):
+            assert shapes(P.plain_config(c, 64), Z, P.ROWS, P.ROWS)[-1] == shape, (shape, c)
+        assert shapes(P.gated_config(Z.dense(ff=ff), 64), Z, P.ROWS)[2] == shape, (shape, ff)
+        assert shapes(P.gated_config(Z.moe(experts=2, top=2, ff=grouped, shared=0), 64), Z, P.ROWS)[3] == shape, (shape, grouped)
+    for shape, (experts, top) in P.FEW.items():
+        assert shapes(P.gated_config(Z.moe(experts=experts, top=top, ff=192, shared=0), 64), Z, P.ROWS)[-2:] == [shape] * 2, shape
+    for shape, (rows, width) in P.RESIDUAL.items():
+        assert [x for x in shapes(P.residual_config(width), T, rows)][1::2] == [shape] * 2, shape
+
+
 if __name__ == '__main__':
     globals()[sys.argv[2]](Stub(sys.argv[1]), *sys.argv[3:])
     print('ok')
@@ -179,3 +204,6 @@ else:
 
     def test_more_wanted_rows_than_a_grid_dimension(stub):
         run(stub, 'many_small_rows')
+
+    def test_tile_shapes_of_the_product_tests(stub):
+        run(stub, 'tile_shapes')
