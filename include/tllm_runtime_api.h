@@ -101,7 +101,9 @@ int32_t tllm_session_vocab_size(tllm_session_t s);
  * (the reference syncs every step, generation.py:963).
  *   input_ids     HOST int32 [B, max_input_len] (padded with pad_id), input_lengths HOST int32 [B];
  *   output_ids    HOST int32 [B, max_input_len + max_new_tokens]: the prompt followed by the generated ids;
- *   end_id < 0 disables early stopping (benchmarks).  Blocks until the ids are on the host. */
+ *   end_id < 0 disables early stopping (benchmarks).  Blocks until the ids are on the host.
+ * fp16 and weight-only layers sum in an order that follows the batch (generation: up to 4 sequences, int4 weights 2, or more), so a
+ * sequence's fp16 values agree alone and in a batch to their rounding, not to the bit; the int8 products of SmoothQuant are exact. */
 int32_t tllm_session_generate(tllm_session_t s, const int32_t* input_ids, const int32_t* input_lengths,
     int32_t max_new_tokens, int32_t end_id, int32_t pad_id, int32_t* output_ids, tllm_stream_t stream);
 

@@ -120,7 +120,9 @@ typedef struct
 } tllm_stack_batch_t;
 
 /* Runs one step.  logits_out: host fp32 [n_want, vocab] or NULL; next_ids_out: host int32 [n_want] (arg-max of each wanted row, the
- * greedy sampler) or NULL.  Every index is checked on the host before anything is launched. */
+ * greedy sampler) or NULL.  Every index is checked on the host before anything is launched.  The kernels of a step, and with them the
+ * order of a row's fp32 sums, follow the step's sizes: the same step gives the same bits, a request in other company (other tokens, or
+ * portions cut elsewhere) the same values to the element type's rounding. */
 int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* batch, float* logits_out, int32_t* next_ids_out, void* stream);
 
 /* Geometry the cache manager needs. */

@@ -8,6 +8,10 @@
 //                     activation row's chunks in registers; fp32 accumulation, DPP reduction; few columns, M <= 8: its form whose waves split K;
 //   float32         : fma_tile_kernel - 64 x 64 tiles of plain fp32 FMAs through LDS (no reduced-precision matrix mode), any shape;
 //                     also the fallback for bfloat16 operands whose rows are not 16-byte aligned.
+//
+// A row's fp32 sums run in the order of the form that serves the call, so its last bits follow the rows beside it: one row, 2 .. 31 and more are
+// different orders in bfloat16, a grouped product of few rows splits K over 4 or 8 waves by how many products the launch holds, and a
+// product of few tiles is cut along K by how many there are.  Rows of one launch do not depend on each other.
 #include "dev_utils.h"
 #include "gemm_glds_impl.h"
 #include "gemm_seam.h"

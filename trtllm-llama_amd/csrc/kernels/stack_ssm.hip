@@ -584,7 +584,9 @@ int launch_stack_ssm_conv(const StackSsmParams& p, hipStream_t stream)
     else if (!ssm_ok(p, "stack_ssm_conv"))
         return -1;
     const int CH = p.conv_channels > 0 ? p.conv_channels : p.heads * p.vdim + 2 * p.groups * p.state;
-    // prompts of 4 taps (the usual number) in runs of rows
+    // Prompts of 4 taps in runs of rows, from 64 on (6144 channels, us: 32 rows 6.7 by a row per workgroup; 63 rows 10.9, 64 in runs 6.4; 1021 rows
+    // 14.7, 1672 rows 19.8).  The models measured here have 4 taps; other numbers keep a row per workgroup (1021 rows 25 us at 3
+    // taps, 106 at 8), since each would be two instantiations more.
     constexpr int RUN = 8;
     const int64_t col = p.conv_channels > 0 ? p.conv_col : p.heads * p.vdim;
     const uintptr_t piece = p.dtype == DT_BF16 ? 7 : 15;
