@@ -17,8 +17,8 @@
 // product without moving, and what comes from scratch is 16 bytes per lane.  One barrier per chunk, where the waves' partial o (and S^T k)
 // meet; the next chunk's operands are in flight under this one's products.
 //
-// Measured (us, both launches, 16 heads): HGRN2 128 x 128, 1024 rows 1024 -> 68; delta rule 128 x 128, three prompts of 683 rows in all 1740 1193 -> 119;
-// Mamba-2 64 heads 128 x 64, 1021 rows 400 -> 70.
+// Measured (us, both launches, 16 heads): HGRN2 128 x 128, 1024 rows 1024 -> 68; delta rule 128 x 128, three prompts of 683 rows in all 1740 1193 -> 123;
+// Mamba-2 64 heads 128 x 64, 1021 rows 400 -> 78.
 #include "dev_utils.h"
 #include "launch_util.h"
 #include "stack_chunk.h"
@@ -524,31 +524,15 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
             else
                 S[n] = S[n] * o.b[n];
         }
-        // The zeros of P and T above their diagonals meet every row in a matrix product, and 0 times an infinity or a NaN is a NaN: where a row
-        // has one, the outputs are formed again row by row, without what follows a row (the state takes every row in any case).  All waves hold
-        // the same x, so that the branch is the workgroup's.  (Delta rule: u overflows only where x is near it, T's entries are below 2^15.)
-        const bool large = any_large(x);
-        if (large)
-        {
-            if constexpr (MODE == DELTA)
-                out = lower_product(o.p, lower_product(o.t, x, 0, 4, out), 0, 4, out);
-            else
-            {
-                po[buf][wid][lane] = lower_product(o.p, u, wid, wid + 1, past); // (nobody reads this chunk's po ahead of the barrier below)
-                __syncthreads();
-            }
-        }
         if constexpr (MODE == DELTA)
         {
             u = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 u = __builtin_amdgcn_mfma_f32_16x16x4f32(o.t[i], x[i], u, 0, 0, 0);
-            f32x4 pu = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                pu = __builtin_amdgcn_mfma_f32_16x16x4f32(o.p[i], u[i], pu, 0, 0, 0);
-            out = large ? out : pu;
+                out = __builtin_amdgcn_mfma_f32_16x16x4f32(o.p[i], u[i], out, 0, 0, 0);
         }
         const f32x4 us = MODE == SSM ? u * o.ws : u;
 #pragma unroll
@@ -558,7 +542,28 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
                 S[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kt[n][i], us[i], S[n], 0, 0, 0);
         // wave w finishes rows 4 g + w
         const float* pf = reinterpret_cast<const float*>(&po[buf][0][0]);
-        float y = ((pf[lane * 4 + wid] + pf[256 + lane * 4 + wid]) + (pf[512 + lane * 4 + wid] + pf[768 + lane * 4 + wid])) + pick(out, wid);
+        auto waves_sum = [&] { return (pf[lane * 4 + wid] + pf[256 + lane * 4 + wid]) + (pf[512 + lane * 4 + wid] + pf[768 + lane * 4 + wid]); };
+        float y = waves_sum() + pick(out, wid);
+        // The zeros of P and T above their diagonals meet every row in a matrix product, and 0 times an infinity or a NaN is a NaN: where a row
+        // has one, the outputs are formed again row by row, without what follows a row (the state takes every row in any case).  All waves hold
+        // the same x, so that the branch is the workgroup's.  (Delta rule: u overflows only where x is near it, T's entries are below 2^15.)
+        // Asked behind the chunk's products: a branch among them takes the next request's addresses and the state's factors out of their
+        // shadow, 60 us for the walk of HGRN2 128 x 128 over 1024 rows instead of 50.
+        if (any_large(x))
+        {
+            if constexpr (MODE == DELTA)
+            {
+                const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+                y = waves_sum() + pick(lower_product(o.p, lower_product(o.t, x, 0, 4, none), 0, 4, none), wid);
+            }
+            else
+            {
+                __syncthreads(); // (every wave has read the sums above)
+                po[buf][wid][lane] = lower_product(o.p, x, wid, wid + 1, past);
+                __syncthreads();
+                y = waves_sum();
+            }
+        }
         const int row = j * R + 4 * g4 + wid;
         if constexpr (MODE == SSM)
         {
