@@ -4,8 +4,8 @@
 //                     (v_mfma_f32_32x32x16_bf16), tile shape by the same rounds x area rule as the fp16 form;
 //   bfloat16, other M >= 32: the register-staged MFMA tiles of gemm_mfma.hip;
 //   bfloat16, M <= 31: slim_kernel below - HBM-bound, the weight-streaming MFMA main loop of gemm_slim_impl.h;
-//   bfloat16, M = 1 but for long rows of few columns: skinny_kernel - a wave streams 2 weight rows with 16-byte non-temporal loads and keeps the
-//                     activation row's chunks in registers; fp32 accumulation, DPP reduction; few columns, M <= 8: its form whose waves split K;
+//   bfloat16, M = 1:  row_kernel - dot products on the vector pipe, K split over a workgroup's waves; fp32 accumulation, DPP reduction;
+//   bfloat16, 2 <= M <= 8, few columns: skinny_ksplit_kernel, the same for several rows;
 //   float32         : fma_tile_kernel - 64 x 64 tiles of plain fp32 FMAs through LDS (no reduced-precision matrix mode), any shape;
 //                     also the fallback for bfloat16 operands whose rows are not 16-byte aligned.
 //
@@ -79,9 +79,9 @@ __device__ __forceinline__ void seam_pair(const StackGemmParams& p, int row, int
     seam_store_pair<DT == DT_FLOAT>(p.seam, p.act, p.c, p.ldc, p.out_f32 != 0, row, col, v0, v1, has1);
 }
 
-// operands of product b of a batched launch
+// operands of product b of a batched launch; first >= 0: of a grouped one whose rows the caller has looked up
 template <int DT>
-__device__ __forceinline__ StackGemmParams batch_slice(StackGemmParams p, int64_t b)
+__device__ __forceinline__ StackGemmParams batch_slice(StackGemmParams p, int64_t b, int first = -1, int rows = 0)
 {
     constexpr int ES = DT == DT_BF16 ? 2 : 4;
     p.a = reinterpret_cast<const char*>(p.a) + b * p.stride_a * ES;
@@ -91,8 +91,8 @@ __device__ __forceinline__ StackGemmParams batch_slice(StackGemmParams p, int64_
     if (p.group_off)
     {
         // grouped form: this product's rows are a range of a and c that the device knows
-        const int64_t o = p.group_off[b];
-        p.M = p.group_off[b + 1] - (int) o;
+        const int64_t o = first >= 0 ? first : p.group_off[b];
+        p.M = first >= 0 ? rows : p.group_off[b + 1] - (int) o;
         if (p.a_rows)
             p.a_rows += o;
         else
@@ -166,65 +166,191 @@ __global__ __launch_bounds__(256) void fma_tile_kernel(const StackGemmParams p_i
 
 // Group blockIdx.z of a grouped launch whose grid holds fewer products than there are groups: the blockIdx.z-th one that has rows (a step of
 // few tokens reaches few experts; 32 x 352 workgroups of which 4 x 352 have work cost more to start than to run).  -1: there is none.
-__device__ __forceinline__ int nth_group(const int32_t* off, int groups, int nth)
+// first, rows: where its rows begin and how many they are.
+__device__ __forceinline__ int nth_group(const int32_t* off, int groups, int nth, int& first, int& rows)
 {
     const int lane = threadIdx.x & 63;
     for (int g0 = 0; g0 < groups; g0 += 64)
     {
         const int g = g0 + lane;
-        uint64_t has = __ballot(g < groups && off[g + 1] > off[g]);
+        const int lo = g < groups ? off[g] : 0, hi = g < groups ? off[g + 1] : 0;
+        uint64_t has = __ballot(hi > lo);
         const int n = __popcll(has);
         if (nth < n)
         {
             for (; nth > 0; --nth)
                 has &= has - 1;
-            return g0 + __ffsll((unsigned long long) has) - 1;
+            const int at = __ffsll((unsigned long long) has) - 1;
+            first = __builtin_amdgcn_readlane(lo, at);
+            rows = __builtin_amdgcn_readlane(hi, at) - first;
+            return g0 + at;
         }
         nth -= n;
     }
     return -1;
 }
 
-// bfloat16, one row: 4 waves per workgroup, SK_R weight rows per wave
+// bfloat16, one row: KS waves share SK_R rows of W (one pair of columns), wave w the 1 KiB chunks w, w + KS, ... of each, and 4 / KS such teams make
+// a workgroup.  NC chunks per wave and row, with the activations that face them, are requested before the first is used: a product of up to
+// 512 KS NC columns of A is one trip to memory per wave, and the next workgroups' trips overlap it.  Bound by the weights' stream.  What it replaced were whole
+// rows per wave, a chunk of 2 rows at a time, and for long rows of few columns the matrix pipe; us, cold weights, N x K:
+//   2048 x 2048 3.5 (4.6)    2048 x 5504 6.0 (8.5)    4096 x 4096 7.0 (8.5)    4096 x 11008 16.5 (19.0)    10304 x 2048 8.0 (8.9)
+//   10240 x 4096 13.6 (15.5)    22016 x 4096 26.4 = 6.8 TB/s (31.1)    32000 x 2048 20.0 (21.4)
+// 4 rows per team measured the same within 4 %, 8 waves per team too, 8 of both up to 60 % worse.
 constexpr int SK_R = 2;
 
-__global__ __launch_bounds__(256) void skinny_kernel(const StackGemmParams p_in, int groups)
+// What the epilogue of columns n and n + 1 of the one row reads, requested with the weights; raw, so that nothing waits for it here.
+struct RowSeam
 {
-    int b = blockIdx.z;
-    if (groups && (b = nth_group(p_in.group_off, groups, b)) < 0)
-        return;
-    const StackGemmParams p = batch_slice<DT_BF16>(p_in, b);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int n0 = (blockIdx.x * 4 + wid) * SK_R;
-    if (n0 >= p.N || p.M <= 0)
-        return;
-    float acc[SK_R] = {0.f, 0.f};
-    const uint16_t* a = reinterpret_cast<const uint16_t*>(p.a) + (int64_t) (p.a_rows ? p.a_rows[0] : 0) * p.lda;
-    const uint16_t* w = reinterpret_cast<const uint16_t*>(p.w);
-    for (int k = lane * 8; k < p.K; k += 64 * 8)
+    float r[2], b[2];
+    uint16_t z[2];
+};
+__device__ __forceinline__ RowSeam row_seam_request(const StackGemmParams& p, int n)
+{
+    RowSeam o = {};
+    const int n1 = n + 1 < p.N ? n + 1 : n;
+    const float* bias = p.resid ? p.gate_bias : p.bias;
+    if (bias)
     {
-        uint4 wv[SK_R];
-#pragma unroll
-        for (int r = 0; r < SK_R; ++r)
-            wv[r] = n0 + r < p.N ? ld_nt16(w + (int64_t) (n0 + r) * p.ldw + k) : make_uint4(0, 0, 0, 0);
-        const uint4 xv = *reinterpret_cast<const uint4*>(a + k);
-        const uint32_t xs[4] = {xv.x, xv.y, xv.z, xv.w};
-#pragma unroll
-        for (int r = 0; r < SK_R; ++r)
+        o.b[0] = bias[n];
+        o.b[1] = bias[n1];
+    }
+    if (p.resid)
+    {
+        o.r[0] = p.resid[n];
+        o.r[1] = p.resid[n1];
+        if (p.gate)
         {
-            const uint32_t ws[4] = {wv[r].x, wv[r].y, wv[r].z, wv[r].w};
+            o.z[0] = reinterpret_cast<const uint16_t*>(p.gate)[n];
+            o.z[1] = reinterpret_cast<const uint16_t*>(p.gate)[n1];
+        }
+    }
+    return o;
+}
+// seam_pair of row 0 with those operands
+__device__ __forceinline__ void row_seam(const StackGemmParams& p, const RowSeam& o, int n, float v0, float v1)
+{
+    if (!p.resid)
+    {
+        seam_store_pair<false>(p.seam, p.act, p.c, p.ldc, p.out_f32 != 0, 0, n, v0 + o.b[0], v1 + o.b[1], n + 1 < p.N);
+        return;
+    }
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 2; ++i)
+    {
+        const float g = p.gate ? 1.f / (1.f + expf(-(bf2f(o.z[i]) + o.b[i]))) : 1.f;
+        if (n + i < p.N)
+            p.resid[n + i] = o.r[i] + g * (i ? v1 : v0);
+    }
+}
+
+template <int KS, int NC>
+__global__ __launch_bounds__(256) void row_kernel(const StackGemmParams p_in, int groups)
+{
+    constexpr int TEAMS = 4 / KS;
+    __shared__ float part[4][SK_R];
+    int b = blockIdx.z, first = -1, rows = 0;
+    if (groups && (b = nth_group(p_in.group_off, groups, b, first, rows)) < 0)
+        return;
+    const StackGemmParams p = batch_slice<DT_BF16>(p_in, b, first, rows);
+    if (p.M <= 0)
+        return;
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kw = wid % KS;
+    const int n0 = (blockIdx.x * TEAMS + wid / KS) * SK_R; // (a team beyond N repeats the last row and stores nothing)
+    const uint16_t* a = reinterpret_cast<const uint16_t*>(p.a) + (int64_t) (p.a_rows ? p.a_rows[0] : 0) * p.lda;
+    const uint16_t* w[SK_R];
+#pragma unroll
+    for (int r = 0; r < SK_R; ++r)
+        w[r] = reinterpret_cast<const uint16_t*>(p.w) + (int64_t) (n0 + r < p.N ? n0 + r : p.N - 1) * p.ldw;
+    const RowSeam ops = row_seam_request(p, n0 < p.N ? n0 : p.N - 1);
+    float acc[SK_R] = {0.f, 0.f};
+    for (int c0 = kw; c0 * 512 < p.K; c0 += KS * NC)
+    {
+        uint4 wv[NC][SK_R], xv[NC];
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+        {
+            int k = (c0 + i * KS) * 512 + lane * 8;
+            k = k < p.K ? k : 0; // (loads without a branch; what they bring beyond K is dropped below)
+#pragma unroll
+            for (int r = 0; r < SK_R; ++r)
+                wv[i][r] = ld_nt16(w[r] + k);
+            xv[i] = *reinterpret_cast<const uint4*>(a + k);
+        }
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+        {
+            const bool in = (c0 + i * KS) * 512 + lane * 8 < p.K; // (no branch: behind one the compiler would request a chunk where it is used)
+            const uint32_t xs[4] = {in ? xv[i].x : 0u, in ? xv[i].y : 0u, in ? xv[i].z : 0u, in ? xv[i].w : 0u};
+#pragma unroll
+            for (int r = 0; r < SK_R; ++r)
             {
-                acc[r] = fmaf(__builtin_bit_cast(float, xs[i] << 16), __builtin_bit_cast(float, ws[i] << 16), acc[r]);
-                acc[r] = fmaf(__builtin_bit_cast(float, xs[i] & 0xffff0000u), __builtin_bit_cast(float, ws[i] & 0xffff0000u), acc[r]);
+                const uint32_t ws[4] = {in ? wv[i][r].x : 0u, in ? wv[i][r].y : 0u, in ? wv[i][r].z : 0u, in ? wv[i][r].w : 0u};
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                {
+                    acc[r] = fmaf(__builtin_bit_cast(float, xs[q] << 16), __builtin_bit_cast(float, ws[q] << 16), acc[r]);
+                    acc[r] = fmaf(__builtin_bit_cast(float, xs[q] & 0xffff0000u), __builtin_bit_cast(float, ws[q] & 0xffff0000u), acc[r]);
+                }
             }
         }
     }
-    static_assert(SK_R == 2, "a wave's rows are one pair of columns");
+    static_assert(SK_R == 2, "a team's rows are one pair of columns");
     const float s0 = wave_sum(acc[0]), s1 = wave_sum(acc[1]);
+    if constexpr (KS == 1)
+    {
+        if (lane == 0 && n0 < p.N)
+            row_seam(p, ops, n0, s0, s1);
+        return;
+    }
     if (lane == 0)
-        seam_pair<DT_BF16>(p, 0, n0, s0, s1);
+    {
+        part[wid][0] = s0;
+        part[wid][1] = s1;
+    }
+    __syncthreads();
+    if (lane == 0 && kw == 0 && n0 < p.N)
+    {
+        float v0 = part[wid][0], v1 = part[wid][1];
+#pragma unroll
+        for (int k = 1; k < KS; ++k)
+        {
+            v0 += part[wid + k][0];
+            v1 += part[wid + k][1];
+        }
+        row_seam(p, ops, n0, v0, v1);
+    }
+}
+
+// A wave's chunks at once are all it has up to 12288 columns of A, then portions of 3.  Rows of up to 2048 columns are shared by 2 or 4 waves only where
+// that leaves the chip room to take all workgroups in at once; otherwise, and where a workgroup first looks up its group, a wave has rows of its own and a
+// workgroup lives longer (32000 x 2048 21.6 us by two waves a row, 22.2 by four; 4 grouped products of 2816 x 2048 10.3 against 12.1;
+// 2048 x 2048 4.8 by two, 4.6 by four).
+void launch_row(const StackGemmParams& p, int products, int groups, hipStream_t stream)
+{
+    auto go = [&](auto kernel, int ks) {
+        const int cols = SK_R * (4 / ks);
+        hipLaunchKernelGGL(kernel, dim3((p.N + cols - 1) / cols, 1, products), dim3(256), 0, stream, p, groups);
+    };
+    const int chunks = (p.K + 511) / 512;
+    const bool many = p.group_off || (int64_t) p.N * products > 16 * launch_util::device_cus();
+    if (chunks <= 1)
+        go(row_kernel<1, 1>, 1);
+    else if (chunks <= 2)
+        many ? go(row_kernel<1, 2>, 1) : go(row_kernel<2, 1>, 2);
+    else if (chunks <= 3)
+        many ? go(row_kernel<1, 3>, 1) : go(row_kernel<4, 1>, 4);
+    else if (chunks <= 4)
+        many ? go(row_kernel<1, 4>, 1) : go(row_kernel<4, 1>, 4);
+    else if (chunks <= 8)
+        p.group_off ? go(row_kernel<2, 4>, 2) : go(row_kernel<4, 2>, 4);
+    else if (chunks <= 12 || chunks > 24)
+        go(row_kernel<4, 3>, 4);
+    else if (chunks <= 16)
+        go(row_kernel<4, 4>, 4);
+    else
+        go(row_kernel<4, 6>, 4);
 }
 
 // bfloat16, M <= 16 * MT rows: the main loop of gemm_slim_impl.h, a workgroup per 16 columns and product
@@ -232,10 +358,10 @@ template <int MT, int D, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void slim_kernel(const StackGemmParams p_in, int groups)
 {
     __shared__ __attribute__((aligned(16))) char lds[slim::lds_bytes<MT, WAVES>()];
-    int b = blockIdx.z;
-    if (groups && (b = nth_group(p_in.group_off, groups, b)) < 0)
+    int b = blockIdx.z, first = -1, rows = 0;
+    if (groups && (b = nth_group(p_in.group_off, groups, b, first, rows)) < 0)
         return;
-    const StackGemmParams p = batch_slice<DT_BF16>(p_in, b);
+    const StackGemmParams p = batch_slice<DT_BF16>(p_in, b, first, rows);
     if (p.M <= 0)
         return;
     const int lane = threadIdx.x & 63, n0 = blockIdx.x * 16;
@@ -265,8 +391,7 @@ void launch_slim(const StackGemmParams& p, int products, int groups, hipStream_t
     hipLaunchKernelGGL((slim_kernel<MT, D, WAVES>), dim3((p.N + 15) / 16, 1, products), dim3(WAVES * 64), 0, stream, p, groups);
 }
 
-// The same for products of few rows of W (a token input's gate): a workgroup per SK_R rows whose 4 waves split K, so that the weights are
-// requested by four times the waves; their sums meet in LDS.
+// Several rows through few columns (a token input's gate): a workgroup per SK_R rows of W whose 4 waves split K; their sums meet in LDS.
 template <int MR>
 __global__ __launch_bounds__(256) void skinny_ksplit_kernel(const StackGemmParams p)
 {
@@ -435,24 +560,20 @@ int launch_stack_gemm(const StackGemmParams& p_in, hipStream_t stream)
         const bool few = p.group_off && p.group_total < p.batch;
         const int products = few ? p.group_total : p.batch, groups = few ? p.batch : 0;
         const int64_t slim_wgs = (int64_t) ((p.N + 15) / 16) * products;
+        if (p.M <= 1)
+        {
+            launch_row(p, products, groups, stream);
+            return launched("stack_gemm row");
+        }
         if (p.batch == 1 && !p.group_off && p.M <= 8 && (p.N + 7) / 8 * 2 <= cus && p.K >= 2048)
         {
-            // 1024 x 2048: 3.4 / 4.0 / 5.2 us at one / four / eight rows, the MFMA form 5.1 .. 6.2
+            // 1024 x 2048: 4.0 / 5.2 us at four / eight rows, the MFMA form 5.1 .. 6.2
             const dim3 kg((p.N + SK_R - 1) / SK_R);
-            if (p.M <= 1)
-                hipLaunchKernelGGL((skinny_ksplit_kernel<1>), kg, dim3(256), 0, stream, p);
-            else if (p.M <= 4)
+            if (p.M <= 4)
                 hipLaunchKernelGGL((skinny_ksplit_kernel<4>), kg, dim3(256), 0, stream, p);
             else
                 hipLaunchKernelGGL((skinny_ksplit_kernel<8>), kg, dim3(256), 0, stream, p);
             return launched("stack_gemm skinny (K over waves)");
-        }
-        if (p.M <= 1 && (slim_wgs > cus || p.K < 4096))
-        {
-            // one row: 32000 x 2048 22.4 us against the MFMA form's 28.0, 11008 x 2048 10.4 / 12.3, 2048 x 2048 5.4 / 6.2; long rows of few
-            // columns want the MFMA form, whose waves split K: 4096 x 4096 9.7 against 10.8, 4096 x 11008 20.3 / 21.4, 2048 x 5504 9.7 / 10.3
-            hipLaunchKernelGGL(skinny_kernel, dim3((p.N + 4 * SK_R - 1) / (4 * SK_R), 1, products), dim3(256), 0, stream, p, groups);
-            return launched("stack_gemm skinny");
         }
         const bool many = slim_wgs * 4 >= cus * 5; // (gemm_slim_impl.h)
         if (p.M <= 16)

@@ -1823,8 +1823,8 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         u.N = up_cols;
         u.K = Wd;
         u.a = mp.a_sorted ? s->moe_a : s->h1;
-        u.a_rows = mp.a_sorted ? nullptr : mp.tok_of_slot;
-        u.lda = Wd;
+        u.a_rows = mp.a_sorted || T == 1 ? nullptr : mp.tok_of_slot;
+        u.lda = mp.a_sorted || T > 1 ? Wd : 0; // (every slot of a lone token reads its row: nothing to look up)
         u.w = l.w_gu;
         u.c = s->act;
         u.ldc = l.ff;
