@@ -126,6 +126,18 @@ int launch_stack_pass_entry(float* x, const float* add, const float* row, int32_
 // gather (row r reads x[rows[r]]).  y2 / w2 may be null.
 int launch_stack_group_rmsnorm(void* y1, void* y2, const float* x, const int32_t* rows, const float* w1, const float* w2, int32_t dtype,
     int32_t n_rows, int32_t width, int32_t groups, float eps, hipStream_t stream);
+// A routed mixture's sum that has not been formed yet: row t of what it stands for is (has_row ? (keep ? sigmoid(keep[t]) : 1) y[t] : 0) plus the
+// outputs of the token's experts (launch_stack_moe_combine's terms and order).  The norm that reads the sum forms it (in rows that it does not take in
+// 16-byte pieces: has it formed, in y, by a launch ahead of its own).
+struct StackExpertSum
+{
+    const float* ys = nullptr; // [slots, width]; null: y is what it is
+    const int32_t* slot_of_pair = nullptr;
+    const float* topk_w = nullptr;
+    const void* h = nullptr; // an identity's output: row t of the experts' input (may be the row that the norm writes)
+    const float* keep = nullptr;
+    int32_t tokens = 0, top = 0, weight_input = 0, has_row = 0;
+};
 // Hyper-connected residual streams xs[s] = x + s * stream_stride (fp32 [tokens, width] each, `streams` >= 1 of them; one stream with
 // mix = out = in = 1 is the plain residual sum).  In one pass over a row:
 //   1. y != null: a sublayer's result lands, all streams at once from the old ones: xs[t] <- sum_s mix[s * streams + t] xs[s] + out[t] y
@@ -140,7 +152,8 @@ struct StackHyperParams
     int32_t tokens = 0, width = 0, streams = 1;
     float* x = nullptr;
     int64_t stream_stride = 0;
-    const float* y = nullptr;   // [tokens, width] or null
+    float* y = nullptr;         // [tokens, width] or null
+    StackExpertSum sum;         // y stands for it
     const float* mix = nullptr; // [streams, streams], indexed [from, to]
     const float* out = nullptr; // [streams]
     const float* in = nullptr;  // [streams] or null
@@ -163,7 +176,8 @@ struct StackLandParams
     int32_t dtype = DT_BF16;
     int32_t tokens = 0, width = 0;
     float* x = nullptr;
-    const float* y = nullptr;      // [tokens, width] or null
+    float* y = nullptr;            // [tokens, width] or null
+    StackExpertSum sum;            // y stands for it
     const void* table = nullptr;   // [vocab, width] of the element type or null
     const int32_t* ids = nullptr;  // [tokens]
     int32_t vocab = 0;

@@ -1532,6 +1532,63 @@ int launch_stack_token_shift(const StackShiftParams& p, hipStream_t stream)
 
 namespace
 {
+// Row t of a mixture's sum (StackExpertSum), K float4 pieces per thread from piece tid on, nt apart; u holds y's row where it has a part.  Terms and
+// their order are moe_combine_vec_kernel's.  A launch of its own for the sum took 2.7 us a token's layer (width 2048, top 4), 10 .. 13 us at 1720
+// tokens, and wrote and read its row once more.
+template <int DT, int K>
+__device__ __forceinline__ void expert_sum(const StackExpertSum& m, int t, int width, int tid, int nt, float4 (&u)[K])
+{
+    constexpr int AHEAD = 4;
+    const float keep = m.keep ? 1.f / (1.f + expf(-m.keep[t])) : 1.f;
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        u[k] = m.has_row ? make_float4(u[k].x * keep, u[k].y * keep, u[k].z * keep, u[k].w * keep) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int j0 = 0; j0 < m.top; j0 += AHEAD)
+    {
+        int slot[AHEAD];
+        float w[AHEAD];
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j)
+        {
+            const int64_t pair = (int64_t) t * m.top + (j0 + j < m.top ? j0 + j : j0);
+            slot[j] = m.slot_of_pair[pair];
+            w[j] = m.weight_input && slot[j] >= 0 ? 1.f : m.topk_w[pair]; // an input-weighted expert's output is summed as it is
+        }
+        float4 v[K][AHEAD];
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j)
+            {
+                const int c = 4 * (tid + k * nt);
+                if (c >= width)
+                    v[k][j] = make_float4(0.f, 0.f, 0.f, 0.f);
+                else if (slot[j] >= 0)
+                    v[k][j] = *reinterpret_cast<const float4*>(m.ys + (int64_t) slot[j] * width + c);
+                else if constexpr (DT == DT_BF16)
+                {
+                    const uint2 b = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(m.h) + (int64_t) t * width + c);
+                    v[k][j] = make_float4(__builtin_bit_cast(float, b.x << 16), __builtin_bit_cast(float, b.x & 0xffff0000u),
+                        __builtin_bit_cast(float, b.y << 16), __builtin_bit_cast(float, b.y & 0xffff0000u));
+                }
+                else
+                    v[k][j] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(m.h) + (int64_t) t * width + c);
+            }
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j)
+            {
+                if (j0 + j >= m.top)
+                    break;
+                u[k].x = fmaf(w[j], v[k][j].x, u[k].x);
+                u[k].y = fmaf(w[j], v[k][j].y, u[k].y);
+                u[k].z = fmaf(w[j], v[k][j].z, u[k].z);
+                u[k].w = fmaf(w[j], v[k][j].w, u[k].w);
+            }
+    }
+}
+
 // The form for rows of a multiple of 4 up to HV_K * 4096 elements: up to 1024 threads, a thread owns HV_K float4 columns of every
 // stream and has ALL of them in flight before its first store (the streams are read and written through the same pointer, so in
 // a loop every store would fence the loads behind it); the combined row stays in registers.
@@ -1542,7 +1599,8 @@ __global__ __launch_bounds__(1024) void hyper_norm_vec_kernel(const StackHyperPa
 {
     __shared__ float red[32];
     const int t = p.rows ? p.rows[blockIdx.x] : blockIdx.x, tid = threadIdx.x, S = p.streams, W4 = p.width >> 2, NT = blockDim.x;
-    float4 xs[HV_K][SM], yv[HV_K], u[HV_K];
+    constexpr bool EARLY = SM <= 2; // the norm's weights come in with the row (more streams: no registers left for them)
+    float4 xs[HV_K][SM], yv[HV_K], u[HV_K], wv[HV_K];
 #pragma unroll
     for (int k = 0; k < HV_K; ++k)
     {
@@ -1552,9 +1610,13 @@ __global__ __launch_bounds__(1024) void hyper_norm_vec_kernel(const StackHyperPa
         for (int s = 0; s < SM; ++s)
             xs[k][s] = (s < S && c4 < W4) ? reinterpret_cast<const float4*>(p.x + s * p.stream_stride + (int64_t) t * p.width)[c4]
                                           : make_float4(0.f, 0.f, 0.f, 0.f);
-        if (p.y && c4 < W4)
+        if (p.y && c4 < W4 && (!p.sum.ys || p.sum.has_row))
             yv[k] = reinterpret_cast<const float4*>(p.y + (int64_t) t * p.width)[c4];
+        if (EARLY)
+            wv[k] = p.w && c4 < W4 ? reinterpret_cast<const float4*>(p.w)[c4] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
+    if (p.y && p.sum.ys)
+        expert_sum<DT, HV_K>(p.sum, t, p.width, tid, NT, yv);
     float cm[SM][SM], co[SM], ci[SM];
 #pragma unroll
     for (int a = 0; a < SM; ++a)
@@ -1613,7 +1675,7 @@ __global__ __launch_bounds__(1024) void hyper_norm_vec_kernel(const StackHyperPa
         const int c4 = tid + k * NT;
         if (c4 < W4)
         {
-            const float4 w = reinterpret_cast<const float4*>(p.w)[c4];
+            const float4 w = EARLY ? wv[k] : reinterpret_cast<const float4*>(p.w)[c4];
             const int64_t o = (int64_t) blockIdx.x * p.width + 4 * c4;
             if (p.h32)
                 *reinterpret_cast<float4*>(p.h32 + o) = make_float4(u[k].x * inv * w.x, u[k].y * inv * w.y, u[k].z * inv * w.z, u[k].w * inv * w.w);
@@ -1686,12 +1748,14 @@ __global__ __launch_bounds__(1024) void land_vec_kernel(const StackLandParams p)
             u[k] = land_table4<DT>(p.table, trow + 4 * c4);
             u[k].x *= p.scale, u[k].y *= p.scale, u[k].z *= p.scale, u[k].w *= p.scale;
         }
-        else if (on && p.y)
+        else if (on && p.y && (!p.sum.ys || p.sum.has_row))
             u[k] = reinterpret_cast<const float4*>(p.y + row)[c4];
         yn[k] = on && p.y_norm ? reinterpret_cast<const float4*>(p.y_norm)[c4] : zero;
         ar[k] = on && p.add_row ? reinterpret_cast<const float4*>(p.add_row)[c4] : zero;
         wv[k] = on && p.w ? reinterpret_cast<const float4*>(p.w)[c4] : zero;
     }
+    if (p.sum.ys)
+        expert_sum<DT, K>(p.sum, t, p.width, tid, NT, u);
     if (p.y_norm)
     {
         float ss = 0.f;
@@ -1804,19 +1868,37 @@ __global__ __launch_bounds__(256) void land_kernel(const StackLandParams p)
 
 } // namespace
 
-int launch_stack_land(const StackLandParams& p, hipStream_t stream)
+// y = the sum, for a norm that does not form it itself
+static int form_expert_sum(const StackExpertSum& m, float* y, int32_t dtype, int32_t width, hipStream_t stream)
 {
+    StackMoeParams mp;
+    mp.dtype = dtype;
+    mp.tokens = m.tokens;
+    mp.width = width;
+    mp.experts = mp.top = m.top;
+    mp.weight_input = m.weight_input;
+    mp.h = m.h;
+    mp.topk_w = const_cast<float*>(m.topk_w);
+    mp.slot_of_pair = const_cast<int32_t*>(m.slot_of_pair);
+    mp.accumulate = m.has_row;
+    mp.accumulate_gate = m.keep;
+    return launch_stack_moe_combine(mp, m.ys, y, stream);
+}
+
+int launch_stack_land(const StackLandParams& p_in, hipStream_t stream)
+{
+    StackLandParams p = p_in;
     if (p.tokens <= 0)
         return 0;
     if (!known_dtype(p.dtype, "stack_land"))
         return -1;
-    if (p.width < 1 || !p.x || (p.table && (!p.ids || p.vocab < 1 || p.y)) || (p.y_norm && !p.table && !p.y))
+    if (p.width < 1 || !p.x || (p.table && (!p.ids || p.vocab < 1 || p.y)) || (p.y_norm && !p.table && !p.y) || (p.sum.ys && !p.y))
     {
         set_error("stack_land: width %d, or a missing operand", p.width);
         return -1;
     }
     uintptr_t bits = 0;
-    for (const void* q : {(const void*) p.x, (const void*) p.y, p.table, (const void*) p.y_norm, (const void*) p.tap, (const void*) p.add_row, (const void*) p.h, (const void*) p.w})
+    for (const void* q : {(const void*) p.x, (const void*) p.y, p.table, (const void*) p.y_norm, (const void*) p.tap, (const void*) p.add_row, (const void*) p.h, (const void*) p.w, (const void*) p.sum.ys, p.sum.h})
         bits |= reinterpret_cast<uintptr_t>(q);
     if (p.width % 4 == 0 && p.width <= HV_K * 4096 && !(bits & 15))
     {
@@ -1834,6 +1916,9 @@ int launch_stack_land(const StackLandParams& p, hipStream_t stream)
 #undef TLLM_LAND
         return launched("stack_land");
     }
+    if (p.sum.ys && form_expert_sum(p.sum, p.y, p.dtype, p.width, stream))
+        return -1;
+    p.sum = StackExpertSum();
     const size_t lds = sizeof(float) * (size_t) p.width;
     if (lds > 60 * 1024)
     {
@@ -1847,8 +1932,9 @@ int launch_stack_land(const StackLandParams& p, hipStream_t stream)
     return launched("stack_land");
 }
 
-int launch_stack_hyper_norm(const StackHyperParams& p, hipStream_t stream)
+int launch_stack_hyper_norm(const StackHyperParams& p_in, hipStream_t stream)
 {
+    StackHyperParams p = p_in;
     if (p.tokens <= 0)
         return 0;
     if (!known_dtype(p.dtype, "stack_hyper_norm"))
@@ -1860,7 +1946,7 @@ int launch_stack_hyper_norm(const StackHyperParams& p, hipStream_t stream)
     }
     const bool al16 = !(reinterpret_cast<uintptr_t>(p.x) & 15) && !(reinterpret_cast<uintptr_t>(p.y) & 15) && !(reinterpret_cast<uintptr_t>(p.h) & 15)
         && !(reinterpret_cast<uintptr_t>(p.w) & 15) && !(reinterpret_cast<uintptr_t>(p.sum_out) & 15) && !(reinterpret_cast<uintptr_t>(p.h32) & 15)
-        && p.stream_stride % 4 == 0;
+        && p.stream_stride % 4 == 0 && !((reinterpret_cast<uintptr_t>(p.sum.ys) | reinterpret_cast<uintptr_t>(p.sum.h)) & 15);
     if (p.width % 4 == 0 && p.width <= HV_K * 4096 && al16)
     {
         const int nt = std::min(1024, (p.width / 4 + 63) / 64 * 64);
@@ -1870,6 +1956,9 @@ int launch_stack_hyper_norm(const StackHyperParams& p, hipStream_t stream)
             launch_hyper_vec<DT_FLOAT>(p, nt, stream);
         return launched("stack_hyper_norm");
     }
+    if (p.sum.ys && form_expert_sum(p.sum, p.y, p.dtype, p.width, stream))
+        return -1;
+    p.sum = StackExpertSum();
     const size_t lds = sizeof(float) * (size_t) p.width;
     if (lds > 64 * 1024)
     {

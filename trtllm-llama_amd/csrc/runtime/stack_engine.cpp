@@ -1779,9 +1779,9 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         return (launch_stack_rope_kv(a, stream) || launch_stack_attention(a, stream)) ? -1 : 0;
     };
 
-    // the routed feed-forward on h1: y32 = its output, or (accumulate) x += it, x_el = the resulting rows in the element type.  With
-    // residual=plain the router's logits are there already.
-    auto run_moe = [&](const Layer& l, float* y, bool accumulate, void* y_el) -> int {
+    // the routed feed-forward on h1: y = its output, or (accumulate) y += it, x_el = the resulting rows in the element type; later != null: what y
+    // stands for, for the norm that reads it.  With residual=plain the router's logits are there already.
+    auto run_moe = [&](const Layer& l, float* y, bool accumulate, void* y_el, StackExpertSum* later) -> int {
         const size_t pairs = (size_t) T * l.top;
         StackMoeParams mp;
         mp.dtype = s->dtype;
@@ -1852,8 +1852,23 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         dn.group_off = mp.group_off;
         dn.group_total = u.group_total;
         dn.group_rows = u.group_rows;
-        return (launch_stack_gemm(dn, stream) || launch_stack_moe_combine(mp, s->moe_y, y, stream)) ? -1 : 0;
+        if (launch_stack_gemm(dn, stream))
+            return -1;
+        if (!later)
+            return launch_stack_moe_combine(mp, s->moe_y, y, stream);
+        later->ys = s->moe_y;
+        later->slot_of_pair = mp.slot_of_pair;
+        later->topk_w = mp.topk_w;
+        later->h = mp.h;
+        later->keep = mp.accumulate_gate;
+        later->tokens = T;
+        later->top = l.top;
+        later->weight_input = mp.weight_input;
+        later->has_row = mp.accumulate;
+        return 0;
     };
+
+    StackExpertSum left_sum; // what y32 stands for where the last sublayer was a mixture of experts
 
     // the feed-forwards of sequential blocks: h1 -> y32
     auto seq_dense = [&](const Layer& l) -> int {
@@ -1939,7 +1954,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             if (launch_stack_gemm(sd, stream))
                 return -1;
         }
-        return run_moe(l, s->y32, l.shared_ff > 0, nullptr);
+        return run_moe(l, s->y32, l.shared_ff > 0, nullptr, &left_sum);
     };
 
     // residual=plain: what the last sublayer or token input left to land in y32, and the next norm, in one launch
@@ -1962,6 +1977,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         else if (land_y)
         {
             lp.y = s->y32;
+            lp.sum = left_sum;
             lp.y_norm = land_norm;
             lp.y_scale = s->resid_mult;
         }
@@ -1973,6 +1989,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         lp.rows = rows;
         land_y = false;
         land_norm = nullptr;
+        left_sum = StackExpertSum();
         return launch_stack_land(lp, stream);
     };
 
@@ -1990,6 +2007,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         if (pending)
         {
             hp.y = s->y32;
+            hp.sum = left_sum;
             hp.mix = pending->mix;
             hp.out = pending->out;
         }
@@ -2000,6 +2018,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         hp.sum_out = sum_out;
         hp.h32 = h32;
         pending = nullptr;
+        left_sum = StackExpertSum();
         return launch_stack_hyper_norm(hp, stream);
     };
 
@@ -2036,7 +2055,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
                 if (launch_stack_gemm(o, stream))
                     return -1;
             }
-            if (l.ff > 0 && run_moe(l, s->x, true, s->side_dim ? s->x_el : nullptr))
+            if (l.ff > 0 && run_moe(l, s->x, true, s->side_dim ? s->x_el : nullptr, nullptr))
                 return -1;
             if (s->side_dim > 0)
             {
@@ -2229,6 +2248,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             if (pending)
             {
                 hp.y = s->y32;
+                hp.sum = left_sum;
                 hp.mix = pending->mix;
                 hp.out = pending->out;
             }
