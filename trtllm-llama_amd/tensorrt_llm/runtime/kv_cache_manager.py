@@ -148,18 +148,25 @@ class KVCacheManager(object):
     def reserve(self, sequence: GenerationSequence, total_tokens: int):
         """Ragged batches: make `sequence` (known or new) hold blocks for `total_tokens` tokens.  A prompt arrives in portions of
         any size, so the blocks are taken as the portions come, not for the whole prompt at once."""
-        if sequence not in self.blocks_manager._owned and sequence not in self.sequences:
+        owned = self.blocks_manager._owned.get(sequence)
+        if owned is None and sequence not in self.sequences:
             sequence.batch_idx = len(self.sequences)
             self.sequences.append(sequence)
             self.lens.append(0)
-        have = self.blocks_manager.get_number_blocks(sequence) if sequence in self.blocks_manager._owned else 0
+        at = sequence.batch_idx  # its place, unless the caller counts its batch another way
+        if not (0 <= at < len(self.sequences) and self.sequences[at] is sequence):
+            at = self.sequences.index(sequence)
+        have = len(owned[0]) if owned is not None else 0
         need = -(-total_tokens // self.tokens_per_block)
+        if need <= have:
+            self.lens[at] = total_tokens
+            return
         if need - have > self.blocks_manager.num_free_blocks():
             raise RuntimeError(f"Can't allocate new block for KV cache: sequence {sequence.get_seq_idx()} needs {need - have} more, "
                                f'{self.blocks_manager.num_free_blocks()} are free')
         for _ in range(need - have):
             self.blocks_manager.allocate(sequence, share_across_beam=True)
-        self.lens[self.sequences.index(sequence)] = total_tokens
+        self.lens[at] = total_tokens
 
     def release(self, sequence: GenerationSequence):
         """Give back everything `sequence` holds (ragged batches: a sequence ends when its owner says so)."""
