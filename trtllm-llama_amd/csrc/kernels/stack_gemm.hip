@@ -353,30 +353,26 @@ void launch_row(const StackGemmParams& p, int products, int groups, hipStream_t 
         go(row_kernel<4, 6>, 4);
 }
 
-// bfloat16, M <= 16 * MT rows: the main loop of gemm_slim_impl.h, a workgroup per 16 columns and product
-template <int MT, int D, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void slim_kernel(const StackGemmParams p_in, int groups)
+// bfloat16, 2 .. 31 rows: the main loop of gemm_slim_impl.h, a workgroup per S::cols columns and product
+template <class S>
+__global__ __launch_bounds__(S::waves * 64) void slim_kernel(const StackGemmParams p_in, int groups)
 {
-    __shared__ __attribute__((aligned(16))) char lds[slim::lds_bytes<MT, WAVES>()];
+    extern __shared__ __attribute__((aligned(16))) char slim_lds[];
     int b = blockIdx.z, first = -1, rows = 0;
     if (groups && (b = nth_group(p_in.group_off, groups, b, first, rows)) < 0)
         return;
     const StackGemmParams p = batch_slice<DT_BF16>(p_in, b, first, rows);
     if (p.M <= 0)
         return;
-    const int lane = threadIdx.x & 63, n0 = blockIdx.x * 16;
-    const char* xrow[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-    {
-        int m = 16 * t + (lane & 15);
-        m = m < p.M ? m : p.M - 1;
-        xrow[t] = reinterpret_cast<const char*>(p.a) + (int64_t) (p.a_rows ? p.a_rows[m] : m) * p.lda * 2;
-    }
-    slim::product<W_BF16, MT, D, WAVES>(lds, reinterpret_cast<const char*>(p.w) + (int64_t) n0 * p.ldw * 2, p.ldw * 2, p.N - n0, p.K * 2, xrow,
+    const int lane = threadIdx.x & 63, n0 = blockIdx.x * S::cols;
+    slim::stream<W_BF16, S>(slim_lds, reinterpret_cast<const char*>(p.w) + (int64_t) n0 * p.ldw * 2, p.ldw * 2, p.N - n0, p.K * 2,
+        [&](int m) {
+            m = m < p.M ? m : p.M - 1;
+            return reinterpret_cast<const char*>(p.a) + (int64_t) (p.a_rows ? p.a_rows[m] : m) * p.lda * 2;
+        },
         [&](int t, const slim::f32x4& acc) {
-            const int row = 16 * t + (lane & 15), col = n0 + 4 * (lane >> 4);
-            if (row >= p.M)
+            const int row = 16 * t + (lane & 15), c = 4 * (lane >> 4), col = n0 + c;
+            if (row >= p.M || row >= S::mt * S::cols || c >= S::cols)
                 return;
             if (col < p.N)
                 seam_pair<DT_BF16>(p, row, col, acc[0], acc[1]);
@@ -385,10 +381,13 @@ __global__ __launch_bounds__(WAVES * 64) void slim_kernel(const StackGemmParams 
         });
 }
 
-template <int MT, int D, int WAVES>
 void launch_slim(const StackGemmParams& p, int products, int groups, hipStream_t stream)
 {
-    hipLaunchKernelGGL((slim_kernel<MT, D, WAVES>), dim3((p.N + 15) / 16, 1, products), dim3(WAVES * 64), 0, stream, p, groups);
+    slim::pick_shape(p.M, p.N, products, (int64_t) p.K * 2, p.group_off != nullptr, launch_util::device_cus(), [&](auto shape) {
+        using S = decltype(shape);
+        launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(&slim_kernel<S>), S::lds_bytes);
+        hipLaunchKernelGGL((slim_kernel<S>), dim3((p.N + S::cols - 1) / S::cols, 1, products), dim3(S::waves * 64), S::lds_bytes, stream, p, groups);
+    });
 }
 
 // Several rows through few columns (a token input's gate): a workgroup per SK_R rows of W whose 4 waves split K; their sums meet in LDS.
@@ -559,7 +558,6 @@ int launch_stack_gemm(const StackGemmParams& p_in, hipStream_t stream)
         // a grouped step of few rows: as many products as groups can have rows
         const bool few = p.group_off && p.group_total < p.batch;
         const int products = few ? p.group_total : p.batch, groups = few ? p.batch : 0;
-        const int64_t slim_wgs = (int64_t) ((p.N + 15) / 16) * products;
         if (p.M <= 1)
         {
             launch_row(p, products, groups, stream);
@@ -575,11 +573,7 @@ int launch_stack_gemm(const StackGemmParams& p_in, hipStream_t stream)
                 hipLaunchKernelGGL((skinny_ksplit_kernel<8>), kg, dim3(256), 0, stream, p);
             return launched("stack_gemm skinny (K over waves)");
         }
-        const bool many = slim_wgs * 4 >= cus * 5; // (gemm_slim_impl.h)
-        if (p.M <= 16)
-            many ? launch_slim<1, 1, 4>(p, products, groups, stream) : launch_slim<1, 2, 8>(p, products, groups, stream);
-        else
-            many ? launch_slim<2, 1, 4>(p, products, groups, stream) : launch_slim<2, 1, 8>(p, products, groups, stream);
+        launch_slim(p, products, groups, stream);
         return launched("stack_gemm slim");
     }
     const int64_t tiles128 = (int64_t) ((p.M + 127) / 128) * ((p.N + 127) / 128);
