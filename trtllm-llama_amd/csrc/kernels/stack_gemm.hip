@@ -17,6 +17,7 @@
 #include "gemm_seam.h"
 #include "gemm_slim_impl.h"
 #include "stack_kernels.h"
+#include "stack_route_impl.h"
 
 namespace tllm
 {
@@ -244,17 +245,11 @@ __device__ __forceinline__ void row_seam(const StackGemmParams& p, const RowSeam
     }
 }
 
-template <int KS, int NC>
-__global__ __launch_bounds__(256) void row_kernel(const StackGemmParams p_in, int groups)
+// SCALED: the row counts as scale times itself, rounded to bfloat16.  part: LDS
+template <int KS, int NC, bool SCALED>
+__device__ __forceinline__ void row_product(const StackGemmParams& p, float scale, float (&part)[4][SK_R])
 {
     constexpr int TEAMS = 4 / KS;
-    __shared__ float part[4][SK_R];
-    int b = blockIdx.z, first = -1, rows = 0;
-    if (groups && (b = nth_group(p_in.group_off, groups, b, first, rows)) < 0)
-        return;
-    const StackGemmParams p = batch_slice<DT_BF16>(p_in, b, first, rows);
-    if (p.M <= 0)
-        return;
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kw = wid % KS;
     const int n0 = (blockIdx.x * TEAMS + wid / KS) * SK_R; // (a team beyond N repeats the last row and stores nothing)
@@ -282,7 +277,11 @@ __global__ __launch_bounds__(256) void row_kernel(const StackGemmParams p_in, in
         for (int i = 0; i < NC; ++i)
         {
             const bool in = (c0 + i * KS) * 512 + lane * 8 < p.K; // (no branch: behind one the compiler would request a chunk where it is used)
-            const uint32_t xs[4] = {in ? xv[i].x : 0u, in ? xv[i].y : 0u, in ? xv[i].z : 0u, in ? xv[i].w : 0u};
+            uint32_t xs[4] = {in ? xv[i].x : 0u, in ? xv[i].y : 0u, in ? xv[i].z : 0u, in ? xv[i].w : 0u};
+            if constexpr (SCALED)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    xs[q] = (uint32_t) f2bf(scale * __builtin_bit_cast(float, xs[q] << 16)) | ((uint32_t) f2bf(scale * __builtin_bit_cast(float, xs[q] & 0xffff0000u)) << 16);
 #pragma unroll
             for (int r = 0; r < SK_R; ++r)
             {
@@ -323,34 +322,98 @@ __global__ __launch_bounds__(256) void row_kernel(const StackGemmParams p_in, in
     }
 }
 
+template <int KS, int NC>
+__global__ __launch_bounds__(256) void row_kernel(const StackGemmParams p_in, int groups)
+{
+    __shared__ float part[4][SK_R];
+    int b = blockIdx.z, first = -1, rows = 0;
+    if (groups && (b = nth_group(p_in.group_off, groups, b, first, rows)) < 0)
+        return;
+    const StackGemmParams p = batch_slice<DT_BF16>(p_in, b, first, rows);
+    if (p.M > 0)
+        row_product<KS, NC, false>(p, 1.f, part);
+}
+
+// A lone token's experts, product z = choice z.  up: every wave chooses from the logits by itself (some 0.8 us in front of its weights' requests), which
+// replaces a launch that orders pairs: a last workgroup that waits for all logits, chooses, orders and copies.  Choice, order and products of
+// a layer of 32 + 2 outputs, width 2048, in a step of one token: 9.5 us for the router's launch, 4.9 for its logits alone.
+template <int KS, int NC>
+__global__ __launch_bounds__(256) void lone_up_kernel(const StackGemmParams p_in, const StackMoeParams m)
+{
+    __shared__ float part[4][SK_R];
+    const int lane = threadIdx.x & 63, z = blockIdx.z, o = lane < m.experts + m.identity ? lane : 0;
+    const Chosen c = choose_in_wave(m, m.logits[o] + (m.bias ? m.bias[o] : 0.f), m.correction ? m.correction[o] : 0.f, lane);
+    if (blockIdx.x == 0 && z == 0 && (int) threadIdx.x < m.top)
+    {
+        m.topk_idx[lane] = c.output;
+        m.topk_w[lane] = c.weight;
+        m.slot_of_pair[lane] = c.output < m.experts ? lane : -1;
+    }
+    const int e = __builtin_amdgcn_readlane(c.output, z);
+    if (e >= m.experts)
+        return;
+    const float scale = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c.weight), z));
+    StackGemmParams p = p_in;
+    p.w = reinterpret_cast<const uint16_t*>(p.w) + e * p.stride_w;
+    p.c = reinterpret_cast<char*>(p.c) + z * p.ldc * (p.out_f32 ? 4 : 2);
+    if (m.weight_input)
+        row_product<KS, NC, true>(p, scale, part);
+    else
+        row_product<KS, NC, false>(p, 1.f, part);
+}
+
+template <int KS, int NC>
+__global__ __launch_bounds__(256) void lone_down_kernel(const StackGemmParams p_in, const int32_t* choice, int experts)
+{
+    __shared__ float part[4][SK_R];
+    const int z = blockIdx.z, e = choice[z];
+    if (e >= experts)
+        return;
+    StackGemmParams p = p_in;
+    p.a = reinterpret_cast<const uint16_t*>(p.a) + z * p.lda;
+    p.w = reinterpret_cast<const uint16_t*>(p.w) + e * p.stride_w;
+    p.c = reinterpret_cast<char*>(p.c) + z * p.ldc * (p.out_f32 ? 4 : 2);
+    row_product<KS, NC, false>(p, 1.f, part);
+}
+
 // A wave's chunks at once are all it has up to 12288 columns of A, then portions of 3.  Rows of up to 2048 columns are shared by 2 or 4 waves only where
 // that leaves the chip room to take all workgroups in at once; otherwise, and where a workgroup first looks up its group, a wave has rows of its own and a
 // workgroup lives longer (32000 x 2048 21.6 us by two waves a row, 22.2 by four; 4 grouped products of 2816 x 2048 10.3 against 12.1;
 // 2048 x 2048 4.8 by two, 4.6 by four).
+template <int KS_, int NC_>
+struct RowShape
+{
+    static constexpr int KS = KS_, NC = NC_, cols = SK_R * (4 / KS_);
+};
+template <class F>
+void pick_row_shape(int64_t n, int k, int products, bool looks_up, F f)
+{
+    const int chunks = (k + 511) / 512;
+    const bool many = looks_up || n * products > 16 * launch_util::device_cus();
+    if (chunks <= 1)
+        f(RowShape<1, 1>());
+    else if (chunks <= 2)
+        many ? f(RowShape<1, 2>()) : f(RowShape<2, 1>());
+    else if (chunks <= 3)
+        many ? f(RowShape<1, 3>()) : f(RowShape<4, 1>());
+    else if (chunks <= 4)
+        many ? f(RowShape<1, 4>()) : f(RowShape<4, 1>());
+    else if (chunks <= 8)
+        looks_up ? f(RowShape<2, 4>()) : f(RowShape<4, 2>());
+    else if (chunks <= 12 || chunks > 24)
+        f(RowShape<4, 3>());
+    else if (chunks <= 16)
+        f(RowShape<4, 4>());
+    else
+        f(RowShape<4, 6>());
+}
+
 void launch_row(const StackGemmParams& p, int products, int groups, hipStream_t stream)
 {
-    auto go = [&](auto kernel, int ks) {
-        const int cols = SK_R * (4 / ks);
-        hipLaunchKernelGGL(kernel, dim3((p.N + cols - 1) / cols, 1, products), dim3(256), 0, stream, p, groups);
-    };
-    const int chunks = (p.K + 511) / 512;
-    const bool many = p.group_off || (int64_t) p.N * products > 16 * launch_util::device_cus();
-    if (chunks <= 1)
-        go(row_kernel<1, 1>, 1);
-    else if (chunks <= 2)
-        many ? go(row_kernel<1, 2>, 1) : go(row_kernel<2, 1>, 2);
-    else if (chunks <= 3)
-        many ? go(row_kernel<1, 3>, 1) : go(row_kernel<4, 1>, 4);
-    else if (chunks <= 4)
-        many ? go(row_kernel<1, 4>, 1) : go(row_kernel<4, 1>, 4);
-    else if (chunks <= 8)
-        p.group_off ? go(row_kernel<2, 4>, 2) : go(row_kernel<4, 2>, 4);
-    else if (chunks <= 12 || chunks > 24)
-        go(row_kernel<4, 3>, 4);
-    else if (chunks <= 16)
-        go(row_kernel<4, 4>, 4);
-    else
-        go(row_kernel<4, 6>, 4);
+    pick_row_shape(p.N, p.K, products, p.group_off != nullptr, [&](auto shape) {
+        using S = decltype(shape);
+        hipLaunchKernelGGL((row_kernel<S::KS, S::NC>), dim3((p.N + S::cols - 1) / S::cols, 1, products), dim3(256), 0, stream, p, groups);
+    });
 }
 
 // bfloat16, 2 .. 31 rows: the main loop of gemm_slim_impl.h, a workgroup per S::cols columns and product
@@ -518,6 +581,39 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
 }
 
 } // namespace
+
+bool stack_lone_serves(const StackMoeParams& m, const StackGemmParams& up, const StackGemmParams& down)
+{
+    auto rows_of_pieces = [](const StackGemmParams& p) {
+        return p.K > 0 && p.N > 0 && p.K % 8 == 0 && p.lda % 8 == 0 && p.stride_w % 8 == 0 && p.ldw == 0 && p.c && !p.resid && !p.bias && p.seam.n_sec == 0
+            && !((reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.w)) & 15) && (p.act < ACT_GATE_SILU || !(p.N & 1));
+    };
+    return m.tokens == 1 && m.dtype == DT_BF16 && m.experts + m.identity <= LONE_OUT && rows_of_pieces(up) && rows_of_pieces(down);
+}
+
+int launch_stack_lone_up(const StackMoeParams& m, const StackGemmParams& p_in, hipStream_t stream)
+{
+    StackGemmParams p = p_in;
+    p.M = 1;
+    p.ldw = p.K;
+    pick_row_shape(p.N, p.K, m.top, true, [&](auto shape) {
+        using S = decltype(shape);
+        hipLaunchKernelGGL((lone_up_kernel<S::KS, S::NC>), dim3((p.N + S::cols - 1) / S::cols, 1, m.top), dim3(256), 0, stream, p, m);
+    });
+    return launched("stack_lone_up");
+}
+
+int launch_stack_lone_down(const StackMoeParams& m, const StackGemmParams& p_in, hipStream_t stream)
+{
+    StackGemmParams p = p_in;
+    p.M = 1;
+    p.ldw = p.K;
+    pick_row_shape(p.N, p.K, m.top, true, [&](auto shape) {
+        using S = decltype(shape);
+        hipLaunchKernelGGL((lone_down_kernel<S::KS, S::NC>), dim3((p.N + S::cols - 1) / S::cols, 1, m.top), dim3(256), 0, stream, p, m.topk_idx, m.experts);
+    });
+    return launched("stack_lone_down");
+}
 
 int launch_stack_gemm(const StackGemmParams& p_in, hipStream_t stream)
 {

@@ -3,6 +3,7 @@
 #include "dev_utils.h"
 #include "launch_util.h"
 #include "stack_kernels.h"
+#include "stack_route_impl.h"
 #include <algorithm>
 
 namespace tllm
@@ -41,28 +42,6 @@ inline int launched(const char* what)
         return -1;
     }
     return 0;
-}
-
-// the lane that holds the largest value of the wave, the lowest index among equals; every lane gets (value, index).  The maximum goes
-// through DPP moves, and a lane that holds it alone gives its index by a lane read: a twelve-shuffle tree costs twice the time of a choice.
-__device__ __forceinline__ void wave_argmax(float& v, int& idx)
-{
-    const float m = wave_max(v);
-    const uint64_t at = __ballot(v == m);
-    if (__popcll(at) == 1)
-        idx = __builtin_amdgcn_readlane(idx, (int) __builtin_ctzll(at));
-    else
-    {
-        int best = v == m ? idx : 0x7fffffff;
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1)
-        {
-            const int o = __shfl_xor(best, d, 64);
-            best = o < best ? o : best;
-        }
-        idx = best;
-    }
-    v = m;
 }
 
 constexpr int RT = 8;         // tokens per logits workgroup: a router row is read once for all of them
@@ -833,6 +812,20 @@ int launch_stack_moe_sort(const StackMoeParams& p, hipStream_t stream)
         return rc;
     hipLaunchKernelGGL(moe_gather_kernel, dim3(p.tokens * p.top), dim3(256), 0, stream, p, row_bytes);
     return launched("stack_moe_gather");
+}
+
+int launch_stack_moe_logits(const StackMoeParams& p, hipStream_t stream)
+{
+    if (p.tokens <= 0)
+        return 0;
+    if (!moe_ok(p, "stack_moe_logits"))
+        return -1;
+    const dim3 lg((p.experts + p.identity + 3) / 4, (p.tokens + RT - 1) / RT);
+    if (p.dtype == DT_BF16)
+        hipLaunchKernelGGL((moe_logits_kernel<DT_BF16>), lg, dim3(256), 0, stream, p, p.logits);
+    else
+        hipLaunchKernelGGL((moe_logits_kernel<DT_FLOAT>), lg, dim3(256), 0, stream, p, p.logits);
+    return launched("stack_moe_logits");
 }
 
 int launch_stack_moe_plan(const StackMoeParams& p, hipStream_t stream)

@@ -1813,8 +1813,6 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         mp.accumulate = accumulate ? 1 : 0;
         mp.accumulate_gate = l.shared_gate ? s->shared_z : nullptr;
         mp.y_el = y_el;
-        if (launch_stack_moe_plan(mp, stream))
-            return -1;
         // per expert: gate and up on its rows with silu(gate) * up (or relu(up)^2) in the epilogue, down in fp32; an expert's rows are at most one per token
         const int up_cols = l.expert_relu2 ? l.ff : 2 * l.ff;
         StackGemmParams u;
@@ -1834,8 +1832,6 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         u.group_off = mp.group_off;
         u.group_total = (int) pairs;
         u.group_rows = (int) std::min<int64_t>(T, (pairs + l.experts - 1) / l.experts);
-        if (launch_stack_gemm(u, stream))
-            return -1;
         StackGemmParams dn;
         dn.dtype = s->dtype;
         dn.out_f32 = 1;
@@ -1852,7 +1848,14 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         dn.group_off = mp.group_off;
         dn.group_total = u.group_total;
         dn.group_rows = u.group_rows;
-        if (launch_stack_gemm(dn, stream))
+        StackGemmParams lone = u; // (reads the token's row itself, also where it counts weighted)
+        lone.a = s->h1;
+        if (stack_lone_serves(mp, lone, dn))
+        {
+            if ((!mp.have_logits && launch_stack_moe_logits(mp, stream)) || launch_stack_lone_up(mp, lone, stream) || launch_stack_lone_down(mp, dn, stream))
+                return -1;
+        }
+        else if (launch_stack_moe_plan(mp, stream) || launch_stack_gemm(u, stream) || launch_stack_gemm(dn, stream))
             return -1;
         if (!later)
             return launch_stack_moe_combine(mp, s->moe_y, y, stream);
