@@ -1,0 +1,18 @@
+"""Grouped bfloat16 products whose groups fit one 256-row tile (launch_glds_bf16 of stack_gemm.hip takes 256 x 256 tiles where that saves a round of
+workgroups: 8 groups of 200 rows on average x 8176 columns on 256 CUs): groups that end inside the tile, columns that end inside it, one stage of K and
+several.  Bounds as in test_gpu_product_tiles."""
+import pytest
+
+import ruzinex_cases as Z
+import test_gpu_ruzinex as R
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('rows', [752, 800])
+@pytest.mark.parametrize('k', [64, 320])
+def test_groups_of_one_wide_tile(k, rows):
+    cfg = Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=Z.moe(experts=8, top=2, ff=4088, shared=0))], width=k)
+    toks = R.tokens_for(cfg, rows, 97)
+    w = R.weights_for(cfg, 98, 'bfloat16', toks)
+    R.check_rows(R.replay(R.session_for(cfg, w, 'bfloat16'), {'a': toks}, [[('a', rows)]])['a'], toks, w, cfg, 'bfloat16')
