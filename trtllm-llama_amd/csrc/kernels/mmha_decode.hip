@@ -452,7 +452,15 @@ __global__ __launch_bounds__(256) void mmha_partial_kernel(const MmhaParams p, f
             L += sm_l[g] * sm_w[g];
             O += sm_o[g][d] * sm_w[g];
         }
-        if (tail)
+        if (tail && nact == 1) // uniform
+        {
+            const uint16_t h16 = f2h(O * (1.f / (L + 1.e-6f))); // (what the merge makes of one partial)
+            const int64_t o = ((int64_t) b * H + h) * DH + d;
+            reinterpret_cast<uint16_t*>(p.out)[o] = h16;
+            if (p.tail_out_q8)
+                reinterpret_cast<int8_t*>(p.tail_out_q8)[o] = f2i8_rni_sat(h2f(h16) * p.tail_quant_scale[0]);
+        }
+        else if (tail)
         {
             sm_out[d] = O;
             if (d == 0) // (m, l) as ONE 8-byte write-through store
@@ -466,7 +474,9 @@ __global__ __launch_bounds__(256) void mmha_partial_kernel(const MmhaParams p, f
                 ws_ml[pi] = make_float2(M, L);
         }
     }
-    if (!tail)
+    // A sequence within one split has nothing to merge: it leaves at once, without the stores, the ticket and the loads below, 1.6 us of a launch's 7.6
+    // at 8 heads and 10 tokens.
+    if (!tail || nact == 1)
         return;
     // write-through (sc1) 16-byte stores of the partial: the merging workgroup may sit on another XCD, whose L2 never sees this
     // one's; scalar write-through stores are one fabric write each (guide: dword ~6 x the dwordx4 time per byte)

@@ -1738,6 +1738,9 @@ int32_t tllm_session_setup_beam(tllm_session_t s, int32_t batch_size, int32_t be
             s->attn_nit = 16;
             if (mmha_split_layout(s->Dh, Smax, 12, B, s->Hr, &tc, &ns, &off) == 0 && ns <= 8)
                 s->attn_nit = 12;
+            // (a cache within one split of the shortest form: its code is a third of the others', and a launch of few cycles is bound by fetching it)
+            if (mmha_split_layout(s->Dh, Smax, 4, B, s->Hr, &tc, &ns, &off) == 0 && ns == 1)
+                s->attn_nit = 4;
             s->attn_tail = true;
             RUN(s->dalloc(reinterpret_cast<void**>(&s->attn_tickets), (size_t) B * s->Hr * 4));
             HIP_OK(hipMemset(s->attn_tickets, 0, (size_t) B * s->Hr * 4));
