@@ -52,12 +52,12 @@ constexpr int FEW_TOKENS = RT; // steps of this many tokens or fewer are routed 
 
 // acc[r] = this lane's share of router row e times the rows t0 .. t0 + nt of h; lanes split the width in float4 pieces where rows are
 // 16-byte aligned
-template <int DT>
-__device__ __forceinline__ void router_row(const StackMoeParams& p, int e, int t0, int nt, int lane, float (&acc)[RT])
+template <int DT, int NR = RT>
+__device__ __forceinline__ void router_row(const StackMoeParams& p, int e, int t0, int nt, int lane, float (&acc)[NR])
 {
     const int W = p.width;
 #pragma unroll
-    for (int r = 0; r < RT; ++r)
+    for (int r = 0; r < NR; ++r)
         acc[r] = 0.f;
     const float* wr = p.router_w + (int64_t) e * W;
     if ((W & 7) == 0)
@@ -75,7 +75,7 @@ __device__ __forceinline__ void router_row(const StackMoeParams& p, int e, int t
                 w[a][1] = *reinterpret_cast<const float4*>(wr + k + 4);
             }
 #pragma unroll
-            for (int r = 0; r < RT; ++r)
+            for (int r = 0; r < NR; ++r)
             {
                 if (r >= nt)
                     break;
@@ -122,26 +122,27 @@ __device__ __forceinline__ void router_row(const StackMoeParams& p, int e, int t
         {
             const float wv = wr[k];
 #pragma unroll
-            for (int r = 0; r < RT; ++r)
+            for (int r = 0; r < NR; ++r)
                 if (r < nt)
                     acc[r] = fmaf(wv, ld_el<DT>(p.h, (int64_t) (t0 + r) * W + k), acc[r]);
         }
     }
 }
 
-// Router logits, fp32: workgroup (x, y) = 4 router rows (one per wave) x RT tokens.  z [tokens, outputs].
-template <int DT>
+// Router logits, fp32: workgroup (x, y) = 4 router rows (one per wave) x NR tokens (one: a lone token's, without the
+// code of eight, which such a launch spends its time fetching).  z [tokens, outputs].
+template <int DT, int NR>
 __global__ __launch_bounds__(256) void moe_logits_kernel(const StackMoeParams p, float* z)
 {
     const int NE = p.experts + p.identity;
-    const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, t0 = blockIdx.y * RT;
+    const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, t0 = blockIdx.y * NR;
     if (e >= NE)
         return;
-    const int nt = p.tokens - t0 < RT ? p.tokens - t0 : RT;
-    float acc[RT];
-    router_row<DT>(p, e, t0, nt, lane, acc);
+    const int nt = NR > 1 && p.tokens - t0 < NR ? p.tokens - t0 : NR;
+    float acc[NR];
+    router_row<DT, NR>(p, e, t0, nt, lane, acc);
 #pragma unroll
-    for (int r = 0; r < RT; ++r)
+    for (int r = 0; r < NR; ++r)
     {
         const float sum = wave_sum(acc[r]);
         if (lane == 0 && r < nt)
@@ -783,9 +784,9 @@ int launch_stack_moe_route(const StackMoeParams& p, hipStream_t stream)
             hipLaunchKernelGGL((moe_logits_mfma_kernel<DT_FLOAT>), mg, dim3(512), 0, stream, p, p.logits);
     }
     else if (p.dtype == DT_BF16)
-        hipLaunchKernelGGL((moe_logits_kernel<DT_BF16>), lg, dim3(256), 0, stream, p, p.logits);
+        hipLaunchKernelGGL((moe_logits_kernel<DT_BF16, RT>), lg, dim3(256), 0, stream, p, p.logits);
     else
-        hipLaunchKernelGGL((moe_logits_kernel<DT_FLOAT>), lg, dim3(256), 0, stream, p, p.logits);
+        hipLaunchKernelGGL((moe_logits_kernel<DT_FLOAT, RT>), lg, dim3(256), 0, stream, p, p.logits);
     if (launched("stack_moe_logits"))
         return -1;
     hipLaunchKernelGGL(moe_select_kernel, dim3((p.tokens + 3) / 4), dim3(256), sizeof(float) * 2 * 4 * NE, stream, p, p.logits);
@@ -820,11 +821,11 @@ int launch_stack_moe_logits(const StackMoeParams& p, hipStream_t stream)
         return 0;
     if (!moe_ok(p, "stack_moe_logits"))
         return -1;
-    const dim3 lg((p.experts + p.identity + 3) / 4, (p.tokens + RT - 1) / RT);
+    const dim3 lg((p.experts + p.identity + 3) / 4, p.tokens);
     if (p.dtype == DT_BF16)
-        hipLaunchKernelGGL((moe_logits_kernel<DT_BF16>), lg, dim3(256), 0, stream, p, p.logits);
+        hipLaunchKernelGGL((moe_logits_kernel<DT_BF16, 1>), lg, dim3(256), 0, stream, p, p.logits);
     else
-        hipLaunchKernelGGL((moe_logits_kernel<DT_FLOAT>), lg, dim3(256), 0, stream, p, p.logits);
+        hipLaunchKernelGGL((moe_logits_kernel<DT_FLOAT, 1>), lg, dim3(256), 0, stream, p, p.logits);
     return launched("stack_moe_logits");
 }
 

@@ -1589,20 +1589,22 @@ __device__ __forceinline__ void expert_sum(const StackExpertSum& m, int t, int w
     }
 }
 
-// The form for rows of a multiple of 4 up to HV_K * 4096 elements: up to 1024 threads, a thread owns HV_K float4 columns of every
+// The form for rows of a multiple of 4 up to HV_K * 4096 elements: up to 1024 threads, a thread owns K float4 columns of every
 // stream and has ALL of them in flight before its first store (the streams are read and written through the same pointer, so in
-// a loop every store would fence the loads behind it); the combined row stays in registers.
+// a loop every store would fence the loads behind it); the combined row stays in registers.  SUM: y may be a sum that is still to be formed.  In a
+// decode step such a launch comes once between streams of weights and is bound by fetching its code, some 0.3 us a KiB, so that neither a second
+// column nor the sum is compiled in where it is not needed.
 constexpr int HV_K = 2;
 
-template <int DT, int SM>
+template <int DT, int SM, int K, bool SUM>
 __global__ __launch_bounds__(1024) void hyper_norm_vec_kernel(const StackHyperParams p)
 {
     __shared__ float red[32];
     const int t = p.rows ? p.rows[blockIdx.x] : blockIdx.x, tid = threadIdx.x, S = p.streams, W4 = p.width >> 2, NT = blockDim.x;
     constexpr bool EARLY = SM <= 2; // the norm's weights come in with the row (more streams: no registers left for them)
-    float4 xs[HV_K][SM], yv[HV_K], u[HV_K], wv[HV_K];
+    float4 xs[K][SM], yv[K], u[K], wv[K];
 #pragma unroll
-    for (int k = 0; k < HV_K; ++k)
+    for (int k = 0; k < K; ++k)
     {
         const int c4 = tid + k * NT;
         yv[k] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1610,13 +1612,14 @@ __global__ __launch_bounds__(1024) void hyper_norm_vec_kernel(const StackHyperPa
         for (int s = 0; s < SM; ++s)
             xs[k][s] = (s < S && c4 < W4) ? reinterpret_cast<const float4*>(p.x + s * p.stream_stride + (int64_t) t * p.width)[c4]
                                           : make_float4(0.f, 0.f, 0.f, 0.f);
-        if (p.y && c4 < W4 && (!p.sum.ys || p.sum.has_row))
+        if (p.y && c4 < W4 && (!SUM || !p.sum.ys || p.sum.has_row))
             yv[k] = reinterpret_cast<const float4*>(p.y + (int64_t) t * p.width)[c4];
         if (EARLY)
             wv[k] = p.w && c4 < W4 ? reinterpret_cast<const float4*>(p.w)[c4] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    if (p.y && p.sum.ys)
-        expert_sum<DT, HV_K>(p.sum, t, p.width, tid, NT, yv);
+    if constexpr (SUM)
+        if (p.y && p.sum.ys)
+            expert_sum<DT, K>(p.sum, t, p.width, tid, NT, yv);
     float cm[SM][SM], co[SM], ci[SM];
 #pragma unroll
     for (int a = 0; a < SM; ++a)
@@ -1629,7 +1632,7 @@ __global__ __launch_bounds__(1024) void hyper_norm_vec_kernel(const StackHyperPa
     }
     float ss = 0.f;
 #pragma unroll
-    for (int k = 0; k < HV_K; ++k)
+    for (int k = 0; k < K; ++k)
     {
         const int c4 = tid + k * NT;
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1670,7 +1673,7 @@ __global__ __launch_bounds__(1024) void hyper_norm_vec_kernel(const StackHyperPa
     ss = block_sum(ss, red);
     const float inv = 1.f / sqrtf(ss / (float) p.width + p.eps);
 #pragma unroll
-    for (int k = 0; k < HV_K; ++k)
+    for (int k = 0; k < K; ++k)
     {
         const int c4 = tid + k * NT;
         if (c4 < W4)
@@ -1695,14 +1698,17 @@ __global__ __launch_bounds__(1024) void hyper_norm_vec_kernel(const StackHyperPa
 template <int DT>
 void launch_hyper_vec(const StackHyperParams& p, int nt, hipStream_t stream)
 {
-    if (p.streams <= 1)
-        hipLaunchKernelGGL((hyper_norm_vec_kernel<DT, 1>), dim3(p.tokens), dim3(nt), 0, stream, p);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.tokens), dim3(nt), 0, stream, p); };
+    if (p.streams <= 1 && p.width <= 4096)
+        p.sum.ys ? go(hyper_norm_vec_kernel<DT, 1, 1, true>) : go(hyper_norm_vec_kernel<DT, 1, 1, false>);
+    else if (p.streams <= 1)
+        go(hyper_norm_vec_kernel<DT, 1, HV_K, true>);
     else if (p.streams <= 2)
-        hipLaunchKernelGGL((hyper_norm_vec_kernel<DT, 2>), dim3(p.tokens), dim3(nt), 0, stream, p);
+        go(hyper_norm_vec_kernel<DT, 2, HV_K, true>);
     else if (p.streams <= 4)
-        hipLaunchKernelGGL((hyper_norm_vec_kernel<DT, 4>), dim3(p.tokens), dim3(nt), 0, stream, p);
+        go(hyper_norm_vec_kernel<DT, 4, HV_K, true>);
     else
-        hipLaunchKernelGGL((hyper_norm_vec_kernel<DT, 8>), dim3(p.tokens), dim3(nt), 0, stream, p);
+        go(hyper_norm_vec_kernel<DT, 8, HV_K, true>);
 }
 
 // One plain residual stream (StackLandParams): a row stays in registers between its loads, the norm of what lands, the addition and
@@ -1720,8 +1726,8 @@ __device__ __forceinline__ float4 land_table4(const void* table, int64_t i)
         return *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(table) + i);
 }
 
-// K float4 pieces of the row per thread
-template <int DT, int K>
+// K float4 pieces of the row per thread; SUM: as above
+template <int DT, int K, bool SUM>
 __global__ __launch_bounds__(1024) void land_vec_kernel(const StackLandParams p)
 {
     __shared__ float red[32], red2[32];
@@ -1748,13 +1754,13 @@ __global__ __launch_bounds__(1024) void land_vec_kernel(const StackLandParams p)
             u[k] = land_table4<DT>(p.table, trow + 4 * c4);
             u[k].x *= p.scale, u[k].y *= p.scale, u[k].z *= p.scale, u[k].w *= p.scale;
         }
-        else if (on && p.y && (!p.sum.ys || p.sum.has_row))
+        else if (on && p.y && (!SUM || p.sum.has_row))
             u[k] = reinterpret_cast<const float4*>(p.y + row)[c4];
         yn[k] = on && p.y_norm ? reinterpret_cast<const float4*>(p.y_norm)[c4] : zero;
         ar[k] = on && p.add_row ? reinterpret_cast<const float4*>(p.add_row)[c4] : zero;
         wv[k] = on && p.w ? reinterpret_cast<const float4*>(p.w)[c4] : zero;
     }
-    if (p.sum.ys)
+    if constexpr (SUM)
         expert_sum<DT, K>(p.sum, t, p.width, tid, NT, u);
     if (p.y_norm)
     {
@@ -1904,16 +1910,15 @@ int launch_stack_land(const StackLandParams& p_in, hipStream_t stream)
     {
         const int k = p.width > 4096 || p.tokens >= 64 ? 2 : 1; // many rows: fewer waves meet at a row's barriers
         const int nt = std::min(1024, (p.width / 4 + 64 * k - 1) / (64 * k) * 64);
-#define TLLM_LAND(DT, K) hipLaunchKernelGGL((land_vec_kernel<DT, K>), dim3(p.tokens), dim3(nt), 0, stream, p)
+auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.tokens), dim3(nt), 0, stream, p); };
         if (p.dtype == DT_BF16 && k == 1)
-            TLLM_LAND(DT_BF16, 1);
+            p.sum.ys ? go(land_vec_kernel<DT_BF16, 1, true>) : go(land_vec_kernel<DT_BF16, 1, false>);
         else if (p.dtype == DT_BF16)
-            TLLM_LAND(DT_BF16, 2);
+            p.sum.ys ? go(land_vec_kernel<DT_BF16, 2, true>) : go(land_vec_kernel<DT_BF16, 2, false>);
         else if (k == 1)
-            TLLM_LAND(DT_FLOAT, 1);
+            p.sum.ys ? go(land_vec_kernel<DT_FLOAT, 1, true>) : go(land_vec_kernel<DT_FLOAT, 1, false>);
         else
-            TLLM_LAND(DT_FLOAT, 2);
-#undef TLLM_LAND
+            p.sum.ys ? go(land_vec_kernel<DT_FLOAT, 2, true>) : go(land_vec_kernel<DT_FLOAT, 2, false>);
         return launched("stack_land");
     }
     if (p.sum.ys && form_expert_sum(p.sum, p.y, p.dtype, p.width, stream))
