@@ -1,6 +1,6 @@
 // Products of few rows on the LLaMA path: fp16, SmoothQuant int8, weight-only int8 / int4 weights through the weight-streaming main loop of
 // gemm_slim_impl.h.  Short prompts and plain calls of 5 .. 31 rows (int4 weights 3 .. 31), generation steps of 5 .. 32 sequences with fp16 or
-// weight-only weights (int4 3 .. 32).  The epilogue has the rounding points of the tiles in gemm_mfma.hip.  The sums' order is not the
+// weight-only weights (int4 3 .. 32; fp16 products without a norm ahead or SwiGLU behind from 3).  The epilogue has the rounding points of the tiles in gemm_mfma.hip.  The sums' order is not the
 // streaming GEMV's, which serves fewer rows: a sequence's fp16 rows differ in their last bits with the number of rows beside it.
 #include "gemm_slim_impl.h"
 #include "kernels.h"
@@ -135,9 +135,10 @@ int launch_wt(const GemmParams& p, hipStream_t stream)
 } // namespace
 
 // Rows from which this form is the quicker one (the streaming GEMV's time grows with the rows: dot products on the vector pipe, and LDS for
-// every row's activations).  Cold weights, us at 4 / 5 / 8 rows by the GEMV and at 9 here: fp16 4096 x 4096 9.3 / 11.5 / 12.0, 9.8; fp16
-// 4096 x 11008 19.9 / 36.8 / 39.3, 19.8; SmoothQuant 4096 x 11008 12.9 / 15.5 / 16.5, 12.7; int8 weights 12288 x 4096 16.0 / 28.6 / 28.9,
-// 16.8; int4 weights 12288 x 4096 at 2 / 4 / 5 rows 16.4 / 31.5 / 195, 15.0.
+// every row's activations).  Cold weights, us at 4 / 5 / 8 rows by the GEMV and at 8 here (timed with bfloat16): fp16 4096 x 4096 9.3 / 11.5 /
+// 12.0, 7.8; fp16 4096 x 11008 19.9 / 36.8 / 39.3, 18.7 (from 3 rows where there is nothing but the product to do: session.cpp's gemv); at 9
+// here: SmoothQuant 4096 x 11008 12.9 / 15.5 / 16.5, 12.7; int8 weights 12288 x 4096 16.0 / 28.6 / 28.9, 16.8; int4 weights 12288 x 4096 at
+// 2 / 4 / 5 rows 16.4 / 31.5 / 195, 15.0.
 int gemm_slim_rows(int wtype)
 {
     return wtype == W_INT4_WOQ ? 3 : 5;

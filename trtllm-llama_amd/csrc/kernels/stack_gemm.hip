@@ -4,14 +4,16 @@
 //                     (v_mfma_f32_32x32x16_bf16), tile shape by the same rounds x area rule as the fp16 form;
 //   bfloat16, other M >= 32: the register-staged MFMA tiles of gemm_mfma.hip;
 //   bfloat16, M <= 31: slim_kernel below - HBM-bound, the weight-streaming MFMA main loop of gemm_slim_impl.h;
-//   bfloat16, M = 1:  row_kernel - dot products on the vector pipe, K split over a workgroup's waves; fp32 accumulation, DPP reduction;
-//   bfloat16, 2 <= M <= 8, few columns: skinny_ksplit_kernel, the same for several rows;
+//   bfloat16, M = 1:  row_kernel - dot products on the vector pipe, K split over a workgroup's waves; fp32 accumulation, DPP reduction
+//                     (a lone token's experts: lone_up_kernel, lone_down_kernel);
+//   bfloat16, 2 <= M <= 8, few columns of long rows: skinny_ksplit_kernel, the same for several rows;
 //   float32         : fma_tile_kernel - 64 x 64 tiles of plain fp32 FMAs through LDS (no reduced-precision matrix mode), any shape;
 //                     also the fallback for bfloat16 operands whose rows are not 16-byte aligned.
 //
 // A row's fp32 sums run in the order of the form that serves the call, so its last bits follow the rows beside it: one row, 2 .. 31 and more are
-// different orders in bfloat16, a grouped product of few rows splits K over 4 or 8 waves by how many products the launch holds, and a
-// product of few tiles is cut along K by how many there are.  Rows of one launch do not depend on each other.
+// different orders in bfloat16, one of 2 .. 31 splits K over 2, 4 or 8 waves by its rows and by how many workgroups its launch holds
+// (slim::pick_shape), one row's over 1 .. 4 by its columns and products (pick_row_shape), and a product of few tiles is cut along K by how many
+// there are.  Rows of one launch do not depend on each other.
 #include "dev_utils.h"
 #include "gemm_glds_impl.h"
 #include "gemm_seam.h"
@@ -337,7 +339,7 @@ __global__ __launch_bounds__(256) void row_kernel(const StackGemmParams p_in, in
 
 // A lone token's experts, product z = choice z.  up: every wave chooses from the logits by itself (some 0.8 us in front of its weights' requests), which
 // replaces a launch that orders pairs: a last workgroup that waits for all logits, chooses, orders and copies.  Choice, order and products of
-// a layer of 32 + 2 outputs, width 2048, in a step of one token: 9.5 us for the router's launch, 4.9 for its logits alone.
+// a layer of 32 + 2 outputs, width 2048, in a step of one token: 9.5 us for the router's launch, 3.7 for its logits alone.
 template <int KS, int NC>
 __global__ __launch_bounds__(256) void lone_up_kernel(const StackGemmParams p_in, const StackMoeParams m)
 {
@@ -672,7 +674,8 @@ int launch_stack_gemm(const StackGemmParams& p_in, hipStream_t stream)
         }
         if (p.batch == 1 && !p.group_off && p.M <= 8 && (p.N + 7) / 8 * 2 <= cus && p.K >= 2048)
         {
-            // 1024 x 2048: 4.0 / 5.2 us at four / eight rows, the MFMA form 5.1 .. 6.2
+            // us at 2 / 4 / 8 rows, in brackets slim_kernel: 256 x 2048 3.5 / 3.6 / 4.5 (4.8 / 4.8 / 4.9), 1024 x 2048 3.9 / 4.1 / 5.1 (5.0 / 5.0 / 5.1),
+            // 1024 x 4096 5.0 / 5.3 / 6.7 (6.3 / 6.3 / 6.5)
             const dim3 kg((p.N + SK_R - 1) / SK_R);
             if (p.M <= 4)
                 hipLaunchKernelGGL((skinny_ksplit_kernel<4>), kg, dim3(256), 0, stream, p);

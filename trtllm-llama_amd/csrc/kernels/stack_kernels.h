@@ -21,7 +21,7 @@ constexpr int32_t DT_BF16 = 7; // nvinfer1::DataType::kBF16
 
 // ---------------------------------------------------------------------------------------------
 // Dense product C[m,n] = sum_k A[m,k] * W[n,k] for the stack engine, with the layer's seam in the epilogue.
-//   dtype DT_BF16: MFMA tiles (gemm_mfma.hip, v_mfma_f32_32x32x16_bf16) for M > 8, the streaming skinny kernel below it;
+//   dtype DT_BF16: MFMA tiles (v_mfma_f32_32x32x16_bf16) for M >= 32, weight-streaming kernels below it (stack_gemm.hip);
 //   dtype DT_FLOAT: fp32 FMA tiles (stack_gemm.hip).
 // Epilogue, when `resid` is set: resid[m, n] += sigmoid(gate[m, n] + gate_bias[n]) * C[m, n]  (fp32 residual stream, the
 // sublayer's gate taken from another projection's columns); nothing is written to `c` then.  Otherwise `bias` (fp32 [N]) is added
