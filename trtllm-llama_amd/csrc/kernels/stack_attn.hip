@@ -136,39 +136,42 @@ __device__ __forceinline__ int walk_block(const BlockWalk& w, int v)
 
 // Scores of one 32-key block of one map -> its P^T fragment, with the online-softmax state of the lane's query row brought up to
 // date.  `masked` is wave-uniform: only blocks that reach past the first row's position, or start before the last row's first
-// visible key, compare keys with positions.
+// visible key, compare keys with positions.  Each option is one branch around its eight scores: with the options tested score by score the
+// loop held two scalar branches per score and option, and the code of options that a model does not have was fetched all the same (attn_tile_kernel of
+// two maps of 64 x 128 14.9 KB, 10.2 this way with the split form on its own; prompts of latent keys 320 x 256, 1021 rows 58.4 -> 49.5 us, 2048 rows
+// 110.9 -> 94.7, three of 1021 rows in the wide form 189.9 -> 163.4).
 template <int VT>
 __device__ __forceinline__ uint4 softmax_block(f32x4 (&s)[2], float& m_run, float& l_run, f32x4 (&acc)[VT], const HeadMods& hm, bool masked,
     int key_lane0, int qpos, int klo)
 {
-    float bm = -INFINITY;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
+#define EACH_SCORE _Pragma("unroll") for (int t = 0; t < 2; ++t) _Pragma("unroll") for (int i = 0; i < 4; ++i)
+    if (hm.cap2 > 0.f)
+    {
+        // cap * tanh(x / cap) with tanh(y) = (e^{2y} - 1) / (e^{2y} + 1); cap_arg = scale / cap * 2 log2 e
+        EACH_SCORE
         {
-            float v;
-            if (hm.cap2 > 0.f)
-            {
-                // cap * tanh(x / cap) with tanh(y) = (e^{2y} - 1) / (e^{2y} + 1); cap_arg = scale / cap * 2 log2 e
-                const float t2 = __builtin_amdgcn_exp2f(fminf(fmaxf(s[t][i] * hm.cap_arg, -43.f), 43.f));
-                v = hm.cap2 * (t2 - 1.f) * __builtin_amdgcn_rcpf(t2 + 1.f);
-            }
-            else
-                v = s[t][i] * hm.scale2;
-            const int kidx = key_lane0 + t * 16 + i;
-            if (hm.pen)
-            {
-                const float dist = (float) (qpos - kidx);
-                v -= hm.slope2 * dist;
-                if (hm.r1 != 0.f)
-                    v -= hm.r1 * __builtin_amdgcn_logf(fmaxf(1.f + hm.r2 * dist, 1e-30f));
-            }
-            if (masked && (kidx > qpos || (kidx < klo && kidx >= hm.keep)))
-                v = -INFINITY;
-            s[t][i] = v;
-            bm = fmaxf(bm, v);
+            const float t2 = __builtin_amdgcn_exp2f(fminf(fmaxf(s[t][i] * hm.cap_arg, -43.f), 43.f));
+            s[t][i] = hm.cap2 * (t2 - 1.f) * __builtin_amdgcn_rcpf(t2 + 1.f);
         }
+    }
+    else
+        EACH_SCORE s[t][i] *= hm.scale2;
+    if (hm.pen)
+    {
+        EACH_SCORE s[t][i] -= hm.slope2 * (float) (qpos - (key_lane0 + t * 16 + i));
+        if (hm.r1 != 0.f)
+            EACH_SCORE s[t][i] -= hm.r1 * __builtin_amdgcn_logf(fmaxf(1.f + hm.r2 * (float) (qpos - (key_lane0 + t * 16 + i)), 1e-30f));
+    }
+    if (masked)
+        EACH_SCORE
+        {
+            const int kidx = key_lane0 + t * 16 + i;
+            if (kidx > qpos || (kidx < klo && kidx >= hm.keep))
+                s[t][i] = -INFINITY;
+        }
+    float bm = -INFINITY;
+    EACH_SCORE bm = fmaxf(bm, s[t][i]);
+#undef EACH_SCORE
     if (hm.sigm)
     {
         // every key's weight stands alone: 1 / (1 + 2^-(score2 + offset2)); a hidden key's is 2^-inf = 0
@@ -227,17 +230,20 @@ __device__ __forceinline__ float out_gate_of(const StackAttnParams& p, int64_t t
     return 1.f / (1.f + __expf(-z));
 }
 
-template <int MAPS, int DK, int VT, int NW>
-__global__ __launch_bounds__(NW * 64) void attn_tile_kernel(const StackAttnParams p, int below_count, int ks, int head_rows)
+template <int MAPS, int DK, int VT, int NW, bool SPLIT>
+__global__ __launch_bounds__(NW * 64, 3 * MAPS * DK + (1 + MAPS) * VT <= 42 ? 2 : 1) void attn_tile_kernel(const StackAttnParams p, int below_count, int ks, int head_rows)
 {
     // VP: 16 floats behind a row's channels put the 16 rows x 4 pieces that a wave stores at once on all banks alike.  (Rows of V floats, a
     // float per store, met on one bank 16 at a time: one decoded token took 10.7 us with two maps of 64 x 128 at 154 keys, 13.7 us with
-    // latent keys of 320 x 256 under a window of 512; 8.1 and 11.5 us this way.)
+    // latent keys of 320 x 256 under a window of 512; 8.1 and 11.5 us this way.)  SPLIT is the instance of ks > 1: a launch of few cycles is bound by
+    // fetching its code, and each form carried the other's end; two waves per SIMD where the operands' registers allow it keep the accumulators out
+    // of the accumulation registers, from which every block's rescaling moved them back and forth (two maps of 64 x 128 8.3 -> 7.4 us, five requests
+    // of 300 keys 12.4 -> 11.5, one map of 128 x 128 in one round 5.9 -> 5.4; 192 x 128 in two splits 7.6 as before).
     constexpr int D = DK * 32, V = VT * 16, VP = V + 16;
     extern __shared__ float lds[];
     float* o_part = lds;                          // [NW][MAPS][16][VP]
     float* ml_part = lds + NW * MAPS * 16 * VP;    // [NW][MAPS][16][2]
-    // ks == 1: blockIdx.x is the entry's 16-row tile.  ks > 1 (decoding steps: every entry one tile): blockIdx.x is the key split -
+    // Not SPLIT: blockIdx.x is the entry's 16-row tile.  SPLIT (ks > 1; decoding steps: every entry one tile): blockIdx.x is the key split -
     // workgroup `split` of an (entry, head) takes the key blocks split * NW + w, + ks * NW, ... and leaves an unnormalised partial
     // (max, sum, O per map and row) in split_ws; attn_split_merge_kernel finishes the rows.
     // head_rows (a step of single decoded tokens whose heads share key/value heads and have no numbers inside the score): the tile's 16
@@ -246,8 +252,8 @@ __global__ __launch_bounds__(NW * 64) void attn_tile_kernel(const StackAttnParam
     const int e = blockIdx.y, group = p.heads / p.kv_heads;
     const int hbase = head_rows ? blockIdx.z / head_rows * group + blockIdx.z % head_rows * 16 : 0, h = head_rows ? hbase : blockIdx.z;
     const int hend = head_rows ? min(hbase + 16, ((int) blockIdx.z / head_rows + 1) * group) : p.heads; // behind the set's last head
-    const int r0 = (ks > 1 || head_rows) ? 0 : blockIdx.x * 16;
-    const int split = ks > 1 ? blockIdx.x : 0;
+    const int r0 = (SPLIT || head_rows) ? 0 : blockIdx.x * 16;
+    const int split = SPLIT ? blockIdx.x : 0;
     const int count = p.ent_count[e];
     if (r0 >= count || count >= below_count) // entries of below_count rows and more are the prefill form's
         return;
@@ -307,7 +313,7 @@ __global__ __launch_bounds__(NW * 64) void attn_tile_kernel(const StackAttnParam
             }
     };
     const BlockWalk bw = block_walk(p, pos0 + r0, nblk);
-    const int vb0 = split * NW + w, kstep = ks * NW;
+    const int vb0 = split * NW + w, kstep = SPLIT ? ks * NW : NW;
     int kb_next = vb0 < bw.n ? walk_block(bw, vb0) : 0;
     int blk = vb0 < bw.n ? table[kb_next * 32 / page] : 0;
     if (vb0 < bw.n)
@@ -399,7 +405,7 @@ __global__ __launch_bounds__(NW * 64) void attn_tile_kernel(const StackAttnParam
                 wgt[m][ww] = 1.f; // sigmoid weights: the waves' sums simply add
             L += wgt[m][ww] * ml_part[((ww * MAPS + m) * 16 + row) * 2 + 1];
         }
-        if (ks > 1)
+        if constexpr (SPLIT)
         {
             // partial of this split: weights stay relative to the split's own maximum, nothing is divided yet
             if (sub == 0 && out_ok)
@@ -418,7 +424,7 @@ __global__ __launch_bounds__(NW * 64) void attn_tile_kernel(const StackAttnParam
         }
     }
     constexpr int CPT = (V + TPR - 1) / TPR;
-    if (ks > 1)
+    if constexpr (SPLIT)
     {
         if (out_ok)
         {
@@ -1370,8 +1376,6 @@ int launch_tile(const StackAttnParams& p, hipStream_t stream)
 {
     constexpr int NW = 4;
     const size_t lds = sizeof(float) * ((size_t) NW * MAPS * 16 * (VT * 16 + 16) + (size_t) NW * MAPS * 16 * 2);
-    const void* fn = reinterpret_cast<const void*>(&attn_tile_kernel<MAPS, DK, VT, NW>);
-    launch_util::ensure_dynamic_lds(fn, lds);
     // entries of PREFILL_ROWS rows and more go to the staged form, the rest (decoded tokens, short portions) to the key-split form;
     // a mixed step launches both, each skipping the other's entries
     static const int PREFILL_ROWS = [] {
@@ -1456,7 +1460,9 @@ int launch_tile(const StackAttnParams& p, hipStream_t stream)
                 ks = std::min(kMaxSplits, (nblk + NW - 1) / NW);
         }
         const dim3 grid(ks > 1 ? ks : (small_rows + 15) / 16, p.entries, gz);
-        hipLaunchKernelGGL((attn_tile_kernel<MAPS, DK, VT, NW>), grid, dim3(NW * 64), lds, stream, p, PREFILL_ROWS, ks, head_rows);
+        const auto tile = ks > 1 ? attn_tile_kernel<MAPS, DK, VT, NW, true> : attn_tile_kernel<MAPS, DK, VT, NW, false>;
+        launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(tile), lds);
+        hipLaunchKernelGGL(tile, grid, dim3(NW * 64), lds, stream, p, PREFILL_ROWS, ks, head_rows);
         if (ks > 1)
             hipLaunchKernelGGL((attn_split_merge_kernel<MAPS>), dim3(p.tokens, p.heads), dim3(64), 0, stream, p, ks, PREFILL_ROWS);
     }
