@@ -2,7 +2,8 @@
 //
 //   bfloat16, M >= 32, K % 64 == 0: the LDS-DMA staged MFMA tiles of gemm_glds_impl.h instantiated for bfloat16 operands
 //                     (v_mfma_f32_32x32x16_bf16), tile shape by the same rounds x area rule as the fp16 form;
-//   bfloat16, other M >= 32: the register-staged MFMA tiles of gemm_mfma.hip;
+//   bfloat16, other M >= 32: fp32 results as far as whole stages go by the same tiles, the rest of K by fma_tile_kernel; 16-bit results by the
+//                     register-staged MFMA tiles of gemm_mfma.hip;
 //   bfloat16, M <= 31: slim_kernel below - HBM-bound, the weight-streaming MFMA main loop of gemm_slim_impl.h;
 //   bfloat16, M = 1:  row_kernel - dot products on the vector pipe, K split over a workgroup's waves; fp32 accumulation, DPP reduction
 //                     (a lone token's experts: lone_up_kernel, lone_down_kernel);
@@ -685,6 +686,30 @@ int launch_stack_gemm(const StackGemmParams& p_in, hipStream_t stream)
         }
         launch_slim(p, products, groups, stream);
         return launched("stack_gemm slim");
+    }
+    if (aligned && p.M >= 32 && p.batch == 1 && !p.group_off && p.K % 64 && p.K > 64 && (p.resid || (p.out_f32 && p.act == ACT_NONE && p.seam.n_sec == 0)))
+    {
+        // rows that end inside a 128-byte stage: the LDS-DMA tiles take the whole stages, plain FMAs add what is left of K (8 .. 56 columns, exact products,
+        // bound by the fp32 result's way there and back) to it.  From one whole stage on quicker than the register-staged tiles, whose 64-byte slabs take
+        // 2 us each whatever the shape, us at M x N x K, in brackets those: 292 x 1536 x 4128 34 (278), x 1376 21 (107), x 288 15 (39), x 72 12 (28);
+        // 41 x 512 x 4128 31 (266); 4096 x 512 x 1376 30 (111); 4096 x 1536 x 4128 86 (755), x 72 32 (49).  16-bit results, which would be rounded
+        // twice, stay with them.
+        StackGemmParams whole = p, rest = p;
+        whole.K = p.K / 64 * 64;
+        rest.K = p.K - whole.K;
+        rest.a = reinterpret_cast<const uint16_t*>(p.a) + whole.K;
+        rest.w = reinterpret_cast<const uint16_t*>(p.w) + whole.K;
+        rest.split_ws = nullptr;
+        if (!p.resid)
+        {
+            rest.resid = reinterpret_cast<float*>(p.c);
+            rest.ldr = p.ldc;
+            rest.gate = nullptr;
+        }
+        if (launch_stack_gemm(whole, stream))
+            return -1;
+        hipLaunchKernelGGL((fma_tile_kernel<DT_BF16>), tiles, dim3(256), 0, stream, rest);
+        return launched("stack_gemm rest of K");
     }
     const int64_t tiles128 = (int64_t) ((p.M + 127) / 128) * ((p.N + 127) / 128);
     if (aligned && p.split_ws && p.batch == 1 && p.M >= 32 && tiles128 * 2 <= launch_util::device_cus())
