@@ -183,6 +183,28 @@ def tile_shapes(stub):
         assert [x for x in shapes(P.residual_config(width), T, rows)][1::2] == [shape] * 2, shape
 
 
+def norms_without_a_sum(stub):
+    """A norm of any number of streams carries the code of the experts' sum only where there is one to form."""
+    import narurax_cases as N
+    import ruzinex_cases as Z
+    import vetipel_cases as V
+
+    def summing(cfg, cases):
+        s = engine(cfg, cases, max_tokens=256, max_sequences=1)
+        stub.forget()
+        step(s, 'a', 40)
+        found = [re.search(r'(?:hyper_norm|land)_vec_kernelI.*Lb([01])E', k) for k in stub.kernels()]
+        assert any(found)
+        return {m[1] for m in found if m}
+
+    for width in (96, 4104):
+        for streams in (1, 2, 3, 8):
+            assert summing(V.make_config([V.window_layer()] * 2, width=width, streams=streams), V) == {'0'}, (width, streams)
+        assert summing(Z.make_config([Z.layer(mlp=Z.dense(ff=24))], width=width), Z) == {'0'}
+        for cases, layer in ((N, N.attn_layer(mlp=N.moe())), (Z, Z.layer(mlp=Z.moe()))):
+            assert summing(cases.make_config([layer] * 2, width=width), cases) == {'0', '1'}, (width, cases)
+
+
 if __name__ == '__main__':
     globals()[sys.argv[2]](Stub(sys.argv[1]), *sys.argv[3:])
     print('ok')
@@ -207,3 +229,6 @@ else:
 
     def test_tile_shapes_of_the_product_tests(stub):
         run(stub, 'tile_shapes')
+
+    def test_norms_without_an_experts_sum_do_not_carry_its_code(stub):
+        run(stub, 'norms_without_a_sum')

@@ -1592,8 +1592,8 @@ __device__ __forceinline__ void expert_sum(const StackExpertSum& m, int t, int w
 // The form for rows of a multiple of 4 up to HV_K * 4096 elements: up to 1024 threads, a thread owns K float4 columns of every
 // stream and has ALL of them in flight before its first store (the streams are read and written through the same pointer, so in
 // a loop every store would fence the loads behind it); the combined row stays in registers.  SUM: y may be a sum that is still to be formed.  In a
-// decode step such a launch comes once between streams of weights and is bound by fetching its code, some 0.3 us a KiB, so that neither a second
-// column nor the sum is compiled in where it is not needed.
+// decode step such a launch comes once between streams of weights and is bound by fetching its code, some 0.3 us a KiB, so that the sum is compiled
+// in only where there is one to form, and with one stream a second column only for rows of more than 4096.
 constexpr int HV_K = 2;
 
 template <int DT, int SM, int K, bool SUM>
@@ -1702,13 +1702,13 @@ void launch_hyper_vec(const StackHyperParams& p, int nt, hipStream_t stream)
     if (p.streams <= 1 && p.width <= 4096)
         p.sum.ys ? go(hyper_norm_vec_kernel<DT, 1, 1, true>) : go(hyper_norm_vec_kernel<DT, 1, 1, false>);
     else if (p.streams <= 1)
-        go(hyper_norm_vec_kernel<DT, 1, HV_K, true>);
+        p.sum.ys ? go(hyper_norm_vec_kernel<DT, 1, HV_K, true>) : go(hyper_norm_vec_kernel<DT, 1, HV_K, false>);
     else if (p.streams <= 2)
-        go(hyper_norm_vec_kernel<DT, 2, HV_K, true>);
+        p.sum.ys ? go(hyper_norm_vec_kernel<DT, 2, HV_K, true>) : go(hyper_norm_vec_kernel<DT, 2, HV_K, false>);
     else if (p.streams <= 4)
-        go(hyper_norm_vec_kernel<DT, 4, HV_K, true>);
+        p.sum.ys ? go(hyper_norm_vec_kernel<DT, 4, HV_K, true>) : go(hyper_norm_vec_kernel<DT, 4, HV_K, false>);
     else
-        go(hyper_norm_vec_kernel<DT, 8, HV_K, true>);
+        p.sum.ys ? go(hyper_norm_vec_kernel<DT, 8, HV_K, true>) : go(hyper_norm_vec_kernel<DT, 8, HV_K, false>);
 }
 
 // One plain residual stream (StackLandParams): a row stays in registers between its loads, the norm of what lands, the addition and
@@ -1910,7 +1910,7 @@ int launch_stack_land(const StackLandParams& p_in, hipStream_t stream)
     {
         const int k = p.width > 4096 || p.tokens >= 64 ? 2 : 1; // many rows: fewer waves meet at a row's barriers
         const int nt = std::min(1024, (p.width / 4 + 64 * k - 1) / (64 * k) * 64);
-auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.tokens), dim3(nt), 0, stream, p); };
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.tokens), dim3(nt), 0, stream, p); };
         if (p.dtype == DT_BF16 && k == 1)
             p.sum.ys ? go(land_vec_kernel<DT_BF16, 1, true>) : go(land_vec_kernel<DT_BF16, 1, false>);
         else if (p.dtype == DT_BF16)
