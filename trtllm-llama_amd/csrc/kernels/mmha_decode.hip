@@ -454,7 +454,7 @@ __global__ __launch_bounds__(256) void mmha_partial_kernel(const MmhaParams p, f
         }
         if (tail && nact == 1) // uniform
         {
-            const uint16_t h16 = f2h(O * (1.f / (L + 1.e-6f))); // (what the merge makes of one partial)
+            const uint16_t h16 = f2h(M == -INFINITY ? 0.f : O * (1.f / (L + 1.e-6f))); // (what the merge makes of one partial: no score is a number, no key counts)
             const int64_t o = ((int64_t) b * H + h) * DH + d;
             reinterpret_cast<uint16_t*>(p.out)[o] = h16;
             if (p.tail_out_q8)
