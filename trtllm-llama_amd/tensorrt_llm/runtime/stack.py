@@ -163,12 +163,10 @@ class StackEngine:
         n, e, w = len(tokens), len(counts), len(want_rows)
         assert table.ndim == 2 and table.shape[0] == e == len(pos0) == len(slots)
         # the step's arrays side by side in one: one address to look up
-        at = (0, n, n + e, n + 2 * e, n + 3 * e, n + 3 * e + table.size)
-        meta = np.empty(at[5] + w, np.int32)
-        for i, a in enumerate((tokens, counts, pos0, slots, table.reshape(-1))):
-            meta[at[i]:at[i + 1]] = np.asarray(a)
-        if w:
-            meta[at[5]:] = np.asarray(want_rows)
+        at = (0, n, n + e, n + 2 * e, n + 3 * e, n + 3 * e + table.size, n + 3 * e + table.size + w)
+        meta = np.empty(at[6], np.int32)
+        for i, a in enumerate((tokens, counts, pos0, slots, table, want_rows)):
+            meta[at[i]:at[i + 1]] = np.asarray(a).reshape(-1)[:at[i + 1] - at[i]]  # (whatever its shape, as its memory has it)
         p = meta.ctypes.data
         b = Batch(n, e, w, table.shape[1], p, p + 4 * at[1], p + 4 * at[2], p + 4 * at[3], p + 4 * at[4], p + 4 * at[5] if w else None)
         logits, at_logits = self._rows.rows(w, self.vocab) if (return_logits and w) else (None, None)
