@@ -1,61 +1,43 @@
-"""The memory behind a step's rows (runtime/stack.py): no GPU, no engine."""
+"""The rows that a step hands back belong to whoever asked for them (runtime/stack.py): no GPU, the native side is the recorder of
+test_stack_step_arguments."""
 import gc
 import threading
 
 import numpy as np
 
-from tensorrt_llm.runtime.stack import _RowPool
+from test_stack_step_arguments import WANT, engine  # noqa: F401  (a fixture)
 
 
-def test_rows_are_handed_out_again_only_when_nobody_looks_at_them():
-    pool = _RowPool()
-    a, at = pool.rows(3, 50)
-    assert a.shape == (3, 50) and a.dtype == np.float32 and a.ctypes.data == at and a.flags.c_contiguous and a.flags.writeable
+def rows(e):
+    return e.step(*WANT[:4], np.array(WANT[4]).reshape(2, 3), WANT[5])[0]
+
+
+def test_rows_own_their_memory(engine):  # noqa: F811
+    a = rows(engine)
+    assert a.base is None and a.flags.owndata and a.flags.c_contiguous and a.flags.writeable and type(a) is np.ndarray
+    a.resize((3, 7))
+    assert (a[:2] == np.arange(14).reshape(2, 7)).all() and (a[2] == 0).all()
+
+
+def test_rows_of_one_step_are_not_those_of_another(engine):  # noqa: F811
+    a = rows(engine)
     a[:] = 7.0
-    view, buffer = a[1][10:20], memoryview(a)
+    view, buffer = a[1][2:5], memoryview(a)
     del a
     gc.collect()
-    b, at_b = pool.rows(3, 50)
-    assert at_b != at
-    b[:] = 1.0
+    b = [rows(engine) for _ in range(50)]
+    for x in b:
+        x[:] = 1.0
     assert (view == 7.0).all() and (np.asarray(buffer) == 7.0).all()
-    del view
-    assert pool.rows(3, 50)[1] not in (at, at_b)
-    del buffer
-    gc.collect()
-    assert pool.rows(3, 50)[1] == at
-    assert pool.rows(2, 50)[1] != at
+    assert len({x.ctypes.data for x in b}) == 50
 
 
-def test_what_waits_is_bounded_and_other_sizes_give_way():
-    pool = _RowPool()
-    for n in (1, 2, 3):
-        held = [pool.rows(n, 1 << 18)[0] for _ in range(40)]
-        del held
-        gc.collect()
-        assert sum(k * len(v) for k, v in pool._idle.items()) <= pool.LIMIT
-        assert pool._idle[n << 20]
-    held = pool.rows(64, 1 << 18)[0]
-    held[:] = 0.0
-    del held
-    assert sum(k * len(v) for k, v in pool._idle.items()) <= pool.LIMIT
-
-
-def test_rows_outlive_their_pool():
-    pool = _RowPool()
-    a, _ = pool.rows(2, 30)
-    a[:] = 5.0
-    del pool
-    gc.collect()
-    assert (a == 5.0).all()
-
-
-def test_threads():
-    pool, bad = _RowPool(), []
+def test_threads(engine):  # noqa: F811
+    bad = []
 
     def work(i):
-        for k in range(300):
-            a, _ = pool.rows(1 + k % 3, 64)
+        for _ in range(300):
+            a = rows(engine)
             a[:] = i
             if not (a == i).all():
                 bad.append(i)

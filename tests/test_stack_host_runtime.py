@@ -136,6 +136,30 @@ def pinned_rows(stub):
     assert stub.pinned_bytes() <= (8 << 20) + 65 * 64 * 8 + (64 << 10)
 
 
+def rows_to_the_edge(stub):
+    """The caller's rows begin and end at the edge of what may be written, whatever their size; a step of that many rows stays within them."""
+    import mmap
+    import rofozen_cases as M
+    import tensorrt_llm.runtime.stack as stack
+    libc = ctypes.CDLL(None)
+    for vocab in (16, 1024, 1027, 32000):
+        s = engine(M.make_config([M.mamba_layer(heads=2, vdim=8, state=16, groups=1)], vocab=vocab), M, max_tokens=256, max_sequences=4)
+        tokens, zero, one, wanted = np.ones(3, np.int32), np.zeros(4, np.int32), np.full(1, 3, np.int32), np.arange(3, dtype=np.int32)
+        for want in (1, 3):
+            n, page = want * vocab * 4, mmap.PAGESIZE
+            pages = -(-n // page)
+            m = mmap.mmap(-1, (pages + 2) * page)
+            base = ctypes.addressof(ctypes.c_char.from_buffer(m))
+            for closed in (base, base + (pages + 1) * page):
+                assert libc.mprotect(ctypes.c_void_p(closed), page, 0) == 0
+            for at in (base + page, base + (pages + 1) * page - n):
+                b = stack.Batch(3, 1, want, 1, tokens.ctypes.data, one.ctypes.data, zero.ctypes.data, zero.ctypes.data, zero.ctypes.data,
+                                wanted.ctypes.data)
+                stub.forget()
+                assert stack.load_library().tllm_stack_step(s.engine._h, ctypes.byref(b), at, None, None) == 0
+                assert any('deliver' in k for k in stub.kernels())
+
+
 def huge_step(stub):
     """One prompt of 131072 tokens beside 300 decoded ones, 64 heads: tiles x entries x heads of one launch are more than a grid's x dimension takes."""
     import ruzinex_cases as Z
@@ -220,6 +244,9 @@ else:
 
     def test_pinned_rows(stub):
         run(stub, 'pinned_rows')
+
+    def test_rows_that_end_where_memory_does(stub):
+        run(stub, 'rows_to_the_edge')
 
     def test_a_step_with_more_tiles_than_a_grid_dimension(stub):
         run(stub, 'huge_step')

@@ -37,8 +37,6 @@ def engine(monkeypatch):
     monkeypatch.setattr(stack, 'load_library', lambda *a, **k: lib)
     e = object.__new__(stack.StackEngine)
     e._h, e.vocab, e.lib = 1, lib.vocab, lib
-    if hasattr(stack, '_RowPool'):
-        e._rows = stack._RowPool()
     yield e
     e._h = None
 

@@ -138,6 +138,16 @@ struct Run
     float* shift_carry = nullptr;              // token shift: the sequence's last normed row, [slots, width]
 };
 
+// The caller's rows are mostly memory that the system has yet to give: their pages come in while the GPU works, with what they hold unchanged,
+// instead of behind it.
+void bring_in(float* rows, size_t bytes)
+{
+    volatile char* p = reinterpret_cast<volatile char*>(rows);
+    for (size_t at = 0; at < bytes; at += 4096)
+        p[at] = p[at];
+    p[bytes - 1] = p[bytes - 1];
+}
+
 } // namespace
 
 struct tllm_stack
@@ -2293,6 +2303,8 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         if (!deliver && next_ids_out)
             HIP_OK(hipMemcpyAsync(next_ids_out, s->ids_out, (size_t) NW * 4, hipMemcpyDeviceToHost, stream));
     }
+    if (deliver && logits_out)
+        bring_in(logits_out, (size_t) NW * s->vocab * 4);
     HIP_OK(hipStreamSynchronize(stream));
     if (deliver && logits_out)
         std::memcpy(logits_out, s->land_rows, (size_t) NW * s->vocab * 4);

@@ -6,8 +6,6 @@ caller that drives `RaggedGenerationSession.step` itself."""
 import ctypes
 import os
 import subprocess
-import threading
-import weakref
 from typing import Dict, Optional, Sequence
 
 import numpy as np
@@ -77,50 +75,6 @@ def last_error() -> str:
     return load_library().tllm_last_error().decode('utf-8', 'replace')
 
 
-class _Lease:
-    """What every array over a block of the pool hangs on, views and all (numpy keeps it as their base); the block goes back with the last of them."""
-    __slots__ = ('pool', 'block', '__array_interface__')
-
-    def __init__(self, pool, block, shape):
-        self.pool, self.block = weakref.ref(pool), block
-        self.__array_interface__ = {'version': 3, 'shape': shape, 'typestr': '<f4', 'data': (block[1], False)}
-
-    def __del__(self):
-        pool = self.pool()
-        if pool is not None:
-            pool.give_back(self.block)
-
-
-class _RowPool:
-    """Memory of result rows that is handed out again once no array looks at it any more: a fresh row of 32000 logits takes 65 us to fault in, a
-    warm one 2 us to fill.  At most `LIMIT` bytes wait here, and they go with the engine; rows that are still looked at stay theirs."""
-    LIMIT = 32 << 20
-
-    def __init__(self):
-        self._idle = {}  # bytes of a block -> the blocks of that size (memory, its address) that nobody looks at
-        self._lock = threading.RLock()  # (an array can end while this thread is in here)
-
-    def give_back(self, block):
-        n = block[0].nbytes
-        with self._lock:
-            if sum(k * len(v) for k, v in self._idle.items()) + n > self.LIMIT:
-                self._idle = {k: v for k, v in self._idle.items() if k == n}  # sizes that steps no longer ask for
-                if n * (len(self._idle.get(n, ())) + 1) > self.LIMIT:
-                    return
-            self._idle.setdefault(n, []).append(block)
-
-    def rows(self, n: int, width: int):
-        """An fp32 array [n, width] and its address."""
-        need = n * width * 4
-        with self._lock:
-            waiting = self._idle.get(need)
-            block = waiting.pop() if waiting else None
-        if block is None:
-            memory = np.empty(need, np.uint8)
-            block = (memory, memory.ctypes.data)
-        return np.asarray(_Lease(self, block, (n, width))), block[1]
-
-
 class StackEngine:
     """config: flat dict of the keys include/tllm_stack_api.h lists; tensors: name -> (numpy array, 'float32' | 'bfloat16')
     where a bfloat16 tensor is carried as uint16 bit patterns."""
@@ -153,7 +107,6 @@ class StackEngine:
         self.layer_runs = lib.tllm_stack_layer_runs(self._h)
         self.width = int(config['width'])
         self._last_tokens = 0
-        self._rows = _RowPool()
 
     def step(self, tokens: Sequence[int], counts: Sequence[int], pos0: Sequence[int], slots: Sequence[int], block_table,
              want_rows: Sequence[int], return_logits: bool = True, stream: int = 0):
@@ -169,9 +122,10 @@ class StackEngine:
             meta[at[i]:at[i + 1]] = np.asarray(a).reshape(-1)[:at[i + 1] - at[i]]  # (whatever its shape, as its memory has it)
         p = meta.ctypes.data
         b = Batch(n, e, w, table.shape[1], p, p + 4 * at[1], p + 4 * at[2], p + 4 * at[3], p + 4 * at[4], p + 4 * at[5] if w else None)
-        logits, at_logits = self._rows.rows(w, self.vocab) if (return_logits and w) else (None, None)
+        logits = np.empty((w, self.vocab), np.float32) if (return_logits and w) else None
         ids = np.empty(w, np.int32)
-        rc = load_library().tllm_stack_step(self._h, ctypes.byref(b), at_logits, ids.ctypes.data if w else None, stream)
+        rc = load_library().tllm_stack_step(self._h, ctypes.byref(b), logits.ctypes.data if logits is not None else None,
+                                            ids.ctypes.data if w else None, stream)
         if rc:
             raise RuntimeError(f'tllm_stack_step failed: {last_error()}')
         self._last_tokens = n
