@@ -68,3 +68,31 @@ def test_exhaustion_and_limits():
         KVCacheManager([pool], 2, 6, 8)  # tokens_per_block must be a power of two
     with pytest.raises(ValueError):
         KVCacheManager([pool], 2, 4, 8, beam_width=2).add_sequence(GenerationSequence(0, 0), 5)
+
+
+def test_reserve_finds_a_sequence_however_its_caller_counts_the_batch():
+    mgr = KVCacheManager([], 32, 4, 8)
+    seqs = [GenerationSequence(i, i) for i in range(3)]
+    for s in seqs:
+        mgr.reserve(s, 5)
+    counts = [None, -1, 2, 7, 'row 3', np.int64(1), True]
+    known = [GenerationSequence(10 + i, c) for i, c in enumerate(counts)]
+    for s in known:
+        mgr.add_sequence(s, 3)
+    for n in (6, 9):
+        for i, s in enumerate(known):
+            mgr.reserve(s, n + i % 2)
+    assert mgr.lens == [5, 5, 5] + [9 + i % 2 for i in range(len(known))] and [s.batch_idx for s in known] == counts
+    mgr.reserve(GenerationSequence(1, 1), 11)  # equal is the same sequence
+    assert mgr.lens[1] == 11 and len(mgr.sequences) == 3 + len(known)
+    assert mgr.blocks_manager.get_number_blocks(seqs[1]) == 3
+
+
+def test_reserve_counts_the_blocks_of_the_place_that_a_sequence_takes():
+    mgr = KVCacheManager([], 8, 4, 8)
+    mgr.reserve(GenerationSequence(0, 0), 4)
+    for _ in range(2):  # held for sequence 5 in row 1, ahead of its first tokens
+        mgr.blocks_manager.allocate(GenerationSequence(5, 1))
+    late = GenerationSequence(5, 9)
+    mgr.reserve(late, 12)
+    assert late.batch_idx == 1 and mgr.blocks_manager.get_number_blocks(late) == 3 and mgr.blocks_manager.num_free_blocks() == 4

@@ -148,13 +148,13 @@ class KVCacheManager(object):
     def reserve(self, sequence: GenerationSequence, total_tokens: int):
         """Ragged batches: make `sequence` (known or new) hold blocks for `total_tokens` tokens.  A prompt arrives in portions of
         any size, so the blocks are taken as the portions come, not for the whole prompt at once."""
-        owned = self.blocks_manager._owned.get(sequence)
-        if owned is None and sequence not in self.sequences:
+        if sequence not in self.blocks_manager._owned and sequence not in self.sequences:
             sequence.batch_idx = len(self.sequences)
             self.sequences.append(sequence)
             self.lens.append(0)
-        at = sequence.batch_idx  # its place, unless the caller counts its batch another way
-        if not (0 <= at < len(self.sequences) and self.sequences[at] is sequence):
+        owned = self.blocks_manager._owned.get(sequence)
+        at = sequence.batch_idx  # its place, unless the caller counts its batch another way, with numbers or without
+        if not (type(at) is int and 0 <= at < len(self.sequences) and self.sequences[at] is sequence):
             at = self.sequences.index(sequence)
         have = len(owned[0]) if owned is not None else 0
         need = -(-total_tokens // self.tokens_per_block)
