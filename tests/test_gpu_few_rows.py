@@ -1,6 +1,7 @@
-"""Products of few rows (2 .. 31; LLaMA: from 5, int4 weights from 3) through the weight-streaming MFMA kernels (gemm_slim_impl.h): LLaMA plugins in every weight type and the stack
-engine, at the edges of the row tiles (9, 16, 17, 31 rows), ragged columns, rows of W that end inside a 256-byte block or are shorter
-than the waves' first round, and both launch shapes (from 5120 columns on)."""
+"""Products of few rows (2 .. 31; LLaMA: from 5, int4 weights and fp16 O / down of a generation step from 3) through the weight-streaming MFMA kernels
+(gemm_slim_impl.h): LLaMA plugins in every weight type and the stack engine, at the edges of the row tiles (9, 16, 17, 31 rows), ragged columns, rows
+of W that end inside a 256-byte block or are shorter than the waves' first round.  Weight-only weights: both launch shapes (from 5120 columns on);
+the launch shapes of the others are test_gpu_slim_shapes.py's."""
 import numpy as np
 import pytest
 import torch

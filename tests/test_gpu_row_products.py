@@ -1,6 +1,6 @@
 """Products of one row (row_kernel of stack_gemm.hip): K of less than one 512-column chunk, of whole chunks and one 16-byte piece more at every number
 of chunks per wave and of waves per row, beyond the longest row that is requested at once; odd columns, and columns enough that a wave has rows of its
-own; the plain, gated, grouped and residual epilogues.  Bounds as in test_gpu_product_tiles."""
+own; the plain (against an exactly known row), gated, grouped and residual epilogues.  Bounds of the others as in the designs' own tests."""
 import numpy as np
 import pytest
 
@@ -8,6 +8,7 @@ import ruzinex_cases as Z
 import test_gpu_ruzinex as R
 import test_gpu_tolenex as GT
 import tolenex_cases as T
+from test_gpu_slim_shapes import check_head, known_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -18,18 +19,10 @@ LENGTHS = [8, 504, 512, 520, 1024, 1032, 1536, 1544, 2048, 2056, 4096, 4104, 614
 @pytest.mark.parametrize('k', LENGTHS)
 @pytest.mark.parametrize('columns', [37, 4101])
 def test_plain_product(columns, k):
-    cfg = Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32)], width=k, vocab=columns)
-    toks = R.tokens_for(cfg, 1, 5)
-    w = Z.random_weights(cfg, 6)
-    s = R.session_for(cfg, w, 'bfloat16', debug_mode=True)
+    s, toks, h, w = known_rows(columns, k, 1)
     got, _ = s.step([('a', toks, [0])])
-    x = s.engine.tap(0).astype(np.float64)
-    h = R.to_bf16(x / np.sqrt((x * x).mean(1, keepdims=True) + cfg['norm']['eps']) * w['final.norm'])
-    want = h @ w['embed'].astype(np.float64).T
-    e = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
-    assert (e < 2.0 ** -8 + k * 2.0 ** -24).all(), f'off by {e.max():.3g}'
-    worst = np.abs(got - want) / (np.abs(h) @ np.abs(w['embed'].astype(np.float64)).T)
-    assert (worst < 2.0 ** -8 + k * 2.0 ** -24).all(), f'place {worst.argmax()} is off by {worst.max():.3g} of its terms'
+    np.testing.assert_array_equal(s.engine.tap(0), w[:1])
+    check_head(got, h, w)
 
 
 @pytest.mark.parametrize('k,ff', [(72, 504), (520, 1032), (1032, 1536), (1544, 2056), (2056, 520), (4104, 64)])

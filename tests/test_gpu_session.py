@@ -577,7 +577,7 @@ def test_one_layer_at_larger_llama_dimensions_vs_oracle(mode, int8_kv, dims):
     """The layer dimensions of LLaMA-30B (D 6656, 52 heads, FFN 17920) and 65B (D 8192, 64 heads, FFN 22016) - what `build.py --n_embd
     --n_head --inter_size` of the reference accepts - with a ragged batch of 5 (the GEMV's 8-row bucket; with fp16 activations its rows
     exceed a CU's LDS and go through in slabs, gemv.hip): rows of 13 - 43 KiB, the third activation-vector bucket for the
-    down-projection, 52 / 64 heads in the attention launch and its in-launch merge.  Context + 3 generation steps (eager and graph)
+    down-projection, 52 / 64 heads in the attention launch (28 slots: one split, no merge).  Context + 3 generation steps (eager and graph)
     against the oracle on identical weights and scales."""
     H, D, I = {'30b': (52, 6656, 17920), '65b': (64, 8192, 22016)}[dims]
     cfg, w = synth_model(29, L=1, H=H, D=D, I=I, V=512)

@@ -1,6 +1,7 @@
 """Products of 2 .. 31 rows in every launch shape of the weight-streaming form (pick_shape of gemm_slim_impl.h): on both sides of its lines in rows
 (8, 16), columns (2048, 4096 on 256 CUs) and length of a row (4096 bytes), with columns that end inside a workgroup and rows that end inside a
-block, in its second run, or give some waves no block.  Bounds as in test_gpu_few_rows and test_gpu_product_tiles."""
+block, in its second run, or give some waves no block.  The stack engine's against exactly known rows; bounds of the plugins as in
+test_gpu_few_rows."""
 import numpy as np
 import pytest
 import torch
@@ -17,20 +18,31 @@ ROWS = [2, 8, 9, 16, 17, 31]
 COLUMNS = [2045, 3003, 4101]
 
 
+def known_rows(n, k, m):
+    """A session, a prompt of m tokens and the bfloat16 rows h that its head multiplies, known exactly: the layer adds nothing to embeddings of +- 1,
+    whose norm is 1 / sqrt(1 + eps), 5e-6 below 1, and takes every bfloat16 weight back to itself."""
+    cfg = Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32)], width=k, vocab=n)
+    w = Z.random_weights(cfg, 6)
+    w['l0.mix.o'][:] = 0
+    signs = np.random.default_rng(5).integers(0, 2, (m, k)) * 2.0 - 1
+    w['embed'][:m] = signs
+    return R.session_for(cfg, w, 'bfloat16', debug_mode=True), list(range(m)), signs * w['final.norm'], w['embed'].astype(np.float64)
+
+
+def check_head(got, h, w):
+    """Sums of k products that are exact in fp32: each is off by no more than k roundings of what its terms come to."""
+    worst = np.abs(got - h @ w.T) / (np.abs(h) @ np.abs(w).T)
+    assert (worst < h.shape[1] * 2.0 ** -24).all(), f'place {np.unravel_index(worst.argmax(), worst.shape)} is off by {worst.max():.3g} of its terms'
+
+
 @pytest.mark.parametrize('k', [8, 136, 264, 2048, 2056, 4360])
 @pytest.mark.parametrize('n', COLUMNS)
 @pytest.mark.parametrize('m', ROWS)
 def test_stack_products(m, n, k):
-    cfg = Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32)], width=k, vocab=n)
-    toks = R.tokens_for(cfg, m, 5)
-    w = Z.random_weights(cfg, 6)
-    s = R.session_for(cfg, w, 'bfloat16', debug_mode=True)
+    s, toks, h, w = known_rows(n, k, m)
     got, _ = s.step([('a', toks, list(range(m)))])
-    x = s.engine.tap(0).astype(np.float64)
-    h = R.to_bf16(x / np.sqrt((x * x).mean(1, keepdims=True) + cfg['norm']['eps']) * w['final.norm'])
-    want = h @ w['embed'].astype(np.float64).T
-    worst = np.abs(got - want) / (np.abs(h) @ np.abs(w['embed'].astype(np.float64)).T)
-    assert (worst < 2.0 ** -8 + k * 2.0 ** -24).all(), f'place {np.unravel_index(worst.argmax(), worst.shape)} is off by {worst.max():.3g} of its terms'
+    np.testing.assert_array_equal(s.engine.tap(0), w[:m])
+    check_head(got, h, w)
 
 
 @pytest.mark.parametrize('k', [64, 544, 4112, 8208])
