@@ -1,5 +1,5 @@
 """Products of 2 .. 31 rows in every launch shape of the weight-streaming form (pick_shape of gemm_slim_impl.h): on both sides of its lines in rows
-(8, 16), columns (2048, 4096 on 256 CUs) and length of a row (4096 bytes), with columns that end inside a workgroup and rows that end inside a
+(8, 16), columns (2048, 4096, 12288, 16384 on 256 CUs) and length of a row (512, 1024, 4096 bytes), with columns that end inside a workgroup and rows that end inside a
 block, in its second run, or give some waves no block.  The stack engine's against exactly known rows; bounds of the plugins as in
 test_gpu_few_rows."""
 import numpy as np
@@ -18,7 +18,7 @@ ROWS = [2, 8, 9, 16, 17, 31]
 COLUMNS = [2045, 3003, 4101]
 
 
-def known_rows(n, k, m):
+def known_rows(n, k, m, **kw):
     """A session, a prompt of m tokens and the bfloat16 rows h that its head multiplies, known exactly: the layer adds nothing to embeddings of +- 1,
     whose norm is 1 / sqrt(1 + eps), 5e-6 below 1, and takes every bfloat16 weight back to itself."""
     cfg = Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32)], width=k, vocab=n)
@@ -26,7 +26,7 @@ def known_rows(n, k, m):
     w['l0.mix.o'][:] = 0
     signs = np.random.default_rng(5).integers(0, 2, (m, k)) * 2.0 - 1
     w['embed'][:m] = signs
-    return R.session_for(cfg, w, 'bfloat16', debug_mode=True), list(range(m)), signs * w['final.norm'], w['embed'].astype(np.float64)
+    return R.session_for(cfg, w, 'bfloat16', debug_mode=True, **kw), list(range(m)), signs * w['final.norm'], w['embed'].astype(np.float64)
 
 
 def check_head(got, h, w):
@@ -43,6 +43,16 @@ def test_stack_products(m, n, k):
     got, _ = s.step([('a', toks, list(range(m)))])
     np.testing.assert_array_equal(s.engine.tap(0), w[:m])
     check_head(got, h, w)
+
+
+@pytest.mark.parametrize('k', [8, 72, 264, 520, 1544, 2040, 2048, 2056])
+@pytest.mark.parametrize('n', [12301, 16371])
+def test_stack_products_of_many_columns(n, k):
+    """More than three, and four, workgroups of 16 columns per CU."""
+    s, toks, h, w = known_rows(n, k, max(ROWS), max_sequences=len(ROWS))
+    for m in ROWS:
+        got, _ = s.step([(m, toks[:m], list(range(m)))])
+        check_head(got, h[:m], w)
 
 
 @pytest.mark.parametrize('k', [64, 544, 4112, 8208])

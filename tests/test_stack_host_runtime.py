@@ -229,6 +229,38 @@ def norms_without_a_sum(stub):
             assert summing(cases.make_config([layer] * 2, width=width), cases) == {'0', '1'}, (width, cases)
 
 
+def few_row_forms(stub):
+    """Products of 2 .. 31 rows take the form that their rows, columns, length of a row and products call for (gemm_slim_impl.h), on 256 CUs."""
+    import ruzinex_cases as Z
+
+    class Zeros:  # (nothing is computed)
+        standard_normal = staticmethod(lambda shape: np.zeros(shape, np.float32))
+    np.random.default_rng = lambda seed: Zeros
+
+    def forms(s, rows, want=1):
+        stub.forget()
+        step(s, 'a', rows, want)
+        found = [re.search(r'slim_(group)_kernelILi(\d)|slim_kernel.*ShapeILi(\d+)ELi(\d)ELi(\d)ELi(\d)', k) for k in stub.kernels()]
+        return [m[2] if m[1] else tuple(map(int, m.groups()[2:])) for m in found if m]
+
+    for n, k, shapes in ((16384, 64, ((16, 2, 1, 2), (16, 2, 1, 4), (16, 2, 1, 8))), (16384, 512, ((16, 2, 1, 2), (16, 2, 1, 4), (16, 2, 1, 8))),
+                         (16384, 2040, ((16, 2, 1, 2), (16, 2, 2, 4), (16, 2, 1, 8))), (16384, 2048, ((8, 4, 1, 4), (16, 2, 2, 4), (16, 2, 1, 8))),
+                         (16384, 2056, ((16, 4, 2, 2), (16, 4, 2, 4), (16, 2, 1, 8))), (16385, 2056, ((16, 4, 2, 2), (16, 4, 2, 4), (16, 2, 2, 8))),
+                         (16368, 64, ((16, 2, 2, 2), (16, 2, 2, 4), (16, 2, 1, 8))), (12288, 64, ((16, 2, 2, 2), (16, 2, 2, 4), (16, 2, 2, 8))),
+                         (5504, 1536, ((16, 2, 2, 2), (16, 2, 2, 4), (16, 2, 2, 8))), (4096, 256, ((16, 2, 2, 2), (16, 4, 2, 4), (16, 4, 2, 8))),
+                         (4096, 264, ((16, 8, 2, 2), (16, 4, 2, 4), (16, 4, 2, 8))), (2048, 264, ((8, 4, 2, 4), (16, 4, 2, 4), (16, 4, 2, 8)))):
+        s = engine(Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32)], width=k, vocab=n), Z, max_tokens=256, max_sequences=1)
+        for rows, shape in zip(((2, 8), (9, 16), (17, 31)), shapes):
+            assert [forms(s, m, m)[-1] for m in rows] == [shape] * 2, (n, k, rows)
+    # 32 experts that all tokens go to: gated columns, then the width's
+    for ff, width, want in ((520, 1032, ('1', '1', '1', '1', '2', '2')), (520, 2056, ((16, 4, 2, 2), '1', '1', '1', '2', '2')),
+                            (128, 512, ((16, 2, 2, 2), (16, 2, 1, 2), (16, 2, 2, 4), '1', (16, 2, 2, 8), '2'))):
+        mlp = Z.moe(experts=32, top=32, ff=ff, shared=0)
+        s = engine(Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=mlp)], width=width), Z, max_tokens=256, max_sequences=1)
+        got = tuple(f for m in (8, 16, 31) for f in forms(s, m, 0)[-2:])
+        assert got == want, (ff, width, got)
+
+
 if __name__ == '__main__':
     globals()[sys.argv[2]](Stub(sys.argv[1]), *sys.argv[3:])
     print('ok')
@@ -259,3 +291,6 @@ else:
 
     def test_norms_without_an_experts_sum_do_not_carry_its_code(stub):
         run(stub, 'norms_without_a_sum')
+
+    def test_forms_of_products_of_few_rows(stub):
+        run(stub, 'few_row_forms')

@@ -10,13 +10,13 @@
 // stream(): both operands come by LDS-DMA, D blocks ahead in a ring of the wave's own, so that a lane holds no block in registers (40 .. 50
 // VGPRs, and what is in flight per CU is what its LDS holds) and rows of A are requested once per workgroup, 4 rows x 256 bytes an instruction.
 // product(): a block ahead in registers, A straight from the cache in fragment geometry; for weight-only types, whose rows of A are 2 and 4 times
-// as long as W's.
+// as long as W's, and for grouped products whose groups have few rows (groups_by_registers).
 //
 // Time hardly depends on M up to 8 rows.  Measured, cold weights, back to back, us, bfloat16, N x K at 8 / 16 / 31 rows, in brackets the register form:
 //   2048 x 2048 4.0 / 5.0 / 6.1 (5.3 / 6.1 / 7.5)    2048 x 5504 7.5 / 9.0 / 11.2 (9.1 / 10.6 / 15.1)    4352 x 2048 6.7 / 7.2 / 8.9 (9.5 / 11.1 / 13.5)
 //   11008 x 2048 10.8 / 11.2 / 13.5 (12.1 / 13.6 / 18.6)    4096 x 4096 7.8 / 8.9 / 10.5 (9.1 / 9.9 / 12.9)    4096 x 11008 18.7 / 19.9 / 23.2 (19.6 / 21.6 / 28.4)
 //   22016 x 4096 30.3 = 5.9 TB/s / 34.2 / 44.1 (32.1 / 39.5 / 59.5)    32000 x 2048 24.6 / 27.4 / 35.7 (28.7 / 31.8 / 43.7)
-// The launch shapes (Shape below) are chosen from these: few columns want narrow workgroups (2048 x 2048, 8 rows: 8 columns 4.0, 16 columns 4.6 us);
+// The launch shapes (Shape below) for long rows are chosen from these: few columns want narrow workgroups (2048 x 2048, 8 rows: 8 columns 4.0, 16 columns 4.6 us);
 // up to a workgroup per CU 8 waves (4096 x 4096 7.8 against 8.5 for 4); more workgroups than CUs fewer waves of fewer blocks, as requests
 // beyond what fills the memory system only thrash (4352 x 2048, 8 rows: 8 columns by 4 waves one block ahead 6.7, 16 columns by 4 waves 7.2, by 8 waves
 // 7.7; 31 rows by 2 waves 8.9, by 4 waves 10.5), but long rows still 4 (22016 x 4096, 16 rows: 34.2 against 40.2 for 2).
@@ -103,14 +103,24 @@ struct Shape
     static_assert((COLS == 16 || (COLS == 8 && XI == 4)) && ring >= mt * 1024, "narrow workgroups hold up to 8 rows of A");
     static constexpr int lds_bytes = WAVES_ * ring;
 };
-// calls f with the shape for m rows, n columns of `products` products and rows of W of `wbytes` bytes; grouped: a workgroup looks up its product first
+// calls f with the shape for m rows, n columns of `products` products and rows of W of `wbytes` bytes; grouped: a workgroup looks up its product first.
+// Rows below 4 KiB end within a few blocks a wave: there what counts is how many workgroups a CU holds, so two waves, and from four workgroups per CU on
+// a single block ahead; us at 8 rows, in brackets the shapes for longer rows: 32000 x 64 5.1 (14.4), x 512 9.0 (15.4), x 1792 21.6 (25.0), 11008 x 256
+// 4.7 (7.7), x 1792 9.7 (12.0), 2048 x 64 3.8 (4.3); at 16 rows 32000 x 256 6.8 (9.5).  Rows of 4 KiB, each on the same memory channels as the one
+// before, want 8 columns in 512-byte runs up to 8 rows: 8192 x 2048 9.9 (16 columns 11.0), 32000 x 2048 at 2 rows 24.9 (27.4).  31 rows by 2 waves two blocks ahead
+// fill a third of a CU's LDS: beyond three workgroups per CU one block ahead, 13056 x 128 5.1 (7.3), 16384 x 2048 18.3 (23.5), x 11008 84 (99), of
+// long rows up to four per CU (22016 x 11008 126, 121 with two).
 template <class F>
 inline auto pick_shape(int m, int64_t n, int64_t products, int64_t wbytes, bool grouped, int cus, F f)
 {
     const int64_t wgs = (n + 15) / 16 * products;
-    const bool many = wgs > cus, brief = wbytes <= 4096;
+    const bool many = wgs > cus, crowd = wgs >= 4 * cus, brief = wbytes <= 4096;
     if (m <= 8)
     {
+        if (crowd && (grouped ? brief : wbytes < 4096))
+            return f(Shape<16, 2, 1, 2>());
+        if (wbytes <= 512 || (many && (grouped ? wbytes <= 1024 : wbytes < 4096)))
+            return f(Shape<16, 2, 2, 2>());
         if (wgs * 2 <= cus)
             return f(Shape<8, 4, 2, 4>());
         if (!many)
@@ -118,8 +128,24 @@ inline auto pick_shape(int m, int64_t n, int64_t products, int64_t wbytes, bool 
         return brief && !grouped ? f(Shape<8, 4, 1, 4>()) : f(Shape<16, 4, 2, 2>());
     }
     if (m <= 16)
+    {
+        if (crowd && wbytes <= 1024)
+            return f(Shape<16, 2, 1, 4>());
         return many && brief ? f(Shape<16, 2, 2, 4>()) : f(Shape<16, 4, 2, 4>());
+    }
+    if (wgs > 3 * cus && (brief || wgs <= 4 * cus))
+        return f(Shape<16, 2, 1, 8>());
     return many ? f(Shape<16, 2, 2, 8>()) : f(Shape<16, 4, 2, 8>());
+}
+// Whether grouped products of up to m rows go through product(), 4 waves: a group mostly has a row or two of them, and stream() brings all 8, 16 or
+// 32 rows of A that its shape has room for to LDS for each.  32 groups, 4 of them per token, weights cold, us, in brackets stream(); N x K at 8 tokens:
+// 2816 x 256 10.7 (17.8), x 1024 21.1 (24.5), x 2048 42.1 (45.2), x 3072 54.6 (53.2); at 16 tokens 2816 x 512 15.6 (21.3), x 2048 55.3 (61.4), x 4096
+// 100 (100); at 31 tokens 1408 x 512 14.3 (17.2), x 2048 41.9 (43.2), x 4096 64.6 (69.4).  Fewer workgroups, 704 x 2048 at 8 tokens 15.7 (15.0); 256 x 512 at 16
+// and 31 4.9 (5.0), 6.7 (5.4), x 2048 10.9 (10.8), 12.6 (11.9).
+inline bool groups_by_registers(int m, int64_t n, int64_t products, int64_t wbytes, int cus)
+{
+    const int64_t wgs = (n + 15) / 16 * products;
+    return m > 8 ? wgs > 2 * cus : wgs >= 8 * cus && wbytes <= 4096;
 }
 
 // one LDS-DMA instruction: 64 lanes x 16 bytes -> LDS [lds_byte + lane * 16] (inline asm: for the builtin the compiler waits for everything in

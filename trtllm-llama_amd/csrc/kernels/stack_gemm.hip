@@ -448,8 +448,46 @@ __global__ __launch_bounds__(S::waves * 64) void slim_kernel(const StackGemmPara
         });
 }
 
+// Grouped, up to 16 * MT rows a group (groups_by_registers): the same with a block ahead in registers
+template <int MT>
+__global__ __launch_bounds__(256) void slim_group_kernel(const StackGemmParams p_in, int groups)
+{
+    __shared__ __attribute__((aligned(16))) char lds[slim::lds_bytes<MT, 4>()];
+    int b = blockIdx.z, first = -1, rows = 0;
+    if (groups && (b = nth_group(p_in.group_off, groups, b, first, rows)) < 0)
+        return;
+    const StackGemmParams p = batch_slice<DT_BF16>(p_in, b, first, rows);
+    if (p.M <= 0)
+        return;
+    const int lane = threadIdx.x & 63, n0 = blockIdx.x * 16;
+    const char* xrow[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+    {
+        int m = 16 * t + (lane & 15);
+        m = m < p.M ? m : p.M - 1;
+        xrow[t] = reinterpret_cast<const char*>(p.a) + (int64_t) (p.a_rows ? p.a_rows[m] : m) * p.lda * 2;
+    }
+    slim::product<W_BF16, MT, 4>(lds, reinterpret_cast<const char*>(p.w) + (int64_t) n0 * p.ldw * 2, p.ldw * 2, p.N - n0, p.K * 2, xrow,
+        [&](int t, const slim::f32x4& acc) {
+            const int row = 16 * t + (lane & 15), col = n0 + 4 * (lane >> 4);
+            if (row >= p.M)
+                return;
+            if (col < p.N)
+                seam_pair<DT_BF16>(p, row, col, acc[0], acc[1]);
+            if (col + 2 < p.N)
+                seam_pair<DT_BF16>(p, row, col + 2, acc[2], acc[3]);
+        });
+}
+
 void launch_slim(const StackGemmParams& p, int products, int groups, hipStream_t stream)
 {
+    if (p.group_off && slim::groups_by_registers(p.M, p.N, products, (int64_t) p.K * 2, launch_util::device_cus()))
+    {
+        const auto kernel = p.M <= 16 ? slim_group_kernel<1> : slim_group_kernel<2>;
+        hipLaunchKernelGGL(kernel, dim3((p.N + 15) / 16, 1, products), dim3(256), 0, stream, p, groups);
+        return;
+    }
     slim::pick_shape(p.M, p.N, products, (int64_t) p.K * 2, p.group_off != nullptr, launch_util::device_cus(), [&](auto shape) {
         using S = decltype(shape);
         launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(&slim_kernel<S>), S::lds_bytes);
