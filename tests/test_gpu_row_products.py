@@ -25,7 +25,7 @@ def test_plain_product(columns, k):
     check_head(got, h, w)
 
 
-@pytest.mark.parametrize('k,ff', [(72, 504), (520, 1032), (1032, 1536), (1544, 2056), (2056, 520), (4104, 64)])
+@pytest.mark.parametrize('k,ff', [(72, 504), (520, 1032), (1032, 1536), (1544, 2056), (2056, 520), (4104, 64), (2056, 704), (2312, 1408), (3072, 1400)])
 @pytest.mark.parametrize('kind', ['dense', 'moe', 'shared'])
 def test_gated_and_grouped_products(kind, k, ff):
     mlp = {'dense': Z.dense(ff=ff), 'moe': Z.moe(experts=70, top=3, ff=ff, shared=0), 'shared': Z.moe(experts=3, top=2, ff=ff, shared=ff)}[kind]

@@ -261,6 +261,24 @@ def few_row_forms(stub):
         assert got == want, (ff, width, got)
 
 
+def lone_row_forms(stub):
+    """One row through experts that an ordering launch has looked up (over 64 outputs): a row of W by one wave or several, in one portion or more, by its
+    length and by how many there are (pick_row_shape of stack_gemm.hip)."""
+    import ruzinex_cases as Z
+
+    class Zeros:  # (nothing is computed)
+        standard_normal = staticmethod(lambda shape: np.zeros(shape, np.float32))
+    np.random.default_rng = lambda seed: Zeros
+    for width, ff, want in ((2048, 8, (1, 4)), (2056, 8, (2, 3)), (3072, 8, (2, 3)), (3080, 8, (2, 4)), (2056, 64, (2, 3)), (2056, 72, (1, 6)), (2056, 128, (1, 6)),
+                            (2056, 136, (1, 3))):
+        cfg = Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=Z.moe(experts=65, top=32, ff=ff, shared=0))], width=width)
+        s = engine(cfg, Z, max_tokens=256, max_sequences=1)
+        stub.forget()
+        step(s, 'a', 1, 0)
+        found = [re.search(r'row_kernelILi(\d)ELi(\d)', k) for k in stub.kernels()]
+        assert [tuple(map(int, m.groups())) for m in found if m][-2] == want, (width, ff)
+
+
 if __name__ == '__main__':
     globals()[sys.argv[2]](Stub(sys.argv[1]), *sys.argv[3:])
     print('ok')
@@ -294,3 +312,6 @@ else:
 
     def test_forms_of_products_of_few_rows(stub):
         run(stub, 'few_row_forms')
+
+    def test_forms_of_a_lone_row_through_groups(stub):
+        run(stub, 'lone_row_forms')

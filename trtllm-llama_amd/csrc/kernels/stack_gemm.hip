@@ -383,7 +383,8 @@ __global__ __launch_bounds__(256) void lone_down_kernel(const StackGemmParams p_
 // A wave's chunks at once are all it has up to 12288 columns of A, then portions of 3.  Rows of up to 2048 columns are shared by 2 or 4 waves only where
 // that leaves the chip room to take all workgroups in at once; otherwise, and where a workgroup first looks up its group, a wave has rows of its own and a
 // workgroup lives longer (32000 x 2048 21.6 us by two waves a row, 22.2 by four; 4 grouped products of 2816 x 2048 10.3 against 12.1;
-// 2048 x 2048 4.8 by two, 4.6 by four).
+// 2048 x 2048 4.8 by two, 4.6 by four).  Grouped rows of 5 and 6 chunks: by two waves of 3, by one of 6, by one in two portions, us for 4 products: 704 x
+// 2304 5.5 / - / -, 1408 x 2304 7.7 / 7.4 / -, 2816 x 2304 12.3 / 12.4 / 11.5, 5504 x 2304 19.7 / 19.9 / 18.5 (by two waves of 4, as longer rows: 5.8, 8.2, 12.7, 21.1).
 template <int KS_, int NC_>
 struct RowShape
 {
@@ -392,8 +393,8 @@ struct RowShape
 template <class F>
 void pick_row_shape(int64_t n, int k, int products, bool looks_up, F f)
 {
-    const int chunks = (k + 511) / 512;
-    const bool many = looks_up || n * products > 16 * launch_util::device_cus();
+    const int chunks = (k + 511) / 512, cus = launch_util::device_cus();
+    const bool many = looks_up || n * products > 16 * cus;
     if (chunks <= 1)
         f(RowShape<1, 1>());
     else if (chunks <= 2)
@@ -402,6 +403,11 @@ void pick_row_shape(int64_t n, int k, int products, bool looks_up, F f)
         many ? f(RowShape<1, 3>()) : f(RowShape<4, 1>());
     else if (chunks <= 4)
         many ? f(RowShape<1, 4>()) : f(RowShape<4, 1>());
+    else if (chunks <= 6 && looks_up)
+    {
+        const int64_t rows = n * products;
+        rows > 32 * cus ? f(RowShape<1, 3>()) : rows > 16 * cus ? f(RowShape<1, 6>()) : f(RowShape<2, 3>());
+    }
     else if (chunks <= 8)
         looks_up ? f(RowShape<2, 4>()) : f(RowShape<4, 2>());
     else if (chunks <= 12 || chunks > 24)
