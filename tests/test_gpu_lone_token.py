@@ -1,5 +1,5 @@
 """Steps of one token whose experts' products choose for themselves (stack_gemm.hip lone_up_kernel, choose_in_wave): one output and as many as a wave
-has lanes, and one more (which takes the ordering launch); groups; identities; every output chosen; equal scores (the lowest outputs win); rows of less
+has lanes, and one more (which takes the ordering launch); 8 choices, and more (which take it too); groups; identities; every output chosen; equal scores (the lowest outputs win); rows of less
 than a chunk and of several; the choice by softmax and by sigmoid, biased and corrected, weights on the input and on the output, a shared expert
 beside; and steps of more tokens in between."""
 import numpy as np
@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
 
 STEPS = [[('a', k)] for k in (1, 1, 2, 1)]
 ROUTERS = [dict(experts=1, identity=0, top=1, count=1, keep=1), dict(experts=6, identity=3, top=2, count=3, keep=2), dict(experts=17, identity=0, top=3, count=1, keep=1),
-           dict(experts=60, identity=4, top=2, count=8, keep=3), dict(experts=64, identity=0, top=64, count=1, keep=1), dict(experts=65, identity=0, top=3, count=1, keep=1)]
+           dict(experts=60, identity=4, top=2, count=8, keep=3), dict(experts=64, identity=0, top=64, count=1, keep=1), dict(experts=64, identity=0, top=8, count=1, keep=1),
+           dict(experts=5, identity=3, top=8, count=1, keep=1), dict(experts=65, identity=0, top=3, count=1, keep=1)]
 
 
 def run(mod, cfg, w, toks):
@@ -43,7 +44,7 @@ def test_corrected_softmax_and_identities(router, width, ff, equal):
     run(mod, cfg, w, toks)
 
 
-@pytest.mark.parametrize('experts,top', [(1, 1), (11, 4), (9, 9)])
+@pytest.mark.parametrize('experts,top', [(1, 1), (11, 4), (8, 8), (9, 9)])
 @pytest.mark.parametrize('width,ff', [(72, 8), (1032, 520)])
 def test_sigmoid_and_input_weights(experts, top, width, ff):
     Z, mod = narurax_cases, test_gpu_narurax

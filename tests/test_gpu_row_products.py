@@ -25,11 +25,19 @@ def test_plain_product(columns, k):
     check_head(got, h, w)
 
 
-@pytest.mark.parametrize('k,ff', [(72, 504), (520, 1032), (1032, 1536), (1544, 2056), (2056, 520), (4104, 64), (2056, 704), (2312, 1408), (3072, 1400)])
+@pytest.mark.parametrize('k,ff', [(72, 504), (520, 1032), (1032, 1536), (1544, 2056), (2056, 520), (4104, 64)])
 @pytest.mark.parametrize('kind', ['dense', 'moe', 'shared'])
 def test_gated_and_grouped_products(kind, k, ff):
     mlp = {'dense': Z.dense(ff=ff), 'moe': Z.moe(experts=70, top=3, ff=ff, shared=0), 'shared': Z.moe(experts=3, top=2, ff=ff, shared=ff)}[kind]
     cfg = Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=mlp)], width=k, vocab=61)
+    toks = R.tokens_for(cfg, 3, 97)
+    w = R.weights_for(cfg, 98, 'bfloat16', toks)
+    R.check_rows(R.replay(R.session_for(cfg, w, 'bfloat16'), {'a': toks}, ONE)['a'], toks, w, cfg, 'bfloat16')
+
+
+@pytest.mark.parametrize('k,ff', [(2056, 8), (2560, 72), (2056, 136), (3072, 136)])
+def test_rows_of_a_few_chunks_through_many_groups(k, ff):
+    cfg = Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=Z.moe(experts=65, top=32, ff=ff, shared=0))], width=k, vocab=61)
     toks = R.tokens_for(cfg, 3, 97)
     w = R.weights_for(cfg, 98, 'bfloat16', toks)
     R.check_rows(R.replay(R.session_for(cfg, w, 'bfloat16'), {'a': toks}, ONE)['a'], toks, w, cfg, 'bfloat16')

@@ -261,6 +261,16 @@ def few_row_forms(stub):
         assert got == want, (ff, width, got)
 
 
+def lone_choices(stub):
+    """A lone token's products choose for themselves up to 64 outputs and 8 choices; beyond, a launch orders the pairs."""
+    import ruzinex_cases as Z
+    for experts, top, lone in ((1, 1, True), (8, 8, True), (64, 8, True), (64, 9, False), (9, 9, False), (64, 64, False), (65, 2, False)):
+        s = engine(Z.make_config([Z.layer(mlp=Z.moe(experts=experts, top=top, ff=24))]), Z, max_tokens=256, max_sequences=1)
+        stub.forget()
+        step(s, 'a', 1, 0)
+        assert any('lone_up_kernel' in k for k in stub.kernels()) == lone, (experts, top)
+
+
 def lone_row_forms(stub):
     """One row through experts that an ordering launch has looked up (over 64 outputs): a row of W by one wave or several, in one portion or more, by its
     length and by how many there are (pick_row_shape of stack_gemm.hip)."""
@@ -315,3 +325,6 @@ else:
 
     def test_forms_of_a_lone_row_through_groups(stub):
         run(stub, 'lone_row_forms')
+
+    def test_who_chooses_for_a_lone_token(stub):
+        run(stub, 'lone_choices')

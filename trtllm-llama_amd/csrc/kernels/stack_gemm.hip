@@ -646,7 +646,10 @@ bool stack_lone_serves(const StackMoeParams& m, const StackGemmParams& up, const
         return p.K > 0 && p.N > 0 && p.K % 8 == 0 && p.lda % 8 == 0 && p.stride_w % 8 == 0 && p.ldw == 0 && p.c && !p.resid && !p.bias && p.seam.n_sec == 0
             && !((reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.w)) & 15) && (p.act < ACT_GATE_SILU || !(p.N & 1));
     };
-    return m.tokens == 1 && m.dtype == DT_BF16 && m.experts + m.identity <= LONE_OUT && rows_of_pieces(up) && rows_of_pieces(down);
+    // (every wave of the first products makes all choices: with many of them that costs more than the launch it saves.  Steps of 3 layers of 64 experts, us,
+    // in brackets with the ordering launch; width x ff 1024 x 704, 4 choices 161 - 164 (165 - 184), 8 172 - 175 (179 - 199), 16 214 - 216 (209 - 219), 64 776
+    // (376); 2048 x 1408 172 - 186 (188 - 210), 230 - 233 (229 - 246), 312 - 315 (299 - 320), 1490 (740))
+    return m.tokens == 1 && m.dtype == DT_BF16 && m.experts + m.identity <= LONE_OUT && m.top <= 8 && rows_of_pieces(up) && rows_of_pieces(down);
 }
 
 int launch_stack_lone_up(const StackMoeParams& m, const StackGemmParams& p_in, hipStream_t stream)

@@ -440,7 +440,7 @@ int launch_stack_moe_plan(const StackMoeParams& p, hipStream_t stream);
 // A step of one token needs no order of its pairs: product z of its experts' first matrices (up) chooses for itself from the logits and takes choice z
 // (slot z; slot_of_pair, topk_idx and topk_w are left for what follows), product z of their second ones (down) the same.  up / down: as for
 // launch_stack_gemm, batch the number of choices, stride_w from expert to expert, a of `up` the token's row, everything else row z.  Where
-// stack_lone_serves (bfloat16, up to 64 outputs, rows in 16-byte pieces).
+// stack_lone_serves (bfloat16, up to 64 outputs, 8 of them chosen, rows in 16-byte pieces).
 bool stack_lone_serves(const StackMoeParams& m, const StackGemmParams& up, const StackGemmParams& down);
 int launch_stack_lone_up(const StackMoeParams& m, const StackGemmParams& up, hipStream_t stream);
 int launch_stack_lone_down(const StackMoeParams& m, const StackGemmParams& down, hipStream_t stream);
