@@ -271,6 +271,25 @@ def lone_choices(stub):
         assert any('lone_up_kernel' in k for k in stub.kernels()) == lone, (experts, top)
 
 
+def who_sums(stub):
+    """The experts' rows of few tokens are summed by the norm behind them, very many of them by a launch of its own."""
+    import narurax_cases as N
+    import ruzinex_cases as Z
+
+    class Zeros:  # (nothing is computed)
+        standard_normal = staticmethod(lambda shape: np.zeros(shape, np.float32))
+        integers = staticmethod(lambda *a, **k: np.zeros(k.get('size', a[-1] if a else 1), np.int64))
+        uniform = staticmethod(lambda lo, hi, size=None: np.full(size, lo, np.float32))
+    np.random.default_rng = lambda seed: Zeros
+    for width, top, tokens, apart in ((2048, 64, 1, False), (2056, 64, 1, True), (2056, 64, 64, True), (2056, 64, 65, False), (4104, 32, 8, True), (4104, 31, 8, False)):
+        for cases, layer in ((Z, Z.layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=Z.moe(experts=64, top=top, ff=8, shared=0))),
+                             (N, N.attn_layer(heads=2, kv_heads=1, dim=32, mlp=N.moe(experts=64, top=top, ff=8)))):
+            s = engine(cases.make_config([layer], width=width), cases, max_tokens=256, max_sequences=1)
+            stub.forget()
+            step(s, 'a', tokens)
+            assert any('moe_combine' in k for k in stub.kernels()) == apart, (width, top, tokens, cases)
+
+
 def lone_row_forms(stub):
     """One row through experts that an ordering launch has looked up (over 64 outputs): a row of W by one wave or several, in one portion or more, by its
     length and by how many there are (pick_row_shape of stack_gemm.hip)."""
@@ -328,3 +347,6 @@ else:
 
     def test_who_chooses_for_a_lone_token(stub):
         run(stub, 'lone_choices')
+
+    def test_who_sums_the_experts_rows(stub):
+        run(stub, 'who_sums')

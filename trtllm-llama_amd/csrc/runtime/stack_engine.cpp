@@ -1867,7 +1867,10 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         }
         else if (launch_stack_moe_plan(mp, stream) || launch_stack_gemm(u, stream) || launch_stack_gemm(dn, stream))
             return -1;
-        if (!later)
+        // (in the norm one workgroup forms a row's sum: few tokens with very many choices are better off with the combining launch, which spreads a row.
+        // A layer's norms and sum, us, in the norm / apart: 64 rows of 6144, 1 token 31.4 / 27.6, 8 33.4 / 28.5, 64 36.4 / 33.3, 128 42 either way; 32 rows of
+        // 6144 21.0 / 20.0, 23.0 / 22.1, 26.0 / 26.1)
+        if (!later || (T <= 64 && (int64_t) l.top * Wd > 128 * 1024))
             return launch_stack_moe_combine(mp, s->moe_y, y, stream);
         later->ys = s->moe_y;
         later->slot_of_pair = mp.slot_of_pair;
