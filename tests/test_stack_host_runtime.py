@@ -271,6 +271,20 @@ def lone_choices(stub):
         assert any('lone_up_kernel' in k for k in stub.kernels()) == lone, (experts, top)
 
 
+def group_tiles(stub):
+    """Tiles of grouped products by rounds of 256 workgroups: a few tiles beyond whole rounds are no round."""
+    import ruzinex_cases as Z
+    for experts, top, tokens, ff, want in ((32, 2, 1700, 1024, (128, 256)), (16, 2, 1021, 1408, (128, 256)), (16, 8, 700, 2048, (128, 256)),
+                                           (32, 2, 2048, 1024, (256, 256)), (16, 2, 1200, 1408, (256, 256)), (32, 4, 1700, 1024, (256, 256))):
+        mlp = Z.moe(experts=experts, top=top, ff=ff, shared=0)
+        s = engine(Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=mlp)], width=64), Z, max_tokens=4096, max_sequences=1)
+        stub.forget()
+        step(s, 'a', tokens, 0)
+        found = [re.search(r'gemm_glds_kernelILi\d+ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)', k) for k in stub.kernels()]
+        shapes = [(32 * int(m[1]) * int(m[3]), 32 * int(m[2]) * int(m[4])) for m in found if m]
+        assert shapes[-2] == want, (experts, top, tokens, ff, shapes)
+
+
 def who_sums(stub):
     """The experts' rows of few tokens are summed by the norm behind them, very many of them by a launch of its own."""
     import narurax_cases as N
@@ -350,3 +364,6 @@ else:
 
     def test_who_sums_the_experts_rows(stub):
         run(stub, 'who_sums')
+
+    def test_tiles_of_grouped_products(stub):
+        run(stub, 'group_tiles')

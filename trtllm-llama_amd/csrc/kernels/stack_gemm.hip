@@ -611,16 +611,18 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
     // Grouped: m_expected rows in a group on average (g.M is their bound); up to three 128-row tiles the groups' last ones decide.  32 groups of 8096 rows: 128 x 256 151 us against 160 for 128 x 128 and
     // 167 for 256 x 192 (N 2816, K 2048), 255 / 307 / 291 (4096, 2752); of 1944 rows 128 x 128 92 us, the wider ones 95 and more (2816, 2048).
     // 256 x 256 only where it saves rounds: 32 groups of 6700 rows 60.5 us in one round against 66.6 in two (N 2048, K 1408), 145 in two against 125 in
-    // three (2816, 2048).  A group's rows spread around the average by its root.
+    // three (2816, 2048).  A group's rows spread around the average by its root; a round of the last few tiles, most of them nearly empty, does not count
+    // against the smaller ones (16 groups of 128 rows on average, N 2816, K 2048: 1.03 rounds of 128 x 256 51 us, 0.69 of 256 x 256 65; 16 of 350, 4096, 1024: 3.03
+    // 69, 2.0 78).  Over 280 products of 8 .. 64 groups where the wide ones are taken they have 0.82 - 0.99 of the other's time.
     if (m_expected > 0 && m_expected <= 384)
     {
-        auto cost = [&](int bm, int bn, double f) {
+        auto cost = [&](int bm, int bn, double f, double rest) {
             double tiles = 0.0;
             for (int at = 0; at < 3 * m_expected; at += bm) // a tile for every group of more than `at` rows
                 tiles += at ? 0.5 * std::erfc((at - m_expected) / std::sqrt(2.0 * m_expected)) : 1.0;
-            return std::ceil(tiles * g.batch * ((g.N + bn - 1) / bn) / cus - 0.02) * bm * bn * f;
+            return std::ceil(tiles * g.batch * ((g.N + bn - 1) / bn) / cus - rest) * bm * bn * f;
         };
-        pick = m_expected <= 64 ? 0 : cost(256, 256, shapes[2].f) < cost(128, 256, shapes[3].f) ? 2 : 3;
+        pick = m_expected <= 64 ? 0 : cost(256, 256, shapes[2].f, 0.02) < cost(128, 256, shapes[3].f, 0.08) ? 2 : 3;
     }
     if (g.act == ACT_SCALE_CAP || g.act == ACT_GELU_MUL)
         pick = 0; // the shape whose epilogue has them
