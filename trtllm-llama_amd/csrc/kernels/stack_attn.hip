@@ -236,9 +236,10 @@ __global__ __launch_bounds__(NW * 64, 3 * MAPS * DK + (1 + MAPS) * VT <= 42 ? 2 
     // VP: 16 floats behind a row's channels put the 16 rows x 4 pieces that a wave stores at once on all banks alike.  (Rows of V floats, a
     // float per store, met on one bank 16 at a time: one decoded token took 10.7 us with two maps of 64 x 128 at 154 keys, 13.7 us with
     // latent keys of 320 x 256 under a window of 512; 8.1 and 11.5 us this way.)  SPLIT is the instance of ks > 1: a launch of few cycles is bound by
-    // fetching its code, and each form carried the other's end; two waves per SIMD where the operands' registers allow it keep the accumulators out
-    // of the accumulation registers, from which every block's rescaling moved them back and forth (two maps of 64 x 128 8.3 -> 7.4 us, five requests
-    // of 300 keys 12.4 -> 11.5, one map of 128 x 128 in one round 5.9 -> 5.4; 192 x 128 in two splits 7.6 as before).
+    // fetching its code, and each form carried the other's end.  Two waves per SIMD where the operands leave room: Q and two key tiles of every map (3 MAPS
+    // DK), a value tile and the accumulators ((1 + MAPS) VT) take 4 registers each, and some 55 are needed beside them, so up to 42 x 4 fit 256 (one map of 192 x
+    // 192: 222; two of 128 x 128, 48 x 4, want 254 and more).  That keeps the accumulators out of the accumulation registers, from which every block's
+    // rescaling moved them back and forth (two maps of 64 x 128 8.3 -> 7.4 us, five requests of 300 keys 12.4 -> 11.5, one map of 128 x 128 in one round 5.9 -> 5.4; 192 x 128 in two splits 7.6 as before).
     constexpr int D = DK * 32, V = VT * 16, VP = V + 16;
     extern __shared__ float lds[];
     float* o_part = lds;                          // [NW][MAPS][16][VP]

@@ -200,7 +200,9 @@ __device__ __forceinline__ int nth_group(const int32_t* off, int groups, int nth
 // 512 KS NC columns of A is one trip to memory per wave, and the next workgroups' trips overlap it.  Bound by the weights' stream.  What it replaced were whole
 // rows per wave, a chunk of 2 rows at a time, and for long rows of few columns the matrix pipe; us, cold weights, N x K:
 //   2048 x 2048 3.5 (4.6)    2048 x 5504 6.0 (8.5)    4096 x 4096 7.0 (8.5)    4096 x 11008 16.5 (19.0)    10304 x 2048 8.0 (8.9)
-//   10240 x 4096 13.6 (15.5)    22016 x 4096 26.4 = 6.8 TB/s (31.1)    32000 x 2048 20.0 (21.4)
+//   10240 x 4096 13.6 (15.5)    22016 x 4096 26.4 = 6.8 TB/s (31.1)    32000 x 2048 20.0 (21.4); of rows below 512 bytes the new form has many a bit slower:
+//   16384 x 128 5.3 (4.7)    32000 x 256 8.2 (7.4)
+// These are repetitions, whose code is warm; between a step's other kernels 2048 x 2048 takes 4.6, 4096 x 4096 8.7, 10304 x 2048 10.4, 32000 x 2048 21.6.
 // 4 rows per team measured the same within 4 %, 8 waves per team too, 8 of both up to 60 % worse.
 constexpr int SK_R = 2;
 

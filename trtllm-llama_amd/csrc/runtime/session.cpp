@@ -497,7 +497,9 @@ struct tllm_session
         const float* in_qscale, const void* residual, const float* epi_scale, void* y, int64_t ldy, int out_dtype,
         const Linear* up, hipStream_t st, const float* row_scales = nullptr)
     {
-        // (fp16 without a norm ahead: generation with 8 layers of width 4096 takes 18.3 ms by the GEMV, 18.6 here at 2 sequences, 19.6 and 19.4 at 3, 20.3 and 19.9 at 4)
+        // (fp16 without a norm ahead, us a step of 3 / 4 sequences by the GEMV and here: 8 layers of width 1024 265.5 / 280.6 and 261.0 / 270.6, 2048 373.9 / 395.4
+        // and 367.6 / 383.3, 4096 765 / 792 and 752 / 772, 5120 1100 / 1144 and 1102 / 1143; 4 layers of 3072 301 / 314 and 302 / 314, 4352 502 / 525 and 499 /
+        // 519, 6656 854 / 878 and 839 / 859, 8192 1423 / 1446 and 1225 / 1250.  At 2 sequences the GEMV: 4096 18.3 ms of 24 steps, 18.6 here)
         const int from = L.wtype == W_FP16 && pro == PRO_NONE && epi != EPI_SWIGLU && out_dtype == DT_HALF ? 3 : gemm_slim_rows(L.wtype);
         if (L.wtype != W_INT8_SQ && M >= from && M <= 32 && !row_scales && !tap_dst)
         {
