@@ -4,7 +4,9 @@ own; the plain (against an exactly known row), gated, grouped and residual epilo
 import numpy as np
 import pytest
 
+import rofozen_cases as M
 import ruzinex_cases as Z
+import test_gpu_rofozen as RF
 import test_gpu_ruzinex as R
 import test_gpu_tolenex as GT
 import tolenex_cases as T
@@ -25,6 +27,20 @@ def test_plain_product(columns, k):
     check_head(got, h, w)
 
 
+@pytest.mark.parametrize('k', [8, 72, 256, 264, 504, 512])
+@pytest.mark.parametrize('columns', [10761, 16387])
+def test_short_rows_of_many_columns(columns, k):
+    test_plain_product(columns, k)
+
+
+@pytest.mark.parametrize('heads,dim,kv_rank', [(64, 16, 171), (128, 32, 88), (64, 260, 258)])
+def test_short_rows_of_many_heads(heads, dim, kv_rank):
+    cfg = M.make_config([M.latent_layer(heads=heads, dim=dim, vdim=16, kv_rank=kv_rank)])
+    toks = RF.tokens_for(cfg, 3, 97)
+    w = M.random_weights(cfg, 98)
+    RF.check_rows(RF.replay(RF.session_for(cfg, w, 'bfloat16'), {'a': toks}, ONE)['a'], toks, w, cfg, 'bfloat16')
+
+
 @pytest.mark.parametrize('k,ff', [(72, 504), (520, 1032), (1032, 1536), (1544, 2056), (2056, 520), (4104, 64)])
 @pytest.mark.parametrize('kind', ['dense', 'moe', 'shared'])
 def test_gated_and_grouped_products(kind, k, ff):
@@ -35,7 +51,7 @@ def test_gated_and_grouped_products(kind, k, ff):
     R.check_rows(R.replay(R.session_for(cfg, w, 'bfloat16'), {'a': toks}, ONE)['a'], toks, w, cfg, 'bfloat16')
 
 
-@pytest.mark.parametrize('k,ff', [(2056, 8), (2560, 72), (2056, 136), (3072, 136)])
+@pytest.mark.parametrize('k,ff', [(2056, 8), (2560, 72), (2056, 136), (3072, 136), (256, 176)])
 def test_rows_of_a_few_chunks_through_many_groups(k, ff):
     cfg = Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=Z.moe(experts=65, top=32, ff=ff, shared=0))], width=k, vocab=61)
     toks = R.tokens_for(cfg, 3, 97)

@@ -319,7 +319,12 @@ def lone_row_forms(stub):
         stub.forget()
         step(s, 'a', 1, 0)
         found = [re.search(r'row_kernelILi(\d)ELi(\d)', k) for k in stub.kernels()]
-        assert [tuple(map(int, m.groups())) for m in found if m][-2] == want, (width, ff)
+        assert [tuple(map(int, m.groups())) for m in found if m][-1] == want, (width, ff)  # (the down products: row_short_kernel)
+    for columns, k, short in ((10752, 256, False), (10753, 256, True), (10753, 264, False), (16384, 512, False), (16385, 512, True), (16385, 520, False)):
+        s = engine(Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32)], width=k, vocab=columns), Z, max_tokens=256, max_sequences=1)
+        stub.forget()
+        step(s, 'a', 1)
+        assert any('row_short_kernel' in k for k in stub.kernels()) == short, (columns, k)
 
 
 if __name__ == '__main__':

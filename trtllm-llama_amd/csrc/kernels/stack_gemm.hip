@@ -340,6 +340,54 @@ __global__ __launch_bounds__(256) void row_kernel(const StackGemmParams p_in, in
         row_product<KS, NC, false>(p, 1.f, part);
 }
 
+// Rows of W of one chunk where there are very many (a head's vocabulary on a narrow stream, the per-head products of latent attention): a wave has
+// SHORT_PAIRS pairs of columns, all requested at once, and half as many workgroups come and go, which is what bounds such a launch.  us, in brackets
+// row_kernel<1, 1>, whole rows by the waves in turn before that: 32000 x 64 6.8 (8.1, 7.2)    32000 x 256 6.9 (8.3, 7.4)    32000 x 512 8.2 (8.8, 8.8)
+//   128 heads of 512 x 128 11.1 (14.0, 12.2)    64 of 512 x 256 6.9 (8.4, 7.5)    4 pairs: 10.2, 7.5
+constexpr int SHORT_PAIRS = 2, SHORT_COLS = 4 * SK_R * SHORT_PAIRS;
+
+__global__ __launch_bounds__(256) void row_short_kernel(const StackGemmParams p_in, int groups)
+{
+    int b = blockIdx.z, first = -1, rows = 0;
+    if (groups && (b = nth_group(p_in.group_off, groups, b, first, rows)) < 0)
+        return;
+    const StackGemmParams p = batch_slice<DT_BF16>(p_in, b, first, rows);
+    const int lane = threadIdx.x & 63, n0 = (blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * SK_R * SHORT_PAIRS;
+    if (p.M <= 0 || n0 >= p.N)
+        return;
+    const uint16_t* a = reinterpret_cast<const uint16_t*>(p.a) + (int64_t) (p.a_rows ? p.a_rows[0] : 0) * p.lda;
+    const bool in = lane * 8 < p.K;
+    const int k = in ? lane * 8 : 0;
+    uint4 wv[SK_R * SHORT_PAIRS];
+#pragma unroll
+    for (int r = 0; r < SK_R * SHORT_PAIRS; ++r)
+        wv[r] = ld_nt16(reinterpret_cast<const uint16_t*>(p.w) + (int64_t) (n0 + r < p.N ? n0 + r : p.N - 1) * p.ldw + k);
+    const uint4 xv = *reinterpret_cast<const uint4*>(a + k);
+    RowSeam ops[SHORT_PAIRS];
+#pragma unroll
+    for (int i = 0; i < SHORT_PAIRS; ++i)
+        ops[i] = row_seam_request(p, n0 + SK_R * i < p.N ? n0 + SK_R * i : p.N - 1);
+    const uint32_t xs[4] = {in ? xv.x : 0u, in ? xv.y : 0u, in ? xv.z : 0u, in ? xv.w : 0u};
+    float sum[SK_R * SHORT_PAIRS];
+#pragma unroll
+    for (int r = 0; r < SK_R * SHORT_PAIRS; ++r)
+    {
+        const uint32_t ws[4] = {in ? wv[r].x : 0u, in ? wv[r].y : 0u, in ? wv[r].z : 0u, in ? wv[r].w : 0u};
+        float acc = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+        {
+            acc = fmaf(__builtin_bit_cast(float, xs[q] << 16), __builtin_bit_cast(float, ws[q] << 16), acc);
+            acc = fmaf(__builtin_bit_cast(float, xs[q] & 0xffff0000u), __builtin_bit_cast(float, ws[q] & 0xffff0000u), acc);
+        }
+        sum[r] = wave_sum(acc);
+    }
+#pragma unroll
+    for (int i = 0; i < SHORT_PAIRS; ++i)
+        if (lane == 0 && n0 + SK_R * i < p.N)
+            row_seam(p, ops[i], n0 + SK_R * i, sum[SK_R * i], sum[SK_R * i + 1]);
+}
+
 // A lone token's experts, product z = choice z.  up: every wave chooses from the logits by itself (some 0.8 us in front of its weights' requests), which
 // replaces a launch that orders pairs: a last workgroup that waits for all logits, chooses, orders and copies.  Choice, order and products of
 // a layer of 32 + 2 outputs, width 2048, in a step of one token: 9.5 us for the router's launch, 3.7 for its logits alone.
@@ -422,6 +470,12 @@ void pick_row_shape(int64_t n, int k, int products, bool looks_up, F f)
 
 void launch_row(const StackGemmParams& p, int products, int groups, hipStream_t stream)
 {
+    // (us by row_kernel and here: 10240 x 256 4.3 and 4.6, 11008 x 256 4.7 and 4.6, 16384 x 256 5.4 and 5.0, x 512 5.6 and 5.9, 20000 x 512 7.0 and 6.5)
+    if (p.K <= 512 && (int64_t) p.N * products > (p.K <= 256 ? 42 : 64) * launch_util::device_cus())
+    {
+        hipLaunchKernelGGL(row_short_kernel, dim3((p.N + SHORT_COLS - 1) / SHORT_COLS, 1, products), dim3(256), 0, stream, p, groups);
+        return;
+    }
     pick_row_shape(p.N, p.K, products, p.group_off != nullptr, [&](auto shape) {
         using S = decltype(shape);
         hipLaunchKernelGGL((row_kernel<S::KS, S::NC>), dim3((p.N + S::cols - 1) / S::cols, 1, products), dim3(256), 0, stream, p, groups);
