@@ -1,7 +1,7 @@
 """Steps of one token whose experts' products choose for themselves (stack_gemm.hip lone_up_kernel, choose_in_wave): one output and as many as a wave
-has lanes, and one more (which takes the ordering launch); 8 choices, and more (which take it too); groups; identities; every output chosen; equal scores (the lowest outputs win); rows of less
-than a chunk and of several; the choice by softmax and by sigmoid, biased and corrected, weights on the input and on the output, a shared expert
-beside; and steps of more tokens in between."""
+has lanes, and one more (which takes the ordering launch); 8 choices, and more (which take it too); groups; identities; every output chosen; equal scores
+(the lowest outputs win); rows of less than a chunk and of several; the choice by softmax and by sigmoid, biased and corrected, weights on the input and
+on the output, a shared expert beside; and steps of more tokens in between."""
 import numpy as np
 import pytest
 

@@ -4,9 +4,10 @@
 //                     (v_mfma_f32_32x32x16_bf16), tile shape by the same rounds x area rule as the fp16 form;
 //   bfloat16, other M >= 32: fp32 results as far as whole stages go by the same tiles, the rest of K by fma_tile_kernel; 16-bit results by the
 //                     register-staged MFMA tiles of gemm_mfma.hip;
-//   bfloat16, M <= 31: slim_kernel below - HBM-bound, the weight-streaming MFMA main loop of gemm_slim_impl.h;
-//   bfloat16, M = 1:  row_kernel - dot products on the vector pipe, K split over a workgroup's waves; fp32 accumulation, DPP reduction
-//                     (a lone token's experts: lone_up_kernel, lone_down_kernel);
+//   bfloat16, M <= 31: slim_kernel below - HBM-bound, the weight-streaming MFMA main loop of gemm_slim_impl.h; grouped products of many workgroups
+//                     slim_group_kernel, the same with its block in registers;
+//   bfloat16, M = 1:  row_kernel - dot products on the vector pipe, K split over a workgroup's waves; fp32 accumulation, DPP reduction; very many rows of
+//                     one chunk: row_short_kernel (a lone token's experts: lone_up_kernel, lone_down_kernel);
 //   bfloat16, 2 <= M <= 8, few columns of long rows: skinny_ksplit_kernel, the same for several rows;
 //   float32         : fma_tile_kernel - 64 x 64 tiles of plain fp32 FMAs through LDS (no reduced-precision matrix mode), any shape;
 //                     also the fallback for bfloat16 operands whose rows are not 16-byte aligned.
