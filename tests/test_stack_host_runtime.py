@@ -207,6 +207,42 @@ def tile_shapes(stub):
         assert [x for x in shapes(P.residual_config(width), T, rows)][1::2] == [shape] * 2, shape
 
 
+def wide_tiles(stub):
+    """The sizes of test_gpu_wide_tiles.py take the 256 x 256 tiles of gemm_wide_impl.h: (ways out of wide::Out, grouped) of a step's products."""
+    import ruzinex_cases as Z
+    import sodudra_cases as S
+    import test_gpu_product_tiles as P
+    import test_gpu_wide_tiles as G
+    import tolenex_cases as T
+
+    class Zeros:  # (nothing is computed)
+        standard_normal = uniform = staticmethod(lambda *a, size=None, **k: np.zeros(size if size is not None else a[-1], np.float32))
+    np.random.default_rng = lambda seed: Zeros
+    for cases in (S, T, Z):
+        cases.bf16_round = lambda x: x
+    store, gated, fp32, resid, resid_gate = range(5)
+
+    def outs(cfg, cases, *steps):
+        s = engine(cfg, cases, max_tokens=4096, max_batch_tokens=4096, max_sequences=1)
+        for rows, want in steps:
+            stub.forget()
+            step(s, 'a', rows, want)
+            found = [re.search(r'wide_kernelILi\d+ELi(\d+)ELb([01])', k) for k in stub.kernels()]
+            yield {(int(m[1]), int(m[2])) for m in found if m}
+
+    for k in sorted({k for _, k in G.PLAIN}):
+        for found in outs(P.plain_config(G.COLUMNS, k), Z, *((rows, rows) for rows, at in G.PLAIN if at == k)):
+            assert (fp32, 0) in found, k
+    rows, k = G.PLAIN[0]
+    assert not next(outs(P.plain_config(G.COLUMNS - 1, k), Z, (rows, rows)))
+    assert (gated, 0) in next(outs(G.gated_config(), Z, (G.GATED[0], 1)))
+    for tokens, *sizes in G.GROUPED:
+        assert (gated, 1) in next(outs(G.grouped_config(*sizes), Z, (tokens, 1))), sizes
+    assert (fp32, 1) in next(outs(G.grouped_config(*G.GROUPED[-1][1:]), Z, (G.GROUPED[-1][0], 1)))
+    assert (resid_gate, 0) in next(outs(G.residual_config(T), T, (G.RESIDUAL[0], 1)))
+    assert (resid, 0) in next(outs(G.residual_config(S), S, (G.RESIDUAL[0], 1)))
+
+
 def norms_without_a_sum(stub):
     """A norm of any number of streams carries the code of the experts' sum only where there is one to form."""
     import narurax_cases as N
@@ -372,3 +408,6 @@ else:
 
     def test_tiles_of_grouped_products(stub):
         run(stub, 'group_tiles')
+
+    def test_sizes_of_the_wide_tile_tests(stub):
+        run(stub, 'wide_tiles')

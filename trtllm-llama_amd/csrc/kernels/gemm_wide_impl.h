@@ -1,0 +1,665 @@
+// Products of many rows on 256 x 256 tiles:  C[m,n] = epi( sum_k A[m,k] * W[n,k] ), both operands with K contiguous; bfloat16, fp16 or int8 (the three
+// share one geometry: a K-tile is 128 BYTES of every row, a k-step 64 of them, and v_mfma_*_16x16x{32,32,64} takes 16 bytes a lane).  A header, so that
+// the translation units that instantiate it for their operand types share one source.  Everything has internal linkage.
+//
+// What bounds it, and what follows from that (2048 x 4096 x 4096, 128 workgroups, clocks per K-tile of one CU, of which its 512 MFMAs are 2048):
+//   * Lock-step stages (barrier, read fragments, multiply) took 3650, the sum of LDS reads and MFMAs: every wave read at the same time.  Here the fragments of
+//     the blocks ahead are requested BETWEEN the MFMAs, pinned there, a ring of four A blocks ahead of their use; MFMAs and reads alone 2350.
+//   * The operands' way from L2 to LDS alone takes 2260 - 2400 (27 bytes per clock and CU; with 64-byte rows of half as long a K-tile 2900), which is why the tile is the
+//     largest that the accumulators allow, rows are whole 128-byte lines, and a K-tile is requested 1.5 K-tiles before its use: A has three buffers, W
+//     two, 160 KB together.  W's fragments of a k-step stay in registers, so its buffer is free again halfway through the K-tile: the first of two barriers a
+//     K-tile hands over W(t) and A(t - 1) to K-tile t + 2, the second says that K-tile t + 1 has landed.
+//   * 16 x 16 MFMAs of twice the depth move half the accumulator traffic of 32 x 32 ones: alone 1.96 against 1.82 PFLOP/s in bfloat16, and where the chip is full
+//     its clock falls with its power, 2.2 against 2.0 GHz in the same lock-step kernel.
+// All together 2640 - 2700 clocks.  bfloat16, us, in brackets what the lock-step tiles of 32 x 32 MFMAs took: 2048 x 22016 x 4096 gated 285 (350; in a step 315 (353)),
+// 4096 x 4096 x 4096 111 (123), 4096 x 8192 x 4096 210 = 1.31 PFLOP/s (265), 1024 x 13056 x 2048 gated 60 (63).
+// Tried and slower: the DMA two at a time (+8 %), W's ahead of A's or in turn with them (+10 %), a fifth 64-byte stage, setprio by wave half.
+#pragma once
+#include "dev_utils.h"
+#include "gemm_seam.h"
+#include "kernels.h"
+#include "launch_util.h"
+#include <algorithm>
+#include <cmath>
+
+namespace tllm
+{
+namespace kernels
+{
+namespace
+{
+namespace wide
+{
+using namespace dev;
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) void lds_ptr;
+typedef const __attribute__((address_space(3))) u32x4* lds_frag;
+
+constexpr int BM = 256, BN = 256, WN = 4, WAVES = 8;
+constexpr int NA = 8, NB = 4;               // 16-row blocks of A and of W of a wave (2 x 4 waves)
+constexpr int UNIT = 256 * 128;             // bytes of one operand's K-tile
+constexpr int LDS_BYTES = 5 * UNIT;         // A: three buffers, W: two
+constexpr int AHEAD = 3, RING = 4;          // A blocks requested ahead of their use
+constexpr int MID = 5;                      // block of the first k-step in front of which W(t) and A(t - 1) are handed over
+constexpr int DMA_A = 4, DMA_W = 4;         // LDS-DMA instructions of a wave and K-tile (8 rows each)
+
+// 64 lanes x 16 bytes, wave-uniform base + a lane's 32-bit offset -> LDS [lds_byte + lane * 16]; in asm, as hipcc would wait for the builtin's in
+// front of the next ds_read (it cannot know that it writes another buffer)
+__device__ __forceinline__ void load16(const char* base, uint32_t off, uint32_t lds_byte)
+{
+    uint32_t m0_keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(m0_keep) : "v"(off), "s"(base), "s"(lds_byte) : "memory");
+}
+
+// LDS image of a K-tile: [row][8 pieces of 16 bytes], piece c of a row at c ^ swz(row).  The lane groups of a ds_read_b128 ({0-3, 12-15, 20-27},
+// {4-11, 16-19, 28-31} and + 32) then meet 16 different 16-byte slots.  A lane's row of an A block is lane & 15; of a W block w_row().
+__device__ __forceinline__ int a_swz(int row)
+{
+    return (row & 2) | ((row & 8) >> 1);
+}
+// Row of W's tile (of the wave's 64) that MFMA row i of block j takes, and with it where a lane's four results of that block go, of row lane & 15.
+// PAIRS: blocks 2q and 2q + 1 are together 8 neighbouring columns, 32 q + 8 (lane >> 4) and on: 16 bytes of a 16-bit row; otherwise block j is the 4
+// columns 16 j + 4 (lane >> 4) and on: 16 bytes of an fp32 row.  Either way a store covers 64 neighbouring bytes of 16 rows.
+template <bool PAIRS>
+__device__ __forceinline__ int w_row(int j, int i)
+{
+    return PAIRS ? 32 * (j >> 1) + 8 * (i >> 2) + 4 * (j & 1) + (i & 3) : 16 * j + i;
+}
+template <bool PAIRS>
+__device__ __forceinline__ int w_swz(int row)
+{
+    return PAIRS ? (row & 2) | ((row & 16) >> 2) : a_swz(row);
+}
+
+template <int WT>
+struct Acc
+{
+    using type = typename std::conditional<WT == W_INT8_SQ, i32x4, f32x4>::type;
+};
+template <int WT>
+__device__ __forceinline__ typename Acc<WT>::type mfma(const u32x4& w, const u32x4& a, const typename Acc<WT>::type& c)
+{
+    if constexpr (WT == W_INT8_SQ)
+        return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, w), __builtin_bit_cast(i32x4, a), c, 0, 0, 0);
+    else if constexpr (WT == W_BF16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, a), c, 0, 0, 0);
+}
+
+template <int N>
+__device__ __forceinline__ void wait_vm_and_meet()
+{
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// One wave's part of a tile: its operands' sources and its accumulators.
+template <int WT, bool PAIRS>
+struct Tile
+{
+    using acc_t = typename Acc<WT>::type;
+    const char *a, *w;      // wave-uniform bases
+    uint32_t ao[DMA_A], wo[DMA_W]; // a lane's offsets of its DMA instructions
+    uint32_t lds;           // LDS address of the buffers
+    int nt, wid, lane;
+    acc_t acc[NA][NB];
+
+    __device__ __forceinline__ void dma_a(int i, int t, uint32_t buf) const
+    {
+        load16(a + (int64_t) t * 128, ao[i], buf + (uint32_t) (i * WAVES + wid) * 1024);
+    }
+    __device__ __forceinline__ void dma_w(int i, int t, uint32_t buf) const
+    {
+        load16(w + (int64_t) t * 128, wo[i], buf + (uint32_t) (i * WAVES + wid) * 1024);
+    }
+    // HALF: the tile has up to 128 rows, the second half of A is not fetched
+    template <bool HALF>
+    static constexpr int dmas()
+    {
+        return (HALF ? DMA_A / 2 : DMA_A) + DMA_W;
+    }
+    // instruction i of K-tile t (A's first, see above)
+    template <bool HALF>
+    __device__ __forceinline__ void dma(int i, int t, uint32_t abuf, uint32_t wbuf) const
+    {
+        constexpr int FIRST_W = HALF ? DMA_A / 2 : DMA_A;
+        i < FIRST_W ? dma_a(i, t, abuf) : dma_w(i - FIRST_W, t, wbuf);
+    }
+    // K-tiles 0 and 1
+    __device__ __forceinline__ void head(bool half) const
+    {
+        for (int t = 0; t < 2 && t < nt; ++t)
+        {
+            const uint32_t ab = lds + (uint32_t) t * UNIT, wb = lds + (uint32_t) (3 + t) * UNIT;
+#pragma unroll
+            for (int i = 0; i < DMA_A / 2; ++i)
+                dma_a(i, t, ab);
+            if (!half)
+#pragma unroll
+                for (int i = DMA_A / 2; i < DMA_A; ++i)
+                    dma_a(i, t, ab);
+#pragma unroll
+            for (int i = 0; i < DMA_W; ++i)
+                dma_w(i, t, wb);
+        }
+    }
+
+    // The K loop, behind a barrier that says that K-tile 0 has landed.  Ends with every wave past its last LDS read.
+    template <bool HALF>
+    __device__ __forceinline__ void loop()
+    {
+        uint32_t A0 = lds, A1 = lds + UNIT, A2 = lds + 2 * UNIT, W0 = lds + 3 * UNIT, W1 = lds + 4 * UNIT; // of K-tiles t, t + 1, t + 2 and t, t + 1
+        constexpr int DMAS = dmas<HALF>();
+        const int wm = wid / WN, wn = wid % WN;
+        if (HALF && wm == 1) // no rows: this wave only fetches
+        {
+            for (int t = 0; t < nt; ++t)
+            {
+                asm volatile("s_barrier" ::: "memory");
+                if (t + 2 < nt)
+                {
+#pragma unroll
+                    for (int i = 0; i < DMAS; ++i)
+                        dma<HALF>(i, t + 2, A2, W0);
+                    wait_vm_and_meet<DMAS>();
+                }
+                else
+                    wait_vm_and_meet<0>();
+                const uint32_t x = A0, y = W0;
+                A0 = A1, A1 = A2, A2 = x, W0 = W1, W1 = y;
+            }
+            asm volatile("s_barrier" ::: "memory");
+            return;
+        }
+        const int i16 = lane & 15, k4 = lane >> 4;
+        const uint32_t al = (uint32_t) ((wm * NA * 16 + i16) * 128), wl = (uint32_t) ((wn * NB * 16 + w_row<PAIRS>(0, i16)) * 128);
+        const uint32_t as = a_swz(i16), ws = w_swz<PAIRS>(w_row<PAIRS>(0, i16));
+        const uint32_t a_k0 = al + ((k4 ^ as) << 4), a_k1 = al + (((4 + k4) ^ as) << 4), w_k0 = wl + ((k4 ^ ws) << 4), w_k1 = wl + (((4 + k4) ^ ws) << 4);
+        auto a_at = [](uint32_t base, int block) { return *(lds_frag) (uintptr_t) (base + block * 2048); };
+        auto w_at = [](uint32_t base, int j) { return *(lds_frag) (uintptr_t) (base + w_row<PAIRS>(j, 0) * 128); };
+        u32x4 fa[RING], fw[2][NB]; // fw: by k-step
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            fw[0][j] = w_at(W0 + w_k0, j);
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+            fa[i] = a_at(A0 + a_k0, i);
+        for (int t = 0; t < nt; ++t)
+        {
+            const uint32_t ra0 = A0 + a_k0, ra1 = A0 + a_k1, ran = A1 + a_k0, rw1 = W0 + w_k1, rwn = W1 + w_k0;
+            const bool more = t + 2 < nt;
+            // every step is pinned (sched_barrier): left to itself the compiler gathers the reads in front of the MFMAs
+#pragma unroll
+            for (int i = 0; i < NA; ++i) // k-step 0
+            {
+                if (i == MID)
+                {
+                    // W's fragments of k-step 1 have arrived (the A blocks requested behind them may still be under way): nobody reads W(t), or A(t - 1), any more
+                    asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(MID - 2) : "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                {
+                    acc[i][j] = mfma<WT>(fw[0][j], fa[i % RING], acc[i][j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (j == 0)
+                        fa[(i + AHEAD) % RING] = i + AHEAD < NA ? a_at(ra0, i + AHEAD) : a_at(ra1, i + AHEAD - NA);
+                    if (i < 2 && (j == 1 || j == 2))
+                        fw[1][i * 2 + j - 1] = w_at(rw1, i * 2 + j - 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (i >= MID)
+                {
+                    if (more && i - MID < DMAS)
+                        dma<HALF>(i - MID, t + 2, A2, W0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < NA; ++i) // k-step 1
+            {
+                if (i == NA - AHEAD)
+                {
+                    // K-tile t + 1 has landed: this wave's by the count (K-tile t + 2's stay under way; five of them are requested behind here), everyone's by the barrier
+                    constexpr int BEHIND = DMAS - (NA - AHEAD) - (NA - MID) > 0 ? DMAS - (NA - AHEAD) - (NA - MID) : 0;
+                    if (more)
+                        wait_vm_and_meet<DMAS - BEHIND>();
+                    else
+                        wait_vm_and_meet<0>();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                {
+                    acc[i][j] = mfma<WT>(fw[1][j], fa[i % RING], acc[i][j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (j == 0)
+                        fa[(i + AHEAD) % RING] = i + AHEAD < NA ? a_at(ra1, i + AHEAD) : a_at(ran, i + AHEAD - NA);
+                    const int q = (i - (NA - AHEAD)) * (NB - 1) + j - 1; // (behind the last K-tile: old data, not used)
+                    if (i >= NA - AHEAD && j >= 1 && q < NB)
+                        fw[0][q] = w_at(rwn, q);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (more && i + NA - MID < DMAS)
+                    dma<HALF>(i + NA - MID, t + 2, A2, W0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const uint32_t x = A0, y = W0;
+            A0 = A1, A1 = A2, A2 = x, W0 = W1, W1 = y;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+};
+
+// Where the tiles of a launch are.  Tiles are numbered product by product (or group by group), inside one by bands of eight row tiles, rows fastest; in each round
+// of the grid an XCD (workgroups go round them) takes a contiguous range of the numbers, so that the 32 tiles that it works on share 8 + 4 operand panels in its L2.
+struct Place
+{
+    int product, m0, n0, rows, first; // rows: of the product; first: grouped, where they begin
+};
+__device__ __forceinline__ int rows_to_tiles(int rows)
+{
+    return (rows + BM - 1) / BM;
+}
+
+template <bool GROUPED>
+struct Places
+{
+    int tiles_n, total;
+    int first, count, own, incl; // grouped, of group `lane` (of 64): where its rows begin, how many, its row tiles, those of all groups up to it
+
+    __device__ __forceinline__ void chunk(const GemmParams& p, int g0, int before, int lane)
+    {
+        const int g = g0 + lane < p.batch ? g0 + lane : p.batch - 1, lo = p.group_off[g], hi = p.group_off[g + 1];
+        first = lo;
+        count = hi - lo;
+        own = g0 + lane < p.batch ? rows_to_tiles(count) : 0;
+        incl = own;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1)
+        {
+            const int o = __shfl_up(incl, d, 64);
+            incl += lane >= d ? o : 0;
+        }
+        incl += before;
+    }
+    __device__ __forceinline__ void begin(const GemmParams& p, int lane)
+    {
+        tiles_n = (p.N + BN - 1) / BN;
+        if constexpr (!GROUPED)
+        {
+            total = rows_to_tiles(p.M) * tiles_n * p.batch;
+            return;
+        }
+        int before = 0;
+        for (int g0 = 0; g0 < p.batch; g0 += 64)
+        {
+            chunk(p, g0, before, lane);
+            before = __builtin_amdgcn_readlane(incl, 63);
+        }
+        total = before * tiles_n;
+    }
+    // the tile of this workgroup's round r; false: there is none left
+    __device__ __forceinline__ bool at(const GemmParams& p, int r, int lane, Place& o)
+    {
+        const int grid = gridDim.x, begin = r * grid, c = blockIdx.x, size = total - begin < grid ? total - begin : grid;
+        if (c >= size)
+            return false;
+        const int q = size >> 3, rest = size & 7, xcd = c & 7;
+        int id = begin + (xcd < rest ? xcd * (q + 1) : rest * (q + 1) + (xcd - rest) * q) + (c >> 3);
+        o.product = o.first = 0;
+        o.rows = p.M;
+        if constexpr (GROUPED)
+        {
+            uint64_t mask;
+            for (int g0 = 0, before = 0;; g0 += 64)
+            {
+                if (p.batch > 64)
+                    chunk(p, g0, before, lane); // (else the registers hold the only one)
+                o.product = g0;
+                mask = __builtin_amdgcn_ballot_w64(id < incl * tiles_n);
+                if (mask != 0 || g0 + 64 >= p.batch)
+                    break;
+                before = __builtin_amdgcn_readlane(incl, 63);
+            }
+            const int g = mask ? __builtin_ctzll(mask) : 63;
+            id -= (__builtin_amdgcn_readlane(incl, g) - __builtin_amdgcn_readlane(own, g)) * tiles_n;
+            o.product += g;
+            o.first = __builtin_amdgcn_readlane(first, g);
+            o.rows = __builtin_amdgcn_readlane(count, g);
+        }
+        const int tiles_m = rows_to_tiles(o.rows);
+        if (!GROUPED && p.batch > 1)
+        {
+            o.product = id / (tiles_m * tiles_n);
+            id -= o.product * (tiles_m * tiles_n);
+        }
+        constexpr int BAND = 8;
+        int band = 0, high = tiles_m;
+        if (tiles_m > BAND)
+        {
+            band = id / (BAND * tiles_n);
+            id -= band * (BAND * tiles_n);
+            high = tiles_m - band * BAND < BAND ? tiles_m - band * BAND : BAND;
+        }
+        const int tn = id / high;
+        o.m0 = (band * BAND + id - tn * high) * BM;
+        o.n0 = tn * BN;
+        return true;
+    }
+};
+
+// How the results leave: a kernel instance each, as an epilogue's instructions are fetched cold once a tile.
+enum Out
+{
+    OUT_STORE, // c and the output sections: mostly 16-bit rows, bias, relu^2
+    OUT_GATED, // gated pairs of columns in front of the first section, 16-bit rows
+    OUT_FP32,  // fp32 c alone
+    OUT_RESID, // added to the fp32 residual
+    OUT_RESID_GATE // ... behind a sigmoid gate
+};
+constexpr bool out_pairs(int out)
+{
+    return out == OUT_STORE || out == OUT_GATED;
+}
+
+__device__ __forceinline__ float4 load4(const float* p)
+{
+    return *reinterpret_cast<const float4*>(p);
+}
+__device__ __forceinline__ void store8(float* p, const float (&v)[8])
+{
+    reinterpret_cast<float4*>(p)[0] = make_float4(v[0], v[1], v[2], v[3]);
+    reinterpret_cast<float4*>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
+}
+__device__ __forceinline__ uint32_t bf_pair(float a, float b)
+{
+    return (uint32_t) f2bf(a) | ((uint32_t) f2bf(b) << 16);
+}
+__device__ __forceinline__ void store8(uint16_t* p, const float (&v)[8])
+{
+    *reinterpret_cast<uint4*>(p) = make_uint4(bf_pair(v[0], v[1]), bf_pair(v[2], v[3]), bf_pair(v[4], v[5]), bf_pair(v[6], v[7]));
+}
+
+// bfloat16 products: the stack engine's layer seam.  p.N, offsets and addresses are whole 16-byte pieces (serves()); c: of this product
+template <int OUT>
+__device__ __forceinline__ void leave_pairs(const GemmParams& p, const Tile<W_BF16, true>& t, void* c, int row0, int col0, int rows)
+{
+#pragma unroll
+    for (int jp = 0; jp < NB / 2; ++jp)
+    {
+        const int col = col0 + 32 * jp + 8 * (t.lane >> 4);
+        if (col >= p.N)
+            continue;
+        float b[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (p.bias)
+        {
+            const float4 x = load4(p.bias + col), y = load4(p.bias + col + 4);
+            b[0] = x.x, b[1] = x.y, b[2] = x.z, b[3] = x.w, b[4] = y.x, b[5] = y.y, b[6] = y.z, b[7] = y.w;
+        }
+        const SeamOut so = seam_out<false>(p.seam, p.act, c, p.ldc, p.out_dtype != DT_BFLOAT16, col);
+        auto value = [&](float (&v)[8], int i) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                v[e] = t.acc[i][2 * jp + (e >> 2)][e & 3] + b[e];
+        };
+        auto rows_out = [&](auto* to) {
+#pragma unroll
+            for (int i = 0; i < NA; ++i)
+            {
+                float v[8];
+                value(v, i);
+                if (so.act == GEMM_ACT_RELU2)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        v[e] = seam_relu2(v[e]);
+                if (row0 + i * 16 < rows)
+                    store8(to + (int64_t) (row0 + i * 16) * so.ldc + col, v);
+            }
+        };
+        if (OUT == OUT_GATED && seam_gated(so.act))
+        {
+#pragma unroll
+            for (int i = 0; i < NA; ++i)
+            {
+                float v[8], g[4];
+                value(v, i);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    g[e] = seam_gate<false>(p.act, v[2 * e], v[2 * e + 1]);
+                if (row0 + i * 16 < rows)
+                    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(so.c) + (int64_t) (row0 + i * 16) * so.ldc + (col >> 1)) = make_uint2(bf_pair(g[0], g[1]), bf_pair(g[2], g[3]));
+            }
+        }
+        else if (so.f32)
+            rows_out(reinterpret_cast<float*>(so.c));
+        else
+            rows_out(reinterpret_cast<uint16_t*>(so.c));
+    }
+}
+template <int OUT>
+__device__ __forceinline__ void leave_fp32(const GemmParams& p, const Tile<W_BF16, false>& t, void* c, int row0, int col0, int rows)
+{
+    float* out = OUT == OUT_FP32 ? reinterpret_cast<float*>(c) : p.resid;
+    const int64_t ld = OUT == OUT_FP32 ? p.ldc : p.ldr;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+    {
+        const int col = col0 + 16 * j + 4 * (t.lane >> 4);
+        if (col >= p.N)
+            continue;
+        const float* bias = OUT == OUT_RESID_GATE ? p.gate_bias : p.bias;
+        float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (OUT != OUT_RESID && bias)
+            b = load4(bias + col);
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+        {
+            const int64_t row = row0 + i * 16;
+            if (row >= rows)
+                continue;
+            float* at = out + row * ld + col;
+            float v[4] = {t.acc[i][j][0], t.acc[i][j][1], t.acc[i][j][2], t.acc[i][j][3]};
+            if constexpr (OUT == OUT_FP32)
+                *reinterpret_cast<float4*>(at) = make_float4(v[0] + b.x, v[1] + b.y, v[2] + b.z, v[3] + b.w);
+            else
+            {
+                const float4 o = load4(at);
+                if constexpr (OUT == OUT_RESID_GATE)
+                {
+                    const uint2 z = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(p.gate) + row * p.ldg + col);
+                    v[0] *= 1.f / (1.f + __expf(-(__builtin_bit_cast(float, z.x << 16) + b.x)));
+                    v[1] *= 1.f / (1.f + __expf(-(__builtin_bit_cast(float, z.x & 0xffff0000u) + b.y)));
+                    v[2] *= 1.f / (1.f + __expf(-(__builtin_bit_cast(float, z.y << 16) + b.z)));
+                    v[3] *= 1.f / (1.f + __expf(-(__builtin_bit_cast(float, z.y & 0xffff0000u) + b.w)));
+                }
+                *reinterpret_cast<float4*>(at) = make_float4(o.x + v[0], o.y + v[1], o.z + v[2], o.w + v[3]);
+            }
+        }
+    }
+}
+
+// Persistent: a workgroup per CU (fewer where that makes the rounds even) walks its tiles; the next tile's first two K-tiles are under way while this
+// one's results leave, straight from the accumulators (16 rows x 64 bytes a store, no LDS).  The code in front of the first request runs cold: one copy
+// of it serves the first tile and the others (2.2 us with two, a batch's and a group's places in one instance and K-tile 1's requests unrolled).
+template <int WT, int OUT, bool GROUPED>
+__global__ __launch_bounds__(64 * WAVES) void wide_kernel(const GemmParams p)
+{
+    extern __shared__ __attribute__((aligned(16))) char wide_lds[];
+    constexpr int ES = WT == W_INT8_SQ ? 1 : 2;
+    constexpr bool PAIRS = out_pairs(OUT);
+    using T = Tile<WT, PAIRS>;
+    T t;
+    t.lane = threadIdx.x & 63;
+    t.wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    t.lds = (uint32_t) (uintptr_t) (lds_ptr*) wide_lds;
+    t.nt = p.K * ES / 128;
+    Places<GROUPED> places;
+    places.begin(p, t.lane);
+    Place now = {}, next;
+    for (int round = 0;; ++round)
+    {
+        const bool more = places.at(p, round, t.lane, next);
+        const bool half = next.rows - next.m0 <= BM / 2;
+        if (more)
+        {
+            const int row8 = t.wid * 8 + (t.lane >> 3), piece = t.lane & 7;
+            t.a = reinterpret_cast<const char*>(p.a);
+            t.w = reinterpret_cast<const char*>(p.w);
+            if (WT == W_BF16 && (GROUPED || p.batch > 1))
+            {
+                t.a += GROUPED ? 0 : next.product * p.batch_a;
+                t.w += next.product * p.batch_w;
+            }
+#pragma unroll
+            for (int i = 0; i < DMA_A; ++i)
+            {
+                const int row = i * WAVES * 8 + row8, m = next.m0 + row;
+                int r = next.first + (m < next.rows ? m : next.rows - 1);
+                if (GROUPED && p.a_rows)
+                    r = p.a_rows[r];
+                t.ao[i] = (uint32_t) r * (uint32_t) (p.lda * ES) + ((piece ^ a_swz(row)) << 4);
+            }
+#pragma unroll
+            for (int i = 0; i < DMA_W; ++i)
+            {
+                const int row = i * WAVES * 8 + row8, n = next.n0 + row < p.N ? next.n0 + row : p.N - 1;
+                t.wo[i] = (uint32_t) n * (uint32_t) p.ldw + ((piece ^ w_swz<PAIRS>(row)) << 4);
+            }
+            t.head(half);
+        }
+        if (round > 0)
+        {
+            char* c = reinterpret_cast<char*>(p.c);
+            if constexpr (WT == W_BF16)
+            {
+                c += GROUPED ? now.first * p.ldc * (p.out_dtype == DT_FLOAT ? 4 : 2) : now.product * p.batch_c;
+                const int row0 = now.m0 + t.wid / WN * (NA * 16) + (t.lane & 15), col0 = now.n0 + t.wid % WN * (NB * 16);
+                if constexpr (PAIRS)
+                    leave_pairs<OUT>(p, t, c, row0, col0, now.rows);
+                else
+                    leave_fp32<OUT>(p, t, c, row0, col0, now.rows);
+            }
+        }
+        if (!more)
+            return;
+        now = next;
+        if (round == 0 && t.nt > 1)
+        {
+            if (half)
+                wait_vm_and_meet<T::template dmas<true>()>();
+            else
+                wait_vm_and_meet<T::template dmas<false>()>();
+        }
+        else
+            wait_vm_and_meet<0>(); // (the results of the tile before have left, too)
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+                t.acc[i][j] = typename T::acc_t{0, 0, 0, 0};
+        if (half)
+            t.template loop<true>();
+        else
+            t.template loop<false>();
+    }
+}
+
+inline bool aligned16(const void* p)
+{
+    return !(reinterpret_cast<uintptr_t>(p) & 15);
+}
+
+// what the kernel takes: everything that leaves does so in whole 16-byte pieces
+template <int WT>
+bool serves(const GemmParams& p)
+{
+    constexpr int ES = WT == W_INT8_SQ ? 1 : 2;
+    if (p.wtype != WT || p.K <= 0 || (p.K * ES) % 128 || !aligned16(p.a) || !aligned16(p.w) || (p.lda * ES) % 16 || p.ldw % 16 || p.N % 8)
+        return false;
+    // 32-bit offsets of the operands' rows (gathered rows: any of the a that the caller has; its extent is not known here)
+    const int64_t rows = p.group_off ? p.group_total : p.M;
+    if (rows * p.lda * ES >= (1ll << 31) || (int64_t) p.N * p.ldw >= (1ll << 31))
+        return false;
+    if constexpr (WT == W_BF16)
+    {
+        const int c_es = p.out_dtype == DT_FLOAT ? 4 : 2;
+        if (p.batch > 1 && (p.batch_a % 16 || p.batch_w % 16 || p.batch_c % 16))
+            return false;
+        if (p.resid)
+            return aligned16(p.resid) && p.ldr % 4 == 0 && (!p.gate || (aligned16(p.gate) && p.ldg % 8 == 0 && aligned16(p.gate_bias)));
+        if ((p.out_dtype != DT_BFLOAT16 && p.out_dtype != DT_FLOAT) || !aligned16(p.bias) || (p.act != GEMM_ACT_NONE && p.act != GEMM_ACT_RELU2 && p.act < GEMM_ACT_GATE_SILU))
+            return false;
+        const bool gated = p.act >= GEMM_ACT_GATE_SILU;
+        if ((p.seam.n_sec == 0 || p.seam.sec[0].col0 > 0)
+            && (!aligned16(p.c) || p.ldc % (gated ? 8 : 16 / c_es) || (gated && p.out_dtype != DT_BFLOAT16)))
+            return false;
+        for (int s = 0; s < p.seam.n_sec; ++s)
+        {
+            const GemmSection& k = p.seam.sec[s];
+            if (k.col0 % 8 || !aligned16(k.c) || k.ldc % (k.f32 ? 4 : 8) || (k.act != GEMM_ACT_NONE && k.act != GEMM_ACT_RELU2))
+                return false;
+        }
+        return true;
+    }
+    return false;
+}
+
+// at most this many tiles (grouped: full ones, and one begun in every group that has rows)
+inline int64_t most_tiles(const GemmParams& p)
+{
+    const int64_t cols = (p.N + BN - 1) / BN;
+    if (p.group_off)
+        return (p.group_total / BM + std::min<int64_t>(p.batch, p.group_total)) * cols;
+    return (int64_t) ((p.M + BM - 1) / BM) * cols * p.batch;
+}
+
+// What a plain or batched product costs on these tiles, in K-tiles of a lock-step 256 x 256 tile on a full chip (1.77 us each): the fewer CUs have one, the
+// faster they run (their common power and L2; 1.2 us a K-tile with 128 of 256, 1.36 with 192, 1.5 with all), and the launch, its first requests and the results
+// take the time of eight.  A tile of up to 128 rows costs two thirds.
+inline double cost(const GemmParams& p, int es)
+{
+    const double tiles = (double) most_tiles(p), cus = launch_util::device_cus(), rounds = std::ceil(tiles / cus), fill = tiles / rounds / cus;
+    return rounds * ((double) ((int64_t) p.K * es / 128) * (0.56 + 0.29 * fill) * (p.M <= BM / 2 ? 0.65 : 1.0) + 1.0) + 7.0;
+}
+
+template <int WT, int OUT, bool GROUPED = false>
+int launch_out(const GemmParams& p, hipStream_t stream)
+{
+    const auto kernel = wide_kernel<WT, OUT, GROUPED>;
+    launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), LDS_BYTES);
+    const int64_t tiles = most_tiles(p), cus = launch_util::device_cus(), rounds = (tiles + cus - 1) / cus;
+    // even rounds: no workgroup has more than one tile more than another, and where some CUs have nothing to do the others run faster.  Grouped: a tile a
+    // workgroup, as tiles of few rows and of many follow one another (in rounds the same within 2 %)
+    const int64_t grid = GROUPED ? tiles : (tiles + rounds - 1) / rounds;
+    hipLaunchKernelGGL(kernel, dim3((unsigned) grid), dim3(64 * WAVES), LDS_BYTES, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+    {
+        set_error("gemm_wide launch failed: %s", hipGetErrorString(e));
+        return -1;
+    }
+    return 0;
+}
+
+// p: serves<W_BF16>(p)
+inline int launch_bf16(const GemmParams& p, hipStream_t stream)
+{
+    const bool fp32 = p.out_dtype == DT_FLOAT && p.seam.n_sec == 0 && p.act == GEMM_ACT_NONE;
+    if (p.group_off)
+        return p.act >= GEMM_ACT_GATE_SILU ? launch_out<W_BF16, OUT_GATED, true>(p, stream) : fp32 ? launch_out<W_BF16, OUT_FP32, true>(p, stream) : launch_out<W_BF16, OUT_STORE, true>(p, stream);
+    if (p.resid)
+        return p.gate ? launch_out<W_BF16, OUT_RESID_GATE>(p, stream) : launch_out<W_BF16, OUT_RESID>(p, stream);
+    return p.act >= GEMM_ACT_GATE_SILU ? launch_out<W_BF16, OUT_GATED>(p, stream) : fp32 ? launch_out<W_BF16, OUT_FP32>(p, stream) : launch_out<W_BF16, OUT_STORE>(p, stream);
+}
+
+} // namespace wide
+} // namespace
+} // namespace kernels
+} // namespace tllm

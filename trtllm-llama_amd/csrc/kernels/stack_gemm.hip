@@ -20,6 +20,7 @@
 #include "gemm_glds_impl.h"
 #include "gemm_seam.h"
 #include "gemm_slim_impl.h"
+#include "gemm_wide_impl.h"
 #include "stack_kernels.h"
 #include "stack_route_impl.h"
 #include <cmath>
@@ -680,6 +681,29 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
             return std::ceil(tiles * g.batch * ((g.N + bn - 1) / bn) / cus - rest) * bm * bn * f;
         };
         pick = m_expected <= 64 ? 0 : cost(256, 256, shapes[2].f, 0.02) < cost(128, 256, shapes[3].f, 0.08) ? 2 : 3;
+    }
+    // 256 x 256 tiles of gemm_wide_impl.h.  Grouped: where groups have two of them (32 groups, us, in brackets the shapes above: 16384 rows, N 2816, K 2048 227 (282), 12000
+    // 176 (202), 16384 rows, 704, 512 24 (34)).  Groups of one tile read their weights alone, from HBM, which a K-tile and a half ahead does not hide: 8192 rows,
+    // 5504, 4096 took 542 (500) in a step, the same rows of fewer columns by themselves 133 (141) at 2816, 2048 and 126 (121) with 6700 rows.
+    if (wide::serves<W_BF16>(g))
+    {
+        if (m_expected > 0)
+        {
+            // rounds of all groups' tiles, the last one of a group being there as often as not
+            auto tiles = [&](int bm, int bn) { return (std::ceil(m_expected / (double) bm) + 0.4) * g.batch * ((g.N + bn - 1) / bn) / cus; };
+            const Shape& sh = shapes[pick];
+            const double kt = g.K / 64;
+            if (m_expected >= 384 && std::max(1.0, tiles(256, 256)) * (kt * 0.85 + 1.5) + 4.0 < std::max(1.0, tiles(sh.bm, sh.bn)) * (kt * sh.bm * sh.bn * sh.f / 65536.0 + 4.0))
+                return wide::launch_bf16(g, stream);
+        }
+        else if (!g.group_off)
+        {
+            const Shape& sh = shapes[pick];
+            const int64_t tiles = (int64_t) ((g.M + sh.bm - 1) / sh.bm) * ((g.N + sh.bn - 1) / sh.bn) * (g.batch > 1 ? g.batch : 1);
+            // (a round of the lock-step tiles pays its first requests and its results each time: 2.5 K-tiles)
+            if (wide::cost(g, 2) < (double) ((tiles + cus - 1) / cus) * ((double) (g.K / 64) * sh.bm * sh.bn * sh.f / 65536.0 + 2.5))
+                return wide::launch_bf16(g, stream);
+        }
     }
     if (g.act == ACT_SCALE_CAP || g.act == ACT_GELU_MUL)
         pick = 0; // the shape whose epilogue has them
