@@ -33,6 +33,8 @@ using namespace dev;
 int gemm_tune_cfg = 0; // test/bench override of the tile shape (0 = heuristic)
 int launch_gemm_sqp(const GemmParams& p, int cfg, hipStream_t stream); // gemm_sqp.hip: phased SmoothQuant kernel, ids 13..
 int launch_gemm_f16p(const GemmParams& p, int cfg, hipStream_t stream); // gemm_sqp.hip: the same pipeline on fp16 operands, ids 50..
+int launch_gemm_wide(const GemmParams& p, hipStream_t stream); // gemm_wide.hip: 256 x 256 tiles of both types, id 80
+bool gemm_wide_beats(const GemmParams& p, double other);
 extern void* gemm_clock_probe;                                              // gemm_sqp.hip (microbench hook)
 
 namespace
@@ -53,6 +55,7 @@ constexpr int kPhased256x128 = 42;
 constexpr Shape kShapes[] = {{8, 128, 128, 1.40, 1.80}, {6, 256, 192, 1.0, 1.0}, {2, 256, 256, 1.04, 1.30}, {4, 128, 256, 1.39, 1.60},
     {kPhased256x128, 256, 128, 1.08, 1.37}};
 constexpr int kNumCfg = 12;
+constexpr int kWide = 80;
 
 template <int WT>
 int launch_wt(const GemmParams& p, int cfg, hipStream_t stream)
@@ -107,7 +110,7 @@ static bool glds_serves(const GemmParams& p)
 // The static rule: fewest workgroup rounds over the CUs x the tile's area x what a tile of that kind costs per area (the 128-wide
 // lock-step tiles pay ~40 % for their lower MFMA : LDS ratio and their exposed prologue / epilogue).  `phased_ok` = false leaves
 // out the tile that exists in gemm_sqp.hip only (its launcher refused the problem: alignment, 32-bit DMA offsets).
-static int static_shape_cfg(const GemmParams& p, bool phased_ok = true)
+static int static_shape_cfg(const GemmParams& p, bool phased_ok = true, bool wide_ok = true)
 {
     const int cus = launch_util::device_cus();
     double best = 1e30;
@@ -127,7 +130,10 @@ static int static_shape_cfg(const GemmParams& p, bool phased_ok = true)
             cfg = s.id;
         }
     }
-    return cfg;
+    // the tiles of gemm_wide.hip: both costs in K-tiles of 256 x 256 (a phased 256 x 192 tile takes 1.28 us a K-tile), the other kernels' first requests and
+    // results those of three
+    const double k_tiles = (double) ((int64_t) p.K * (p.wtype == W_INT8_SQ ? 1 : 2) / 128);
+    return wide_ok && gemm_wide_beats(p, best * 0.96 / 65536.0 * k_tiles + 3.0) ? kWide : cfg;
 }
 
 // the kernel id launch_gemm_glds runs for this problem when no profile entry exists (the tactic profiler's incumbent)
@@ -152,6 +158,8 @@ int launch_gemm_cfg(const GemmParams& p, int cfg, hipStream_t stream)
     if (!glds_serves(p))
         return 1;
     const bool sq = p.wtype == W_INT8_SQ;
+    if (cfg == kWide)
+        return launch_gemm_wide(p, stream);
     if ((cfg >= 1 && cfg <= kNumCfg) || cfg == 36 || cfg == 37)
     {
         // a tile far larger than the problem only burns time in the sweep
@@ -177,7 +185,7 @@ int launch_gemm_glds(const GemmParams& p, hipStream_t stream)
     const bool glds_id = (cfg >= 1 && cfg <= kNumCfg) || cfg == 36 || cfg == 37; // ids served by this file's table
     if (cfg > kNumCfg && !glds_id)
     {
-        const int r = sq ? launch_gemm_sqp(p, cfg, stream) : launch_gemm_f16p(p, cfg, stream);
+        const int r = cfg == kWide ? launch_gemm_wide(p, stream) : sq ? launch_gemm_sqp(p, cfg, stream) : launch_gemm_f16p(p, cfg, stream);
         if (r <= 0)
             return r;
         cfg = 0; // not served there (shape / alignment): the heuristic below picks a lock-step shape
@@ -185,6 +193,8 @@ int launch_gemm_glds(const GemmParams& p, hipStream_t stream)
     if (cfg <= 0 || !((cfg >= 1 && cfg <= kNumCfg) || cfg == 36 || cfg == 37))
     {
         cfg = static_shape_cfg(p);
+        if (cfg == kWide)
+            return launch_gemm_wide(p, stream);
         if (cfg == kPhased256x128)
         {
             // one round of 256 x 128 tiles where 128 x 128 would take two (O / down at M = 2048: 34 vs 44 us, 84 vs 107 us)
@@ -193,7 +203,7 @@ int launch_gemm_glds(const GemmParams& p, hipStream_t stream)
                 r = sq ? launch_gemm_sqp(p, 42, stream) : launch_gemm_f16p(p, 54, stream);
             if (r <= 0)
                 return r;
-            cfg = static_shape_cfg(p, false);
+            cfg = static_shape_cfg(p, false, false);
         }
     }
     if (!sq && cfg == 6 && gemm_tune_cfg <= 0 && !from_table)

@@ -13,6 +13,8 @@
 //     its clock falls with its power, 2.2 against 2.0 GHz in the same lock-step kernel.
 // All together 2640 - 2700 clocks.  bfloat16, us, in brackets what the lock-step tiles of 32 x 32 MFMAs took: 2048 x 22016 x 4096 gated 285 (350; in a step 315 (353)),
 // 4096 x 4096 x 4096 111 (123), 4096 x 8192 x 4096 210 = 1.31 PFLOP/s (265), 1024 x 13056 x 2048 gated 60 (63).
+// fp16, in brackets the best of the phased forms of gemm_sqp.hip and of the lock-step ones: 1200 x 12288 x 4096 103 (120), 1200 x 11008 x 4096 95 (112); int8 4096 x 12288 x 4096
+// 171 (184), 4096 x 4096 x 4096 59 (67), 4096 x 4096 x 11008 147 = 2.51 POP/s (168).  At 1024 rows, where 256 x 192 tiles fill the chip once, those are quicker (fp16 QKV 87, here 92).
 // Tried and slower: the DMA two at a time (+8 %), W's ahead of A's or in turn with them (+10 %), a fifth 64-byte stage, setprio by wave half.
 #pragma once
 #include "dev_utils.h"
@@ -268,7 +270,7 @@ __device__ __forceinline__ int rows_to_tiles(int rows)
     return (rows + BM - 1) / BM;
 }
 
-template <bool GROUPED>
+template <bool GROUPED, int COLS>
 struct Places
 {
     int tiles_n, total;
@@ -291,7 +293,7 @@ struct Places
     }
     __device__ __forceinline__ void begin(const GemmParams& p, int lane)
     {
-        tiles_n = (p.N + BN - 1) / BN;
+        tiles_n = (p.N + COLS - 1) / COLS;
         if constexpr (!GROUPED)
         {
             total = rows_to_tiles(p.M) * tiles_n * p.batch;
@@ -350,7 +352,7 @@ struct Places
         }
         const int tn = id / high;
         o.m0 = (band * BAND + id - tn * high) * BM;
-        o.n0 = tn * BN;
+        o.n0 = tn * COLS;
         return true;
     }
 };
@@ -362,11 +364,13 @@ enum Out
     OUT_GATED, // gated pairs of columns in front of the first section, 16-bit rows
     OUT_FP32,  // fp32 c alone
     OUT_RESID, // added to the fp32 residual
-    OUT_RESID_GATE // ... behind a sigmoid gate
+    OUT_RESID_GATE, // ... behind a sigmoid gate
+    OUT_HALF,  // fp16 rows of fp16 or int8 products: scales, fp16 residual or SwiGLU gate
+    OUT_DUAL   // two int8 products of the same rows: SwiGLU of both, quantised to int8
 };
 constexpr bool out_pairs(int out)
 {
-    return out == OUT_STORE || out == OUT_GATED;
+    return out != OUT_FP32 && out != OUT_RESID && out != OUT_RESID_GATE;
 }
 
 __device__ __forceinline__ float4 load4(const float* p)
@@ -485,6 +489,122 @@ __device__ __forceinline__ void leave_fp32(const GemmParams& p, const Tile<W_BF1
     }
 }
 
+// fp16 and int8 products: the scales of a lane's columns and rows, requested ahead of the K loop (behind it they would wait for the next tile's first requests)
+template <int WT, int OUT>
+struct Scales
+{
+    // int8: factors of the columns of block pair q (OUT_DUAL: of the first and the second product) and of the rows; fp16: weight-only's of a column
+    float col[NB / 2][8], row[WT == W_INT8_SQ && OUT == OUT_HALF ? NA : 1];
+
+    __device__ __forceinline__ void request(const GemmParams& p, int row0, int col0, int rows, int lane)
+    {
+#pragma unroll
+        for (int q = 0; q < NB / 2; ++q)
+        {
+            int c = col0 + (OUT == OUT_DUAL ? 0 : 32 * q) + 8 * (lane >> 4);
+            c = c < p.N ? c : 0;
+            if constexpr (WT == W_INT8_SQ)
+            {
+                const float* from = reinterpret_cast<const float*>(OUT == OUT_DUAL && q ? p.scale_col2 : p.scale_col);
+                if (p.per_channel)
+                {
+                    const float4 x = load4(from + c), y = load4(from + c + 4);
+                    col[q][0] = x.x, col[q][1] = x.y, col[q][2] = x.z, col[q][3] = x.w, col[q][4] = y.x, col[q][5] = y.y, col[q][6] = y.z, col[q][7] = y.w;
+                }
+                else
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        col[q][e] = from[0];
+            }
+            else
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    col[q][e] = p.scale_col ? h2f(reinterpret_cast<const uint16_t*>(p.scale_col)[c + e]) : 1.f;
+        }
+        if constexpr (WT == W_INT8_SQ)
+#pragma unroll
+            for (int i = 0; i < (int) (sizeof(row) / sizeof(row[0])); ++i)
+            {
+                const int m = row0 + i * 16;
+                row[i] = p.scale_row[OUT == OUT_HALF && p.per_token ? (m < rows ? m : rows - 1) : 0];
+            }
+    }
+};
+__device__ __forceinline__ uint32_t half_pair(float a, float b)
+{
+    return (uint32_t) f2h(a) | ((uint32_t) f2h(b) << 16);
+}
+template <int WT>
+__device__ __forceinline__ void leave_half(const GemmParams& p, const Tile<WT, true>& t, const Scales<WT, OUT_HALF>& sc, int row0, int col0, int rows)
+{
+    auto out = [&](auto finish) {
+#pragma unroll
+        for (int q = 0; q < NB / 2; ++q)
+        {
+            const int col = col0 + 32 * q + 8 * (t.lane >> 4);
+            if (col >= p.N)
+                continue;
+#pragma unroll
+            for (int i = 0; i < NA; ++i)
+            {
+                if (row0 + i * 16 >= rows)
+                    continue;
+                float v[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                {
+                    const auto a = t.acc[i][2 * q + (e >> 2)][e & 3];
+                    if constexpr (WT == W_INT8_SQ)
+                        v[e] = (float) a * (sc.col[q][e] * sc.row[i]);
+                    else
+                        v[e] = a * sc.col[q][e];
+                }
+                const int64_t at = (int64_t) (row0 + i * 16) * p.ldc + col;
+                *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.c) + at)
+                    = finish(make_uint4(half_pair(v[0], v[1]), half_pair(v[2], v[3]), half_pair(v[4], v[5]), half_pair(v[6], v[7])), at);
+            }
+        }
+    };
+    if (p.residual)
+        out([&](const uint4& v, int64_t at) {
+            const uint4 r = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.residual) + at);
+            const uint32_t a[4] = {v.x, v.y, v.z, v.w}, b[4] = {r.x, r.y, r.z, r.w};
+            uint32_t o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                o[e] = half_pair(h2f((uint16_t) (a[e] & 0xffffu)) + h2f((uint16_t) (b[e] & 0xffffu)), h2f((uint16_t) (a[e] >> 16)) + h2f((uint16_t) (b[e] >> 16)));
+            return make_uint4(o[0], o[1], o[2], o[3]);
+        });
+    else if (WT == W_FP16 && p.silu_gate)
+        out([&](const uint4& v, int64_t at) { return epi_silu_gate8(v, *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.silu_gate) + at)); });
+    else
+        out([](const uint4& v, int64_t) { return v; });
+}
+// rounded where two fp16 products, SwiGLU in fp16 and the static quantiser would round
+__device__ __forceinline__ void leave_dual(const GemmParams& p, const Tile<W_INT8_SQ, true>& t, const Scales<W_INT8_SQ, OUT_DUAL>& sc, int row0, int col0, int rows)
+{
+    const int col = col0 + 8 * (t.lane >> 4);
+    if (col >= p.N)
+        return;
+    const float qs = p.swiglu_qscale[0], sr2 = p.scale_row2 ? p.scale_row2[0] : p.scale_row[0];
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+    {
+        uint32_t o[2] = {0, 0};
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+        {
+            const float g16 = h2f(f2h((float) t.acc[i][e >> 2][e & 3] * (sc.col[0][e] * sc.row[0])));
+            const float u16 = h2f(f2h((float) t.acc[i][2 + (e >> 2)][e & 3] * (sc.col[1][e] * sr2)));
+            const float a16 = h2f(f2h(g16 / (1.f + __expf(-g16))));
+            const float o16 = h2f(f2h(a16 * u16));
+            o[e >> 2] |= ((uint32_t) (uint8_t) f2i8_rni_sat(o16 * qs)) << (8 * (e & 3));
+        }
+        if (row0 + i * 16 < rows)
+            *reinterpret_cast<uint2*>(reinterpret_cast<int8_t*>(p.c) + (int64_t) (row0 + i * 16) * p.ldc + col) = make_uint2(o[0], o[1]);
+    }
+}
+
 // Persistent: a workgroup per CU (fewer where that makes the rounds even) walks its tiles; the next tile's first two K-tiles are under way while this
 // one's results leave, straight from the accumulators (16 rows x 64 bytes a store, no LDS).  The code in front of the first request runs cold: one copy
 // of it serves the first tile and the others (2.2 us with two, a batch's and a group's places in one instance and K-tile 1's requests unrolled).
@@ -500,9 +620,11 @@ __global__ __launch_bounds__(64 * WAVES) void wide_kernel(const GemmParams p)
     t.wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     t.lds = (uint32_t) (uintptr_t) (lds_ptr*) wide_lds;
     t.nt = p.K * ES / 128;
-    Places<GROUPED> places;
+    constexpr bool DUAL = OUT == OUT_DUAL;
+    Places<GROUPED, DUAL ? BN / 2 : BN> places;
     places.begin(p, t.lane);
     Place now = {}, next;
+    Scales<WT, OUT> scales;
     for (int round = 0;; ++round)
     {
         const bool more = places.at(p, round, t.lane, next);
@@ -511,7 +633,7 @@ __global__ __launch_bounds__(64 * WAVES) void wide_kernel(const GemmParams p)
         {
             const int row8 = t.wid * 8 + (t.lane >> 3), piece = t.lane & 7;
             t.a = reinterpret_cast<const char*>(p.a);
-            t.w = reinterpret_cast<const char*>(p.w);
+            t.w = reinterpret_cast<const char*>(DUAL && t.wid >= WAVES / 2 ? p.w2 : p.w);
             if (WT == W_BF16 && (GROUPED || p.batch > 1))
             {
                 t.a += GROUPED ? 0 : next.product * p.batch_a;
@@ -529,23 +651,28 @@ __global__ __launch_bounds__(64 * WAVES) void wide_kernel(const GemmParams p)
 #pragma unroll
             for (int i = 0; i < DMA_W; ++i)
             {
-                const int row = i * WAVES * 8 + row8, n = next.n0 + row < p.N ? next.n0 + row : p.N - 1;
+                // two products: the first 32 of a wave's 64 rows are the first matrix's, the others the second one's
+                const int row = i * WAVES * 8 + row8, col = next.n0 + (DUAL ? 32 * i + (row8 & 31) : row), n = col < p.N ? col : p.N - 1;
                 t.wo[i] = (uint32_t) n * (uint32_t) p.ldw + ((piece ^ w_swz<PAIRS>(row)) << 4);
             }
             t.head(half);
         }
+        const int row0 = now.m0 + t.wid / WN * (NA * 16) + (t.lane & 15), col0 = now.n0 + t.wid % WN * (DUAL ? NB * 8 : NB * 16);
         if (round > 0)
         {
-            char* c = reinterpret_cast<char*>(p.c);
             if constexpr (WT == W_BF16)
             {
+                char* c = reinterpret_cast<char*>(p.c);
                 c += GROUPED ? now.first * p.ldc * (p.out_dtype == DT_FLOAT ? 4 : 2) : now.product * p.batch_c;
-                const int row0 = now.m0 + t.wid / WN * (NA * 16) + (t.lane & 15), col0 = now.n0 + t.wid % WN * (NB * 16);
                 if constexpr (PAIRS)
                     leave_pairs<OUT>(p, t, c, row0, col0, now.rows);
                 else
                     leave_fp32<OUT>(p, t, c, row0, col0, now.rows);
             }
+            else if constexpr (DUAL)
+                leave_dual(p, t, scales, row0, col0, now.rows);
+            else
+                leave_half<WT>(p, t, scales, row0, col0, now.rows);
         }
         if (!more)
             return;
@@ -559,6 +686,8 @@ __global__ __launch_bounds__(64 * WAVES) void wide_kernel(const GemmParams p)
         }
         else
             wait_vm_and_meet<0>(); // (the results of the tile before have left, too)
+        if constexpr (WT != W_BF16)
+            scales.request(p, now.m0 + t.wid / WN * (NA * 16) + (t.lane & 15), now.n0 + t.wid % WN * (DUAL ? NB * 8 : NB * 16), now.rows, t.lane);
 #pragma unroll
         for (int i = 0; i < NA; ++i)
 #pragma unroll
@@ -608,13 +737,25 @@ bool serves(const GemmParams& p)
         }
         return true;
     }
-    return false;
+    else
+    {
+        const bool dual = WT == W_INT8_SQ && p.w2;
+        if (p.out_dtype != DT_HALF && !dual)
+            return false;
+        if (p.ldc % 8 || reinterpret_cast<uintptr_t>(p.c) % (dual ? 8 : 16) || (p.residual && (dual || !aligned16(p.residual))) || (p.silu_gate && (WT != W_FP16 || p.residual || !aligned16(p.silu_gate))))
+            return false;
+        if constexpr (WT == W_INT8_SQ)
+            return p.scale_col && p.scale_row && (!p.per_channel || aligned16(p.scale_col))
+                && (!dual || (p.scale_col2 && p.swiglu_qscale && !p.per_token && aligned16(p.w2) && (!p.per_channel || aligned16(p.scale_col2))));
+        return true;
+    }
 }
 
 // at most this many tiles (grouped: full ones, and one begun in every group that has rows)
 inline int64_t most_tiles(const GemmParams& p)
 {
-    const int64_t cols = (p.N + BN - 1) / BN;
+    const int of_tile = p.wtype == W_INT8_SQ && p.w2 ? BN / 2 : BN;
+    const int64_t cols = (p.N + of_tile - 1) / of_tile;
     if (p.group_off)
         return (p.group_total / BM + std::min<int64_t>(p.batch, p.group_total)) * cols;
     return (int64_t) ((p.M + BM - 1) / BM) * cols * p.batch;
@@ -648,15 +789,23 @@ int launch_out(const GemmParams& p, hipStream_t stream)
     return 0;
 }
 
-// p: serves<W_BF16>(p)
-inline int launch_bf16(const GemmParams& p, hipStream_t stream)
+// p: serves<WT>(p)
+template <int WT>
+int launch(const GemmParams& p, hipStream_t stream)
 {
-    const bool fp32 = p.out_dtype == DT_FLOAT && p.seam.n_sec == 0 && p.act == GEMM_ACT_NONE;
-    if (p.group_off)
-        return p.act >= GEMM_ACT_GATE_SILU ? launch_out<W_BF16, OUT_GATED, true>(p, stream) : fp32 ? launch_out<W_BF16, OUT_FP32, true>(p, stream) : launch_out<W_BF16, OUT_STORE, true>(p, stream);
-    if (p.resid)
-        return p.gate ? launch_out<W_BF16, OUT_RESID_GATE>(p, stream) : launch_out<W_BF16, OUT_RESID>(p, stream);
-    return p.act >= GEMM_ACT_GATE_SILU ? launch_out<W_BF16, OUT_GATED>(p, stream) : fp32 ? launch_out<W_BF16, OUT_FP32>(p, stream) : launch_out<W_BF16, OUT_STORE>(p, stream);
+    if constexpr (WT == W_BF16)
+    {
+        const bool gated = p.act >= GEMM_ACT_GATE_SILU, fp32 = p.out_dtype == DT_FLOAT && p.seam.n_sec == 0 && p.act == GEMM_ACT_NONE;
+        if (p.group_off)
+            return gated ? launch_out<WT, OUT_GATED, true>(p, stream) : fp32 ? launch_out<WT, OUT_FP32, true>(p, stream) : launch_out<WT, OUT_STORE, true>(p, stream);
+        if (p.resid)
+            return p.gate ? launch_out<WT, OUT_RESID_GATE>(p, stream) : launch_out<WT, OUT_RESID>(p, stream);
+        return gated ? launch_out<WT, OUT_GATED>(p, stream) : fp32 ? launch_out<WT, OUT_FP32>(p, stream) : launch_out<WT, OUT_STORE>(p, stream);
+    }
+    else if constexpr (WT == W_INT8_SQ)
+        return p.w2 ? launch_out<WT, OUT_DUAL>(p, stream) : launch_out<WT, OUT_HALF>(p, stream);
+    else
+        return launch_out<WT, OUT_HALF>(p, stream);
 }
 
 } // namespace wide

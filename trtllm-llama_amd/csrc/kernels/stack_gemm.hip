@@ -694,7 +694,7 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
             const Shape& sh = shapes[pick];
             const double kt = g.K / 64;
             if (m_expected >= 384 && std::max(1.0, tiles(256, 256)) * (kt * 0.85 + 1.5) + 4.0 < std::max(1.0, tiles(sh.bm, sh.bn)) * (kt * sh.bm * sh.bn * sh.f / 65536.0 + 4.0))
-                return wide::launch_bf16(g, stream);
+                return wide::launch<W_BF16>(g, stream);
         }
         else if (!g.group_off)
         {
@@ -702,7 +702,7 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
             const int64_t tiles = (int64_t) ((g.M + sh.bm - 1) / sh.bm) * ((g.N + sh.bn - 1) / sh.bn) * (g.batch > 1 ? g.batch : 1);
             // (a round of the lock-step tiles pays its first requests and its results each time: 2.5 K-tiles)
             if (wide::cost(g, 2) < (double) ((tiles + cus - 1) / cus) * ((double) (g.K / 64) * sh.bm * sh.bn * sh.f / 65536.0 + 2.5))
-                return wide::launch_bf16(g, stream);
+                return wide::launch<W_BF16>(g, stream);
         }
     }
     if (g.act == ACT_SCALE_CAP || g.act == ACT_GELU_MUL)
