@@ -22,6 +22,7 @@
 #include "gemm_slim_impl.h"
 #include "gemm_wide_impl.h"
 #include "stack_kernels.h"
+#include "stack_norm_impl.h"
 #include "stack_route_impl.h"
 #include <cmath>
 
@@ -390,6 +391,72 @@ __global__ __launch_bounds__(256) void row_short_kernel(const StackGemmParams p_
             row_seam(p, ops[i], n0 + SK_R * i, sum[SK_R * i], sum[SK_R * i + 1]);
 }
 
+// row_kernel whose row is formed here (StackRowNorm) instead of by a launch of its own in front, which costs its start and 2.3 us for some hundred cycles of work: the
+// row is requested ahead of the weights and normed while they are under way.  K <= 512 KS NC.  Rows of more than 2048 values by whole waves, 8 columns a workgroup, as
+// every workgroup reads the row (10240 x 4096 by 2 columns a workgroup 21.6), but for few columns.  us in a step of one token, norm + product and here: 10304 x 2048 2.3 + 11.0, 10.7;
+// 11008 x 2048 2.3 + 11.2, 11.2; 10240 x 4096 4.6 + 14.7, 17.1; 16384 x 4096 4.6 + 21.0, 23.8.
+template <int KS, int NC, int NP>
+__global__ __launch_bounds__(256) void row_norm_kernel(const StackGemmParams p, const StackRowNorm n)
+{
+    constexpr int TEAMS = 4 / KS;
+    __shared__ __attribute__((aligned(16))) uint16_t row[NP * 1024];
+    __shared__ float red[4], part[4][SK_R];
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kw = wid % KS;
+    const int n0 = (blockIdx.x * TEAMS + wid / KS) * SK_R;
+    LoneRow<NP> lone;
+    lone.request(n, p.K);
+    uint4 wv[NC][SK_R];
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+    {
+        const int k = (kw + i * KS) * 512 + lane * 8;
+#pragma unroll
+        for (int r = 0; r < SK_R; ++r)
+            wv[i][r] = ld_nt16(reinterpret_cast<const uint16_t*>(p.w) + (int64_t) (n0 + r < p.N ? n0 + r : p.N - 1) * p.ldw + (k < p.K ? k : 0));
+    }
+    const RowSeam ops = row_seam_request(p, n0 < p.N ? n0 : p.N - 1);
+    lone.finish(n, p.K, row, red, blockIdx.x == 0);
+    float acc[SK_R] = {0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+    {
+        const int k = (kw + i * KS) * 512 + lane * 8;
+        const bool in = k < p.K;
+        const uint4 xv = *reinterpret_cast<const uint4*>(row + (in ? k : 0));
+        const uint32_t xs[4] = {in ? xv.x : 0u, in ? xv.y : 0u, in ? xv.z : 0u, in ? xv.w : 0u};
+#pragma unroll
+        for (int r = 0; r < SK_R; ++r)
+        {
+            const uint32_t ws[4] = {in ? wv[i][r].x : 0u, in ? wv[i][r].y : 0u, in ? wv[i][r].z : 0u, in ? wv[i][r].w : 0u};
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+            {
+                acc[r] = fmaf(__builtin_bit_cast(float, xs[q] << 16), __builtin_bit_cast(float, ws[q] << 16), acc[r]);
+                acc[r] = fmaf(__builtin_bit_cast(float, xs[q] & 0xffff0000u), __builtin_bit_cast(float, ws[q] & 0xffff0000u), acc[r]);
+            }
+        }
+    }
+    float v0 = wave_sum(acc[0]), v1 = wave_sum(acc[1]);
+    if constexpr (KS > 1)
+    {
+        if (lane == 0)
+        {
+            part[wid][0] = v0;
+            part[wid][1] = v1;
+        }
+        __syncthreads();
+        v0 = part[wid - kw][0], v1 = part[wid - kw][1];
+#pragma unroll
+        for (int k = 1; k < KS; ++k)
+        {
+            v0 += part[wid - kw + k][0];
+            v1 += part[wid - kw + k][1];
+        }
+    }
+    if (lane == 0 && kw == 0 && n0 < p.N)
+        row_seam(p, ops, n0, v0, v1);
+}
+
 // A lone token's experts, product z = choice z.  up: every wave chooses from the logits by itself (some 0.8 us in front of its weights' requests), which
 // replaces a launch that orders pairs: a last workgroup that waits for all logits, chooses, orders and copies.  Choice, order and products of
 // a layer of 32 + 2 outputs, width 2048, in a step of one token: 9.5 us for the router's launch, 3.7 for its logits alone.
@@ -722,6 +789,41 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
 }
 
 } // namespace
+
+bool stack_row_norm_serves(const StackRowNorm& n, int dtype, int width)
+{
+    auto pieces = [](const void* p) { return !(reinterpret_cast<uintptr_t>(p) & 15); };
+    return dtype == DT_BF16 && width % 16 == 0 && width > 0 && width <= 4096 && (n.groups == 1 || n.groups == 2 || n.groups == 4) && n.x && n.w && pieces(n.x) && pieces(n.y)
+        && pieces(n.w) && pieces(n.w2) && pieces(n.h) && pieces(n.h2) && pieces(n.x_out) && (!n.y || (n.mix && n.out && n.x_out && n.x_out != n.x)) && (!n.h2 || n.w2);
+}
+
+int launch_stack_row_gemm(const StackGemmParams& p_in, const StackRowNorm& n, hipStream_t stream)
+{
+    StackGemmParams p = p_in;
+    if (p.ldw == 0)
+        p.ldw = p.K;
+    if (p.M != 1 || p.batch != 1 || p.group_off || p.a_rows || p.N <= 0 || !p.w || (!p.c && !p.resid) || !stack_row_norm_serves(n, p.dtype, p.K) || (reinterpret_cast<uintptr_t>(p.w) & 15)
+        || p.ldw % 8 || p.ldw < p.K || p.ldw >= (1 << 26) || p.act == ACT_GELU_MUL || p.act == ACT_SCALE_CAP
+        || (p.act >= ACT_GATE_SILU && (p.resid || ((p.seam.n_sec > 0 ? p.seam.sec[0].col0 : p.N) & 1))))
+        return 1;
+    const bool many = p.N > 16 * launch_util::device_cus(); // as in pick_row_shape
+    auto go = [&](auto shape, auto np) {
+        using S = decltype(shape);
+        hipLaunchKernelGGL((row_norm_kernel<S::KS, S::NC, decltype(np)::value>), dim3((p.N + S::cols - 1) / S::cols), dim3(256), 0, stream, p, n);
+    };
+    using Quarter1 = std::integral_constant<int, 1>; // pieces of a lane
+    using Quarter2 = std::integral_constant<int, 2>;
+    using Quarter4 = std::integral_constant<int, 4>;
+    if (p.K <= 512)
+        go(RowShape<1, 1>(), Quarter1());
+    else if (p.K <= 1024)
+        many ? go(RowShape<1, 2>(), Quarter1()) : go(RowShape<2, 1>(), Quarter1());
+    else if (p.K <= 2048)
+        many ? go(RowShape<1, 4>(), Quarter2()) : go(RowShape<4, 1>(), Quarter2());
+    else
+        p.N < 8 * launch_util::device_cus() ? go(RowShape<4, 2>(), Quarter4()) : go(RowShape<1, 8>(), Quarter4());
+    return launched("stack_gemm row and norm");
+}
 
 bool stack_lone_serves(const StackMoeParams& m, const StackGemmParams& up, const StackGemmParams& down)
 {

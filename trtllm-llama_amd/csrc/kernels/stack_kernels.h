@@ -68,6 +68,24 @@ struct StackGemmParams
     int32_t group_rows = 0; // the rows a group is expected to have (tile shapes are chosen for it), 0: M
 };
 int launch_stack_gemm(const StackGemmParams& p, hipStream_t stream);
+// A lone token's row as the one launch reads it that needs it: every workgroup forms v = x, or mix[0] x + out[0] y where there is a y, and
+//   row = bfloat16(u / sqrt(mean(u^2) + eps) * w),  u = in[0] v (in null: v), the mean over each of `groups` (1, 2 or 4) parts of the row.
+// The first workgroup leaves v in x_out (not x itself, which others still read; with a y only), the row in h and the row of weights w2 in h2, where they are set.
+// bfloat16, rows of up to 4096 values in whole pieces of 16 (stack_row_norm_serves).
+struct StackRowNorm
+{
+    const float* x = nullptr;
+    const float* y = nullptr;
+    const float *mix = nullptr, *out = nullptr, *in = nullptr;
+    const float *w = nullptr, *w2 = nullptr;
+    float eps = 1e-5f;
+    int32_t groups = 1;
+    float* x_out = nullptr;
+    void *h = nullptr, *h2 = nullptr;
+};
+bool stack_row_norm_serves(const StackRowNorm& n, int dtype, int width);
+// launch_stack_gemm of one row, that row (a is not read); 1: not served, nothing was launched
+int launch_stack_row_gemm(const StackGemmParams& p, const StackRowNorm& n, hipStream_t stream);
 
 // ---------------------------------------------------------------------------------------------
 // Pointwise pieces.
@@ -445,6 +463,7 @@ bool stack_lone_serves(const StackMoeParams& m, const StackGemmParams& up, const
 int launch_stack_lone_up(const StackMoeParams& m, const StackGemmParams& up, hipStream_t stream);
 int launch_stack_lone_down(const StackMoeParams& m, const StackGemmParams& down, hipStream_t stream);
 int launch_stack_moe_logits(const StackMoeParams& p, hipStream_t stream); // the router's logits alone
+int launch_stack_moe_logits(const StackMoeParams& p, const StackRowNorm& n, hipStream_t stream); // of one token, whose row h they form
 int launch_stack_moe_combine(const StackMoeParams& p, const float* y_sorted, float* y, hipStream_t stream);
 
 // ---------------------------------------------------------------------------------------------

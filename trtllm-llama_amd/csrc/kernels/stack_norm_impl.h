@@ -1,0 +1,97 @@
+// A lone token's normed row, formed by the workgroups that read it (stack_kernels.h, StackRowNorm): shared by its products (stack_gemm.hip) and its
+// router's logits (stack_moe.hip).  Everything has internal linkage.
+#pragma once
+#include "dev_utils.h"
+#include "stack_kernels.h"
+
+namespace tllm
+{
+namespace kernels
+{
+namespace
+{
+using namespace dev;
+
+// A workgroup of 4 waves; wave q has the q-th quarter of the row, NP pieces of 4 values a lane, so that up to 4 parts with a norm each end where a wave does.
+template <int NP>
+struct LoneRow
+{
+    float4 x[NP], y[NP], w[NP];
+    float cm, co, ci;
+
+    __device__ __forceinline__ static int piece(int width, int k, bool& on)
+    {
+        const int quarter = width >> 4, i = (threadIdx.x & 63) + 64 * k;
+        on = i < quarter;
+        return (int) (threadIdx.x >> 6) * quarter + (on ? i : 0);
+    }
+    // all loads, without a branch that they would wait behind; ahead of the operands that they are to arrive before
+    __device__ __forceinline__ void request(const StackRowNorm& n, int width)
+    {
+        const float* y_or_x = n.y ? n.y : n.x;
+        cm = n.y ? n.mix[0] : 1.f;
+        co = n.y ? n.out[0] : 0.f;
+        ci = n.in ? n.in[0] : 1.f;
+#pragma unroll
+        for (int k = 0; k < NP; ++k)
+        {
+            bool on;
+            const int c = piece(width, k, on);
+            x[k] = reinterpret_cast<const float4*>(n.x)[c];
+            y[k] = reinterpret_cast<const float4*>(y_or_x)[c];
+            w[k] = reinterpret_cast<const float4*>(n.w)[c];
+        }
+        asm volatile("" ::: "memory"); // (what is requested next does not go in front)
+    }
+    // row: LDS [width], the normed row in bfloat16; red: LDS [4].  first: this workgroup also leaves what later launches read.
+    __device__ __forceinline__ void finish(const StackRowNorm& n, int width, uint16_t* row, float* red, bool first)
+    {
+        const int wid = threadIdx.x >> 6;
+        float ss = 0.f;
+#pragma unroll
+        for (int k = 0; k < NP; ++k)
+        {
+            bool on;
+            const int c = piece(width, k, on);
+            float4 v = x[k];
+            if (n.y)
+            {
+                v = make_float4(fmaf(co, y[k].x, cm * v.x), fmaf(co, y[k].y, cm * v.y), fmaf(co, y[k].z, cm * v.z), fmaf(co, y[k].w, cm * v.w));
+                if (first && on)
+                    reinterpret_cast<float4*>(n.x_out)[c] = v;
+            }
+            v = make_float4(ci * v.x, ci * v.y, ci * v.z, ci * v.w);
+            x[k] = v;
+            ss += on ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f;
+        }
+        ss = wave_sum(ss);
+        if ((threadIdx.x & 63) == 0)
+            red[wid] = ss;
+        __syncthreads();
+        ss = n.groups == 4 ? red[wid] : n.groups == 2 ? red[wid & 2] + red[wid | 1] : (red[0] + red[1]) + (red[2] + red[3]);
+        const float inv = 1.f / sqrtf(ss / (float) (width / n.groups) + n.eps);
+#pragma unroll
+        for (int k = 0; k < NP; ++k)
+        {
+            bool on;
+            const int c = piece(width, k, on);
+            auto normed = [&](const float4& s) {
+                return make_uint2((uint32_t) f2bf(x[k].x * inv * s.x) | ((uint32_t) f2bf(x[k].y * inv * s.y) << 16),
+                    (uint32_t) f2bf(x[k].z * inv * s.z) | ((uint32_t) f2bf(x[k].w * inv * s.w) << 16));
+            };
+            if (!on)
+                continue;
+            const uint2 h = normed(w[k]);
+            reinterpret_cast<uint2*>(row)[c] = h;
+            if (first && n.h)
+                reinterpret_cast<uint2*>(n.h)[c] = h;
+            if (first && n.h2)
+                reinterpret_cast<uint2*>(n.h2)[c] = normed(reinterpret_cast<const float4*>(n.w2)[c]);
+        }
+        __syncthreads();
+    }
+};
+
+} // namespace
+} // namespace kernels
+} // namespace tllm

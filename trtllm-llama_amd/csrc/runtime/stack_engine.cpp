@@ -1473,7 +1473,8 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
     s->tap_tokens = T;
 
     // P1 = h1 W_mix^T, then the mixer: its context rows land in s->ctx, ld_ctx elements apart
-    auto run_mixer = [&](const Layer& l, const Run& r) -> int {
+    // first(g): launches it, its row in s->h1 or formed on the way
+    auto run_mixer = [&](const Layer& l, const Run& r, auto first) -> int {
         const int64_t ld_ctx = l.n_ctx + (s->side_by_side && l.kind == MIX_LATENT ? l.shared_ff : 0);
         StackGemmParams g;
         g.dtype = s->dtype;
@@ -1504,7 +1505,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             sec.f32 = 1;
             g.N += l.n_route;
         }
-        if (launch_stack_gemm(g, stream))
+        if (first(g))
             return -1;
         if (l.kind == MIX_DELTA)
         {
@@ -1790,8 +1791,9 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
     };
 
     // the routed feed-forward on h1: y = its output, or (accumulate) y += it, x_el = the resulting rows in the element type; later != null: what y
-    // stands for, for the norm that reads it.  With residual=plain the router's logits are there already.
-    auto run_moe = [&](const Layer& l, float* y, bool accumulate, void* y_el, StackExpertSum* later) -> int {
+    // stands for, for the norm that reads it.  With residual=plain the router's logits are there already.  form(mp): h1 is still to be formed, by a launch of its own
+    // or (mp != null) by the one of mp's logits; 1: those are there.
+    auto run_moe = [&](const Layer& l, float* y, bool accumulate, void* y_el, StackExpertSum* later, auto form) -> int {
         const size_t pairs = (size_t) T * l.top;
         StackMoeParams mp;
         mp.dtype = s->dtype;
@@ -1860,9 +1862,13 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         dn.group_rows = u.group_rows;
         StackGemmParams lone = u; // (reads the token's row itself, also where it counts weighted)
         lone.a = s->h1;
-        if (stack_lone_serves(mp, lone, dn))
+        const bool choosing = stack_lone_serves(mp, lone, dn);
+        const int formed = form(choosing && !mp.have_logits ? &mp : nullptr);
+        if (formed < 0)
+            return -1;
+        if (choosing)
         {
-            if ((!mp.have_logits && launch_stack_moe_logits(mp, stream)) || launch_stack_lone_up(mp, lone, stream) || launch_stack_lone_down(mp, dn, stream))
+            if ((!mp.have_logits && !formed && launch_stack_moe_logits(mp, stream)) || launch_stack_lone_up(mp, lone, stream) || launch_stack_lone_down(mp, dn, stream))
                 return -1;
         }
         else if (launch_stack_moe_plan(mp, stream) || launch_stack_gemm(u, stream) || launch_stack_gemm(dn, stream))
@@ -1886,8 +1892,11 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
 
     StackExpertSum left_sum; // what y32 stands for where the last sublayer was a mixture of experts
 
+    auto product = [&](const StackGemmParams& g) { return launch_stack_gemm(g, stream); };
+    auto formed_before = [](const StackMoeParams*) { return 0; };
+
     // the feed-forwards of sequential blocks: h1 -> y32
-    auto seq_dense = [&](const Layer& l) -> int {
+    auto seq_dense = [&](const Layer& l, auto first) -> int {
         StackGemmParams u;
         u.dtype = s->dtype;
         u.M = T;
@@ -1899,7 +1908,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         u.c = s->act;
         u.ldc = l.ff;
         u.act = l.mlp == MLP_RELU2 ? ACT_RELU2 : ACT_GATE_GELU;
-        if (launch_stack_gemm(u, stream))
+        if (first(u))
             return -1;
         StackGemmParams dn;
         dn.dtype = s->dtype;
@@ -1914,10 +1923,13 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         dn.ldc = Wd;
         return launch_stack_gemm(dn, stream);
     };
-    auto seq_moe = [&](const Layer& l) -> int {
+    auto seq_moe = [&](const Layer& l, auto form) -> int {
         // what reads the row beside the experts, one product: the shared expert's first matrices, with residual=plain the router's logits,
         // the shared expert's gate (both in fp32)
         const int n_z = s->plain ? l.experts + l.identity : 0;
+        const bool alone = l.n_shared + n_z == 0; // nothing but the routed layer reads h1
+        if (!alone && form(nullptr) < 0)
+            return -1;
         StackGemmParams u;
         u.dtype = s->dtype;
         u.M = T;
@@ -1970,7 +1982,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             if (launch_stack_gemm(sd, stream))
                 return -1;
         }
-        return run_moe(l, s->y32, l.shared_ff > 0, nullptr, &left_sum);
+        return run_moe(l, s->y32, l.shared_ff > 0, nullptr, &left_sum, [&](const StackMoeParams* mp) { return alone ? form(mp) : 0; });
     };
 
     // residual=plain: what the last sublayer or token input left to land in y32, and the next norm, in one launch
@@ -2012,13 +2024,14 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
     // residual=hyper: the sublayer result in y32 that has not yet been folded into the streams, and the launch that folds it,
     // combines the streams for the next reader and norms the combination
     const HyperW* pending = nullptr;
+    float* xs = s->x; // the streams; a lone token's single one changes places with x0 where a launch folds a result in that others read at the same time
     auto hyper = [&](const float* in, void* h, const float* w, float* sum_out, float* h32 = nullptr) -> int {
         StackHyperParams hp;
         hp.dtype = s->dtype;
         hp.tokens = T;
         hp.width = Wd;
         hp.streams = s->streams;
-        hp.x = s->x;
+        hp.x = xs;
         hp.stream_stride = stream_stride;
         if (pending)
         {
@@ -2038,6 +2051,33 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         return launch_stack_hyper_norm(hp, stream);
     };
 
+    // A lone token's normed row is formed by the launch that reads it, launch(row), where that is the only one, or the first and leaves it for the others; 1: it is not.
+    // (what waits for the stream as a sum of experts is formed once, by the norm's own launch)
+    auto lone_row = [&](const float* in, const float* w, void* h, auto launch) -> int {
+        if (T != 1 || !s->hyper || s->streams != 1 || s->taps || (pending && left_sum.ys))
+            return 1;
+        StackRowNorm n;
+        n.x = xs;
+        if (pending)
+        {
+            n.y = s->y32;
+            n.mix = pending->mix;
+            n.out = pending->out;
+            n.x_out = xs == s->x ? s->x0 : s->x;
+        }
+        n.in = in;
+        n.w = w;
+        n.eps = s->eps;
+        n.h = h;
+        const int rc = launch(n);
+        if (rc == 0)
+        {
+            xs = pending ? n.x_out : xs;
+            pending = nullptr;
+        }
+        return rc;
+    };
+
     for (size_t ri = 0; ri < s->runs.size(); ++ri)
     {
         const Run& r = s->runs[ri];
@@ -2047,7 +2087,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             if (land(s->h1, l.norm1, r.enters_pass ? s->loop_step + (size_t) r.pass * Wd : nullptr, nullptr, T,
                     s->taps && ri > 0 ? s->tap + (ri - 1) * (size_t) T * Wd : nullptr, ri == 0))
                 return -1;
-            if (run_mixer(l, r))
+            if (run_mixer(l, r, product))
                 return -1;
             const bool joint = l.kind == MIX_LATENT && l.shared_ff > 0;
             StackGemmParams o; // x += [ctx | a_shared] [Wo | Wshared_down]^T
@@ -2071,7 +2111,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
                 if (launch_stack_gemm(o, stream))
                     return -1;
             }
-            if (l.ff > 0 && run_moe(l, s->x, true, s->side_dim ? s->x_el : nullptr, nullptr))
+            if (l.ff > 0 && run_moe(l, s->x, true, s->side_dim ? s->x_el : nullptr, nullptr, formed_before))
                 return -1;
             if (s->side_dim > 0)
             {
@@ -2140,15 +2180,26 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
                 if (hyper(l.hc[0].in, nullptr, l.norm1, nullptr, s->h32) || launch_stack_token_shift(sh, stream))
                     return -1;
             }
-            else if (hyper(l.hc[0].in, s->h1, l.norm1, nullptr))
-                return -1;
             // a sublayer's result waits in y32 for the next launch that reads the stream
             auto leave = [&](int sub) {
                 pending = &l.hc[sub];
                 land_y = true;
                 land_norm = sub ? l.norm2b : l.norm1b;
             };
-            if (run_mixer(l, r))
+            // g reads the row that norm1 or norm2 forms; with residual=plain and behind a token shift it is there
+            auto normed = [&](const StackGemmParams& g, int sub) -> int {
+                const float *in = l.hc[sub].in, *w = sub ? l.norm2 : l.norm1;
+                if (!s->plain && !(s->token_shift && sub == 0))
+                {
+                    const int rc = lone_row(in, w, nullptr, [&](const StackRowNorm& n) { return launch_stack_row_gemm(g, n, stream); });
+                    if (rc <= 0)
+                        return rc;
+                    if (hyper(in, s->h1, w, nullptr))
+                        return -1;
+                }
+                return launch_stack_gemm(g, stream);
+            };
+            if (run_mixer(l, r, [&](const StackGemmParams& g) { return normed(g, 0); }))
                 return -1;
             StackGemmParams o; // y = ctx Wo^T in fp32: the residual sum is 32-bit
             o.dtype = s->dtype;
@@ -2167,9 +2218,17 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             leave(0);
             if (l.ff > 0)
             {
-                if (s->plain ? land(s->h1, l.norm2, nullptr, nullptr, T, nullptr, false) : hyper(l.hc[1].in, s->h1, l.norm2, nullptr))
+                if (s->plain && land(s->h1, l.norm2, nullptr, nullptr, T, nullptr, false))
                     return -1;
-                if (l.mlp == MLP_MOE ? seq_moe(l) : seq_dense(l))
+                auto form = [&](const StackMoeParams* mp) -> int {
+                    if (s->plain)
+                        return 0;
+                    const int rc = mp ? lone_row(l.hc[1].in, l.norm2, s->h1, [&](const StackRowNorm& n) {
+                        return stack_row_norm_serves(n, s->dtype, Wd) ? launch_stack_moe_logits(*mp, n, stream) : 1;
+                    }) : 1;
+                    return rc <= 0 ? (rc == 0 ? 1 : -1) : hyper(l.hc[1].in, s->h1, l.norm2, nullptr);
+                };
+                if (l.mlp == MLP_MOE ? seq_moe(l, form) : seq_dense(l, [&](const StackGemmParams& g) { return normed(g, 1); }))
                     return -1;
                 leave(1);
             }
@@ -2180,10 +2239,26 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         if (r.enters_pass
             && launch_stack_pass_entry(s->x, r.pass > 0 ? s->x0 : nullptr, s->loop_step + (size_t) r.pass * Wd, T, Wd, stream))
             return -1;
-        if (launch_stack_group_rmsnorm(s->h1, l.ff > 0 ? s->h2 : nullptr, s->x, nullptr, l.norm1, l.norm2, s->dtype, T, Wd, s->groups, s->eps,
-                stream))
-            return -1;
-        if (run_mixer(l, r))
+        auto normed = [&](const StackGemmParams& g) -> int {
+            if (T == 1)
+            {
+                StackRowNorm n;
+                n.x = s->x;
+                n.w = l.norm1;
+                n.w2 = l.norm2;
+                n.h2 = l.ff > 0 ? s->h2 : nullptr;
+                n.eps = s->eps;
+                n.groups = s->groups;
+                const int rc = launch_stack_row_gemm(g, n, stream);
+                if (rc <= 0)
+                    return rc;
+            }
+            return launch_stack_group_rmsnorm(s->h1, l.ff > 0 ? s->h2 : nullptr, s->x, nullptr, l.norm1, l.norm2, s->dtype, T, Wd, s->groups, s->eps, stream)
+                    || launch_stack_gemm(g, stream)
+                ? -1
+                : 0;
+        };
+        if (run_mixer(l, r, normed))
             return -1;
         // x += sigmoid(P1[rg1] + b1) * (ctx Wo^T)
         StackGemmParams o;
@@ -2259,7 +2334,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             hp.tokens = NW;
             hp.width = Wd;
             hp.streams = s->streams;
-            hp.x = s->x;
+            hp.x = xs;
             hp.stream_stride = stream_stride;
             if (pending)
             {
