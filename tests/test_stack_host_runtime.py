@@ -243,6 +243,40 @@ def wide_tiles(stub):
     assert (resid, 0) in next(outs(G.residual_config(S), S, (G.RESIDUAL[0], 1)))
 
 
+def row_tiles(stub):
+    """The sizes of test_gpu_row_tiles.py take the tiles of gemm_wide_impl.h that they are listed under."""
+    import ruzinex_cases as Z
+    import sodudra_cases as S
+    import test_gpu_product_tiles as P
+    import test_gpu_row_tiles as G
+    import tolenex_cases as T
+
+    class Zeros:  # (nothing is computed)
+        standard_normal = uniform = staticmethod(lambda *a, size=None, **k: np.zeros(size if size is not None else a[-1], np.float32))
+    np.random.default_rng = lambda seed: Zeros
+    for cases in (S, T, Z):
+        cases.bf16_round = lambda x: x
+    store, gated, fp32, resid, resid_gate = range(5)
+
+    def tiles(cfg, cases, rows, want=1):
+        s = engine(cfg, cases, max_tokens=2048, max_sequences=1)
+        stub.forget()
+        step(s, 'a', rows, want)
+        found = [re.search(r'4wide\d+gemm_glds_kernelILi\d+ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi\d+ELi(\d+)', k) for k in stub.kernels()]
+        return [(32 * int(m[1]) * int(m[3]), 32 * int(m[2]) * int(m[4]), int(m[5])) for m in found if m]
+
+    for shape, columns in G.COLUMNS.items():
+        assert tiles(P.plain_config(columns, 64), Z, P.ROWS, P.ROWS)[-1] == (*shape, fp32)
+        assert (*shape, gated) in tiles(G.shared_config(G.SHARED[shape]), Z, P.ROWS), shape
+    s = engine(G.shared_config(*G.WIDE_SHARED), Z, max_tokens=2048, max_sequences=1)
+    stub.forget()
+    step(s, 'a', P.ROWS, 1)
+    assert any(f'wide_kernelILi4ELi{gated}ELb0' in k for k in stub.kernels())
+    for shape, (rows, width) in G.RESIDUAL.items():
+        assert (*shape, resid) in tiles(G.residual_config(width), S, rows), shape
+        assert (*shape, resid_gate) in tiles(P.residual_config(width), T, rows), shape
+
+
 def norms_without_a_sum(stub):
     """A norm of any number of streams carries the code of the experts' sum only where there is one to form."""
     import narurax_cases as N
@@ -408,6 +442,9 @@ else:
 
     def test_tiles_of_grouped_products(stub):
         run(stub, 'group_tiles')
+
+    def test_sizes_of_the_row_tile_tests(stub):
+        run(stub, 'row_tiles')
 
     def test_sizes_of_the_wide_tile_tests(stub):
         run(stub, 'wide_tiles')

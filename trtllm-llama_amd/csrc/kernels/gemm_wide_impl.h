@@ -1,4 +1,4 @@
-// Products of many rows on 256 x 256 tiles:  C[m,n] = epi( sum_k A[m,k] * W[n,k] ), both operands with K contiguous; bfloat16, fp16 or int8 (the three
+// Products of many rows on 256 x 256 tiles (those of 128 rows behind them):  C[m,n] = epi( sum_k A[m,k] * W[n,k] ), both operands with K contiguous; bfloat16, fp16 or int8 (the three
 // share one geometry: a K-tile is 128 BYTES of every row, a k-step 64 of them, and v_mfma_*_16x16x{32,32,64} takes 16 bytes a lane).  A header, so that
 // the translation units that instantiate it for their operand types share one source.  Everything has internal linkage.
 //
@@ -18,6 +18,7 @@
 // Tried and slower: the DMA two at a time (+8 %), W's ahead of A's or in turn with them (+10 %), a fifth 64-byte stage, setprio by wave half.
 #pragma once
 #include "dev_utils.h"
+#include "gemm_glds_impl.h"
 #include "gemm_seam.h"
 #include "kernels.h"
 #include "launch_util.h"
@@ -391,14 +392,14 @@ __device__ __forceinline__ void store8(uint16_t* p, const float (&v)[8])
     *reinterpret_cast<uint4*>(p) = make_uint4(bf_pair(v[0], v[1]), bf_pair(v[2], v[3]), bf_pair(v[4], v[5]), bf_pair(v[6], v[7]));
 }
 
-// bfloat16 products: the stack engine's layer seam.  p.N, offsets and addresses are whole 16-byte pieces (serves()); c: of this product
-template <int OUT>
-__device__ __forceinline__ void leave_pairs(const GemmParams& p, const Tile<W_BF16, true>& t, void* c, int row0, int col0, int rows)
+// bfloat16 products: the stack engine's layer seam.  Offsets and addresses are whole 16-byte pieces, fp32 sections without an activation apart (serves()); c: of this product
+template <int OUT, int NA, int NB>
+__device__ __forceinline__ void leave_pairs(const GemmParams& p, const f32x4 (&acc)[NA][NB], int lane, void* c, int row0, int col0, int rows)
 {
 #pragma unroll
     for (int jp = 0; jp < NB / 2; ++jp)
     {
-        const int col = col0 + 32 * jp + 8 * (t.lane >> 4);
+        const int col = col0 + 32 * jp + 8 * (lane >> 4);
         if (col >= p.N)
             continue;
         float b[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -411,7 +412,7 @@ __device__ __forceinline__ void leave_pairs(const GemmParams& p, const Tile<W_BF
         auto value = [&](float (&v)[8], int i) {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                v[e] = t.acc[i][2 * jp + (e >> 2)][e & 3] + b[e];
+                v[e] = acc[i][2 * jp + (e >> 2)][e & 3] + b[e];
         };
         auto rows_out = [&](auto* to) {
 #pragma unroll
@@ -442,20 +443,31 @@ __device__ __forceinline__ void leave_pairs(const GemmParams& p, const Tile<W_BF
             }
         }
         else if (so.f32)
-            rows_out(reinterpret_cast<float*>(so.c));
+        {
+            float* to = reinterpret_cast<float*>(so.c);
+            if (col + 8 <= p.N && !((reinterpret_cast<uintptr_t>(to + col) | (so.ldc << 2)) & 15))
+                rows_out(to);
+            else // a section of a few columns
+#pragma unroll
+                for (int i = 0; i < NA; ++i)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (col + e < p.N && row0 + i * 16 < rows)
+                            to[(int64_t) (row0 + i * 16) * so.ldc + col + e] = acc[i][2 * jp + (e >> 2)][e & 3] + b[e];
+        }
         else
             rows_out(reinterpret_cast<uint16_t*>(so.c));
     }
 }
-template <int OUT>
-__device__ __forceinline__ void leave_fp32(const GemmParams& p, const Tile<W_BF16, false>& t, void* c, int row0, int col0, int rows)
+template <int OUT, int NA, int NB>
+__device__ __forceinline__ void leave_fp32(const GemmParams& p, const f32x4 (&acc)[NA][NB], int lane, void* c, int row0, int col0, int rows)
 {
     float* out = OUT == OUT_FP32 ? reinterpret_cast<float*>(c) : p.resid;
     const int64_t ld = OUT == OUT_FP32 ? p.ldc : p.ldr;
 #pragma unroll
     for (int j = 0; j < NB; ++j)
     {
-        const int col = col0 + 16 * j + 4 * (t.lane >> 4);
+        const int col = col0 + 16 * j + 4 * (lane >> 4);
         if (col >= p.N)
             continue;
         const float* bias = OUT == OUT_RESID_GATE ? p.gate_bias : p.bias;
@@ -469,7 +481,7 @@ __device__ __forceinline__ void leave_fp32(const GemmParams& p, const Tile<W_BF1
             if (row >= rows)
                 continue;
             float* at = out + row * ld + col;
-            float v[4] = {t.acc[i][j][0], t.acc[i][j][1], t.acc[i][j][2], t.acc[i][j][3]};
+            float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
             if constexpr (OUT == OUT_FP32)
                 *reinterpret_cast<float4*>(at) = make_float4(v[0] + b.x, v[1] + b.y, v[2] + b.z, v[3] + b.w);
             else
@@ -665,9 +677,9 @@ __global__ __launch_bounds__(64 * WAVES) void wide_kernel(const GemmParams p)
                 char* c = reinterpret_cast<char*>(p.c);
                 c += GROUPED ? now.first * p.ldc * (p.out_dtype == DT_FLOAT ? 4 : 2) : now.product * p.batch_c;
                 if constexpr (PAIRS)
-                    leave_pairs<OUT>(p, t, c, row0, col0, now.rows);
+                    leave_pairs<OUT>(p, t.acc, t.lane, c, row0, col0, now.rows);
                 else
-                    leave_fp32<OUT>(p, t, c, row0, col0, now.rows);
+                    leave_fp32<OUT>(p, t.acc, t.lane, c, row0, col0, now.rows);
             }
             else if constexpr (DUAL)
                 leave_dual(p, t, scales, row0, col0, now.rows);
@@ -700,6 +712,204 @@ __global__ __launch_bounds__(64 * WAVES) void wide_kernel(const GemmParams p)
     }
 }
 
+// Tiles of 128 rows, for products of few tiles and groups of few rows: bfloat16, a tile a workgroup of 8 waves, S whole stages of 128-byte rows, results straight from the
+// accumulators as above.  PINNED: reads between the MFMAs, one barrier a K-tile (128 x 256 and 128 x 192); otherwise a k-step's reads in front of its MFMAs, which
+// the SIMD's other wave covers (128 x 128 and 128 x 64: pinned reads gave them nothing).  Bound by the operands' way from L2 and, once a wave's MFMAs are queued, by
+// them: 128 x 256 1600 - 1800 clocks a K-tile, 1024 of them MFMAs.  us in a step, in brackets the lock-step tiles of 32 x 32 MFMAs whose results went through LDS:
+//   128 x 256  2048 x 4096 x 4096 65 (70), x 11008 168 (180), 1672 x 4096 x 2048 35 (41), 32 groups of 8192 rows, 5504, 4096 493 (514), of 6688 rows, 2816, 2048 127 (126)
+//   128 x 192  1024 x 6912 x 2048 29.5 (31.9), 2048 x 8832 x 4096 161 (165)      128 x 128  1672 x 2048 x 2048 14.5 (17.8)
+//   128 x 64   1024 x 2048 x 4096 and x 6528, behind a gate into the residual 29.8 (31.7)
+template <int WT, int WM, int WN, int MT, int NT, int S, int OUT, bool GROUPED, bool PINNED>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParams p_in)
+{
+    constexpr bool PAIRS = out_pairs(OUT);
+    constexpr int NA = 2 * MT, NB = 2 * NT;
+    constexpr int NW = WM * WN, BM = WM * NA * 16, BN = WN * NB * 16, STAGE = (BM + BN) * 128, DMAS = (BM + BN) / 8 / NW, DMA_A = BM / 8 / NW;
+    static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole instructions");
+    extern __shared__ __attribute__((aligned(16))) char wide_lds[];
+    GemmParams p = p_in;
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wid / WN, wn = wid % WN;
+    int64_t product = blockIdx.y;
+    int id = blockIdx.x;
+    if constexpr (GROUPED)
+    {
+        const GroupTile gt = group_tile<BM>(p, (p.N + BN - 1) / BN, id);
+        if (gt.group < 0)
+            return; // behind the last tile
+        product = gt.group;
+        id = gt.tile;
+        const int64_t o = p.group_off[product];
+        p.M = p.group_off[product + 1] - (int) o;
+        if (p.a_rows)
+            p.a_rows += o;
+        else
+            p.a = reinterpret_cast<const char*>(p.a) + o * p.lda * 2;
+        p.c = reinterpret_cast<char*>(p.c) + o * p.ldc * (p.out_dtype == DT_FLOAT ? 4 : 2);
+    }
+    else
+    {
+        // each XCD a contiguous range of the tiles, row tiles fastest: those that share a panel of W run side by side on one L2
+        const int q = gridDim.x >> 3, r = gridDim.x & 7, xcd = id & 7;
+        id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (id >> 3);
+        p.a = reinterpret_cast<const char*>(p.a) + product * p.batch_a;
+        p.c = reinterpret_cast<char*>(p.c) + product * p.batch_c;
+    }
+    const char* w = reinterpret_cast<const char*>(p.w) + product * p.batch_w;
+    const int tiles_m = (p.M + BM - 1) / BM, tn = id / tiles_m, m0 = (id - tn * tiles_m) * BM, n0 = tn * BN, nt = p.K / 64;
+    const uint32_t lds = (uint32_t) (uintptr_t) (lds_ptr*) wide_lds;
+    uint32_t from[DMAS];
+#pragma unroll
+    for (int i = 0; i < DMAS; ++i)
+    {
+        const int row = ((i < DMA_A ? i : i - DMA_A) * NW + wid) * 8 + (lane >> 3);
+        if (i < DMA_A)
+        {
+            int r = m0 + row < p.M ? m0 + row : p.M - 1;
+            if (GROUPED && p.a_rows)
+                r = p.a_rows[r];
+            from[i] = (uint32_t) r * (uint32_t) (p.lda * 2) + (((lane & 7) ^ a_swz(row)) << 4);
+        }
+        else
+            from[i] = (uint32_t) (n0 + row < p.N ? n0 + row : p.N - 1) * (uint32_t) p.ldw + (((lane & 7) ^ w_swz<PAIRS>(row)) << 4);
+    }
+    auto dma = [&](int i, int t, uint32_t stage) {
+        load16((i < DMA_A ? reinterpret_cast<const char*>(p.a) : w) + (int64_t) t * 128, from[i], stage + (uint32_t) (i * NW + wid) * 1024);
+    };
+    f32x4 acc[NA][NB];
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int i16 = lane & 15, k4 = lane >> 4;
+    const uint32_t al = (uint32_t) ((wm * NA * 16 + i16) * 128), wl = (uint32_t) (BM * 128 + (wn * NB * 16 + w_row<PAIRS>(0, i16)) * 128);
+    const uint32_t as = a_swz(i16), ws = w_swz<PAIRS>(w_row<PAIRS>(0, i16));
+    const uint32_t a_k[2] = {al + ((k4 ^ as) << 4), al + (((4 + k4) ^ as) << 4)}, w_k[2] = {wl + ((k4 ^ ws) << 4), wl + (((4 + k4) ^ ws) << 4)};
+    auto a_at = [](uint32_t base, int block) { return *(lds_frag) (uintptr_t) (base + block * 2048); };
+    auto w_at = [](uint32_t base, int j) { return *(lds_frag) (uintptr_t) (base + w_row<PAIRS>(j, 0) * 128); };
+    const uint32_t end = lds + S * STAGE;
+    if constexpr (PINNED)
+    {
+        constexpr int BLOCKS = 2 * NA, L = BLOCKS >= 8 ? 3 : 2, HAND_OVER = BLOCKS - L;
+#pragma unroll
+        for (int t = 0; t < S; ++t)
+            if (t < nt)
+#pragma unroll
+                for (int i = 0; i < DMAS; ++i)
+                    dma(i, t, lds + t * STAGE);
+        if (nt >= S)
+            wait_vm_and_meet<(S - 1) * DMAS>();
+        else
+            wait_vm_and_meet<0>();
+        u32x4 fa[BLOCKS + L], fw[2][NB]; // fa: by block, those of the next stage behind; renamed, not kept
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            fw[0][j] = w_at(lds + w_k[0], j);
+#pragma unroll
+        for (int i = 0; i < L; ++i)
+            fa[i] = a_at(lds + a_k[0], i);
+        uint32_t cur = lds, before = lds;
+        for (int t = 0; t < nt; ++t)
+        {
+            const uint32_t next = cur + STAGE == end ? lds : cur + STAGE;
+            const uint32_t ra[3] = {cur + a_k[0], cur + a_k[1], next + a_k[0]}, rw1 = cur + w_k[1], rwn = next + w_k[0];
+#pragma unroll
+            for (int g = 0; g < BLOCKS; ++g)
+            {
+                if (g == HAND_OVER)
+                {
+                    // stage t + 1 has landed, nobody reads stage t any more: its room is for stage t + S
+                    if (t + S - 1 < nt)
+                        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * DMAS) : "memory");
+                    else
+                        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                {
+                    acc[g % NA][j] = mfma<WT>(fw[g / NA][j], fa[g], acc[g % NA][j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (j == 0)
+                        fa[g + L] = a_at(ra[(g + L) / NA], (g + L) % NA);
+                    else
+                    {
+                        const int q = g * (NB - 1) + j - 1, qn = q - HAND_OVER * (NB - 1);
+                        if (q < NB)
+                            fw[1][q] = w_at(rw1, q);
+                        if (qn >= 0 && qn < NB) // (behind the last stage: old data, not used)
+                            fw[0][qn] = w_at(rwn, qn);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // stage t - 1 + S, into the room that the hand-over from t - 1 to t released
+#pragma unroll
+                for (int i = 0; i < DMAS; ++i)
+                    if (g < HAND_OVER && i * HAND_OVER / DMAS == g)
+                    {
+                        if (t >= 1 && t - 1 + S < nt)
+                            dma(i, t - 1 + S, before);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
+#pragma unroll
+            for (int i = 0; i < L; ++i)
+                fa[i] = fa[BLOCKS + i];
+            before = cur;
+            cur = next;
+        }
+    }
+    else
+    {
+        constexpr int AHEAD_STAGES = S - 1, PARTS = 2;
+#pragma unroll
+        for (int t = 0; t < AHEAD_STAGES; ++t)
+            if (t < nt)
+#pragma unroll
+                for (int i = 0; i < DMAS; ++i)
+                    dma(i, t, lds + t * STAGE);
+        uint32_t cur = lds, into = lds + AHEAD_STAGES * STAGE;
+        for (int t = 0; t < nt; ++t)
+        {
+            // stage t has landed (the younger ones stay under way), and nobody reads stage t - 1 any more, whose room the next requests take
+            if (t + AHEAD_STAGES - 1 < nt)
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((AHEAD_STAGES - 1) * DMAS) : "memory");
+            else
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+            {
+                u32x4 fa[NA], fw[NB];
+#pragma unroll
+                for (int i = 0; i < NA; ++i)
+                    fa[i] = a_at(cur + a_k[k], i);
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    fw[j] = w_at(cur + w_k[k], j);
+                __builtin_amdgcn_sched_barrier(0);
+                if (t + AHEAD_STAGES < nt)
+#pragma unroll
+                    for (int i = 0; i < DMAS; ++i)
+                        if (i % PARTS == k)
+                            dma(i, t + AHEAD_STAGES, into);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < NA; ++i)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j)
+                        acc[i][j] = mfma<WT>(fw[j], fa[i], acc[i][j]);
+            }
+            cur = cur + STAGE == end ? lds : cur + STAGE;
+            into = into + STAGE == end ? lds : into + STAGE;
+        }
+    }
+    const int row0 = m0 + wm * (NA * 16) + i16, col0 = n0 + wn * (NB * 16);
+    if constexpr (PAIRS)
+        leave_pairs<OUT>(p, acc, lane, p.c, row0, col0, p.M);
+    else
+        leave_fp32<OUT>(p, acc, lane, p.c, row0, col0, p.M);
+}
+
 inline bool aligned16(const void* p)
 {
     return !(reinterpret_cast<uintptr_t>(p) & 15);
@@ -710,7 +920,10 @@ template <int WT>
 bool serves(const GemmParams& p)
 {
     constexpr int ES = WT == W_INT8_SQ ? 1 : 2;
-    if (p.wtype != WT || p.K <= 0 || (p.K * ES) % 128 || !aligned16(p.a) || !aligned16(p.w) || (p.lda * ES) % 16 || p.ldw % 16 || p.N % 8)
+    if (p.wtype != WT || p.K <= 0 || (p.K * ES) % 128 || !aligned16(p.a) || !aligned16(p.w) || (p.lda * ES) % 16 || p.ldw % 16)
+        return false;
+    const GemmSection* last = WT == W_BF16 && p.seam.n_sec > 0 ? &p.seam.sec[p.seam.n_sec - 1] : nullptr;
+    if (p.N % 8 && (!last || last->col0 > p.N - p.N % 8 || !last->f32 || p.bias)) // (columns that are no whole piece: one by one, in the last section)
         return false;
     // 32-bit offsets of the operands' rows (gathered rows: any of the a that the caller has; its extent is not known here)
     const int64_t rows = p.group_off ? p.group_total : p.M;
@@ -732,7 +945,9 @@ bool serves(const GemmParams& p)
         for (int s = 0; s < p.seam.n_sec; ++s)
         {
             const GemmSection& k = p.seam.sec[s];
-            if (k.col0 % 8 || !aligned16(k.c) || k.ldc % (k.f32 ? 4 : 8) || (k.act != GEMM_ACT_NONE && k.act != GEMM_ACT_RELU2))
+            if (k.col0 % 8 || (k.act != GEMM_ACT_NONE && k.act != GEMM_ACT_RELU2))
+                return false;
+            if ((!k.f32 || k.act != GEMM_ACT_NONE) && (p.N % 8 || !aligned16(k.c) || k.ldc % (k.f32 ? 4 : 8)))
                 return false;
         }
         return true;
@@ -806,6 +1021,42 @@ int launch(const GemmParams& p, hipStream_t stream)
         return p.w2 ? launch_out<WT, OUT_DUAL>(p, stream) : launch_out<WT, OUT_HALF>(p, stream);
     else
         return launch_out<WT, OUT_HALF>(p, stream);
+}
+
+template <int OUT, bool GROUPED, int WM, int WN, int MT, int NT, int S, bool PINNED>
+int launch_row128_out(const GemmParams& p, hipStream_t stream)
+{
+    constexpr int BM = WM * MT * 32, BN = WN * NT * 32;
+    constexpr size_t lds = (size_t) S * (BM + BN) * 128;
+    static_assert(BM == 128 && lds <= LDS_BYTES, "LDS");
+    const auto kernel = gemm_glds_kernel<W_BF16, WM, WN, MT, NT, S, OUT, GROUPED, PINNED>;
+    launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
+    const int64_t cols = (p.N + BN - 1) / BN;
+    // grouped: at most this many row tiles, full ones, and one begun in every group that has rows
+    const int64_t tiles = GROUPED ? (p.group_total / BM + std::min<int64_t>(p.batch, p.group_total)) * cols : (p.M + BM - 1) / BM * cols;
+    hipLaunchKernelGGL(kernel, dim3((unsigned) tiles, GROUPED ? 1 : p.batch), dim3(64 * WM * WN), lds, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+    {
+        set_error("gemm tiles of 128 rows: launch failed: %s", hipGetErrorString(e));
+        return -1;
+    }
+    return 0;
+}
+// p: serves<W_BF16>(p)
+template <int WM, int WN, int MT, int NT, int S, bool PINNED>
+int launch_row128(const GemmParams& p, hipStream_t stream)
+{
+    const bool gated = p.act >= GEMM_ACT_GATE_SILU, fp32 = p.out_dtype == DT_FLOAT && p.seam.n_sec == 0 && p.act == GEMM_ACT_NONE;
+    if (p.group_off)
+        return gated ? launch_row128_out<OUT_GATED, true, WM, WN, MT, NT, S, PINNED>(p, stream)
+            : fp32   ? launch_row128_out<OUT_FP32, true, WM, WN, MT, NT, S, PINNED>(p, stream)
+                     : launch_row128_out<OUT_STORE, true, WM, WN, MT, NT, S, PINNED>(p, stream);
+    if (p.resid)
+        return p.gate ? launch_row128_out<OUT_RESID_GATE, false, WM, WN, MT, NT, S, PINNED>(p, stream) : launch_row128_out<OUT_RESID, false, WM, WN, MT, NT, S, PINNED>(p, stream);
+    return gated ? launch_row128_out<OUT_GATED, false, WM, WN, MT, NT, S, PINNED>(p, stream)
+        : fp32   ? launch_row128_out<OUT_FP32, false, WM, WN, MT, NT, S, PINNED>(p, stream)
+                 : launch_row128_out<OUT_STORE, false, WM, WN, MT, NT, S, PINNED>(p, stream);
 }
 
 } // namespace wide

@@ -1,13 +1,13 @@
 // Products of the stack engine (stack_kernels.h): C[m,n] = sum_k A[m,k] * W[n,k] with the layer seam in the epilogue.
 //
-//   bfloat16, M >= 32, K % 64 == 0: the LDS-DMA staged MFMA tiles of gemm_glds_impl.h instantiated for bfloat16 operands
-//                     (v_mfma_f32_32x32x16_bf16), tile shape by the same rounds x area rule as the fp16 form;
+//   bfloat16, M >= 32, K % 64 == 0: LDS-DMA staged MFMA tiles, shape by rounds x area: gemm_wide_impl.h where results leave in 16-byte pieces, otherwise
+//                     gemm_glds_impl.h (v_mfma_f32_32x32x16_bf16);
 //   bfloat16, other M >= 32: fp32 results as far as whole stages go by the same tiles, the rest of K by fma_tile_kernel; 16-bit results by the
 //                     register-staged MFMA tiles of gemm_mfma.hip;
 //   bfloat16, M <= 31: slim_kernel below - HBM-bound, the weight-streaming MFMA main loop of gemm_slim_impl.h; grouped products of many workgroups
 //                     slim_group_kernel, the same with its block in registers;
 //   bfloat16, M = 1:  row_kernel - dot products on the vector pipe, K split over a workgroup's waves; fp32 accumulation, DPP reduction; very many rows of
-//                     one chunk: row_short_kernel (a lone token's experts: lone_up_kernel, lone_down_kernel);
+//                     one chunk: row_short_kernel (a lone token's experts: lone_up_kernel, lone_down_kernel; behind its norm: row_norm_kernel);
 //   bfloat16, 2 <= M <= 8, few columns of long rows: skinny_ksplit_kernel, the same for several rows;
 //   float32         : fma_tile_kernel - 64 x 64 tiles of plain fp32 FMAs through LDS (no reduced-precision matrix mode), any shape;
 //                     also the fallback for bfloat16 operands whose rows are not 16-byte aligned.
@@ -706,11 +706,10 @@ inline int launched(const char* what)
     return 0;
 }
 
-// The tile shapes of the LDS-DMA kernel, all with stages of whole 128-byte lines and 8 waves, and what a tile of each kind costs per area when
-// the chip is full of them (measured, relative to 256 x 256; M 2048 .. 512, N 2048 .. 22016, K 2048 .. 11008): fewest workgroup rounds x
-// area x cost.  us, M x N x K, in brackets the 64-byte stages and 4-wave tiles these replaced:
-//   1024 x 2048 x 5504   128 x 64  38 (49)      2048 x 4096 x 4096   128 x 256  62 (81)      2048 x 22016 x 4096   256 x 256  332 (380)
-//   1024 x 6144 x 2048   128 x 192 30 (43)      2048 x 6144 x 4096   256 x 192  94 (102)     1024 x 13056 x 2048   256 x 256   57 (61)
+// The tile shapes of the LDS-DMA kernels, all with stages of whole 128-byte lines and 8 waves, and what a tile of each kind costs per area when
+// the chip is full of them (measured, relative to lock-step 256 x 256; M 2048 .. 512, N 2048 .. 22016, K 2048 .. 11008): fewest workgroup rounds x
+// area x cost.  row_tiles: those of 128 rows by gemm_wide_impl.h, 4 - 18 % quicker than the lock-step ones of gemm_glds_impl.h (figures there), which stay for
+// what leaves in other pieces (columns that are no multiple of 8, rows off 16 bytes) and for 256 rows x 192, where the 16 x 16 form gained nothing.
 int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0)
 {
     struct Shape
@@ -718,7 +717,10 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
         int id, bm, bn;
         double f;
     };
-    static const Shape shapes[] = {{0, 128, 128, 1.49}, {1, 256, 192, 1.16}, {2, 256, 256, 1.0}, {3, 128, 256, 1.15}, {4, 128, 192, 1.28}, {5, 128, 64, 2.15}};
+    static const Shape lock_step[] = {{0, 128, 128, 1.49}, {1, 256, 192, 1.16}, {2, 256, 256, 1.0}, {3, 128, 256, 1.15}, {4, 128, 192, 1.28}, {5, 128, 64, 2.15}};
+    static const Shape row_tiles[] = {{0, 128, 128, 1.37}, {1, 256, 192, 1.16}, {2, 256, 256, 1.0}, {3, 128, 256, 1.07}, {4, 128, 192, 1.22}, {5, 128, 64, 2.05}};
+    const bool served = wide::serves<W_BF16>(g);
+    const Shape (&shapes)[6] = served ? row_tiles : lock_step;
     const int cus = launch_util::device_cus();
     double best = 1e30;
     int pick = 0;
@@ -752,7 +754,7 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
     // 256 x 256 tiles of gemm_wide_impl.h.  Grouped: where groups have two of them (32 groups, us, in brackets the shapes above: 16384 rows, N 2816, K 2048 227 (282), 12000
     // 176 (202), 16384 rows, 704, 512 24 (34)).  Groups of one tile read their weights alone, from HBM, which a K-tile and a half ahead does not hide: 8192 rows,
     // 5504, 4096 took 542 (500) in a step, the same rows of fewer columns by themselves 133 (141) at 2816, 2048 and 126 (121) with 6700 rows.
-    if (wide::serves<W_BF16>(g))
+    if (served)
     {
         if (m_expected > 0)
         {
@@ -772,6 +774,14 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
                 return wide::launch<W_BF16>(g, stream);
         }
     }
+    if (served)
+        switch (pick)
+        {
+        case 0: return wide::launch_row128<2, 4, 2, 1, 4, false>(g, stream);
+        case 3: return wide::launch_row128<2, 4, 2, 2, 3, true>(g, stream);
+        case 4: return wide::launch_row128<4, 2, 1, 3, 4, true>(g, stream);
+        case 5: return wide::launch_row128<4, 2, 1, 1, 4, false>(g, stream);
+        }
     if (g.act == ACT_SCALE_CAP || g.act == ACT_GELU_MUL)
         pick = 0; // the shape whose epilogue has them
     const int gated = g.act >= ACT_GATE_SILU ? (g.seam.n_sec > 0 ? g.seam.sec[0].col0 : g.N) : 0;
