@@ -277,6 +277,24 @@ def row_tiles(stub):
         assert (*shape, resid_gate) in tiles(P.residual_config(width), T, rows), shape
 
 
+def convolution_of_single_rows(stub):
+    """A step of one row per entry has no launch for a convolution of 4 taps, whatever the layers of test_gpu_conv_step.py; other steps and other taps do."""
+    import test_gpu_conv_step as G
+    import narurax_cases as N
+    import rofozen_cases as M
+    for name, layer in G.LAYERS.items():
+        cases = N if name.startswith('delta') else M
+        for taps in (4, 3):
+            layer['mixer']['conv'] = taps
+            s = engine(cases.make_config([layer]), cases, max_tokens=64, max_sequences=2)
+            for rows in (5, 1, 1, 2):
+                stub.forget()
+                step(s, 'a', rows)
+                kernels = stub.kernels()
+                assert any('ssm_conv' in k for k in kernels) == (rows > 1 or taps != 4), (name, taps, rows)
+                assert any(re.search(r'(ssm|delta)_step_kernelILi7ELb1', k) for k in kernels) == (rows == 1 and taps == 4), (name, taps, rows)
+
+
 def norms_without_a_sum(stub):
     """A norm of any number of streams carries the code of the experts' sum only where there is one to form."""
     import narurax_cases as N
@@ -442,6 +460,9 @@ else:
 
     def test_tiles_of_grouped_products(stub):
         run(stub, 'group_tiles')
+
+    def test_convolution_of_single_rows(stub):
+        run(stub, 'convolution_of_single_rows')
 
     def test_sizes_of_the_row_tile_tests(stub):
         run(stub, 'row_tiles')

@@ -4,6 +4,7 @@
 #include "dev_utils.h"
 #include "launch_util.h"
 #include "stack_chunk.h"
+#include "stack_conv_impl.h"
 #include "stack_kernels.h"
 #include <algorithm>
 #include <cstdlib>
@@ -294,7 +295,8 @@ __global__ __launch_bounds__(256) void delta_out_kernel(const StackDeltaParams p
 // reads.  Thread (r, c) keeps rows 8 r .. 8 r + 7 of columns 4 c .. 4 c + 3; the state comes in 16-byte pieces that are requested ahead of
 // the unit norms and decays, and the two sums over rows meet in LDS.  8 heads of 128 x 128, one entry: 6.1 us, as a walk of one row
 // and a norm 9.1 + 2.9 us.
-template <int DT>
+// CONV: the row's convolution, too (stack_conv_impl.h); the first head of those that share q and k writes their raw inputs.
+template <int DT, bool CONV>
 __global__ __launch_bounds__(1024) void delta_step_kernel(const StackDeltaParams p)
 {
     extern __shared__ float sm[];
@@ -302,7 +304,8 @@ __global__ __launch_bounds__(1024) void delta_step_kernel(const StackDeltaParams
     const int D = p.dim, V = p.vdim, R = D >> 3, CT = V >> 2, NT = blockDim.x;
     float* qs = sm;              // [D]
     float* ks = qs + D;          // [D]
-    float* gs = ks + D;          // [D]
+    float* vs = ks + D;          // CONV: [V]
+    float* gs = CONV ? vs + V : vs; // [D]
     float* part = gs + D;        // [R][V] of S^T k
     float* opart = part + R * V; // [R][V] of S^T q
     const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
@@ -326,17 +329,33 @@ __global__ __launch_bounds__(1024) void delta_step_kernel(const StackDeltaParams
             S[j] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
     float v[4];
+    if constexpr (!CONV)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        v[i] = ld_el<DT>(p.x, row * CH + 2 * QK + h * V + 4 * c + i);
+        for (int i = 0; i < 4; ++i)
+            v[i] = ld_el<DT>(p.x, row * CH + 2 * QK + h * V + 4 * c + i);
     const float beta = 1.f / (1.f + expf(-ld_el<DT>(p.beta_raw, row * p.ld_beta + h))), rate = expf(p.a_log[h]);
+    if constexpr (CONV)
+    {
+        // q, k and v lie one behind the other
+        constexpr int ES = DT == DT_BF16 ? 2 : 4;
+        conv_step<DT>(reinterpret_cast<const char*>(p.x_raw) + row * p.ld_raw * ES, p.conv_state + (int64_t) p.ent_slot[e] * p.taps * CH, p.conv_w, nullptr, CH, p.ent_pos0[e],
+            2 * D + V, qs, [&](int i) { return i < D ? hk * D + i : i < 2 * D ? QK + hk * D + i - D : 2 * QK + h * V + i - 2 * D; },
+            [&](int i) { return i >= 2 * D || h % (p.heads / p.qk_heads) == 0; });
+    }
     for (int d = tid; d < D; d += NT)
     {
-        qs[d] = ld_el<DT>(p.x, row * CH + hk * D + d);
-        ks[d] = ld_el<DT>(p.x, row * CH + QK + hk * D + d);
+        if constexpr (!CONV)
+        {
+            qs[d] = ld_el<DT>(p.x, row * CH + hk * D + d);
+            ks[d] = ld_el<DT>(p.x, row * CH + QK + hk * D + d);
+        }
         gs[d] = decay_of<DT>(rate, p.decay_raw[(row * p.heads + h) * D + d] + p.dt_bias[h * D + d]);
     }
     __syncthreads();
+    if constexpr (CONV)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            v[i] = vs[4 * c + i];
     float sq = 0.f, sk = 0.f; // (every wave for itself)
     for (int d = lane; d < D; d += 64)
     {
@@ -487,26 +506,49 @@ bool stack_delta_serves(int32_t dim, int32_t vdim)
     return dim >= 1 && vdim >= 1 && dim <= 512 && delta_shape(dim, vdim).nsz > 0; // 16 staged rows of q, k and the decay within 128 KiB of LDS
 }
 
+static int one_row_threads(const StackDeltaParams& p)
+{
+    return (p.vdim / 4 * (p.dim / 8) + 63) / 64 * 64;
+}
+static size_t one_row_lds(const StackDeltaParams& p, bool convolve)
+{
+    return sizeof(float) * (3 * (size_t) p.dim + 2 * (size_t) (p.dim / 8) * p.vdim + (convolve ? p.vdim : 0));
+}
+static bool one_row(const StackDeltaParams& p, bool convolve)
+{
+    return p.max_count == 1 && p.dim % 8 == 0 && p.vdim % 4 == 0 && one_row_threads(p) <= 1024 && one_row_lds(p, convolve) <= 64 * 1024;
+}
+
+bool stack_delta_convolves(const StackDeltaParams& p)
+{
+    return one_row(p, true) && p.taps == 4 && !(reinterpret_cast<uintptr_t>(p.conv_w) & 15);
+}
+
 int launch_stack_delta(const StackDeltaParams& p, hipStream_t stream)
 {
-    const int threads = (p.vdim / 4 * (p.dim / 8) + 63) / 64 * 64;
-    const size_t lds = sizeof(float) * (3 * (size_t) p.dim + 2 * (size_t) (p.dim / 8) * p.vdim);
-    if (p.max_count != 1 || p.dim % 8 || p.vdim % 4 || threads > 1024 || lds > 64 * 1024)
+    const bool convolve = p.x_raw != nullptr;
+    if (convolve && (!stack_delta_convolves(p) || !p.conv_w || !p.conv_state))
+    {
+        set_error("stack_delta: the convolution of %d taps goes with steps of one row of 4, its weights and its state", p.taps);
+        return -1;
+    }
+    if (!one_row(p, convolve))
         return (launch_stack_delta_scan(p, stream) || launch_stack_delta_out(p, stream)) ? -1 : 0;
     if (p.tokens <= 0 || p.entries <= 0)
         return 0;
     if (!delta_ok(p, "stack_delta"))
         return -1;
-    if (!p.x || !p.beta_raw || !p.decay_raw || !p.dt_bias || !p.a_log || !p.state || !p.ent_slot || !p.ent_first || !p.ent_pos0 || !p.gate_raw
+    if ((!p.x && !convolve) || !p.beta_raw || !p.decay_raw || !p.dt_bias || !p.a_log || !p.state || !p.ent_slot || !p.ent_first || !p.ent_pos0 || !p.gate_raw
         || !p.norm_w || !p.out)
     {
         set_error("stack_delta: a missing operand");
         return -1;
     }
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.entries, p.heads), dim3(one_row_threads(p)), one_row_lds(p, convolve), stream, p); };
     if (p.dtype == DT_BF16)
-        hipLaunchKernelGGL((delta_step_kernel<DT_BF16>), dim3(p.entries, p.heads), dim3(threads), lds, stream, p);
+        convolve ? go(delta_step_kernel<DT_BF16, true>) : go(delta_step_kernel<DT_BF16, false>);
     else
-        hipLaunchKernelGGL((delta_step_kernel<DT_FLOAT>), dim3(p.entries, p.heads), dim3(threads), lds, stream, p);
+        convolve ? go(delta_step_kernel<DT_FLOAT, true>) : go(delta_step_kernel<DT_FLOAT, false>);
     return launched("stack_delta (one row)");
 }
 

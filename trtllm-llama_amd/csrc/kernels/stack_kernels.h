@@ -370,8 +370,9 @@ bool stack_hgrn2_serves(int32_t dim, int32_t vdim); // shapes one of its two for
 // ---------------------------------------------------------------------------------------------
 // Selective state-space layer (Mamba-2): proj [tokens, ldp] = [z: inner | x: inner | B: groups * state | C: groups * state |
 // dt: heads], inner = heads * vdim.  x, B, C pass a causal convolution over `taps` tokens per channel (conv_w [channels, taps], the
-// last column meets the current token; bias) and silu: launch_stack_ssm_conv writes them to xbc [tokens, channels] and moves the
-// sequence's last taps - 1 raw inputs into conv_state [slots, taps - 1, channels].  launch_stack_ssm_scan: per head h (reading group
+// last column meets the current token; bias) and silu: launch_stack_ssm_conv writes them to xbc [tokens, channels] and the
+// sequence's last taps - 1 raw inputs into conv_state [slots, taps, channels], position q's in row q mod taps; where stack_ssm_convolves, the scan does
+// both itself (convolve) and xbc stays as it is.  launch_stack_ssm_scan: per head h (reading group
 // h / (heads / groups)), with dt = softplus(dt + dt_bias[h]):
 //   S <- exp(-exp(a_log[h]) dt) S + dt B x^T   (S [state, vdim], fp32, one per slot),   y = S^T C + d_skip[h] x,
 // and y32 [tokens, inner] = y * silu(z) in fp32 (the grouped norm behind it is launch_stack_group_rmsnorm).  An entry whose pos0 is 0
@@ -389,7 +390,8 @@ struct StackSsmParams
     const float* dt_bias = nullptr; // [heads]
     const float* a_log = nullptr;   // [heads]
     const float* d_skip = nullptr;  // [heads]
-    float* conv_state = nullptr;    // [slots, taps - 1, channels]
+    float* conv_state = nullptr;    // [slots, taps, channels]
+    int32_t convolve = 0;           // scan: 1: of the raw columns of proj, whose convolution it forms (stack_ssm_convolves)
     float* ssm_state = nullptr;     // [slots, heads, state, vdim]
     void* xbc = nullptr;            // scratch [tokens, channels], element type
     float* y32 = nullptr;           // [tokens, inner]
@@ -409,6 +411,7 @@ struct StackSsmParams
 };
 int launch_stack_ssm_conv(const StackSsmParams& p, hipStream_t stream);
 int launch_stack_ssm_scan(const StackSsmParams& p, hipStream_t stream);
+bool stack_ssm_convolves(const StackSsmParams& p); // a step of one row per entry, 4 taps
 bool stack_ssm_serves(int32_t vdim, int32_t state, int32_t taps);
 
 // ---------------------------------------------------------------------------------------------
@@ -501,7 +504,14 @@ struct StackDeltaParams
     int32_t max_count = 0;            // host: the largest ent_count of the step
     float* chunk_ws = nullptr;        // optional scratch of the chunked form, as above
     size_t chunk_floats = 0;
+    // launch_stack_delta alone, of the raw columns: x comes from the convolution of x_raw (x_raw[t * ld_raw + channel]), as in StackSsmParams; null: from x
+    const void* x_raw = nullptr;
+    int64_t ld_raw = 0;
+    const float* conv_w = nullptr;
+    float* conv_state = nullptr;
+    int32_t taps = 0;
 };
+bool stack_delta_convolves(const StackDeltaParams& p); // a step of one row per entry, 4 taps
 // both, in one launch for a step of single rows
 int launch_stack_delta(const StackDeltaParams& p, hipStream_t stream);
 int launch_stack_delta_scan(const StackDeltaParams& p, hipStream_t stream);

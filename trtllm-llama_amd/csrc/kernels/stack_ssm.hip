@@ -4,6 +4,7 @@
 #include "dev_utils.h"
 #include "launch_util.h"
 #include "stack_chunk.h"
+#include "stack_conv_impl.h"
 #include "stack_kernels.h"
 #include <algorithm>
 #include <cstdlib>
@@ -53,18 +54,21 @@ inline int launched(const char* what)
 
 constexpr int MAX_TAPS = 16;
 
-// An entry's first taps - 1 rows of channel c, which reach into the sequence's tail of raw inputs, and the new tail: one thread per (entry,
-// channel) reads the old tail before it writes, so the launch has no ordering between workgroups to keep
+// An entry's first taps - 1 rows of channel c, which reach into the sequence's last raw inputs, and the new ones: one thread per (entry,
+// channel) reads the old ones before it writes, so the launch has no ordering between workgroups to keep
 template <int DT>
 __device__ __forceinline__ void conv_edges(const StackSsmParams& p, int e, int c, int CH, int64_t col, const float* w, float bias)
 {
     const int K = p.taps;
-    const int first = p.ent_first[e], count = p.ent_count[e];
-    float* tail = p.conv_state + (int64_t) p.ent_slot[e] * (K - 1) * CH + c;
+    const int first = p.ent_first[e], count = p.ent_count[e], pos0 = p.ent_pos0[e];
+    float* ring = p.conv_state + (int64_t) p.ent_slot[e] * K * CH + c; // position q's in row q mod K
     float old[MAX_TAPS - 1];
 #pragma unroll
     for (int j = 0; j < MAX_TAPS - 1; ++j)
-        old[j] = (j < K - 1 && p.ent_pos0[e] > 0) ? tail[(int64_t) j * CH] : 0.f;
+    {
+        const int q = pos0 - (K - 1) + j;
+        old[j] = (j < K - 1 && q >= 0) ? ring[(int64_t) (q % K) * CH] : 0.f;
+    }
     // input at index i of the entry (negative: the tail; old[K - 1 + i])
     auto input = [&](int i) -> float {
         if (i >= 0)
@@ -83,8 +87,8 @@ __device__ __forceinline__ void conv_edges(const StackSsmParams& p, int e, int c
             acc = fmaf(w[k], input(i - (K - 1) + k), acc);
         st_el<DT>(p.xbc, (int64_t) (first + i) * CH + c, silu_f(acc));
     }
-    for (int j = 0; j < K - 1; ++j)
-        tail[(int64_t) j * CH] = input(count - (K - 1) + j);
+    for (int i = count - head; i < count; ++i)
+        ring[(int64_t) ((pos0 + i) % K) * CH] = input(i);
 }
 
 // Workgroups [0, tokens): row t, 256 channels each (blockIdx.y): rows that lie at least taps - 1 tokens into their entry read
@@ -453,10 +457,11 @@ __global__ __launch_bounds__(1024) void ssm_scan_pipe_kernel(const StackSsmParam
 // (entry, head), thread (r, c) keeps rows 8 r .. 8 r + 7 of columns 4 c .. 4 c + 3: the state comes in 16-byte pieces, B and C as one
 // 8-value read each, all requested before the step size is known; one barrier for the sum over rows.  64 heads of 128 x 64, one
 // entry: 4.4 us, 7.9 us as a walk of one row.
-template <int DT>
+// CONV: the row's convolution, too (stack_conv_impl.h); the first head of a group writes B's and C's raw inputs.
+template <int DT, bool CONV>
 __global__ __launch_bounds__(1024) void ssm_step_kernel(const StackSsmParams p)
 {
-    extern __shared__ float part[]; // [N / 8][PH]
+    extern __shared__ float part[]; // [N / 8][PH]; CONV: the row's x [PH], B [N], C [N] behind it
     const int PH = p.vdim, N = p.state, H = p.heads, G = p.groups;
     const int inner = H * PH, GN = G * N, CH = inner + 2 * GN;
     const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, CT = PH >> 2;
@@ -476,16 +481,8 @@ __global__ __launch_bounds__(1024) void ssm_step_kernel(const StackSsmParams p)
             return v;
     };
     const Raw rdt = prj[2 * inner + 2 * GN + h];
-    Raw4 rb[2], rc[2];
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-    {
-        rb[k] = *reinterpret_cast<const Raw4*>(xbc + bcol + 4 * k);
-        rc[k] = *reinterpret_cast<const Raw4*>(xbc + bcol + GN + 4 * k);
-    }
-    const Raw4 rx = *reinterpret_cast<const Raw4*>(xbc + xcol + 4 * c);
     const int v = tid < PH ? tid : PH - 1; // the column this thread finishes
-    const Raw vx = xbc[xcol + v], vz = prj[h * PH + v];
+    const Raw vz = prj[h * PH + v];
     float4 S[8];
     if (p.ent_pos0[e] > 0)
     {
@@ -499,14 +496,60 @@ __global__ __launch_bounds__(1024) void ssm_step_kernel(const StackSsmParams p)
         for (int j = 0; j < 8; ++j)
             S[j] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
+    float* conv = part + (N >> 3) * PH;
+    Raw4 rb[2], rc[2], rx;
+    Raw vx;
+    if constexpr (CONV)
+    {
+        const int g = h / (H / G);
+        conv_step<DT>(prj + inner, p.conv_state + (int64_t) p.ent_slot[e] * p.taps * CH, p.conv_w, p.conv_b, CH, p.ent_pos0[e], PH + 2 * N, conv,
+            [&](int i) { return i < PH ? h * PH + i : inner + g * N + (i - PH < N ? i - PH : GN + i - PH - N); }, [&](int i) { return i < PH || h % (H / G) == 0; });
+    }
+    else
+    {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+        {
+            rb[k] = *reinterpret_cast<const Raw4*>(xbc + bcol + 4 * k);
+            rc[k] = *reinterpret_cast<const Raw4*>(xbc + bcol + GN + 4 * k);
+        }
+        rx = *reinterpret_cast<const Raw4*>(xbc + xcol + 4 * c);
+        vx = xbc[xcol + v];
+    }
     const float z = cvt(rdt) + p.dt_bias[h], dt = z > 20.f ? z : log1pf(expf(z));
     const float a = expf(-expf(p.a_log[h]) * dt);
-    const float x[4] = {cvt(rx[0]) * dt, cvt(rx[1]) * dt, cvt(rx[2]) * dt, cvt(rx[3]) * dt};
+    float x[4], b8[8], c8[8];
+    if constexpr (CONV)
+    {
+        __syncthreads();
+        const int r8 = 8 * (live ? r : 0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            x[j] = conv[4 * c + j] * dt;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+        {
+            b8[j] = conv[PH + r8 + j];
+            c8[j] = conv[PH + N + r8 + j];
+        }
+    }
+    else
+    {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            x[j] = cvt(rx[j]) * dt;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+        {
+            b8[j] = cvt(rb[j >> 2][j & 3]);
+            c8[j] = cvt(rc[j >> 2][j & 3]);
+        }
+    }
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
     {
-        const float b = cvt(rb[j >> 2][j & 3]), cc = cvt(rc[j >> 2][j & 3]);
+        const float b = b8[j], cc = c8[j];
         S[j].x = fmaf(a, S[j].x, b * x[0]);
         S[j].y = fmaf(a, S[j].y, b * x[1]);
         S[j].z = fmaf(a, S[j].z, b * x[2]);
@@ -529,7 +572,12 @@ __global__ __launch_bounds__(1024) void ssm_step_kernel(const StackSsmParams p)
         float y = 0.f;
         for (int k = 0; k < N >> 3; ++k)
             y += part[k * PH + i];
-        const float xi = i == tid ? cvt(vx) : cvt(xbc[xcol + i]), zi = i == tid ? cvt(vz) : cvt(prj[h * PH + i]);
+        float xi;
+        if constexpr (CONV)
+            xi = conv[i];
+        else
+            xi = i == tid ? cvt(vx) : cvt(xbc[xcol + i]);
+        const float zi = i == tid ? cvt(vz) : cvt(prj[h * PH + i]);
         p.y32[row * inner + h * PH + i] = fmaf(p.d_skip[h], xi, y) * silu_f(zi);
     }
 }
@@ -566,6 +614,16 @@ static bool ssm_ok(const StackSsmParams& p, const char* what)
         return false;
     }
     return true;
+}
+
+static bool one_row(const StackSsmParams& p)
+{
+    return p.max_count == 1 && p.state % 8 == 0 && p.vdim % 4 == 0 && (p.heads * p.vdim) % 8 == 0;
+}
+
+bool stack_ssm_convolves(const StackSsmParams& p)
+{
+    return one_row(p) && p.taps == 4 && !(reinterpret_cast<uintptr_t>(p.conv_w) & 15);
 }
 
 int launch_stack_ssm_conv(const StackSsmParams& p, hipStream_t stream)
@@ -616,20 +674,26 @@ int launch_stack_ssm_scan(const StackSsmParams& p, hipStream_t stream)
         return 0;
     if (!ssm_ok(p, "stack_ssm_scan"))
         return -1;
+    if (p.convolve && !stack_ssm_convolves(p))
+    {
+        set_error("stack_ssm_scan: the convolution of %d taps goes with steps of one row of 4", p.taps);
+        return -1;
+    }
     {
         const int rc = launch_stack_chunk_ssm(p, stream); // prompts: 16 rows at a time through matrix products
         if (rc <= 0)
             return rc;
     }
-    if (p.max_count == 1 && p.state % 8 == 0 && p.vdim % 4 == 0 && (p.heads * p.vdim) % 8 == 0)
+    if (one_row(p))
     {
         // (a thread per 8 x 4 values of state: at most 1024, the shapes that are served have at most 1024 x 32)
         const int threads = (p.vdim / 4 * (p.state / 8) + 63) / 64 * 64;
-        const size_t lds = sizeof(float) * (size_t) (p.state / 8) * p.vdim;
+        const size_t lds = sizeof(float) * ((size_t) (p.state / 8) * p.vdim + (p.convolve ? p.vdim + 2 * p.state : 0));
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.entries, p.heads), dim3(threads), lds, stream, p); };
         if (p.dtype == DT_BF16)
-            hipLaunchKernelGGL((ssm_step_kernel<DT_BF16>), dim3(p.entries, p.heads), dim3(threads), lds, stream, p);
+            p.convolve ? go(ssm_step_kernel<DT_BF16, true>) : go(ssm_step_kernel<DT_BF16, false>);
         else
-            hipLaunchKernelGGL((ssm_step_kernel<DT_FLOAT>), dim3(p.entries, p.heads), dim3(threads), lds, stream, p);
+            p.convolve ? go(ssm_step_kernel<DT_FLOAT, true>) : go(ssm_step_kernel<DT_FLOAT, false>);
         return launched("stack_ssm_scan (one row)");
     }
     static const bool plain_only = [] {

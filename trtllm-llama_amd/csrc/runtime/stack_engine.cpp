@@ -134,7 +134,7 @@ struct Run
     bool enters_pass = false;
     void *k_pool = nullptr, *v_pool = nullptr; // attention
     float* state = nullptr;                    // hgrn2, mamba2
-    float* conv_state = nullptr;               // mamba2, delta_rule: the last taps - 1 inputs of the convolution
+    float* conv_state = nullptr;               // mamba2, delta_rule: the last inputs of the convolution, in a ring of taps rows
     float* shift_carry = nullptr;              // token shift: the sequence's last normed row, [slots, width]
 };
 
@@ -1330,7 +1330,7 @@ int32_t tllm_stack_finalize(tllm_stack_t s)
         {
             void *st = nullptr, *cv = nullptr;
             if (alloc_zero(s, (size_t) s->slots * l.heads * l.dim * l.vdim * 4, &st)
-                || alloc_zero(s, (size_t) s->slots * (l.taps - 1) * l.n_conv * 4, &cv))
+                || alloc_zero(s, (size_t) s->slots * l.taps * l.n_conv * 4, &cv))
                 return -1;
             r.state = (float*) st;
             r.conv_state = (float*) cv;
@@ -1528,7 +1528,16 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             sp.ent_first = d_first;
             sp.ent_count = d_count;
             sp.ent_pos0 = d_pos0;
-            if (launch_stack_ssm_conv(sp, stream))
+            StackDeltaParams dp;
+            dp.max_count = max_count;
+            dp.dim = l.dim;
+            dp.vdim = l.vdim;
+            dp.taps = l.taps;
+            dp.conv_w = l.conv_w;
+            dp.conv_state = r.conv_state;
+            dp.ld_raw = l.n_mix;
+            dp.x_raw = stack_delta_convolves(dp) ? s->proj : nullptr;
+            if (!dp.x_raw && launch_stack_ssm_conv(sp, stream))
                 return -1;
             // the two low-rank projections' second halves, in fp32: the decay's pre-activation and the output gate's
             const int col_b = l.n_conv, col_a = col_b + l.n_beta, col_g = col_a + l.decay_rank;
@@ -1553,14 +1562,11 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             lr.ldc = lr.N;
             if (launch_stack_gemm(lr, stream))
                 return -1;
-            StackDeltaParams dp;
             dp.dtype = s->dtype;
             dp.tokens = T;
             dp.entries = E;
             dp.heads = l.heads;
             dp.qk_heads = l.kv_heads;
-            dp.dim = l.dim;
-            dp.vdim = l.vdim;
             dp.x = s->xbc;
             dp.beta_raw = (const char*) s->proj + (size_t) col_b * s->es;
             dp.ld_beta = l.n_mix;
@@ -1577,7 +1583,6 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             dp.ent_first = d_first;
             dp.ent_count = d_count;
             dp.ent_pos0 = d_pos0;
-            dp.max_count = max_count;
             dp.chunk_ws = s->chunk_ws;
             dp.chunk_floats = s->chunk_floats;
             return launch_stack_delta(dp, stream);
@@ -1614,7 +1619,8 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             sp.chunk_ws = s->chunk_ws;
             sp.chunk_floats = s->chunk_floats;
             // convolution + silu (and the sequence's new tail), the recurrence with skip and gate, the norm in parts of the row
-            if (launch_stack_ssm_conv(sp, stream) || launch_stack_ssm_scan(sp, stream))
+            sp.convolve = stack_ssm_convolves(sp);
+            if ((!sp.convolve && launch_stack_ssm_conv(sp, stream)) || launch_stack_ssm_scan(sp, stream))
                 return -1;
             return launch_stack_group_rmsnorm(s->ctx, nullptr, s->o32, nullptr, l.hnorm, nullptr, s->dtype, T, l.n_ctx, l.ssm_norm_groups, s->eps,
                 stream);
