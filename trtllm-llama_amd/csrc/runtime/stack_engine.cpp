@@ -121,6 +121,7 @@ struct Layer
           *d_skip = nullptr, *router_w = nullptr, *correction = nullptr, *talkw = nullptr, *q_norm = nullptr, *k_norm = nullptr, *o_biasv = nullptr,
           *shift = nullptr;
     void *w_a2 = nullptr, *w_g2 = nullptr; // delta_rule: the second halves of the decay's and the gate's low-rank projections
+    bool low_pair = false;                 // ... of one shape: both in w_a2, one product of two
     void* w_uq = nullptr;
     void *w_shared_up = nullptr, *w_shared_down = nullptr; // shared expert (where it is not part of w_mix / w_o)
     void *side_gate = nullptr, *side_proj = nullptr;       // per-layer token input
@@ -215,7 +216,7 @@ struct tllm_stack
     void free_scratch()
     {
         void* all[] = {chunk_ws, v_first, shared_z, split_ws, x_el, side_act, act_sh, route_z, x, x0, o32, logits, tap, y32, h1, h2, proj, q, ctx, act, hw, lat, ints, ids_out, xbc, cq, qfull, moe_a, moe_y, moe_w, moe_i,
-            h32, dl_a, dl_g, pairs};
+            h32, dl_a, pairs};
         for (void* p : all)
             if (p)
                 (void) hipFree(p);
@@ -443,8 +444,9 @@ int ensure_scratch(tllm_stack* s, int tokens, int want, int n_ints)
         HIP_OK(hipMalloc(&s->qfull, T * std::max(s->max_qfull, 1) * es));
         HIP_OK(hipMalloc((void**) &s->h32, (s->token_shift ? T * wd : 1) * 4));
         HIP_OK(hipMalloc(&s->pairs, T * std::max(s->max_pairs, 1) * es));
-        HIP_OK(hipMalloc((void**) &s->dl_a, T * std::max(s->max_hd, 1) * 4));
-        HIP_OK(hipMalloc((void**) &s->dl_g, (s->max_hd ? T * std::max(s->max_ctx, 1) : 1) * 4));
+        const size_t n_a = (T * std::max(s->max_hd, 1) + 63) / 64 * 64;
+        HIP_OK(hipMalloc((void**) &s->dl_a, (n_a + (s->max_hd ? T * std::max(s->max_ctx, 1) : 1)) * 4)); // one block: a product of two writes both
+        s->dl_g = s->dl_a + n_a;
         {
             // a mixture of experts works on one row per (token, chosen expert)
             const size_t pairs = T * (size_t) std::max(s->max_top, 1);
@@ -1033,6 +1035,7 @@ int32_t tllm_stack_finalize(tllm_stack_t s)
                              *cv = need(s, p + "mix.v.conv", {HV, l.taps});
             if (!wq || !wk || !wv || !wb || !a1 || !a2 || !g1 || !g2 || !wo || !cq || !ck || !cv)
                 return -1;
+            l.low_pair = HD == HV && l.decay_rank == l.gate_rank;
             HostTensor pad_b, pad_end; // zero rows: beta's columns up to a multiple of 8, the projection's up to a multiple of 8
             pad_b.dims = {l.n_beta - l.heads, Wd};
             pad_b.v.assign((size_t) pad_b.numel(), 0.f);
@@ -1041,8 +1044,8 @@ int32_t tllm_stack_finalize(tllm_stack_t s)
             std::vector<float> taps(cq->v);
             taps.insert(taps.end(), ck->v.begin(), ck->v.end());
             taps.insert(taps.end(), cv->v.begin(), cv->v.end());
-            if (upload_rows(s, {wq, wk, wv, wb, &pad_b, a1, g1, &pad_end}, &l.w_mix) || upload_rows(s, {wo}, &l.w_o) || upload_rows(s, {a2}, &l.w_a2)
-                || upload_rows(s, {g2}, &l.w_g2) || upload_f32(s, taps.data(), taps.size(), &l.conv_w) || vec("mix.dt_bias", HD, &l.dt_bias)
+            if (upload_rows(s, {wq, wk, wv, wb, &pad_b, a1, g1, &pad_end}, &l.w_mix) || upload_rows(s, {wo}, &l.w_o)
+                || (l.low_pair ? upload_rows(s, {a2, g2}, &l.w_a2) : upload_rows(s, {a2}, &l.w_a2) || upload_rows(s, {g2}, &l.w_g2)) || upload_f32(s, taps.data(), taps.size(), &l.conv_w) || vec("mix.dt_bias", HD, &l.dt_bias)
                 || vec("mix.A_log", l.heads, &l.a_log) || vec("mix.norm", l.vdim, &l.hnorm))
                 return -1;
         }
@@ -1552,6 +1555,14 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             lr.w = l.w_a2;
             lr.c = s->dl_a;
             lr.ldc = lr.N;
+            if (l.low_pair)
+            {
+                // (a launch instead of two, us: one row, 1024 x 128 3.3 + 3.6, 3.6; 1672 rows 7.7 + 7.7, 13)
+                lr.batch = 2;
+                lr.stride_a = l.decay_rank;
+                lr.stride_w = (int64_t) lr.N * lr.K;
+                lr.stride_c = s->dl_g - s->dl_a;
+            }
             if (launch_stack_gemm(lr, stream))
                 return -1;
             lr.N = l.n_ctx;
@@ -1560,7 +1571,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             lr.w = l.w_g2;
             lr.c = s->dl_g;
             lr.ldc = lr.N;
-            if (launch_stack_gemm(lr, stream))
+            if (!l.low_pair && launch_stack_gemm(lr, stream))
                 return -1;
             dp.dtype = s->dtype;
             dp.tokens = T;
