@@ -394,7 +394,8 @@ __global__ __launch_bounds__(256) void row_short_kernel(const StackGemmParams p_
 // row_kernel whose row is formed here (StackRowNorm) instead of by a launch of its own in front, which costs its start and 2.3 us for some hundred cycles of work: the
 // row is requested ahead of the weights and normed while they are under way.  K <= 512 KS NC.  Rows of more than 2048 values by whole waves, 8 columns a workgroup, as
 // every workgroup reads the row (10240 x 4096 by 2 columns a workgroup 21.6), but for few columns.  us in a step of one token, norm + product and here: 10304 x 2048 2.3 + 11.0, 10.7;
-// 11008 x 2048 2.3 + 11.2, 11.2; 10240 x 4096 4.6 + 14.7, 17.1; 16384 x 4096 4.6 + 21.0, 23.8.
+// 11008 x 2048 2.3 + 11.2, 11.2; 10240 x 4096 4.6 + 14.7, 17.1; 16384 x 4096 4.6 + 21.0, 23.8;
+// 2048 x 4096, 8 parts 3.3 + 5.9, 5.8 (by 4 columns a workgroup 6.5, by 2 7.3).
 template <int KS, int NC, int NP>
 __global__ __launch_bounds__(256) void row_norm_kernel(const StackGemmParams p, const StackRowNorm n)
 {
@@ -803,7 +804,7 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
 bool stack_row_norm_serves(const StackRowNorm& n, int dtype, int width)
 {
     auto pieces = [](const void* p) { return !(reinterpret_cast<uintptr_t>(p) & 15); };
-    return dtype == DT_BF16 && width % 16 == 0 && width > 0 && width <= 4096 && (n.groups == 1 || n.groups == 2 || n.groups == 4) && n.x && n.w && pieces(n.x) && pieces(n.y)
+    return dtype == DT_BF16 && width % 16 == 0 && width > 0 && width <= 4096 && (n.groups == 1 || n.groups == 2 || n.groups == 4 || (n.groups == 8 && width % 2048 == 0)) && n.x && n.w && pieces(n.x) && pieces(n.y)
         && pieces(n.w) && pieces(n.w2) && pieces(n.h) && pieces(n.h2) && pieces(n.x_out) && (!n.y || (n.mix && n.out && n.x_out && n.x_out != n.x)) && (!n.h2 || n.w2);
 }
 

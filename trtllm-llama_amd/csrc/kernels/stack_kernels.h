@@ -69,7 +69,7 @@ struct StackGemmParams
 };
 int launch_stack_gemm(const StackGemmParams& p, hipStream_t stream);
 // A lone token's row as the one launch reads it that needs it: every workgroup forms v = x, or mix[0] x + out[0] y where there is a y, and
-//   row = bfloat16(u / sqrt(mean(u^2) + eps) * w),  u = in[0] v (in null: v), the mean over each of `groups` (1, 2 or 4) parts of the row.
+//   row = bfloat16(u / sqrt(mean(u^2) + eps) * w),  u = in[0] v (in null: v), the mean over each of `groups` (1, 2, 4; 8 of rows of 2048 or 4096) parts of the row.
 // The first workgroup leaves v in x_out (not x itself, which others still read; with a y only), the row in h and the row of weights w2 in h2, where they are set.
 // bfloat16, rows of up to 4096 values in whole pieces of 16 (stack_row_norm_serves).
 struct StackRowNorm

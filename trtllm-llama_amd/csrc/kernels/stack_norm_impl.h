@@ -12,7 +12,8 @@ namespace
 {
 using namespace dev;
 
-// A workgroup of 4 waves; wave q has the q-th quarter of the row, NP pieces of 4 values a lane, so that up to 4 parts with a norm each end where a wave does.
+// A workgroup of 4 waves; wave q has the q-th quarter of the row, NP pieces of 4 values a lane, so that up to 4 parts with a norm each end where a wave does, and 8 (whole
+// pieces of the wave each) where half of its pieces do.
 template <int NP>
 struct LoneRow
 {
@@ -47,12 +48,14 @@ struct LoneRow
     __device__ __forceinline__ void finish(const StackRowNorm& n, int width, uint16_t* row, float* red, bool first)
     {
         const int wid = threadIdx.x >> 6;
-        float ss = 0.f;
+        float ss = 0.f, front = 0.f; // front: of the first half of the pieces
 #pragma unroll
         for (int k = 0; k < NP; ++k)
         {
             bool on;
             const int c = piece(width, k, on);
+            if (k == NP / 2)
+                front = ss, ss = 0.f;
             float4 v = x[k];
             if (n.y)
             {
@@ -64,20 +67,30 @@ struct LoneRow
             x[k] = v;
             ss += on ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f;
         }
-        ss = wave_sum(ss);
-        if ((threadIdx.x & 63) == 0)
-            red[wid] = ss;
-        __syncthreads();
-        ss = n.groups == 4 ? red[wid] : n.groups == 2 ? red[wid & 2] + red[wid | 1] : (red[0] + red[1]) + (red[2] + red[3]);
-        const float inv = 1.f / sqrtf(ss / (float) (width / n.groups) + n.eps);
+        float inv_front, inv;
+        if (n.groups == 8)
+        {
+            inv_front = 1.f / sqrtf(wave_sum(front) / (float) (width >> 3) + n.eps);
+            inv = 1.f / sqrtf(wave_sum(ss) / (float) (width >> 3) + n.eps);
+        }
+        else
+        {
+            ss = wave_sum(front + ss);
+            if ((threadIdx.x & 63) == 0)
+                red[wid] = ss;
+            __syncthreads();
+            ss = n.groups == 4 ? red[wid] : n.groups == 2 ? red[wid & 2] + red[wid | 1] : (red[0] + red[1]) + (red[2] + red[3]);
+            inv_front = inv = 1.f / sqrtf(ss / (float) (width / n.groups) + n.eps);
+        }
 #pragma unroll
         for (int k = 0; k < NP; ++k)
         {
             bool on;
             const int c = piece(width, k, on);
+            const float by = k < NP / 2 ? inv_front : inv;
             auto normed = [&](const float4& s) {
-                return make_uint2((uint32_t) f2bf(x[k].x * inv * s.x) | ((uint32_t) f2bf(x[k].y * inv * s.y) << 16),
-                    (uint32_t) f2bf(x[k].z * inv * s.z) | ((uint32_t) f2bf(x[k].w * inv * s.w) << 16));
+                return make_uint2((uint32_t) f2bf(x[k].x * by * s.x) | ((uint32_t) f2bf(x[k].y * by * s.y) << 16),
+                    (uint32_t) f2bf(x[k].z * by * s.z) | ((uint32_t) f2bf(x[k].w * by * s.w) << 16));
             };
             if (!on)
                 continue;

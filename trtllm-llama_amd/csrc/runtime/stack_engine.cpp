@@ -1477,7 +1477,10 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
 
     // P1 = h1 W_mix^T, then the mixer: its context rows land in s->ctx, ld_ctx elements apart
     // first(g): launches it, its row in s->h1 or formed on the way
+    StackRowNorm mixed;   // what the out-projection forms ctx from where the mixer left it raw
+    bool raw_ctx = false;
     auto run_mixer = [&](const Layer& l, const Run& r, auto first) -> int {
+        raw_ctx = false;
         const int64_t ld_ctx = l.n_ctx + (s->side_by_side && l.kind == MIX_LATENT ? l.shared_ff : 0);
         StackGemmParams g;
         g.dtype = s->dtype;
@@ -1633,6 +1636,17 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             sp.convolve = stack_ssm_convolves(sp);
             if ((!sp.convolve && launch_stack_ssm_conv(sp, stream)) || launch_stack_ssm_scan(sp, stream))
                 return -1;
+            if (T == 1 && !s->side_by_side)
+            {
+                // (by the out-projection)
+                mixed.x = s->o32;
+                mixed.w = l.hnorm;
+                mixed.eps = s->eps;
+                mixed.groups = l.ssm_norm_groups;
+                raw_ctx = stack_row_norm_serves(mixed, s->dtype, l.n_ctx);
+                if (raw_ctx)
+                    return 0;
+            }
             return launch_stack_group_rmsnorm(s->ctx, nullptr, s->o32, nullptr, l.hnorm, nullptr, s->dtype, T, l.n_ctx, l.ssm_norm_groups, s->eps,
                 stream);
         }
@@ -1911,6 +1925,18 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
 
     auto product = [&](const StackGemmParams& g) { return launch_stack_gemm(g, stream); };
     auto formed_before = [](const StackMoeParams*) { return 0; };
+    // a layer's out-projection, behind its mixer
+    auto out_product = [&](const StackGemmParams& g) -> int {
+        if (raw_ctx)
+        {
+            const int rc = launch_stack_row_gemm(g, mixed, stream);
+            if (rc <= 0)
+                return rc;
+            if (launch_stack_group_rmsnorm(s->ctx, nullptr, mixed.x, nullptr, mixed.w, nullptr, s->dtype, T, g.K, mixed.groups, mixed.eps, stream))
+                return -1;
+        }
+        return launch_stack_gemm(g, stream);
+    };
 
     // the feed-forwards of sequential blocks: h1 -> y32
     auto seq_dense = [&](const Layer& l, auto first) -> int {
@@ -2230,7 +2256,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             o.c = s->y32;
             o.ldc = Wd;
             o.bias = l.o_biasv;
-            if (launch_stack_gemm(o, stream))
+            if (out_product(o))
                 return -1;
             leave(0);
             if (l.ff > 0)
@@ -2291,7 +2317,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         o.gate = (const char*) s->proj + (size_t) (l.n_q + l.n_k + l.n_v) * s->es;
         o.ldg = l.n_mix;
         o.gate_bias = l.rg1_b;
-        if (launch_stack_gemm(o, stream))
+        if (out_product(o))
             return -1;
         if (l.ff > 0)
         {
