@@ -181,7 +181,12 @@ struct StackHyperParams
     float* sum_out = nullptr;
     float* h32 = nullptr;          // [tokens, width] or null: the normed row in fp32 as well (a token shift reads it)
     const int32_t* rows = nullptr; // [tokens] or null
+    // carry != null: the token shift of StackShiftParams behind the norm, in a step of one row per entry (row t is entry t's), where stack_hyper_shifts
+    const float* mu = nullptr;
+    float* carry = nullptr;
+    const int32_t *ent_slot = nullptr, *ent_pos0 = nullptr;
 };
+bool stack_hyper_shifts(const StackHyperParams& p); // one stream, rows of whole pieces
 int launch_stack_hyper_norm(const StackHyperParams& p, hipStream_t stream);
 // What lands on one plain residual stream between two sublayers, and the next sublayer's norm, in one pass over a row (fp32):
 //   1. u = y, or table row ids[t] * scale (then the stream starts here: x is not read);  y_norm != null: u = u / sqrt(mean(u^2) + eps) * y_norm;

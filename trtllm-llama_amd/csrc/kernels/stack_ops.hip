@@ -1596,17 +1596,27 @@ __device__ __forceinline__ void expert_sum(const StackExpertSum& m, int t, int w
 // in only where there is one to form, and with one stream a second column only for rows of more than 4096.
 constexpr int HV_K = 2;
 
-template <int DT, int SM, int K, bool SUM>
+// SHIFT: the token shift of a step with one row per entry behind the norm, its carry and blend requested with the row (one stream, as where a shift is used).
+// One row of 1024: 2.9 + 2.2 us as two launches, 3.2.
+template <int DT, int SM, int K, bool SHIFT, bool SUM>
 __global__ __launch_bounds__(1024) void hyper_norm_vec_kernel(const StackHyperParams p)
 {
+    static_assert(!SHIFT || SM == 1, "one stream");
     __shared__ float red[32];
     const int t = p.rows ? p.rows[blockIdx.x] : blockIdx.x, tid = threadIdx.x, S = p.streams, W4 = p.width >> 2, NT = blockDim.x;
     constexpr bool EARLY = SM <= 2; // the norm's weights come in with the row (more streams: no registers left for them)
-    float4 xs[K][SM], yv[K], u[K], wv[K];
+    float4 xs[K][SM], yv[K], u[K], wv[K], mu[SHIFT ? K : 1], old[SHIFT ? K : 1];
+    float4* carry = SHIFT ? reinterpret_cast<float4*>(p.carry + (int64_t) p.ent_slot[t] * p.width) : nullptr;
+    const bool fresh = SHIFT && p.ent_pos0[t] == 0;
 #pragma unroll
     for (int k = 0; k < K; ++k)
     {
         const int c4 = tid + k * NT;
+        if constexpr (SHIFT)
+        {
+            mu[k] = reinterpret_cast<const float4*>(p.mu)[c4 < W4 ? c4 : 0];
+            old[k] = fresh ? make_float4(0.f, 0.f, 0.f, 0.f) : carry[c4 < W4 ? c4 : 0];
+        }
         yv[k] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int s = 0; s < SM; ++s)
@@ -1684,13 +1694,17 @@ __global__ __launch_bounds__(1024) void hyper_norm_vec_kernel(const StackHyperPa
                 *reinterpret_cast<float4*>(p.h32 + o) = make_float4(u[k].x * inv * w.x, u[k].y * inv * w.y, u[k].z * inv * w.z, u[k].w * inv * w.w);
             if (!p.h)
                 continue;
+            float4 n = make_float4(u[k].x * inv * w.x, u[k].y * inv * w.y, u[k].z * inv * w.z, u[k].w * inv * w.w);
+            if constexpr (SHIFT)
+            {
+                carry[c4] = n;
+                n = make_float4(n.x + (old[k].x - n.x) * mu[k].x, n.y + (old[k].y - n.y) * mu[k].y, n.z + (old[k].z - n.z) * mu[k].z, n.w + (old[k].w - n.w) * mu[k].w);
+            }
             if (DT == DT_BF16)
                 *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(p.h) + o)
-                    = make_uint2((uint32_t) f2bf(u[k].x * inv * w.x) | ((uint32_t) f2bf(u[k].y * inv * w.y) << 16),
-                        (uint32_t) f2bf(u[k].z * inv * w.z) | ((uint32_t) f2bf(u[k].w * inv * w.w) << 16));
+                    = make_uint2((uint32_t) f2bf(n.x) | ((uint32_t) f2bf(n.y) << 16), (uint32_t) f2bf(n.z) | ((uint32_t) f2bf(n.w) << 16));
             else
-                *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.h) + o)
-                    = make_float4(u[k].x * inv * w.x, u[k].y * inv * w.y, u[k].z * inv * w.z, u[k].w * inv * w.w);
+                *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.h) + o) = n;
         }
     }
 }
@@ -1699,16 +1713,25 @@ template <int DT>
 void launch_hyper_vec(const StackHyperParams& p, int nt, hipStream_t stream)
 {
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.tokens), dim3(nt), 0, stream, p); };
+    auto with = [&](auto streams, auto pieces) {
+        constexpr int SM = decltype(streams)::value, K = decltype(pieces)::value;
+        if constexpr (SM == 1)
+            if (p.carry)
+                return p.sum.ys ? go(hyper_norm_vec_kernel<DT, SM, K, true, true>) : go(hyper_norm_vec_kernel<DT, SM, K, true, false>);
+        p.sum.ys ? go(hyper_norm_vec_kernel<DT, SM, K, false, true>) : go(hyper_norm_vec_kernel<DT, SM, K, false, false>);
+    };
+    using One = std::integral_constant<int, 1>;
+    using Most = std::integral_constant<int, HV_K>;
     if (p.streams <= 1 && p.width <= 4096)
-        p.sum.ys ? go(hyper_norm_vec_kernel<DT, 1, 1, true>) : go(hyper_norm_vec_kernel<DT, 1, 1, false>);
+        with(One(), One());
     else if (p.streams <= 1)
-        p.sum.ys ? go(hyper_norm_vec_kernel<DT, 1, HV_K, true>) : go(hyper_norm_vec_kernel<DT, 1, HV_K, false>);
+        with(One(), Most());
     else if (p.streams <= 2)
-        p.sum.ys ? go(hyper_norm_vec_kernel<DT, 2, HV_K, true>) : go(hyper_norm_vec_kernel<DT, 2, HV_K, false>);
+        with(std::integral_constant<int, 2>(), Most());
     else if (p.streams <= 4)
-        p.sum.ys ? go(hyper_norm_vec_kernel<DT, 4, HV_K, true>) : go(hyper_norm_vec_kernel<DT, 4, HV_K, false>);
+        with(std::integral_constant<int, 4>(), Most());
     else
-        p.sum.ys ? go(hyper_norm_vec_kernel<DT, 8, HV_K, true>) : go(hyper_norm_vec_kernel<DT, 8, HV_K, false>);
+        with(std::integral_constant<int, 8>(), Most());
 }
 
 // One plain residual stream (StackLandParams): a row stays in registers between its loads, the norm of what lands, the addition and
@@ -1937,6 +1960,18 @@ int launch_stack_land(const StackLandParams& p_in, hipStream_t stream)
     return launched("stack_land");
 }
 
+static bool hyper_vec_serves(const StackHyperParams& p)
+{
+    return p.width % 4 == 0 && p.width <= HV_K * 4096 && p.stream_stride % 4 == 0
+        && !((reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.y) | reinterpret_cast<uintptr_t>(p.h) | reinterpret_cast<uintptr_t>(p.w) | reinterpret_cast<uintptr_t>(p.sum_out)
+                 | reinterpret_cast<uintptr_t>(p.h32) | reinterpret_cast<uintptr_t>(p.sum.ys) | reinterpret_cast<uintptr_t>(p.sum.h)) & 15);
+}
+bool stack_hyper_shifts(const StackHyperParams& p)
+{
+    return hyper_vec_serves(p) && p.streams == 1 && p.h && !p.h32 && !p.rows && p.mu && p.carry && p.ent_slot && p.ent_pos0
+        && !((reinterpret_cast<uintptr_t>(p.mu) | reinterpret_cast<uintptr_t>(p.carry)) & 15);
+}
+
 int launch_stack_hyper_norm(const StackHyperParams& p_in, hipStream_t stream)
 {
     StackHyperParams p = p_in;
@@ -1949,10 +1984,12 @@ int launch_stack_hyper_norm(const StackHyperParams& p_in, hipStream_t stream)
         set_error("stack_hyper_norm: %d streams (1 .. %d) of width %d, or a missing operand", p.streams, HY_MAXS, p.width);
         return -1;
     }
-    const bool al16 = !(reinterpret_cast<uintptr_t>(p.x) & 15) && !(reinterpret_cast<uintptr_t>(p.y) & 15) && !(reinterpret_cast<uintptr_t>(p.h) & 15)
-        && !(reinterpret_cast<uintptr_t>(p.w) & 15) && !(reinterpret_cast<uintptr_t>(p.sum_out) & 15) && !(reinterpret_cast<uintptr_t>(p.h32) & 15)
-        && p.stream_stride % 4 == 0 && !((reinterpret_cast<uintptr_t>(p.sum.ys) | reinterpret_cast<uintptr_t>(p.sum.h)) & 15);
-    if (p.width % 4 == 0 && p.width <= HV_K * 4096 && al16)
+    if (p.carry && !stack_hyper_shifts(p))
+    {
+        set_error("stack_hyper_norm: %d streams of width %d, or an operand that the token shift does not go with", p.streams, p.width);
+        return -1;
+    }
+    if (hyper_vec_serves(p))
     {
         const int nt = std::min(1024, (p.width / 4 + 63) / 64 * 64);
         if (p.dtype == DT_BF16)

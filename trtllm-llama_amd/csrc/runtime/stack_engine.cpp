@@ -2068,7 +2068,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
     // combines the streams for the next reader and norms the combination
     const HyperW* pending = nullptr;
     float* xs = s->x; // the streams; a lone token's single one changes places with x0 where a launch folds a result in that others read at the same time
-    auto hyper = [&](const float* in, void* h, const float* w, float* sum_out, float* h32 = nullptr) -> int {
+    auto hyper_of = [&](const float* in, void* h, const float* w, float* sum_out) -> StackHyperParams {
         StackHyperParams hp;
         hp.dtype = s->dtype;
         hp.tokens = T;
@@ -2088,11 +2088,14 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         hp.w = w;
         hp.eps = s->eps;
         hp.sum_out = sum_out;
-        hp.h32 = h32;
+        return hp;
+    };
+    auto hyper_norm = [&](const StackHyperParams& hp) -> int {
         pending = nullptr;
         left_sum = StackExpertSum();
         return launch_stack_hyper_norm(hp, stream);
     };
+    auto hyper = [&](const float* in, void* h, const float* w, float* sum_out) { return hyper_norm(hyper_of(in, h, w, sum_out)); };
 
     // A lone token's normed row is formed by the launch that reads it, launch(row), where that is the only one, or the first and leaves it for the others; 1: it is not.
     // (what waits for the stream as a sum of experts is formed once, by the norm's own launch)
@@ -2204,24 +2207,41 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             }
             else if (s->token_shift)
             {
-                // the norm leaves its row in fp32; the mixer reads it blended with the previous token's
-                StackShiftParams sh;
-                sh.dtype = s->dtype;
-                sh.tokens = T;
-                sh.entries = E;
-                sh.width = Wd;
-                sh.n = s->h32;
-                sh.mu = l.shift;
-                sh.carry = r.shift_carry;
-                sh.h = s->h1;
-                sh.tok_entry = d_tent;
-                sh.tok_pos = d_tpos;
-                sh.ent_slot = d_slot;
-                sh.ent_first = d_first;
-                sh.ent_count = d_count;
-                sh.ent_pos0 = d_pos0;
-                if (hyper(l.hc[0].in, nullptr, l.norm1, nullptr, s->h32) || launch_stack_token_shift(sh, stream))
+                // the mixer reads the normed row blended with the previous token's: in the norm's launch, or of rows that it leaves in fp32
+                StackHyperParams hp = hyper_of(l.hc[0].in, s->h1, l.norm1, nullptr);
+                hp.mu = l.shift;
+                hp.carry = r.shift_carry;
+                hp.ent_slot = d_slot;
+                hp.ent_pos0 = d_pos0;
+                const bool together = max_count == 1 && stack_hyper_shifts(hp);
+                if (!together)
+                {
+                    hp.carry = nullptr;
+                    hp.h = nullptr;
+                    hp.h32 = s->h32;
+                }
+                if (hyper_norm(hp))
                     return -1;
+                if (!together)
+                {
+                    StackShiftParams sh;
+                    sh.dtype = s->dtype;
+                    sh.tokens = T;
+                    sh.entries = E;
+                    sh.width = Wd;
+                    sh.n = s->h32;
+                    sh.mu = l.shift;
+                    sh.carry = r.shift_carry;
+                    sh.h = s->h1;
+                    sh.tok_entry = d_tent;
+                    sh.tok_pos = d_tpos;
+                    sh.ent_slot = d_slot;
+                    sh.ent_first = d_first;
+                    sh.ent_count = d_count;
+                    sh.ent_pos0 = d_pos0;
+                    if (launch_stack_token_shift(sh, stream))
+                        return -1;
+                }
             }
             // a sublayer's result waits in y32 for the next launch that reads the stream
             auto leave = [&](int sub) {
