@@ -118,6 +118,24 @@ int launch_stack_embed(float* x, float* keep, const int32_t* ids, const void* ta
 // buckets (64-bit arithmetic), or the extra row `buckets` where prev[t] < 0 (a sequence's first token).  pair_table [buckets + 1, width].
 int launch_stack_pair_embed(float* x, const int32_t* ids, const int32_t* prev, const void* pair_table, int32_t dtype, int32_t tokens,
     int32_t width, int32_t buckets, int32_t mul_prev, int32_t mul_cur, hipStream_t stream, int32_t copies = 1, int64_t copy_stride = 0);
+// launch_stack_fetch, launch_stack_embed and (pair_table) launch_stack_pair_embed in one launch, for a step of few tokens whose rows are whole pieces
+// (stack_begin_serves).
+struct StackBegin
+{
+    static constexpr int TOKENS = 16;
+    int32_t dtype = DT_BF16;
+    int32_t* dst = nullptr;
+    const int32_t* host = nullptr;
+    int32_t n = 0;
+    int32_t ids[TOKENS] = {}, prev[TOKENS] = {};
+    float *x = nullptr, *keep = nullptr;
+    const void *table = nullptr, *pair_table = nullptr;
+    int32_t tokens = 0, width = 0, vocab = 0, buckets = 0, mul_prev = 0, mul_cur = 0, copies = 1;
+    int64_t copy_stride = 0;
+    float scale = 1.f;
+};
+bool stack_begin_serves(const StackBegin& p);
+int launch_stack_begin(const StackBegin& p, hipStream_t stream);
 // Token shift: h[t, :] = n[t, :] + (n[t - 1, :] - n[t, :]) * mu[:] over fp32 rows n (a norm's output), t - 1 the previous token of the
 // same sequence: the row above inside an entry, for an entry's first row the sequence's carried row carry[slot, :] (zeros when the
 // entry starts its sequence).  The carry then takes the entry's last row of n.  h in the element type; n is not changed.

@@ -230,6 +230,46 @@ __global__ __launch_bounds__(256) void pair_embed_kernel(float* x, const int32_t
     }
 }
 
+// The start of a step in one launch: workgroups [0, fetches) bring its metadata in, the others form the streams' first rows from ids that come with the launch's parameters.
+// A step of a token pays for launches: fetch, embedding, pair embedding 2.3 + 1.5 + 2.3 us (width 1024) and here 2.9.  (From the host's image, as the metadata comes,
+// a row's id takes its own way over PCIe: 3.9 us a token, 22 1021.)  PAIR: with the pair embedding.
+template <int DT, bool PAIR>
+__global__ __launch_bounds__(256) void begin_kernel(const StackBegin p, int fetches)
+{
+#pragma clang fp contract(off) // (as two launches round)
+    if ((int) blockIdx.x < fetches)
+    {
+        const int i = blockIdx.x * 256 + threadIdx.x;
+        if (blockIdx.y == 0 && i < p.n >> 2)
+            reinterpret_cast<int4*>(p.dst)[i] = reinterpret_cast<const int4*>(p.host)[i];
+        return;
+    }
+    const int t = blockIdx.x - fetches, c = (blockIdx.y * 256 + threadIdx.x) * 8;
+    const int id = p.ids[t], prev = PAIR ? p.prev[t] : 0;
+    if (c >= p.width)
+        return;
+    float v[8], q[8];
+    if constexpr (PAIR)
+        ld8<DT>(p.pair_table, (prev >= 0 ? ((int64_t) prev * p.mul_prev + (int64_t) id * p.mul_cur) % p.buckets : p.buckets) * p.width + c, q);
+    ld8<DT>(p.table, (int64_t) (id < 0 ? 0 : id >= p.vocab ? p.vocab - 1 : id) * p.width + c, v);
+    const int64_t o = (int64_t) t * p.width + c;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        v[k] *= p.scale;
+    auto leave = [&](float* to) {
+        reinterpret_cast<float4*>(to + o)[0] = make_float4(v[0], v[1], v[2], v[3]);
+        reinterpret_cast<float4*>(to + o)[1] = make_float4(v[4], v[5], v[6], v[7]);
+    };
+    if (p.keep)
+        leave(p.keep);
+    if constexpr (PAIR)
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            v[k] += q[k];
+    for (int k = 0; k < p.copies; ++k)
+        leave(p.x + k * p.copy_stride);
+}
+
 // Token shift.  Workgroups [0, tokens): rows behind their entry's first read the step's own rows.  Workgroups [tokens, tokens +
 // entries): an entry's first row, which reads the sequence's carried row, and the new carry - one thread per (entry, channel) reads
 // the old carry before it writes, so the launch has no ordering between workgroups to keep.
@@ -1508,6 +1548,28 @@ int launch_stack_pair_embed(float* x, const int32_t* ids, const int32_t* prev, c
         hipLaunchKernelGGL((pair_embed_kernel<DT_FLOAT>), dim3(tokens), dim3(256), 0, stream, x, ids, prev, pair_table, width, buckets, mul_prev,
             mul_cur, copies, copy_stride);
     return launched("stack_pair_embed");
+}
+
+bool stack_begin_serves(const StackBegin& p)
+{
+    auto pieces = [](const void* q) { return !(reinterpret_cast<uintptr_t>(q) & 15); };
+    return (p.dtype == DT_BF16 || p.dtype == DT_FLOAT) && p.tokens > 0 && p.tokens <= StackBegin::TOKENS && p.n > 0 && p.n % 4 == 0 && p.dst && p.host && pieces(p.dst) && pieces(p.host) && p.x && p.table
+        && p.width > 0 && p.width % 8 == 0 && p.copies > 0 && p.copy_stride % 4 == 0 && pieces(p.x) && pieces(p.keep) && pieces(p.table) && pieces(p.pair_table) && (!p.pair_table || p.buckets > 0);
+}
+int launch_stack_begin(const StackBegin& p, hipStream_t stream)
+{
+    if (!stack_begin_serves(p))
+    {
+        set_error("stack_begin: %d tokens of width %d, %d values, or an operand that does not go with it", p.tokens, p.width, p.n);
+        return -1;
+    }
+    const int fetches = (p.n / 4 + 255) / 256;
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(fetches + p.tokens, (p.width / 8 + 255) / 256), dim3(256), 0, stream, p, fetches); };
+    if (p.dtype == DT_BF16)
+        p.pair_table ? go(begin_kernel<DT_BF16, true>) : go(begin_kernel<DT_BF16, false>);
+    else
+        p.pair_table ? go(begin_kernel<DT_FLOAT, true>) : go(begin_kernel<DT_FLOAT, false>);
+    return launched("stack_begin");
 }
 
 int launch_stack_token_shift(const StackShiftParams& p, hipStream_t stream)

@@ -1456,8 +1456,6 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
     }
     for (int i = 0; i < NW; ++i)
         h_want[i] = b->want_rows[i];
-    if (launch_stack_fetch(s->ints, h, (int) (n_ints + 3) / 4 * 4, stream))
-        return -1;
     const int32_t* d = s->ints;
     const int32_t *d_tok = d, *d_tent = d + T, *d_tpos = d + 2 * T, *d_first = d + 3 * T, *d_count = d_first + E, *d_pos0 = d_count + E,
                   *d_slot = d_pos0 + E, *d_table = d_slot + E, *d_want = d_table + (size_t) E * MB, *d_prev = d_want + NW;
@@ -1465,13 +1463,37 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
     const int Wd = s->width;
     const bool looped = s->loop_stop > s->loop_start;
     const int64_t stream_stride = (int64_t) T * Wd;
-    if (!s->plain // (a plain residual starts in the launch of its first norm)
-        && launch_stack_embed(s->x, looped && s->loop_times > 1 ? s->x0 : nullptr, d_tok, s->embed, s->dtype, T, Wd, s->vocab, s->emb_scale, stream,
-            s->streams, stream_stride))
-        return -1;
-    if (s->pair_buckets > 0
-        && launch_stack_pair_embed(s->x, d_tok, d_prev, s->pair_table, s->dtype, T, Wd, s->pair_buckets, s->pair_mul_prev, s->pair_mul_cur, stream,
-            s->streams, stream_stride))
+    StackBegin begin;
+    begin.dtype = s->dtype;
+    begin.dst = s->ints;
+    begin.host = h;
+    begin.n = (int) (n_ints + 3) / 4 * 4;
+    std::memcpy(begin.ids, h_tok, (size_t) std::min(T, StackBegin::TOKENS) * 4);
+    std::memcpy(begin.prev, h_prev, (size_t) std::min(T, StackBegin::TOKENS) * 4);
+    begin.x = s->x;
+    begin.keep = looped && s->loop_times > 1 ? s->x0 : nullptr;
+    begin.table = s->embed;
+    begin.pair_table = s->pair_buckets > 0 ? s->pair_table : nullptr;
+    begin.tokens = T;
+    begin.width = Wd;
+    begin.vocab = s->vocab;
+    begin.buckets = s->pair_buckets;
+    begin.mul_prev = s->pair_mul_prev;
+    begin.mul_cur = s->pair_mul_cur;
+    begin.copies = s->streams;
+    begin.copy_stride = stream_stride;
+    begin.scale = s->emb_scale;
+    if (!s->plain && stack_begin_serves(begin)) // (a plain residual starts in the launch of its first norm)
+    {
+        if (launch_stack_begin(begin, stream))
+            return -1;
+    }
+    else if (launch_stack_fetch(begin.dst, begin.host, begin.n, stream)
+        || (!s->plain
+            && launch_stack_embed(begin.x, begin.keep, d_tok, s->embed, s->dtype, T, Wd, s->vocab, s->emb_scale, stream, s->streams, stream_stride))
+        || (s->pair_buckets > 0
+            && launch_stack_pair_embed(s->x, d_tok, d_prev, s->pair_table, s->dtype, T, Wd, s->pair_buckets, s->pair_mul_prev, s->pair_mul_cur, stream,
+                s->streams, stream_stride)))
         return -1;
     s->tap_tokens = T;
 
