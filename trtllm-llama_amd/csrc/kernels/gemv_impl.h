@@ -212,8 +212,13 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a)
     };
 
     // ------------------------------------------------------------------ t = 0: every x-independent request
-    uint4 xv[kNXV], gv[kNXV];
-    auto load_x_row = [&](int m) {
+    // Several rows of up to 4096 halfs all come at once, in front of the weights: one after the other each waited behind the weight tile for a round trip of its own,
+    // and for its own barriers (4 rows of fp16, us: 12288 x 4096 21.2 that way, 19.3 here; 2 x 11008 x 4096 32.9, 32.0).  Longer rows take too many registers that
+    // way (two rows of 6 vectors 197 for 134, a wave less per SIMD).
+    constexpr bool AT_ONCE = MB > 1 && kNXV <= kNXVSmall;
+    constexpr int ROWS = AT_ONCE ? MB : 1;
+    uint4 xv[ROWS][kNXV], gv[kNXV];
+    auto load_x_row = [&](int m, uint4 (&x)[kNXV]) {
         if constexpr (X_HALF)
         {
             const uint16_t* xg = reinterpret_cast<const uint16_t*>(p.x) + (int64_t) m * p.ldx;
@@ -224,7 +229,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a)
                 // value inside a conditional block made hipcc wait for each of these loads in turn - two serialised round
                 // trips before the first weight tile was even requested.  Vectors beyond K are zeroed by mask_x().
                 const int k = (tid + j * 256) * 8;
-                xv[j] = *reinterpret_cast<const uint4*>(xg + (k < K ? k : K - 8));
+                x[j] = *reinterpret_cast<const uint4*>(xg + (k < K ? k : K - 8));
             }
         }
         else
@@ -235,21 +240,23 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a)
             for (int j = 0; j < kNXV; ++j)
             {
                 const int k = (tid + j * 256) * 16;
-                xv[j] = *reinterpret_cast<const uint4*>(xg + (k < K ? k : K - 16));
+                x[j] = *reinterpret_cast<const uint4*>(xg + (k < K ? k : K - 16));
             }
         }
     };
     // zero the activation vectors beyond K (after the loads have been issued)
-    auto mask_x = [&]() {
+    auto mask_x = [&](uint4 (&x)[kNXV]) {
         constexpr int XVEC = X_HALF ? 8 : 16;
 #pragma unroll
         for (int j = 0; j < kNXV; ++j)
         {
             const bool ok = (tid + j * 256) * XVEC < K;
-            xv[j] = make_uint4(ok ? xv[j].x : 0u, ok ? xv[j].y : 0u, ok ? xv[j].z : 0u, ok ? xv[j].w : 0u);
+            x[j] = make_uint4(ok ? x[j].x : 0u, ok ? x[j].y : 0u, ok ? x[j].z : 0u, ok ? x[j].w : 0u);
         }
     };
-    load_x_row(0);
+#pragma unroll
+    for (int m = 0; m < ROWS; ++m)
+        load_x_row(m < p.M ? m : 0, xv[m]);
     if constexpr (PK == PK_NORM)
     {
         const uint16_t* gam = reinterpret_cast<const uint16_t*>(p.gamma);
@@ -353,55 +360,36 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a)
 #pragma unroll
     for (int m = 0; m < MB; ++m)
         row_scale[m] = 1.f;
+    auto sum_squares = [&](int m, const uint4 (&x)[kNXV]) {
+        float ss = 0.f;
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
-    {
-        if (m >= p.M) // uniform
-            continue;
-        if (m > 0)
-            load_x_row(m);
-        mask_x();
-        if constexpr (!X_HALF)
+        for (int j = 0; j < kNXV; ++j)
         {
+            const uint32_t ws[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
 #pragma unroll
-            for (int j = 0; j < kNXV; ++j)
+            for (int q = 0; q < 4; ++q)
             {
-                const int k = (tid + j * 256) * 16;
-                if (k < Kp)
-                    *reinterpret_cast<uint4*>(xs + (size_t) m * Kp + k) = xv[j];
+                const h2_t h = u32_as_h2(ws[q]);
+                const float f0 = (float) h.x, f1 = (float) h.y;
+                ss += f0 * f0 + f1 * f1;
             }
-            continue;
         }
+        ss = wave_sum(ss);
+        if (lane == 0)
+            red[m * 4 + wid] = ss;
+    };
+    // behind the sums of squares: the row as the dots see it, and where it is quantised by its own largest value, that
+    auto normalise = [&](int m, uint4 (&x)[kNXV]) {
         float inv = 1.f;
         if constexpr (PK == PK_NORM)
-        {
-            float ss = 0.f;
-#pragma unroll
-            for (int j = 0; j < kNXV; ++j)
-            {
-                const uint32_t ws[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                {
-                    const h2_t h = u32_as_h2(ws[q]);
-                    const float f0 = (float) h.x, f1 = (float) h.y;
-                    ss += f0 * f0 + f1 * f1;
-                }
-            }
-            ss = wave_sum(ss);
-            if (lane == 0)
-                red[m * 4 + wid] = ss;
-            __syncthreads();
-            ss = red[m * 4] + red[m * 4 + 1] + red[m * 4 + 2] + red[m * 4 + 3];
-            inv = 1.0f / sqrtf(ss / (float) K + p.eps);
-        }
+            inv = 1.0f / sqrtf((red[m * 4] + red[m * 4 + 1] + red[m * 4 + 2] + red[m * 4 + 3]) / (float) K + p.eps);
         float amax = 0.f;
         if (PK == PK_NORM || q_dyn)
         {
 #pragma unroll
             for (int j = 0; j < kNXV; ++j)
             {
-                uint32_t xs4[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+                uint32_t xs4[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
                 const uint32_t gs4[4] = {gv[j].x, gv[j].y, gv[j].z, gv[j].w};
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
@@ -417,10 +405,9 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a)
                     }
                     amax = fmaxf(amax, fmaxf(fabsf((float) h.x), fabsf((float) h.y)));
                 }
-                xv[j] = make_uint4(xs4[0], xs4[1], xs4[2], xs4[3]);
+                x[j] = make_uint4(xs4[0], xs4[1], xs4[2], xs4[3]);
             }
         }
-        float qs = pro_q;
         if constexpr (SQ)
         {
             if (q_dyn) // uniform
@@ -428,8 +415,16 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a)
                 amax = wave_max(amax);
                 if (lane == 0)
                     red[32 + m * 4 + wid] = amax;
-                __syncthreads();
-                amax = fmaxf(fmaxf(red[32 + m * 4], red[32 + m * 4 + 1]), fmaxf(red[32 + m * 4 + 2], red[32 + m * 4 + 3]));
+            }
+        }
+    };
+    auto leave = [&](int m, const uint4 (&x)[kNXV]) {
+        float qs = pro_q;
+        if constexpr (SQ)
+        {
+            if (q_dyn)
+            {
+                float amax = fmaxf(fmaxf(red[32 + m * 4], red[32 + m * 4 + 1]), fmaxf(red[32 + m * 4 + 2], red[32 + m * 4 + 3]));
                 amax = fmaxf(amax, h2f(f2h(1e-6f))); // T localMax = 1e-6f (K/quantization.cu:101)
                 qs = 127.f / amax;
                 row_scale[m] = amax / 127.f;
@@ -445,7 +440,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a)
 #pragma unroll
             for (int j = 0; j < kNXV; ++j)
             {
-                const uint32_t ws[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+                const uint32_t ws[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                 {
@@ -469,7 +464,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a)
             {
                 if constexpr (SQ)
                 {
-                    const uint32_t ws[4] = {xv[j].x, xv[j].y, xv[j].z, xv[j].w};
+                    const uint32_t ws[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
                     uint32_t o[2] = {0, 0};
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
@@ -482,10 +477,56 @@ __global__ __launch_bounds__(256) void gemv_kernel(const GemvArgs a)
                     *reinterpret_cast<uint2*>(xs + (size_t) m * Kp + k) = make_uint2(o[0], o[1]);
                 }
                 else
-                    *reinterpret_cast<uint4*>(xs + ((size_t) m * Kp + k) * 2) = xv[j];
+                    *reinterpret_cast<uint4*>(xs + ((size_t) m * Kp + k) * 2) = x[j];
             }
         }
-    }
+    };
+    // rows m0 .. m0 + ROWS - 1, which are in registers
+    auto rows_in = [&](int m0) {
+#pragma unroll
+        for (int m = 0; m < ROWS; ++m)
+        {
+            mask_x(xv[m]);
+            if constexpr (!X_HALF)
+            {
+#pragma unroll
+                for (int j = 0; j < kNXV; ++j)
+                {
+                    const int k = (tid + j * 256) * 16;
+                    if (k < Kp && m0 + m < p.M)
+                        *reinterpret_cast<uint4*>(xs + (size_t) (m0 + m) * Kp + k) = xv[m][j];
+                }
+            }
+            else if constexpr (PK == PK_NORM)
+                sum_squares(m0 + m, xv[m]);
+        }
+        if constexpr (X_HALF)
+        {
+            if constexpr (PK == PK_NORM)
+                __syncthreads();
+#pragma unroll
+            for (int m = 0; m < ROWS; ++m)
+                normalise(m0 + m, xv[m]);
+            if (q_dyn) // uniform
+                __syncthreads();
+#pragma unroll
+            for (int m = 0; m < ROWS; ++m)
+                if (m0 + m < p.M) // uniform
+                    leave(m0 + m, xv[m]);
+        }
+    };
+    if constexpr (AT_ONCE)
+        rows_in(0);
+    else
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+        {
+            if (m >= p.M) // uniform
+                continue;
+            if (m > 0)
+                load_x_row(m, xv[0]);
+            rows_in(m);
+        }
     __syncthreads();
     if (blockIdx.x == 0 && p.x_pro_out && PK != PK_COPY)
     {
