@@ -95,11 +95,13 @@ int launch_stack_fetch(int32_t* dst, const int32_t* host_src, int32_t n, hipStre
 // A few wanted rows leave for pinned host memory in one launch: rows (null: not wanted) receives logits [n, vocab], choice
 // [n, stack_choice_parts(vocab)] the largest value of each part of a row and its lowest place (0x7fffffff: none), from which
 // stack_choose picks on the host: the largest, the lowest place among equals, 0 in a row without a number.
-struct StackChoice
+// A part has arrived, row values and all, once its choice differs from stack_no_choice, which the host leaves there ahead of the launch.
+struct alignas(8) StackChoice
 {
     float value;
     int32_t at;
 };
+constexpr StackChoice stack_no_choice{0.f, -1};
 int stack_choice_parts(int32_t vocab);
 int launch_stack_deliver(float* rows, StackChoice* choice, const float* logits, int32_t n, int32_t vocab, hipStream_t stream);
 inline int32_t stack_choose(const StackChoice* c, int parts)

@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256) void fetch_kernel(int4* dst, const int4* src, 
 
 // Workgroup (part, row): `len` logits of a row go to pinned host memory while their largest is looked for; a row's parts meet on the
 // host.  One row of 32000: 5.1 us with the copy; a workgroup per row took 5.9 us
-// for the choice alone, with two copy commands behind it.
+// for the choice alone, with two copy commands behind it.  The part's choice, one 8-byte store behind everything else, says that it is there.
 template <bool VEC>
 __global__ __launch_bounds__(256) void deliver_kernel(float* rows, StackChoice* choice, const float* logits, int vocab, int len)
 {
@@ -160,12 +160,15 @@ __global__ __launch_bounds__(256) void deliver_kernel(float* rows, StackChoice* 
     }
     if ((tid & 63) == 0)
         part[tid >> 6] = StackChoice{best, at};
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // this wave's part of the row has left
     __syncthreads();
     if (tid != 0)
         return;
     for (int w = 1; w < 4; ++w)
         look(part[w].value, part[w].at);
-    choice[blockIdx.y * gridDim.x + blockIdx.x] = StackChoice{best, at};
+    __threadfence_system();
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(choice + blockIdx.y * gridDim.x + blockIdx.x), __builtin_bit_cast(uint64_t, StackChoice{best, at}), __ATOMIC_RELAXED,
+        __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 template <int DT>
