@@ -2,7 +2,8 @@
 //   a few   -> the streaming GEMV (gemv.hip), the decode path;
 //   M 5..31 -> (int4 weights 3..31) the weight-streaming MFMA product (gemm_slim.hip): a 19-token prompt's projections are bound by the weights,
 //              not by MFMA tiles (weight-only int8, 12288 x 4096 at 19 rows: 26 us; the 128 x 128 register-staged tiles took 116);
-//   M >= 32 -> MFMA tiles: LDS-DMA staged (gemm_glds.hip: SQ / fp16, K-bytes % 128 == 0; gemm_woq.hip: weight-only), else register staged
+//   M >= 32 -> MFMA tiles: LDS-DMA staged (gemm_glds.hip: SQ / fp16, K-bytes % 128 == 0, and its phased and wide forms gemm_sqp.hip, gemm_wide.hip; gemm_woq.hip:
+//              weight-only), else register staged
 //              with in-flight dequantisation (gemm_mfma.hip: odd K);
 //   shapes that none of these serves -> 8-row GEMV slabs.
 #include "dev_utils.h"

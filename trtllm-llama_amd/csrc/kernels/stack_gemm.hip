@@ -754,7 +754,7 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
     }
     // 256 x 256 tiles of gemm_wide_impl.h.  Grouped: where groups have two of them (32 groups, us, in brackets the shapes above: 16384 rows, N 2816, K 2048 227 (282), 12000
     // 176 (202), 16384 rows, 704, 512 24 (34)).  Groups of one tile read their weights alone, from HBM, which a K-tile and a half ahead does not hide: 8192 rows,
-    // 5504, 4096 took 542 (500) in a step, the same rows of fewer columns by themselves 133 (141) at 2816, 2048 and 126 (121) with 6700 rows.
+    // 5504, 4096 took 542 (500, by the tiles of 128 rows 490) in a step, the same rows of fewer columns by themselves 133 (141) at 2816, 2048 and 126 (121) with 6700 rows.
     if (served)
     {
         if (m_expected > 0)
