@@ -1,6 +1,7 @@
 """The tiles of 128 rows and 16 x 16 MFMAs of gemm_wide_impl.h: the forms that test_gpu_product_tiles.py does not reach.  fp32 rows in whole pieces with K of one
 stage, of as many as the ring holds, of one more and of three rings; fp32 sections of 16 columns and of one behind gated columns, of the 256 x 256 tiles too; the
-fp32 residual without a gate, and with one in tiles of 256 columns.  Which sizes take which shape is what test_stack_host_runtime.py checks, without a GPU."""
+fp32 residual without a gate, and with one in tiles of 256 columns; how a gated result is rounded.  Which sizes take which shape is what test_stack_host_runtime.py checks, without a GPU."""
+import numpy as np
 import pytest
 
 import ruzinex_cases as Z
@@ -9,6 +10,7 @@ import test_gpu_product_tiles as P
 import test_gpu_ruzinex as R
 import test_gpu_sodudra
 import test_gpu_tolenex
+import test_gpu_wide_tiles as W
 import tolenex_cases as T
 
 pytestmark = pytest.mark.gpu
@@ -58,3 +60,24 @@ def test_gated_residual():
     w = T.random_weights(cfg, 6)
     s = test_gpu_tolenex.session_for(cfg, w, 'bfloat16', max_tokens=2048)
     test_gpu_tolenex.check_rows(T.replay(s, {'a': toks}, [[('a', rows)]])['a'], toks, w, cfg, 'bfloat16')
+
+
+@pytest.mark.parametrize('rows,cfg', [(rows, P.residual_config(width)) for rows, width in sorted(RESIDUAL.values())] + [(W.RESIDUAL[0], W.residual_config(T))],
+                         ids=[*map(str, sorted(RESIDUAL)), '256 x 256'])
+def test_gate_and_residual_round_apart(rows, cfg):
+    """x + g v as two operations in fp32, the same bits by every tile.  The second matrix picks one value v of a row for columns n and n + half, and x is zero in the second
+    half, which then holds g v as it was rounded."""
+    half, width, ff = cfg['width'] // 2, cfg['width'], cfg['layers'][0]['mlp']['ff']
+    w = T.random_weights(cfg, 6)
+    columns = np.arange(width)
+    w['embed'][:, half:] = 0
+    w['l0.mix.o'][:] = w['l0.rg2'][:] = w['l0.mlp.down'][:] = 0
+    w['l0.mlp.down'][columns, columns % half % ff] = 1
+    w['l0.rg2.b'][:] = 0.3125
+    toks = test_gpu_tolenex.tokens_for(cfg, rows, 5)
+    s = test_gpu_tolenex.session_for(cfg, w, 'bfloat16', max_tokens=4096, max_batch_tokens=4096, max_sequences=1, debug_mode=True)
+    s.step([('a', toks, [0])])
+    x, scaled = w['embed'][toks, :half] * np.float32(cfg['embedding']['scale']), s.engine.tap(0)
+    apart = x + scaled[:, half:]
+    assert (scaled[:, half:] != 0).mean() > 0.9 and (apart.view(np.uint32) & 0xff != 0).mean() > 0.5
+    np.testing.assert_array_equal(scaled[:, :half], apart)

@@ -462,6 +462,7 @@ __device__ __forceinline__ void leave_pairs(const GemmParams& p, const f32x4 (&a
 template <int OUT, int NA, int NB>
 __device__ __forceinline__ void leave_fp32(const GemmParams& p, const f32x4 (&acc)[NA][NB], int lane, void* c, int row0, int col0, int rows)
 {
+#pragma clang fp contract(off) // (the gated product is rounded before it is added, as gemm_glds_impl.h leaves it)
     float* out = OUT == OUT_FP32 ? reinterpret_cast<float*>(c) : p.resid;
     const int64_t ld = OUT == OUT_FP32 ? p.ldc : p.ldr;
 #pragma unroll
