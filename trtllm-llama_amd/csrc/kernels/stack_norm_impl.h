@@ -12,6 +12,15 @@ namespace
 {
 using namespace dev;
 
+// x^2 + y^2 + z^2 + w^2 with its contraction written out, x^2 or y^2 rounded first: left to the compiler, which of the two turned over with the code around it, and with it the
+// last bit of a norm.  A row's sum of squares has the same bits in every launch that forms it.
+template <bool X_FIRST>
+__device__ __forceinline__ float sum_squares4(const float4& v)
+{
+    const float xy = X_FIRST ? fmaf(v.y, v.y, v.x * v.x) : fmaf(v.x, v.x, v.y * v.y);
+    return fmaf(v.w, v.w, fmaf(v.z, v.z, xy));
+}
+
 // A workgroup of 4 waves; wave q has the q-th quarter of the row, NP pieces of 4 values a lane, so that up to 4 parts with a norm each end where a wave does, and 8 (whole
 // pieces of the wave each) where half of its pieces do.
 template <int NP>

@@ -4,6 +4,7 @@
 #include "dev_utils.h"
 #include "stack_chunk.h"
 #include "stack_kernels.h"
+#include "stack_norm_impl.h"
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -1741,7 +1742,7 @@ __global__ __launch_bounds__(1024) void hyper_norm_vec_kernel(const StackHyperPa
         u[k] = acc;
         if (p.sum_out && c4 < W4)
             reinterpret_cast<float4*>(p.sum_out + (int64_t) t * p.width)[c4] = acc;
-        ss += acc.x * acc.x + acc.y * acc.y + acc.z * acc.z + acc.w * acc.w;
+        ss += sum_squares4<DT == DT_BF16 && SM <= 2>(acc);
     }
     if (!p.h && !p.h32)
         return;
