@@ -136,7 +136,7 @@ int64_t tllm_stack_weight_bytes(tllm_stack_t s);
  * routed feed-forward the experts that the step's tokens reach when every choice falls on another expert */
 int64_t tllm_stack_step_bytes(tllm_stack_t s, int32_t n_tokens, int64_t context_tokens, int32_t n_entries);
 
-/* debug_taps=1: the residual stream behind layer run `run` of the last step (the sum of the streams, if there are several), fp32
+/* debug_taps=1 (every norm has a launch of its own then; the results are the same bits): the residual stream behind layer run `run` of the last step (the sum of the streams, if there are several), fp32
  * [n_tokens, width], to host memory. */
 int32_t tllm_stack_get_tap(tllm_stack_t s, int32_t run, float* out, size_t n_floats);
 

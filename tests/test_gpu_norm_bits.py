@@ -5,7 +5,11 @@ import numpy as np
 import pytest
 
 import narurax_cases as N
+import rofozen_cases as F
 import test_gpu_narurax
+import test_gpu_rofozen
+import test_gpu_tolenex
+import tolenex_cases as T
 from tolenex_cases import bf16_round
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +70,29 @@ def test_norm_of_one_stream(width):
     assert (want != other).any()
     s = test_gpu_narurax.session_for(cfg, w, 'bfloat16', max_tokens=2048, max_sequences=1)
     np.testing.assert_array_equal(s.step([('a', toks, list(range(len(toks))))])[0], want)
+
+
+def small(**kw):
+    return dict(heads=2, vdim=16, state=16, groups=1, norm_groups=1, **kw)
+
+
+LONE = {
+    **{f'one stream of {width}': (F, F.make_config([F.mamba_layer(**small(mlp=F.dense(ff=40))), F.latent_layer(mlp=F.moe(experts=4, identity=2, top=2, count=1, keep=1)),
+                                                    F.mamba_layer(**small(mlp=None)), F.mamba_layer(**small(mlp=F.dense(ff=24)))], width=width)) for width in (96, 1024, 1040, 2048, 3088, 4096)},
+    'one stream of 4096 and many columns': (F, F.make_config([F.mamba_layer(heads=70, vdim=32, state=8, groups=1, norm_groups=1, mlp=F.dense(ff=40))] * 2, width=4096)),
+    **{f'{groups} parts of {width}': (T, T.make_config([T.attention_layer(heads=2, kv_heads=1, dim=16, vdim=16, rot_dims=8, ff=40), T.hgrn2_layer(heads=2, dim=16, vdim=16, ff=24)],
+                                                       width=width, groups=groups)) for width, groups in ((96, 1), (96, 2), (1040, 4), (2048, 1), (2064, 2), (2048, 8), (4096, 1), (4096, 4), (4096, 8))},
+    **{f'{parts} parts of {heads * vdim} behind a state': (F, F.make_config([F.mamba_layer(heads=heads, vdim=vdim, state=8, groups=1, norm_groups=parts)] * 3, width=96))
+       for heads, vdim, parts in ((2, 8, 1), (4, 16, 4), (32, 64, 1), (32, 64, 2), (32, 64, 8), (64, 64, 4), (64, 64, 8))},
+}
+
+
+@pytest.mark.parametrize('name', LONE)
+def test_lone_rows(name):
+    """A lone token's rows normed by the launches that read them, and (taps: every norm has a launch) by launches of their own: the same logits to the last bit."""
+    cases, cfg = LONE[name]
+    w = cases.random_weights(cfg, 5)
+    mod = test_gpu_rofozen if cases is F else test_gpu_tolenex
+    toks = mod.tokens_for(cfg, 200, 7)
+    rows = [[s.step([('a', [t], [0])])[0] for t in toks] for s in (mod.session_for(cfg, w, 'bfloat16', max_sequences=1, debug_mode=mode) for mode in (False, True))]
+    np.testing.assert_array_equal(*map(np.concatenate, rows))

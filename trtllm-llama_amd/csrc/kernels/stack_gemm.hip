@@ -396,15 +396,16 @@ __global__ __launch_bounds__(256) void row_short_kernel(const StackGemmParams p_
 // every workgroup reads the row (10240 x 4096 by 2 columns a workgroup 21.6), but for few columns.  us in a step of one token, norm + product and here: 10304 x 2048 2.3 + 11.0, 10.7;
 // 11008 x 2048 2.3 + 11.2, 11.2; 10240 x 4096 4.6 + 14.7, 17.1; 16384 x 4096 4.6 + 21.0, 23.8;
 // 2048 x 4096, 8 parts 3.3 + 5.9, 5.8 (by 4 columns a workgroup 6.5, by 2 7.3).
-template <int KS, int NC, int NP>
+template <int KS, int NC, int NP, int PARTS>
 __global__ __launch_bounds__(256) void row_norm_kernel(const StackGemmParams p, const StackRowNorm n)
 {
     constexpr int TEAMS = 4 / KS;
+    constexpr int SUMS = KS == 1 && NC > 4 ? 4 : 1; // of a wave: K in the parts, and their order, of row_kernel's waves, which share rows of more than 2048
     __shared__ __attribute__((aligned(16))) uint16_t row[NP * 1024];
-    __shared__ float red[4], part[4][SK_R];
+    __shared__ float red[LoneRow<NP, PARTS>::SUMS], part[4][SK_R];
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kw = wid % KS;
     const int n0 = (blockIdx.x * TEAMS + wid / KS) * SK_R;
-    LoneRow<NP> lone;
+    LoneRow<NP, PARTS> lone;
     lone.request(n, p.K);
     uint4 wv[NC][SK_R];
 #pragma unroll
@@ -417,7 +418,7 @@ __global__ __launch_bounds__(256) void row_norm_kernel(const StackGemmParams p, 
     }
     const RowSeam ops = row_seam_request(p, n0 < p.N ? n0 : p.N - 1);
     lone.finish(n, p.K, row, red, blockIdx.x == 0);
-    float acc[SK_R] = {0.f, 0.f};
+    float acc[SUMS][SK_R] = {};
 #pragma unroll
     for (int i = 0; i < NC; ++i)
     {
@@ -432,12 +433,18 @@ __global__ __launch_bounds__(256) void row_norm_kernel(const StackGemmParams p, 
 #pragma unroll
             for (int q = 0; q < 4; ++q)
             {
-                acc[r] = fmaf(__builtin_bit_cast(float, xs[q] << 16), __builtin_bit_cast(float, ws[q] << 16), acc[r]);
-                acc[r] = fmaf(__builtin_bit_cast(float, xs[q] & 0xffff0000u), __builtin_bit_cast(float, ws[q] & 0xffff0000u), acc[r]);
+                acc[i % SUMS][r] = fmaf(__builtin_bit_cast(float, xs[q] << 16), __builtin_bit_cast(float, ws[q] << 16), acc[i % SUMS][r]);
+                acc[i % SUMS][r] = fmaf(__builtin_bit_cast(float, xs[q] & 0xffff0000u), __builtin_bit_cast(float, ws[q] & 0xffff0000u), acc[i % SUMS][r]);
             }
         }
     }
-    float v0 = wave_sum(acc[0]), v1 = wave_sum(acc[1]);
+    float v0 = wave_sum(acc[0][0]), v1 = wave_sum(acc[0][1]);
+#pragma unroll
+    for (int k = 1; k < SUMS; ++k)
+    {
+        v0 += wave_sum(acc[k][0]);
+        v1 += wave_sum(acc[k][1]);
+    }
     if constexpr (KS > 1)
     {
         if (lane == 0)
@@ -804,8 +811,8 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
 bool stack_row_norm_serves(const StackRowNorm& n, int dtype, int width)
 {
     auto pieces = [](const void* p) { return !(reinterpret_cast<uintptr_t>(p) & 15); };
-    return dtype == DT_BF16 && width % 16 == 0 && width > 0 && width <= 4096 && (n.groups == 1 || n.groups == 2 || n.groups == 4 || (n.groups == 8 && width % 2048 == 0)) && n.x && n.w && pieces(n.x) && pieces(n.y)
-        && pieces(n.w) && pieces(n.w2) && pieces(n.h) && pieces(n.h2) && pieces(n.x_out) && (!n.y || (n.mix && n.out && n.x_out && n.x_out != n.x)) && (!n.h2 || n.w2);
+    return dtype == DT_BF16 && width % 16 == 0 && width > 0 && width <= 4096 && (n.parts == 0 || ((n.parts == 1 || n.parts == 2 || n.parts == 4 || (n.parts == 8 && width % 2048 == 0)) && !n.y && !n.in)) && n.x && n.w && pieces(n.x) && pieces(n.y)
+        && pieces(n.w) && pieces(n.w2) && pieces(n.h) && pieces(n.h2) && pieces(n.x_out) && (!n.y || (n.mix && n.out && n.x_out && n.x_out != n.x)) && (!n.h2 || (n.w2 && n.parts));
 }
 
 int launch_stack_row_gemm(const StackGemmParams& p_in, const StackRowNorm& n, hipStream_t stream)
@@ -820,7 +827,18 @@ int launch_stack_row_gemm(const StackGemmParams& p_in, const StackRowNorm& n, hi
     const bool many = p.N > 16 * launch_util::device_cus(); // as in pick_row_shape
     auto go = [&](auto shape, auto np) {
         using S = decltype(shape);
-        hipLaunchKernelGGL((row_norm_kernel<S::KS, S::NC, decltype(np)::value>), dim3((p.N + S::cols - 1) / S::cols), dim3(256), 0, stream, p, n);
+        constexpr int NP = decltype(np)::value;
+        auto in = [&](auto parts) { hipLaunchKernelGGL((row_norm_kernel<S::KS, S::NC, NP, decltype(parts)::value>), dim3((p.N + S::cols - 1) / S::cols), dim3(256), 0, stream, p, n); };
+        switch (n.parts)
+        {
+        case 0: return in(std::integral_constant<int, 0>());
+        case 1: return in(std::integral_constant<int, 1>());
+        case 2: return in(std::integral_constant<int, 2>());
+        case 4: return in(std::integral_constant<int, 4>());
+        default:
+            if constexpr (NP > 1)
+                in(std::integral_constant<int, 8>());
+        }
     };
     using Quarter1 = std::integral_constant<int, 1>; // pieces of a lane
     using Quarter2 = std::integral_constant<int, 2>;

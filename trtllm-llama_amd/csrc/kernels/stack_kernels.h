@@ -69,8 +69,9 @@ struct StackGemmParams
 };
 int launch_stack_gemm(const StackGemmParams& p, hipStream_t stream);
 // A lone token's row as the one launch reads it that needs it: every workgroup forms v = x, or mix[0] x + out[0] y where there is a y, and
-//   row = bfloat16(u / sqrt(mean(u^2) + eps) * w),  u = in[0] v (in null: v), the mean over each of `groups` (1, 2, 4; 8 of rows of 2048 or 4096) parts of the row.
-// The first workgroup leaves v in x_out (not x itself, which others still read; with a y only), the row in h and the row of weights w2 in h2, where they are set.
+//   row = bfloat16(u / sqrt(mean(u^2) + eps) * w),  u = in[0] v (in null: v), to the bits of the launch whose place it takes: parts 0: of launch_stack_hyper_norm; 1, 2, 4
+// (8 of rows of 2048 or 4096): of launch_stack_group_rmsnorm, the mean over each of so many parts of the row, without y and in.
+// The first workgroup leaves v in x_out (not x itself, which others still read; with a y only), the row in h and the row of weights w2 in h2 (in parts only), where they are set.
 // bfloat16, rows of up to 4096 values in whole pieces of 16 (stack_row_norm_serves).
 struct StackRowNorm
 {
@@ -79,7 +80,7 @@ struct StackRowNorm
     const float *mix = nullptr, *out = nullptr, *in = nullptr;
     const float *w = nullptr, *w2 = nullptr;
     float eps = 1e-5f;
-    int32_t groups = 1;
+    int32_t parts = 0;
     float* x_out = nullptr;
     void *h = nullptr, *h2 = nullptr;
 };

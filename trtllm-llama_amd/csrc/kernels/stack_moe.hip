@@ -158,9 +158,9 @@ __global__ __launch_bounds__(256) void moe_logits_norm_kernel(const StackMoePara
 {
     constexpr int PIECES = 2 * NP; // of 512 values, all requested at once
     __shared__ __attribute__((aligned(16))) uint16_t row[NP * 1024];
-    __shared__ float red[4];
+    __shared__ float red[LoneRow<NP, 0>::SUMS];
     const int NE = p.experts + p.identity, W = p.width, lane = threadIdx.x & 63, e = blockIdx.x * 4 + (threadIdx.x >> 6);
-    LoneRow<NP> lone;
+    LoneRow<NP, 0> lone;
     lone.request(n, W);
     const float* wr = p.router_w + (int64_t) (e < NE ? e : NE - 1) * W;
     float4 w[PIECES][2];
@@ -874,7 +874,7 @@ int launch_stack_moe_logits(const StackMoeParams& p, hipStream_t stream)
 
 int launch_stack_moe_logits(const StackMoeParams& p, const StackRowNorm& n, hipStream_t stream)
 {
-    if (p.tokens != 1 || !stack_row_norm_serves(n, p.dtype, p.width) || !moe_ok(p, "stack_moe_logits"))
+    if (p.tokens != 1 || n.parts || !stack_row_norm_serves(n, p.dtype, p.width) || !moe_ok(p, "stack_moe_logits"))
     {
         set_error("stack_moe_logits: %d tokens of width %d, or a missing operand", p.tokens, p.width);
         return -1;

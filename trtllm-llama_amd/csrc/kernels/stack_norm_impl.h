@@ -3,6 +3,7 @@
 #pragma once
 #include "dev_utils.h"
 #include "stack_kernels.h"
+#include <type_traits>
 
 namespace tllm
 {
@@ -21,21 +22,37 @@ __device__ __forceinline__ float sum_squares4(const float4& v)
     return fmaf(v.w, v.w, fmaf(v.z, v.z, xy));
 }
 
-// A workgroup of 4 waves; wave q has the q-th quarter of the row, NP pieces of 4 values a lane, so that up to 4 parts with a norm each end where a wave does, and 8 (whole
-// pieces of the wave each) where half of its pieces do.
-template <int NP>
-struct LoneRow
+// the squares of a thread's values of a part, likewise: the second one's first
+template <int N>
+__device__ __forceinline__ float sum_squares(const float (&v)[N])
 {
+    float ss = v[0] * v[0];
+    if constexpr (N > 1)
+        ss = fmaf(v[0], v[0], v[1] * v[1]);
+#pragma unroll
+    for (int k = 2; k < N; ++k)
+        ss = fmaf(v[k], v[k], ss);
+    return ss;
+}
+
+// Both forms: request() asks for the row, ahead of the operands that it is to arrive before and without a branch that a load would wait behind; finish() leaves it in `row`, LDS
+// [width] in bfloat16.  red: LDS, SUMS floats.  first: this workgroup also leaves what later launches read.  The sums of squares run in the order of the launch whose place
+// is taken, so that a row has the same bits either way; what that costs (a sum over a wave a piece instead of one in all) passes while the weights are under way.
+
+// A row of one stream, as hyper_norm_vec_kernel: a lane's float4, 64 lanes, the 256 values of each wave in turn.  The workgroup's 4 waves have NP such pieces each.
+template <int NP>
+struct StreamRow
+{
+    static constexpr int SUMS = 4 * NP;
     float4 x[NP], y[NP], w[NP];
     float cm, co, ci;
 
     __device__ __forceinline__ static int piece(int width, int k, bool& on)
     {
-        const int quarter = width >> 4, i = (threadIdx.x & 63) + 64 * k;
-        on = i < quarter;
-        return (int) (threadIdx.x >> 6) * quarter + (on ? i : 0);
+        const int c = threadIdx.x + 256 * k;
+        on = c < width >> 2;
+        return on ? c : 0;
     }
-    // all loads, without a branch that they would wait behind; ahead of the operands that they are to arrive before
     __device__ __forceinline__ void request(const StackRowNorm& n, int width)
     {
         const float* y_or_x = n.y ? n.y : n.x;
@@ -53,18 +70,13 @@ struct LoneRow
         }
         asm volatile("" ::: "memory"); // (what is requested next does not go in front)
     }
-    // row: LDS [width], the normed row in bfloat16; red: LDS [4].  first: this workgroup also leaves what later launches read.
     __device__ __forceinline__ void finish(const StackRowNorm& n, int width, uint16_t* row, float* red, bool first)
     {
-        const int wid = threadIdx.x >> 6;
-        float ss = 0.f, front = 0.f; // front: of the first half of the pieces
 #pragma unroll
         for (int k = 0; k < NP; ++k)
         {
             bool on;
             const int c = piece(width, k, on);
-            if (k == NP / 2)
-                front = ss, ss = 0.f;
             float4 v = x[k];
             if (n.y)
             {
@@ -72,47 +84,104 @@ struct LoneRow
                 if (first && on)
                     reinterpret_cast<float4*>(n.x_out)[c] = v;
             }
-            v = make_float4(ci * v.x, ci * v.y, ci * v.z, ci * v.w);
-            x[k] = v;
-            ss += on ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f;
-        }
-        float inv_front, inv;
-        if (n.groups == 8)
-        {
-            inv_front = 1.f / sqrtf(wave_sum(front) / (float) (width >> 3) + n.eps);
-            inv = 1.f / sqrtf(wave_sum(ss) / (float) (width >> 3) + n.eps);
-        }
-        else
-        {
-            ss = wave_sum(front + ss);
+            x[k] = make_float4(ci * v.x, ci * v.y, ci * v.z, ci * v.w);
+            const float ss = wave_sum(on ? sum_squares4<true>(x[k]) : 0.f);
             if ((threadIdx.x & 63) == 0)
-                red[wid] = ss;
-            __syncthreads();
-            ss = n.groups == 4 ? red[wid] : n.groups == 2 ? red[wid & 2] + red[wid | 1] : (red[0] + red[1]) + (red[2] + red[3]);
-            inv_front = inv = 1.f / sqrtf(ss / (float) (width / n.groups) + n.eps);
+                red[4 * k + (threadIdx.x >> 6)] = ss;
         }
+        __syncthreads();
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < SUMS; ++i)
+            ss += red[i];
+        const float inv = 1.f / sqrtf(ss / (float) width + n.eps);
 #pragma unroll
         for (int k = 0; k < NP; ++k)
         {
             bool on;
             const int c = piece(width, k, on);
-            const float by = k < NP / 2 ? inv_front : inv;
-            auto normed = [&](const float4& s) {
-                return make_uint2((uint32_t) f2bf(x[k].x * by * s.x) | ((uint32_t) f2bf(x[k].y * by * s.y) << 16),
-                    (uint32_t) f2bf(x[k].z * by * s.z) | ((uint32_t) f2bf(x[k].w * by * s.w) << 16));
-            };
             if (!on)
                 continue;
-            const uint2 h = normed(w[k]);
+            const uint2 h = make_uint2((uint32_t) f2bf(x[k].x * inv * w[k].x) | ((uint32_t) f2bf(x[k].y * inv * w[k].y) << 16),
+                (uint32_t) f2bf(x[k].z * inv * w[k].z) | ((uint32_t) f2bf(x[k].w * inv * w[k].w) << 16));
             reinterpret_cast<uint2*>(row)[c] = h;
             if (first && n.h)
                 reinterpret_cast<uint2*>(n.h)[c] = h;
-            if (first && n.h2)
-                reinterpret_cast<uint2*>(n.h2)[c] = normed(reinterpret_cast<const float4*>(n.w2)[c]);
         }
         __syncthreads();
     }
 };
+
+// A row in PARTS with a norm each, as group_rmsnorm_kernel: thread t has values t, t + 256, ... of a part, 64 lanes, 4 waves.  A part has up to 256 EACH values.
+template <int NP, int PARTS>
+struct PartsRow
+{
+    static constexpr int SUMS = 4 * PARTS, EACH = 4 * NP / PARTS;
+    static_assert(EACH * PARTS == 4 * NP, "whole parts");
+    float x[PARTS][EACH], w[PARTS][EACH];
+
+    __device__ __forceinline__ static int place(int width, int g, int k, bool& on)
+    {
+        const int part = width / PARTS, i = threadIdx.x + 256 * k;
+        on = i < part;
+        return on ? g * part + i : 0;
+    }
+    __device__ __forceinline__ void request(const StackRowNorm& n, int width)
+    {
+#pragma unroll
+        for (int g = 0; g < PARTS; ++g)
+#pragma unroll
+            for (int k = 0; k < EACH; ++k)
+            {
+                bool on;
+                const int i = place(width, g, k, on);
+                x[g][k] = n.x[i];
+                w[g][k] = n.w[i];
+            }
+        asm volatile("" ::: "memory");
+    }
+    __device__ __forceinline__ void finish(const StackRowNorm& n, int width, uint16_t* row, float* red, bool first)
+    {
+#pragma unroll
+        for (int g = 0; g < PARTS; ++g)
+        {
+#pragma unroll
+            for (int k = 0; k < EACH; ++k)
+            {
+                bool on;
+                place(width, g, k, on);
+                x[g][k] = on ? x[g][k] : 0.f;
+            }
+            const float ss = wave_sum(sum_squares(x[g]));
+            if ((threadIdx.x & 63) == 0)
+                red[4 * g + (threadIdx.x >> 6)] = ss;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < PARTS; ++g)
+        {
+            const float ss = ((red[4 * g] + red[4 * g + 1]) + red[4 * g + 2]) + red[4 * g + 3];
+            const float inv = 1.f / sqrtf(ss / (float) (width / PARTS) + n.eps);
+#pragma unroll
+            for (int k = 0; k < EACH; ++k)
+            {
+                bool on;
+                const int i = place(width, g, k, on);
+                if (!on)
+                    continue;
+                const float v = x[g][k] * inv;
+                row[i] = f2bf(v * w[g][k]);
+                if (first && n.h)
+                    reinterpret_cast<uint16_t*>(n.h)[i] = f2bf(v * w[g][k]);
+                if (first && n.h2)
+                    reinterpret_cast<uint16_t*>(n.h2)[i] = f2bf(v * n.w2[i]);
+            }
+        }
+        __syncthreads();
+    }
+};
+template <int NP, int PARTS>
+using LoneRow = typename std::conditional<PARTS == 0, StreamRow<NP>, PartsRow<NP, PARTS ? PARTS : 1>>::type;
 
 } // namespace
 } // namespace kernels

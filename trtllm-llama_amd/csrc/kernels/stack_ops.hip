@@ -403,16 +403,16 @@ __global__ __launch_bounds__(GN_T) void group_rmsnorm_kernel(void* y1, void* y2,
     const int r = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
     const int gs = width / groups;
     const float* xg = x + (int64_t) (rows ? rows[r] : r) * width + g * gs;
-    float v[GN_EPT], ss = 0.f;
+    float v[GN_EPT];
 #pragma unroll
     for (int k = 0; k < GN_EPT; ++k)
     {
         const int i = tid + k * GN_T;
         v[k] = i < gs ? xg[i] : 0.f;
-        ss += v[k] * v[k];
     }
+    float ss = sum_squares(v);
     for (int i = tid + GN_EPT * GN_T; i < gs; i += GN_T) // groups beyond GN_T * GN_EPT elements: the tail is read twice
-        ss += xg[i] * xg[i];
+        ss = fmaf(xg[i], xg[i], ss);
     ss = block_sum(ss, red);
     const float inv = 1.f / sqrtf(ss / (float) gs + eps);
 #pragma unroll

@@ -1690,13 +1690,13 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             sp.convolve = stack_ssm_convolves(sp);
             if ((!sp.convolve && launch_stack_ssm_conv(sp, stream)) || launch_stack_ssm_scan(sp, stream))
                 return -1;
-            if (T == 1 && !s->side_by_side)
+            if (T == 1 && !s->side_by_side && !s->taps)
             {
                 // (by the out-projection)
                 mixed.x = s->o32;
                 mixed.w = l.hnorm;
                 mixed.eps = s->eps;
-                mixed.groups = l.ssm_norm_groups;
+                mixed.parts = l.ssm_norm_groups;
                 raw_ctx = stack_row_norm_serves(mixed, s->dtype, l.n_ctx);
                 if (raw_ctx)
                     return 0;
@@ -1986,7 +1986,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             const int rc = launch_stack_row_gemm(g, mixed, stream);
             if (rc <= 0)
                 return rc;
-            if (launch_stack_group_rmsnorm(s->ctx, nullptr, mixed.x, nullptr, mixed.w, nullptr, s->dtype, T, g.K, mixed.groups, mixed.eps, stream))
+            if (launch_stack_group_rmsnorm(s->ctx, nullptr, mixed.x, nullptr, mixed.w, nullptr, s->dtype, T, g.K, mixed.parts, mixed.eps, stream))
                 return -1;
         }
         return launch_stack_gemm(g, stream);
@@ -2152,7 +2152,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
     auto hyper = [&](const float* in, void* h, const float* w, float* sum_out) { return hyper_norm(hyper_of(in, h, w, sum_out)); };
 
     // A lone token's normed row is formed by the launch that reads it, launch(row), where that is the only one, or the first and leaves it for the others; 1: it is not.
-    // (what waits for the stream as a sum of experts is formed once, by the norm's own launch)
+    // (what waits for the stream as a sum of experts is formed once, by the norm's own launch; with taps every norm has one, here and below)
     auto lone_row = [&](const float* in, const float* w, void* h, auto launch) -> int {
         if (T != 1 || !s->hyper || s->streams != 1 || s->taps || (pending && left_sum.ys))
             return 1;
@@ -2357,7 +2357,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             && launch_stack_pass_entry(s->x, r.pass > 0 ? s->x0 : nullptr, s->loop_step + (size_t) r.pass * Wd, T, Wd, stream))
             return -1;
         auto normed = [&](const StackGemmParams& g) -> int {
-            if (T == 1)
+            if (T == 1 && !s->taps)
             {
                 StackRowNorm n;
                 n.x = s->x;
@@ -2365,7 +2365,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
                 n.w2 = l.norm2;
                 n.h2 = l.ff > 0 ? s->h2 : nullptr;
                 n.eps = s->eps;
-                n.groups = s->groups;
+                n.parts = s->groups;
                 const int rc = launch_stack_row_gemm(g, n, stream);
                 if (rc <= 0)
                     return rc;
