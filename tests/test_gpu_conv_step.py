@@ -1,6 +1,6 @@
 """Steps of one row per entry, where the recurrence's step kernel forms the convolution itself (stack_conv_impl.h) on a ring of raw inputs that prompts write as well:
 sequences that begin with single tokens or with prompts of 1 .. 5, steps of single rows behind steps of several in between, a slot that an earlier sequence used,
-channels that heads share and such that fill a workgroup's threads several times."""
+channels that heads share and such that fill a workgroup's threads several times; positions that do not continue a sequence."""
 import numpy as np
 import pytest
 
@@ -46,3 +46,24 @@ def test_steps_of_single_rows(layer, dtype):
         got = test.replay(s, toks, schedule(reqs, starts))
         for name in toks:
             test.check_rows(got[name], toks[name], w, cfg, dtype, f'{layer} {name}')
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('taps', [3, 4])
+@pytest.mark.parametrize('layer', ['shared', 'delta shared'])
+def test_positions_that_do_not_continue(layer, taps, dtype):
+    """The convolution's history is what the sequence was fed last, whatever positions its caller counts: the same bits as with positions that continue."""
+    cases, test = (N, test_gpu_narurax) if layer.startswith('delta') else (M, test_gpu_rofozen)
+    kind = dict(LAYERS[layer], mixer=dict(LAYERS[layer]['mixer'], conv=taps))
+    cfg = cases.make_config([kind, kind])
+    w = test.weights_for(cfg, 5, dtype)
+    toks, rows = test.tokens_for(cfg, 24, 6), (5, 1, 1, 1, 3, 1, 1, 1, 2, 6, 1, 1)
+    got = []
+    for places in (None, (0, 9, 9, 9, 4, 5, 30, 31, 1, 2, 1, 8)):
+        e = test.session_for(cfg, w, dtype, max_sequences=2).engine
+        out, at = [], 0
+        for k, n in enumerate(rows):
+            out.append(e.step(toks[at:at + n], [n], [places[k] if places else at], [1], [[0]], list(range(n)))[0])
+            at += n
+        got.append(np.concatenate(out))
+    np.testing.assert_array_equal(*got)

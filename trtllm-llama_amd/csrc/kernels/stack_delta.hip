@@ -338,7 +338,7 @@ __global__ __launch_bounds__(1024) void delta_step_kernel(const StackDeltaParams
     {
         // q, k and v lie one behind the other
         constexpr int ES = DT == DT_BF16 ? 2 : 4;
-        conv_step<DT>(reinterpret_cast<const char*>(p.x_raw) + row * p.ld_raw * ES, p.conv_state + (int64_t) p.ent_slot[e] * p.taps * CH, p.conv_w, nullptr, CH, p.ent_pos0[e],
+        conv_step<DT>(reinterpret_cast<const char*>(p.x_raw) + row * p.ld_raw * ES, p.conv_state + (int64_t) p.ent_slot[e] * p.taps * CH, p.conv_w, nullptr, CH, p.ent_fed[e],
             2 * D + V, qs, [&](int i) { return i < D ? hk * D + i : i < 2 * D ? QK + hk * D + i - D : 2 * QK + h * V + i - 2 * D; },
             [&](int i) { return i >= 2 * D || h % (p.heads / p.qk_heads) == 0; });
     }
@@ -527,7 +527,7 @@ bool stack_delta_convolves(const StackDeltaParams& p)
 int launch_stack_delta(const StackDeltaParams& p, hipStream_t stream)
 {
     const bool convolve = p.x_raw != nullptr;
-    if (convolve && (!stack_delta_convolves(p) || !p.conv_w || !p.conv_state))
+    if (convolve && (!stack_delta_convolves(p) || !p.conv_w || !p.conv_state || !p.ent_fed))
     {
         set_error("stack_delta: the convolution of %d taps goes with steps of one row of 4, its weights and its state", p.taps);
         return -1;

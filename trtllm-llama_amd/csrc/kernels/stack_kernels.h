@@ -397,7 +397,7 @@ bool stack_hgrn2_serves(int32_t dim, int32_t vdim); // shapes one of its two for
 // Selective state-space layer (Mamba-2): proj [tokens, ldp] = [z: inner | x: inner | B: groups * state | C: groups * state |
 // dt: heads], inner = heads * vdim.  x, B, C pass a causal convolution over `taps` tokens per channel (conv_w [channels, taps], the
 // last column meets the current token; bias) and silu: launch_stack_ssm_conv writes them to xbc [tokens, channels] and the
-// sequence's last taps - 1 raw inputs into conv_state [slots, taps, channels], position q's in row q mod taps; where stack_ssm_convolves, the scan does
+// sequence's last taps - 1 raw inputs into conv_state [slots, taps, channels], its row q's in row q mod taps; where stack_ssm_convolves, the scan does
 // both itself (convolve) and xbc stays as it is.  launch_stack_ssm_scan: per head h (reading group
 // h / (heads / groups)), with dt = softplus(dt + dt_bias[h]):
 //   S <- exp(-exp(a_log[h]) dt) S + dt B x^T   (S [state, vdim], fp32, one per slot),   y = S^T C + d_skip[h] x,
@@ -431,6 +431,7 @@ struct StackSsmParams
     const int32_t* ent_first = nullptr;
     const int32_t* ent_count = nullptr;
     const int32_t* ent_pos0 = nullptr;
+    const int32_t* ent_fed = nullptr; // convolution: rows that the sequence has had (0 where pos0 is)
     int32_t max_count = 0;          // host: the largest ent_count of the step
     float* chunk_ws = nullptr;      // optional scratch of the chunked form, as above
     size_t chunk_floats = 0;
@@ -536,6 +537,7 @@ struct StackDeltaParams
     const float* conv_w = nullptr;
     float* conv_state = nullptr;
     int32_t taps = 0;
+    const int32_t* ent_fed = nullptr;
 };
 bool stack_delta_convolves(const StackDeltaParams& p); // a step of one row per entry, 4 taps
 // both, in one launch for a step of single rows

@@ -60,13 +60,13 @@ template <int DT>
 __device__ __forceinline__ void conv_edges(const StackSsmParams& p, int e, int c, int CH, int64_t col, const float* w, float bias)
 {
     const int K = p.taps;
-    const int first = p.ent_first[e], count = p.ent_count[e], pos0 = p.ent_pos0[e];
-    float* ring = p.conv_state + (int64_t) p.ent_slot[e] * K * CH + c; // position q's in row q mod K
+    const int first = p.ent_first[e], count = p.ent_count[e], fed = p.ent_fed[e];
+    float* ring = p.conv_state + (int64_t) p.ent_slot[e] * K * CH + c; // the sequence's row q in row q mod K
     float old[MAX_TAPS - 1];
 #pragma unroll
     for (int j = 0; j < MAX_TAPS - 1; ++j)
     {
-        const int q = pos0 - (K - 1) + j;
+        const int q = fed - (K - 1) + j;
         old[j] = (j < K - 1 && q >= 0) ? ring[(int64_t) (q % K) * CH] : 0.f;
     }
     // input at index i of the entry (negative: the tail; old[K - 1 + i])
@@ -88,7 +88,7 @@ __device__ __forceinline__ void conv_edges(const StackSsmParams& p, int e, int c
         st_el<DT>(p.xbc, (int64_t) (first + i) * CH + c, silu_f(acc));
     }
     for (int i = count - head; i < count; ++i)
-        ring[(int64_t) ((pos0 + i) % K) * CH] = input(i);
+        ring[(int64_t) ((fed + i) % K) * CH] = input(i);
 }
 
 // Workgroups [0, tokens): row t, 256 channels each (blockIdx.y): rows that lie at least taps - 1 tokens into their entry read
@@ -502,7 +502,7 @@ __global__ __launch_bounds__(1024) void ssm_step_kernel(const StackSsmParams p)
     if constexpr (CONV)
     {
         const int g = h / (H / G);
-        conv_step<DT>(prj + inner, p.conv_state + (int64_t) p.ent_slot[e] * p.taps * CH, p.conv_w, p.conv_b, CH, p.ent_pos0[e], PH + 2 * N, conv,
+        conv_step<DT>(prj + inner, p.conv_state + (int64_t) p.ent_slot[e] * p.taps * CH, p.conv_w, p.conv_b, CH, p.ent_fed[e], PH + 2 * N, conv,
             [&](int i) { return i < PH ? h * PH + i : inner + g * N + (i - PH < N ? i - PH : GN + i - PH - N); }, [&](int i) { return i < PH || h % (H / G) == 0; });
     }
     else
@@ -633,7 +633,7 @@ int launch_stack_ssm_conv(const StackSsmParams& p, hipStream_t stream)
     if (p.conv_channels > 0)
     {
         // the convolution alone, over a range of columns of another layer kind's projection
-        if ((p.dtype != DT_BF16 && p.dtype != DT_FLOAT) || p.taps < 1 || p.taps > MAX_TAPS || p.conv_col < 0 || !p.conv_w || !p.conv_state || !p.xbc)
+        if ((p.dtype != DT_BF16 && p.dtype != DT_FLOAT) || p.taps < 1 || p.taps > MAX_TAPS || p.conv_col < 0 || !p.conv_w || !p.conv_state || !p.xbc || !p.ent_fed)
         {
             set_error("stack_ssm_conv: %d channels, %d taps (1 .. %d), or a missing operand", p.conv_channels, p.taps, MAX_TAPS);
             return -1;
@@ -674,9 +674,9 @@ int launch_stack_ssm_scan(const StackSsmParams& p, hipStream_t stream)
         return 0;
     if (!ssm_ok(p, "stack_ssm_scan"))
         return -1;
-    if (p.convolve && !stack_ssm_convolves(p))
+    if (p.convolve && (!stack_ssm_convolves(p) || !p.ent_fed))
     {
-        set_error("stack_ssm_scan: the convolution of %d taps goes with steps of one row of 4", p.taps);
+        set_error("stack_ssm_scan: the convolution of %d taps goes with steps of one row of 4, and where their rings stand", p.taps);
         return -1;
     }
     {

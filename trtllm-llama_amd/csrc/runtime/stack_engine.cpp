@@ -136,7 +136,7 @@ struct Run
     bool enters_pass = false;
     void *k_pool = nullptr, *v_pool = nullptr; // attention
     float* state = nullptr;                    // hgrn2, mamba2
-    float* conv_state = nullptr;               // mamba2, delta_rule: the last inputs of the convolution, in a ring of taps rows
+    float* conv_state = nullptr;               // mamba2, delta_rule: the last inputs of the convolution, in a ring of taps rows (fed)
     float* shift_carry = nullptr;              // token shift: the sequence's last normed row, [slots, width]
 };
 
@@ -224,6 +224,7 @@ struct tllm_stack
     int pair_buckets = 0, pair_mul_prev = 0, pair_mul_cur = 0, token_shift = 0;
     void* pair_table = nullptr;
     std::vector<int32_t> last_tok;
+    std::vector<int32_t> fed; // rows that every slot's sequence has had: where its convolutions' rings of raw inputs stand, whatever positions the caller counts
     float *h32 = nullptr, *dl_a = nullptr, *dl_g = nullptr;
     void* pairs = nullptr; // talking heads: every query head's weights over every value head's rows, [tokens, heads * kv_heads * vdim]
     int max_hd = 0, max_pairs = 0, max_sh = 0;
@@ -615,6 +616,7 @@ tllm_stack_t tllm_stack_create(const char* config_text)
     if (s->pair_buckets < 0 || (s->token_shift && !s->hyper) || (s->pair_buckets && s->plain))
         return fail("pair_buckets >= 0, not with residual=plain; the token shift is built for block=sequential");
     s->last_tok.assign((size_t) s->slots, -1);
+    s->fed.assign((size_t) s->slots, 0);
     if (s->loop_times < 1 || s->loop_start < 0 || s->loop_stop < s->loop_start || s->loop_stop > L)
         return fail("the loop must satisfy 0 <= loop_start <= loop_stop <= num_layers, loop_times >= 1");
     s->layers.resize(L);
@@ -1459,13 +1461,13 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         s->open = false;
     }
     // ---- metadata: one packed int32 image, one copy
-    const size_t n_ints = (size_t) 4 * T + (size_t) 4 * E + (size_t) E * MB + NW;
+    const size_t n_ints = (size_t) 4 * T + (size_t) 5 * E + (size_t) E * MB + NW;
     if (ensure_scratch(s, T, std::max(NW, 1), (int) (n_ints + 3) / 4 * 4))
         return -1;
     const bool deliver = (logits_out || next_ids_out) && ensure_landing(s, NW);
     int32_t* h = s->pinned;
     int32_t *h_tok = h, *h_tent = h + T, *h_tpos = h + 2 * T, *h_first = h + 3 * T, *h_count = h_first + E, *h_pos0 = h_count + E,
-            *h_slot = h_pos0 + E, *h_table = h_slot + E, *h_want = h_table + (size_t) E * MB, *h_prev = h_want + NW;
+            *h_slot = h_pos0 + E, *h_fed = h_slot + E, *h_table = h_fed + E, *h_want = h_table + (size_t) E * MB, *h_prev = h_want + NW;
     std::memcpy(h_tok, b->tokens, (size_t) T * 4);
     int row = 0;
     for (int e = 0; e < E; ++e)
@@ -1474,6 +1476,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         h_count[e] = b->ent_count[e];
         h_pos0[e] = b->ent_pos0[e];
         h_slot[e] = b->ent_slot[e];
+        h_fed[e] = b->ent_pos0[e] > 0 ? s->fed[(size_t) b->ent_slot[e]] : 0;
         for (int i = 0; i < b->ent_count[e]; ++i, ++row)
         {
             h_tent[row] = e;
@@ -1490,7 +1493,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         h_want[i] = b->want_rows[i];
     const int32_t* d = s->ints;
     const int32_t *d_tok = d, *d_tent = d + T, *d_tpos = d + 2 * T, *d_first = d + 3 * T, *d_count = d_first + E, *d_pos0 = d_count + E,
-                  *d_slot = d_pos0 + E, *d_table = d_slot + E, *d_want = d_table + (size_t) E * MB, *d_prev = d_want + NW;
+                  *d_slot = d_pos0 + E, *d_fed = d_slot + E, *d_table = d_fed + E, *d_want = d_table + (size_t) E * MB, *d_prev = d_want + NW;
 
     const int Wd = s->width;
     const bool looped = s->loop_stop > s->loop_start;
@@ -1588,6 +1591,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             sp.ent_first = d_first;
             sp.ent_count = d_count;
             sp.ent_pos0 = d_pos0;
+            sp.ent_fed = d_fed;
             StackDeltaParams dp;
             dp.max_count = max_count;
             dp.dim = l.dim;
@@ -1651,6 +1655,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             dp.ent_first = d_first;
             dp.ent_count = d_count;
             dp.ent_pos0 = d_pos0;
+            dp.ent_fed = d_fed;
             dp.chunk_ws = s->chunk_ws;
             dp.chunk_floats = s->chunk_floats;
             return launch_stack_delta(dp, stream);
@@ -1683,6 +1688,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             sp.ent_first = d_first;
             sp.ent_count = d_count;
             sp.ent_pos0 = d_pos0;
+            sp.ent_fed = d_fed;
             sp.max_count = max_count;
             sp.chunk_ws = s->chunk_ws;
             sp.chunk_floats = s->chunk_floats;
@@ -2515,6 +2521,12 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         const int parts = stack_choice_parts(s->vocab);
         for (int i = 0; i < NW; ++i)
             next_ids_out[i] = stack_choose(s->land_choice + (size_t) i * parts, parts);
+    }
+    for (int e = 0; e < E; ++e)
+    {
+        constexpr int FAR = 1 << 30, TURNS = FAR / 720720 * 720720; // (whole turns of a ring of up to 16 rows)
+        const int rows = h_fed[e] + b->ent_count[e];
+        s->fed[(size_t) b->ent_slot[e]] = rows < FAR ? rows : rows - TURNS;
     }
     return 0;
 }
