@@ -67,3 +67,20 @@ def test_another_stream_from_step_to_step():
         rows.append(s.step([('a', [t], [0])])[0])
         at.append(t)
     G.check(np.concatenate(rows), O.logits(toks, G.as_f64(w), cfg), G.F32_TOL)
+
+
+def test_streams_in_turn_give_the_same_bits():
+    """Steps that write and read states, caches and scratch of some size, on three streams in turn and on one."""
+    cfg = F.make_config([F.mamba_layer(heads=16, vdim=64, state=64, groups=2, norm_groups=2, mlp=F.dense(ff=2048)), F.latent_layer(heads=8, dim=64, vdim=64, kv_rank=128, size=0)] * 2, width=1024, vocab=8192)
+    w = F.random_weights(cfg, 3)
+    toks, rows = G.tokens_for(cfg, 400, 6), ([1] * 9 + [31]) * 10
+    streams, got = [torch.cuda.Stream() for _ in range(3)], []
+    for many in (True, False):
+        s = G.session_for(cfg, w, 'bfloat16')
+        step, out, at = s.engine.step, [], 0
+        for k, n in enumerate(rows):
+            s.engine.step = lambda *a, **kw: step(*a, **dict(kw, stream=streams[k % 3 if many else 0].cuda_stream))
+            out.append(s.step([('a', toks[at:at + n], [n - 1])])[0])
+            at += n
+        got.append(np.concatenate(out))
+    np.testing.assert_array_equal(*got)

@@ -136,6 +136,19 @@ def pinned_rows(stub):
     assert stub.pinned_bytes() <= (8 << 20) + 65 * 64 * 8 + (64 << 10)
 
 
+def streams_in_turn(stub):
+    """A step behind one that returned with its rows, on another stream, waits for nothing else on the device."""
+    import rofozen_cases as M
+    s = engine(M.make_config([M.mamba_layer(heads=2, vdim=8, state=16, groups=1)]), M, max_tokens=64, max_sequences=1)
+    take = s.engine.step
+    s.step([('a', [1], [0])])  # (makes its scratch)
+    syncs = stub.device_syncs()
+    for stream in (0, 64, 64, 128, 0):
+        s.engine.step = lambda *a, **k: take(*a, **dict(k, stream=stream))
+        s.step([('a', [1], [0])])
+    assert stub.device_syncs() == syncs
+
+
 def rows_to_the_edge(stub):
     """The caller's rows begin and end at the edge of what may be written, whatever their size; a step of that many rows stays within them."""
     import mmap
@@ -430,6 +443,9 @@ else:
 
     def test_pinned_rows(stub):
         run(stub, 'pinned_rows')
+
+    def test_steps_on_streams_in_turn(stub):
+        run(stub, 'streams_in_turn')
 
     def test_rows_that_end_where_memory_does(stub):
         run(stub, 'rows_to_the_edge')

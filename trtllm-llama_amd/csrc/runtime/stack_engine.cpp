@@ -141,9 +141,12 @@ struct Run
 };
 
 // Rows go on to the caller as they land in pinned memory, while those behind them are still on their way, and without the runtime's wait for the end of the stream: a marker
-// behind the last launch, the wait for it and its wake-up took 12 - 30 us a step (a step of one row of 32000: 329 us with it, 317; eight rows 567, 545).  Whoever
-// needs the stream's end (taps, another stream, errors of the launches) waits for it as before.  -> how many of the rows: the wait ends after SPIN, a core's time, behind
-// which the runtime's own counts for little.
+// behind the last launch, the wait for it and its wake-up took 12 - 30 us a step (a step of one row of 32000: 329 us with it, 317; eight rows 567, 545).  -> how many of the
+// rows: the wait ends after SPIN, a core's time, behind which the runtime's own counts for little.
+//
+// What may follow, on whichever stream: a part's choice is stored behind a release at system scope, by the last launch of its step, so that all which that stream ran
+// before comes ahead of the host's acquire here, and of what the host launches from then on.  Left of the step is the end of a launch that has read and written all it will.
+// (So no event behind every step, a marker in the streams of all for the few who change theirs.)
 int copy_as_they_land(float* to, const float* landing, const StackChoice* choice, int rows, int vocab)
 {
     constexpr auto SPIN = std::chrono::milliseconds(2);
@@ -213,8 +216,6 @@ struct tllm_stack
     // pinned host memory that a few wanted rows are delivered to: the parts' choices, then the logits
     StackChoice* land_choice = nullptr;
     float* land_rows = nullptr;
-    bool open = false;               // the last step returned with its rows, without waiting for its stream
-    hipStream_t open_stream = nullptr;
     int land_cap = 0; // rows
     void *xbc = nullptr, *cq = nullptr, *qfull = nullptr, *moe_a = nullptr;
     float *moe_y = nullptr, *moe_w = nullptr;
@@ -1455,11 +1456,6 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             set_error("tllm_stack_step: wanted row %d is outside the batch of %d", b->want_rows[i], T);
             return -1;
         }
-    if (s->open && s->open_stream != stream)
-    {
-        HIP_OK(hipDeviceSynchronize()); // (the step before ended with its rows, on another stream, which need not be there any more)
-        s->open = false;
-    }
     // ---- metadata: one packed int32 image, one copy
     const size_t n_ints = (size_t) 4 * T + (size_t) 5 * E + (size_t) E * MB + NW;
     if (ensure_scratch(s, T, std::max(NW, 1), (int) (n_ints + 3) / 4 * 4))
@@ -2509,10 +2505,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
     if (deliver && logits_out)
         bring_in(logits_out, (size_t) NW * s->vocab * 4);
     const int there = deliver ? copy_as_they_land(logits_out, s->land_rows, s->land_choice, NW, s->vocab) : 0; // rows
-    // (behind the rows nothing but the end of their launch is left)
-    s->open = deliver && there == NW && !s->taps;
-    s->open_stream = stream;
-    if (!s->open)
+    if (!deliver || there < NW || s->taps)
         HIP_OK(hipStreamSynchronize(stream));
     if (deliver && logits_out && there < NW)
         std::memcpy(logits_out + (size_t) there * s->vocab, s->land_rows + (size_t) there * s->vocab, (size_t) (NW - there) * s->vocab * 4);
