@@ -22,7 +22,7 @@ std::map<void*, size_t> g_device, g_pinned;
 std::map<const void*, std::string> g_names;
 std::string g_launched;
 size_t g_live = 0, g_budget = ~size_t(0), g_largest = 0;
-int g_host_mallocs = 0, g_syncs = 0;
+int g_host_mallocs = 0, g_syncs = 0, g_stream_syncs = 0;
 hipError_t g_last = hipSuccess;
 
 hipError_t done(hipError_t e)
@@ -59,6 +59,7 @@ int stub_has_allocation(size_t bytes)
 }
 int stub_host_mallocs() { return g_host_mallocs; }
 int stub_device_syncs() { return g_syncs; }
+int stub_stream_syncs() { return g_stream_syncs; }
 size_t stub_pinned_bytes()
 {
     size_t n = 0;
@@ -91,7 +92,7 @@ hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return s
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { return std::memmove(d, s, n), hipSuccess; }
 hipError_t hipMemset(void*, int, size_t) { return hipSuccess; }
 hipError_t hipDeviceSynchronize() { return ++g_syncs, hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return ++g_stream_syncs, hipSuccess; }
 hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }

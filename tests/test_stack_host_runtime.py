@@ -149,6 +149,23 @@ def streams_in_turn(stub):
     assert stub.device_syncs() == syncs
 
 
+def who_waits(stub):
+    """The host watches for a step's rows unless the step's products alone take longer than it would: of 2 ms at 1.31 PFLOP/s in bfloat16, 0.15 in fp32."""
+    import ruzinex_cases as Z
+
+    class Zeros:  # (nothing is computed)
+        standard_normal = staticmethod(lambda shape: np.zeros(shape, np.float32))
+    np.random.default_rng = lambda seed: Zeros
+    for dtype, rate in (('bfloat16', 1.31e15), ('float32', 0.15e15)):
+        width, ff, d = 1024, 6144, 32
+        s = engine(Z.make_config([Z.layer(heads=2, kv_heads=1, dim=d, vdim=d, mlp=Z.dense(ff=ff))], width=width, vocab=64), Z, dtype=dtype, max_tokens=140000, max_batch_tokens=140000, max_sequences=1)
+        edge = 2e-3 * rate / (2 * width * (3 * ff + 6 * d))
+        for tokens, watches in ((1, True), (int(0.98 * edge), True), (int(1.02 * edge), False)):
+            before = stub.stream_syncs()
+            step(s, 'a', tokens)
+            assert stub.stream_syncs() - before == (0 if watches else 1), (dtype, tokens)
+
+
 def rows_to_the_edge(stub):
     """The caller's rows begin and end at the edge of what may be written, whatever their size; a step of that many rows stays within them."""
     import mmap
@@ -446,6 +463,9 @@ else:
 
     def test_steps_on_streams_in_turn(stub):
         run(stub, 'streams_in_turn')
+
+    def test_who_waits_for_a_steps_rows(stub):
+        run(stub, 'who_waits')
 
     def test_rows_that_end_where_memory_does(stub):
         run(stub, 'rows_to_the_edge')
