@@ -40,7 +40,8 @@
  * Element type bfloat16: weights, activations and caches in bfloat16, fp32 accumulation, and fp32 for the residual stream, norms,
  * scores and softmax, rotation angles, gates of a recurrence and its state.  float32: everything in fp32 with plain FMAs.
  *
- * Errors: NULL / non-zero + tllm_last_error().  Nothing synchronises except tllm_stack_step (it returns host results).
+ * Errors: NULL / non-zero + tllm_last_error().  Nothing waits for the device but tllm_stack_step, which returns host results, calls that make a step's scratch larger, and
+ * tllm_stack_get_tap.
  */
 #ifndef TLLM_STACK_API_H
 #define TLLM_STACK_API_H
@@ -122,7 +123,11 @@ typedef struct
 /* Runs one step.  logits_out: host fp32 [n_want, vocab] or NULL; next_ids_out: host int32 [n_want] (arg-max of each wanted row, the
  * greedy sampler) or NULL.  Every index is checked on the host before anything is launched.  The kernels of a step, and with them the
  * order of a row's fp32 sums, follow the step's sizes: the same step gives the same bits, a request in other company (other tokens, or
- * portions cut elsewhere) the same values to the element type's rounding. */
+ * portions cut elsewhere) the same values to the element type's rounding.
+ * On return the results are complete and so is all that the step does to caches and states, on whatever stream the next step comes; its
+ * last launch, which brought the results, may still be about to end, so that `stream` need not be idle.  The call waits for nothing but its own work: it watches
+ * up to 8 MiB of rows arrive, with a core, for at most 2 ms, and waits for `stream` beyond that, with more rows, none or taps, and where the step's products alone
+ * take longer.  An error of the device is this call's: results that do not arrive are waited for with `stream`. */
 int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* batch, float* logits_out, int32_t* next_ids_out, void* stream);
 
 /* Geometry the cache manager needs. */
