@@ -325,6 +325,27 @@ def convolution_of_single_rows(stub):
                 assert any(re.search(r'(ssm|delta)_step_kernelILi7ELb1', k) for k in kernels) == (rows == 1 and taps == 4), (name, taps, rows)
 
 
+def low_rank_pairs(stub):
+    """A delta layer's two low-rank pairs are one product of two where one launch serves it; rows of tiles that end inside a stage of 64 go one by one, not by the
+    register-staged tiles."""
+    import narurax_cases as N
+    from tensorrt_llm.runtime import RaggedGenerationSession
+    for rank in (8, 40, 64, 72, 96, 128):
+        cfg = N.make_config([N.delta_layer(heads=2, kv_heads=1, dim=96, vdim=96)], width=256)
+        s = RaggedGenerationSession(N.as_model(cfg, N.random_weights(cfg, 1, ranks=(rank, rank))), dtype='bfloat16', max_tokens=256, max_sequences=1)
+        for rows in (1, 8, 31, 32, 40):
+            stub.forget()
+            step(s, 'a', rows)
+            kernels = stub.kernels()
+            first = next(i for i, k in enumerate(kernels) if 'token_shift' in k or re.search(r'hyper_norm_vec_kernelILi7ELi1ELi1ELb1', k)) + 1  # the mixer's first product
+            last = next(i for i, k in enumerate(kernels) if re.search(r'delta_(scan|step)', k))
+            found = [k for k in kernels[first + 1:last] if 'conv' not in k]
+            if rows < 32 or rank % 64 == 0:
+                assert len(found) == 1, (rank, rows, found)
+            elif rank > 64:
+                assert [bool(re.search('gemm_glds', k)) for k in found] == [True, False] * 2 and all('fma_tile' in k for k in found[1::2]), (rank, rows, found)
+
+
 def norms_without_a_sum(stub):
     """A norm of any number of streams carries the code of the experts' sum only where there is one to form."""
     import narurax_cases as N
@@ -499,6 +520,9 @@ else:
 
     def test_convolution_of_single_rows(stub):
         run(stub, 'convolution_of_single_rows')
+
+    def test_low_rank_pairs(stub):
+        run(stub, 'low_rank_pairs')
 
     def test_sizes_of_the_row_tile_tests(stub):
         run(stub, 'row_tiles')

@@ -122,7 +122,7 @@ struct Layer
           *d_skip = nullptr, *router_w = nullptr, *correction = nullptr, *talkw = nullptr, *q_norm = nullptr, *k_norm = nullptr, *o_biasv = nullptr,
           *shift = nullptr;
     void *w_a2 = nullptr, *w_g2 = nullptr; // delta_rule: the second halves of the decay's and the gate's low-rank projections
-    bool low_pair = false;                 // ... of one shape: both in w_a2, one product of two
+    bool low_pair = false;                 // ... of one shape: both in w_a2, one product of two where one launch serves it
     void* w_uq = nullptr;
     void *w_shared_up = nullptr, *w_shared_down = nullptr; // shared expert (where it is not part of w_mix / w_o)
     void *side_gate = nullptr, *side_proj = nullptr;       // per-layer token input
@@ -1621,9 +1621,12 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             lr.w = l.w_a2;
             lr.c = s->dl_a;
             lr.ldc = lr.N;
-            if (l.low_pair)
+            // (a launch instead of two, us: one row, 1024 x 128 3.3 + 3.6, 3.6; 1672 rows 7.7 + 7.7, 13.  Tiles take a pair in one launch where a row is whole stages of 64; rows
+            // that end inside one go one by one, by whole stages and a rest, as a pair would
+            // not: rank 96, 4 layers of width 1536, 300 rows 690 as pairs and 550 one by one, 2000 rows 1580 and 1470)
+            const bool pair = l.low_pair && (T < 32 || l.decay_rank % 64 == 0);
+            if (pair)
             {
-                // (a launch instead of two, us: one row, 1024 x 128 3.3 + 3.6, 3.6; 1672 rows 7.7 + 7.7, 13)
                 lr.batch = 2;
                 lr.stride_a = l.decay_rank;
                 lr.stride_w = (int64_t) lr.N * lr.K;
@@ -1634,10 +1637,10 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
             lr.N = l.n_ctx;
             lr.K = l.gate_rank;
             lr.a = (const char*) s->proj + (size_t) col_g * s->es;
-            lr.w = l.w_g2;
+            lr.w = l.low_pair ? (const char*) l.w_a2 + (size_t) l.n_ctx * l.gate_rank * s->es : l.w_g2;
             lr.c = s->dl_g;
             lr.ldc = lr.N;
-            if (!l.low_pair && launch_stack_gemm(lr, stream))
+            if (!pair && launch_stack_gemm(lr, stream))
                 return -1;
             dp.dtype = s->dtype;
             dp.tokens = T;
