@@ -1,5 +1,5 @@
-// A HIP runtime for tests of the stack engine's host side on a machine without a GPU: loaded ahead of libtllm_stack_engine.so, it takes the
-// place of the 20 runtime calls that the library makes.  Device memory is host memory within a budget, launches are recorded and compute
+// A HIP runtime for tests of the engines' host side on a machine without a GPU: loaded ahead of libtllm_stack_engine.so, it takes the
+// place of the 20 runtime calls that the library makes, and ahead of libnvinfer_plugin_tensorrt_llm.so of those of a LLaMA session's set-up and context phase.  Device memory is host memory within a budget, launches are recorded and compute
 // nothing, but that wanted rows land: all of them zeros.  Launch limits are the runtime's documented ones: fewer than 2^32 threads per grid dimension, 65535 workgroups in y and z.
 #include <hip/hip_runtime_api.h>
 #include <cstdint>
@@ -91,6 +91,12 @@ hipError_t hipHostFree(void* p) { return release(g_pinned, p); }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { return std::memmove(d, s, n), hipSuccess; }
 hipError_t hipMemset(void*, int, size_t) { return hipSuccess; }
+hipError_t hipMemsetAsync(void*, int, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return *e = reinterpret_cast<hipEvent_t>(new int(0)), hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { return delete reinterpret_cast<int*>(e), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.f, hipSuccess; } // (all kernels are as quick)
 hipError_t hipDeviceSynchronize() { return ++g_syncs, hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return ++g_stream_syncs, hipSuccess; }
 hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }

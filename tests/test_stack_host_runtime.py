@@ -325,6 +325,28 @@ def convolution_of_single_rows(stub):
                 assert any(re.search(r'(ssm|delta)_step_kernelILi7ELb1', k) for k in kernels) == (rows == 1 and taps == 4), (name, taps, rows)
 
 
+def packed_prompts(stub):
+    """Batches of test_gpu_ragged_prompts.py that leave their padding rows out, and such that do not; products of either have a kernel that was chosen by measuring."""
+    import test_gpu_ragged_prompts as G
+    from tensorrt_llm.plugin import capi
+    lib = capi.load_library()
+    lib.tllm_gemm_tactic_lookup.restype = ctypes.c_int32
+    for mode, wtype in (('fp16', 0), ('sq_static_pc', 3)):
+        _, session = G.sessions(mode, 1)
+        s = session(4, G.S)
+        for lens in G.BATCHES:
+            stub.forget()
+            s.context(np.zeros((4, G.S), np.int32), np.array(lens, np.int32))
+            assert any('gather_rows' in k for k in stub.kernels()) == (sum(lens) <= 1232), (mode, lens)
+        s.close()
+        lib.tllm_gemm_tactics_clear()
+        for prompt, packed in ((330, 1000), (G.S, 1024), (G.S, 1232)):
+            s = session(4, prompt)
+            assert lib.tllm_gemm_tactic_lookup(wtype, 4 * prompt, 6144, 2048) > 0 and lib.tllm_gemm_tactic_lookup(wtype, packed, 6144, 2048) > 0, (mode, prompt, packed)
+            s.close()
+            lib.tllm_gemm_tactics_clear()
+
+
 def low_rank_pairs(stub):
     """A delta layer's two low-rank pairs are one product of two where one launch serves it; rows of tiles that end inside a stage of 64 go one by one, not by the
     register-staged tiles."""
@@ -520,6 +542,9 @@ else:
 
     def test_convolution_of_single_rows(stub):
         run(stub, 'convolution_of_single_rows')
+
+    def test_packed_prompts(stub):
+        run(stub, 'packed_prompts')
 
     def test_low_rank_pairs(stub):
         run(stub, 'low_rank_pairs')
