@@ -11,6 +11,7 @@ from tensorrt_llm.plugin import capi
 
 pytestmark = pytest.mark.gpu
 WIDE = 80
+MLP = (3900, 11000, 4096)                                       # rows, columns, K of the two products
 
 
 class GemmParams(ctypes.Structure):
@@ -85,21 +86,42 @@ def test_scales_of_a_whole_matrix(wide, per_channel, per_token):
     product(wide, 300, 520, 3, True, per_channel, per_token)
 
 
+def fused(lib, m, n, k, a, w1, w2, s1, s2, sr, qs):
+    out = torch.full((m, n), 77, dtype=torch.int8, device='cuda')
+    q = GemmParams(3, 2, m, n, k, a.data_ptr(), k, w1.data_ptr(), k, s1.data_ptr(), sr.data_ptr(), 1, 0, out.data_ptr(), n)
+    assert lib.tllm_gemm_swiglu_quant(ctypes.byref(q), w2.data_ptr(), s2.data_ptr(), qs.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0, capi.last_error()
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize('k_tiles', [1, 2, 3, 4, 5, 6, 7, 13])
+@pytest.mark.parametrize('m', [33, 128, 129, 300, 640])
+def test_two_products_of_an_mlp(wide, m, k_tiles):
+    """Against products of whole numbers, rounded to fp16 where two launches and the static quantiser round.  The kernel's exponential is another: a value of 11 bits may round the
+    other way, 2^-11 of up to 127 quantised, which moves a byte by one where it lies that close to a half: 0.06 on either side at the largest, 1 byte in 100 if all of
+    the 11 bits of one value in ten turn over."""
+    torch.manual_seed(m + k_tiles)
+    n, k = 520, 128 * k_tiles
+    a, w1, w2 = int8(m, k), int8(n, k), int8(n, k)
+    s1, s2 = (torch.randint(1, 13, (n,), device='cuda').float() * 2e-5 / k_tiles ** 0.5 for _ in range(2))
+    sr, qs = torch.tensor([0.75], device='cuda'), torch.tensor([23.0], device='cuda')
+    g, u = (((a.double() @ w.double().t()).float() * (s * sr)).half().float() for w, s in ((w1, s1), (w2, s2)))
+    want = ((g / (1 + torch.exp(-g))).half().float() * u).half().float().mul(qs).round().clamp(-128, 127)
+    d = (fused(wide, m, n, k, a, w1, w2, s1, s2, sr, qs).float() - want).abs()
+    assert d.max() <= 1 and (d > 0).float().mean() < 1e-2 and want.unique().numel() > 100 and (want.abs() < 127).float().mean() > 0.5
+
+
 def test_fused_int8_mlp(wide):
-    """Rows, columns and K for which the rule takes these tiles: the same bytes as by the one-tile-per-workgroup form."""
+    """Rows, columns and K for which the rule takes these tiles (test_stack_host_runtime.py): the same bytes as by the one-tile-per-workgroup form."""
     torch.manual_seed(5)
-    m, n, k = 3900, 11000, 4096
+    m, n, k = MLP
     a, w1, w2 = int8(m, k), int8(n, k), int8(n, k)
     s1, s2 = (torch.randint(1, 13, (n,), device='cuda').float() * 2e-6 for _ in range(2))
     sr, qs = torch.tensor([0.75], device='cuda'), torch.tensor([23.0], device='cuda')
     got = []
     for cfg in (0, -2):
         wide.tllm_gemm_set_tile_cfg(cfg)
-        out = torch.full((m, n), 77, dtype=torch.int8, device='cuda')
-        q = GemmParams(3, 2, m, n, k, a.data_ptr(), k, w1.data_ptr(), k, s1.data_ptr(), sr.data_ptr(), 1, 0, out.data_ptr(), n)
-        assert wide.tllm_gemm_swiglu_quant(ctypes.byref(q), w2.data_ptr(), s2.data_ptr(), qs.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0, capi.last_error()
-        torch.cuda.synchronize()
-        got.append(out)
+        got.append(fused(wide, m, n, k, a, w1, w2, s1, s2, sr, qs))
     assert torch.equal(*got) and got[0].unique().numel() > 100
 
 

@@ -347,6 +347,21 @@ def packed_prompts(stub):
             lib.tllm_gemm_tactics_clear()
 
 
+def two_int8_products(stub):
+    """The sizes of test_gpu_wide_half.py's MLP take the tiles of gemm_wide.hip by their cost, or by their id; the one-tile form and small ones do not."""
+    import test_gpu_wide_half as G
+    from tensorrt_llm.plugin import capi
+    lib = capi.load_library()
+    lib.tllm_gemm_swiglu_quant.argtypes = [ctypes.POINTER(G.GemmParams)] + [ctypes.c_void_p] * 4
+    for cfg, (m, n, k), wide in ((0, G.MLP, True), (-2, G.MLP, False), (0, (300, 520, 384), False), (G.WIDE, (300, 520, 384), True)):
+        lib.tllm_gemm_set_tile_cfg(0)
+        lib.tllm_gemm_set_tile_cfg(cfg)
+        stub.forget()
+        q = G.GemmParams(3, 2, m, n, k, 4096, k, 4096, k, 4096, 4096, 1, 0, 4096, n)
+        assert lib.tllm_gemm_swiglu_quant(ctypes.byref(q), 4096, 4096, 4096, None) == 0
+        assert [bool(re.search('wide_kernelILi3ELi6', x)) for x in stub.kernels()] == [wide], (cfg, m)
+
+
 def low_rank_pairs(stub):
     """A delta layer's two low-rank pairs are one product of two where one launch serves it; rows of tiles that end inside a stage of 64 go one by one, not by the
     register-staged tiles."""
@@ -545,6 +560,9 @@ else:
 
     def test_packed_prompts(stub):
         run(stub, 'packed_prompts')
+
+    def test_two_int8_products(stub):
+        run(stub, 'two_int8_products')
 
     def test_low_rank_pairs(stub):
         run(stub, 'low_rank_pairs')

@@ -1016,6 +1016,7 @@ int launch_sqp(const GemmParams& pin, hipStream_t stream)
 
 int launch_gemm_wide(const GemmParams& p, hipStream_t stream); // gemm_wide.hip
 bool gemm_wide_beats(const GemmParams& p, double other);
+extern int gemm_tune_cfg; // gemm_glds.hip
 
 // A/B hook (tllm_gemm_set_tile_cfg(-2) / (-3)): the fused SwiGLU GEMM in its one-tile-per-workgroup form
 bool gemm_swiglu_one_tile = false;
@@ -1152,12 +1153,13 @@ int launch_gemm_swiglu(const GemmParams& p, hipStream_t stream)
         return 1;
     if (!gemm_swiglu_one_tile)
     {
-        // 256 x 128 columns of both matrices by the tiles of gemm_wide.hip where that is quicker than 256 x 96 by the persistent form below (1.28 us a K-tile and round)
+        // 256 x 128 columns of both matrices by the tiles of gemm_wide.hip where that is quicker than 256 x 96 by the persistent form below (1.28 us a K-tile and round), or
+        // where those are asked for by their id
         const int cus = launch_util::device_cus();
         const int64_t tiles = (int64_t) ((p.M + 255) / 256) * ((p.N + 95) / 96);
         GemmParams q = p;
         q.out_dtype = DT_HALF;
-        if (gemm_wide_beats(q, (double) ((tiles + cus - 1) / cus) * (p.K / 128) * 0.723 + 3.0))
+        if (gemm_wide_beats(q, gemm_tune_cfg == 80 ? 1e30 : (double) ((tiles + cus - 1) / cus) * (p.K / 128) * 0.723 + 3.0))
             return launch_gemm_wide(q, stream);
     }
     // 256 rows x 96 columns of both matrices; int8 output on 16-byte rows: the persistent form (r05)
