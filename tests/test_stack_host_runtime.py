@@ -325,6 +325,58 @@ def convolution_of_single_rows(stub):
                 assert any(re.search(r'(ssm|delta)_step_kernelILi7ELb1', k) for k in kernels) == (rows == 1 and taps == 4), (name, taps, rows)
 
 
+def in_lone_steps(stub, pattern, cfg, cases, dtype='bfloat16', rows=1):
+    """-> matches of `pattern` among the kernels of a step of `rows` tokens behind a prompt."""
+    s = engine(cfg, cases, dtype, max_tokens=64, max_sequences=1)
+    s.step([('a', [1, 2, 3], [0])])
+    stub.forget()
+    s.step([('a', [1] * rows, [0])])
+    return [m for m in (re.search(pattern, k) for k in stub.kernels()) if m]
+
+
+def lone_norms(stub):
+    """A lone token's rows are normed by their readers at the sizes that test_gpu_lone_norm.py and test_gpu_lone_out_norm.py list for it, and not just outside."""
+    import rofozen_cases as F
+    import tolenex_cases as T
+
+    class Zeros:  # (nothing is computed)
+        standard_normal = staticmethod(lambda shape: np.zeros(shape, np.float32))
+        uniform = staticmethod(lambda lo, hi, size=None: np.full(size, lo, np.float32))
+    np.random.default_rng = lambda seed: Zeros
+    row_norm = r'row_norm_kernelILi\d+ELi\d+ELi\d+ELi(\d+)E'
+    mamba = dict(heads=2, vdim=12, state=16, groups=1, norm_groups=1)  # (rows of 24: their own norm has a launch)
+    for width in (16, 96, 104, 512, 528, 1024, 1040, 2048, 2064, 4096, 4112):
+        served = width % 16 == 0 and width <= 4096
+        cfg = F.make_config([F.mamba_layer(mlp=F.dense(ff=40), **mamba), F.latent_layer(mlp=F.moe(experts=4, identity=2, top=2, count=1, keep=1))], width=width)
+        assert [m[1] for m in in_lone_steps(stub, row_norm, cfg, F)] == ['0'] * 3 * served, width  # two mixers' first products and a feed-forward's
+        assert len(in_lone_steps(stub, 'moe_logits_norm_kernel', cfg, F)) == served, width
+        assert not in_lone_steps(stub, 'row_norm|logits_norm', cfg, F, 'float32') and not in_lone_steps(stub, 'row_norm|logits_norm', cfg, F, rows=2)
+    for width, parts, served in ((96, 1, 1), (96, 2, 1), (96, 4, 1), (96, 3, 0), (1040, 2, 1), (1040, 4, 1), (2048, 4, 1), (4096, 1, 1), (4096, 4, 1), (4112, 4, 0), (1024, 8, 0), (2048, 8, 1), (4096, 8, 1)):
+        cfg = T.make_config([T.attention_layer(heads=2, kv_heads=1, dim=16, vdim=16, rot_dims=8, ff=40)], width=width, groups=parts)
+        assert [m[1] for m in in_lone_steps(stub, row_norm, cfg, T)] == [str(parts)] * served, (width, parts)
+    for heads, vdim, parts, served in ((2, 8, 1, 1), (4, 16, 4, 1), (4, 18, 4, 0), (6, 16, 3, 0), (8, 64, 8, 0), (32, 64, 1, 1), (32, 64, 8, 1), (32, 96, 8, 0), (64, 64, 4, 1), (64, 64, 8, 1), (64, 66, 8, 0)):
+        cfg = F.make_config([F.mamba_layer(heads=heads, vdim=vdim, state=8, groups=1, norm_groups=parts)], width=100)  # (the layer's own rows are no whole pieces)
+        assert [m[1] for m in in_lone_steps(stub, row_norm, cfg, F)] == [str(parts)] * served, (heads, vdim, parts)
+
+
+def shifts_and_starts(stub):
+    """The token shift inside its norm's launch, and the start of a step in one, at the sizes of test_gpu_shift_step.py and test_gpu_step_start.py."""
+    import narurax_cases as N
+    delta = dict(heads=2, kv_heads=1, dim=8, vdim=8)
+    for width in (96, 98, 260, 4096, 4100, 8192, 8196):
+        cfg = N.make_config([N.delta_layer(**delta)] * 2, width=width)
+        for dtype in ('bfloat16', 'float32'):
+            together = width % 4 == 0 and width <= 8192
+            assert len(in_lone_steps(stub, r'hyper_norm_vec_kernelILi\d+ELi1ELi\d+ELb1', cfg, N, dtype)) == 2 * together, (width, dtype)
+            assert len(in_lone_steps(stub, 'token_shift_kernel', cfg, N, dtype)) == 2 * (not together), (width, dtype)
+            assert len(in_lone_steps(stub, 'token_shift_kernel', cfg, N, dtype, rows=2)) == 2
+    for width in (8, 96, 100, 2056):
+        cfg = N.make_config([N.delta_layer(**delta)], width=width)
+        for rows in (1, 16, 17):
+            one = width % 8 == 0 and rows <= 16
+            assert [len(in_lone_steps(stub, name, cfg, N, rows=rows)) for name in ('begin_kernel', 'fetch_kernel', 'embed')] == ([1, 0, 0] if one else [0, 1, 2]), (width, rows)
+
+
 def packed_prompts(stub):
     """Batches of test_gpu_ragged_prompts.py that leave their padding rows out, and such that do not; products of either have a kernel that was chosen by measuring."""
     import test_gpu_ragged_prompts as G
@@ -557,6 +609,12 @@ else:
 
     def test_convolution_of_single_rows(stub):
         run(stub, 'convolution_of_single_rows')
+
+    def test_lone_norms(stub):
+        run(stub, 'lone_norms')
+
+    def test_shifts_and_starts(stub):
+        run(stub, 'shifts_and_starts')
 
     def test_packed_prompts(stub):
         run(stub, 'packed_prompts')
