@@ -229,10 +229,10 @@ struct Tile
             {
                 if (i == NA - AHEAD)
                 {
-                    // K-tile t + 1 has landed: this wave's by the count (K-tile t + 2's stay under way; five of them are requested behind here), everyone's by the barrier
-                    constexpr int BEHIND = DMAS - (NA - AHEAD) - (NA - MID) > 0 ? DMAS - (NA - AHEAD) - (NA - MID) : 0;
+                    // K-tile t + 1 has landed: this wave's by the count (all of K-tile t + 2's have been requested and stay under way), everyone's by the barrier
+                    static_assert(DMAS <= (NA - MID) + (NA - AHEAD), "a K-tile's requests end in front of this wait");
                     if (more)
-                        wait_vm_and_meet<DMAS - BEHIND>();
+                        wait_vm_and_meet<DMAS>();
                     else
                         wait_vm_and_meet<0>();
                     __builtin_amdgcn_sched_barrier(0);
@@ -720,9 +720,11 @@ __global__ __launch_bounds__(64 * WAVES) void wide_kernel(const GemmParams p)
 //   128 x 256  2048 x 4096 x 4096 65 (70), x 11008 168 (180), 1672 x 4096 x 2048 35 (41), 32 groups of 8192 rows, 5504, 4096 493 (514), of 6688 rows, 2816, 2048 127 (126)
 //   128 x 192  1024 x 6912 x 2048 29.5 (31.9), 2048 x 8832 x 4096 161 (165)      128 x 128  1672 x 2048 x 2048 14.5 (17.8)
 //   128 x 64   1024 x 2048 x 4096 and x 6528, behind a gate into the residual 29.8 (31.7)
+// (Named as the lock-step form: whoever reads a tile from a kernel's name finds it in the same arguments; wide:: tells the two apart.)
 template <int WT, int WM, int WN, int MT, int NT, int S, int OUT, bool GROUPED, bool PINNED>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParams p_in)
 {
+    static_assert(WT == W_BF16, "a K-tile is 64 values of 2 bytes, results leave through the stack engine's seam");
     constexpr bool PAIRS = out_pairs(OUT);
     constexpr int NA = 2 * MT, NB = 2 * NT;
     constexpr int NW = WM * WN, BM = WM * NA * 16, BN = WN * NB * 16, STAGE = (BM + BN) * 128, DMAS = (BM + BN) / 8 / NW, DMA_A = BM / 8 / NW;
