@@ -10,7 +10,7 @@ from test_gpu_session import synth_model
 
 pytestmark = pytest.mark.gpu
 S, NEW = 352, 4
-BATCHES = [(352, 176, 240, 350), (352, 352, 352, 352), (352, 352, 352, 177), (352, 352, 352, 176), (352, 1, 352, 2)]  # 1408 rows, 11 x 48 tiles: up to 1232 pack
+BATCHES = [(352, 176, 240, 350), (352, 352, 352, 352), (352, 352, 352, 177), (352, 352, 352, 176), (352, 1, 352, 2), (1, 3, 1, 1)]  # 1408 rows, 11 x 48 tiles: up to 1232 pack
 
 
 def sessions(mode, int8_kv):

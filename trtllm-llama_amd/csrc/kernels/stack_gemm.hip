@@ -393,16 +393,17 @@ __global__ __launch_bounds__(256) void row_short_kernel(const StackGemmParams p_
 
 // row_kernel whose row is formed here (StackRowNorm) instead of by a launch of its own in front, which costs its start and 2.3 us for some hundred cycles of work: the
 // row is requested ahead of the weights and normed while they are under way.  K <= 512 KS NC.  Rows of more than 2048 values by whole waves, 8 columns a workgroup, as
-// every workgroup reads the row (10240 x 4096 by 2 columns a workgroup 21.6), but for few columns.  us in a step of one token, norm + product and here: 10304 x 2048 2.3 + 11.0, 10.7;
-// 11008 x 2048 2.3 + 11.2, 11.2; 10240 x 4096 4.6 + 14.7, 17.1; 16384 x 4096 4.6 + 21.0, 23.8;
-// 2048 x 4096, 8 parts 3.3 + 5.9, 5.8 (by 4 columns a workgroup 6.5, by 2 7.3).
+// every workgroup reads the row (10240 x 4096 by 2 columns a workgroup 21.6), but for few columns.  us in a step of one token, norm + product and here: 10304 x 2048 2.3 + 11.0, 10.5;
+// 11008 x 2048 2.3 + 11.2, 11.1; 10240 x 4096, 4 parts 4.6 + 14.7, 17.5; 16384 x 4096, 4 parts 4.6 + 21.0, 24.5;
+// 2048 x 4096, 8 parts 3.3 + 5.9, 7.0 (with sums in another order, of quarters of a row, 5.8; so by 4 columns a workgroup 6.5, by 2 7.3).
 template <int KS, int NC, int NP, int PARTS>
 __global__ __launch_bounds__(256) void row_norm_kernel(const StackGemmParams p, const StackRowNorm n)
 {
     constexpr int TEAMS = 4 / KS;
     constexpr int SUMS = KS == 1 && NC > 4 ? 4 : 1; // of a wave: K in the parts, and their order, of row_kernel's waves, which share rows of more than 2048
     __shared__ __attribute__((aligned(16))) uint16_t row[NP * 1024];
-    __shared__ float red[LoneRow<NP, PARTS>::SUMS], part[4][SK_R];
+    __shared__ __attribute__((aligned(16))) float red[LoneRow<NP, PARTS>::SUMS];
+    __shared__ float part[4][SK_R];
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kw = wid % KS;
     const int n0 = (blockIdx.x * TEAMS + wid / KS) * SK_R;
     LoneRow<NP, PARTS> lone;

@@ -152,13 +152,13 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const StackMoeParams p,
 }
 
 // A lone token's, its row formed here (StackRowNorm) while the router's rows are under way: lane l has values 8 l .. of every 512, in the order of router_row.
-// 34 outputs of width 2048 in a step: 3.4 us for what took 2.3 and 3.3.
+// 34 outputs of width 2048 in a step: 3.5 us for what took 2.3 and 3.3.
 template <int NP>
 __global__ __launch_bounds__(256) void moe_logits_norm_kernel(const StackMoeParams p, const StackRowNorm n)
 {
     constexpr int PIECES = 2 * NP; // of 512 values, all requested at once
     __shared__ __attribute__((aligned(16))) uint16_t row[NP * 1024];
-    __shared__ float red[LoneRow<NP, 0>::SUMS];
+    __shared__ __attribute__((aligned(16))) float red[LoneRow<NP, 0>::SUMS];
     const int NE = p.experts + p.identity, W = p.width, lane = threadIdx.x & 63, e = blockIdx.x * 4 + (threadIdx.x >> 6);
     LoneRow<NP, 0> lone;
     lone.request(n, W);

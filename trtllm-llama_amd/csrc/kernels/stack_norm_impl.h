@@ -36,7 +36,7 @@ __device__ __forceinline__ float sum_squares(const float (&v)[N])
 }
 
 // Both forms: request() asks for the row, ahead of the operands that it is to arrive before and without a branch that a load would wait behind; finish() leaves it in `row`, LDS
-// [width] in bfloat16.  red: LDS, SUMS floats.  first: this workgroup also leaves what later launches read.  The sums of squares run in the order of the launch whose place
+// [width] in bfloat16.  red: LDS, SUMS floats on 16 bytes.  first: this workgroup also leaves what later launches read.  The sums of squares run in the order of the launch whose place
 // is taken, so that a row has the same bits either way; what that costs (a sum over a wave a piece instead of one in all) passes while the weights are under way.
 
 // A row of one stream, as hyper_norm_vec_kernel: a lane's float4, 64 lanes, the 256 values of each wave in turn.  The workgroup's 4 waves have NP such pieces each.
@@ -157,11 +157,12 @@ struct PartsRow
                 red[4 * g + (threadIdx.x >> 6)] = ss;
         }
         __syncthreads();
+        const float4 r = reinterpret_cast<const float4*>(red)[threadIdx.x & (PARTS - 1)]; // (lane g has part g's root: one sequence of instructions instead of PARTS)
+        const float root = 1.f / sqrtf((((r.x + r.y) + r.z) + r.w) / (float) (width / PARTS) + n.eps);
 #pragma unroll
         for (int g = 0; g < PARTS; ++g)
         {
-            const float ss = ((red[4 * g] + red[4 * g + 1]) + red[4 * g + 2]) + red[4 * g + 3];
-            const float inv = 1.f / sqrtf(ss / (float) (width / PARTS) + n.eps);
+            const float inv = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, root), g));
 #pragma unroll
             for (int k = 0; k < EACH; ++k)
             {
