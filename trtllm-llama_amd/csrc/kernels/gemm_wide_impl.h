@@ -913,6 +913,271 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParam
         leave_fp32<OUT>(p, acc, lane, p.c, row0, col0, p.M);
 }
 
+// Tiles of up to 288 rows x 192 columns, for groups of a few hundred rows: bfloat16, 8 waves of 2 x 4, a wave the row blocks wm, wm + 2, ... and 48 columns.  A group's rows
+// are cut into as few tiles as take them, of equal height in steps of 32 rows; a wave's blocks are a template of the loop, so that a tile fetches and multiplies no more rows than it has.
+//   Bound by the operands' way from L2 (28 bytes per clock and CU) and the weights' from HBM.  Tiles of 128 rows bring a group's weights in two or three times, the last one for
+// a few rows as often as not; 256 x 256 ones once, but a group of a few rows more costs two thirds of another tile, and a tile is a third of a round: that is why a tile is
+// as high as three buffers of A and two of W's 192 columns let it be.  Reads and requests as in the 256 x 256 loop: 1.5 K-tiles ahead, W's buffer handed back within the K-tile.
+// us, 32 groups, random sizes, cold weights, in brackets 128 x 256 and 256 x 256: 8192 rows, 5504, 4096 390 (476, 523; 330 with weights from L2), 4096, 2752 216 (272, 295), 6900 rows,
+// 2816, 2048 111 (122, 130; 84 with weights from L2), of 12000 rows, 4224, 3072 338 (392, 400).
+// Tried and no quicker: W asked for two K-tiles ahead and A three where they fit (nothing: it is not the latency), weights' requests marked nt, K begun at another place by each column of
+// tiles (100 -> 87 at 4084 rows, 2816, 2048, whose rows of 4096 bytes meet few memory channels, 390 -> 460 at 5504, 4096).
+template <int NA>
+struct TallLoop
+{
+    static constexpr int NB = 3, BLOCKS = 2 * NA, AHEAD = NA >= 5 ? 3 : 2, HAND_OVER = BLOCKS - AHEAD, MID = NA >= 5 ? 3 : 2;
+    static constexpr int DMA_A = (NA + 1) / 2, DMA_W = 3, DMAS = DMA_A + DMA_W, SLOTS = (HAND_OVER - MID) * NB;
+    static constexpr bool ODD = NA % 2 != 0; // the last of A's requests is there in half of the waves only
+};
+constexpr int TALL_BM = 288, TALL_BN = 192, TALL_A = TALL_BM * 128, TALL_W = TALL_BN * 128, TALL_LDS = 3 * TALL_A + 2 * TALL_W;
+// Row of W's tile (of the wave's 48) that MFMA row i of block j takes: a lane's results of the three blocks are 12 neighbouring columns.
+__device__ __forceinline__ int tall_w_row(int j, int i)
+{
+    return 12 * (i >> 2) + 4 * j + (i & 3);
+}
+__device__ __forceinline__ int tall_w_swz(int row) // of 192
+{
+    return (row & 2) | (row % 48 >= 24 ? 4 : 0);
+}
+struct TallTile
+{
+    const char *a, *w;
+    uint32_t ao[5], wo[3], lds;
+    int nt, wid, lane;
+    f32x4 acc[9][3];
+
+    template <int NA>
+    __device__ __forceinline__ void dma(int i, int t, uint32_t abuf, uint32_t wbuf) const
+    {
+        using L = TallLoop<NA>;
+        if (i >= L::DMA_A)
+            load16(w + (int64_t) t * 128, wo[i - L::DMA_A], wbuf + (uint32_t) ((i - L::DMA_A) * 8 + wid) * 1024);
+        else if (!L::ODD || i < L::DMA_A - 1 || wid < 4)
+            load16(a + (int64_t) t * 128, ao[i], abuf + (uint32_t) (i * 8 + wid) * 1024);
+    }
+    // this wave's requests are in but for the last K-tile's, everyone's behind the barrier
+    template <int NA>
+    __device__ __forceinline__ void landed() const
+    {
+        using L = TallLoop<NA>;
+        if (L::ODD && wid >= 4)
+            wait_vm_and_meet<L::DMAS - 1>();
+        else
+            wait_vm_and_meet<L::DMAS>();
+    }
+    template <int NA>
+    __device__ __forceinline__ void run()
+    {
+        using L = TallLoop<NA>;
+        constexpr int NB = L::NB;
+        static_assert(L::SLOTS > 0 && L::AHEAD * (NB - 1) >= NB, "requests between the two barriers, the next k-step's fragments behind the second");
+        uint32_t A0 = lds, A1 = lds + TALL_A, A2 = lds + 2 * TALL_A, W0 = lds + 3 * TALL_A, W1 = W0 + TALL_W; // of K-tiles t, t + 1, t + 2 and t, t + 1
+#pragma unroll
+        for (int i = 0; i < L::DMAS; ++i)
+            dma<NA>(i, 0, A0, W0);
+        if (nt > 1)
+        {
+#pragma unroll
+            for (int i = 0; i < L::DMAS; ++i)
+                dma<NA>(i, 1, A1, W1);
+            landed<NA>();
+        }
+        else
+            wait_vm_and_meet<0>();
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+                acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int i16 = lane & 15, k4 = lane >> 4, wm = wid >> 2, wn = wid & 3;
+        const uint32_t al = (uint32_t) ((16 * wm + i16) * 128), wl = (uint32_t) ((48 * wn + tall_w_row(0, i16)) * 128);
+        const uint32_t as = a_swz(i16), ws = tall_w_swz(tall_w_row(0, i16));
+        const uint32_t a_k0 = al + ((k4 ^ as) << 4), a_k1 = al + (((4 + k4) ^ as) << 4), w_k0 = wl + ((k4 ^ ws) << 4), w_k1 = wl + (((4 + k4) ^ ws) << 4);
+        auto a_at = [](uint32_t base, int block) { return *(lds_frag) (uintptr_t) (base + block * 4096); };
+        auto w_at = [](uint32_t base, int j) { return *(lds_frag) (uintptr_t) (base + j * 512); };
+        u32x4 fa[L::BLOCKS + L::AHEAD], fw[2][NB];
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            fw[0][j] = w_at(W0 + w_k0, j);
+#pragma unroll
+        for (int i = 0; i < L::AHEAD; ++i)
+            fa[i] = a_at(A0 + a_k0, i);
+        for (int t = 0; t < nt; ++t)
+        {
+            const uint32_t ra[3] = {A0 + a_k0, A0 + a_k1, A1 + a_k0}, rw1 = W0 + w_k1, rwn = W1 + w_k0;
+            const bool more = t + 2 < nt;
+#pragma unroll
+            for (int g = 0; g < L::BLOCKS; ++g)
+            {
+                if (g == L::MID)
+                {
+                    // W's fragments of k-step 1 have arrived (A blocks requested behind them may be under way): nobody reads W(t), or A(t - 1), any more
+                    asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(L::MID - 2) : "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (g == L::HAND_OVER)
+                {
+                    // K-tile t + 1 has landed
+                    if (more)
+                        landed<NA>();
+                    else
+                        wait_vm_and_meet<0>();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                {
+                    acc[g % NA][j] = mfma<W_BF16>(fw[g / NA][j], fa[g], acc[g % NA][j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (j == 0)
+                        fa[g + L::AHEAD] = a_at(ra[(g + L::AHEAD) / NA], (g + L::AHEAD) % NA);
+                    else
+                    {
+                        const int q = g * (NB - 1) + j - 1, qn = q - L::HAND_OVER * (NB - 1);
+                        if (q < NB)
+                            fw[1][q] = w_at(rw1, q);
+                        if (qn >= 0 && qn < NB) // (behind the last K-tile: old data, not used)
+                            fw[0][qn] = w_at(rwn, qn);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < L::DMAS; ++i)
+                        if (more && g >= L::MID && g < L::HAND_OVER && i * L::SLOTS / L::DMAS == (g - L::MID) * NB + j)
+                            dma<NA>(i, t + 2, A2, W0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < L::AHEAD; ++i)
+                fa[i] = fa[L::BLOCKS + i];
+            const uint32_t x = A0, y = W0;
+            A0 = A1, A1 = A2, A2 = x, W0 = W1, W1 = y;
+        }
+    }
+    template <int OUT, int NA>
+    __device__ __forceinline__ void leave(const GemmParams& p, char* c, int row0, int col, int rows) const
+    {
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+        {
+            const int row = row0 + 32 * i;
+            if (row >= rows)
+                continue;
+            const bool all = col + 12 <= p.N;
+            uint32_t o[6];
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+            {
+                const f32x4 v = acc[i][j];
+                if constexpr (OUT == OUT_GATED)
+                    o[j] = bf_pair(seam_gate<false>(p.act, v[0], v[1]), seam_gate<false>(p.act, v[2], v[3]));
+                else if constexpr (OUT == OUT_STORE)
+                {
+                    const bool sq = p.act == GEMM_ACT_RELU2;
+                    o[2 * j] = bf_pair(sq ? seam_relu2(v[0]) : v[0], sq ? seam_relu2(v[1]) : v[1]);
+                    o[2 * j + 1] = bf_pair(sq ? seam_relu2(v[2]) : v[2], sq ? seam_relu2(v[3]) : v[3]);
+                }
+                else if (col + 4 * j < p.N)
+                    *reinterpret_cast<float4*>(c + ((int64_t) row * p.ldc + col + 4 * j) * 4) = make_float4(v[0], v[1], v[2], v[3]);
+            }
+            if constexpr (OUT == OUT_GATED)
+            {
+                uint32_t* to = reinterpret_cast<uint32_t*>(c + ((int64_t) row * p.ldc + (col >> 1)) * 2);
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                    if (all || col + 4 * j < p.N)
+                        to[j] = o[j];
+            }
+            else if constexpr (OUT == OUT_STORE)
+            {
+                uint2* to = reinterpret_cast<uint2*>(c + ((int64_t) row * p.ldc + col) * 2);
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                    if (all || col + 4 * j < p.N)
+                        to[j] = make_uint2(o[2 * j], o[2 * j + 1]);
+            }
+        }
+    }
+};
+template <int OUT>
+__global__ __launch_bounds__(64 * WAVES) void tall_kernel(const GemmParams p)
+{
+    extern __shared__ __attribute__((aligned(16))) char wide_lds[];
+    const GroupTile gt = group_tile<TALL_BM>(p, (p.N + TALL_BN - 1) / TALL_BN, blockIdx.x);
+    if (gt.group < 0)
+        return; // behind the last tile
+    const int first = p.group_off[gt.group], rows = p.group_off[gt.group + 1] - first;
+    const int tiles_m = (rows + TALL_BM - 1) / TALL_BM, tn = gt.tile / tiles_m, height = ((rows + tiles_m - 1) / tiles_m + 31) / 32 * 32;
+    const int m0 = (gt.tile - tn * tiles_m) * height, n0 = tn * TALL_BN;
+    if (m0 >= rows)
+        return; // (many rows, rounded up to whole steps)
+    const int blocks = (min(height, rows - m0) + 31) / 32; // of a wave
+    TallTile t;
+    t.lane = threadIdx.x & 63;
+    t.wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    t.lds = (uint32_t) (uintptr_t) (lds_ptr*) wide_lds;
+    t.nt = p.K / 64;
+    t.a = reinterpret_cast<const char*>(p.a);
+    t.w = reinterpret_cast<const char*>(p.w) + gt.group * p.batch_w;
+    const int row8 = t.wid * 8 + (t.lane >> 3), piece = t.lane & 7;
+#pragma unroll
+    for (int i = 0; i < 5; ++i)
+    {
+        const int row = i * 64 + row8, m = m0 + row;
+        int r = first + (m < rows ? m : rows - 1);
+        if (p.a_rows)
+            r = p.a_rows[r];
+        t.ao[i] = (uint32_t) r * (uint32_t) (p.lda * 2) + ((piece ^ a_swz(row)) << 4);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+    {
+        const int row = i * 64 + row8, col = n0 + row, n = col < p.N ? col : p.N - 1;
+        t.wo[i] = (uint32_t) n * (uint32_t) p.ldw + ((piece ^ tall_w_swz(row)) << 4);
+    }
+    char* c = reinterpret_cast<char*>(p.c) + first * p.ldc * (OUT == OUT_FP32 ? 4 : 2);
+    const int row0 = m0 + 16 * (t.wid >> 2) + (t.lane & 15), col = n0 + 48 * (t.wid & 3) + 12 * (t.lane >> 4);
+    auto go = [&](auto na) {
+        constexpr int NA = decltype(na)::value;
+        t.run<NA>();
+        t.leave<OUT, NA>(p, c, row0, col, rows);
+    };
+    switch (blocks)
+    {
+    case 9: return go(std::integral_constant<int, 9>());
+    case 8: return go(std::integral_constant<int, 8>());
+    case 7: return go(std::integral_constant<int, 7>());
+    case 6: return go(std::integral_constant<int, 6>());
+    case 5: return go(std::integral_constant<int, 5>());
+    case 4: return go(std::integral_constant<int, 4>());
+    default: return go(std::integral_constant<int, 3>());
+    }
+}
+template <int OUT>
+int launch_tall_out(const GemmParams& p, hipStream_t stream)
+{
+    launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(tall_kernel<OUT>), TALL_LDS);
+    const int64_t tiles = (p.group_total / TALL_BM + std::min<int64_t>(p.batch, p.group_total)) * ((p.N + TALL_BN - 1) / TALL_BN);
+    hipLaunchKernelGGL(tall_kernel<OUT>, dim3((unsigned) tiles), dim3(64 * WAVES), TALL_LDS, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+    {
+        set_error("gemm tall tiles: launch failed: %s", hipGetErrorString(e));
+        return -1;
+    }
+    return 0;
+}
+// p: serves<W_BF16>(p)
+inline bool tall_serves(const GemmParams& p)
+{
+    return p.group_off && !p.resid && !p.bias && p.seam.n_sec == 0 && (p.act == GEMM_ACT_NONE || p.act == GEMM_ACT_RELU2 || p.act >= GEMM_ACT_GATE_SILU) && (p.out_dtype == DT_BFLOAT16 || p.act == GEMM_ACT_NONE);
+}
+// p: tall_serves(p)
+inline int launch_tall(const GemmParams& p, hipStream_t stream)
+{
+    return p.act >= GEMM_ACT_GATE_SILU ? launch_tall_out<OUT_GATED>(p, stream) : p.out_dtype == DT_FLOAT ? launch_tall_out<OUT_FP32>(p, stream) : launch_tall_out<OUT_STORE>(p, stream);
+}
+
 inline bool aligned16(const void* p)
 {
     return !(reinterpret_cast<uintptr_t>(p) & 15);

@@ -715,6 +715,51 @@ inline int launched(const char* what)
     return 0;
 }
 
+// Rows of a group are expected to spread around m by its root: how many tiles of `high` rows a group has on average.
+inline double expected_tiles(int m, int high)
+{
+    double tiles = 1.0;
+    for (int at = high; at < 3 * m + 16; at += high) // one more for every group of more than `at` rows
+        tiles += 0.5 * std::erfc((at - m) / std::sqrt(2.0 * m));
+    return tiles;
+}
+// The tiles of a grouped product of gemm_wide_impl.h by what they are expected to take, us: rounds of the chip x (a tile's launch, first requests and results, and its K-tiles), or
+// the weights' way from HBM (5.1 TB/s), whichever is longer, rounded off between the two.  Fitted to 180 products of 8 .. 64 groups of 40 .. 600 rows, N 512 .. 5504, K 512 .. 4096,
+// cold weights, of each form, within 6 - 11 %; the forms that it picks have 0.91 of the time that the pick of one shape by rounds and area had, the best ones 0.90.
+// us, 128 x 256 / 256 x 256 / up to 288 x 192: 32 groups of 256 rows, 5504, 4096 476 / 523 / 390, 4096, 2752 272 / 295 / 216; of 216, 2816, 2048 122 / 130 / 111, 2048, 1408 58 / 44 / 63;
+// of 375, 4224, 3072 392 / 400 / 338; of 94 184 / 192 / 166; of 128, 2816, 2048 97 / 117 / 100, 2048, 1408 46 / 39 / 46.
+enum GroupForm
+{
+    GROUP_128x128, // up to 64 rows
+    GROUP_128x256,
+    GROUP_256x256,
+    GROUP_TALL
+};
+GroupForm pick_group_form(const GemmParams& g, int m)
+{
+    const double kt = g.K / 64, cus = launch_util::device_cus(), weights = (double) g.batch * g.N * g.K * 2 / 5.1e6;
+    auto us = [&](int high, int wide, double fixed, double k_tile) {
+        const double tiles = expected_tiles(m, high) * g.batch * ((g.N + wide - 1) / wide) / cus;
+        const double a = std::max(1.0, std::ceil(tiles - 0.03)) * (fixed + kt * k_tile), b = fixed + weights;
+        return std::sqrt(std::sqrt(a * a * a * a + b * b * b * b));
+    };
+    GroupForm form = GROUP_128x256;
+    double best = us(128, 256, 6.6, 0.86);
+    auto offer = [&](GroupForm f, double t) {
+        if (t < best)
+        {
+            best = t;
+            form = f;
+        }
+    };
+    if (m <= 64)
+        offer(GROUP_128x128, us(128, 128, 5.5, 0.45));
+    offer(GROUP_256x256, us(256, 256, 7.5, m + 1.5 * std::sqrt(m) <= 128 ? 0.95 : 1.36));
+    if (wide::tall_serves(g))
+        offer(GROUP_TALL, us(wide::TALL_BM, wide::TALL_BN, 7.1, 0.34 + 0.004 * std::min<double>(wide::TALL_BM, m / expected_tiles(m, wide::TALL_BM))));
+    return form;
+}
+
 // The tile shapes of the LDS-DMA kernels, all with stages of whole 128-byte lines and 8 waves, and what a tile of each kind costs per area when
 // the chip is full of them (measured, relative to lock-step 256 x 256; M 2048 .. 512, N 2048 .. 22016, K 2048 .. 11008): fewest workgroup rounds x
 // area x cost.  row_tiles: those of 128 rows by gemm_wide_impl.h, 4 - 18 % quicker than the lock-step ones of gemm_glds_impl.h (figures there), which stay for
@@ -744,25 +789,22 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
             pick = sh.id;
         }
     }
-    // Grouped: m_expected rows in a group on average (g.M is their bound); up to three 128-row tiles the groups' last ones decide.  32 groups of 8096 rows: 128 x 256 151 us against 160 for 128 x 128 and
-    // 167 for 256 x 192 (N 2816, K 2048), 255 / 307 / 291 (4096, 2752); of 1944 rows 128 x 128 92 us, the wider ones 95 and more (2816, 2048).
-    // 256 x 256 only where it saves rounds: 32 groups of 6700 rows 60.5 us in one round against 66.6 in two (N 2048, K 1408), 145 in two against 125 in
-    // three (2816, 2048).  A group's rows spread around the average by its root; a round of the last few tiles, most of them nearly empty, does not count
-    // against the smaller ones (16 groups of 128 rows on average, N 2816, K 2048: 1.03 rounds of 128 x 256 51 us, 0.69 of 256 x 256 65; 16 of 350, 4096, 1024: 3.03
-    // 69, 2.0 78).  Over 280 products of 8 .. 64 groups where the wide ones are taken they have 0.82 - 0.99 of the other's time.
-    if (m_expected > 0 && m_expected <= 384)
+    // Grouped: m_expected rows in a group on average (g.M is their bound).  Of more than 384 the shapes above, too (16 of 453, 512, 1024 128 x 128 15.2 us, 128 x 256 20.7).
+    // Lock-step tiles, us: 32 groups of 8096 rows 128 x 256 151 against 160 for 128 x 128 and 167 for 256 x 192 (N 2816, K 2048), of 1944 rows 128 x 128 92, the wider ones 95 and more.
+    if (m_expected > 0 && (served || m_expected <= 384))
     {
-        auto cost = [&](int bm, int bn, double f, double rest) {
-            double tiles = 0.0;
-            for (int at = 0; at < 3 * m_expected; at += bm) // a tile for every group of more than `at` rows
-                tiles += at ? 0.5 * std::erfc((at - m_expected) / std::sqrt(2.0 * m_expected)) : 1.0;
-            return std::ceil(tiles * g.batch * ((g.N + bn - 1) / bn) / cus - rest) * bm * bn * f;
-        };
-        pick = m_expected <= 64 ? 0 : cost(256, 256, shapes[2].f, 0.02) < cost(128, 256, shapes[3].f, 0.08) ? 2 : 3;
+        auto rounds = [&](int high, double rest) { return std::ceil(expected_tiles(m_expected, high) * g.batch * ((g.N + 255) / 256) / cus - rest); };
+        const GroupForm form = served ? pick_group_form(g, m_expected)
+            : m_expected <= 64        ? GROUP_128x128
+            : rounds(256, 0.02) * 256 * lock_step[2].f < rounds(128, 0.08) * 128 * lock_step[3].f ? GROUP_256x256 : GROUP_128x256;
+        if (form == GROUP_TALL)
+            return wide::launch_tall(g, stream);
+        if (served && form == GROUP_256x256)
+            return wide::launch<W_BF16>(g, stream);
+        if (m_expected <= 384)
+            pick = form == GROUP_128x128 ? 0 : form == GROUP_256x256 ? 2 : 3;
     }
-    // 256 x 256 tiles of gemm_wide_impl.h.  Grouped: where groups have two of them (32 groups, us, in brackets the shapes above: 16384 rows, N 2816, K 2048 227 (282), 12000
-    // 176 (202), 16384 rows, 704, 512 24 (34)).  Groups of one tile read their weights alone, from HBM, which a K-tile and a half ahead does not hide: 8192 rows,
-    // 5504, 4096 took 542 (500, by the tiles of 128 rows 490) in a step, the same rows of fewer columns by themselves 133 (141) at 2816, 2048 and 126 (121) with 6700 rows.
+    // 256 x 256 tiles of gemm_wide_impl.h
     if (served)
     {
         if (m_expected > 0)
