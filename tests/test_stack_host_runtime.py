@@ -513,6 +513,20 @@ def group_tiles(stub):
         assert shapes[-2] == want, (experts, top, tokens, ff, shapes)
 
 
+def tall_tiles(stub):
+    """Which of test_gpu_group_tiles.py's products with rows of 512 values and more take tiles of up to 288 x 192: (gated columns, the width's)."""
+    import ruzinex_cases as Z
+    for width in (512, 576):
+        mlp = Z.moe(experts=8, top=8, ff=2944, shared=0)
+        s = engine(Z.make_config([Z.layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=mlp)], width=width), Z, max_tokens=1024, max_sequences=1)
+        for tokens, want in ((72, (True, True)), (97, (False, True)), (129, (True, False)), (288, (True, False)), (330, (True, False))):
+            stub.forget()
+            step(s, 'a', tokens, 0)
+            found = [k for k in stub.kernels() if re.search(r'gemm_glds_kernelI|wide_kernelI', k)]
+            assert tuple('4tall16gemm_glds_kernelILi4ELi9ELi6ELi1ELi1E' in k for k in found[-2:]) == want, (width, tokens, found[-2:])
+        s.release('a')
+
+
 def who_sums(stub):
     """The experts' rows of few tokens are summed by the norm behind them, very many of them by a launch of its own."""
     import narurax_cases as N
@@ -603,6 +617,9 @@ else:
 
     def test_who_sums_the_experts_rows(stub):
         run(stub, 'who_sums')
+
+    def test_tall_tiles_of_grouped_products(stub):
+        run(stub, 'tall_tiles')
 
     def test_tiles_of_grouped_products(stub):
         run(stub, 'group_tiles')

@@ -1099,9 +1099,13 @@ struct TallTile
         }
     }
 };
-template <int OUT>
-__global__ __launch_bounds__(64 * WAVES) void tall_kernel(const GemmParams p)
+namespace tall
 {
+// (named like the other two, 32 WM MT rows x 32 WN NT columns)
+template <int WT, int WM, int WN, int MT, int NT, int OUT>
+__global__ __launch_bounds__(64 * WAVES) void gemm_glds_kernel(const GemmParams p)
+{
+    static_assert(WT == W_BF16 && 32 * WM * MT == TALL_BM && 32 * WN * NT == TALL_BN, "one shape");
     extern __shared__ __attribute__((aligned(16))) char wide_lds[];
     const GroupTile gt = group_tile<TALL_BM>(p, (p.N + TALL_BN - 1) / TALL_BN, blockIdx.x);
     if (gt.group < 0)
@@ -1153,12 +1157,14 @@ __global__ __launch_bounds__(64 * WAVES) void tall_kernel(const GemmParams p)
     default: return go(std::integral_constant<int, 3>());
     }
 }
+} // namespace tall
 template <int OUT>
 int launch_tall_out(const GemmParams& p, hipStream_t stream)
 {
-    launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(tall_kernel<OUT>), TALL_LDS);
+    const auto kernel = tall::gemm_glds_kernel<W_BF16, 9, 6, 1, 1, OUT>;
+    launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), TALL_LDS);
     const int64_t tiles = (p.group_total / TALL_BM + std::min<int64_t>(p.batch, p.group_total)) * ((p.N + TALL_BN - 1) / TALL_BN);
-    hipLaunchKernelGGL(tall_kernel<OUT>, dim3((unsigned) tiles), dim3(64 * WAVES), TALL_LDS, stream, p);
+    hipLaunchKernelGGL(kernel, dim3((unsigned) tiles), dim3(64 * WAVES), TALL_LDS, stream, p);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess)
     {

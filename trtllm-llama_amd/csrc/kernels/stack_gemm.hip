@@ -789,20 +789,25 @@ int launch_glds_bf16(const GemmParams& g, hipStream_t stream, int m_expected = 0
             pick = sh.id;
         }
     }
-    // Grouped: m_expected rows in a group on average (g.M is their bound).  Of more than 384 the shapes above, too (16 of 453, 512, 1024 128 x 128 15.2 us, 128 x 256 20.7).
-    // Lock-step tiles, us: 32 groups of 8096 rows 128 x 256 151 against 160 for 128 x 128 and 167 for 256 x 192 (N 2816, K 2048), of 1944 rows 128 x 128 92, the wider ones 95 and more.
-    if (m_expected > 0 && (served || m_expected <= 384))
+    // Grouped: m_expected rows in a group on average (g.M is their bound); up to three 128-row tiles the groups' last ones decide.  32 groups of 8096 rows: 128 x 256 151 us against 160 for
+    // 128 x 128 and 167 for 256 x 192 (N 2816, K 2048); of 1944 rows 128 x 128 92 us, the wider ones 95 and more.  256 x 256 only where it saves rounds; a round of the last few tiles,
+    // most of them nearly empty, does not count against the smaller ones.
+    if (m_expected > 0 && m_expected <= 384)
     {
-        auto rounds = [&](int high, double rest) { return std::ceil(expected_tiles(m_expected, high) * g.batch * ((g.N + 255) / 256) / cus - rest); };
-        const GroupForm form = served ? pick_group_form(g, m_expected)
-            : m_expected <= 64        ? GROUP_128x128
-            : rounds(256, 0.02) * 256 * lock_step[2].f < rounds(128, 0.08) * 128 * lock_step[3].f ? GROUP_256x256 : GROUP_128x256;
+        auto cost = [&](int bm, double f, double rest) { return std::ceil(expected_tiles(m_expected, bm) * g.batch * ((g.N + 255) / 256) / cus - rest) * bm * f; };
+        pick = m_expected <= 64 ? 0 : cost(256, shapes[2].f, 0.02) < cost(128, shapes[3].f, 0.08) ? 2 : 3;
+    }
+    // Up to two tall tiles of rows of 512 values and more, where K-tiles count and not a tile's start (and which the times are fitted to): by time.  Of more than 384 rows the shapes
+    // above, too (16 groups of 453, 512, 1024 128 x 128 15.2 us, 128 x 256 20.7).
+    if (served && m_expected > 0 && m_expected <= 2 * wide::TALL_BM && g.K >= 512)
+    {
+        const GroupForm form = pick_group_form(g, m_expected);
         if (form == GROUP_TALL)
             return wide::launch_tall(g, stream);
-        if (served && form == GROUP_256x256)
+        if (form == GROUP_256x256)
             return wide::launch<W_BF16>(g, stream);
         if (m_expected <= 384)
-            pick = form == GROUP_128x128 ? 0 : form == GROUP_256x256 ? 2 : 3;
+            pick = form == GROUP_128x128 ? 0 : 3;
     }
     // 256 x 256 tiles of gemm_wide_impl.h
     if (served)
