@@ -61,3 +61,14 @@ def test_vectors_of_every_form_reach_the_engine(engine, form):
 def test_no_wanted_rows(engine):
     logits, ids = engine.step(*WANT[:4], [[1], [2]], [])
     assert logits is None and ids.shape == (0,) and engine.lib.got[5] == []
+
+
+@pytest.mark.parametrize('bad', [2 ** 31, 7.9, np.int64(-2 ** 31 - 1), True])
+def test_lists_that_are_no_whole_numbers_of_32_bits_reach_the_engine_as_numpy_casts_them(engine, bad):
+    tokens = [5, bad, 7, 8]
+    table = np.array(WANT[4], np.int32).reshape(2, 3)
+    table.flags.writeable = False
+    engine.step(tokens, *WANT[1:4], table, WANT[5])
+    want = np.empty(4, np.int32)
+    want[:] = np.asarray(tokens)
+    assert engine.lib.got == [want.tolist()] + WANT[1:]

@@ -190,7 +190,7 @@ class RaggedGenerationSession(object):
         that give back what they hold after this step.  Returns (logits fp32 [wanted, vocab] or None, next ids int32 [wanted]),
         rows in the order of the entries and of their `want`."""
         tokens, counts, pos0, slots, want_rows, seqs = [], [], [], [], [], []
-        seen = set()
+        seen, longest = set(), 0
         for rid, toks, want in entries:
             toks = [int(t) for t in toks]
             if not toks:
@@ -198,29 +198,30 @@ class RaggedGenerationSession(object):
             if rid in seen:
                 raise ValueError(f'request {rid} appears twice in one step')
             seen.add(rid)
-            if rid not in self._seq:
-                self._seq[rid] = self._Sequence(self._next_seq_idx, len(self._seq))
+            seq = self._seq.get(rid)
+            if seq is None:
+                seq = self._seq[rid] = self._Sequence(self._next_seq_idx, len(self._seq))
                 self._next_seq_idx += 1
                 self._len[rid] = 0
-            seq = self._seq[rid]
+            n, at = len(toks), self._len[rid]
             slot = self.slots.acquire(seq)
-            self.cache.reserve(seq, self._len[rid] + len(toks))
+            self.cache.reserve(seq, at + n)
             for w in want:
-                if not 0 <= int(w) < len(toks):
-                    raise ValueError(f'request {rid}: wanted place {w} is outside its {len(toks)} tokens')
+                if not 0 <= int(w) < n:
+                    raise ValueError(f'request {rid}: wanted place {w} is outside its {n} tokens')
                 want_rows.append(len(tokens) + int(w))
             tokens += toks
-            counts.append(len(toks))
-            pos0.append(self._len[rid])
+            counts.append(n)
+            pos0.append(at)
             slots.append(slot)
             seqs.append(seq)
+            longest = max(longest, at + n)
         out = (None, np.empty(0, np.int32))
         if entries:
-            max_blocks = max(-(-(p + c) // self.page_size) for p, c in zip(pos0, counts))
-            table = self.cache.blocks_manager.block_table(seqs, max_blocks)
+            table = self.cache.blocks_manager.block_table(seqs, -(-longest // self.page_size))
             out = self.engine.step(tokens, counts, pos0, slots, table, want_rows, return_logits=return_logits)
-            for (rid, toks, _) in entries:
-                self._len[rid] += len(toks)
+            for (rid, _, _), n in zip(entries, counts):
+                self._len[rid] += n
         for rid in end:
             self.release(rid)
         return out

@@ -104,11 +104,15 @@ class BlocksManager(object):
 
     def block_table(self, owners: List[GenerationSequence], max_blocks: int):
         """int32 [len(owners), max_blocks] of block ids (beam 0), zero-padded: what an engine that addresses blocks by id takes."""
-        table = np.zeros((len(owners), max_blocks), np.int32)
-        for i, owner in enumerate(owners):
-            ids = self._owned.get(owner, [[]])[0]
-            table[i, :len(ids)] = ids
-        return table
+        flat = []
+        for owner in owners:
+            rows = self._owned.get(owner)
+            ids = rows[0] if rows else []
+            if len(ids) > max_blocks:
+                raise ValueError(f'sequence {owner.get_seq_idx()} holds {len(ids)} blocks, the table has room for {max_blocks}')
+            flat += ids
+            flat += [0] * (max_blocks - len(ids))
+        return np.array(flat, np.int32).reshape(len(owners), max_blocks)
 
     # -- what the kernels consume
     def get_pointer_array(self, pool_idx: int):
@@ -148,11 +152,12 @@ class KVCacheManager(object):
     def reserve(self, sequence: GenerationSequence, total_tokens: int):
         """Ragged batches: make `sequence` (known or new) hold blocks for `total_tokens` tokens.  A prompt arrives in portions of
         any size, so the blocks are taken as the portions come, not for the whole prompt at once."""
-        if sequence not in self.blocks_manager._owned and sequence not in self.sequences:
+        owned = self.blocks_manager._owned.get(sequence)
+        if owned is None and sequence not in self.sequences:
             sequence.batch_idx = len(self.sequences)
             self.sequences.append(sequence)
             self.lens.append(0)
-        owned = self.blocks_manager._owned.get(sequence)
+            owned = self.blocks_manager._owned.get(sequence)  # (what is held for the place that it has now)
         at = sequence.batch_idx  # its place, unless the caller counts its batch another way, with numbers or without
         if not (type(at) is int and 0 <= at < len(self.sequences) and self.sequences[at] is sequence):
             at = self.sequences.index(sequence)
@@ -216,8 +221,9 @@ class StateSlotManager(object):
         return len(self._free)
 
     def acquire(self, sequence: GenerationSequence) -> int:
-        if sequence in self._owner:
-            return self._owner[sequence]
+        slot = self._owner.get(sequence)
+        if slot is not None:
+            return slot
         if not self._free:
             raise RuntimeError(f'all {self.slots} state slots are in use')
         slot = min(self._free)

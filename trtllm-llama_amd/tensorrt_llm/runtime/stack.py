@@ -3,6 +3,7 @@
 `StackEngine` owns a tllm_stack_t.  It is the compute half only - which page and which state slot a sequence uses is the
 business of the cache managers in kv_cache_manager.py, and what a step contains that of the scheduler (scheduler.py) or of a
 caller that drives `RaggedGenerationSession.step` itself."""
+import array
 import ctypes
 import os
 import subprocess
@@ -25,6 +26,10 @@ def build_library(jobs: Optional[int] = None):
     csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.dirname(os.path.realpath(__file__)))), 'csrc')
     jobs = jobs or min(16, os.cpu_count() or 1)
     subprocess.run(['make', '-C', csrc, 'stack', '-j', str(jobs)], check=True, stdout=subprocess.DEVNULL)
+
+
+def _address(a: np.ndarray) -> int:
+    return ctypes.addressof(ctypes.c_char.from_buffer(a)) if a.flags.writeable and a.size else a.ctypes.data  # (half the time of the latter)
 
 
 class Batch(ctypes.Structure):
@@ -112,20 +117,30 @@ class StackEngine:
              want_rows: Sequence[int], return_logits: bool = True, stream: int = 0):
         """One packed step.  block_table: int32 [entries, max_blocks].  Returns (logits fp32 [n_want, vocab] or None,
         next ids int32 [n_want]): the arg-max of every wanted row is the greedy sampler's choice."""
-        table = np.asarray(block_table)
         n, e, w = len(tokens), len(counts), len(want_rows)
+        table = block_table if type(block_table) is np.ndarray else np.asarray(block_table)
         assert table.ndim == 2 and table.shape[0] == e == len(pos0) == len(slots)
         # the step's arrays side by side in one: one address to look up
-        at = (0, n, n + e, n + 2 * e, n + 3 * e, n + 3 * e + table.size, n + 3 * e + table.size + w)
-        meta = np.empty(at[6], np.int32)
-        for i, a in enumerate((tokens, counts, pos0, slots, table, want_rows)):
-            meta[at[i]:at[i + 1]] = np.asarray(a).reshape(-1)[:at[i + 1] - at[i]]  # (whatever its shape, as its memory has it)
-        p = meta.ctypes.data
-        b = Batch(n, e, w, table.shape[1], p, p + 4 * at[1], p + 4 * at[2], p + 4 * at[3], p + 4 * at[4], p + 4 * at[5] if w else None)
+        at = (0, n, n + e, n + 2 * e, n + 3 * e, n + 3 * e + w, n + 3 * e + w + table.size)
+        vectors = (tokens, counts, pos0, slots, want_rows)
+        meta = None
+        if all(type(v) is list for v in vectors):
+            try:  # lists of whole numbers, as the session hands them over: 2 us where numpy takes 9
+                meta = array.array('i', tokens + counts + pos0 + slots + want_rows)
+            except (TypeError, OverflowError):
+                pass
+        if meta is not None and table.dtype == np.int32 and table.flags.c_contiguous:
+            p, p_table = meta.buffer_info()[0], _address(table)
+        else:
+            meta = np.empty(at[6], np.int32)
+            for i, a in enumerate(vectors + (table,)):
+                meta[at[i]:at[i + 1]] = np.asarray(a).reshape(-1)[:at[i + 1] - at[i]]  # (whatever its shape, as its memory has it)
+            p = _address(meta)
+            p_table = p + 4 * at[5]
+        b = Batch(n, e, w, table.shape[1], p, p + 4 * at[1], p + 4 * at[2], p + 4 * at[3], p_table, p + 4 * at[4] if w else None)
         logits = np.empty((w, self.vocab), np.float32) if (return_logits and w) else None
         ids = np.empty(w, np.int32)
-        rc = load_library().tllm_stack_step(self._h, ctypes.byref(b), logits.ctypes.data if logits is not None else None,
-                                            ids.ctypes.data if w else None, stream)
+        rc = load_library().tllm_stack_step(self._h, ctypes.byref(b), _address(logits) if logits is not None else None, _address(ids) if w else None, stream)
         if rc:
             raise RuntimeError(f'tllm_stack_step failed: {last_error()}')
         self._last_tokens = n
