@@ -106,3 +106,12 @@ def test_a_row_without_finite_numbers_leaves_the_earlier_ones_alone(kind, dtype,
     assert not np.isfinite(got['a'][where]).all()
     check_request(mod, kind, got['a'][:where], toks[:where], w, cfg, dtype, 'a')
     check_request(mod, kind, got['b'], other, w, cfg, dtype, 'b')
+
+
+# Eight chunks between two barriers (chunk_scan_kernel, dim up to 128): portions that end in, on and behind an eighth chunk, one that begins with carried state, waves without a chunk.
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('dim,vdim', [(64, 24), (128, 16)])
+@pytest.mark.parametrize('kind', ['hgrn2', 'mamba2'])
+def test_portions_around_eight_chunks(kind, dim, vdim, dtype, monkeypatch):
+    monkeypatch.setitem(SCHEDULES, 'eights', [[('a', 112), ('b', 128)], [('a', 129), ('b', 32)], [('a', 127), ('b', 257)], [('a', 144), ('b', 1)]])
+    run(kind, dim, vdim, dtype, 'eights')

@@ -11,14 +11,14 @@
 // mode) in both element types.
 //
 // Two launches.  chunk_prepare_kernel / ssm_prepare_kernel: a workgroup per (chunk, head), resp. (chunk, group), all chunks at once: gates, unit
-// norms, the decayed vectors, P, M and T into scratch.  chunk_walk_kernel: a workgroup per (entry, head, 16 columns of V) walks the chunks; its
+// norms, the decayed vectors, P, M and T into scratch.  chunk_scan_kernel (HGRN2 and Mamba-2 with D up to 128) or chunk_walk_kernel: a workgroup per (entry, head, 16 columns of V) walks the chunks; its
 // four waves keep the state's rows in turn, 16 at a time, in registers in the MFMA's accumulator layout (lane: column lane & 15, rows 4 (lane >> 4)
 // + i), which is also its B-operand layout when the four K = 4 steps of 16 rows take rows 4 g + i in step i: S, u and v go from product to
 // product without moving, and what comes from scratch is 16 bytes per lane.  One barrier per chunk, where the waves' partial o (and S^T k)
 // meet; the next chunk's operands are in flight under this one's products.
 //
-// Measured (us, both launches, 16 heads): HGRN2 128 x 128, 1024 rows 1024 -> 68; delta rule 128 x 128, three prompts of 683 rows in all 1740 1193 -> 123;
-// Mamba-2 64 heads 128 x 64, 1021 rows 400 -> 78.
+// Measured (us, both launches, 16 heads): HGRN2 128 x 128, 1024 rows 1024 -> 57; delta rule 128 x 128, three prompts of 683 rows in all 1740 1193 -> 123;
+// Mamba-2 64 heads 128 x 64, 1021 rows 400 -> 57.
 #include "dev_utils.h"
 #include "launch_util.h"
 #include "stack_chunk.h"
@@ -607,6 +607,191 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
     }
 }
 
+// The walk of HGRN2 and Mamba-2, where what a chunk adds to the state does not hang on the state (u is there from the start): one workgroup per (entry, head, 16 columns of V), eight
+// chunks between two barriers, D up to 128.  Wave w carries tile w of the state (16 rows) through the eight: K^T U of its rows, q S of its rows into LDS, S <- b S + K^T U; behind the barrier
+// it sums chunk w's parts and finishes its rows.  The chain is a multiply-add per chunk, operands are asked for eight chunks ahead in the registers that they have just left, and a SIMD's two
+// waves cover each other.  Bound by the operands' way to the CU (every 16 columns bring 16 KB of q and k a chunk: 17 - 20 bytes per clock) ahead of the MFMAs (68 of 32 clocks on four SIMDs a
+// chunk): 1300 clocks a chunk.  Both launches, us, in brackets with chunk_walk_kernel: HGRN2 16 heads 128 x 128, 1021 rows 57 (69), Mamba-2 64 heads 128 x 64 57 (76).
+// With four waves and a barrier per chunk (chunk_walk_kernel, which the delta rule and larger D keep) a chunk's products, the barrier and the sums over the waves stood one after the
+// other, 2100 clocks a chunk.  Tried on the way: a wave per chunk with all rows of the state, the state handed on through LDS (63 and 63; four waves 66 and 70: LDS and the fold beside idle MFMAs).
+constexpr int SCAN = 8; // chunks at a time, waves
+template <int DT, int MODE, int TILES>
+__global__ __launch_bounds__(64 * SCAN) void chunk_scan_kernel(const ChunkArgs a)
+{
+    static_assert(MODE != DELTA && TILES <= 2, "u hangs on the state; a wave per tile");
+    constexpr int D = TILES * 64, NT = TILES * 4;
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    f32x4* part = reinterpret_cast<f32x4*>(sm);  // [2][8][NT][64] q S by turn, chunk, tile, lane
+    f32x4* us = part + 2 * SCAN * NT * 64;       // [2][8][64] u by turn and chunk, SSM: dt_s f_{s+1} ... f_16 u
+    const int e = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c16 = lane & 15, g4 = lane >> 4;
+    const int v = blockIdx.z * 16 + c16, V = a.V, vc = v < V ? v : V - 1;
+    const int first = a.ent_first[e], count = a.ent_count[e], last = (count + R - 1) / R - 1;
+    if (last < 0)
+        return;
+    const int64_t slot0 = first / R + e;
+    const int grp = MODE == SSM ? h / (a.heads / a.groups) : 0;
+    const int tile = NT == SCAN ? wid : wid % NT; // (waves beyond the tiles go along; what they form is not used)
+    float* st = a.state + (((int64_t) a.ent_slot[e] * a.heads + h) * D + 16 * tile + 4 * g4) * V + v;
+    const bool live = v < V, carry = a.ent_pos0[e] > 0;
+
+    f32x4 S;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        S[i] = live && carry ? st[(int64_t) i * V] : 0.f;
+    const float dsk = MODE == SSM ? a.d_skip[h] : 0.f;
+
+    typedef typename std::conditional<DT == DT_BF16, uint16_t, float>::type Raw;
+    const Raw* vsrc = reinterpret_cast<const Raw*>(MODE == HGRN ? a.proj : a.xbc);
+    const int64_t vld = MODE == HGRN ? a.ldp : a.ldx;
+    const int64_t vcol = (MODE == HGRN ? 2 * a.heads * D : 0) + h * V + vc;
+    f32x4 kt[SCAN], q[SCAN], b[SCAN], p, bt, ws; // by chunk, of this wave's tile; of this wave's chunk
+    Raw vr[4], zr[4];
+    auto row_of = [&](int j, int i) { return (int64_t) (first + min(j * R + 4 * g4 + i, count - 1)); };
+    auto request_kt = [&](int c, int j) {
+        const int64_t kg = MODE == SSM ? (slot0 + j) * a.groups + grp : (slot0 + j) * a.heads + h;
+        kt[c] = *reinterpret_cast<const f32x4*>(a.kt + kg * D * R + (16 * tile + c16) * R + 4 * g4);
+    };
+    auto request_q = [&](int c, int j) {
+        const int64_t ch = (slot0 + j) * a.heads + h, kg = MODE == SSM ? (slot0 + j) * a.groups + grp : ch;
+        q[c] = *reinterpret_cast<const f32x4*>(a.qt + kg * R * D + c16 * D + 16 * tile + 4 * g4);
+        if constexpr (MODE == SSM)
+            b[c][0] = a.bc[ch * 48 + 2 * R];
+        else
+            b[c] = *reinterpret_cast<const f32x4*>(a.bc + ch * D + 16 * tile + 4 * g4);
+    };
+    auto leave_part = [&](int turn, int c, const f32x4& o) {
+        if (NT == SCAN || wid < NT)
+            part[((turn * SCAN + c) * NT + tile) * 64 + lane] = o;
+    };
+    auto request_u = [&](int j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            vr[i] = vsrc[row_of(j, i) * vld + vcol];
+        if constexpr (MODE == SSM)
+            ws = *reinterpret_cast<const f32x4*>(a.bc + ((slot0 + j) * a.heads + h) * 48 + R + 4 * g4);
+    };
+    auto request_output = [&](int j) {
+        const int64_t ch = (slot0 + j) * a.heads + h;
+        p = *reinterpret_cast<const f32x4*>(a.pm + ch * R * R + c16 * R + 4 * g4);
+        if constexpr (MODE == SSM)
+        {
+            bt = *reinterpret_cast<const f32x4*>(a.bc + ch * 48 + 4 * g4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                zr[i] = reinterpret_cast<const Raw*>(a.proj)[row_of(j, i) * a.ldp + h * V + vc];
+        }
+    };
+    auto cvt = [](Raw r) -> float {
+        if constexpr (DT == DT_BF16)
+            return bf2f(r);
+        else
+            return r;
+    };
+    // this wave's chunk's u, for all tiles
+    auto leave_u = [&](int turn) {
+        f32x4 u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            u[i] = cvt(vr[i]);
+        us[(turn * SCAN + wid) * 64 + lane] = MODE == SSM ? u * ws : u;
+        return u;
+    };
+
+    request_u(min(wid, last));
+    __builtin_amdgcn_sched_barrier(0); // (requests in the order in which they are used: the waits count them)
+#pragma unroll
+    for (int c = 0; c < SCAN; ++c)
+    {
+        if (c == 0)
+            request_kt(0, 0);
+        request_q(c, min(c, last));
+        if (c + 1 < SCAN)
+            request_kt(c + 1, min(c + 1, last));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    request_output(min(wid, last));
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 u = leave_u(0);
+    __syncthreads();
+    for (int j0 = 0, turn = 0; j0 <= last; j0 += SCAN, turn ^= 1)
+    {
+        const int j = j0 + wid, next = min(j + SCAN, last); // (past the end the last chunk's operands, nothing of which counts)
+        request_u(next);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 uc[SCAN];
+#pragma unroll
+        for (int c = 0; c < SCAN; ++c)
+            uc[c] = us[(turn * SCAN + c) * 64 + lane];
+        // chunk c's q S beside chunk c + 1's K^T U: what S waits for was formed a chunk ahead
+        f32x4 x = {0.f, 0.f, 0.f, 0.f}, o_before = x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            x = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[0][i], uc[0][i], x, 0, 0, 0);
+        request_kt(0, min(j0 + SCAN, last));
+#pragma unroll
+        for (int c = 0; c < SCAN; ++c)
+        {
+            f32x4 o = {0.f, 0.f, 0.f, 0.f}, x_next = o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                o = __builtin_amdgcn_mfma_f32_16x16x4f32(q[c][i], S[i], o, 0, 0, 0);
+                if (c + 1 < SCAN)
+                    x_next = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[c + 1][i], uc[c + 1][i], x_next, 0, 0, 0);
+            }
+            const f32x4 after = MODE == SSM ? S * b[c][0] + x : S * b[c] + x;
+            S = j0 + c <= last ? after : S;
+            if (c > 0)
+                leave_part(turn, c - 1, o_before);
+            x = x_next;
+            o_before = o;
+            __builtin_amdgcn_sched_barrier(0);
+            const int after_j = min(j0 + SCAN + c, last);
+            request_q(c, after_j);
+            if (c + 1 < SCAN)
+                request_kt(c + 1, min(j0 + SCAN + c + 1, last));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        leave_part(turn, SCAN - 1, o_before);
+        const f32x4 u_next = leave_u(turn ^ 1);
+        __syncthreads();
+        f32x4 past = part[(turn * SCAN + wid) * NT * 64 + lane];
+#pragma unroll
+        for (int n = 1; n < NT; ++n)
+            past = past + part[((turn * SCAN + wid) * NT + n) * 64 + lane];
+        if constexpr (MODE == SSM)
+            past = past * bt;
+        f32x4 y = past;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            y = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i], u[i], y, 0, 0, 0);
+        // the zeros of P above its diagonal meet every row: as in chunk_walk_kernel, a chunk with an infinity or a NaN row by row
+        if (any_large(u))
+            y = lower_product(p, u, 0, 4, past);
+        if constexpr (MODE == SSM)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                const float z = cvt(zr[i]);
+                y[i] = fmaf(dsk, u[i], y[i]) * (z / (1.f + expf(-z)));
+            }
+        if (live && j <= last)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (j * R + 4 * g4 + i < count)
+                    a.out[(int64_t) (first + j * R + 4 * g4 + i) * (a.heads * V) + h * V + v] = y[i];
+        __builtin_amdgcn_sched_barrier(0);
+        request_output(next);
+        __builtin_amdgcn_sched_barrier(0);
+        u = u_next;
+    }
+    if (live && wid < NT)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            st[(int64_t) i * V] = S[i];
+}
+
 inline int launched(const char* what)
 {
     const hipError_t e = hipGetLastError();
@@ -622,6 +807,15 @@ template <int DT, int MODE>
 void walk(const ChunkArgs& a, hipStream_t stream)
 {
     const dim3 grid(a.entries, a.heads, (a.V + 15) / 16);
+    if constexpr (MODE != DELTA)
+        if (a.D <= 128)
+        {
+            const auto kernel = a.D == 64 ? chunk_scan_kernel<DT, MODE, 1> : chunk_scan_kernel<DT, MODE, 2>;
+            const size_t lds = sizeof(f32x4) * 2 * SCAN * 64 * ((size_t) a.D / 16 + 1);
+            launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
+            hipLaunchKernelGGL(kernel, grid, dim3(64 * SCAN), lds, stream, a);
+            return;
+        }
     switch (a.D / 64)
     {
     case 1: hipLaunchKernelGGL((chunk_walk_kernel<DT, MODE, 1>), grid, dim3(256), 0, stream, a); break;
