@@ -11,13 +11,13 @@
 // mode) in both element types.
 //
 // Two launches.  chunk_prepare_kernel / ssm_prepare_kernel: a workgroup per (chunk, head), resp. (chunk, group), all chunks at once: gates, unit
-// norms, the decayed vectors, P, M and T into scratch.  chunk_scan_kernel (HGRN2 and Mamba-2 with D up to 128) or chunk_walk_kernel: a workgroup per (entry, head, 16 columns of V) walks the chunks; its
+// norms, the decayed vectors, P, M and T into scratch.  chunk_scan_kernel (HGRN2 and Mamba-2 with D up to 128), chunk_walk_kernel (beyond) and delta_walk_kernel: a workgroup per (entry, head, 16 columns of V) walks the chunks; its
 // four waves keep the state's rows in turn, 16 at a time, in registers in the MFMA's accumulator layout (lane: column lane & 15, rows 4 (lane >> 4)
 // + i), which is also its B-operand layout when the four K = 4 steps of 16 rows take rows 4 g + i in step i: S, u and v go from product to
 // product without moving, and what comes from scratch is 16 bytes per lane.  One barrier per chunk, where the waves' partial o (and S^T k)
 // meet; the next chunk's operands are in flight under this one's products.
 //
-// Measured (us, both launches, 16 heads): HGRN2 128 x 128, 1024 rows 1024 -> 57; delta rule 128 x 128, three prompts of 683 rows in all 1740 1193 -> 123;
+// Measured (us, both launches, 16 heads): HGRN2 128 x 128, 1024 rows 1024 -> 57; delta rule 128 x 128, three prompts of 683 rows in all 1740 1193 -> 109;
 // Mamba-2 64 heads 128 x 64, 1021 rows 400 -> 57.
 #include "dev_utils.h"
 #include "launch_util.h"
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256) void chunk_prepare_kernel(const ChunkArgs a)
 #pragma unroll
         for (int half = 0; half < 2; ++half)
         {
-            const int t = half ? R - 1 - tp : tp;
+            const int t = half ? R - 1 - tp : tp, rows = half ? R : R / 2; // (rows: unrolled, as is half)
             float pa[R], ma[R];
 #pragma unroll
             for (int s = 0; s < R; ++s)
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(256) void chunk_prepare_kernel(const ChunkArgs a)
             {
                 float2 q = *reinterpret_cast<const float2*>(qs + t * D + d), k = *reinterpret_cast<const float2*>(ks + t * D + d);
 #pragma unroll
-                for (int s = R - 1; s >= 0; --s)
+                for (int s = rows - 1; s >= 0; --s)
                 {
                     if (s > t)
                         continue;
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void chunk_prepare_kernel(const ChunkArgs a)
                 }
             }
 #pragma unroll
-            for (int s = 0; s < R; ++s)
+            for (int s = 0; s < rows; ++s)
             {
                 pa[s] = group_sum<32>(pa[s]);
                 if (MODE == DELTA)
@@ -412,11 +412,12 @@ __device__ __forceinline__ f32x4 lower_product(const f32x4& m, const f32x4& x, i
     return acc;
 }
 
-// One workgroup per (entry, head, 16 columns of V): TILES * 64 rows of state (D), wave w keeps rows 16 (w + 4 j) .. + 16
+// HGRN2 and Mamba-2 with D beyond 128.  One workgroup per (entry, head, 16 columns of V): TILES * 64 rows of state (D), wave w keeps rows 16 (w + 4 j) .. + 16
 template <int DT, int MODE, int TILES>
 __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
 {
-    __shared__ f32x4 po[2][4][64], pr[MODE == DELTA ? 2 : 1][MODE == DELTA ? 4 : 1][64];
+    static_assert(MODE != DELTA, "delta_walk_kernel");
+    __shared__ f32x4 po[2][4][64];
     constexpr int D = TILES * 64;
     const int e = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int c16 = lane & 15, g4 = lane >> 4;
@@ -439,14 +440,14 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
     typedef typename std::conditional<DT == DT_BF16, uint16_t, float>::type Raw;
     struct Ops
     {
-        f32x4 q[TILES], kb[MODE == DELTA ? TILES : 1], kt[TILES], b[MODE == SSM ? 1 : TILES], p, t;
+        f32x4 q[TILES], kt[TILES], b[MODE == SSM ? 1 : TILES], p;
         f32x4 bt, ws; // SSM: b_t of this lane's rows, dt_s f_{s+1} ... f_16
         Raw v[4], z;
         float b16;
     };
     const Raw* vsrc = reinterpret_cast<const Raw*>(MODE == HGRN ? a.proj : a.xbc);
     const int64_t vld = MODE == HGRN ? a.ldp : a.ldx;
-    const int64_t vcol = (MODE == HGRN ? 2 * a.heads * D : MODE == DELTA ? 2 * a.qk_heads * D : 0) + h * V + vc;
+    const int64_t vcol = (MODE == HGRN ? 2 * a.heads * D : 0) + h * V + vc;
     auto request = [&](int j, Ops& o) {
         const int64_t slot = slot0 + j, ch = slot * a.heads + h, kg = MODE == SSM ? slot * a.groups + grp : ch;
 #pragma unroll
@@ -457,12 +458,8 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
             o.q[n] = *reinterpret_cast<const f32x4*>(a.qt + (kg * R + c16) * D + d0 + 4 * g4);
             if constexpr (MODE != SSM)
                 o.b[n] = *reinterpret_cast<const f32x4*>(a.bc + ch * D + d0 + 4 * g4);
-            if constexpr (MODE == DELTA)
-                o.kb[n] = *reinterpret_cast<const f32x4*>(a.kb + (ch * R + c16) * D + d0 + 4 * g4);
         }
         o.p = *reinterpret_cast<const f32x4*>(a.pm + ch * R * R + c16 * R + 4 * g4);
-        if constexpr (MODE == DELTA)
-            o.t = *reinterpret_cast<const f32x4*>(a.tm + ch * R * R + c16 * R + 4 * g4);
         if constexpr (MODE == SSM)
         {
             o.bt = *reinterpret_cast<const f32x4*>(a.bc + ch * 48 + 4 * g4);
@@ -488,34 +485,22 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
         for (int i = 0; i < 4; ++i)
             u[i] = cvt(o.v[i]);
         // two sums per product: a product's next step waits for the one before
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc1 = acc, accr = acc, accr1 = acc;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc1 = acc;
 #pragma unroll
         for (int n = 0; n < TILES; ++n)
 #pragma unroll
             for (int i = 0; i < 4; i += 2)
             {
-                if constexpr (MODE == DELTA)
-                {
-                    accr = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kb[n][i], S[n][i], accr, 0, 0, 0);
-                    accr1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kb[n][i + 1], S[n][i + 1], accr1, 0, 0, 0);
-                }
                 acc = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[n][i], S[n][i], acc, 0, 0, 0);
                 acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[n][i + 1], S[n][i + 1], acc1, 0, 0, 0);
             }
         acc = acc + acc1;
-        accr = accr + accr1;
         if constexpr (MODE == SSM)
             acc = acc * o.bt;
         const f32x4 past = acc; // what the rows ahead of the chunk give
-        if constexpr (MODE != DELTA) // this wave's quarter of P u
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pick(o.p, wid), pick(u, wid), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pick(o.p, wid), pick(u, wid), acc, 0, 0, 0); // this wave's quarter of P u
         po[buf][wid][lane] = acc;
-        if constexpr (MODE == DELTA)
-            pr[buf][wid][lane] = accr;
         __syncthreads();
-        f32x4 out = {0.f, 0.f, 0.f, 0.f}, x = u;
-        if constexpr (MODE == DELTA)
-            x = u - ((pr[buf][0][lane] + pr[buf][1][lane]) + (pr[buf][2][lane] + pr[buf][3][lane]));
 #pragma unroll
         for (int n = 0; n < TILES; ++n)
         {
@@ -523,16 +508,6 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
                 S[n] = S[n] * o.b16;
             else
                 S[n] = S[n] * o.b[n];
-        }
-        if constexpr (MODE == DELTA)
-        {
-            u = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                u = __builtin_amdgcn_mfma_f32_16x16x4f32(o.t[i], x[i], u, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                out = __builtin_amdgcn_mfma_f32_16x16x4f32(o.p[i], u[i], out, 0, 0, 0);
         }
         const f32x4 us = MODE == SSM ? u * o.ws : u;
 #pragma unroll
@@ -543,26 +518,18 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
         // wave w finishes rows 4 g + w
         const float* pf = reinterpret_cast<const float*>(&po[buf][0][0]);
         auto waves_sum = [&] { return (pf[lane * 4 + wid] + pf[256 + lane * 4 + wid]) + (pf[512 + lane * 4 + wid] + pf[768 + lane * 4 + wid]); };
-        float y = waves_sum() + pick(out, wid);
-        // The zeros of P and T above their diagonals meet every row in a matrix product, and 0 times an infinity or a NaN is a NaN: where a row
+        float y = waves_sum();
+        // The zeros of P above its diagonal meet every row in a matrix product, and 0 times an infinity or a NaN is a NaN: where a row
         // has one, the outputs are formed again row by row, without what follows a row (the state takes every row in any case).  All waves hold
-        // the same x, so that the branch is the workgroup's.  (Delta rule: u overflows only where x is near it, T's entries are below 2^15.)
+        // the same u, so that the branch is the workgroup's.
         // Asked behind the chunk's products: a branch among them takes the next request's addresses and the state's factors out of their
         // shadow, 60 us for the walk of HGRN2 128 x 128 over 1024 rows instead of 50.
-        if (any_large(x))
+        if (any_large(u))
         {
-            if constexpr (MODE == DELTA)
-            {
-                const f32x4 none = {0.f, 0.f, 0.f, 0.f};
-                y = waves_sum() + pick(lower_product(o.p, lower_product(o.t, x, 0, 4, none), 0, 4, none), wid);
-            }
-            else
-            {
-                __syncthreads(); // (every wave has read the sums above)
-                po[buf][wid][lane] = lower_product(o.p, x, wid, wid + 1, past);
-                __syncthreads();
-                y = waves_sum();
-            }
+            __syncthreads(); // (every wave has read the sums above)
+            po[buf][wid][lane] = lower_product(o.p, u, wid, wid + 1, past);
+            __syncthreads();
+            y = waves_sum();
         }
         const int row = j * R + 4 * g4 + wid;
         if constexpr (MODE == SSM)
@@ -607,12 +574,194 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
     }
 }
 
+// The walk of the delta rule, whose u hangs on the state: one workgroup per (entry, head, 16 columns of V), wave w keeps rows 16 (w + 4 j) .. + 16 of the state.  The chain of a chunk is
+// (b k)^T S of a wave's rows, their sum over the waves through LDS, T on what is left of v, and S's update; everything else stands beside it: q's product with S covers the way
+// through LDS, a wave adds its quarter of P u to it, and the sums over the waves become outputs a chunk later, behind that chunk's one barrier.  With everything in the order of the formulas
+// and three sets of operands 1.35 us a chunk where a CU has one workgroup, here 1.15 (a chunk brings 27 KB).  Both launches, us, in brackets that form: 16 heads 128 x 128, one prompt of 683 rows 67 (76), three of
+// 1672 in all 96 (108), 24 heads 136 (158), eight of 240 92 (100).  32 columns a workgroup, which halve what its operands bring, made the chain longer: 109, 120, 167, 89.
+template <int DT, int TILES>
+__global__ __launch_bounds__(256, 2) void delta_walk_kernel(const ChunkArgs a)
+{
+    __shared__ f32x4 po[2][4][64], pr[2][4][64];
+    constexpr int D = TILES * 64;
+    const int e = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c16 = lane & 15, g4 = lane >> 4;
+    const int v = blockIdx.z * 16 + c16, V = a.V, vc = v < V ? v : V - 1;
+    const int first = a.ent_first[e], count = a.ent_count[e], last = (count + R - 1) / R - 1;
+    if (last < 0)
+        return;
+    const int64_t slot0 = first / R + e;
+    float* st = a.state + ((int64_t) a.ent_slot[e] * a.heads + h) * D * V;
+    const bool live = v < V, carry = a.ent_pos0[e] > 0;
+
+    f32x4 S[TILES];
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            S[j][i] = live && carry ? st[(int64_t) (16 * (wid + 4 * j) + 4 * g4 + i) * V + v] : 0.f;
+
+    // a chunk's operands as this lane holds them; `raw` ones are converted where they are used, so that nothing waits at its load
+    typedef typename std::conditional<DT == DT_BF16, uint16_t, float>::type Raw;
+    struct Ops
+    {
+        f32x4 q[TILES], kb[TILES], kt[TILES], b[TILES], p, t;
+        Raw v[4];
+    };
+    const Raw* vsrc = reinterpret_cast<const Raw*>(a.xbc) + 2 * a.qk_heads * D + h * V + vc;
+    const int64_t vrow0 = (int64_t) first * a.ldx;
+    auto request_kb = [&](int j, Ops& o) {
+        const float* kb = a.kb + ((slot0 + j) * a.heads + h) * R * D;
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
+            o.kb[n] = *reinterpret_cast<const f32x4*>(kb + c16 * D + 16 * (wid + 4 * n) + 4 * g4);
+    };
+    auto request_q = [&](int j, Ops& o) {
+        const float* q = a.qt + ((slot0 + j) * a.heads + h) * R * D;
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
+            o.q[n] = *reinterpret_cast<const f32x4*>(q + c16 * D + 16 * (wid + 4 * n) + 4 * g4);
+    };
+    auto request_v = [&](int j, Ops& o) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            o.v[i] = vsrc[vrow0 + (int64_t) min(j * R + 4 * g4 + i, count - 1) * a.ldx];
+        o.t = *reinterpret_cast<const f32x4*>(a.tm + ((slot0 + j) * a.heads + h) * R * R + c16 * R + 4 * g4);
+    };
+    auto request_k = [&](int j, Ops& o) {
+        const int64_t ch = (slot0 + j) * a.heads + h;
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
+        {
+            o.b[n] = *reinterpret_cast<const f32x4*>(a.bc + ch * D + 16 * (wid + 4 * n) + 4 * g4);
+            o.kt[n] = *reinterpret_cast<const f32x4*>(a.kt + (ch * D + 16 * (wid + 4 * n) + c16) * R + 4 * g4);
+        }
+        o.p = *reinterpret_cast<const f32x4*>(a.pm + ch * R * R + c16 * R + 4 * g4);
+    };
+    auto cvt = [](Raw r) -> float {
+        if constexpr (DT == DT_BF16)
+            return bf2f(r);
+        else
+            return r;
+    };
+    // wave w finishes rows 4 g + w of chunk j, behind a barrier that its sums are ahead of
+    auto finish = [&](int j) {
+        const float* pf = reinterpret_cast<const float*>(&po[j & 1][0][0]);
+        const float y = (pf[lane * 4 + wid] + pf[256 + lane * 4 + wid]) + (pf[512 + lane * 4 + wid] + pf[768 + lane * 4 + wid]);
+        const int row = j * R + 4 * g4 + wid;
+        if (live && row < count)
+            a.out[(int64_t) (first + row) * (a.heads * V) + h * V + v] = y;
+    };
+
+    auto chunk = [&](int j, int buf, Ops& o) {
+        const int next = min(j + 2, last);
+        // two sums per product: a product's next step waits for the one before
+        f32x4 accr = {0.f, 0.f, 0.f, 0.f}, accr1 = accr, acc = accr, acc1 = accr;
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2)
+            {
+                accr = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kb[n][i], S[n][i], accr, 0, 0, 0);
+                accr1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kb[n][i + 1], S[n][i + 1], accr1, 0, 0, 0);
+            }
+        pr[buf][wid][lane] = accr + accr1;
+        __builtin_amdgcn_sched_barrier(0);
+        request_kb(next, o);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        const f32x4 r0 = pr[buf][0][lane], r1 = pr[buf][1][lane], r2 = pr[buf][2][lane], r3 = pr[buf][3][lane];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2)
+            {
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[n][i], S[n][i], acc, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[n][i + 1], S[n][i + 1], acc1, 0, 0, 0);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            x[i] = cvt(o.v[i]) - ((r0[i] + r1[i]) + (r2[i] + r3[i]));
+        f32x4 u = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            u = __builtin_amdgcn_mfma_f32_16x16x4f32(o.t[i], x[i], u, 0, 0, 0);
+        acc = acc + acc1;
+#pragma unroll
+        for (int n = 0; n < TILES; ++n)
+            S[n] = S[n] * o.b[n];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int n = 0; n < TILES; ++n)
+                S[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kt[n][i], u[i], S[n], 0, 0, 0);
+        f32x4 part = __builtin_amdgcn_mfma_f32_16x16x4f32(pick(o.p, wid), pick(u, wid), acc, 0, 0, 0); // with this wave's quarter of P u
+        // The zeros of P and T above their diagonals meet every row in a matrix product, and 0 times an infinity or a NaN is a NaN: where a row
+        // has one, P u is formed again row by row, without what follows a row (the state takes every row in any case).  All waves hold
+        // the same x.  (u overflows only where x is near it, T's entries are below 2^15.)
+        if (any_large(x))
+        {
+            const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+            part = wid == 0 ? lower_product(o.p, lower_product(o.t, x, 0, 4, none), 0, 4, acc) : acc;
+        }
+        po[buf][wid][lane] = part;
+        __builtin_amdgcn_sched_barrier(0);
+        request_q(next, o);
+        __builtin_amdgcn_sched_barrier(0);
+        request_v(next, o);
+        __builtin_amdgcn_sched_barrier(0);
+        request_k(next, o);
+        __builtin_amdgcn_sched_barrier(0);
+        if (j > 0)
+            finish(j - 1);
+    };
+
+    // Two sets of operands, each requested again as it is used, two chunks ahead and in that order: the waits count.  Every request is made (past the end the last chunk's once more):
+    // one under a condition would have the compiler wait as if it had not been made, for all that is in flight.
+    Ops o0, o1;
+    auto request = [&](int j, Ops& o) {
+        request_kb(j, o);
+        __builtin_amdgcn_sched_barrier(0);
+        request_q(j, o);
+        __builtin_amdgcn_sched_barrier(0);
+        request_v(j, o);
+        __builtin_amdgcn_sched_barrier(0);
+        request_k(j, o);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    request(0, o0);
+    request(min(1, last), o1);
+    for (int j = 0;; j += 2)
+    {
+        chunk(j, 0, o0);
+        if (j + 1 > last)
+            break;
+        chunk(j + 1, 1, o1);
+        if (j + 2 > last)
+            break;
+    }
+    __syncthreads();
+    finish(last);
+    if (live)
+    {
+#pragma unroll
+        for (int j = 0; j < TILES; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                st[(int64_t) (16 * (wid + 4 * j) + 4 * g4 + i) * V + v] = S[j][i];
+    }
+}
+
 // The walk of HGRN2 and Mamba-2, where what a chunk adds to the state does not hang on the state (u is there from the start): one workgroup per (entry, head, 16 columns of V), eight
 // chunks between two barriers, D up to 128.  Wave w carries tile w of the state (16 rows) through the eight: K^T U of its rows, q S of its rows into LDS, S <- b S + K^T U; behind the barrier
 // it sums chunk w's parts and finishes its rows.  The chain is a multiply-add per chunk, operands are asked for eight chunks ahead in the registers that they have just left, and a SIMD's two
 // waves cover each other.  Bound by the operands' way to the CU (every 16 columns bring 16 KB of q and k a chunk: 17 - 20 bytes per clock) ahead of the MFMAs (68 of 32 clocks on four SIMDs a
 // chunk): 1300 clocks a chunk.  Both launches, us, in brackets with chunk_walk_kernel: HGRN2 16 heads 128 x 128, 1021 rows 57 (69), Mamba-2 64 heads 128 x 64 57 (76).
-// With four waves and a barrier per chunk (chunk_walk_kernel, which the delta rule and larger D keep) a chunk's products, the barrier and the sums over the waves stood one after the
+// With four waves and a barrier per chunk (chunk_walk_kernel, which larger D keep) a chunk's products, the barrier and the sums over the waves stood one after the
 // other, 2100 clocks a chunk.  Tried on the way: a wave per chunk with all rows of the state, the state handed on through LDS (63 and 63; four waves 66 and 70: LDS and the fold beside idle MFMAs).
 constexpr int SCAN = 8; // chunks at a time, waves
 template <int DT, int MODE, int TILES>
@@ -816,13 +965,17 @@ void walk(const ChunkArgs& a, hipStream_t stream)
             hipLaunchKernelGGL(kernel, grid, dim3(64 * SCAN), lds, stream, a);
             return;
         }
-    switch (a.D / 64)
-    {
-    case 1: hipLaunchKernelGGL((chunk_walk_kernel<DT, MODE, 1>), grid, dim3(256), 0, stream, a); break;
-    case 2: hipLaunchKernelGGL((chunk_walk_kernel<DT, MODE, 2>), grid, dim3(256), 0, stream, a); break;
-    case 3: hipLaunchKernelGGL((chunk_walk_kernel<DT, MODE, 3>), grid, dim3(256), 0, stream, a); break;
-    default: hipLaunchKernelGGL((chunk_walk_kernel<DT, MODE, 4>), grid, dim3(256), 0, stream, a); break;
-    }
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a); };
+    if constexpr (MODE == DELTA)
+        switch (a.D / 64)
+        {
+        case 1: return go(delta_walk_kernel<DT, 1>);
+        case 2: return go(delta_walk_kernel<DT, 2>);
+        case 3: return go(delta_walk_kernel<DT, 3>);
+        default: return go(delta_walk_kernel<DT, 4>);
+        }
+    else
+        a.D == 192 ? go(chunk_walk_kernel<DT, MODE, 3>) : go(chunk_walk_kernel<DT, MODE, 4>);
 }
 
 template <int DT, int MODE>
