@@ -108,7 +108,7 @@ def test_a_row_without_finite_numbers_leaves_the_earlier_ones_alone(kind, dtype,
     check_request(mod, kind, got['b'], other, w, cfg, dtype, 'b')
 
 
-# Eight chunks between two barriers (chunk_scan_kernel, dim up to 128): portions that end in, on and behind an eighth chunk, one that begins with carried state, waves without a chunk.
+# Eight chunks between two barriers (eight_chunk_walk_kernel, dim up to 128): portions that end in, on and behind an eighth chunk, one that begins with carried state, waves without a chunk.
 @pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
 @pytest.mark.parametrize('dim,vdim', [(64, 24), (128, 16)])
 @pytest.mark.parametrize('kind', ['hgrn2', 'mamba2'])

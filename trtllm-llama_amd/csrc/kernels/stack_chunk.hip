@@ -11,7 +11,7 @@
 // mode) in both element types.
 //
 // Two launches.  chunk_prepare_kernel / ssm_prepare_kernel: a workgroup per (chunk, head), resp. (chunk, group), all chunks at once: gates, unit
-// norms, the decayed vectors, P, M and T into scratch.  chunk_scan_kernel (HGRN2 and Mamba-2 with D up to 128), chunk_walk_kernel (beyond) and delta_walk_kernel: a workgroup per (entry, head, 16 columns of V) walks the chunks; its
+// norms, the decayed vectors, P, M and T into scratch.  eight_chunk_walk_kernel (HGRN2 and Mamba-2 with D up to 128), chunk_walk_kernel (beyond) and delta_chunk_walk_kernel: a workgroup per (entry, head, 16 columns of V) walks the chunks; its
 // four waves keep the state's rows in turn, 16 at a time, in registers in the MFMA's accumulator layout (lane: column lane & 15, rows 4 (lane >> 4)
 // + i), which is also its B-operand layout when the four K = 4 steps of 16 rows take rows 4 g + i in step i: S, u and v go from product to
 // product without moving, and what comes from scratch is 16 bytes per lane.  One barrier per chunk, where the waves' partial o (and S^T k)
@@ -416,7 +416,7 @@ __device__ __forceinline__ f32x4 lower_product(const f32x4& m, const f32x4& x, i
 template <int DT, int MODE, int TILES>
 __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
 {
-    static_assert(MODE != DELTA, "delta_walk_kernel");
+    static_assert(MODE != DELTA, "delta_chunk_walk_kernel");
     __shared__ f32x4 po[2][4][64];
     constexpr int D = TILES * 64;
     const int e = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -580,7 +580,7 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
 // and three sets of operands 1.35 us a chunk where a CU has one workgroup, here 1.15 (a chunk brings 27 KB).  Both launches, us, in brackets that form: 16 heads 128 x 128, one prompt of 683 rows 67 (76), three of
 // 1672 in all 96 (108), 24 heads 136 (158), eight of 240 92 (100).  32 columns a workgroup, which halve what its operands bring, made the chain longer: 109, 120, 167, 89.
 template <int DT, int TILES>
-__global__ __launch_bounds__(256, 2) void delta_walk_kernel(const ChunkArgs a)
+__global__ __launch_bounds__(256, 2) void delta_chunk_walk_kernel(const ChunkArgs a)
 {
     __shared__ f32x4 po[2][4][64], pr[2][4][64];
     constexpr int D = TILES * 64;
@@ -765,7 +765,7 @@ __global__ __launch_bounds__(256, 2) void delta_walk_kernel(const ChunkArgs a)
 // other, 2100 clocks a chunk.  Tried on the way: a wave per chunk with all rows of the state, the state handed on through LDS (63 and 63; four waves 66 and 70: LDS and the fold beside idle MFMAs).
 constexpr int SCAN = 8; // chunks at a time, waves
 template <int DT, int MODE, int TILES>
-__global__ __launch_bounds__(64 * SCAN) void chunk_scan_kernel(const ChunkArgs a)
+__global__ __launch_bounds__(64 * SCAN) void eight_chunk_walk_kernel(const ChunkArgs a)
 {
     static_assert(MODE != DELTA && TILES <= 2, "u hangs on the state; a wave per tile");
     constexpr int D = TILES * 64, NT = TILES * 4;
@@ -959,7 +959,7 @@ void walk(const ChunkArgs& a, hipStream_t stream)
     if constexpr (MODE != DELTA)
         if (a.D <= 128)
         {
-            const auto kernel = a.D == 64 ? chunk_scan_kernel<DT, MODE, 1> : chunk_scan_kernel<DT, MODE, 2>;
+            const auto kernel = a.D == 64 ? eight_chunk_walk_kernel<DT, MODE, 1> : eight_chunk_walk_kernel<DT, MODE, 2>;
             const size_t lds = sizeof(f32x4) * 2 * SCAN * 64 * ((size_t) a.D / 16 + 1);
             launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
             hipLaunchKernelGGL(kernel, grid, dim3(64 * SCAN), lds, stream, a);
@@ -969,10 +969,10 @@ void walk(const ChunkArgs& a, hipStream_t stream)
     if constexpr (MODE == DELTA)
         switch (a.D / 64)
         {
-        case 1: return go(delta_walk_kernel<DT, 1>);
-        case 2: return go(delta_walk_kernel<DT, 2>);
-        case 3: return go(delta_walk_kernel<DT, 3>);
-        default: return go(delta_walk_kernel<DT, 4>);
+        case 1: return go(delta_chunk_walk_kernel<DT, 1>);
+        case 2: return go(delta_chunk_walk_kernel<DT, 2>);
+        case 3: return go(delta_chunk_walk_kernel<DT, 3>);
+        default: return go(delta_chunk_walk_kernel<DT, 4>);
         }
     else
         a.D == 192 ? go(chunk_walk_kernel<DT, MODE, 3>) : go(chunk_walk_kernel<DT, MODE, 4>);
