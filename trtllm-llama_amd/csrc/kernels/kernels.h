@@ -527,6 +527,8 @@ int launch_beam_step(const BeamParams& p, hipStream_t stream);
 int launch_fill_random(void* dst, int32_t dtype, int64_t n, uint32_t seed, float scale, hipStream_t stream);
 // int32 fill
 int launch_fill_i32(int32_t* dst, int32_t value, int64_t n, hipStream_t stream);
+// dst[i] = host_src[i] of pinned host memory, n a multiple of 4, both 16-byte aligned
+int launch_fetch(int32_t* dst, const int32_t* host_src, int64_t n, hipStream_t stream);
 
 } // namespace kernels
 } // namespace tllm

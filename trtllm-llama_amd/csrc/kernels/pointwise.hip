@@ -849,6 +849,13 @@ __global__ __launch_bounds__(256) void fill_random_kernel(void* dst, int dtype, 
     }
 }
 
+__global__ __launch_bounds__(256) void fetch_ints_kernel(int4* dst, const int4* src, int64_t n4)
+{
+    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+    if (i < n4)
+        dst[i] = src[i];
+}
+
 __global__ void fill_i32_kernel(int32_t* dst, int32_t v, int64_t n)
 {
     for (int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t) gridDim.x * blockDim.x)
@@ -1129,6 +1136,19 @@ int launch_fill_random(void* dst, int32_t dtype, int64_t n, uint32_t seed, float
         return 0;
     hipLaunchKernelGGL(fill_random_kernel, dim3(grid_for(n)), dim3(256), 0, stream, dst, dtype, n, seed, scale);
     return check_launch("fill_random");
+}
+
+int launch_fetch(int32_t* dst, const int32_t* host_src, int64_t n, hipStream_t stream)
+{
+    if (n <= 0)
+        return 0;
+    if (n % 4 || ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(host_src)) & 15))
+    {
+        set_error("fetch: %lld values, not in whole 16-byte pieces", (long long) n);
+        return -1;
+    }
+    hipLaunchKernelGGL(fetch_ints_kernel, dim3((unsigned) ((n / 4 + 255) / 256)), dim3(256), 0, stream, reinterpret_cast<int4*>(dst), reinterpret_cast<const int4*>(host_src), n / 4);
+    return check_launch("fetch");
 }
 
 int launch_fill_i32(int32_t* dst, int32_t value, int64_t n, hipStream_t stream)

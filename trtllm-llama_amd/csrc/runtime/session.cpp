@@ -220,6 +220,15 @@ struct tllm_session
     // split runs with its own combine launch
     bool attn_tail = false;
     uint32_t* attn_tickets = nullptr;
+    // What a request starts from (lengths, ids, mask, flags) side by side on the device and as the host writes it, in pinned memory: one launch brings it over
+    int32_t *start_dev = nullptr, *start_host = nullptr;
+    size_t start_ints = 0;
+    bool start_read = false;         // a launch on start_stream reads start_host, or has read it
+    hipStream_t start_stream = nullptr;
+    int32_t* start_of(const void* dev) const
+    {
+        return start_host + (static_cast<const int32_t*>(dev) - start_dev);
+    }
     // r05: batch-1 greedy decode of a SmoothQuant engine runs the QKV projection, RoPE, the cache append and the attention of a head
     // in ONE launch (kernels/qkv_attn_fused.hip); session key fuse_qkv_attention = 0 keeps the two launches (A/B, parity tests)
     int fuse_qkv_cfg = -1;          // -1 auto, 0 off
@@ -248,6 +257,7 @@ struct tllm_session
     int end_id = -1;
     hipGraphExec_t graph = nullptr;
     hipStream_t graph_stream = nullptr;
+    int graph_end_id = -1;         // baked into the captured sampler node
     uint64_t graph_comm_gen = 0;   // comm::p2p::generation() the step graph was captured under
     uint64_t comm_err_seen = 0;    // comm::p2p::error_generation() at this session's last check_comm
     hipStream_t own_stream = nullptr; // used when the caller passes the NULL stream (it cannot be captured)
@@ -303,6 +313,7 @@ struct tllm_session
             (void) hipStreamDestroy(own_stream);
         if (graph)
             (void) hipGraphExecDestroy(graph);
+        free_start();
         for (auto p : allocs)
             (void) hipFree(p);
         for (auto& kv : tensors)
@@ -332,9 +343,20 @@ struct tllm_session
             (void) hipGraphExecDestroy(graph);
             graph = nullptr;
         }
+        free_start();
         for (auto p : allocs)
             (void) hipFree(p);
         allocs.clear();
+    }
+
+    void free_start()
+    {
+        if (start_read)
+            (void) hipDeviceSynchronize(); // (a request may still be under way)
+        if (start_host)
+            (void) hipHostFree(start_host);
+        start_read = false;
+        start_host = nullptr;
     }
 
     const TensorRec* find(const std::string& name, bool required = true)
@@ -1719,17 +1741,27 @@ int32_t tllm_session_setup_beam(tllm_session_t s, int32_t batch_size, int32_t be
             HIP_OK(hipMemset(s->tap_buf[w], 0, nb));
         }
     }
-    RUN(s->dalloc(&s->cu_dev, (size_t) (Bc + 1) * 4));
-    RUN(s->dalloc(&s->last_rows, (size_t) Bc * 4));
     RUN(s->dalloc(&s->mmha_ws, mmha_workspace_size(B, s->Hr, s->Dh, Smax) + 256));
     HIP_OK(hipMemset(s->mmha_ws, 0, mmha_workspace_size(B, s->Hr, s->Dh, Smax) + 256));
-    RUN(s->dalloc(&s->ids_in, M * 4));
     RUN(s->dalloc(&s->cur_ids, (size_t) B * 4));
-    RUN(s->dalloc(&s->out_ids, (size_t) B * Smax * 4));
-    RUN(s->dalloc(&s->seq_len, (size_t) B * 4));
-    RUN(s->dalloc(&s->in_len, (size_t) B * 4));
-    RUN(s->dalloc(&s->last_tok, (size_t) Bc * 4));
-    RUN(s->dalloc(&s->in_len_ctx, (size_t) Bc * 4));
+    {
+        // (the prompts' ids last: of packed ones fewer are brought)
+        std::vector<std::pair<int32_t**, size_t>> parts = {{&s->cu_dev, (size_t) Bc + 1}, {&s->last_rows, (size_t) Bc}, {&s->seq_len, (size_t) B}, {&s->in_len, (size_t) B}, {&s->last_tok, (size_t) Bc},
+            {&s->in_len_ctx, (size_t) Bc}, {&s->finished, (size_t) B}, {reinterpret_cast<int32_t**>(&s->attn_tickets), (size_t) B * s->Hr}, {&s->out_ids, (size_t) B * Smax}, {&s->masked, (size_t) B * Smax},
+            {&s->ids_in, M}};
+        s->start_ints = 0;
+        for (auto& part : parts)
+            s->start_ints += (part.second + 63) / 64 * 64;
+        RUN(s->dalloc(&s->start_dev, s->start_ints * 4));
+        HIP_OK(hipMemset(s->start_dev, 0, s->start_ints * 4));
+        HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&s->start_host), s->start_ints * 4, hipHostMallocDefault));
+        size_t at = 0;
+        for (auto& part : parts)
+        {
+            *part.first = s->start_dev + at;
+            at += (part.second + 63) / 64 * 64;
+        }
+    }
     s->cum_log_probs = nullptr;
     s->parent_ids = s->cache_ind = nullptr;
     if (s->beam > 1)
@@ -1738,8 +1770,6 @@ int32_t tllm_session_setup_beam(tllm_session_t s, int32_t batch_size, int32_t be
         RUN(s->dalloc(&s->parent_ids, (size_t) B * Smax * 4));
         RUN(s->dalloc(&s->cache_ind, (size_t) B * Smax * 4));
     }
-    RUN(s->dalloc(&s->finished, (size_t) B * 4));
-    RUN(s->dalloc(&s->masked, (size_t) B * Smax * 4));
     s->rope = plugins::rope_table(s->Dh, Smax > s->max_pos ? Smax : s->max_pos, &s->rope_len);
     if (!s->rope)
         return 1;
@@ -1756,7 +1786,6 @@ int32_t tllm_session_setup_beam(tllm_session_t s, int32_t batch_size, int32_t be
         size_t off = 0;
         s->attn_tail = false;
         s->attn_nit = 4;
-        s->attn_tickets = nullptr;
         s->ctx_q8 = nullptr;
         if (mmha_split_layout(s->Dh, Smax, 16, B, s->Hr, &tc, &ns, &off) == 0 && ns <= 16)
         {
@@ -1767,8 +1796,6 @@ int32_t tllm_session_setup_beam(tllm_session_t s, int32_t batch_size, int32_t be
             if (mmha_split_layout(s->Dh, Smax, 4, B, s->Hr, &tc, &ns, &off) == 0 && ns == 1)
                 s->attn_nit = 4;
             s->attn_tail = true;
-            RUN(s->dalloc(reinterpret_cast<void**>(&s->attn_tickets), (size_t) B * s->Hr * 4));
-            HIP_OK(hipMemset(s->attn_tickets, 0, (size_t) B * s->Hr * 4));
             RUN(s->dalloc(&s->ctx_q8, (size_t) B * s->Dr));
         }
         if (mmha_split_layout(s->Dh, Smax, s->attn_nit, B, s->Hr, &tc, &ns, &off))
@@ -1942,46 +1969,51 @@ static int upload_prompt(tllm_session_t s, const int32_t* input_ids, const int32
 {
     // input_ids / input_lengths describe the Bc prompts; the per-sequence generation state is tiled over the beam
     // (generation.py:898-915 _tile_beam_width) - the prompt itself runs once per batch entry
+    // One launch from pinned memory: copies of eleven pieces took 50 us and the GPU's commands between them as long again, ahead of a small model's first launch (a request of 7
+    // tokens and 4 new through four layers of 1024: 598 us, 540 so and with its step graph kept).
     const int B = s->B, Bc = s->Bc, W = s->beam, S = s->max_in, Smax = s->Smax;
-    std::vector<int32_t> lens_c(input_lengths, input_lengths + Bc), lens(B), seq(B, S), zeros(B, 0);
-    std::vector<int32_t> mask((size_t) B * Smax, 0), out((size_t) B * Smax, 0);
+    for (int b = 0; b < Bc; ++b)
+        if (input_lengths[b] < 1 || input_lengths[b] > S)
+        {
+            set_error("session: input_lengths[%d]=%d out of range [1, %d]", b, input_lengths[b], S);
+            return 1;
+        }
+    if (s->start_read) // (by the request before)
+        HIP_OK(s->start_stream == st ? hipStreamSynchronize(st) : hipDeviceSynchronize());
+    std::fill_n(s->start_host, s->start_of(s->ids_in) - s->start_host, 0); // (flags, tickets: the in-launch merge re-arms itself per launch, this covers a step that never finished)
+    int32_t *lens = s->start_of(s->in_len), *mask = s->start_of(s->masked), *out = s->start_of(s->out_ids), *ids = s->start_of(s->ids_in);
+    std::fill_n(s->start_of(s->seq_len), B, S);
+    std::copy_n(input_lengths, Bc, s->start_of(s->in_len_ctx));
+    std::copy_n(input_lengths, Bc, s->start_of(s->last_tok));
     for (int bb = 0; bb < B; ++bb)
     {
         const int b = bb / W;
-        lens[bb] = lens_c[b];
-        if (lens[bb] < 1 || lens[bb] > S)
-        {
-            set_error("session: input_lengths[%d]=%d out of range [1, %d]", b, lens[bb], S);
-            return 1;
-        }
+        lens[bb] = input_lengths[b];
         // masked_tokens[b, len_b:max_in] = 1 (generation.py:812-821)
-        for (int t = lens[bb]; t < S; ++t)
-            mask[(size_t) bb * Smax + t] = 1;
-        for (int t = 0; t < S; ++t)
-            out[(size_t) bb * Smax + t] = input_ids[(size_t) b * S + t];
+        std::fill(mask + (size_t) bb * Smax + lens[bb], mask + (size_t) bb * Smax + S, 1);
+        std::copy_n(input_ids + (size_t) b * S, S, out + (size_t) bb * Smax);
     }
-    std::vector<int32_t> packed_ids, cu(Bc + 1, 0), last(Bc, 0);
-    s->pack_now = s->packs(std::accumulate(lens_c.begin(), lens_c.end(), 0));
+    size_t n_ids = (size_t) Bc * S;
+    s->pack_now = s->packs(std::accumulate(input_lengths, input_lengths + Bc, 0));
     if (s->pack_now)
     {
         // the real tokens back to back; generation keeps the padded cache layout (slots [len, max_in) masked), so only
         // the context phase changes shape (generation.py:556-568 with remove_input_padding)
+        int32_t *cu = s->start_of(s->cu_dev), *last = s->start_of(s->last_rows);
         for (int b = 0; b < Bc; ++b)
         {
-            cu[b + 1] = cu[b] + lens_c[b];
+            std::copy_n(input_ids + (size_t) b * S, input_lengths[b], ids + cu[b]);
+            cu[b + 1] = cu[b] + input_lengths[b];
             last[b] = cu[b + 1] - 1;
-            packed_ids.insert(packed_ids.end(), input_ids + (size_t) b * S, input_ids + (size_t) b * S + lens_c[b]);
         }
         s->ctx_tokens = cu[Bc];
-        HIP_OK(hipMemcpyAsync(s->ids_in, packed_ids.data(), packed_ids.size() * 4, hipMemcpyHostToDevice, st));
-        HIP_OK(hipMemcpyAsync(s->cu_dev, cu.data(), cu.size() * 4, hipMemcpyHostToDevice, st));
-        HIP_OK(hipMemcpyAsync(s->last_rows, last.data(), last.size() * 4, hipMemcpyHostToDevice, st));
+        n_ids = cu[Bc];
     }
     else
-        HIP_OK(hipMemcpyAsync(s->ids_in, input_ids, (size_t) Bc * S * 4, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(s->in_len, lens.data(), B * 4, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(s->in_len_ctx, lens_c.data(), Bc * 4, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(s->last_tok, lens_c.data(), Bc * 4, hipMemcpyHostToDevice, st));
+        std::copy_n(input_ids, n_ids, ids);
+    RUN(launch_fetch(s->start_dev, s->start_host, (s->ids_in - s->start_dev) + (int64_t) (n_ids + 3) / 4 * 4, st));
+    s->start_read = true;
+    s->start_stream = st;
     std::vector<float> cum;
     if (W > 1)
     {
@@ -1992,14 +2024,8 @@ static int upload_prompt(tllm_session_t s, const int32_t* input_ids, const int32
         HIP_OK(hipMemcpyAsync(s->cum_log_probs, cum.data(), B * 4, hipMemcpyHostToDevice, st));
         HIP_OK(hipMemsetAsync(s->parent_ids, 0, (size_t) B * Smax * 4, st));
         HIP_OK(hipMemsetAsync(s->cache_ind, 0, (size_t) B * Smax * 4, st)); // every slot -> hypothesis 0's rows
+        HIP_OK(hipStreamSynchronize(st)); // cum goes out of scope
     }
-    HIP_OK(hipMemcpyAsync(s->seq_len, seq.data(), B * 4, hipMemcpyHostToDevice, st));
-    if (s->attn_tickets) // re-arm the in-launch merge (it re-arms itself per launch; this covers a step that never finished)
-        HIP_OK(hipMemsetAsync(s->attn_tickets, 0, (size_t) B * s->Hr * 4, st));
-    HIP_OK(hipMemcpyAsync(s->finished, zeros.data(), B * 4, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(s->masked, mask.data(), mask.size() * 4, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(s->out_ids, out.data(), out.size() * 4, hipMemcpyHostToDevice, st));
-    HIP_OK(hipStreamSynchronize(st)); // the host vectors above go out of scope
     return 0;
 }
 
@@ -2028,7 +2054,7 @@ int32_t tllm_session_step(tllm_session_t s, int32_t n_steps, int32_t use_graph, 
     hipStream_t st = s->pick(stream);
     // a graph captured while the transport was in another state (enabled / fused seam / a re-created region) holds launches
     // that no longer match what an eager step would issue: capture again
-    if (use_graph && (!s->graph || s->graph_stream != st || (s->tp > 1 && s->graph_comm_gen != comm::p2p::generation())))
+    if (use_graph && (!s->graph || s->graph_stream != st || s->graph_end_id != s->end_id || (s->tp > 1 && s->graph_comm_gen != comm::p2p::generation())))
     {
         if (s->graph)
         {
@@ -2054,6 +2080,7 @@ int32_t tllm_session_step(tllm_session_t s, int32_t n_steps, int32_t use_graph, 
             return 1;
         }
         s->graph_stream = st;
+        s->graph_end_id = s->end_id;
         s->graph_comm_gen = comm::p2p::generation();
     }
     for (int i = 0; i < n_steps; ++i)
@@ -2122,9 +2149,10 @@ static int32_t generate_once(tllm_session_t s, const int32_t* input_ids, const i
     }
     hipStream_t st = s->pick(stream);
     s->end_id = end_id;
-    if (s->graph)
+    const bool comm = s->tp > 1 || s->force_comm;
+    if (comm && s->graph)
     {
-        // end_id is baked into the captured sampler node
+        // (its collectives are those of the transport that was in service)
         (void) hipGraphExecDestroy(s->graph);
         s->graph = nullptr;
     }
@@ -2132,8 +2160,8 @@ static int32_t generate_once(tllm_session_t s, const int32_t* input_ids, const i
     int produced = max_new_tokens > 0 ? 1 : 0; // tokens generated per sequence (the prompt pass yields the first)
     if (max_new_tokens > 1)
     {
-        // first generation step eagerly (also warms lazily-initialised state), the rest from the graph
-        RUN(tllm_session_step(s, 1, 0, stream));
+        // the first request's first generation step eagerly (also warms lazily-initialised state), the rest from the graph
+        RUN(tllm_session_step(s, 1, s->graph && s->graph_stream == st, stream));
         produced = 2;
         if (max_new_tokens > 2)
         {
