@@ -35,6 +35,8 @@ int launch_gemm_sqp(const GemmParams& p, int cfg, hipStream_t stream); // gemm_s
 int launch_gemm_f16p(const GemmParams& p, int cfg, hipStream_t stream); // gemm_sqp.hip: the same pipeline on fp16 operands, ids 50..
 int launch_gemm_wide(const GemmParams& p, hipStream_t stream); // gemm_wide.hip: 256 x 256 tiles of both types, id 80
 bool gemm_wide_beats(const GemmParams& p, double other);
+int launch_gemm_rows128(const GemmParams& p, bool wide_cols, hipStream_t stream); // gemm_wide.hip: 128 x 128 and 128 x 256 tiles of both types, ids 81 and 82
+bool gemm_rows128_serves(const GemmParams& p);
 extern void* gemm_clock_probe;                                              // gemm_sqp.hip (microbench hook)
 
 namespace
@@ -52,10 +54,24 @@ struct Shape
 };
 // id 42 is the phased 256 x 128 tile of gemm_sqp.hip (its fp16 sibling is id 54): it has no lock-step form in this file
 constexpr int kPhased256x128 = 42;
+constexpr int kWide = 80, kRows128 = 81, kRows128Wide = 82;
+// The tiles of 128 rows by 16 x 16 MFMAs (gemm_wide_impl.h) take the place of the lock-step ones of 32 x 32 wherever results leave in whole 16-byte pieces of fp16; us, cold weights,
+// in brackets what the rule took without them: SmoothQuant 128 x 128 at 1024 / 512 x 4096 x 4096 21.1 / 16.2 (23.9 / 20.6), 128 x 256 at 1400 and 640 x 11008 x 4096 68 and 34.6 (84.7
+// and 46.3), 2048 x 4096 x 11008 84 (91); fp16 128 x 128 at 997 x 4096 x 11008 104 (108), 300 x 4096 x 4096 28.5 (33.0), 128 x 256 at 1400 and 640 x 11008 x 4096 122 and 63.5 (162 and 81.6).
+// Equal counts of 128 x 256 and 256 x 128 (fp16): 62 / 58 at 512 x 11008 x 4096, 64 / 66 at 2048 x 4096 x 4096.
 constexpr Shape kShapes[] = {{8, 128, 128, 1.40, 1.80}, {6, 256, 192, 1.0, 1.0}, {2, 256, 256, 1.04, 1.30}, {4, 128, 256, 1.39, 1.60},
-    {kPhased256x128, 256, 128, 1.08, 1.37}};
+    {kPhased256x128, 256, 128, 1.08, 1.37}, {kRows128, 128, 128, 1.32, 1.33}, {kRows128Wide, 128, 256, 1.09, 1.10}};
 constexpr int kNumCfg = 12;
-constexpr int kWide = 80;
+
+// the tiles of gemm_wide.hip, ids 80 ..: as launch_gemm_wide
+int launch_wide_cfg(const GemmParams& p, int cfg, hipStream_t stream)
+{
+    return cfg == kWide ? launch_gemm_wide(p, stream) : launch_gemm_rows128(p, cfg == kRows128Wide, stream);
+}
+bool is_wide(int cfg)
+{
+    return cfg >= kWide && cfg <= kRows128Wide;
+}
 
 template <int WT>
 int launch_wt(const GemmParams& p, int cfg, hipStream_t stream)
@@ -113,11 +129,12 @@ static bool glds_serves(const GemmParams& p)
 static int static_shape_cfg(const GemmParams& p, bool phased_ok = true, bool wide_ok = true)
 {
     const int cus = launch_util::device_cus();
+    const bool rows128 = gemm_rows128_serves(p);
     double best = 1e30;
     int cfg = 8;
     for (const Shape& s : kShapes)
     {
-        if (s.id == kPhased256x128 && !phased_ok)
+        if ((s.id == kPhased256x128 && !phased_ok) || (s.bm == 128 && is_wide(s.id) != rows128))
             continue;
         const int64_t tiles = (int64_t) ((p.M + s.bm - 1) / s.bm) * ((p.N + s.bn - 1) / s.bn);
         // beyond two rounds the 256 x 128 tile loses to 256 x 256 / 256 x 192 (M = 8192: 162 vs 136 us on O, 467 vs 377 on gate / up)
@@ -158,8 +175,8 @@ int launch_gemm_cfg(const GemmParams& p, int cfg, hipStream_t stream)
     if (!glds_serves(p))
         return 1;
     const bool sq = p.wtype == W_INT8_SQ;
-    if (cfg == kWide)
-        return launch_gemm_wide(p, stream);
+    if (is_wide(cfg))
+        return launch_wide_cfg(p, cfg, stream);
     if ((cfg >= 1 && cfg <= kNumCfg) || cfg == 36 || cfg == 37)
     {
         // a tile far larger than the problem only burns time in the sweep
@@ -185,7 +202,7 @@ int launch_gemm_glds(const GemmParams& p, hipStream_t stream)
     const bool glds_id = (cfg >= 1 && cfg <= kNumCfg) || cfg == 36 || cfg == 37; // ids served by this file's table
     if (cfg > kNumCfg && !glds_id)
     {
-        const int r = cfg == kWide ? launch_gemm_wide(p, stream) : sq ? launch_gemm_sqp(p, cfg, stream) : launch_gemm_f16p(p, cfg, stream);
+        const int r = is_wide(cfg) ? launch_wide_cfg(p, cfg, stream) : sq ? launch_gemm_sqp(p, cfg, stream) : launch_gemm_f16p(p, cfg, stream);
         if (r <= 0)
             return r;
         cfg = 0; // not served there (shape / alignment): the heuristic below picks a lock-step shape
@@ -193,8 +210,6 @@ int launch_gemm_glds(const GemmParams& p, hipStream_t stream)
     if (cfg <= 0 || !((cfg >= 1 && cfg <= kNumCfg) || cfg == 36 || cfg == 37))
     {
         cfg = static_shape_cfg(p);
-        if (cfg == kWide)
-            return launch_gemm_wide(p, stream);
         if (cfg == kPhased256x128)
         {
             // one round of 256 x 128 tiles where 128 x 128 would take two (O / down at M = 2048: 34 vs 44 us, 84 vs 107 us)
@@ -205,6 +220,8 @@ int launch_gemm_glds(const GemmParams& p, hipStream_t stream)
                 return r;
             cfg = static_shape_cfg(p, false, false);
         }
+        if (is_wide(cfg)) // (served: the rule has asked)
+            return launch_wide_cfg(p, cfg, stream);
     }
     if (!sq && cfg == 6 && gemm_tune_cfg <= 0 && !from_table)
     {

@@ -40,8 +40,8 @@ std::mutex g_mu;
 std::map<Key, Entry> g_table;
 
 // candidates (the static rule's pick for the problem is the incumbent: see gemm_profile)
-const int kSqCandidates[] = {80, 63, 20, 8, 62, 64, 65, 42, 6, 15, 18, 1, 3, 2, 4}; // 64 / 65: split-K-2 of the 256 x 128 / 128 x 128 tile (r06)
-const int kFp16Candidates[] = {80, 55, 6, 8, 50, 56, 57, 58, 54, 51, 52, 53, 1, 3, 2, 4, 5, 7}; // 50..: the phased pipeline on fp16 operands (gemm_sqp.hip); 80: the 256 x 256 tiles of gemm_wide.hip
+const int kSqCandidates[] = {80, 81, 82, 63, 20, 8, 62, 64, 65, 42, 6, 15, 18, 1, 3, 2, 4}; // 64 / 65: split-K-2 of the 256 x 128 / 128 x 128 tile (r06)
+const int kFp16Candidates[] = {80, 81, 82, 55, 6, 8, 50, 56, 57, 58, 54, 51, 52, 53, 1, 3, 2, 4, 5, 7}; // 50..: the phased pipeline on fp16 operands (gemm_sqp.hip); 80: the 256 x 256 tiles of gemm_wide.hip, 81 / 82: its 128 x 128 / 128 x 256
 
 __global__ void fill_random_kernel(uint32_t* p, size_t n_words, uint32_t seed, int fp16)
 {
@@ -154,6 +154,10 @@ int gemm_profile(int wtype, int M, int N, int K, int* best_cfg, float* best_us, 
         return 0;
     const int es = sq ? 1 : 2;
     const size_t a_bytes = (size_t) M * K * es, w_bytes = (size_t) N * K * es, c_bytes = (size_t) M * N * 2;
+    // Each launch has other weights, as a model's layers have: from HBM, not from the caches that the launch before left them in (fp16, 1024 x 4096 x 11008: the whole-K 128 x 128
+    // tile 105 us and the split 256 x 128 one 94, cold; warm the first one won).
+    constexpr size_t kColdBytes = (size_t) 384 << 20;
+    size_t copies = std::max<size_t>(1, std::min<size_t>(32, kColdBytes / w_bytes));
     char *a = nullptr, *w = nullptr, *c = nullptr;
     float *sc = nullptr, *sr = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -169,15 +173,25 @@ int gemm_profile(int wtype, int M, int N, int K, int* best_cfg, float* best_us, 
     };
     do
     {
-        if (hipMalloc(reinterpret_cast<void**>(&a), a_bytes + 16) != hipSuccess || hipMalloc(reinterpret_cast<void**>(&w), w_bytes + 16) != hipSuccess
-            || hipMalloc(reinterpret_cast<void**>(&c), c_bytes + 16) != hipSuccess || hipMalloc(reinterpret_cast<void**>(&sc), (size_t) N * 4) != hipSuccess
-            || hipMalloc(reinterpret_cast<void**>(&sr), (size_t) M * 4) != hipSuccess)
+        if (hipMalloc(reinterpret_cast<void**>(&a), a_bytes + 16) != hipSuccess || hipMalloc(reinterpret_cast<void**>(&c), c_bytes + 16) != hipSuccess
+            || hipMalloc(reinterpret_cast<void**>(&sc), (size_t) N * 4) != hipSuccess || hipMalloc(reinterpret_cast<void**>(&sr), (size_t) M * 4) != hipSuccess)
         {
             set_error("gemm profile: hipMalloc failed (%d x %d x %d)", M, N, K);
             break;
         }
         hipLaunchKernelGGL(fill_random_kernel, dim3(1024), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(a), a_bytes / 4, 17u, sq ? 0 : 1);
-        hipLaunchKernelGGL(fill_random_kernel, dim3(1024), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(w), w_bytes / 4, 29u, sq ? 0 : 1);
+        while (hipMalloc(reinterpret_cast<void**>(&w), copies * w_bytes + 16) != hipSuccess && copies > 1) // (little memory left: fewer)
+        {
+            (void) hipGetLastError();
+            copies /= 2;
+            w = nullptr;
+        }
+        if (!w)
+        {
+            set_error("gemm profile: hipMalloc failed (%d x %d x %d)", M, N, K);
+            break;
+        }
+        hipLaunchKernelGGL(fill_random_kernel, dim3(1024), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(w), copies * w_bytes / 4, 29u, sq ? 0 : 1);
         std::vector<float> ones((size_t) std::max(M, N), 1e-3f);
         if (hipMemcpyAsync(sc, ones.data(), (size_t) N * 4, hipMemcpyHostToDevice, stream) != hipSuccess
             || hipMemcpyAsync(sr, ones.data(), (size_t) M * 4, hipMemcpyHostToDevice, stream) != hipSuccess
@@ -231,10 +245,14 @@ int gemm_profile(int wtype, int M, int N, int K, int* best_cfg, float* best_us, 
             st_idx = (int) served.size() - 1;
         }
         constexpr int kRounds = 5, kLaunches = 10;
+        size_t next = 0;
         auto time_one = [&](int cfg, float* us) {
             (void) hipEventRecord(e0, stream);
             for (int i = 0; i < kLaunches; ++i)
+            {
+                p.w = w + next++ % copies * w_bytes;
                 (void) launch_gemm_cfg(p, cfg, stream);
+            }
             (void) hipEventRecord(e1, stream);
             float ms = 0.f;
             if (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess)

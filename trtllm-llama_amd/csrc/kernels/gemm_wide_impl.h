@@ -503,7 +503,7 @@ __device__ __forceinline__ void leave_fp32(const GemmParams& p, const f32x4 (&ac
 }
 
 // fp16 and int8 products: the scales of a lane's columns and rows, requested ahead of the K loop (behind it they would wait for the next tile's first requests)
-template <int WT, int OUT>
+template <int WT, int OUT, int NA = wide::NA, int NB = wide::NB>
 struct Scales
 {
     // int8: factors of the columns of block pair q (OUT_DUAL: of the first and the second product) and of the rows; fp16: weight-only's of a column
@@ -547,14 +547,14 @@ __device__ __forceinline__ uint32_t half_pair(float a, float b)
 {
     return (uint32_t) f2h(a) | ((uint32_t) f2h(b) << 16);
 }
-template <int WT>
-__device__ __forceinline__ void leave_half(const GemmParams& p, const Tile<WT, true>& t, const Scales<WT, OUT_HALF>& sc, int row0, int col0, int rows)
+template <int WT, int NA, int NB>
+__device__ __forceinline__ void leave_half(const GemmParams& p, const typename Acc<WT>::type (&acc)[NA][NB], int lane, const Scales<WT, OUT_HALF, NA, NB>& sc, int row0, int col0, int rows)
 {
     auto out = [&](auto finish) {
 #pragma unroll
         for (int q = 0; q < NB / 2; ++q)
         {
-            const int col = col0 + 32 * q + 8 * (t.lane >> 4);
+            const int col = col0 + 32 * q + 8 * (lane >> 4);
             if (col >= p.N)
                 continue;
 #pragma unroll
@@ -566,7 +566,7 @@ __device__ __forceinline__ void leave_half(const GemmParams& p, const Tile<WT, t
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
                 {
-                    const auto a = t.acc[i][2 * q + (e >> 2)][e & 3];
+                    const auto a = acc[i][2 * q + (e >> 2)][e & 3];
                     if constexpr (WT == W_INT8_SQ)
                         v[e] = (float) a * (sc.col[q][e] * sc.row[i]);
                     else
@@ -685,7 +685,7 @@ __global__ __launch_bounds__(64 * WAVES) void wide_kernel(const GemmParams p)
             else if constexpr (DUAL)
                 leave_dual(p, t, scales, row0, col0, now.rows);
             else
-                leave_half<WT>(p, t, scales, row0, col0, now.rows);
+                leave_half<WT, NA, NB>(p, t.acc, t.lane, scales, row0, col0, now.rows);
         }
         if (!more)
             return;
@@ -713,20 +713,21 @@ __global__ __launch_bounds__(64 * WAVES) void wide_kernel(const GemmParams p)
     }
 }
 
-// Tiles of 128 rows, for products of few tiles and groups of few rows: bfloat16, a tile a workgroup of 8 waves, S whole stages of 128-byte rows, results straight from the
+// Tiles of 128 rows, for products of few tiles and groups of few rows: a tile a workgroup of 8 waves, S whole stages of 128-byte rows, results straight from the
 // accumulators as above.  PINNED: reads between the MFMAs, one barrier a K-tile (128 x 256 and 128 x 192); otherwise a k-step's reads in front of its MFMAs, which
 // the SIMD's other wave covers (128 x 128 and 128 x 64: pinned reads gave them nothing).  Bound by the operands' way from L2 and, once a wave's MFMAs are queued, by
 // them: 128 x 256 1600 - 1800 clocks a K-tile, 1024 of them MFMAs.  us in a step, in brackets the lock-step tiles of 32 x 32 MFMAs whose results went through LDS:
 //   128 x 256  2048 x 4096 x 4096 65 (70), x 11008 168 (180), 1672 x 4096 x 2048 35 (41), 32 groups of 8192 rows, 5504, 4096 493 (514), of 6688 rows, 2816, 2048 127 (126)
 //   128 x 192  1024 x 6912 x 2048 29.5 (31.9), 2048 x 8832 x 4096 161 (165)      128 x 128  1672 x 2048 x 2048 14.5 (17.8)
 //   128 x 64   1024 x 2048 x 4096 and x 6528, behind a gate into the residual 29.8 (31.7)
+//   (fp16 and int8, whole fp16 pieces: figures at the rule that picks them, gemm_glds.hip)
 // (Named as the lock-step form: whoever reads a tile from a kernel's name finds it in the same arguments; wide:: tells the two apart.)
 template <int WT, int WM, int WN, int MT, int NT, int S, int OUT, bool GROUPED, bool PINNED>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParams p_in)
 {
-    static_assert(WT == W_BF16, "a K-tile is 64 values of 2 bytes, results leave through the stack engine's seam");
+    static_assert(WT == W_BF16 || (OUT == OUT_HALF && !GROUPED), "what the other two types leave");
     constexpr bool PAIRS = out_pairs(OUT);
-    constexpr int NA = 2 * MT, NB = 2 * NT;
+    constexpr int ES = WT == W_INT8_SQ ? 1 : 2, NA = 2 * MT, NB = 2 * NT;
     constexpr int NW = WM * WN, BM = WM * NA * 16, BN = WN * NB * 16, STAGE = (BM + BN) * 128, DMAS = (BM + BN) / 8 / NW, DMA_A = BM / 8 / NW;
     static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole instructions");
     extern __shared__ __attribute__((aligned(16))) char wide_lds[];
@@ -754,11 +755,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParam
         // each XCD a contiguous range of the tiles, row tiles fastest: those that share a panel of W run side by side on one L2
         const int q = gridDim.x >> 3, r = gridDim.x & 7, xcd = id & 7;
         id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (id >> 3);
-        p.a = reinterpret_cast<const char*>(p.a) + product * p.batch_a;
-        p.c = reinterpret_cast<char*>(p.c) + product * p.batch_c;
+        if constexpr (WT == W_BF16)
+        {
+            p.a = reinterpret_cast<const char*>(p.a) + product * p.batch_a;
+            p.c = reinterpret_cast<char*>(p.c) + product * p.batch_c;
+        }
     }
-    const char* w = reinterpret_cast<const char*>(p.w) + product * p.batch_w;
-    const int tiles_m = (p.M + BM - 1) / BM, tn = id / tiles_m, m0 = (id - tn * tiles_m) * BM, n0 = tn * BN, nt = p.K / 64;
+    const char* w = reinterpret_cast<const char*>(p.w) + (WT == W_BF16 ? product * p.batch_w : 0);
+    const int tiles_m = (p.M + BM - 1) / BM, tn = id / tiles_m, m0 = (id - tn * tiles_m) * BM, n0 = tn * BN, nt = p.K * ES / 128;
     const uint32_t lds = (uint32_t) (uintptr_t) (lds_ptr*) wide_lds;
     uint32_t from[DMAS];
 #pragma unroll
@@ -770,7 +774,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParam
             int r = m0 + row < p.M ? m0 + row : p.M - 1;
             if (GROUPED && p.a_rows)
                 r = p.a_rows[r];
-            from[i] = (uint32_t) r * (uint32_t) (p.lda * 2) + (((lane & 7) ^ a_swz(row)) << 4);
+            from[i] = (uint32_t) r * (uint32_t) (p.lda * ES) + (((lane & 7) ^ a_swz(row)) << 4);
         }
         else
             from[i] = (uint32_t) (n0 + row < p.N ? n0 + row : p.N - 1) * (uint32_t) p.ldw + (((lane & 7) ^ w_swz<PAIRS>(row)) << 4);
@@ -778,12 +782,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParam
     auto dma = [&](int i, int t, uint32_t stage) {
         load16((i < DMA_A ? reinterpret_cast<const char*>(p.a) : w) + (int64_t) t * 128, from[i], stage + (uint32_t) (i * NW + wid) * 1024);
     };
-    f32x4 acc[NA][NB];
+    using acc_t = typename Acc<WT>::type;
+    acc_t acc[NA][NB];
 #pragma unroll
     for (int i = 0; i < NA; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j)
-            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            acc[i][j] = acc_t{0, 0, 0, 0};
     const int i16 = lane & 15, k4 = lane >> 4;
     const uint32_t al = (uint32_t) ((wm * NA * 16 + i16) * 128), wl = (uint32_t) (BM * 128 + (wn * NB * 16 + w_row<PAIRS>(0, i16)) * 128);
     const uint32_t as = a_swz(i16), ws = w_swz<PAIRS>(w_row<PAIRS>(0, i16));
@@ -791,6 +796,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParam
     auto a_at = [](uint32_t base, int block) { return *(lds_frag) (uintptr_t) (base + block * 2048); };
     auto w_at = [](uint32_t base, int j) { return *(lds_frag) (uintptr_t) (base + w_row<PAIRS>(j, 0) * 128); };
     const uint32_t end = lds + S * STAGE;
+    const int row0 = m0 + wm * (NA * 16) + i16, col0 = n0 + wn * (NB * 16);
+    Scales<WT, OUT, NA, NB> scales;
+    if constexpr (WT != W_BF16)
+        scales.request(p, row0, col0, p.M, lane);
     if constexpr (PINNED)
     {
         constexpr int BLOCKS = 2 * NA, L = BLOCKS >= 8 ? 3 : 2, HAND_OVER = BLOCKS - L;
@@ -906,8 +915,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParam
             into = into + STAGE == end ? lds : into + STAGE;
         }
     }
-    const int row0 = m0 + wm * (NA * 16) + i16, col0 = n0 + wn * (NB * 16);
-    if constexpr (PAIRS)
+    if constexpr (WT != W_BF16)
+        leave_half<WT, NA, NB>(p, acc, lane, scales, row0, col0, p.M);
+    else if constexpr (PAIRS)
         leave_pairs<OUT>(p, acc, lane, p.c, row0, col0, p.M);
     else
         leave_fp32<OUT>(p, acc, lane, p.c, row0, col0, p.M);
@@ -1297,18 +1307,18 @@ int launch(const GemmParams& p, hipStream_t stream)
         return launch_out<WT, OUT_HALF>(p, stream);
 }
 
-template <int OUT, bool GROUPED, int WM, int WN, int MT, int NT, int S, bool PINNED>
+template <int WT, int OUT, bool GROUPED, int WM, int WN, int MT, int NT, int S, bool PINNED>
 int launch_row128_out(const GemmParams& p, hipStream_t stream)
 {
     constexpr int BM = WM * MT * 32, BN = WN * NT * 32;
     constexpr size_t lds = (size_t) S * (BM + BN) * 128;
     static_assert(BM == 128 && lds <= LDS_BYTES, "LDS");
-    const auto kernel = gemm_glds_kernel<W_BF16, WM, WN, MT, NT, S, OUT, GROUPED, PINNED>;
+    const auto kernel = gemm_glds_kernel<WT, WM, WN, MT, NT, S, OUT, GROUPED, PINNED>;
     launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
     const int64_t cols = (p.N + BN - 1) / BN;
     // grouped: at most this many row tiles, full ones, and one begun in every group that has rows
     const int64_t tiles = GROUPED ? (p.group_total / BM + std::min<int64_t>(p.batch, p.group_total)) * cols : (p.M + BM - 1) / BM * cols;
-    hipLaunchKernelGGL(kernel, dim3((unsigned) tiles, GROUPED ? 1 : p.batch), dim3(64 * WM * WN), lds, stream, p);
+    hipLaunchKernelGGL(kernel, dim3((unsigned) tiles, GROUPED || WT != W_BF16 ? 1 : p.batch), dim3(64 * WM * WN), lds, stream, p);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess)
     {
@@ -1323,14 +1333,14 @@ int launch_row128(const GemmParams& p, hipStream_t stream)
 {
     const bool gated = p.act >= GEMM_ACT_GATE_SILU, fp32 = p.out_dtype == DT_FLOAT && p.seam.n_sec == 0 && p.act == GEMM_ACT_NONE;
     if (p.group_off)
-        return gated ? launch_row128_out<OUT_GATED, true, WM, WN, MT, NT, S, PINNED>(p, stream)
-            : fp32   ? launch_row128_out<OUT_FP32, true, WM, WN, MT, NT, S, PINNED>(p, stream)
-                     : launch_row128_out<OUT_STORE, true, WM, WN, MT, NT, S, PINNED>(p, stream);
+        return gated ? launch_row128_out<W_BF16, OUT_GATED, true, WM, WN, MT, NT, S, PINNED>(p, stream)
+            : fp32   ? launch_row128_out<W_BF16, OUT_FP32, true, WM, WN, MT, NT, S, PINNED>(p, stream)
+                     : launch_row128_out<W_BF16, OUT_STORE, true, WM, WN, MT, NT, S, PINNED>(p, stream);
     if (p.resid)
-        return p.gate ? launch_row128_out<OUT_RESID_GATE, false, WM, WN, MT, NT, S, PINNED>(p, stream) : launch_row128_out<OUT_RESID, false, WM, WN, MT, NT, S, PINNED>(p, stream);
-    return gated ? launch_row128_out<OUT_GATED, false, WM, WN, MT, NT, S, PINNED>(p, stream)
-        : fp32   ? launch_row128_out<OUT_FP32, false, WM, WN, MT, NT, S, PINNED>(p, stream)
-                 : launch_row128_out<OUT_STORE, false, WM, WN, MT, NT, S, PINNED>(p, stream);
+        return p.gate ? launch_row128_out<W_BF16, OUT_RESID_GATE, false, WM, WN, MT, NT, S, PINNED>(p, stream) : launch_row128_out<W_BF16, OUT_RESID, false, WM, WN, MT, NT, S, PINNED>(p, stream);
+    return gated ? launch_row128_out<W_BF16, OUT_GATED, false, WM, WN, MT, NT, S, PINNED>(p, stream)
+        : fp32   ? launch_row128_out<W_BF16, OUT_FP32, false, WM, WN, MT, NT, S, PINNED>(p, stream)
+                 : launch_row128_out<W_BF16, OUT_STORE, false, WM, WN, MT, NT, S, PINNED>(p, stream);
 }
 
 } // namespace wide
