@@ -707,28 +707,27 @@ __device__ __forceinline__ void softmax_unit(f32x4 (&s)[NN], float& m_run, float
 {
     if (!plain)
     {
+        // (asked once for all scores: a branch at each one leaves its exponential and its reciprocal to wait for each other, 46 us for 37 at 16 heads of 2 x 64 / 128, 1024 rows)
+        auto all = [&](auto&& f) {
 #pragma unroll
-        for (int n = 0; n < NN; ++n)
+            for (int n = 0; n < NN; ++n)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-            {
-                float v;
-                if (hm.cap2 > 0.f)
-                {
-                    const float t2 = __builtin_amdgcn_exp2f(fminf(fmaxf(s[n][i] * hm.cap_arg, -43.f), 43.f)); // (softmax_block)
-                    v = hm.cap2 * (t2 - 1.f) * __builtin_amdgcn_rcpf(t2 + 1.f);
-                }
-                else
-                    v = s[n][i] * hm.scale2;
-                if (hm.pen)
-                {
-                    const float dist = (float) (qpos - (key_lane0 + 32 * (n >> 1) + 4 * (n & 1) + i));
-                    v -= hm.slope2 * dist;
-                    if (hm.r1 != 0.f)
-                        v -= hm.r1 * __builtin_amdgcn_logf(fmaxf(1.f + hm.r2 * dist, 1e-30f));
-                }
-                s[n][i] = v;
-            }
+                for (int i = 0; i < 4; ++i)
+                    s[n][i] = f(s[n][i], key_lane0 + 32 * (n >> 1) + 4 * (n & 1) + i);
+        };
+        if (hm.cap2 > 0.f)
+            all([&](float v, int) {
+                const float t2 = __builtin_amdgcn_exp2f(fminf(fmaxf(v * hm.cap_arg, -43.f), 43.f)); // (softmax_block)
+                return hm.cap2 * (t2 - 1.f) * __builtin_amdgcn_rcpf(t2 + 1.f);
+            });
+        else
+            all([&](float v, int) { return v * hm.scale2; });
+        if (hm.pen)
+        {
+            all([&](float v, int key) { return v - hm.slope2 * (float) (qpos - key); });
+            if (hm.r1 != 0.f)
+                all([&](float v, int key) { return v - hm.r1 * __builtin_amdgcn_logf(fmaxf(1.f + hm.r2 * (float) (qpos - key), 1e-30f)); });
+        }
     }
     if (masked)
     {
@@ -818,23 +817,24 @@ __device__ __forceinline__ uint4 ones_where(const uint4& x)
 //   - tile t of a half unit holds keys 8 (r / 4) + 4 t + r % 4 in row r, so that a lane's eight scores are eight neighbouring keys and the V^T fragment
 //     that meets them is one 16-byte read;
 //   - a row's maximum meets over the lanes by register swaps;
-//   - KS = 2 (few workgroups): eight waves, two to a row tile, each with its half of every unit's keys; they meet behind the last unit.
-// Workgroups: the heaviest tiles of all heads first, the heads of one key/value head on one XCD.
+//   - KS = 2 (few workgroups): two waves to a row tile, each with its half of every unit's keys, a workgroup 32 rows; they meet behind the last unit.
+// Workgroups: the heaviest tiles of all heads first, the heads of one key/value head on one XCD.  Up to two to a CU, workgroup i + CUs shares i's: from tile level `turn` on the lightest
+// come first, so that a CU has 17 units of a prompt's 32 rows, and not 24 or 9.
 // Measured (us): 32 heads over 8, 192 / 128, 2048 rows at contexts 0 and 2048 on average 402 -> 164; 128 / 128 272 -> 151; 16 heads of 2 x 64 / 128 with a soft
-// cap, 1024 rows 90 -> 57.
+// cap, 1024 rows 90 -> 53, with workgroups of 32 rows for 64, on eight waves, and the turn 46, with the soft cap's branch asked once a unit (softmax_unit) 37.
 template <int MAPS, int DK, int VT, int RT, int KS>
-__global__ __launch_bounds__(256 * KS, 2 / KS) void attn_prompt_kernel(const StackAttnParams p, int min_count, int tiles)
+__global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnParams p, int min_count, int tiles, int turn)
 {
-    constexpr int D = DK * 32, V = VT * 16, ROWS = 64 * RT;
+    constexpr int RW = 4 / KS, D = DK * 32, V = VT * 16, ROWS = 16 * RW * RT; // RW: waves of different rows
     constexpr int KPR = D / 8;                                    // 16-byte pieces of a K row
-    constexpr int NW = 4 * KS, NN = 4 / KS;                       // waves; score tiles of 16 keys per wave and unit
+    constexpr int NW = 4, NN = 4 / KS;                            // waves; score tiles of 16 keys per wave and unit
     constexpr int KI = MAPS * KPR / NW, VI = V / 8 / NW;          // DMA instructions per wave and unit
     constexpr int KB = MAPS * 64 * D * 2, BUF = KB + V * 128;     // bytes
     static_assert(KPR % 8 == 0 && V % 64 == 0 && MAPS * KPR % NW == 0, "head sizes");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // blockIdx.x = tile level x (entries x heads), heaviest tiles first; inside a level the key/value heads run fastest
     const int per = p.entries * p.heads;
-    const int level = blockIdx.x / per, q_ = blockIdx.x % per, e = q_ / p.heads, hi = q_ % p.heads;
+    const int at = blockIdx.x / per, level = at < turn ? at : turn + tiles - 1 - at, q_ = blockIdx.x % per, e = q_ / p.heads, hi = q_ % p.heads;
     const int h = p.cross_values ? hi : hi % p.kv_heads * (p.heads / p.kv_heads) + hi / p.kv_heads;
     const int count = p.ent_count[e];
     if (count < min_count)
@@ -844,7 +844,7 @@ __global__ __launch_bounds__(256 * KS, 2 / KS) void attn_prompt_kernel(const Sta
         return;
     const int first = p.ent_first[e], pos0 = p.ent_pos0[e];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int col = lane & 15, g4 = lane >> 4, wr = w & 3, half = w >> 2; // row tile, and which half of a unit's keys (KS = 2)
+    const int col = lane & 15, g4 = lane >> 4, wr = w % RW, half = w / RW; // row tile, and which half of a unit's keys (KS = 2)
     const HeadMap hd = head_map(p, h);
     const int page = p.page, upp = page / 64; // units per page
     const int32_t* table = p.block_table + (int64_t) e * p.max_blocks;
@@ -1040,7 +1040,7 @@ __global__ __launch_bounds__(256 * KS, 2 / KS) void attn_prompt_kernel(const Sta
     }
     if constexpr (KS == 2)
     {
-        // the two halves of the keys meet: waves 4 .. 7 leave theirs in LDS
+        // the two halves of the keys meet: waves RW .. 2 RW - 1 leave theirs in LDS
         static_assert(RT == 1, "one row tile per wave");
         constexpr int PER = (VT * 4 + 2) * 64; // floats per wave and map
         float* x = reinterpret_cast<float*>(smem) + wr * PER * MAPS + lane;
@@ -1115,11 +1115,14 @@ __global__ __launch_bounds__(256 * KS, 2 / KS) void attn_prompt_kernel(const Sta
 template <int MAPS, int DK, int VT, int RT, int KS>
 void launch_prompt(const StackAttnParams& p, int min_count, hipStream_t stream)
 {
-    constexpr size_t stages = 2 * ((size_t) MAPS * 64 * DK * 64 + VT * 16 * 128), merge = KS == 2 ? (size_t) 4 * MAPS * (VT * 4 + 2) * 256 : 0;
+    constexpr int RW = 4 / KS;
+    constexpr size_t stages = 2 * ((size_t) MAPS * 64 * DK * 64 + VT * 16 * 128), merge = KS == 2 ? (size_t) RW * MAPS * (VT * 4 + 2) * 256 : 0;
     constexpr size_t lds = stages > merge ? stages : merge;
     launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_prompt_kernel<MAPS, DK, VT, RT, KS>), lds);
-    const int tiles = (p.max_count + 64 * RT - 1) / (64 * RT);
-    hipLaunchKernelGGL((attn_prompt_kernel<MAPS, DK, VT, RT, KS>), dim3((unsigned) ((int64_t) tiles * p.entries * p.heads)), dim3(256 * KS), lds, stream, p, min_count, tiles);
+    const int tiles = (p.max_count + 16 * RW * RT - 1) / (16 * RW * RT);
+    const int64_t per = (int64_t) p.entries * p.heads, cus = launch_util::device_cus();
+    const int turn = tiles * per <= 2 * cus ? (int) (cus / per) : tiles;
+    hipLaunchKernelGGL((attn_prompt_kernel<MAPS, DK, VT, RT, KS>), dim3((unsigned) (tiles * per)), dim3(256), lds, stream, p, min_count, tiles, turn);
 }
 
 // attn_prefill_wide_kernel: the staged form for one map and long rows (dim of 160 and more), where the fragment reads out of LDS, not
