@@ -876,6 +876,14 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnPara
         my_lo[rt] = rows_ok ? first_visible(p, pos0 + r0[rt]) / 64 : 0;
         klo_last[rt] = rows_ok ? first_visible(p, pos0 + last) : 0;
     }
+    // The queries' fragments are here: a wait for them inside the walk, where the compiler would leave it, is one for the next unit's K and V, too (they are requested in front of it).
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int m = 0; m < MAPS; ++m)
+#pragma unroll
+            for (int ks = 0; ks < DK; ++ks)
+                asm volatile("" : "+v"(qf[rt][m][ks]));
     const int wg_last = tile * ROWS + ROWS - 1 < count ? tile * ROWS + ROWS - 1 : count - 1;
     // the units the workgroup walks: the ones with kept first keys, then from its first row's first visible key on
     const int lo = first_visible(p, pos0 + tile * ROWS) / 64;
@@ -910,7 +918,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnPara
         for (int i = 0; i < VI; ++i)
             dma16(vb, voff[i], lds0 + buf * BUF + KB + i * NW * 1024);
     };
-    auto block_of = [&](int u) { return __builtin_amdgcn_readfirstlane(table[upp == 1 ? u : u / upp]); };
+    auto block_of = [&](int u) { return table[upp == 1 ? u : u / upp]; };
 
     // CAREFUL: a value that is no finite number meets only the rows that see its key (a weight of 0 times it would make it everyone's)
     auto walk = [&](auto careful) {
@@ -926,7 +934,8 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnPara
                 for (int ct = 0; ct < VT; ++ct)
                     acc[rt][m][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
-        request(unit_at(0), block_of(unit_at(0)), 0);
+        request(unit_at(0), __builtin_amdgcn_readfirstlane(block_of(unit_at(0))), 0);
+        // (in a vector register until behind the next unit's wait: earlier, its own would be one for the requests in front of it)
         int blk_next = n_units > 1 ? block_of(unit_at(1)) : 0;
         for (int v = 0; v < n_units; ++v)
         {
@@ -935,7 +944,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnPara
             __syncthreads(); // the unit has landed for every wave, and every wave is through with the one before it
             if (v + 1 < n_units)
             {
-                request(unit_at(v + 1), blk_next, (v + 1) & 1);
+                request(unit_at(v + 1), __builtin_amdgcn_readfirstlane(blk_next), (v + 1) & 1);
                 if (v + 2 < n_units)
                     blk_next = block_of(unit_at(v + 2));
             }
