@@ -820,8 +820,9 @@ __device__ __forceinline__ uint4 ones_where(const uint4& x)
 //   - KS = 2 (few workgroups): two waves to a row tile, each with its half of every unit's keys, a workgroup 32 rows; they meet behind the last unit.
 // Workgroups: the heaviest tiles of all heads first, the heads of one key/value head on one XCD.  Up to two to a CU, workgroup i + CUs shares i's: from tile level `turn` on the lightest
 // come first, so that a CU has 17 units of a prompt's 32 rows, and not 24 or 9.
-// Measured (us): 32 heads over 8, 192 / 128, 2048 rows at contexts 0 and 2048 on average 402 -> 164; 128 / 128 272 -> 151; 16 heads of 2 x 64 / 128 with a soft
-// cap, 1024 rows 90 -> 53, with workgroups of 32 rows for 64, on eight waves, and the turn 46, with the soft cap's branch asked once a unit (softmax_unit) 37.
+// Measured (us): 32 heads over 8, 192 / 128, 2048 rows at contexts 0 and 2048 on average 402 -> 149, without waits for the next unit inside the walk 127; 128 / 128 272 -> 133 -> 114; 16
+// heads of 2 x 64 / 128 with a soft cap, 1024 rows 90 -> 53, with workgroups of 32 rows for 64, on eight waves, and the turn 46, with the soft cap's branch asked once a unit (softmax_unit)
+// 37, without those waits 34.
 template <int MAPS, int DK, int VT, int RT, int KS>
 __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnParams p, int min_count, int tiles, int turn)
 {
@@ -830,6 +831,9 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnPara
     constexpr int NW = 4, NN = 4 / KS;                            // waves; score tiles of 16 keys per wave and unit
     constexpr int KI = MAPS * KPR / NW, VI = V / 8 / NW;          // DMA instructions per wave and unit
     constexpr int KB = MAPS * 64 * D * 2, BUF = KB + V * 128;     // bytes
+    // Fragments read ahead of their products (V's: over the softmax), what 256 registers have room for: left to itself the compiler waits for each pair of them, LDS answers in 100 clocks
+    // and the products of one take 32 (us, 32 heads, 2048 rows at contexts 0 and 2048 on average: 192 / 128 127 -> 118, 128 / 128 114 -> 106).
+    constexpr int AHEAD = RT * DK > 8 ? 3 : 4, V_AHEAD = RT * DK > 8 ? 2 : 4;
     static_assert(KPR % 8 == 0 && V % 64 == 0 && MAPS * KPR % NW == 0, "head sizes");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // blockIdx.x = tile level x (entries x heads), heaviest tiles first; inside a level the key/value heads run fastest
@@ -960,27 +964,50 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnPara
             const char* ks_ = smem + (v & 1) * BUF;
             const char* vs_ = ks_ + KB;
             const int key0 = u * 64 + (KS == 2 ? half * 32 : 0);
-            uint4 pf[RT][MAPS][NN / 2];
+            uint4 pf[RT][MAPS][NN / 2], vf[VT * NN / 2];
+            auto v_at = [&](int x) {
+                const int row = x / (NN / 2) * 16 + col, b = x % (NN / 2);
+                return *reinterpret_cast<const uint4*>(vs_ + row * 128 + ((((KS == 2 ? half : b) * 4 + g4) ^ ((row >> 1) & 7)) << 4));
+            };
 #pragma unroll
             for (int m = 0; m < MAPS; ++m)
             {
                 f32x4 s[RT][NN];
 #pragma unroll
-                for (int n = 0; n < NN; ++n)
-                {
-                    const int r = 32 * (KS == 2 ? half : n >> 1) + 8 * (col >> 2) + 4 * (n & 1) + (col & 3);
-                    const int x = KPR % 16 == 0 ? ((r >> 3) & 3) << 2 | (r & 3) : ((r >> 3) & 3) << 1 | ((r >> 1) & 1);
+                for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                    for (int rt = 0; rt < RT; ++rt)
+                    for (int n = 0; n < NN; ++n)
                         s[rt][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+                // fragments of two score tiles in turn
+                auto k_at = [&](int x) {
+                    const int n = x / (2 * DK) * 2 + x % 2, ks = x / 2 % DK;
+                    const int r = 32 * (KS == 2 ? half : n >> 1) + 8 * (col >> 2) + 4 * (n & 1) + (col & 3);
+                    const int sw = KPR % 16 == 0 ? ((r >> 3) & 3) << 2 | (r & 3) : ((r >> 3) & 3) << 1 | ((r >> 1) & 1);
+                    return *reinterpret_cast<const uint4*>(ks_ + (m * 64 + r) * (D * 2) + (((ks * 4 + g4) ^ sw) << 4));
+                };
+                uint4 kf[NN * DK];
 #pragma unroll
-                    for (int ks = 0; ks < DK; ++ks)
-                    {
-                        const bf16x8 kf = as_bf16x8(*reinterpret_cast<const uint4*>(ks_ + (m * 64 + r) * (D * 2) + (((ks * 4 + g4) ^ x) << 4)));
+                for (int x = 0; x < AHEAD; ++x)
+                    kf[x] = k_at(x);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                        for (int rt = 0; rt < RT; ++rt) // (no branches among the products: a tile that is off has its scores dropped below)
-                            s[rt][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[rt][m][ks], s[rt][n], 0, 0, 0);
-                    }
+                for (int x = 0; x < NN * DK; ++x)
+                {
+                    const int n = x / (2 * DK) * 2 + x % 2, ks = x / 2 % DK;
+                    if (x + AHEAD < NN * DK)
+                        kf[x + AHEAD] = k_at(x + AHEAD);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt) // (no branches among the products: a tile that is off has its scores dropped below)
+                        s[rt][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[x]), qf[rt][m][ks], s[rt][n], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (m == MAPS - 1)
+                {
+#pragma unroll
+                    for (int x = 0; x < V_AHEAD; ++x)
+                        vf[x] = v_at(x);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt)
@@ -998,8 +1025,12 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnPara
 #pragma unroll
                 for (int b = 0; b < NN / 2; ++b)
                 {
-                    const int row = ct * 16 + col;
-                    uint4 vr = *reinterpret_cast<const uint4*>(vs_ + row * 128 + ((((KS == 2 ? half : b) * 4 + g4) ^ ((row >> 1) & 7)) << 4));
+                    constexpr int ALL = VT * NN / 2;
+                    const int x = ct * (NN / 2) + b;
+                    if (x + V_AHEAD < ALL)
+                        vf[x + V_AHEAD] = v_at(x + V_AHEAD);
+                    __builtin_amdgcn_sched_barrier(0);
+                    uint4 vr = vf[x];
                     uint4 vbad = make_uint4(0, 0, 0, 0);
                     if constexpr (CAREFUL)
                         vbad = take_specials(vr);
@@ -1017,6 +1048,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnPara
                                     acc[rt][m][ct][i] = n[i] > 0.f ? __builtin_nanf("") : acc[rt][m][ct][i];
                             }
                         }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
         }
     };
