@@ -8,6 +8,8 @@ namespace tllm
 namespace kernels
 {
 
+extern void* gemm_clock_probe; // gemm_sqp.hip (microbench hook)
+
 // 0 launched, -1 launch error, 1 not served
 int launch_gemm_wide(const GemmParams& p, hipStream_t stream)
 {
@@ -29,10 +31,12 @@ static int launch_rows128_type(const GemmParams& p, bool wide_cols, hipStream_t 
                      : wide::launch_row128_out<WT, wide::OUT_HALF, false, 2, 4, 2, 1, 4, false>(p, stream);
 }
 // tiles of 128 x 128, or of 128 x 256: 0 launched, -1 launch error, 1 not served
-int launch_gemm_rows128(const GemmParams& p, bool wide_cols, hipStream_t stream)
+int launch_gemm_rows128(const GemmParams& p_in, bool wide_cols, hipStream_t stream)
 {
-    if (!gemm_rows128_serves(p))
+    if (!gemm_rows128_serves(p_in))
         return 1;
+    GemmParams p = p_in;
+    p.clock_probe = gemm_clock_probe;
     return p.wtype == W_FP16 ? launch_rows128_type<W_FP16>(p, wide_cols, stream) : launch_rows128_type<W_INT8_SQ>(p, wide_cols, stream);
 }
 

@@ -732,6 +732,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParam
     static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole instructions");
     extern __shared__ __attribute__((aligned(16))) char wide_lds[];
     GemmParams p = p_in;
+    const bool clocked = WT == W_INT8_SQ && p.clock_probe; // (microbench hook)
+    const uint64_t clk0 = clocked ? __builtin_readcyclecounter() : 0, rt0 = clocked ? __builtin_amdgcn_s_memrealtime() : 0;
     const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wid / WN, wn = wid % WN;
     int64_t product = blockIdx.y;
     int id = blockIdx.x;
@@ -916,7 +918,15 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParam
         }
     }
     if constexpr (WT != W_BF16)
+    {
         leave_half<WT, NA, NB>(p, acc, lane, scales, row0, col0, p.M);
+        if (clocked && threadIdx.x == 0)
+        {
+            uint64_t* to = reinterpret_cast<uint64_t*>(p.clock_probe) + 2 * blockIdx.x;
+            to[0] = __builtin_readcyclecounter() - clk0;
+            to[1] = __builtin_amdgcn_s_memrealtime() - rt0;
+        }
+    }
     else if constexpr (PAIRS)
         leave_pairs<OUT>(p, acc, lane, p.c, row0, col0, p.M);
     else
