@@ -1,5 +1,5 @@
 // A HIP runtime for tests of the engines' host side on a machine without a GPU: loaded ahead of libtllm_stack_engine.so, it takes the
-// place of the 20 runtime calls that the library makes, and ahead of libnvinfer_plugin_tensorrt_llm.so of those of a LLaMA session's set-up and context phase.  Device memory is host memory within a budget, launches are recorded and compute
+// place of the 20 runtime calls that the library makes, and ahead of libnvinfer_plugin_tensorrt_llm.so of those of a LLaMA session on one GPU, its step graph included.  Device memory is host memory within a budget, launches are recorded and compute
 // nothing, but that wanted rows land: all of them zeros.  Launch limits are the runtime's documented ones: fewer than 2^32 threads per grid dimension, 65535 workgroups in y and z.
 #include <hip/hip_runtime_api.h>
 #include <cstdint>
@@ -20,9 +20,9 @@ struct Config
 std::vector<Config> g_configs;
 std::map<void*, size_t> g_device, g_pinned;
 std::map<const void*, std::string> g_names;
-std::string g_launched;
-size_t g_live = 0, g_budget = ~size_t(0), g_largest = 0;
-int g_host_mallocs = 0, g_syncs = 0, g_stream_syncs = 0;
+std::string g_launched, *g_captured = nullptr; // (a graph is the names of its kernels)
+size_t g_live = 0, g_budget = ~size_t(0), g_pinned_budget = ~size_t(0), g_largest = 0;
+int g_host_mallocs = 0, g_syncs = 0, g_stream_syncs = 0, g_event_syncs = 0, g_graphs = 0;
 hipError_t g_last = hipSuccess;
 
 hipError_t done(hipError_t e)
@@ -49,6 +49,7 @@ hipError_t release(std::map<void*, size_t>& from, void* p)
 extern "C" {
 // what the tests ask
 void stub_budget(size_t bytes) { g_budget = bytes; }
+void stub_pinned_budget(size_t bytes) { g_pinned_budget = bytes; } // of one allocation
 size_t stub_live() { return g_live; }
 int stub_has_allocation(size_t bytes)
 {
@@ -60,6 +61,8 @@ int stub_has_allocation(size_t bytes)
 int stub_host_mallocs() { return g_host_mallocs; }
 int stub_device_syncs() { return g_syncs; }
 int stub_stream_syncs() { return g_stream_syncs; }
+int stub_event_syncs() { return g_event_syncs; }
+int stub_graphs() { return g_graphs; } // instantiated so far
 size_t stub_pinned_bytes()
 {
     size_t n = 0;
@@ -74,7 +77,7 @@ hipError_t hipMalloc(void** p, size_t n)
 {
     if (n > g_budget || g_live > g_budget - n)
         return done(hipErrorOutOfMemory);
-    *p = std::malloc(n ? n : 1); // (large ones are mapped on demand: nothing computes on them)
+    *p = std::calloc(1, n ? n : 1); // (large ones are mapped on demand: nothing computes on them)
     g_device[*p] = n;
     g_live += n;
     return hipSuccess;
@@ -82,6 +85,8 @@ hipError_t hipMalloc(void** p, size_t n)
 hipError_t hipFree(void* p) { return release(g_device, p); }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned int)
 {
+    if (n > g_pinned_budget)
+        return done(hipErrorOutOfMemory);
     ++g_host_mallocs;
     *p = std::calloc(1, n ? n : 1);
     g_pinned[*p] = n;
@@ -93,12 +98,32 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipSt
 hipError_t hipMemset(void*, int, size_t) { return hipSuccess; }
 hipError_t hipMemsetAsync(void*, int, size_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { return *e = reinterpret_cast<hipEvent_t>(new int(0)), hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { return delete reinterpret_cast<int*>(e), hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return ++g_event_syncs, hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.f, hipSuccess; } // (all kernels are as quick)
 hipError_t hipDeviceSynchronize() { return ++g_syncs, hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return ++g_stream_syncs, hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t* s) { return *s = reinterpret_cast<hipStream_t>(new int(0)), hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { return delete reinterpret_cast<int*>(s), hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return g_captured = new std::string, hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g)
+{
+    *g = reinterpret_cast<hipGraph_t>(g_captured);
+    g_captured = nullptr;
+    return hipSuccess;
+}
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNode_t*, char*, size_t)
+{
+    ++g_graphs;
+    *e = reinterpret_cast<hipGraphExec_t>(new std::string(*reinterpret_cast<std::string*>(g)));
+    return hipSuccess;
+}
+hipError_t hipGraphDestroy(hipGraph_t g) { return delete reinterpret_cast<std::string*>(g), hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) { return delete reinterpret_cast<std::string*>(e), hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) { return g_launched += *reinterpret_cast<std::string*>(e), hipSuccess; }
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) { return *n = 1, hipSuccess; }
 hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
@@ -114,7 +139,7 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
     auto it = g_names.find(f);
     if (it != g_names.end() && it->second.find("deliver_kernel") != std::string::npos)
         std::memset(*static_cast<void**>(args[1]), 0, (size_t) grid.x * grid.y * 8); // every part's choice
-    g_launched += (it == g_names.end() ? std::string("?") : it->second) + "\n";
+    (g_captured ? *g_captured : g_launched) += (it == g_names.end() ? std::string("?") : it->second) + "\n";
     const bool fits = grid.x && grid.y && grid.z && (uint64_t) grid.x * block.x < (1ull << 32) && grid.y <= 65535 && grid.z <= 65535;
     return done(fits ? hipSuccess : hipErrorInvalidConfiguration);
 }

@@ -38,3 +38,21 @@ def test_requests_do_not_depend_on_the_one_before(batch, prompt):
     other.synchronize()
     np.testing.assert_array_equal(s.generate(ids, lens, new), alone[0])
     s.close()
+
+
+@pytest.mark.parametrize('mode', ['fp16', 'sq_static_pc'])
+def test_beam_requests_do_not_depend_on_the_one_before(mode):
+    """The second request's steps are all replayed: its ids, its logits and how many rows of them there are, are the first one's."""
+    many, session = sessions(mode, 0)
+    s = session(2, 9)
+    s.setup(2, 9, NEW, beam_width=3)
+    ids, lens = many[:2, :9].copy(), np.array([9, 4], np.int32)
+    got = []
+    for prompt in (ids, many[2:4, :9].copy(), ids, ids):
+        out = s.generate(prompt, lens, NEW)
+        got.append((out, s.logits()))
+        assert got[-1][1].shape[0] == 6
+    for out, logits in got[2:]:
+        np.testing.assert_array_equal(out, got[0][0])
+        np.testing.assert_array_equal(logits, got[0][1])
+    s.close()

@@ -1,0 +1,63 @@
+"""Host side of a LLaMA session's requests (session.cpp) over the stand-in for the HIP runtime (hip_stub.cpp), without a GPU: nothing is computed, but every allocation, launch, wait and
+captured step is the real code's.  Each scenario runs in a process of its own, with the stand-in loaded ahead of the library."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from test_stack_host_runtime import Stub, stub  # noqa: F401 (fixture)
+
+S, NEW = 16, 6
+
+
+def run(stub, scenario):  # noqa: F811
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), stub, scenario], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+# ------------------------------------------------------------------------------------------------------------ in the child process
+def session(mode='fp16', batch=1, beam=1):
+    import test_gpu_session as G
+    from oracle import quant_oracle as QO
+    from tensorrt_llm.runtime.native import NativeSession
+    cfg, w = G.synth_model(7)
+    ids = np.full((1, 8), 5, np.int32)
+    m = QO.quantise_model(cfg, w, mode, 0, calib_ids=ids, calib_lens=np.array([8], np.int32))
+    s = NativeSession(dict(cfg, quant_mode=m['quant_mode']))
+    for k, v in m['engine_tensors'].items():
+        s.set_tensor(k, v)
+    s.finalize()
+    s.setup(batch, S, NEW, beam_width=beam)
+    return s
+
+
+def request(s, **kw):
+    return s.generate(np.full((s.batch, S), 3, np.int32), np.full(s.batch, S, np.int32), NEW, **kw)
+
+
+def rows_of_logits(stub):  # noqa: F811
+    """The logits behind a request are its last step's, whether its steps were launched or replayed; behind a prompt they are the prompts'."""
+    for batch, beam in ((2, 3), (2, 1)):
+        s = session(batch=batch, beam=beam)
+        for stream in (0, 0, 64, 64):
+            request(s, stream=stream)
+            assert s.logits(stream=stream).shape[0] == batch * beam, (batch, beam, stream)
+        for graph in (False, True, True):
+            s.context(np.full((batch, S), 3, np.int32), np.full(batch, S, np.int32))
+            s.step(0, use_graph=graph)
+            assert s.logits().shape[0] == batch, (batch, beam, graph)
+            s.step(2, use_graph=graph)
+            assert s.logits().shape[0] == batch * beam, (batch, beam, graph)
+        s.close()
+
+
+if __name__ == '__main__':
+    sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+    globals()[sys.argv[2]](Stub(sys.argv[1]))
+    print('ok')
+else:
+    def test_rows_of_logits(stub):  # noqa: F811
+        run(stub, 'rows_of_logits')

@@ -908,12 +908,12 @@ struct tllm_session
         else
             RUN(launch_gather_last_token(last_hidden, x, last_tok, Bc, S, D, st));
         RUN(run_head(last_hidden, Bc, st));
+        logit_rows = Bc;
         return 0;
     }
 
     int run_head(const void* h, int rows, hipStream_t st, bool normalised = false)
     {
-        logit_rows = rows;
         gemv_cls = PC_GEMV_HEAD;
         const int head_rc = gemv(head, rows, normalised ? PRO_NONE : PRO_RMSNORM, EPI_NONE, h, hidden, lnf, nullptr, nullptr, nullptr,
             logits_local, Vr, DT_FLOAT, nullptr, st);
@@ -2089,6 +2089,7 @@ int32_t tllm_session_step(tllm_session_t s, int32_t n_steps, int32_t use_graph, 
             HIP_OK(hipGraphLaunch(s->graph, st));
         else
             RUN(s->run_decode_step(st));
+        s->logit_rows = s->B; // (here: run_decode_step may be recorded now and replayed behind another prompt)
     }
     return 0;
 }
@@ -2520,6 +2521,8 @@ int32_t tllm_session_profile(tllm_session_t s, int32_t n_steps, float* ms_per_cl
     int rc = 0;
     for (int i = 0; i < n_steps && !rc; ++i)
         rc = s->run_decode_step(st);
+    if (!rc)
+        s->logit_rows = s->B;
     s->profiling = false;
     (void) hipStreamSynchronize(st);
     for (int c = 0; c < tllm_session::PC_COUNT; ++c)
