@@ -54,6 +54,31 @@ def rows_of_logits(stub):  # noqa: F811
         s.close()
 
 
+def set_up_without_memory(stub):  # noqa: F811
+    """A set-up that fails for want of memory, on the device or pinned, gives back what it made, and requests behind it are told to set up first."""
+    s = session()
+    request(s)
+    s.setup(1, S, NEW)
+    pinned = stub.pinned_bytes()
+    assert pinned > 0
+    weights = stub.live()  # (an upper bound: with the set-up)
+    for what, size in (('budget', 0), ('budget', weights // 2), ('budget', weights - 4096), ('pinned_budget', pinned - 1)):
+        getattr(stub, what)(size)
+        with pytest.raises(RuntimeError, match='hipMalloc|hipHostMalloc'):
+            s.setup(1, S, NEW)
+        getattr(stub, what)(2 ** 64 - 1)
+        assert stub.pinned_bytes() == 0 and stub.live() < weights, what
+        s.batch, s.max_in, s.max_new = 1, S, NEW
+        for call in (lambda: request(s), lambda: s.context(np.full((1, S), 3, np.int32), np.full(1, S, np.int32)), lambda: s.step(1)):
+            with pytest.raises(RuntimeError, match='setup'):
+                call()
+        s.setup(1, S, NEW)
+        request(s)
+        assert stub.live() == weights and stub.pinned_bytes() == pinned, what
+    s.close()
+    assert stub.pinned_bytes() == 0
+
+
 if __name__ == '__main__':
     sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
     globals()[sys.argv[2]](Stub(sys.argv[1]))
@@ -61,3 +86,6 @@ if __name__ == '__main__':
 else:
     def test_rows_of_logits(stub):  # noqa: F811
         run(stub, 'rows_of_logits')
+
+    def test_set_up_without_memory(stub):  # noqa: F811
+        run(stub, 'set_up_without_memory')

@@ -347,6 +347,12 @@ struct tllm_session
         for (auto p : allocs)
             (void) hipFree(p);
         allocs.clear();
+        for (auto& L : layers)
+        {
+            L.kv = nullptr;
+            L.kv_table = nullptr;
+        }
+        B = 0; // (no call goes on without a set-up)
     }
 
     void free_start()
@@ -356,7 +362,7 @@ struct tllm_session
         if (start_host)
             (void) hipHostFree(start_host);
         start_read = false;
-        start_host = nullptr;
+        start_host = start_dev = nullptr;
     }
 
     const TensorRec* find(const std::string& name, bool required = true)
@@ -1640,6 +1646,8 @@ int32_t tllm_session_setup(tllm_session_t s, int32_t batch_size, int32_t max_inp
     return tllm_session_setup_beam(s, batch_size, 1, max_input_len, max_new_tokens);
 }
 
+static int32_t setup_runtime(tllm_session_t s, int32_t batch_size, int32_t beam_width, int32_t max_input_len, int32_t max_new_tokens);
+
 int32_t tllm_session_setup_beam(tllm_session_t s, int32_t batch_size, int32_t beam_width, int32_t max_input_len,
     int32_t max_new_tokens)
 {
@@ -1661,6 +1669,17 @@ int32_t tllm_session_setup_beam(tllm_session_t s, int32_t batch_size, int32_t be
             max_input_len + max_new_tokens);
         return 1;
     }
+    const int32_t rc = setup_runtime(s, batch_size, beam_width, max_input_len, max_new_tokens);
+    if (rc)
+    {
+        s->free_runtime(); // what was made so far is given back, and later calls are told to set up first
+        (void) hipGetLastError(); // (told: not the next launch's)
+    }
+    return rc;
+}
+
+static int32_t setup_runtime(tllm_session_t s, int32_t batch_size, int32_t beam_width, int32_t max_input_len, int32_t max_new_tokens)
+{
     s->free_runtime();
     s->Bc = batch_size;
     s->beam = beam_width;
