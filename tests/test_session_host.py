@@ -79,6 +79,46 @@ def set_up_without_memory(stub):  # noqa: F811
     assert stub.pinned_bytes() == 0
 
 
+def knobs_between_requests(stub):  # noqa: F811
+    """A request's steps are launched as the knobs of the decode products and its end token say at the time, and recorded anew only where one of them has changed."""
+    from tensorrt_llm.plugin import capi
+    lib = capi.load_library()
+    s = session('sq_static_pc', batch=6)
+
+    def kernels(**kw):
+        stub.forget()
+        request(s, **kw)
+        return stub.kernels()
+
+    def by_mfma(names):
+        return sum('gemv_mfma' in n for n in names)
+
+    first = kernels()
+    assert by_mfma(first) > 0 and kernels() == first
+    graphs = stub.graphs()
+    assert kernels() == first and stub.graphs() == graphs
+    lib.tllm_gemv_set_mfma_rows(0)
+    by_rows = kernels()
+    assert by_mfma(by_rows) == 0 and stub.graphs() == graphs + 1
+    assert kernels() == by_rows and stub.graphs() == graphs + 1
+    lib.tllm_gemv_set_blocks_per_cu(1)  # (the same kernels, by fewer workgroups)
+    assert kernels() == by_rows and stub.graphs() == graphs + 2
+    lib.tllm_gemv_set_blocks_per_cu(0)
+    lib.tllm_gemv_set_mfma_rows(-1)
+    assert kernels() == first and stub.graphs() == graphs + 3
+    for end_id, new in ((400, 1), (400, 0), (-1, 1)):
+        graphs = stub.graphs()
+        assert kernels(end_id=end_id) == first and stub.graphs() == graphs + new, end_id
+    # a step of the caller's own is replayed under the same rule
+    for rows, mfma in ((0, False), (0, False), (5, True)):
+        lib.tllm_gemv_set_mfma_rows(rows)
+        s.context(np.full((6, S), 3, np.int32), np.full(6, S, np.int32))
+        stub.forget()
+        s.step(1, use_graph=True)
+        assert (by_mfma(stub.kernels()) > 0) == mfma, rows
+    s.close()
+
+
 if __name__ == '__main__':
     sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
     globals()[sys.argv[2]](Stub(sys.argv[1]))
@@ -89,3 +129,6 @@ else:
 
     def test_set_up_without_memory(stub):  # noqa: F811
         run(stub, 'set_up_without_memory')
+
+    def test_knobs_between_requests(stub):  # noqa: F811
+        run(stub, 'knobs_between_requests')

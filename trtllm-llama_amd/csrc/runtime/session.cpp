@@ -259,6 +259,7 @@ struct tllm_session
     hipStream_t graph_stream = nullptr;
     int graph_end_id = -1;         // baked into the captured sampler node
     uint64_t graph_comm_gen = 0;   // comm::p2p::generation() the step graph was captured under
+    int graph_mfma_rows = 0, graph_blocks_per_cu = 0; // gemv_mfma_min_rows and gemv_tune_blocks_per_cu as the captured launches were chosen by them
     uint64_t comm_err_seen = 0;    // comm::p2p::error_generation() at this session's last check_comm
     hipStream_t own_stream = nullptr; // used when the caller passes the NULL stream (it cannot be captured)
 
@@ -289,6 +290,13 @@ struct tllm_session
         if (!own_stream)
             (void) hipStreamCreate(&own_stream);
         return own_stream;
+    }
+
+    // The captured step is what an eager one on `st` would launch now: the same end token, choice of products and, between ranks, transport (enabled / fused seam / a re-created region)
+    bool graph_holds(hipStream_t st) const
+    {
+        return graph && graph_stream == st && graph_end_id == end_id && graph_mfma_rows == gemv_mfma_min_rows && graph_blocks_per_cu == gemv_tune_blocks_per_cu
+            && (tp <= 1 || graph_comm_gen == comm::p2p::generation());
     }
 
     template <typename F>
@@ -2071,9 +2079,7 @@ int32_t tllm_session_step(tllm_session_t s, int32_t n_steps, int32_t use_graph, 
         return 1;
     }
     hipStream_t st = s->pick(stream);
-    // a graph captured while the transport was in another state (enabled / fused seam / a re-created region) holds launches
-    // that no longer match what an eager step would issue: capture again
-    if (use_graph && (!s->graph || s->graph_stream != st || s->graph_end_id != s->end_id || (s->tp > 1 && s->graph_comm_gen != comm::p2p::generation())))
+    if (use_graph && !s->graph_holds(st))
     {
         if (s->graph)
         {
@@ -2101,6 +2107,8 @@ int32_t tllm_session_step(tllm_session_t s, int32_t n_steps, int32_t use_graph, 
         s->graph_stream = st;
         s->graph_end_id = s->end_id;
         s->graph_comm_gen = comm::p2p::generation();
+        s->graph_mfma_rows = gemv_mfma_min_rows;
+        s->graph_blocks_per_cu = gemv_tune_blocks_per_cu;
     }
     for (int i = 0; i < n_steps; ++i)
     {
@@ -2180,8 +2188,8 @@ static int32_t generate_once(tllm_session_t s, const int32_t* input_ids, const i
     int produced = max_new_tokens > 0 ? 1 : 0; // tokens generated per sequence (the prompt pass yields the first)
     if (max_new_tokens > 1)
     {
-        // the first request's first generation step eagerly (also warms lazily-initialised state), the rest from the graph
-        RUN(tllm_session_step(s, 1, s->graph && s->graph_stream == st, stream));
+        // without a graph that still holds the first generation step eagerly (also warms lazily-initialised state), the rest from the graph
+        RUN(tllm_session_step(s, 1, s->graph_holds(st), stream));
         produced = 2;
         if (max_new_tokens > 2)
         {
