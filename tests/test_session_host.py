@@ -119,6 +119,18 @@ def knobs_between_requests(stub):  # noqa: F811
     s.close()
 
 
+def prompts_on_streams_in_turn(stub):  # noqa: F811
+    """A prompt waits until the one before it has been read from pinned memory, on whichever stream, and for nothing else on the device."""
+    s = session()
+    for stream in (0, 64, 64, 128, 0):
+        before = stub.device_syncs(), stub.stream_syncs(), stub.event_syncs()
+        s.context(np.full((1, S), 3, np.int32), np.full(1, S, np.int32), stream=stream)
+        assert (stub.device_syncs(), stub.stream_syncs(), stub.event_syncs()) == (before[0], before[1], before[2] + 1), stream
+    device, events = stub.device_syncs(), stub.event_syncs()
+    s.close()
+    assert stub.device_syncs() == device and stub.event_syncs() == events + 1  # (ahead of giving the memory back)
+
+
 if __name__ == '__main__':
     sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
     globals()[sys.argv[2]](Stub(sys.argv[1]))
@@ -132,3 +144,6 @@ else:
 
     def test_knobs_between_requests(stub):  # noqa: F811
         run(stub, 'knobs_between_requests')
+
+    def test_prompts_on_streams_in_turn(stub):  # noqa: F811
+        run(stub, 'prompts_on_streams_in_turn')

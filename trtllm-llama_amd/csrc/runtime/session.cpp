@@ -223,8 +223,7 @@ struct tllm_session
     // What a request starts from (lengths, ids, mask, flags) side by side on the device and as the host writes it, in pinned memory: one launch brings it over
     int32_t *start_dev = nullptr, *start_host = nullptr;
     size_t start_ints = 0;
-    bool start_read = false;         // a launch on start_stream reads start_host, or has read it
-    hipStream_t start_stream = nullptr;
+    hipEvent_t start_read = nullptr; // behind the last launch that reads start_host
     int32_t* start_of(const void* dev) const
     {
         return start_host + (static_cast<const int32_t*>(dev) - start_dev);
@@ -366,10 +365,13 @@ struct tllm_session
     void free_start()
     {
         if (start_read)
-            (void) hipDeviceSynchronize(); // (a request may still be under way)
+        {
+            (void) hipEventSynchronize(start_read);
+            (void) hipEventDestroy(start_read);
+        }
         if (start_host)
             (void) hipHostFree(start_host);
-        start_read = false;
+        start_read = nullptr;
         start_host = start_dev = nullptr;
     }
 
@@ -1782,6 +1784,7 @@ static int32_t setup_runtime(tllm_session_t s, int32_t batch_size, int32_t beam_
         RUN(s->dalloc(&s->start_dev, s->start_ints * 4));
         HIP_OK(hipMemset(s->start_dev, 0, s->start_ints * 4));
         HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&s->start_host), s->start_ints * 4, hipHostMallocDefault));
+        HIP_OK(hipEventCreateWithFlags(&s->start_read, hipEventDisableTiming));
         size_t at = 0;
         for (auto& part : parts)
         {
@@ -2005,8 +2008,7 @@ static int upload_prompt(tllm_session_t s, const int32_t* input_ids, const int32
             set_error("session: input_lengths[%d]=%d out of range [1, %d]", b, input_lengths[b], S);
             return 1;
         }
-    if (s->start_read) // (by the request before)
-        HIP_OK(s->start_stream == st ? hipStreamSynchronize(st) : hipDeviceSynchronize());
+    HIP_OK(hipEventSynchronize(s->start_read)); // the request before has read its own, whichever stream it is on
     std::fill_n(s->start_host, s->start_of(s->ids_in) - s->start_host, 0); // (flags, tickets: the in-launch merge re-arms itself per launch, this covers a step that never finished)
     int32_t *lens = s->start_of(s->in_len), *mask = s->start_of(s->masked), *out = s->start_of(s->out_ids), *ids = s->start_of(s->ids_in);
     std::fill_n(s->start_of(s->seq_len), B, S);
@@ -2039,8 +2041,7 @@ static int upload_prompt(tllm_session_t s, const int32_t* input_ids, const int32
     else
         std::copy_n(input_ids, n_ids, ids);
     RUN(launch_fetch(s->start_dev, s->start_host, (s->ids_in - s->start_dev) + (int64_t) (n_ids + 3) / 4 * 4, st));
-    s->start_read = true;
-    s->start_stream = st;
+    HIP_OK(hipEventRecord(s->start_read, st));
     std::vector<float> cum;
     if (W > 1)
     {
