@@ -527,6 +527,33 @@ def tall_tiles(stub):
         s.release('a')
 
 
+def expected_rows(stub):
+    """Tiles of grouped products follow the rows that a group is expected to have: choices of identity experts are none; a little over two tiles of 128 x 256 rather than two of 256 x 256."""
+    import rofozen_cases as M
+    import ruzinex_cases as Z
+
+    class Zeros:  # (nothing is computed)
+        standard_normal = staticmethod(lambda shape: np.zeros(shape, np.float32))
+        uniform = staticmethod(lambda lo, hi, size=None: np.full(size, lo, np.float32))
+    np.random.default_rng = lambda seed: Zeros
+
+    def forms(cases, layer, width, tokens):
+        s = engine(cases.make_config([layer], width=width), cases, max_tokens=4096, max_sequences=1)
+        stub.forget()
+        step(s, 'a', tokens, 0)
+        return tuple(k for k in stub.kernels() if re.search(r'gemm_glds_kernelI.*Lb1E|tall|wide_kernelI.*Lb1E', k))[-2:]
+
+    mamba = dict(heads=2, vdim=8, state=16, groups=1)
+    for tokens in (96, 160, 200):
+        with_identity = forms(M, M.mamba_layer(**mamba, mlp=M.moe(experts=8, identity=8, top=8, count=1, keep=1, ff=576)), 512, tokens)
+        half, all_ = (forms(M, M.mamba_layer(**mamba, mlp=M.moe(experts=8, identity=0, top=top, count=1, keep=1, ff=576)), 512, tokens) for top in (4, 8))
+        assert with_identity == half, (tokens, with_identity, half)
+        assert tokens != 160 or half != all_, (half, all_)
+    layer = Z.layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=Z.moe(experts=32, top=4, ff=1408, shared=0))
+    for tokens, want in ((1600, 'wide_kernelILi4'), (2304, 'gemm_glds_kernelILi4ELi2ELi4ELi2ELi2E'), (2560, 'gemm_glds_kernelILi4ELi2ELi4ELi2ELi2E')):
+        assert want in forms(Z, layer, 2048, tokens)[-1], (tokens, forms(Z, layer, 2048, tokens))
+
+
 def who_sums(stub):
     """The experts' rows of few tokens are summed by the norm behind them, very many of them by a launch of its own."""
     import narurax_cases as N
@@ -620,6 +647,9 @@ else:
 
     def test_tall_tiles_of_grouped_products(stub):
         run(stub, 'tall_tiles')
+
+    def test_expected_rows_of_grouped_products(stub):
+        run(stub, 'expected_rows')
 
     def test_tiles_of_grouped_products(stub):
         run(stub, 'group_tiles')

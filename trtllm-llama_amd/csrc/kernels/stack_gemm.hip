@@ -724,10 +724,13 @@ inline double expected_tiles(int m, int high)
     return tiles;
 }
 // The tiles of a grouped product of gemm_wide_impl.h by what they are expected to take, us: rounds of the chip x (a tile's launch, first requests and results, and its K-tiles), or
-// the weights' way from HBM (5.1 TB/s), whichever is longer, rounded off between the two.  Fitted to 180 products of 8 .. 64 groups of 40 .. 600 rows, N 512 .. 5504, K 512 .. 4096,
-// cold weights, of each form, within 6 - 11 %; the forms that it picks have 0.91 of the time that the pick of one shape by rounds and area had, the best ones 0.90.
-// us, 128 x 256 / 256 x 256 / up to 288 x 192: 32 groups of 256 rows, 5504, 4096 476 / 523 / 390, 4096, 2752 272 / 295 / 216; of 216, 2816, 2048 122 / 130 / 111, 2048, 1408 58 / 44 / 63;
-// of 375, 4224, 3072 392 / 400 / 338; of 94 184 / 192 / 166; of 128, 2816, 2048 97 / 117 / 100, 2048, 1408 46 / 39 / 46.
+// the weights' way from HBM (5.1 TB/s), whichever is longer, rounded off between the two.  A product by itself may be off by a third, where its random groups just do or don't make
+// another round; what counts is the form.  Checked on 1639 products of 8 .. 64 groups of 40 .. 560 rows, N 704 .. 5504, K 512 .. 4096, cold weights, each with sizes spread by their root (as
+// a balanced router's choices are: 120 rows +- 10) and by another eighth: they take 0.92 of the time of the forms that rounds and area picked (128 x 128, 128 x 256, lock-step 256 x 256); 2
+// in 100, most of which cross from one round to the next, take over 1.03 of it.  A round of few tiles costs a whole one: counted in parts it picked no better.
+// us, 128 x 256 / 256 x 256 / up to 288 x 192, 32 groups of 120 rows, 2816, 2048 94.5 / 110 / 94, of 128 111 / 116 / 95, of 160 112 / 121 / 99, of 216 121 / 122 / 107 (in a step, of 120: 102
+// the first, 97 the last); 2048, 1408 63 / 44 / 57, 62 / 46 / 57, 61 / 51 / 63, 64 / 54 / 78, of 288 89 / 98 / 97; of 256, 5504, 4096 476 / 523 / 390, 4096, 2752 272 / 295 / 216; of 375, 4224, 3072
+// 392 / 400 / 338.
 enum GroupForm
 {
     GROUP_128x128, // up to 64 rows
@@ -754,7 +757,7 @@ GroupForm pick_group_form(const GemmParams& g, int m)
     };
     if (m <= 64)
         offer(GROUP_128x128, us(128, 128, 5.5, 0.45));
-    offer(GROUP_256x256, us(256, 256, 7.5, m + 1.5 * std::sqrt(m) <= 128 ? 0.95 : 1.36));
+    offer(GROUP_256x256, us(256, 256, 9.5, m + 1.5 * std::sqrt(m) <= 128 ? 0.95 : 1.42));
     if (wide::tall_serves(g))
         offer(GROUP_TALL, us(wide::TALL_BM, wide::TALL_BN, 7.1, 0.34 + 0.004 * std::min<double>(wide::TALL_BM, m / expected_tiles(m, wide::TALL_BM))));
     return form;

@@ -1942,7 +1942,7 @@ int32_t tllm_stack_step(tllm_stack_t s, const tllm_stack_batch_t* b, float* logi
         u.stride_w = (int64_t) up_cols * Wd;
         u.group_off = mp.group_off;
         u.group_total = (int) pairs;
-        u.group_rows = (int) std::min<int64_t>(T, (pairs + l.experts - 1) / l.experts);
+        u.group_rows = (int) std::min<int64_t>(T, (pairs + l.experts + l.identity - 1) / (l.experts + l.identity)); // (identity experts' choices are no rows)
         StackGemmParams dn;
         dn.dtype = s->dtype;
         dn.out_f32 = 1;
