@@ -22,7 +22,7 @@ std::map<void*, size_t> g_device, g_pinned;
 std::map<const void*, std::string> g_names;
 std::string g_launched, *g_captured = nullptr; // (a graph is the names of its kernels)
 size_t g_live = 0, g_budget = ~size_t(0), g_pinned_budget = ~size_t(0), g_largest = 0;
-int g_host_mallocs = 0, g_syncs = 0, g_stream_syncs = 0, g_event_syncs = 0, g_graphs = 0;
+int g_host_mallocs = 0, g_syncs = 0, g_stream_syncs = 0, g_event_syncs = 0, g_event_records = 0, g_graphs = 0, g_fail_launches = 0;
 hipError_t g_last = hipSuccess;
 
 hipError_t done(hipError_t e)
@@ -62,6 +62,8 @@ int stub_host_mallocs() { return g_host_mallocs; }
 int stub_device_syncs() { return g_syncs; }
 int stub_stream_syncs() { return g_stream_syncs; }
 int stub_event_syncs() { return g_event_syncs; }
+int stub_event_records() { return g_event_records; }
+void stub_fail_launches(int on) { g_fail_launches = on; }
 int stub_graphs() { return g_graphs; } // instantiated so far
 size_t stub_pinned_bytes()
 {
@@ -100,7 +102,7 @@ hipError_t hipMemsetAsync(void*, int, size_t, hipStream_t) { return hipSuccess; 
 hipError_t hipEventCreate(hipEvent_t* e) { return *e = reinterpret_cast<hipEvent_t>(new int(0)), hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { return delete reinterpret_cast<int*>(e), hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return ++g_event_records, hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return ++g_event_syncs, hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.f, hipSuccess; } // (all kernels are as quick)
 hipError_t hipDeviceSynchronize() { return ++g_syncs, hipSuccess; }
@@ -140,7 +142,7 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
     if (it != g_names.end() && it->second.find("deliver_kernel") != std::string::npos)
         std::memset(*static_cast<void**>(args[1]), 0, (size_t) grid.x * grid.y * 8); // every part's choice
     (g_captured ? *g_captured : g_launched) += (it == g_names.end() ? std::string("?") : it->second) + "\n";
-    const bool fits = grid.x && grid.y && grid.z && (uint64_t) grid.x * block.x < (1ull << 32) && grid.y <= 65535 && grid.z <= 65535;
+    const bool fits = !g_fail_launches && grid.x && grid.y && grid.z && (uint64_t) grid.x * block.x < (1ull << 32) && grid.y <= 65535 && grid.z <= 65535;
     return done(fits ? hipSuccess : hipErrorInvalidConfiguration);
 }
 hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t shared, hipStream_t stream)

@@ -126,6 +126,19 @@ def prompts_on_streams_in_turn(stub):  # noqa: F811
         before = stub.device_syncs(), stub.stream_syncs(), stub.event_syncs()
         s.context(np.full((1, S), 3, np.int32), np.full(1, S, np.int32), stream=stream)
         assert (stub.device_syncs(), stub.stream_syncs(), stub.event_syncs()) == (before[0], before[1], before[2] + 1), stream
+    # a whole request waits for its tokens, and for its stream where it fails: nothing is left to be waited for
+    records, before = stub.event_records(), stub.device_syncs()
+    for stream in (64, 0):
+        request(s, stream=stream)
+    assert (stub.event_records(), stub.device_syncs()) == (records, before)
+    streams = stub.stream_syncs()
+    stub.fail_launches(1)
+    with pytest.raises(RuntimeError, match='launch failed'):
+        request(s)
+    stub.fail_launches(0)
+    assert (stub.event_records(), stub.device_syncs(), stub.stream_syncs()) == (records, before, streams + 1)
+    s.context(np.full((1, S), 3, np.int32), np.full(1, S, np.int32))
+    assert stub.event_records() == records + 1
     device, events = stub.device_syncs(), stub.event_syncs()
     s.close()
     assert stub.device_syncs() == device and stub.event_syncs() == events + 1  # (ahead of giving the memory back)

@@ -223,7 +223,7 @@ struct tllm_session
     // What a request starts from (lengths, ids, mask, flags) side by side on the device and as the host writes it, in pinned memory: one launch brings it over
     int32_t *start_dev = nullptr, *start_host = nullptr;
     size_t start_ints = 0;
-    hipEvent_t start_read = nullptr; // behind the last launch that reads start_host
+    hipEvent_t start_read = nullptr; // behind the last launch that reads start_host and that its call did not wait for
     int32_t* start_of(const void* dev) const
     {
         return start_host + (static_cast<const int32_t*>(dev) - start_dev);
@@ -1995,7 +1995,8 @@ static int check_comm(tllm_session_t s)
     return 0;
 }
 
-static int upload_prompt(tllm_session_t s, const int32_t* input_ids, const int32_t* input_lengths, hipStream_t st)
+// waited_for: the caller does not return before the stream is through (an event costs a small request 9 us of 530)
+static int upload_prompt(tllm_session_t s, const int32_t* input_ids, const int32_t* input_lengths, hipStream_t st, bool waited_for)
 {
     // input_ids / input_lengths describe the Bc prompts; the per-sequence generation state is tiled over the beam
     // (generation.py:898-915 _tile_beam_width) - the prompt itself runs once per batch entry
@@ -2041,7 +2042,8 @@ static int upload_prompt(tllm_session_t s, const int32_t* input_ids, const int32
     else
         std::copy_n(input_ids, n_ids, ids);
     RUN(launch_fetch(s->start_dev, s->start_host, (s->ids_in - s->start_dev) + (int64_t) (n_ids + 3) / 4 * 4, st));
-    HIP_OK(hipEventRecord(s->start_read, st));
+    if (!waited_for)
+        HIP_OK(hipEventRecord(s->start_read, st));
     std::vector<float> cum;
     if (W > 1)
     {
@@ -2057,6 +2059,14 @@ static int upload_prompt(tllm_session_t s, const int32_t* input_ids, const int32
     return 0;
 }
 
+static int run_prompt(tllm_session_t s, const int32_t* input_ids, const int32_t* input_lengths, hipStream_t st, bool waited_for)
+{
+    RUN(upload_prompt(s, input_ids, input_lengths, st, waited_for));
+    RUN(s->run_context(st));
+    RUN(s->run_sampler(0, st));
+    return 0;
+}
+
 int32_t tllm_session_context(tllm_session_t s, const int32_t* input_ids, const int32_t* input_lengths,
     tllm_stream_t stream)
 {
@@ -2065,11 +2075,7 @@ int32_t tllm_session_context(tllm_session_t s, const int32_t* input_ids, const i
         set_error("tllm_session_context: call tllm_session_setup first");
         return 1;
     }
-    hipStream_t st = s->pick(stream);
-    RUN(upload_prompt(s, input_ids, input_lengths, st));
-    RUN(s->run_context(st));
-    RUN(s->run_sampler(0, st));
-    return 0;
+    return run_prompt(s, input_ids, input_lengths, s->pick(stream), false);
 }
 
 int32_t tllm_session_step(tllm_session_t s, int32_t n_steps, int32_t use_graph, tllm_stream_t stream)
@@ -2133,7 +2139,7 @@ int32_t tllm_session_fake_context(tllm_session_t s, int32_t length, uint32_t see
     const int B = s->B, S = s->max_in;
     std::vector<int32_t> ids((size_t) s->Bc * S, 3), lens(s->Bc, length);
     // a padded prompt of `length` real tokens: slots [length, max_in) are masked
-    RUN(upload_prompt(s, ids.data(), lens.data(), st));
+    RUN(upload_prompt(s, ids.data(), lens.data(), st, false));
     for (int i = 0; i < s->num_layers; ++i)
         RUN(launch_fill_random(s->layers[i].kv, s->int8_kv ? DT_INT8 : DT_HALF, s->kv_elems, seed + 7919u * i, 1.0f, st));
     RUN(s->run_sampler(0, st)); // prepares the RoPE row of the first generation step (the ids are overwritten next)
@@ -2151,11 +2157,15 @@ int32_t tllm_session_generate(tllm_session_t s, const int32_t* input_ids, const 
     // A bounded wait of the one-launch projection + attention expired (its grid was not resident at once - another queue's kernels
     // held CUs): the session has fallen back to the two-launch path, the tokens behind the expired wait are invalid.  Greedy
     // generation is a function of the prompt alone, every cache slot is rewritten before it is read: run the request again.
-    const int32_t rc = generate_once(s, input_ids, input_lengths, max_new_tokens, end_id, pad_id, output_ids, stream);
-    if (rc != kFusedTimedOut)
-        return rc;
-    s->fused_retries += 1;
-    return generate_once(s, input_ids, input_lengths, max_new_tokens, end_id, pad_id, output_ids, stream) ? 1 : 0;
+    int32_t rc = generate_once(s, input_ids, input_lengths, max_new_tokens, end_id, pad_id, output_ids, stream);
+    if (rc == kFusedTimedOut) // (known behind a wait for the stream)
+    {
+        s->fused_retries += 1;
+        rc = generate_once(s, input_ids, input_lengths, max_new_tokens, end_id, pad_id, output_ids, stream) ? 1 : 0;
+    }
+    if (rc && s && s->B)
+        (void) hipStreamSynchronize(s->pick(stream)); // (with its tokens a request has waited by itself: upload_prompt)
+    return rc;
 }
 
 int32_t tllm_session_fused_retries(tllm_session_t s)
@@ -2185,7 +2195,7 @@ static int32_t generate_once(tllm_session_t s, const int32_t* input_ids, const i
         (void) hipGraphExecDestroy(s->graph);
         s->graph = nullptr;
     }
-    RUN(tllm_session_context(s, input_ids, input_lengths, stream));
+    RUN(run_prompt(s, input_ids, input_lengths, st, true));
     int produced = max_new_tokens > 0 ? 1 : 0; // tokens generated per sequence (the prompt pass yields the first)
     if (max_new_tokens > 1)
     {
