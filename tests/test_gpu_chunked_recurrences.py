@@ -83,9 +83,12 @@ def test_decays_from_none_to_all_in_one_chunk(kind):
 def test_a_row_without_finite_numbers_leaves_the_earlier_ones_alone(kind, dtype, what, where):
     """Row `where` of a request is NaN in every channel, or its values overflow: the rows before it, in the same chunk too, are what the oracle
     has for the prompt that ends there, and the request beside it is untouched.  (The last place is a chunk of one row.)"""
-    dim, vdim = 64, 24
+    bad_row(kind, dtype, what, where, 64, 24, 97)
+
+
+def bad_row(kind, dtype, what, where, dim, vdim, rows):
     mod, cfg, _ = KINDS[kind](dim, vdim)
-    toks, other = mod.tokens_for(cfg, 97, 3), mod.tokens_for(cfg, 20, 4)
+    toks, other = mod.tokens_for(cfg, rows, 3), mod.tokens_for(cfg, 20, 4)
     bad = next(t for t in range(cfg['vocab']) if t not in toks and t not in other)
     w = mod.random_weights(cfg, 11)
     if what == 'row':
@@ -102,16 +105,38 @@ def test_a_row_without_finite_numbers_leaves_the_earlier_ones_alone(kind, dtype,
         else:
             w['l0.mix.v'][:, 0] = tolenex_cases.bf16_round(np.float32(3e38))
     toks[where] = bad
-    got = mod.replay(mod.session_for(cfg, w, dtype), {'b': other, 'a': toks}, [[('b', 20), ('a', 97)]])
+    got = mod.replay(mod.session_for(cfg, w, dtype), {'b': other, 'a': toks}, [[('b', 20), ('a', rows)]])
     assert not np.isfinite(got['a'][where]).all()
     check_request(mod, kind, got['a'][:where], toks[:where], w, cfg, dtype, 'a')
     check_request(mod, kind, got['b'], other, w, cfg, dtype, 'b')
 
 
-# Eight chunks between two barriers (eight_chunk_walk_kernel, dim up to 128): portions that end in, on and behind an eighth chunk, one that begins with carried state, waves without a chunk.
+# Portions of 112 .. 257 rows: around eight chunks, one that begins with carried state (which walk a step of them has: test_stack_host_runtime.py).
 @pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
 @pytest.mark.parametrize('dim,vdim', [(64, 24), (128, 16)])
 @pytest.mark.parametrize('kind', ['hgrn2', 'mamba2'])
 def test_portions_around_eight_chunks(kind, dim, vdim, dtype, monkeypatch):
     monkeypatch.setitem(SCHEDULES, 'eights', [[('a', 112), ('b', 128)], [('a', 129), ('b', 32)], [('a', 127), ('b', 257)], [('a', 144), ('b', 1)]])
     run(kind, dim, vdim, dtype, 'eights')
+
+
+# The walk of eight chunks between two barriers: full turns and one short of them, entries beside the longest that end in, on and behind a turn or have a single row, carried state; 64 rows
+# of state from 46 chunks (Mamba-2: 24) on.
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('dim,vdim', [(64, 24), (128, 16)])
+@pytest.mark.parametrize('kind', ['hgrn2', 'mamba2'])
+def test_turns_of_eight_chunks(kind, dim, vdim, dtype, monkeypatch):
+    steps = EIGHT_CHUNKS[dim]
+    monkeypatch.setitem(SCHEDULES, 'turns', steps)
+    run(kind, dim, vdim, dtype, 'turns')
+
+
+EIGHT_CHUNKS = {128: [[('a', 128), ('b', 113)], [('a', 129), ('b', 241), ('c', 1)], [('a', 1), ('b', 16), ('c', 313)]], 64: [[('a', 40)], [('a', 752), ('b', 129)]]}
+
+
+@pytest.mark.parametrize('where', [33, 47, 112])
+@pytest.mark.parametrize('what', ['row', 'value'])
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('kind', ['hgrn2', 'mamba2'])
+def test_a_row_without_finite_numbers_in_a_turn_of_eight_chunks(kind, dtype, what, where):
+    bad_row(kind, dtype, what, where, 128, 16, 113)

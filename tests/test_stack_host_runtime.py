@@ -554,6 +554,53 @@ def expected_rows(stub):
         assert want in forms(Z, layer, 2048, tokens)[-1], (tokens, forms(Z, layer, 2048, tokens))
 
 
+def walks_of_portions(stub):
+    """Chunked recurrences take the walk of eight chunks a turn where the longest entry fills its turns and there are no more workgroups than the CUs have room for; the sizes of
+    test_gpu_chunked_recurrences.py."""
+    import rofozen_cases as M
+    import test_gpu_chunked_recurrences as G
+    import tolenex_cases as H
+
+    class Zeros:  # (nothing is computed)
+        standard_normal = staticmethod(lambda shape: np.zeros(shape, np.float32))
+        uniform = staticmethod(lambda lo, hi, size=None: np.full(size, lo, np.float32))
+    np.random.default_rng = lambda seed: Zeros
+
+    def eight(cases, layer, entries):
+        s = engine(cases.make_config([layer]), cases, max_tokens=sum(entries) + 64 * len(entries), max_sequences=len(entries), max_batch_tokens=sum(entries))
+        stub.forget()
+        s.step([(i, [1] * n, []) for i, n in enumerate(entries)])
+        walks = [k for k in stub.kernels() if 'chunk_walk_kernel' in k]
+        assert len(walks) == 1
+        return 'eight_chunk_walk_kernel' in walks[0]
+
+    def hgrn2(heads, dim, vdim):
+        return H, H.hgrn2_layer(heads=heads, dim=dim, vdim=vdim)
+
+    def mamba2(heads, dim, vdim):
+        return M, M.mamba_layer(heads=heads, vdim=vdim, state=dim, groups=2)
+
+    # up to one workgroup a CU
+    for kind in (hgrn2, mamba2):
+        for rows, want in ((32, False), (112, False), (113, True), (128, True), (129, False), (208, False), (209, True), (256, True), (257, False), (304, False), (305, True), (384, True),
+                           (385, False), (400, False), (401, True), (497, True), (1021, True)):
+            assert eight(*kind(16, 128, 128), [rows]) == eight(*kind(16, 128, 128), [rows, 1]) == want, (kind, rows)
+        for dim in (192, 256):
+            assert not eight(*kind(2, dim, 16), [1024])
+    # more of them
+    for kind, rows, want in ((hgrn2, 1024, False), (mamba2, 1024, True), (mamba2, 384, True), (mamba2, 385, False), (mamba2, 368, False), (mamba2, 368 + 1, True), (mamba2, 256, False)):
+        assert eight(*kind(16, 128, 128), [rows] * 3) == eight(*kind(16, 128, 128), [rows] + [1] * 3) == want, (kind, rows)
+        assert not eight(*kind(16, 128, 128), [rows] * 5) and not eight(*kind(16, 128, 128), [rows] + [1] * 7)
+    # 64 rows of state
+    for kind, rows, want in ((hgrn2, 704, False), (hgrn2, 720, False), (hgrn2, 721, True), (hgrn2, 768, True), (hgrn2, 769, False), (mamba2, 368, False), (mamba2, 384, True), (mamba2, 721, True)):
+        assert eight(*kind(16, 64, 64), [rows]) == want, (kind, rows)
+        assert not eight(*kind(16, 64, 64), [rows] * 5)
+    for dim, steps in G.EIGHT_CHUNKS.items():
+        for kind in (hgrn2, mamba2):
+            assert [eight(*kind(4, dim, 16), [n for _, n in step]) for step in steps] == [len(step) > 1 for step in steps], (dim, kind)
+    assert eight(*hgrn2(2, 128, 16), [113, 20]) and eight(*mamba2(4, 128, 16), [113, 20])
+
+
 def who_sums(stub):
     """The experts' rows of few tokens are summed by the norm behind them, very many of them by a launch of its own."""
     import narurax_cases as N
@@ -650,6 +697,9 @@ else:
 
     def test_expected_rows_of_grouped_products(stub):
         run(stub, 'expected_rows')
+
+    def test_walks_of_portions(stub):
+        run(stub, 'walks_of_portions')
 
     def test_tiles_of_grouped_products(stub):
         run(stub, 'group_tiles')

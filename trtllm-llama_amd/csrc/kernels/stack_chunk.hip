@@ -11,11 +11,13 @@
 // mode) in both element types.
 //
 // Two launches.  chunk_prepare_kernel / ssm_prepare_kernel: a workgroup per (chunk, head), resp. (chunk, group), all chunks at once: gates, unit
-// norms, the decayed vectors, P, M and T into scratch.  eight_chunk_walk_kernel (HGRN2 and Mamba-2 with D up to 128), chunk_walk_kernel (beyond) and delta_chunk_walk_kernel: a workgroup per (entry, head, 16 columns of V) walks the chunks; its
-// four waves keep the state's rows in turn, 16 at a time, in registers in the MFMA's accumulator layout (lane: column lane & 15, rows 4 (lane >> 4)
-// + i), which is also its B-operand layout when the four K = 4 steps of 16 rows take rows 4 g + i in step i: S, u and v go from product to
-// product without moving, and what comes from scratch is 16 bytes per lane.  One barrier per chunk, where the waves' partial o (and S^T k)
-// meet; the next chunk's operands are in flight under this one's products.
+// norms, the decayed vectors, P, M and T into scratch.  Then a workgroup per (entry, head, 16 columns of V) walks the chunks; its waves keep the
+// state's rows, 16 at a time, in registers in the MFMA's accumulator layout (lane: column lane & 15, rows 4 (lane >> 4) + i), which is also its
+// B-operand layout when the four K = 4 steps of 16 rows take rows 4 g + i in step i: S, u and v go from product to product without moving, and what
+// comes from scratch is 16 bytes per lane.  chunk_walk_kernel (HGRN2 and Mamba-2) and delta_chunk_walk_kernel: four waves, which take the state's 16
+// rows in turn, and one barrier per chunk, where their partial o (and S^T k) meet; the next chunk's operands are in flight under this one's products.
+// eight_chunk_walk_kernel (HGRN2 and Mamba-2, long portions in few workgroups: eight_chunks_serve): eight waves, one to 16 rows, and a barrier per
+// eight chunks.
 //
 // Measured (us, both launches, 16 heads): HGRN2 128 x 128, 1024 rows 1024 -> 57; delta rule 128 x 128, three prompts of 683 rows in all 1740 1193 -> 109;
 // Mamba-2 64 heads 128 x 64, 1021 rows 400 -> 57.
@@ -51,6 +53,7 @@ constexpr int HGRN = CHUNK_HGRN2, DELTA = CHUNK_DELTA, SSM = CHUNK_SSM;
 struct ChunkArgs
 {
     int32_t heads = 0, D = 0, V = 0, groups = 1, entries = 0, slots = 0;
+    int32_t max_count = 0; // rows of the longest entry
     // HGRN: q at proj column h D, f at heads D + h D, v at 2 heads D + h V.  DELTA: x = [q | k | v].  SSM: xbc = [x | B | C], proj = [z | ... | dt]
     const void* proj = nullptr;
     int64_t ldp = 0;
@@ -412,7 +415,7 @@ __device__ __forceinline__ f32x4 lower_product(const f32x4& m, const f32x4& x, i
     return acc;
 }
 
-// HGRN2 and Mamba-2 with D beyond 128.  One workgroup per (entry, head, 16 columns of V): TILES * 64 rows of state (D), wave w keeps rows 16 (w + 4 j) .. + 16
+// HGRN2 and Mamba-2 where eight_chunks_serve says no.  One workgroup per (entry, head, 16 columns of V): TILES * 64 rows of state (D), wave w keeps rows 16 (w + 4 j) .. + 16
 template <int DT, int MODE, int TILES>
 __global__ __launch_bounds__(256) void chunk_walk_kernel(const ChunkArgs a)
 {
@@ -761,7 +764,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_walk_kernel(const ChunkArg
 // it sums chunk w's parts and finishes its rows.  The chain is a multiply-add per chunk, operands are asked for eight chunks ahead in the registers that they have just left, and a SIMD's two
 // waves cover each other.  Bound by the operands' way to the CU (every 16 columns bring 16 KB of q and k a chunk: 17 - 20 bytes per clock) ahead of the MFMAs (68 of 32 clocks on four SIMDs a
 // chunk): 1300 clocks a chunk.  Both launches, us, in brackets with chunk_walk_kernel: HGRN2 16 heads 128 x 128, 1021 rows 57 (69), Mamba-2 64 heads 128 x 64 57 (76).
-// With four waves and a barrier per chunk (chunk_walk_kernel, which larger D keep) a chunk's products, the barrier and the sums over the waves stood one after the
+// With four waves and a barrier per chunk (chunk_walk_kernel) a chunk's products, the barrier and the sums over the waves stood one after the
 // other, 2100 clocks a chunk.  Tried on the way: a wave per chunk with all rows of the state, the state handed on through LDS (63 and 63; four waves 66 and 70: LDS and the fold beside idle MFMAs).
 constexpr int SCAN = 8; // chunks at a time, waves
 template <int DT, int MODE, int TILES>
@@ -952,12 +955,33 @@ inline int launched(const char* what)
     return 0;
 }
 
+// Whether a step's walk is eight_chunk_walk_kernel.  Its turns are of eight chunks, however few of them an entry has left, and its LDS leaves room for one workgroup of D = 128 on a CU or two
+// of 64, where chunk_walk_kernel's keep each other's waits covered: it is for entries that fill their turns, in no more workgroups than CUs.  Both launches by it, chunk_walk_kernel's as 1, bf16,
+// longest entry of 7 / 8 / 9 / 13 / 14 / 16 / 17 / 19 / 24 / 25 / 32 / 64 chunks:
+//   D 128, up to one workgroup a CU  HGRN2 1.02 / .99 / 1.12 / .99 / .96 / .92 / 1.02 / .98 / .89 / .97 / .86 / .84   Mamba-2 1.00 / .97 / 1.08 / .96 / .93 / .90 / .97 / .93 / .84 / .91 / .81 / .74
+//   D 128, up to two                 HGRN2 1.14 / 1.09 / 1.29 / 1.11 / 1.09 / 1.04 / 1.18 / 1.13 / 1.02 / 1.14 / 1.01 / .98   Mamba-2 1.10 / 1.06 / 1.25 / 1.09 / 1.05 / .99 / 1.13 / 1.07 / .95 / 1.06 / .93 / .88
+//   D 64, up to one                  HGRN2 1.12 / 1.08 / 1.28 / 1.12 / 1.08 / 1.03 / 1.18 / 1.13 / 1.02 / 1.12 / .99 / .96   Mamba-2 1.08 / 1.06 / 1.21 / 1.08 / 1.06 / 1.01 / 1.13 / 1.08 / .98 / 1.07 / .95 / .90
+//   more workgroups: D 128 up to 1.5, D 64 up to 1.9; a step of 512 rows beside 31 single ones 1.04 - 1.09 and 1.5 - 1.8
+// (four and more full rounds of them for Mamba-2, 0.92 at best, are left to chunk_walk_kernel: three are 1.07 - 1.4.)
+template <int MODE>
+bool eight_chunks_serve(const ChunkArgs& a)
+{
+    const int64_t wgs = (int64_t) a.entries * a.heads * ((a.V + 15) / 16), cus = launch_util::device_cus();
+    const int chunks = (a.max_count + R - 1) / R, turns = (chunks + SCAN - 1) / SCAN;
+    if (MODE == DELTA || a.D > 128)
+        return false;
+    if (a.D == 128 && wgs <= cus)
+        return chunks >= 6 * turns + 2;
+    const bool full = 15 * turns <= 2 * chunks; // 7.5 chunks a turn
+    return MODE == SSM ? full && chunks >= 24 && wgs <= (a.D == 128 ? 2 : 1) * cus : full && chunks >= 46 && a.D == 64 && wgs <= cus;
+}
+
 template <int DT, int MODE>
 void walk(const ChunkArgs& a, hipStream_t stream)
 {
     const dim3 grid(a.entries, a.heads, (a.V + 15) / 16);
     if constexpr (MODE != DELTA)
-        if (a.D <= 128)
+        if (eight_chunks_serve<MODE>(a))
         {
             const auto kernel = a.D == 64 ? eight_chunk_walk_kernel<DT, MODE, 1> : eight_chunk_walk_kernel<DT, MODE, 2>;
             const size_t lds = sizeof(f32x4) * 2 * SCAN * 64 * ((size_t) a.D / 16 + 1);
@@ -975,7 +999,13 @@ void walk(const ChunkArgs& a, hipStream_t stream)
         default: return go(delta_chunk_walk_kernel<DT, 4>);
         }
     else
-        a.D == 192 ? go(chunk_walk_kernel<DT, MODE, 3>) : go(chunk_walk_kernel<DT, MODE, 4>);
+        switch (a.D / 64)
+        {
+        case 1: return go(chunk_walk_kernel<DT, MODE, 1>);
+        case 2: return go(chunk_walk_kernel<DT, MODE, 2>);
+        case 3: return go(chunk_walk_kernel<DT, MODE, 3>);
+        default: return go(chunk_walk_kernel<DT, MODE, 4>);
+        }
 }
 
 template <int DT, int MODE>
@@ -1042,6 +1072,7 @@ int launch_stack_chunk_hgrn2(const StackHgrnParams& p, hipStream_t stream)
     a.D = p.dim;
     a.V = p.vdim;
     a.entries = p.entries;
+    a.max_count = p.max_count;
     a.proj = p.proj;
     a.ldp = p.ldp;
     a.f_bias = p.f_bias;
@@ -1065,6 +1096,7 @@ int launch_stack_chunk_delta(const StackDeltaParams& p, hipStream_t stream)
     a.D = p.dim;
     a.V = p.vdim;
     a.entries = p.entries;
+    a.max_count = p.max_count;
     a.xbc = p.x;
     a.ldx = 2 * (int64_t) p.qk_heads * p.dim + (int64_t) p.heads * p.vdim;
     a.decay_raw = p.decay_raw;
@@ -1091,6 +1123,7 @@ int launch_stack_chunk_ssm(const StackSsmParams& p, hipStream_t stream)
     a.D = p.state;
     a.V = p.vdim;
     a.entries = p.entries;
+    a.max_count = p.max_count;
     a.proj = p.proj;
     a.ldp = p.ldp;
     a.xbc = p.xbc;
