@@ -133,8 +133,11 @@ __device__ __forceinline__ float decay_of(float rate, float z)
 constexpr int R = CHUNK_ROWS;
 
 // HGRN2 and delta rule: a workgroup per (chunk, head), D a multiple of 64 up to 256
+// (Rows 0 .. 7 of a chunk meet eight rows of it in the delta rule's P and M, not sixteen, which needs 72 registers if the compiler is held to them: left to itself it takes 82, five
+// workgroups on a CU for six.  us, 16 heads of 128 x 128, 1021 rows, 16 rows always / 82 registers / 72: 25.7 / 24.6 / 24.6; 24 heads, four times 1021 101 / 109 / 98.  HGRN2's P alone is
+// quicker the long way: 32 heads, four times 1021 97 and 105.)
 template <int DT, int MODE>
-__global__ __launch_bounds__(256) void chunk_prepare_kernel(const ChunkArgs a)
+__global__ __launch_bounds__(256, MODE == DELTA ? 6 : 1) void chunk_prepare_kernel(const ChunkArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) float sm[];
     const int D = a.D, h = blockIdx.y, slot = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -207,7 +210,7 @@ __global__ __launch_bounds__(256) void chunk_prepare_kernel(const ChunkArgs a)
 #pragma unroll
         for (int half = 0; half < 2; ++half)
         {
-            const int t = half ? R - 1 - tp : tp, rows = half ? R : R / 2; // (rows: unrolled, as is half)
+            const int t = half ? R - 1 - tp : tp, rows = MODE != DELTA || half ? R : R / 2; // (unrolled, as is half)
             float pa[R], ma[R];
 #pragma unroll
             for (int s = 0; s < R; ++s)
