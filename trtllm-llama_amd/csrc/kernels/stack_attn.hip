@@ -880,14 +880,6 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnPara
         my_lo[rt] = rows_ok ? first_visible(p, pos0 + r0[rt]) / 64 : 0;
         klo_last[rt] = rows_ok ? first_visible(p, pos0 + last) : 0;
     }
-    // The queries' fragments are here: a wait for them inside the walk, where the compiler would leave it, is one for the next unit's K and V, too (they are requested in front of it).
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int m = 0; m < MAPS; ++m)
-#pragma unroll
-            for (int ks = 0; ks < DK; ++ks)
-                asm volatile("" : "+v"(qf[rt][m][ks]));
     const int wg_last = tile * ROWS + ROWS - 1 < count ? tile * ROWS + ROWS - 1 : count - 1;
     // the units the workgroup walks: the ones with kept first keys, then from its first row's first visible key on
     const int lo = first_visible(p, pos0 + tile * ROWS) / 64;
@@ -941,6 +933,16 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnPara
         request(unit_at(0), __builtin_amdgcn_readfirstlane(block_of(unit_at(0))), 0);
         // (in a vector register until behind the next unit's wait: earlier, its own would be one for the requests in front of it)
         int blk_next = n_units > 1 ? block_of(unit_at(1)) : 0;
+        // The queries' fragments are here: a wait for them inside the loop, where the compiler would leave it, is one for the next unit's K and V, too (they are requested in front of it).
+        // Ahead of the first request, their way and the page number's and K's and V's would follow each other: 2.4 % over 1274 steps of up to 8 prompts and 4096 rows, 3 - 7 % of short ones (45 of
+        // those steps took over 1.03 of the time without any such wait; 4 do so, up to 1.05).
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int m = 0; m < MAPS; ++m)
+#pragma unroll
+                for (int ks = 0; ks < DK; ++ks)
+                    asm volatile("" : "+v"(qf[rt][m][ks]));
         for (int v = 0; v < n_units; ++v)
         {
             const int u = unit_at(v);
