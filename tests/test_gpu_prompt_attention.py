@@ -92,6 +92,14 @@ def test_many_workgroups_of_wider_heads(kind, dim, vdim, steps):
     run(kind, 64, 16, dim, vdim, steps)
 
 
+@pytest.mark.parametrize('heads,steps', [(64, [[('a', 200)]]), (32, [[('a', 200), ('b', 90)]]), (32, [[('a', 700)]]), (32, [[('b', 130), ('a', 380)]])],
+                         ids=['shared keys', 'shared keys, two', 'own keys', 'own keys, two'])
+@pytest.mark.parametrize('kind,dim', [('tolenex', 64), ('ruzinex', 128)])
+def test_levels_whose_order_turns(kind, dim, heads, steps):
+    """Up to two workgroups on each of 256 CUs, the lightest first from the fifth (700 rows: the ninth) level of tiles on: two or three levels change places."""
+    run(kind, heads, heads // 4, dim, dim, steps)
+
+
 @pytest.mark.parametrize('page', [32, 128])
 @pytest.mark.parametrize('kind', sorted(KINDS))
 def test_pages_of_other_sizes(kind, page):

@@ -11,6 +11,7 @@
 // Both maps of a differential head run side by side and share the V^T fragments.  fp32: scores, soft cap, softmax state, O.
 #include "dev_utils.h"
 #include "launch_util.h"
+#include "stack_attn_order.h"
 #include "stack_kernels.h"
 #include <algorithm>
 #include <cstdlib>
@@ -838,7 +839,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(const StackAttnPara
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // blockIdx.x = tile level x (entries x heads), heaviest tiles first; inside a level the key/value heads run fastest
     const int per = p.entries * p.heads;
-    const int at = blockIdx.x / per, level = at < turn ? at : turn + tiles - 1 - at, q_ = blockIdx.x % per, e = q_ / p.heads, hi = q_ % p.heads;
+    const int level = prompt_level(blockIdx.x / per, turn, tiles), q_ = blockIdx.x % per, e = q_ / p.heads, hi = q_ % p.heads;
     const int h = p.cross_values ? hi : hi % p.kv_heads * (p.heads / p.kv_heads) + hi / p.kv_heads;
     const int count = p.ent_count[e];
     if (count < min_count)
@@ -1163,8 +1164,8 @@ void launch_prompt(const StackAttnParams& p, int min_count, hipStream_t stream)
     constexpr size_t lds = stages > merge ? stages : merge;
     launch_util::ensure_dynamic_lds(reinterpret_cast<const void*>(&attn_prompt_kernel<MAPS, DK, VT, RT, KS>), lds);
     const int tiles = (p.max_count + 16 * RW * RT - 1) / (16 * RW * RT);
-    const int64_t per = (int64_t) p.entries * p.heads, cus = launch_util::device_cus();
-    const int turn = tiles * per <= 2 * cus ? (int) (cus / per) : tiles;
+    const int64_t per = (int64_t) p.entries * p.heads;
+    const int turn = prompt_turn(tiles, per, launch_util::device_cus());
     hipLaunchKernelGGL((attn_prompt_kernel<MAPS, DK, VT, RT, KS>), dim3((unsigned) (tiles * per)), dim3(256), lds, stream, p, min_count, tiles, turn);
 }
 
