@@ -414,6 +414,21 @@ def two_int8_products(stub):
         assert [bool(re.search('wide_kernelILi3ELi6', x)) for x in stub.kernels()] == [wide], (cfg, m)
 
 
+def int8_products(stub):
+    """SmoothQuant products without a measured choice: the tiles of 128 rows where they save a round or fit better, 256 x 128 at equal counts, one round of 256 x 256 rather than two of 128 x 256."""
+    import test_gpu_wide_half as G
+    from tensorrt_llm.plugin import capi
+    lib = capi.load_library()
+    lib.tllm_gemm.argtypes = [ctypes.POINTER(G.GemmParams), ctypes.c_void_p]
+    for m, n, k, want in ((384, 13824, 5120, 'gemm_sqp'), (512, 11008, 4096, 'gemm_sqp'), (1024, 5120, 5120, 'gemm_sqp'), (2500, 5504, 2048, 'wide_kernelILi3E'), (2500, 6144, 2048, 'wide_kernelILi3E'),
+                          (640, 11008, 4096, 'wide16gemm_glds_kernelILi3ELi2ELi4ELi2ELi2E'), (1400, 11008, 4096, 'wide16gemm_glds_kernelILi3ELi2ELi4ELi2ELi2E'),
+                          (512, 4096, 4096, 'wide16gemm_glds_kernelILi3ELi2ELi4ELi2ELi1E'), (1024, 4096, 4096, 'wide16gemm_glds_kernelILi3ELi2ELi4ELi2ELi1E')):
+        stub.forget()
+        q = G.GemmParams(3, 1, m, n, k, 4096, k, 4096, k, 4096, 4096, 1, 0, 4096, n)
+        assert lib.tllm_gemm(ctypes.byref(q), None) == 0
+        assert want in stub.kernels()[-1], (m, n, k, stub.kernels())
+
+
 def low_rank_pairs(stub):
     """A delta layer's two low-rank pairs are one product of two where one launch serves it; rows of tiles that end inside a stage of 64 go one by one, not by the
     register-staged tiles."""
@@ -718,6 +733,9 @@ else:
 
     def test_two_int8_products(stub):
         run(stub, 'two_int8_products')
+
+    def test_int8_products(stub):
+        run(stub, 'int8_products')
 
     def test_low_rank_pairs(stub):
         run(stub, 'low_rank_pairs')

@@ -58,9 +58,11 @@ constexpr int kWide = 80, kRows128 = 81, kRows128Wide = 82;
 // The tiles of 128 rows by 16 x 16 MFMAs (gemm_wide_impl.h) take the place of the lock-step ones of 32 x 32 wherever results leave in whole 16-byte pieces of fp16; us, cold weights,
 // in brackets what the rule took without them: SmoothQuant 128 x 128 at 1024 / 512 x 4096 x 4096 21.1 / 16.2 (23.9 / 20.6), 128 x 256 at 1400 and 640 x 11008 x 4096 68 and 34.6 (84.7
 // and 46.3), 2048 x 4096 x 11008 84 (91); fp16 128 x 128 at 997 x 4096 x 11008 104 (108), 300 x 4096 x 4096 28.5 (33.0), 128 x 256 at 1400 and 640 x 11008 x 4096 122 and 63.5 (162 and 81.6).
-// Equal counts of 128 x 256 and 256 x 128 (fp16): 62 / 58 at 512 x 11008 x 4096, 64 / 66 at 2048 x 4096 x 4096.
+// Equal counts of 128 x 256 and 256 x 128: fp16 62 / 58 at 512 x 11008 x 4096, 64 / 66 at 2048 x 4096 x 4096; SmoothQuant 45.5 / 39.1 at 384 x 13824 x 5120, 33.4 / 31.8 at 384 x 12288 x 4096,
+// 41.7 / 39.5 at 1024 x 5120 x 5120.  Two rounds of 128 x 256 and one of 256 x 256 (SmoothQuant): 40.2 / 30.9 at 2500 x 5504 x 2048.  Over 308 products of each type (32 .. 4096 rows, N 1024 ..
+// 13824, K 1024 .. 11008, cold weights) the rule's picks take 0.91 (SmoothQuant; fp16 0.95) of the time of its picks without these tiles, none over 1.01 of it, and 1.006 (1.005) of the best's.
 constexpr Shape kShapes[] = {{8, 128, 128, 1.40, 1.80}, {6, 256, 192, 1.0, 1.0}, {2, 256, 256, 1.04, 1.30}, {4, 128, 256, 1.39, 1.60},
-    {kPhased256x128, 256, 128, 1.08, 1.37}, {kRows128, 128, 128, 1.32, 1.33}, {kRows128Wide, 128, 256, 1.09, 1.10}};
+    {kPhased256x128, 256, 128, 1.08, 1.37}, {kRows128, 128, 128, 1.32, 1.50}, {kRows128Wide, 128, 256, 1.09, 1.40}};
 constexpr int kNumCfg = 12;
 
 // the tiles of gemm_wide.hip, ids 80 ..: as launch_gemm_wide
