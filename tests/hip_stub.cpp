@@ -51,6 +51,7 @@ extern "C" {
 void stub_budget(size_t bytes) { g_budget = bytes; }
 void stub_pinned_budget(size_t bytes) { g_pinned_budget = bytes; } // of one allocation
 size_t stub_live() { return g_live; }
+size_t stub_largest() { return g_largest; } // allocation on the device so far
 int stub_has_allocation(size_t bytes)
 {
     for (auto& a : g_device)
@@ -82,6 +83,7 @@ hipError_t hipMalloc(void** p, size_t n)
     *p = std::calloc(1, n ? n : 1); // (large ones are mapped on demand: nothing computes on them)
     g_device[*p] = n;
     g_live += n;
+    g_largest = g_largest < n ? n : g_largest;
     return hipSuccess;
 }
 hipError_t hipFree(void* p) { return release(g_device, p); }

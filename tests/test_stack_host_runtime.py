@@ -31,7 +31,7 @@ class Stub:
     def __init__(self, path):
         self.lib = ctypes.CDLL(path, mode=ctypes.RTLD_GLOBAL)
         self.lib.stub_budget.argtypes = self.lib.stub_has_allocation.argtypes = [ctypes.c_size_t]
-        self.lib.stub_live.restype = self.lib.stub_pinned_bytes.restype = ctypes.c_size_t
+        self.lib.stub_live.restype = self.lib.stub_largest.restype = self.lib.stub_pinned_bytes.restype = ctypes.c_size_t
         self.lib.stub_launched.restype = ctypes.c_char_p
         for p in (os.path.dirname(HERE), os.path.join(os.path.dirname(HERE), 'trtllm-llama_amd'), HERE):
             sys.path.insert(0, p)
@@ -429,6 +429,22 @@ def int8_products(stub):
         assert want in stub.kernels()[-1], (m, n, k, stub.kernels())
 
 
+def cold_weights(stub):
+    """Products are timed on weights that rotate through more than the last-level cache, small ones too; with little memory free on fewer, and are chosen all the same."""
+    from tensorrt_llm.plugin import capi
+    lib = capi.load_library()
+    lib.tllm_gemm_profile.argtypes = [ctypes.c_int32] * 4 + [ctypes.c_void_p] * 3
+    largest = 0
+    for wtype, n, k in ((0, 64, 64), (3, 2752, 1024), (0, 1024, 1024), (0, 4096, 4096)):
+        for budget in (2 ** 64 - 1, 64 << 20):
+            lib.tllm_gemm_tactics_clear()
+            stub.budget(budget)
+            assert lib.tllm_gemm_profile(wtype, 128, n, k, None, None, None) == 0 and lib.tllm_gemm_tactic_lookup(wtype, 128, n, k) > 0, (wtype, n, k)
+            stub.budget(2 ** 64 - 1)
+            largest = max(largest, n * k * (2 if wtype == 0 else 1))
+        assert (384 << 20) - largest <= stub.largest() <= (384 << 20) + 16, (n, k, stub.largest())
+
+
 def low_rank_pairs(stub):
     """A delta layer's two low-rank pairs are one product of two where one launch serves it; rows of tiles that end inside a stage of 64 go one by one, not by the
     register-staged tiles."""
@@ -736,6 +752,9 @@ else:
 
     def test_int8_products(stub):
         run(stub, 'int8_products')
+
+    def test_cold_weights_of_measured_products(stub):
+        run(stub, 'cold_weights')
 
     def test_low_rank_pairs(stub):
         run(stub, 'low_rank_pairs')

@@ -155,9 +155,10 @@ int gemm_profile(int wtype, int M, int N, int K, int* best_cfg, float* best_us, 
     const int es = sq ? 1 : 2;
     const size_t a_bytes = (size_t) M * K * es, w_bytes = (size_t) N * K * es, c_bytes = (size_t) M * N * 2;
     // Each launch has other weights, as a model's layers have: from HBM, not from the caches that the launch before left them in (fp16, 1024 x 4096 x 11008: the whole-K 128 x 128
-    // tile 105 us and the split 256 x 128 one 94, cold; warm the first one won).
+    // tile 105 us and the split 256 x 128 one 94, cold; warm the first one won).  384 MB of them, whatever one takes, pass the last-level cache of 256 MB; with less memory free there are
+    // fewer, and the choice is made on what the caches hold of them.
     constexpr size_t kColdBytes = (size_t) 384 << 20;
-    size_t copies = std::max<size_t>(1, std::min<size_t>(32, kColdBytes / w_bytes));
+    size_t copies = std::max<size_t>(1, kColdBytes / w_bytes);
     char *a = nullptr, *w = nullptr, *c = nullptr;
     float *sc = nullptr, *sr = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
