@@ -934,7 +934,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_glds_kernel(const GemmParam
 }
 
 // Tiles of up to 288 rows x 192 columns, for groups of a few hundred rows: bfloat16, 8 waves of 2 x 4, a wave the row blocks wm, wm + 2, ... and 48 columns.  A group's rows
-// are cut into as few tiles as take them, of equal height in steps of 32 rows; a wave's blocks are a template of the loop, so that a tile fetches and multiplies no more rows than it has.
+// are cut into as few tiles as take them, of equal height in steps of 32 rows; a wave's blocks are a template of the loop, so that a tile fetches and multiplies no more rows than it has
+// (but for tiles of up to 64 rows, which go by the loop of 96).
 //   Bound by the operands' way from L2 (28 bytes per clock and CU) and the weights' from HBM.  Tiles of 128 rows bring a group's weights in two or three times, the last one for
 // a few rows as often as not; 256 x 256 ones once, but a group of a few rows more costs two thirds of another tile, and a tile is a third of a round: that is why a tile is
 // as high as three buffers of A and two of W's 192 columns let it be.  Reads and requests as in the 256 x 256 loop: 1.5 K-tiles ahead, W's buffer handed back within the K-tile.
@@ -995,15 +996,10 @@ struct TallTile
 #pragma unroll
         for (int i = 0; i < L::DMAS; ++i)
             dma<NA>(i, 0, A0, W0);
-        if (nt > 1)
-        {
 #pragma unroll
-            for (int i = 0; i < L::DMAS; ++i)
-                dma<NA>(i, 1, A1, W1);
-            landed<NA>();
-        }
-        else
-            wait_vm_and_meet<0>();
+        for (int i = 0; i < L::DMAS; ++i)
+            dma<NA>(i, 1, A1, W1);
+        landed<NA>();
 #pragma unroll
         for (int i = 0; i < NA; ++i)
 #pragma unroll
@@ -1193,10 +1189,10 @@ int launch_tall_out(const GemmParams& p, hipStream_t stream)
     }
     return 0;
 }
-// p: serves<W_BF16>(p)
+// p: serves<W_BF16>(p); two K-tiles at least (the rule that picks them asks for eight)
 inline bool tall_serves(const GemmParams& p)
 {
-    return p.group_off && !p.resid && !p.bias && p.seam.n_sec == 0 && (p.act == GEMM_ACT_NONE || p.act == GEMM_ACT_RELU2 || p.act >= GEMM_ACT_GATE_SILU) && (p.out_dtype == DT_BFLOAT16 || p.act == GEMM_ACT_NONE);
+    return p.K >= 128 && p.group_off && !p.resid && !p.bias && p.seam.n_sec == 0 && (p.act == GEMM_ACT_NONE || p.act == GEMM_ACT_RELU2 || p.act >= GEMM_ACT_GATE_SILU) && (p.out_dtype == DT_BFLOAT16 || p.act == GEMM_ACT_NONE);
 }
 // p: tall_serves(p)
 inline int launch_tall(const GemmParams& p, hipStream_t stream)
