@@ -558,6 +558,21 @@ def tall_tiles(stub):
         s.release('a')
 
 
+def tall_ungated_tiles(stub):
+    """Experts without a gate on tall tiles, whose results leave as they are: the sizes of test_gpu_group_tiles.py."""
+    import sodudra_cases as S
+    import test_gpu_group_tiles as G
+
+    class Zeros:  # (nothing is computed)
+        standard_normal = staticmethod(lambda shape: np.zeros(shape, np.float32))
+    np.random.default_rng = lambda seed: Zeros
+    s = engine(G.ungated_config(S), S, max_tokens=1024, max_sequences=1)
+    for tokens in G.UNGATED_ROWS:
+        stub.forget()
+        step(s, 'a', tokens, 0)
+        assert any('4tall16gemm_glds_kernelILi4ELi9ELi6ELi1ELi1ELi0E' in k for k in stub.kernels()), tokens
+
+
 def expected_rows(stub):
     """Tiles of grouped products follow the rows that a group is expected to have: choices of identity experts are none; a little over two tiles of 128 x 256 rather than two of 256 x 256."""
     import rofozen_cases as M
@@ -725,6 +740,9 @@ else:
 
     def test_tall_tiles_of_grouped_products(stub):
         run(stub, 'tall_tiles')
+
+    def test_tall_tiles_of_ungated_experts(stub):
+        run(stub, 'tall_ungated_tiles')
 
     def test_expected_rows_of_grouped_products(stub):
         run(stub, 'expected_rows')
