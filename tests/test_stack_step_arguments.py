@@ -72,3 +72,14 @@ def test_lists_that_are_no_whole_numbers_of_32_bits_reach_the_engine_as_numpy_ca
     want = np.empty(4, np.int32)
     want[:] = np.asarray(tokens)
     assert engine.lib.got == [want.tolist()] + WANT[1:]
+
+
+def test_a_table_off_its_alignment_is_copied(engine):
+    room = np.zeros(4 * 6 + 1, np.uint8)
+    table = room[1:].view(np.int32).reshape(2, 3)
+    table[...] = np.reshape(WANT[4], (2, 3))
+    assert not table.flags.aligned and table.flags.c_contiguous
+    at, take = [], engine.lib.tllm_stack_step
+    engine.lib.tllm_stack_step = lambda handle, batch, *a: at.append(batch._obj.block_table) or take(handle, batch, *a)
+    engine.step(*WANT[:4], table, WANT[5])
+    assert engine.lib.got == WANT and at[0] % 4 == 0

@@ -129,7 +129,7 @@ class StackEngine:
                 meta = array.array('i', tokens + counts + pos0 + slots + want_rows)
             except (TypeError, OverflowError):
                 pass
-        if meta is not None and table.dtype == np.int32 and table.flags.c_contiguous:
+        if meta is not None and table.dtype == np.int32 and table.flags.c_contiguous and table.flags.aligned:
             p, p_table = meta.buffer_info()[0], _address(table)
         else:
             meta = np.empty(at[6], np.int32)
