@@ -226,7 +226,8 @@ typedef struct
 } tllm_gemv_params_t;
 
 int32_t tllm_gemv(const tllm_gemv_params_t* p, tllm_stream_t stream);
-/* Test/bench knob: persistent workgroups per CU (0 = occupancy query). */
+/* Test/bench knob: persistent workgroups per CU (0 = occupancy query).  This one and the next hold for every product launched behind the
+ * call; a session's recorded step is recorded anew. */
 void tllm_gemv_set_blocks_per_cu(int32_t n);
 /* Test/bench knob: number of rows (sequences) from which the SmoothQuant decode GEMM runs on the matrix pipe
  * (kernels/gemv_mfma_sq.hip, static activation scales) instead of the skinny vector-ALU kernel: 0 = never, -1 = the default
@@ -237,7 +238,8 @@ void tllm_gemv_set_mfma_rows(int32_t n);
  * SmoothQuant pipeline of kernels/gemm_sqp.hip (20 = 256x192, 42 = 256x128, one tile per workgroup; 63 / 62 their persistent
  * forms, r05; 64 / 65 = 256x128 / 128x128 as two workgroups per tile splitting K, r06; 21..33 are ablations with wrong results on purpose);
  * 50..58: the same pipeline on fp16 operands (50 = 256x192, 54 = 256x128, 55 / 56 persistent, 57 / 58 split-K); 101..106: the weight-only kernel of kernels/gemm_woq.hip (101 = 256x192, 102 = 128x128,
- * 106 = 256x128); -2: the fused SwiGLU GEMM in its one-tile form.  The ids are what tllm_gemm_profile reports. */
+ * 106 = 256x128); 80 / 81 / 82: the 256x256 / 128x128 / 128x256 tiles of 16x16 MFMAs of kernels/gemm_wide.hip, both types;
+ * -2: the fused SwiGLU GEMM in its one-tile form.  The ids are what tllm_gemm_profile reports. */
 void tllm_gemm_set_tile_cfg(int32_t cfg);
 
 /* Kernel-level entry for the prefill GEMMs (kernels/gemm_mfma.hip; M <= 8 goes to the skinny GEMM):
@@ -287,8 +289,9 @@ int64_t tllm_gemm_tactics_export(char* buf, int64_t capacity);
 int32_t tllm_gemm_tactics_import(const char* text);
 void tllm_gemm_tactics_clear(void);
 int32_t tllm_gemm_tactic_lookup(int32_t wtype, int32_t M, int32_t N, int32_t K);
-/* Microbenchmark hook: while set (non-NULL), every workgroup of the phased SmoothQuant GEMM writes {shader cycles, ticks of
- * the constant 100 MHz counter} over its lifetime to device_buffer[2 * workgroup] (uint64) - the clock the chip held. */
+/* Microbenchmark hook: while set (non-NULL), every workgroup of the phased and lock-step SmoothQuant GEMMs and of the tiles of 128 rows
+ * writes {shader cycles, ticks of the constant 100 MHz counter} over its lifetime to device_buffer[2 * workgroup] (uint64) - the clock the
+ * chip held. */
 void tllm_gemm_set_clock_probe(void* device_buffer);
 
 #ifdef __cplusplus
