@@ -729,7 +729,7 @@ inline double expected_tiles(int m, int high)
 // a balanced router's choices are: 120 rows +- 10) and by another eighth: they take 0.92 of the time of the forms that rounds and area picked (128 x 128, 128 x 256, lock-step 256 x 256); 2
 // in 100, most of which cross from one round to the next, take over 1.03 of it.  A round of few tiles costs a whole one: counted in parts it picked no better.
 // us, 128 x 256 / 256 x 256 / up to 288 x 192, 32 groups of 120 rows, 2816, 2048 94.5 / 110 / 94, of 128 111 / 116 / 95, of 160 112 / 121 / 99, of 216 121 / 122 / 107 (in a step, of 120: 102
-// the first, 97 the last); 2048, 1408 63 / 44 / 57, 62 / 46 / 57, 61 / 51 / 63, 64 / 54 / 78, of 288 89 / 98 / 97; of 256, 5504, 4096 476 / 523 / 390, 4096, 2752 272 / 295 / 216; of 375, 4224, 3072
+// the first and 97 the last on one card, 107 and 108 on another); 2048, 1408 63 / 44 / 57, 62 / 46 / 57, 61 / 51 / 63, 64 / 54 / 78, of 288 89 / 98 / 97; of 256, 5504, 4096 476 / 523 / 390, 4096, 2752 272 / 295 / 216; of 375, 4224, 3072
 // 392 / 400 / 338.
 enum GroupForm
 {
